@@ -160,7 +160,7 @@ constexpr int TD_G = 4;    // MFMA k-steps (of 32) per load group: 64 B per lane
 constexpr int TD_SL = 64;  // LDS slots per (wave, query)
 
 __device__ __forceinline__ unsigned td_key(float v, int id) {  // larger = better; empty (id < 0) = 0
-  const unsigned u = __float_as_uint(v);
+  const unsigned u = __float_as_uint(v + 0.f);  // (-0 as 0)
   return id < 0 ? 0u : ((u & 0x80000000u) ? ~u : (u | 0x80000000u));
 }
 __device__ __forceinline__ float td_unkey(unsigned k) {
@@ -451,124 +451,199 @@ topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict_
   st.store(nq, ((size_t)rb * Q + qbase) * K, out_s, out_i);
 }
 
-// Per-query row ranges. ranges [R, 2] (start, end), range_off [Q+1]; rows_per_q_block rows of the
-// query's concatenated ranges per workgroup (grid = (splits, Q)). out [splits, Q, K].
+// A wave's unsorted top-K list in LDS: cs / ci hold TL_SL slots, [0, K) the list, the rest room for what is
+// being added. kth: the K-th best score (-inf while fewer than K rows are in).
+constexpr int TL_SL = 64 + TK_MAX;
+
+struct TopList {
+  float* cs; int* ci;
+  int K, lane;
+  float kth;
+
+  __device__ __forceinline__ void init(float* s, int* i, int k) {
+    cs = s; ci = i; K = k; lane = threadIdx.x & 63; kth = -INFINITY;
+    if (lane < K) { cs[lane] = -INFINITY; ci[lane] = -1; }
+    wave_sync_lds();
+  }
+  // one candidate per lane (id < 0: none); ties at the threshold go to the smaller row id
+  __device__ __forceinline__ void add(float v, int id) {
+    const bool cand = id >= 0 && v >= kth;
+    const unsigned long long m = __ballot(cand);
+    if (!m) return;
+    const int n = __popcll(m);
+    if (n + K > 64) {  // only the best K of the new ones can stay
+      td_cut(cand ? v : -INFINITY, cand ? id : -1, K, lane, cs + 64, ci + 64);
+      const float* s = lane < K ? cs + lane : cs + 64 + (lane - K);
+      const int* i = lane < K ? ci + lane : ci + 64 + (lane - K);
+      v = lane < 2 * K ? *s : -INFINITY;
+      id = lane < 2 * K ? *i : -1;
+    } else {
+      const int pos = K + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+      wave_sync_lds();
+      if (cand) { cs[pos] = v; ci[pos] = id; }
+      wave_sync_lds();
+      v = lane < K + n ? cs[lane] : -INFINITY;
+      id = lane < K + n ? ci[lane] : -1;
+    }
+    kth = td_cut(v, id, K, lane, cs, ci);
+  }
+};
+
+// Per-query row ranges: ranges [R, 2] (start, end) and range_off [Q + 1], or (lists != null) the row ranges
+// off[l] .. off[l + 1] of the query's `probes` lists. rows_per_split rows of the query's concatenated ranges per
+// workgroup (grid = (splits, Q)). out [splits, Q, K], unsorted lists (topk_merge_kernel orders them).
+//
+// A half-wave owns a row (16 B per lane and load, NCH loads), four rows of it are on their way together; 64 rows
+// are scored per step and handed to wave 0, which keeps the list while the others score the next 64 (two buffers,
+// one barrier a step). Bound by the latency of a step for few rows, by HBM for many: the caller splits a query's
+// rows over as many workgroups as fill the chip (388 rows of 8 documents: one workgroup took 105 us, with one load
+// in flight and a shuffle merge of K rounds per 64 rows; 7 workgroups take 15 us. 24 queries over 8 lists of about
+// 780 rows x 768: 162 -> 41 us).
+template <int NCH>
 __global__ void __launch_bounds__(256)
 topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ slots,
                    const bf16_t* __restrict__ Qv, int Q, const int* __restrict__ ranges,
                    const int* __restrict__ range_off, const unsigned* __restrict__ bitmap, int W, float thr,
                    int K, int rows_per_split, float* __restrict__ out_s, int* __restrict__ out_i) {
-  __shared__ float sc[64];
-  __shared__ int sr[64];
-  __shared__ float best[TK_MAX];
-  __shared__ int bidx[TK_MAX];
+  __shared__ float sc[2][64];
+  __shared__ int sr[2][64];
+  __shared__ float cs[TL_SL];
+  __shared__ int ci[TL_SL];
   const int split = blockIdx.x, q = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int half = lane >> 5, l32 = lane & 31;
-  if (tid < TK_MAX) { best[tid] = -INFINITY; bidx[tid] = -1; }
-  // query chunks held in registers: lane handles chunks c = l32 + 32*i
-  constexpr int MAXC = 16;  // d <= 32 * 8 * 16 = 4096
-  const int nch = d / 8;
-  float qv[MAXC][8];
+  TopList top;
+  top.init(cs, ci, K);  // (every wave writes the same empty list; wave 0 keeps it)
+  const int nch = d / 8;  // 16-B chunks of a row; this lane has chunks l32 + 32 i
+  float qv[NCH][8];
 #pragma unroll
-  for (int i = 0; i < MAXC; ++i) {
+  for (int i = 0; i < NCH; ++i) {
     const int c = l32 + 32 * i;
-    if (c < nch) {
-      u32x4_t u = *(const u32x4_t*)(Qv + (size_t)q * d + c * 8);
+    u32x4_t u = *(const u32x4_t*)(Qv + (size_t)q * d + min(c, nch - 1) * 8);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) qv[i][e] = bf2f((bf16_t)((e & 1) ? (u[e >> 1] >> 16) : (u[e >> 1] & 0xffff)));
-    }
+    for (int e = 0; e < 8; ++e) qv[i][e] = bf2f((bf16_t)((e & 1) ? (u[e >> 1] >> 16) : (u[e >> 1] & 0xffff)));
   }
   const int rb = range_off[q], re = range_off[q + 1];
   DA_ASSERT(rb >= 0 && re >= rb);
   const int pbeg = split * rows_per_split, pend = pbeg + rows_per_split;
   __syncthreads();
   // walk the concatenated ranges; position p counts rows across this query's ranges
-  int pos = 0;
+  int pos = 0, buf = 0;
   for (int r = rb; r < re; ++r) {
     const int s0 = ranges[2 * r], s1 = ranges[2 * r + 1];
     const int len = s1 - s0;
     const int lo = max(pbeg, pos), hi = min(pend, pos + len);
     for (int p0 = lo; p0 < hi; p0 += 64) {
-      // 64 rows per iteration: 8 half-waves x 8 rows
-      for (int j = 0; j < 8; ++j) {
-        const int rl = (wid * 2 + half) * 8 + j;
-        const int p = p0 + rl;
-        float dot = 0.f;
-        const int row = s0 + (p - pos);
-        if (p < hi) {
-          const bf16_t* xr = X + (size_t)row * d;
+      // 64 rows per step: 8 half-waves x 8 rows, 4 at a time
 #pragma unroll
-          for (int i = 0; i < MAXC; ++i) {
-            const int c = l32 + 32 * i;
-            if (c < nch) {
-              u32x4_t u = *(const u32x4_t*)(xr + c * 8);
+      for (int j0 = 0; j0 < 8; j0 += 4) {
+        const int rl = (wid * 2 + half) * 8 + j0;
+        u32x4_t u[4][NCH];
 #pragma unroll
-              for (int e = 0; e < 8; ++e)
-                dot += qv[i][e] * bf2f((bf16_t)((e & 1) ? (u[e >> 1] >> 16) : (u[e >> 1] & 0xffff)));
+        for (int j = 0; j < 4; ++j) {  // rows and chunks past the end: the last one's
+          const bf16_t* xr = X + (size_t)(s0 + (min(p0 + rl + j, hi - 1) - pos)) * d;
+#pragma unroll
+          for (int i = 0; i < NCH; ++i) u[j][i] = *(const u32x4_t*)(xr + min(l32 + 32 * i, nch - 1) * 8);
+        }
+        float dot[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+          const bool in = l32 + 32 * i < nch;
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float x = bf2f((bf16_t)((e & 1) ? (u[j][i][e >> 1] >> 16) : (u[j][i][e >> 1] & 0xffff)));
+              const float t = dot[j] + qv[i][e] * x;
+              dot[j] = in ? t : dot[j];
             }
-          }
         }
 #pragma unroll
-        for (int o = 16; o > 0; o >>= 1) dot += __shfl_xor(dot, o, 64);
-        if (l32 == 0) {
-          bool ok = p < hi && dot >= thr;
+        for (int o = 16; o > 0; o >>= 1)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) dot[j] += __shfl_xor(dot[j], o, 64);
+        // lane j of a half-wave hands in row j
+        const float s = (l32 == 0 ? dot[0] : l32 == 1 ? dot[1] : l32 == 2 ? dot[2] : dot[3]);
+        if (l32 < 4) {
+          const int p = p0 + rl + l32, row = s0 + (p - pos);
+          bool ok = p < hi && s >= thr && s != -INFINITY;
           if (ok && slots) {
             const int sl = slots[row];
             ok = sl >= 0 && (!bitmap || ((sl >> 5) < W && ((bitmap[(size_t)q * W + (sl >> 5)] >> (sl & 31)) & 1u)));
           }
-          sc[rl] = ok ? dot : -INFINITY;
-          sr[rl] = ok ? row : -1;
+          sc[buf][rl + l32] = s;
+          sr[buf][rl + l32] = ok ? row : -1;
         }
       }
-      __syncthreads();
-      if (wid == 0) wave_merge_topk(sc[lane], sr[lane], best, bidx, K, lane);
-      __syncthreads();
+      __syncthreads();  // this step's scores are in, and the list has taken the last step's
+      if (wid == 0) top.add(sc[buf][lane], sr[buf][lane]);
+      buf ^= 1;
     }
     pos += len;
     if (pos >= pend) break;
   }
-  if (tid < K) {
-    const size_t o = ((size_t)split * Q + q) * K + tid;
-    out_s[o] = best[tid];
-    out_i[o] = bidx[tid];
+  if (wid == 0) {
+    wave_sync_lds();
+    if (lane < K) {
+      const size_t o = ((size_t)split * Q + q) * K + lane;
+      out_s[o] = cs[lane];
+      out_i[o] = ci[lane];
+    }
   }
 }
 
-// cand [P, Q, K] -> out [Q, K] sorted desc. One workgroup per query; candidates consumed in place.
-__global__ void __launch_bounds__(256)
-topk_merge_kernel(float* __restrict__ cs, int* __restrict__ ci, int P, int Q, int K, float* __restrict__ os,
-                  int* __restrict__ oi) {
-  __shared__ float rv[4];
-  __shared__ int ri[4], rp[4];
-  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+// cand [P, Q, K] -> out [Q, K] sorted desc (ties: smaller row id). One workgroup per query, a wave per 64 candidates
+// up to 16 (TM_WAVES): each wave cuts its share to K, wave 0 joins the lists and orders them by counting the better
+// ones of each. Bound by the chain of cuts (about 1 us each), hence many waves: K rounds of a workgroup-wide argmax
+// with two barriers each took 18 us for 256 parts of K = 5, cuts by 4 waves 23 us, by 16 16.5 us.
+constexpr int TM_WAVES = 16;
+
+__global__ void __launch_bounds__(64 * TM_WAVES)
+topk_merge_kernel(const float* __restrict__ cand_s, const int* __restrict__ cand_i, int P, int Q, int K,
+                  float* __restrict__ os, int* __restrict__ oi) {
+  __shared__ float cs[TM_WAVES][TL_SL];
+  __shared__ int ci[TM_WAVES][TL_SL];
+  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nt = blockDim.x;
   const int n = P * K;
-  for (int r = 0; r < K; ++r) {
-    float bv = -INFINITY; int bi = -1, bp = -1;
-    for (int j = tid; j < n; j += 256) {
-      const int pp = j / K, kk = j % K;
-      const size_t o = ((size_t)pp * Q + q) * K + kk;
-      const float v = cs[o];
-      const int id = ci[o];
-      if (id >= 0 && better(v, id, bv, bi)) { bv = v; bi = id; bp = (int)o; }
+  TopList top;
+  top.init(cs[wid], ci[wid], K);
+  for (int j0 = wid * 64; j0 < n; j0 += nt * 4) {
+    float v[4];
+    int id[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {  // issued together: the lists come from all over the chip's caches
+      const int j = j0 + lane + nt * u, jc = min(j, n - 1);
+      const size_t o = ((size_t)(jc / K) * Q + q) * K + jc % K;
+      v[u] = cand_s[o];
+      id[u] = j < n ? cand_i[o] : -1;
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oid = __shfl_xor(bi, o, 64), op = __shfl_xor(bp, o, 64);
-      if ((oid >= 0 && better(ov, oid, bv, bi)) || (bi < 0 && oid >= 0)) { bv = ov; bi = oid; bp = op; }
-    }
-    if (lane == 0) { rv[wid] = bv; ri[wid] = bi; rp[wid] = bp; }
-    __syncthreads();
-    if (tid == 0) {
-      float fv = rv[0]; int fi = ri[0], fp = rp[0];
-      for (int w = 1; w < 4; ++w)
-        if ((ri[w] >= 0 && better(rv[w], ri[w], fv, fi)) || (fi < 0 && ri[w] >= 0)) { fv = rv[w]; fi = ri[w]; fp = rp[w]; }
-      os[(size_t)q * K + r] = fi >= 0 ? fv : -INFINITY;
-      oi[(size_t)q * K + r] = fi;
-      if (fp >= 0) ci[fp] = -1;  // consume
-    }
-    __syncthreads();
+    for (int u = 0; u < 4; ++u) top.add(v[u], id[u]);
+  }
+  __syncthreads();
+  if (wid) return;
+  const int rest = (nt / 64 - 1) * K;  // the other waves' lists, one after another
+  for (int e0 = 0; e0 < rest; e0 += 64) {
+    const int e = e0 + lane, w = 1 + min(e, max(rest - 1, 0)) / K;
+    top.add(cs[w][e % K], e < rest ? ci[w][e % K] : -1);
+  }
+  wave_sync_lds();
+  const float v = lane < K ? cs[0][lane] : -INFINITY;
+  const int id = lane < K ? ci[0][lane] : -1;
+  int rank = 0;
+  for (int j = 0; j < K; ++j) {
+    const float vj = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), j));
+    const int ij = __builtin_amdgcn_readlane(id, j);
+    rank += ij >= 0 && (better(vj, ij, v, id) || (vj == v && ij == id && j < lane));  // (a row named twice)
+  }
+  const int real = __popcll(__ballot(id >= 0));
+  if (id >= 0) {
+    os[(size_t)q * K + rank] = v;
+    oi[(size_t)q * K + rank] = id;
+  }
+  if (lane >= real && lane < K) {
+    os[(size_t)q * K + lane] = -INFINITY;
+    oi[(size_t)q * K + lane] = -1;
   }
 }
 
@@ -581,6 +656,12 @@ __global__ void kmeans_accum_kernel(const bf16_t* __restrict__ X, int N, int d, 
   if (c < 0) return;
   for (int j = threadIdx.x; j < d; j += blockDim.x) atomicAdd(&sums[(size_t)c * d + j], bf2f(X[(size_t)row * d + j]));
   if (threadIdx.x == 0) atomicAdd(&counts[c], 1.f);
+}
+
+static int topk_merge(const void* cs, const void* ci, int P, int Q, int K, void* out_s, void* out_i, hipStream_t s) {
+  const long waves = min((long)TM_WAVES, max(1L, ((long)P * K + 63) / 64));
+  topk_merge_kernel<<<Q, 64 * (int)waves, 0, s>>>((const float*)cs, (const int*)ci, P, Q, K, (float*)out_s, (int*)out_i);
+  DA_LAUNCH_CHECK();
 }
 
 DA_EXPORT size_t da_topk_dense_ws(int N, int Q, int K, int rows_per_block) {
@@ -604,8 +685,7 @@ DA_EXPORT int da_topk_dense(const void* X, int N, int d, const void* slots, cons
                                            (const unsigned*)bitmap, W, thr, K, rows_per_block, cs, ci);
   int err = (int)hipGetLastError();
   if (err) return err;
-  topk_merge_kernel<<<Q, 256, 0, s>>>(cs, ci, nblk, Q, K, (float*)out_s, (int*)out_i);
-  DA_LAUNCH_CHECK();
+  return topk_merge(cs, ci, nblk, Q, K, out_s, out_i, s);
 }
 
 // The streaming scan (d = 384, 768 or 1024): ws holds (row blocks padded to 8) * 4 * Q * K candidate
@@ -653,34 +733,39 @@ DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slot
 #undef TDS
   int err = (int)hipGetLastError();
   if (err) return err;
-  topk_merge_kernel<<<Q, 256, 0, s>>>(cs, ci, nqb == 1 ? nrb8 : nrb8_mq, Q, K, (float*)out_s, (int*)out_i);
-  DA_LAUNCH_CHECK();
+  return topk_merge(cs, ci, nqb == 1 ? nrb8 : nrb8_mq, Q, K, out_s, out_i, s);
 }
 
 DA_EXPORT int da_topk_ranges(const void* X, int d, const void* slots, const void* Qv, int Q, const void* ranges,
                              const void* range_off, const void* bitmap, int W, float thr, int K, int splits,
                              int rows_per_split, void* ws, void* out_s, void* out_i, void* stream) {
-  if (d % 8 || d > 4096 || K < 1 || K > TK_MAX || splits < 1) return (int)hipErrorInvalidValue;
+  if (d % 8 || d < 8 || d > 4096 || K < 1 || K > TK_MAX || splits < 1 || rows_per_split < 1)
+    return (int)hipErrorInvalidValue;
   if (Q == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   float* cs = (float*)ws;
   int* ci = (int*)(cs + (size_t)splits * Q * K);
   dim3 grid(splits, Q);
-  topk_ranges_kernel<<<grid, 256, 0, s>>>((const bf16_t*)X, d, (const int*)slots, (const bf16_t*)Qv, Q,
-                                          (const int*)ranges, (const int*)range_off, (const unsigned*)bitmap, W, thr,
-                                          K, rows_per_split, cs, ci);
+#define TRG(NCH)                                                                                                    \
+  topk_ranges_kernel<NCH><<<grid, 256, 0, s>>>((const bf16_t*)X, d, (const int*)slots, (const bf16_t*)Qv, Q,        \
+                                               (const int*)ranges, (const int*)range_off, (const unsigned*)bitmap,  \
+                                               W, thr, K, rows_per_split, cs, ci)
+  if (d <= 256) TRG(1);
+  else if (d <= 512) TRG(2);
+  else if (d <= 768) TRG(3);
+  else if (d <= 1024) TRG(4);
+  else if (d <= 2048) TRG(8);
+  else TRG(16);
+#undef TRG
   int err = (int)hipGetLastError();
   if (err) return err;
-  topk_merge_kernel<<<Q, 256, 0, s>>>(cs, ci, splits, Q, K, (float*)out_s, (int*)out_i);
-  DA_LAUNCH_CHECK();
+  return topk_merge(cs, ci, splits, Q, K, out_s, out_i, s);
 }
 
 DA_EXPORT int da_topk_merge(void* cand_s, void* cand_i, int P, int Q, int K, void* out_s, void* out_i, void* stream) {
   if (K < 1 || K > TK_MAX) return (int)hipErrorInvalidValue;
   if (Q == 0) return 0;
-  topk_merge_kernel<<<Q, 256, 0, (hipStream_t)stream>>>((float*)cand_s, (int*)cand_i, P, Q, K, (float*)out_s,
-                                                         (int*)out_i);
-  DA_LAUNCH_CHECK();
+  return topk_merge(cand_s, cand_i, P, Q, K, out_s, out_i, (hipStream_t)stream);
 }
 
 DA_EXPORT int da_kmeans_accum(const void* X, int N, int d, const void* assign, void* sums, void* counts, void* stream) {

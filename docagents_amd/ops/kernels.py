@@ -964,9 +964,11 @@ def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_bloc
 
 
 def topk_ranges(X, Qv, ranges, range_off, K: int, thr: float, max_rows: int, slots=None, bitmap=None,
-                rows_per_split: int = 512):
+                rows_per_split: int | None = None):
     """Top-K per query over its own row ranges. ranges int32 [R, 2], range_off int32 [Q+1];
-    max_rows = max total rows of any query (host int) — sets the split count."""
+    max_rows = max total rows of any query (host int) — sets the split count: rows_per_split rows of a query per
+    workgroup, by default what gives about 1024 workgroups (4 per CU: a workgroup keeps 48 KB of rows on their way),
+    from one step of the kernel (64) to 512."""
     _bf16_cuda(X, "X"); _bf16_cuda(Qv, "Qv")
     N, d = X.shape
     Q = Qv.shape[0]
@@ -981,6 +983,8 @@ def topk_ranges(X, Qv, ranges, range_off, K: int, thr: float, max_rows: int, slo
         _req(slots is not None, "bitmap needs slots")
         _req(bitmap.dtype == torch.int32 and bitmap.shape[0] == Q, "bitmap")
         W = bitmap.shape[1]
+    if rows_per_split is None:
+        rows_per_split = min(512, max(64, math.ceil(max_rows * Q / 1024 / 64) * 64))
     splits = max(1, math.ceil(max_rows / rows_per_split))
     ws = _workspace(splits * Q * K * 8, X.device)
     out_s = torch.empty((Q, K), dtype=torch.float32, device=X.device)
@@ -992,11 +996,11 @@ def topk_ranges(X, Qv, ranges, range_off, K: int, thr: float, max_rows: int, slo
 
 
 def topk_merge(cand_s, cand_i, K: int):
-    """cand [P, Q, K] (consumed) -> [Q, K]."""
+    """cand [P, Q, K] -> the best K of each query, sorted."""
     _req(cand_s.dtype == torch.float32 and cand_i.dtype == torch.int32, "dtypes")
     P, Q, K2 = cand_s.shape
     _req(K2 == K, "K mismatch")
-    cs, ci = cand_s.contiguous().clone(), cand_i.contiguous().clone()
+    cs, ci = cand_s.contiguous(), cand_i.contiguous()
     out_s = torch.empty((Q, K), dtype=torch.float32, device=cs.device)
     out_i = torch.empty((Q, K), dtype=torch.int32, device=cs.device)
     _check(lib().da_topk_merge(_ptr(cs), _ptr(ci), P, Q, K, _ptr(out_s), _ptr(out_i), _stream()), "topk_merge")

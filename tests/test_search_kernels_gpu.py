@@ -1,0 +1,62 @@
+"""The vector index's kernels at the edges of their steps, splits and lists, against 64-bit products and plain sorts."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from docagents_amd.ops import kernels as K  # noqa: E402
+
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("d,Kk,rows", [(8, 1, None), (264, 5, None), (384, 32, 64), (768, 5, None), (1024, 20, 100),
+                                       (1032, 7, None), (4096, 3, None)])
+def test_topk_ranges_edges(d, Kk, rows):
+    """Steps of 64 rows and what is left of them, splits that end inside a range, empty ranges and queries, a range
+    named twice, removed rows and a document filter, every count of 16-B chunks per lane."""
+    torch.manual_seed(d)
+    N, Q = 1500, 6
+    X = torch.nn.functional.normalize(torch.randn(N, d, device=DEV), dim=-1).to(torch.bfloat16)
+    Qv = torch.nn.functional.normalize(torch.randn(Q, d, device=DEV), dim=-1).to(torch.bfloat16)
+    rg = [[0, 1], [3, 3], [10, 74], [100, 165], [1499, 1500], [200, 263], [200, 263], [0, 1500], [7, 7]]
+    ro = [0, 2, 5, 7, 8, 9, 9]
+    ranges = torch.tensor(rg, dtype=torch.int32, device=DEV)
+    roff = torch.tensor(ro, dtype=torch.int32, device=DEV)
+    slots = (torch.arange(N, device=DEV, dtype=torch.int32) // 4).contiguous()
+    slots[::5] = -1
+    bitmap = torch.randint(-2**31, 2**31 - 1, (Q, N // 128 + 1), device=DEV, dtype=torch.int32)
+    dots = Qv.double().cpu() @ X.double().cpu().T
+    tol = d * 2.0 ** -23  # d terms summed in fp32, sum of |terms| at most about 1
+    for sl, bm in ((None, None), (slots, None), (slots, bitmap)):
+        s, i = K.topk_ranges(X, Qv, ranges, roff, Kk, -1.0, max_rows=1500, slots=sl, bitmap=bm, rows_per_split=rows)
+        for q in range(Q):
+            named = [r for a, b in rg[ro[q]:ro[q + 1]] for r in range(a, b)]
+            if sl is not None:
+                named = [r for r in named if sl[r] >= 0]
+            if bm is not None:
+                named = [r for r in named if (int(bm[q, int(sl[r]) >> 5]) >> (int(sl[r]) & 31)) & 1]
+            want = sorted((float(dots[q, r]) for r in named), reverse=True)[:Kk]
+            got = i[q].tolist()
+            assert got[len(want):] == [-1] * (Kk - len(want)) and bool((s[q, len(want):] == -math.inf).all())
+            assert all(g in named for g in got[:len(want)])
+            assert all(got.count(g) <= named.count(g) for g in got[:len(want)])
+            assert torch.allclose(s[q, :len(want)].double().cpu(), torch.tensor(want, dtype=torch.float64), rtol=0, atol=tol)
+            at = torch.tensor([float(dots[q, g]) for g in got[:len(want)]], dtype=torch.float64)
+            assert torch.allclose(s[q, :len(want)].double().cpu(), at, rtol=0, atol=tol)
+
+
+@pytest.mark.parametrize("P,Kk", [(1, 1), (1, 32), (3, 5), (13, 5), (52, 20), (300, 32)])
+def test_topk_merge_orders(P, Kk):
+    """Empty places, ties (the smaller id first, a repeated one kept twice), one list and many: exactly a sort."""
+    torch.manual_seed(P)
+    Q = 3
+    s = (torch.randint(-40, 40, (P, Q, Kk), device=DEV).float() / 8).contiguous()
+    i = torch.randint(-2, 500, (P, Q, Kk), device=DEV, dtype=torch.int32).clamp_min(-1)
+    i[:, 2] = -1
+    os_, oi = K.topk_merge(s, i, Kk)
+    for q in range(Q):
+        c = sorted((-float(a), int(b)) for a, b in zip(s[:, q].flatten(), i[:, q].flatten()) if b >= 0)[:Kk]
+        c += [(math.inf, -1)] * (Kk - len(c))
+        assert [(-float(a), int(b)) for a, b in zip(os_[q], oi[q])] == c
