@@ -135,9 +135,9 @@ topk_dense_kernel(const bf16_t* __restrict__ X, int N, int d, const int* __restr
 //    it do any top-K work (TdWave below).
 //  * Up to 16 queries (one query block): topk_dense_stream_kernel, every wave its own rows, the
 //    rows loaded non-temporally straight into the MFMA A registers.
-//  * 17..64 queries: topk_dense_mq_kernel, the workgroup's 4 waves = 4 query blocks over the SAME
+//  * 17 and more: topk_dense_mq_kernel, the workgroup's 4 waves = 4 (or 8) query blocks over the SAME
 //    rows: each 16-row tile is read from HBM once into LDS and feeds all four waves (B fragments of
-//    a wave's 16 queries live in its registers). Query blocks as separate workgroups over the same
+//    a wave's queries live in its registers). Query blocks as separate workgroups over the same
 //    rows, even dispatched back to back to one XCD, missed in L2 and read the shard once per block
 //    (batch 64: 12.1 ms vs 3.6 ms for batch 1, profiles/r5/index/).
 // out [row blocks (padded to 8), Q, K]: one unsorted top-K list per (workgroup, query), ordered and
@@ -172,41 +172,49 @@ __device__ __forceinline__ void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The top K of the wave's 64 (v, id) (one per lane; id < 0 = empty) into cs/ci[0, K) of a list,
-// unsorted. Returns the K-th best score (-inf while fewer than K are real). Every lane must have
-// read what it passes before the call (the list slots are overwritten).
+// The top K of the wave's 64 (v, id) (one per lane; id < 0 = empty) into cs/ci[0, K) of a list, unsorted, empty
+// places behind them. Returns a bound that the K-th best reaches and the next one does not (-inf while fewer than K
+// are real). Every lane must have read what it passes before the call (the list slots are overwritten).
+// The masks are uniform (scalar unit), and the rounds end at the bit that tells the K-th best from the next: about
+// 16 of 32 rounds for scores of one magnitude.
 __device__ __forceinline__ float td_cut(float v, int id, int K, int lane, float* cs, int* ci) {
   const unsigned key = td_key(v, id);
-  unsigned T = 0;  // the K-th largest key (empty lanes have key 0)
+  unsigned long long act = __ballot(key != 0u), sel = 0ull;
+  unsigned T = 0;  // prefix of the K-th largest key
   int need = K;
-  bool act = true;
-  for (int bt = 31; bt >= 0; --bt) {
-    const bool one = (key >> bt) & 1u;
-    const int c1 = __popcll(__ballot(act && one));
-    if (c1 >= need) { T |= 1u << bt; act = act && one; }
-    else { need -= c1; act = act && !one; }
+  if (__popcll(act) <= K) {
+    sel = act;
+    need = 0;
   }
-  // winners: every key > T, then `need` of the keys == T (smallest row ids; empties: any)
-  unsigned long long sel = __ballot(key > T);
-  unsigned long long eq = __ballot(key == T);
-  need = K - __popcll(sel);
-  if (__popcll(eq) <= need || T == 0u) {
-    for (; need > 0 && eq; --need) { sel |= eq & (~eq + 1); eq &= eq - 1; }
-  } else {  // exact score ties at the threshold (rare): smallest row ids first
-    for (; need > 0; --need) {
-      int m = ((eq >> lane) & 1ull) ? id : 0x7fffffff;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) m = min(m, __shfl_xor(m, o, 64));
-      const unsigned long long w = __ballot(((eq >> lane) & 1ull) && id == m);
-      sel |= w & (~w + 1);
-      eq &= ~(w & (~w + 1));
+  for (int bt = 31; bt >= 0 && need > 0; --bt) {
+    const unsigned long long one = __ballot((key >> bt) & 1u) & act;
+    const int c = __popcll(one);
+    if (c >= need) T |= 1u << bt;
+    if (c > need) {
+      act = one;
+    } else {
+      sel |= one;
+      need -= c;
+      act &= ~one;
     }
   }
+  for (; need > 0; --need) {  // exact ties at the threshold (rare): smallest row ids first
+    int m = ((act >> lane) & 1ull) ? id : 0x7fffffff;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = min(m, __shfl_xor(m, o, 64));
+    unsigned long long w = __ballot(((act >> lane) & 1ull) && id == m);
+    w &= ~w + 1;
+    sel |= w;
+    act &= ~w;
+  }
   const int pos = __builtin_amdgcn_mbcnt_hi((unsigned)(sel >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)sel, 0u));
+  const int real = __popcll(sel);
   wave_sync_lds();
   if ((sel >> lane) & 1ull) { cs[pos] = v; ci[pos] = id; }
+  if (lane >= real && lane < K) { cs[lane] = -INFINITY; ci[lane] = -1; }
   wave_sync_lds();
-  return td_unkey(T);
+  const float t = td_unkey(T);
+  return t != t ? -INFINITY : t;  // (a prefix below -FLT_MAX)
 }
 
 struct TdWave {
@@ -241,10 +249,11 @@ struct TdWave {
     if ((full >> fr) & 1ull) { kth = kn; cnt = 0; }
   }
   // a finished 16 x 16 tile: lane (fr, fg) holds rows row0 + i (row0 = tile base + 4 fg) of query fr
-  // (global query index qrow); rows from `end` on are padding
-  __device__ __forceinline__ void tile(const f32x4_t& acc, int row0, int end, bool qok, float thr,
-                                       const int* __restrict__ slots, const unsigned* __restrict__ bitmap, int W,
-                                       int qrow) {
+  // (global query index qrow); rows from `end` on are padding. slot: the doc slot of row fr of the tile, loaded with
+  // its rows (0 without slots): most tiles of a whole-shard pass have a candidate somewhere, and a load of its slot
+  // here had every wave of the workgroup wait for memory once a tile.
+  __device__ __forceinline__ void tile(const f32x4_t& acc, int row0, int end, bool qok, float thr, int slot,
+                                       const unsigned* __restrict__ bitmap, int W, int qrow) {
     bool cand = false;
 #pragma unroll
     for (int i = 0; i < 4; ++i) cand |= qok && row0 + i < end && acc[i] >= thr && acc[i] > kth;
@@ -254,11 +263,9 @@ struct TdWave {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = row0 + i;
-      bool ok = qok && row < end && acc[i] >= thr && acc[i] > kth;
-      if (ok && slots) {  // removed rows (slot -1) never match; the bitmap filters documents
-        const int sl = slots[row];
-        ok = sl >= 0 && (!bitmap || ((sl >> 5) < W && ((bitmap[(size_t)qrow * W + (sl >> 5)] >> (sl & 31)) & 1u)));
-      }
+      const int sl = __shfl(slot, 4 * fg + i, 64);
+      bool ok = qok && row < end && acc[i] >= thr && acc[i] > kth && sl >= 0;  // removed rows (slot -1) never match
+      if (ok && bitmap) ok = (sl >> 5) < W && ((bitmap[(size_t)qrow * W + (sl >> 5)] >> (sl & 31)) & 1u);
       if (ok) { bs[cnt] = acc[i]; bi[cnt] = row; ++cnt; }
     }
     // a lane's next tile adds <= 4: cut the queries with a sub-buffer past SB - 4
@@ -326,6 +333,7 @@ topk_dense_stream_kernel(const bf16_t* __restrict__ X, int N, const int* __restr
   const int wend = (int)min((long)N, (long)wbeg + rows_per_wave);
   const int ntile = (wend - wbeg + 15) / 16;
   const int lrow = N - 1;
+  const int* sp = slots ? slots : (const int*)X;  // (without slots some word of X: loaded all the same, not used)
   auto gload = [&](u32x4_t (&v)[NG][TD_G], int t) {  // tile t's fragments (rows clamped)
     const int row = min(wbeg + t * 16 + fr, lrow);
     const bf16_t* p = X + (size_t)row * d + fg * 8;
@@ -336,10 +344,13 @@ topk_dense_stream_kernel(const bf16_t* __restrict__ X, int N, const int* __restr
   };
   u32x4_t ring[NG][TD_G];
   gload(ring, 0);
+  int sl_next = sp[min(wbeg + fr, lrow)];
   const bool qok = fr < nq;
   for (int t = 0; t < ntile; ++t) {
     f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const int row_next = min(wbeg + (t + 1) * 16 + fr, lrow);
+    const int sl = slots ? sl_next : 0;
+    sl_next = sp[row_next];
     const bf16_t* pn = X + (size_t)row_next * d + fg * 8;
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
@@ -354,7 +365,7 @@ topk_dense_stream_kernel(const bf16_t* __restrict__ X, int N, const int* __restr
       for (int j = 0; j < TD_G; ++j)
         ring[g][j] = __builtin_nontemporal_load((const u32x4_t*)(pn + (g * TD_G + j) * 32));
     }
-    st.tile(acc, wbeg + t * 16 + fg * 4, wend, qok, thr, slots, bitmap, W, qbase + fr);
+    st.tile(acc, wbeg + t * 16 + fg * 4, wend, qok, thr, sl, bitmap, W, qbase + fr);
   }
   st.finish();
   // the 4 waves' lists -> one per workgroup (wave 0 absorbs the others'), out [rb, Q, K]
@@ -365,14 +376,18 @@ topk_dense_stream_kernel(const bf16_t* __restrict__ X, int N, const int* __restr
   }
 }
 
-// 17..64 queries per workgroup (see above). rows_per_block rows per workgroup (multiple of 16), grid
-// = row blocks (padded to 8) x query groups of 64: the nqg groups of one row block are dispatched to
-// one XCD back to back. A tile: 16 rows x d, 16 B per thread per load (NG loads), TD_PF tiles in
-// flight in registers, written to one of two LDS buffers (16-B chunk c of row r at c ^ (r & 15): the
-// 16 rows one ds_read_b128 lane group reads hit 16 distinct slots), one barrier per tile.
+// 17 and more queries: 64 QB queries per workgroup (QB blocks of 16 per wave: 2 from 65 queries on, so that a shard is
+// read once for up to 128). rows_per_block rows per workgroup (multiple of 16), grid = row blocks (padded to 8) x
+// query groups: the nqg groups of one row block are dispatched to one XCD back to back. A tile: 16 rows x d, 16 B per
+// thread per load (NG loads) and the rows' doc slots, TD_PF tiles in flight in registers, written to one of two LDS
+// buffers (16-B chunk c of row r at c ^ (r & 15): the 16 rows one ds_read_b128 lane group reads hit 16 distinct
+// slots), one barrier per tile. The queries' fragments stay in registers (QB d / 8 of the 512 that one wave per SIMD
+// may have); a wave's two query blocks share the reads of the tile.
+// Bound by HBM: 128 queries x 1.25 M rows x 1024 take @@MQ@@ us (@@MQBW@@ TB/s; 2228 with 64 queries per workgroup, slots
+// loaded where a candidate turned up and cuts of always 32 rounds).
 constexpr int TD_PF = 3;
 
-template <int NG>
+template <int NG, int QB>
 __global__ void __launch_bounds__(256, 1)
 topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict__ slots,
                      const bf16_t* __restrict__ Qv, int Q, const unsigned* __restrict__ bitmap, int W, float thr,
@@ -380,35 +395,42 @@ topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict_
   constexpr int d = NG * 128, NK = d / 32, CPR = d / 8, RB = d * 2, TB = 16 * RB;
   static_assert(16 * CPR == 256 * NG, "one 16-B load per thread per 128 columns");
   __shared__ __attribute__((aligned(16))) char sX[2][TB];
-  __shared__ float cs_all[4][16 * TD_SL];
-  __shared__ int ci_all[4][16 * TD_SL];
+  __shared__ float cs_all[4 * QB][16 * TD_SL];
+  __shared__ int ci_all[4 * QB][16 * TD_SL];
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int fr = lane & 15, fg = lane >> 4;
   const int b = blockIdx.x, per = 8 * nqg;
   const int grp = b / per, rem = b % per;
   const int qg = rem / 8, rb = grp * 8 + rem % 8;
-  const int qbase = (qg * 4 + wid) * 16, nq = max(0, min(16, Q - qbase));
-  const bool qok = fr < nq;
   // this wave's B fragments: query qbase + fr, columns 32 kk + 8 fg .. + 8
-  bf16x8_t bq[NK];
+  bf16x8_t bq[QB][NK];
+  TdWave st[QB];
+  int qbase[QB];
+  bool qok[QB];
 #pragma unroll
-  for (int kk = 0; kk < NK; ++kk)
-    bq[kk] = qok ? *(const bf16x8_t*)(Qv + (size_t)(qbase + fr) * d + kk * 32 + fg * 8)
-                 : bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-  TdWave st;
-  st.init(cs_all[wid], ci_all[wid], K);
+  for (int j = 0; j < QB; ++j) {
+    qbase[j] = (qg * 4 * QB + j * 4 + wid) * 16;
+    qok[j] = qbase[j] + fr < Q;
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk)
+      bq[j][kk] = qok[j] ? *(const bf16x8_t*)(Qv + (size_t)(qbase[j] + fr) * d + kk * 32 + fg * 8)
+                         : bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+    st[j].init(cs_all[j * 4 + wid], ci_all[j * 4 + wid], K);
+  }
 
   const int rbeg = (int)min((long)N, (long)rb * rows_per_block);
   const int rend = (int)min((long)N, (long)rbeg + rows_per_block);
   const int ntile = (rend - rbeg + 15) / 16;
   const int tl = max(ntile - 1, 0), lrow = N - 1;
-  auto gload = [&](u32x4_t (&v)[NG], int t) {  // tile t (rows clamped): thread's chunks tid + 256 i
+  const int* sp = slots ? slots : (const int*)X;  // (without slots some word of X: loaded all the same, not used)
+  auto gload = [&](u32x4_t (&v)[NG], int& sl, int t) {  // tile t (rows clamped): thread's chunks tid + 256 i
 #pragma unroll
     for (int i = 0; i < NG; ++i) {
       const int idx = tid + 256 * i, r = idx / CPR, c = idx % CPR;
       v[i] = __builtin_nontemporal_load((const u32x4_t*)(X + (size_t)min(rbeg + t * 16 + r, lrow) * d + c * 8));
     }
+    sl = sp[min(rbeg + t * 16 + fr, lrow)];
   };
   auto lstore = [&](const u32x4_t (&v)[NG], int buf) {
 #pragma unroll
@@ -419,9 +441,10 @@ topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict_
   };
   __syncthreads();  // the lists' initial values (before any load is in flight: this drains them)
   u32x4_t ring[TD_PF][NG];
+  int slot[TD_PF];
 #pragma unroll
   for (int u = 0; u < TD_PF; ++u) {
-    gload(ring[u], min(u, tl));
+    gload(ring[u], slot[u], min(u, tl));
     asm volatile("" ::: "memory");  // issue order = tile order (counted waits)
   }
   // whole groups of TD_PF tiles (no exit inside the unrolled group: the ring keeps fixed registers);
@@ -430,25 +453,33 @@ topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict_
 #pragma unroll
     for (int u = 0; u < TD_PF; ++u) {
       const int t = t0 + u;
-      const int buf = t & 1;
+      const int buf = t & 1, sl = slots ? slot[u] : 0;
       lstore(ring[u], buf);
-      gload(ring[u], min(t + TD_PF, tl));  // clamped past the end: uniform counts
+      gload(ring[u], slot[u], min(t + TD_PF, tl));  // clamped past the end: uniform counts
       // tile t visible to every wave, and every wave is done with tile t - 2 (same buffer): a raw
       // barrier (__syncthreads() would drain the loads in flight)
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
-      f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      f32x4_t acc[QB];
+#pragma unroll
+      for (int j = 0; j < QB; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       const char* xr = &sX[buf][fr * RB];
 #pragma unroll
       for (int kk = 0; kk < NK; ++kk) {
-        const int c = kk * 4 + fg;
-        acc = mfma16(*(const bf16x8_t*)(xr + ((c ^ fr) << 4)), bq[kk], acc);
+        const bf16x8_t a = *(const bf16x8_t*)(xr + (((kk * 4 + fg) ^ fr) << 4));
+#pragma unroll
+        for (int j = 0; j < QB; ++j) acc[j] = mfma16(a, bq[j][kk], acc[j]);
       }
-      st.tile(acc, rbeg + t * 16 + fg * 4, rend, qok, thr, slots, bitmap, W, qbase + fr);
+#pragma unroll
+      for (int j = 0; j < QB; ++j)
+        st[j].tile(acc[j], rbeg + t * 16 + fg * 4, rend, qok[j], thr, sl, bitmap, W, qbase[j] + fr);
     }
   }
-  st.finish();
-  st.store(nq, ((size_t)rb * Q + qbase) * K, out_s, out_i);
+#pragma unroll
+  for (int j = 0; j < QB; ++j) {
+    st[j].finish();
+    st[j].store(max(0, min(16, Q - qbase[j])), ((size_t)rb * Q + qbase[j]) * K, out_s, out_i);
+  }
 }
 
 // A wave's unsorted top-K list in LDS: cs / ci hold TL_SL slots, [0, K) the list, the rest room for what is
@@ -691,10 +722,14 @@ DA_EXPORT int da_topk_dense(const void* X, int N, int d, const void* slots, cons
 // The streaming scan (d = 384, 768 or 1024): ws holds (row blocks padded to 8) * 4 * Q * K candidate
 // pairs; rows_per_wave % 16 == 0. hipErrorInvalidValue for shapes it does not take (the caller
 // then uses da_topk_dense).
+static long blocks8(long N, long rows) { return ((N + rows - 1) / rows + 7) / 8 * 8; }
+// rows per workgroup of the shared-tile kernel: one workgroup per CU over the whole shard (each pays the early top-K
+// fill once), one tile at least
+static int mq_rows(long N) { return (int)max(16L, (N + 256 * 16 - 1) / (256 * 16) * 16); }
+
 DA_EXPORT size_t da_topk_stream_ws(int N, int Q, int K, int rows_per_wave) {
-  const long nrb = ((long)N + 4L * rows_per_wave - 1) / (4L * rows_per_wave);
-  const long nrb8 = (nrb + 7) / 8 * 8;
-  return (size_t)nrb8 * Q * K * 8;
+  const long parts = Q <= 16 ? blocks8(N, 4L * rows_per_wave) : blocks8(N, mq_rows(N));
+  return (size_t)parts * Q * K * 8;
 }
 
 DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slots, const void* Qv, int Q,
@@ -705,25 +740,23 @@ DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slot
     return (int)hipErrorInvalidValue;
   if (Q == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  const long nrb = ((long)N + 4L * rows_per_wave - 1) / (4L * rows_per_wave);
-  const int nrb8 = (int)((nrb + 7) / 8 * 8);
-  const int nqb = (Q + 15) / 16, nqg = (Q + 63) / 64;  // query blocks of 16 / groups of 64
-  if ((long)nrb8 * nqg > 0x7fffffffL) return (int)hipErrorInvalidValue;
+  const int rpb = mq_rows(N), qper = Q > 64 ? 128 : 64, nqg = (Q + qper - 1) / qper;
+  const long parts = Q <= 16 ? blocks8(N, 4L * rows_per_wave) : blocks8(N, rpb);
+  if (parts * nqg > 0x7fffffffL) return (int)hipErrorInvalidValue;
   float* cs = (float*)ws;
-  int* ci = (int*)(cs + (size_t)nrb8 * Q * K);
-  // shared-tile kernel: one workgroup per CU over the whole shard (~N / 256 rows each; each
-  // workgroup pays the early top-K fill once), never more row blocks than the workspace holds
-  const int rpb = (int)max(4L * rows_per_wave, ((long)N + 256 * 16 - 1) / (256 * 16) * 16);
-  const long nrb_mq = ((long)N + rpb - 1) / rpb;
-  const int nrb8_mq = (int)((nrb_mq + 7) / 8 * 8);
+  int* ci = (int*)(cs + (size_t)parts * Q * K);
+#define TDQ(NG, QB)                                                                                     \
+  topk_dense_mq_kernel<NG, QB><<<(int)parts * nqg, 256, 0, s>>>((const bf16_t*)X, N, (const int*)slots,  \
+      (const bf16_t*)Qv, Q, (const unsigned*)bitmap, W, thr, K, rpb, nqg, cs, ci)
 #define TDS(NG)                                                                                         \
   do {                                                                                                  \
-    if (nqb == 1)                                                                                       \
-      topk_dense_stream_kernel<NG><<<nrb8, 256, 0, s>>>((const bf16_t*)X, N, (const int*)slots,         \
+    if (Q <= 16)                                                                                        \
+      topk_dense_stream_kernel<NG><<<(int)parts, 256, 0, s>>>((const bf16_t*)X, N, (const int*)slots,   \
           (const bf16_t*)Qv, Q, (const unsigned*)bitmap, W, thr, K, rows_per_wave, 1, cs, ci);           \
+    else if (Q <= 64)                                                                                   \
+      TDQ(NG, 1);                                                                                       \
     else                                                                                                \
-      topk_dense_mq_kernel<NG><<<nrb8_mq * nqg, 256, 0, s>>>((const bf16_t*)X, N, (const int*)slots,    \
-          (const bf16_t*)Qv, Q, (const unsigned*)bitmap, W, thr, K, rpb, nqg, cs, ci);                  \
+      TDQ(NG, 2);                                                                                       \
   } while (0)
   switch (d) {
     case 384: TDS(3); break;
@@ -731,9 +764,10 @@ DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slot
     default: TDS(8); break;
   }
 #undef TDS
+#undef TDQ
   int err = (int)hipGetLastError();
   if (err) return err;
-  return topk_merge(cs, ci, nqb == 1 ? nrb8 : nrb8_mq, Q, K, out_s, out_i, s);
+  return topk_merge(cs, ci, (int)parts, Q, K, out_s, out_i, s);
 }
 
 DA_EXPORT int da_topk_ranges(const void* X, int d, const void* slots, const void* Qv, int Q, const void* ranges,

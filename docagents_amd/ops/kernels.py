@@ -942,8 +942,8 @@ def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_bloc
     if d in (384, 768, 1024) and rows_per_block is None and N > 0 and Q <= 256:
         # the streaming scan (search-sized batches over a big shard; k-means assignment, with the
         # rows as the queries, keeps the query-major tiles below): ~16 waves of rows per CU over
-        # the chip (256 CUs), >= 64 rows each
-        rpw = max(64, math.ceil(N / (256 * 16) / 16) * 16)
+        # the chip (256 CUs), one tile of 16 rows each at least (a few hundred centroids)
+        rpw = max(16, math.ceil(N / (256 * 16) / 16) * 16)
         ws = _workspace(int(lib().da_topk_stream_ws(N, Q, K, rpw)), X.device)
         out_s = torch.empty((Q, K), dtype=torch.float32, device=X.device)
         out_i = torch.empty((Q, K), dtype=torch.int32, device=X.device)

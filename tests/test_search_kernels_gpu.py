@@ -60,3 +60,38 @@ def test_topk_merge_orders(P, Kk):
         c = sorted((-float(a), int(b)) for a, b in zip(s[:, q].flatten(), i[:, q].flatten()) if b >= 0)[:Kk]
         c += [(math.inf, -1)] * (Kk - len(c))
         assert [(-float(a), int(b)) for a, b in zip(os_[q], oi[q])] == c
+
+
+@pytest.mark.parametrize("N,d,Q,Kk", [(1, 768, 17, 3), (15, 1024, 65, 32), (512, 384, 24, 8), (513, 768, 16, 5),
+                                      (4097, 1024, 128, 5), (4100, 768, 129, 20), (20011, 384, 70, 1), (70001, 1024, 256, 5)])
+def test_topk_dense_whole_shard(N, d, Q, Kk):
+    """Last tiles and workgroups that are not full, one or two query blocks per wave, query groups that are not full,
+    removed rows and a document filter (slots at an odd address)."""
+    torch.manual_seed(N)
+    X = torch.nn.functional.normalize(torch.randn(N, d, device=DEV), dim=-1).to(torch.bfloat16)
+    Qv = torch.nn.functional.normalize(torch.randn(Q, d, device=DEV), dim=-1).to(torch.bfloat16)
+    slots = torch.empty(N + 1, dtype=torch.int32, device=DEV)[1:]
+    slots.copy_(torch.arange(N, device=DEV) // 3)
+    slots[::5] = -1
+    bitmap = torch.randint(-2**31, 2**31 - 1, (Q, N // 96 + 1), device=DEV, dtype=torch.int32)
+    dots = Qv.double() @ X.double().T
+    tol = d * 2.0 ** -23  # d terms summed in fp32, sum of |terms| at most about 1
+    bits = (bitmap[:, (slots.clamp_min(0) >> 5).long()] >> (slots & 31)) & 1
+    for sl, bm, thr in ((None, None, -1.0), (slots, None, 0.0), (slots, bitmap, -1.0)):
+        s, i = K.topk_dense(X, Qv, Kk, thr, slots=sl, bitmap=bm)
+        ok = torch.ones_like(dots, dtype=torch.bool)
+        if sl is not None:
+            ok &= slots >= 0
+        if bm is not None:
+            ok &= bits.bool()
+        want = dots.masked_fill(~ok, -math.inf).masked_fill(dots < thr - tol, -math.inf)
+        want = torch.nn.functional.pad(want, (0, Kk), value=-math.inf).topk(Kk).values
+        near = (want - thr).abs() <= tol  # a score at the floor may fall on either side
+        real = i >= 0
+        assert bool((real == (want > -math.inf)).logical_or(near).all())
+        assert bool((s[~real] == -math.inf).all()) and bool((i[~real] == -1).all())
+        both = real & (want > -math.inf)
+        assert bool(((s.double() - want).abs() <= tol)[both].all())
+        at = dots.gather(1, i.clamp_min(0).long())
+        assert bool(((s.double() - at).abs() <= tol)[real].all()) and bool(ok.gather(1, i.clamp_min(0).long())[real].all())
+        assert all(len(set(r)) == len(r) for r in ([j for j in row if j >= 0] for row in i.tolist()))
