@@ -253,41 +253,34 @@ class FlatIndex:
             return self.ops.topk_ranges(X, q, rt, ot, k, min_sim, max_rows=maxrows)
 
     def _dense(self, X, q, k, min_sim, slots, doc_filters=None):
-        """MFMA dense scan; doc filter as a bitmap over local doc slots. Removed rows (slot -1) map to
-        a guard slot whose bit is never set."""
-        Q = q.shape[0]
-        nslots = len(self.slot_docs)
-        guard = nslots
-        W = (nslots + 1 + 31) // 32
-        bm = np.zeros((Q, W), dtype=np.uint32)
-        if doc_filters is None:
-            full, rem = divmod(nslots, 32)
-            bm[:, :full] = 0xFFFFFFFF
-            if rem:
-                bm[:, full] = (1 << rem) - 1
-        else:
-            full, rem = divmod(nslots, 32)
-            for i, f in enumerate(doc_filters):
-                if f is None:
-                    bm[i, :full] = 0xFFFFFFFF
-                    if rem:
-                        bm[i, full] = (1 << rem) - 1
-                    continue
-                for d in f:
-                    e = self.docs.get(d)
-                    if e is not None and e.rows:
-                        bm[i, e.slot >> 5] |= np.uint32(1 << (e.slot & 31))
-        bitmap = h2d(bm.view(np.int32), self.device)
-        slots = torch.where(slots < 0, torch.full_like(slots, guard), slots).contiguous()
+        """MFMA dense scan; doc filter as a bitmap over local doc slots (none without a filter: the scan itself
+        leaves out removed rows, slot -1)."""
+        bitmap = None if doc_filters is None else self._bitmap(q.shape[0], doc_filters)
         return self.ops.topk_dense(X, q, k, min_sim, slots=slots, bitmap=bitmap)
 
+    def _bitmap(self, Q, doc_filters):
+        """int32 [Q, words]: bit s of a query's row is set for the doc slots s that its filter names."""
+        nslots = len(self.slot_docs)
+        W = (nslots + 1 + 31) // 32
+        bm = np.zeros((Q, W), dtype=np.uint32)
+        full, rem = divmod(nslots, 32)
+        for i, f in enumerate(doc_filters):
+            if f is None:
+                bm[i, :full] = 0xFFFFFFFF
+                if rem:
+                    bm[i, full] = (1 << rem) - 1
+                continue
+            for d in f:
+                e = self.docs.get(d)
+                if e is not None and e.rows:
+                    bm[i, e.slot >> 5] |= np.uint32(1 << (e.slot & 31))
+        return h2d(bm.view(np.int32), self.device)
+
     def gather_ids(self, rows: torch.Tensor) -> torch.Tensor:
-        """Device: row indices (int32, -1 = none) -> external ids (int64, -1 = none). Indices are
-        clamped into the id table before the gather (a bad row index must never read outside it)."""
+        """Device: row indices (int32, -1 = none) -> external ids (int64, -1 = none; a bad row index never reads
+        outside the id table)."""
         with self.reading():
-            r = rows.long()
-            ok = (r >= 0) & (r < self.n)
-            return torch.where(ok, self.ids_t[r.clamp(0, max(0, self.n - 1))], torch.full_like(r, -1))
+            return self.ops.gather_ids(rows, self.ids_t[:self.n])
 
     def search_ids(self, q: torch.Tensor, k: int, min_sim: float, doc_filters=None):
         """search + gather_ids as ONE read: (scores fp32 [Q, k], external ids int64 [Q, k]) from the

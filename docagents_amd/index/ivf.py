@@ -36,6 +36,13 @@ class IVFFlatIndex(FlatIndex):
         self.centroids = None
         self.trained_n = 0
         self.list_off = None    # np int64 [lists + 1]: list l = rows [list_off[l], list_off[l+1])
+        self.list_off_t = None  # the same, int32 on the device
+        self.most_rows = None   # np int64 [lists + 1]: rows of the p longest lists together
+
+    def _set_lists(self, list_off: np.ndarray) -> None:
+        self.list_off = list_off
+        self.list_off_t = h2d(list_off.astype(np.int32), self.device)
+        self.most_rows = np.concatenate([[0], np.cumsum(np.sort(np.diff(list_off))[::-1])])
 
     # ------------------------------------------------------------------ training
     def _kmeans(self, Xs: torch.Tensor, iters: int) -> torch.Tensor:
@@ -100,8 +107,7 @@ class IVFFlatIndex(FlatIndex):
         assign = self._assign_chunked(self.X[:n])
         order = torch.sort(assign.long(), stable=True).indices
         counts = torch.bincount(assign.long(), minlength=self.lists).cpu().numpy()
-        self.list_off = np.zeros(self.lists + 1, dtype=np.int64)
-        np.cumsum(counts, out=self.list_off[1:])
+        self._set_lists(np.concatenate([[0], np.cumsum(counts)]).astype(np.int64))
         self.X[:n] = self.X[:n].index_select(0, order)
         self.slots_t[:n] = self.slots_t[:n].index_select(0, order)
         self.ids_t[:n] = self.ids_t[:n].index_select(0, order)
@@ -175,7 +181,7 @@ class IVFFlatIndex(FlatIndex):
             self.slot_docs = [f"{doc_prefix}{i}" for i in range(ndocs)]
             self.docs = {d: DocEntry(slot=i) for i, d in enumerate(self.slot_docs)}
             self.n = n_rows
-            self.list_off = off_t.cpu().numpy()
+            self._set_lists(off_t.cpu().numpy())
             self._rebuild_doc_ranges(n_rows)
             self.trained_n = n_rows
             return self
@@ -226,24 +232,10 @@ class IVFFlatIndex(FlatIndex):
                 _, lists = self.ops.topk_dense(self.centroids, q, probes, -2.0)
             else:  # wide probing: centroid scores as one GEMM, then torch top-k
                 lists = torch.topk(self.ops.gemm(q, self.centroids).float(), probes, dim=1).indices.int()
-            lists_h = lists.cpu().numpy()
-            off = self.list_off
-            starts, ends = off[lists_h.clip(0)], off[lists_h.clip(0) + 1]
-            valid = (lists_h >= 0) & (ends > starts)
-            per_q = np.where(valid, ends - starts, 0).sum(axis=1)
-            maxrows = int(per_q.max()) if Q else 0
             bitmap = None if doc_filters is None else self._bitmap(Q, doc_filters)
-            if maxrows > 0:
-                rr = np.stack([starts[valid], ends[valid]], axis=1).astype(np.int32)
-                ro = np.zeros(Q + 1, dtype=np.int32)
-                np.cumsum(valid.sum(axis=1), out=ro[1:])
-                rt = h2d(rr, self.device)
-                ot = h2d(ro, self.device)
-                s1, i1 = self.ops.topk_ranges(self.X, q, rt, ot, k, min_sim, max_rows=maxrows,
-                                              slots=self.slots_t, bitmap=bitmap)
-            else:
-                s1 = torch.full((Q, k), float("-inf"), device=self.device)
-                i1 = torch.full((Q, k), -1, dtype=torch.int32, device=self.device)
+            s1, i1 = self.ops.topk_lists(self.X, q, lists, self.list_off_t, k, min_sim,
+                                         mean_rows=-(-probes * self.trained_n // self.lists),
+                                         max_rows=int(self.most_rows[probes]), slots=self.slots_t, bitmap=bitmap)
             if self.n > self.trained_n:  # delta rows: exact scan
                 d0 = self.trained_n
                 rt = h2d(np.asarray([[d0, self.n]] * Q, dtype=np.int32), self.device)
@@ -252,20 +244,3 @@ class IVFFlatIndex(FlatIndex):
                                               slots=self.slots_t, bitmap=bitmap)
                 s1, i1 = self.ops.topk_merge(torch.stack([s1, s2]), torch.stack([i1, i2]), k)
             return s1, i1
-
-    def _bitmap(self, Q, doc_filters):
-        nslots = len(self.slot_docs)
-        W = (nslots + 1 + 31) // 32
-        bm = np.zeros((Q, W), dtype=np.uint32)
-        full, rem = divmod(nslots, 32)
-        for i, f in enumerate(doc_filters):
-            if f is None:
-                bm[i, :full] = 0xFFFFFFFF
-                if rem:
-                    bm[i, full] = (1 << rem) - 1
-                continue
-            for d in f:
-                e = self.docs.get(d)
-                if e is not None and e.rows:
-                    bm[i, e.slot >> 5] |= np.uint32(1 << (e.slot & 31))
-        return h2d(bm.view(np.int32), self.device)

@@ -414,23 +414,25 @@ topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict_
     qok[j] = qbase[j] + fr < Q;
 #pragma unroll
     for (int kk = 0; kk < NK; ++kk)
-      bq[j][kk] = qok[j] ? *(const bf16x8_t*)(Qv + (size_t)(qbase[j] + fr) * d + kk * 32 + fg * 8)
-                         : bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      bq[j][kk] = *(const bf16x8_t*)(Qv + (size_t)min(qbase[j] + fr, Q - 1) * d + kk * 32 + fg * 8);
     st[j].init(cs_all[j * 4 + wid], ci_all[j * 4 + wid], K);
   }
 
   const int rbeg = (int)min((long)N, (long)rb * rows_per_block);
   const int rend = (int)min((long)N, (long)rbeg + rows_per_block);
   const int ntile = (rend - rbeg + 15) / 16;
-  const int tl = max(ntile - 1, 0), lrow = N - 1;
-  const int* sp = slots ? slots : (const int*)X;  // (without slots some word of X: loaded all the same, not used)
-  auto gload = [&](u32x4_t (&v)[NG], int& sl, int t) {  // tile t (rows clamped): thread's chunks tid + 256 i
+  const int tl = max(ntile - 1, 0);
+  // buffer loads: one scalar offset per tile, rows past the workgroup's last return zeros (masked in tile()).
+  // Without slots some words of X are loaded in their place, and not used.
+  const __amdgpu_buffer_rsrc_t rsx = __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)rbeg * d), (short)0,
+                                                                       (rend - rbeg) * RB, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rss = __builtin_amdgcn_make_buffer_rsrc(
+      slots ? (void*)(slots + rbeg) : (void*)(X + (size_t)rbeg * d), (short)0, (rend - rbeg) * 4, 0x00020000);
+  auto gload = [&](u32x4_t (&v)[NG], int& sl, int t) {  // tile t <= tl: thread's chunks tid + 256 i
 #pragma unroll
-    for (int i = 0; i < NG; ++i) {
-      const int idx = tid + 256 * i, r = idx / CPR, c = idx % CPR;
-      v[i] = __builtin_nontemporal_load((const u32x4_t*)(X + (size_t)min(rbeg + t * 16 + r, lrow) * d + c * 8));
-    }
-    sl = sp[min(rbeg + t * 16 + fr, lrow)];
+    for (int i = 0; i < NG; ++i)
+      v[i] = __builtin_amdgcn_raw_buffer_load_b128(rsx, tid * 16 + i * 4096, t * TB, 2);  // non-temporal
+    sl = __builtin_amdgcn_raw_buffer_load_b32(rss, fr * 4, t * 64, 0);
   };
   auto lstore = [&](const u32x4_t (&v)[NG], int buf) {
 #pragma unroll
@@ -439,6 +441,9 @@ topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict_
       *(u32x4_t*)(&sX[buf][r * RB + ((c ^ (r & 15)) << 4)]) = v[i];
     }
   };
+  int xo[4];  // where chunk 4 kk + fg of row fr is: the swizzle only touches the chunk's low four bits
+#pragma unroll
+  for (int j = 0; j < 4; ++j) xo[j] = fr * RB + (((j * 4 + fg) ^ fr) << 4);
   __syncthreads();  // the lists' initial values (before any load is in flight: this drains them)
   u32x4_t ring[TD_PF][NG];
   int slot[TD_PF];
@@ -463,10 +468,9 @@ topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict_
       f32x4_t acc[QB];
 #pragma unroll
       for (int j = 0; j < QB; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      const char* xr = &sX[buf][fr * RB];
 #pragma unroll
       for (int kk = 0; kk < NK; ++kk) {
-        const bf16x8_t a = *(const bf16x8_t*)(xr + (((kk * 4 + fg) ^ fr) << 4));
+        const bf16x8_t a = *(const bf16x8_t*)(&sX[buf][xo[kk & 3] + (kk >> 2) * 256]);
 #pragma unroll
         for (int j = 0; j < QB; ++j) acc[j] = mfma16(a, bq[j][kk], acc[j]);
       }
@@ -520,8 +524,8 @@ struct TopList {
   }
 };
 
-// Per-query row ranges: ranges [R, 2] (start, end) and range_off [Q + 1], or (lists != null) the row ranges
-// off[l] .. off[l + 1] of the query's `probes` lists. rows_per_split rows of the query's concatenated ranges per
+// Per-query row ranges: ranges [R, 2] (start, end) and range_off [Q + 1], or (lists [Q, probes] != null) rows
+// ranges[l] .. ranges[l + 1] of each list l that the query names (l < 0: none). rows_per_split rows of the query's concatenated ranges per
 // workgroup (grid = (splits, Q)). out [splits, Q, K], unsorted lists (topk_merge_kernel orders them).
 //
 // A half-wave owns a row (16 B per lane and load, NCH loads), four rows of it are on their way together; 64 rows
@@ -534,7 +538,8 @@ template <int NCH>
 __global__ void __launch_bounds__(256)
 topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ slots,
                    const bf16_t* __restrict__ Qv, int Q, const int* __restrict__ ranges,
-                   const int* __restrict__ range_off, const unsigned* __restrict__ bitmap, int W, float thr,
+                   const int* __restrict__ range_off, const int* __restrict__ lists, int probes,
+                   const unsigned* __restrict__ bitmap, int W, float thr,
                    int K, int rows_per_split, float* __restrict__ out_s, int* __restrict__ out_i) {
   __shared__ float sc[2][64];
   __shared__ int sr[2][64];
@@ -554,14 +559,16 @@ topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ 
 #pragma unroll
     for (int e = 0; e < 8; ++e) qv[i][e] = bf2f((bf16_t)((e & 1) ? (u[e >> 1] >> 16) : (u[e >> 1] & 0xffff)));
   }
-  const int rb = range_off[q], re = range_off[q + 1];
+  const int rb = lists ? q * probes : range_off[q], re = lists ? rb + probes : range_off[q + 1];
   DA_ASSERT(rb >= 0 && re >= rb);
   const int pbeg = split * rows_per_split, pend = pbeg + rows_per_split;
   __syncthreads();
   // walk the concatenated ranges; position p counts rows across this query's ranges
   int pos = 0, buf = 0;
   for (int r = rb; r < re; ++r) {
-    const int s0 = ranges[2 * r], s1 = ranges[2 * r + 1];
+    const int l = lists ? lists[r] : 0;
+    if (l < 0) continue;
+    const int s0 = ranges[lists ? l : 2 * r], s1 = ranges[lists ? l + 1 : 2 * r + 1];
     const int len = s1 - s0;
     const int lo = max(pbeg, pos), hi = min(pend, pos + len);
     for (int p0 = lo; p0 < hi; p0 += 64) {
@@ -678,6 +685,16 @@ topk_merge_kernel(const float* __restrict__ cand_s, const int* __restrict__ cand
   }
 }
 
+// out[i] = ids[rows[i]], -1 where rows[i] names no row of [0, N) (a bad row index must never read outside the table).
+// One launch where nine elementwise ones of 2 to 5 us each did it.
+__global__ void __launch_bounds__(256)
+gather_ids_kernel(const int* __restrict__ rows, int n, const long* __restrict__ ids, int N, long* __restrict__ out) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int r = rows[i];
+  out[i] = r >= 0 && r < N ? ids[r] : -1;
+}
+
 // k-means accumulation: sums[assign[i]] += X[i] (fp32), counts[assign[i]] += 1
 __global__ void kmeans_accum_kernel(const bf16_t* __restrict__ X, int N, int d, const int* __restrict__ assign,
                                     float* __restrict__ sums, float* __restrict__ counts) {
@@ -724,8 +741,8 @@ DA_EXPORT int da_topk_dense(const void* X, int N, int d, const void* slots, cons
 // then uses da_topk_dense).
 static long blocks8(long N, long rows) { return ((N + rows - 1) / rows + 7) / 8 * 8; }
 // rows per workgroup of the shared-tile kernel: one workgroup per CU over the whole shard (each pays the early top-K
-// fill once), one tile at least
-static int mq_rows(long N) { return (int)max(16L, (N + 256 * 16 - 1) / (256 * 16) * 16); }
+// fill once), one tile at least, 1 GB at most (its 32-bit offsets)
+static int mq_rows(long N) { return (int)min(524288L, max(16L, (N + 256 * 16 - 1) / (256 * 16) * 16)); }
 
 DA_EXPORT size_t da_topk_stream_ws(int N, int Q, int K, int rows_per_wave) {
   const long parts = Q <= 16 ? blocks8(N, 4L * rows_per_wave) : blocks8(N, mq_rows(N));
@@ -771,9 +788,11 @@ DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slot
 }
 
 DA_EXPORT int da_topk_ranges(const void* X, int d, const void* slots, const void* Qv, int Q, const void* ranges,
-                             const void* range_off, const void* bitmap, int W, float thr, int K, int splits,
-                             int rows_per_split, void* ws, void* out_s, void* out_i, void* stream) {
-  if (d % 8 || d < 8 || d > 4096 || K < 1 || K > TK_MAX || splits < 1 || rows_per_split < 1)
+                             const void* range_off, const void* lists, int probes, const void* bitmap, int W,
+                             float thr, int K, int splits, int rows_per_split, void* ws, void* out_s, void* out_i,
+                             void* stream) {
+  if (d % 8 || d < 8 || d > 4096 || K < 1 || K > TK_MAX || splits < 1 || rows_per_split < 1 ||
+      (!range_off && (!lists || probes < 0)))
     return (int)hipErrorInvalidValue;
   if (Q == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
@@ -782,8 +801,8 @@ DA_EXPORT int da_topk_ranges(const void* X, int d, const void* slots, const void
   dim3 grid(splits, Q);
 #define TRG(NCH)                                                                                                    \
   topk_ranges_kernel<NCH><<<grid, 256, 0, s>>>((const bf16_t*)X, d, (const int*)slots, (const bf16_t*)Qv, Q,        \
-                                               (const int*)ranges, (const int*)range_off, (const unsigned*)bitmap,  \
-                                               W, thr, K, rows_per_split, cs, ci)
+                                               (const int*)ranges, (const int*)range_off, (const int*)lists,        \
+                                               probes, (const unsigned*)bitmap, W, thr, K, rows_per_split, cs, ci)
   if (d <= 256) TRG(1);
   else if (d <= 512) TRG(2);
   else if (d <= 768) TRG(3);
@@ -800,6 +819,14 @@ DA_EXPORT int da_topk_merge(void* cand_s, void* cand_i, int P, int Q, int K, voi
   if (K < 1 || K > TK_MAX) return (int)hipErrorInvalidValue;
   if (Q == 0) return 0;
   return topk_merge(cand_s, cand_i, P, Q, K, out_s, out_i, (hipStream_t)stream);
+}
+
+DA_EXPORT int da_gather_ids(const void* rows, int n, const void* ids, int N, void* out, void* stream) {
+  if (n < 0 || N < 0) return (int)hipErrorInvalidValue;
+  if (n == 0) return 0;
+  gather_ids_kernel<<<(n + 255) / 256, 256, 0, (hipStream_t)stream>>>((const int*)rows, n, (const long*)ids, N,
+                                                                      (long*)out);
+  DA_LAUNCH_CHECK();
 }
 
 DA_EXPORT int da_kmeans_accum(const void* X, int N, int d, const void* assign, void* sums, void* counts, void* stream) {

@@ -69,9 +69,10 @@ _SIGS = {
                       c_int, c_void_p, c_void_p, c_void_p, c_void_p],
     "da_topk_dense_stream": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_float, c_int,
                              c_int, c_void_p, c_void_p, c_void_p, c_void_p],
-    "da_topk_ranges": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
+    "da_topk_ranges": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int,
                        c_float, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
     "da_topk_merge": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
+    "da_gather_ids": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p],
     "da_kmeans_accum": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
     "da_sample_partial": [c_void_p, c_int, c_int, c_int, c_int, c_float, c_uint, c_uint, c_void_p, c_void_p, c_void_p],
     "da_sample_chunked": [c_void_p, c_int, c_int, c_int, c_float, c_uint, c_uint] + [c_void_p] * 10
@@ -967,14 +968,35 @@ def topk_ranges(X, Qv, ranges, range_off, K: int, thr: float, max_rows: int, slo
                 rows_per_split: int | None = None):
     """Top-K per query over its own row ranges. ranges int32 [R, 2], range_off int32 [Q+1];
     max_rows = max total rows of any query (host int) — sets the split count: rows_per_split rows of a query per
-    workgroup, by default what gives about 1024 workgroups (4 per CU: a workgroup keeps 48 KB of rows on their way),
-    from one step of the kernel (64) to 512."""
+    workgroup (default: ``_rows_per_split``)."""
+    _i32(ranges, "ranges"); _i32(range_off, "range_off")
+    _req(range_off.numel() == Qv.shape[0] + 1, "range_off length")
+    return _ranges(X, Qv, ranges, range_off, None, K, thr, max_rows, slots, bitmap,
+                   rows_per_split or _rows_per_split(max_rows, Qv.shape[0]))
+
+
+def topk_lists(X, Qv, lists, list_off, K: int, thr: float, mean_rows: int, max_rows: int, slots=None, bitmap=None):
+    """Top-K per query over the lists it names: lists int32 [Q, probes] (on the device; negative: none), list l =
+    rows list_off[l] .. list_off[l + 1] (int32). mean_rows / max_rows: rows of a query, expected / at most (host
+    ints). The lists never visit the host: nothing waits for the kernel that chose them."""
+    _i32(lists, "lists"); _i32(list_off, "list_off")
+    _req(lists.dim() == 2 and lists.shape[0] == Qv.shape[0], "lists [Q, probes]")
+    # workgroups past a query's rows end at once, but lists of very uneven length must not make too many of them
+    rows = max(_rows_per_split(mean_rows, Qv.shape[0]), math.ceil(max_rows / 512 / 64) * 64)
+    return _ranges(X, Qv, list_off, None, lists, K, thr, max_rows, slots, bitmap, rows)
+
+
+def _rows_per_split(rows: int, Q: int) -> int:
+    """Rows of a query per workgroup of the range scan: what gives about 1024 workgroups (4 per CU: a workgroup keeps
+    48 KB of rows on their way), from one step of the kernel (64) to 512."""
+    return min(512, max(64, math.ceil(rows * Q / 1024 / 64) * 64))
+
+
+def _ranges(X, Qv, ranges, range_off, lists, K, thr, max_rows, slots, bitmap, rows_per_split):
     _bf16_cuda(X, "X"); _bf16_cuda(Qv, "Qv")
     N, d = X.shape
     Q = Qv.shape[0]
     _req(d % 8 == 0 and d <= 4096 and 1 <= K <= 32, "d / K limits")
-    _i32(ranges, "ranges"); _i32(range_off, "range_off")
-    _req(range_off.numel() == Q + 1, "range_off length")
     W = 0
     if slots is not None:
         _i32(slots, "slots")
@@ -983,13 +1005,12 @@ def topk_ranges(X, Qv, ranges, range_off, K: int, thr: float, max_rows: int, slo
         _req(slots is not None, "bitmap needs slots")
         _req(bitmap.dtype == torch.int32 and bitmap.shape[0] == Q, "bitmap")
         W = bitmap.shape[1]
-    if rows_per_split is None:
-        rows_per_split = min(512, max(64, math.ceil(max_rows * Q / 1024 / 64) * 64))
     splits = max(1, math.ceil(max_rows / rows_per_split))
     ws = _workspace(splits * Q * K * 8, X.device)
     out_s = torch.empty((Q, K), dtype=torch.float32, device=X.device)
     out_i = torch.empty((Q, K), dtype=torch.int32, device=X.device)
-    _check(lib().da_topk_ranges(_ptr(X), d, _ptr(slots), _ptr(Qv), Q, _ptr(ranges), _ptr(range_off), _ptr(bitmap),
+    _check(lib().da_topk_ranges(_ptr(X), d, _ptr(slots), _ptr(Qv), Q, _ptr(ranges), _ptr(range_off), _ptr(lists),
+                                0 if lists is None else lists.shape[1], _ptr(bitmap),
                                 W, float(thr), K, splits, rows_per_split, _ptr(ws), _ptr(out_s), _ptr(out_i),
                                 _stream()), "topk_ranges")
     return out_s, out_i
@@ -1005,6 +1026,18 @@ def topk_merge(cand_s, cand_i, K: int):
     out_i = torch.empty((Q, K), dtype=torch.int32, device=cs.device)
     _check(lib().da_topk_merge(_ptr(cs), _ptr(ci), P, Q, K, _ptr(out_s), _ptr(out_i), _stream()), "topk_merge")
     return out_s, out_i
+
+
+def gather_ids(rows, ids):
+    """ids[rows] (int64, in the shape of rows), -1 where a row is outside [0, len(ids))."""
+    _req(rows.is_cuda, "rows must be on GPU")
+    _req(ids.is_cuda and ids.dtype == torch.int64 and ids.is_contiguous() and ids.dim() == 1, "ids must be int64 [N]")
+    if rows.dtype != torch.int32:
+        rows = rows.clamp(-1, 2**31 - 1).int()
+    rows = rows.contiguous()
+    out = torch.empty(rows.shape, dtype=torch.int64, device=rows.device)
+    _check(lib().da_gather_ids(_ptr(rows), rows.numel(), _ptr(ids), ids.numel(), _ptr(out), _stream()), "gather_ids")
+    return out
 
 
 def kmeans_accum(X, assign, sums, counts):

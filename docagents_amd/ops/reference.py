@@ -427,6 +427,13 @@ def topk_ranges(X, Qv, ranges, range_off, K, thr, max_rows=None, slots=None, bit
     return _topk_with_ties(s, K)
 
 
+def topk_lists(X, Qv, lists, list_off, K, thr, mean_rows=None, max_rows=None, slots=None, bitmap=None):
+    off = list_off.tolist()
+    rg = [[off[x], off[x + 1]] if x >= 0 else [0, 0] for q in lists.tolist() for x in q]
+    ro = torch.arange(lists.shape[0] + 1) * lists.shape[1]
+    return topk_ranges(X, Qv, torch.tensor(rg).view(-1, 2), ro, K, thr, slots=slots, bitmap=bitmap)
+
+
 def topk_merge(cand_s, cand_i, K):
     P, Q, _ = cand_s.shape
     s = cand_s.permute(1, 0, 2).reshape(Q, -1)
@@ -439,6 +446,12 @@ def topk_merge(cand_s, cand_i, K):
     vs, ii = torch.gather(s, 1, order)[:, :K], torch.gather(i, 1, order)[:, :K]
     ii = torch.where(torch.isinf(vs), torch.full_like(ii, -1), ii)
     return vs, ii
+
+
+def gather_ids(rows, ids):
+    r = rows.long()
+    ok = (r >= 0) & (r < ids.numel())
+    return torch.where(ok, torch.nn.functional.pad(ids, (0, 1))[torch.where(ok, r, ids.numel())], torch.full_like(r, -1))
 
 
 def kmeans_accum(X, assign, sums, counts):
