@@ -376,47 +376,42 @@ topk_dense_stream_kernel(const bf16_t* __restrict__ X, int N, const int* __restr
   }
 }
 
-// 17 and more queries: 64 QB queries per workgroup (QB blocks of 16 per wave: 2 from 65 queries on, so that a shard is
-// read once for up to 128). rows_per_block rows per workgroup (multiple of 16), grid = row blocks (padded to 8) x
-// query groups: the nqg groups of one row block are dispatched to one XCD back to back. A tile: 16 rows x d, 16 B per
-// thread per load (NG loads) and the rows' doc slots, TD_PF tiles in flight in registers, written to one of two LDS
-// buffers (16-B chunk c of row r at c ^ (r & 15): the 16 rows one ds_read_b128 lane group reads hit 16 distinct
-// slots), one barrier per tile. The queries' fragments stay in registers (QB d / 8 of the 512 that one wave per SIMD
-// may have); a wave's two query blocks share the reads of the tile.
-// Bound by HBM: 128 queries x 1.25 M rows x 1024 take @@MQ@@ us (@@MQBW@@ TB/s; 2228 with 64 queries per workgroup, slots
-// loaded where a candidate turned up and cuts of always 32 rounds).
+// 17 and more queries: NW waves of 16 queries each per workgroup (8 from 65 queries on, so that a shard is read once
+// for up to 128). rows_per_block rows per workgroup (multiple of 16), grid = row blocks (padded to 8) x query groups:
+// the nqg groups of one row block are dispatched to one XCD back to back. A tile: 16 rows x d, 16 B per thread per load
+// (NL loads) and the rows' doc slots, TD_PF tiles in flight in registers, written to one of two LDS buffers (16-B
+// chunk c of row r at c ^ (r & 15): the 16 rows one ds_read_b128 lane group reads hit 16 distinct slots), one barrier
+// per tile. The queries' fragments stay in registers (d / 8 of them).
+// Bound by HBM, and by what a SIMD does between tiles when it has one wave only: a pass of 128 queries x 1.25 M rows x
+// 1024 took 2304 us with 64 queries per workgroup, slots loaded where a candidate turned up and cuts of always 32
+// rounds, 1087 us with 4 waves of 32 queries each, and 808 us (3.2 TB/s) with two waves per SIMD, whose waits overlap.
 constexpr int TD_PF = 3;
 
-template <int NG, int QB>
-__global__ void __launch_bounds__(256, 1)
+template <int NG, int NW>
+__global__ void __launch_bounds__(64 * NW, 1)
 topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict__ slots,
                      const bf16_t* __restrict__ Qv, int Q, const unsigned* __restrict__ bitmap, int W, float thr,
                      int K, int rows_per_block, int nqg, float* __restrict__ out_s, int* __restrict__ out_i) {
-  constexpr int d = NG * 128, NK = d / 32, CPR = d / 8, RB = d * 2, TB = 16 * RB;
-  static_assert(16 * CPR == 256 * NG, "one 16-B load per thread per 128 columns");
+  constexpr int d = NG * 128, NK = d / 32, CPR = d / 8, RB = d * 2, TB = 16 * RB, NT = 64 * NW;
+  constexpr int NL = (16 * CPR + NT - 1) / NT;  // 16-B loads of a thread per tile
   __shared__ __attribute__((aligned(16))) char sX[2][TB];
-  __shared__ float cs_all[4 * QB][16 * TD_SL];
-  __shared__ int ci_all[4 * QB][16 * TD_SL];
+  __shared__ float cs_all[NW][16 * TD_SL];
+  __shared__ int ci_all[NW][16 * TD_SL];
 
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int fr = lane & 15, fg = lane >> 4;
   const int b = blockIdx.x, per = 8 * nqg;
   const int grp = b / per, rem = b % per;
   const int qg = rem / 8, rb = grp * 8 + rem % 8;
+  const int qbase = (qg * NW + wid) * 16, nq = max(0, min(16, Q - qbase));
+  const bool qok = fr < nq;
   // this wave's B fragments: query qbase + fr, columns 32 kk + 8 fg .. + 8
-  bf16x8_t bq[QB][NK];
-  TdWave st[QB];
-  int qbase[QB];
-  bool qok[QB];
+  bf16x8_t bq[NK];
 #pragma unroll
-  for (int j = 0; j < QB; ++j) {
-    qbase[j] = (qg * 4 * QB + j * 4 + wid) * 16;
-    qok[j] = qbase[j] + fr < Q;
-#pragma unroll
-    for (int kk = 0; kk < NK; ++kk)
-      bq[j][kk] = *(const bf16x8_t*)(Qv + (size_t)min(qbase[j] + fr, Q - 1) * d + kk * 32 + fg * 8);
-    st[j].init(cs_all[j * 4 + wid], ci_all[j * 4 + wid], K);
-  }
+  for (int kk = 0; kk < NK; ++kk)
+    bq[kk] = *(const bf16x8_t*)(Qv + (size_t)min(qbase + fr, Q - 1) * d + kk * 32 + fg * 8);
+  TdWave st;
+  st.init(cs_all[wid], ci_all[wid], K);
 
   const int rbeg = (int)min((long)N, (long)rb * rows_per_block);
   const int rend = (int)min((long)N, (long)rbeg + rows_per_block);
@@ -428,24 +423,30 @@ topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict_
                                                                        (rend - rbeg) * RB, 0x00020000);
   const __amdgpu_buffer_rsrc_t rss = __builtin_amdgcn_make_buffer_rsrc(
       slots ? (void*)(slots + rbeg) : (void*)(X + (size_t)rbeg * d), (short)0, (rend - rbeg) * 4, 0x00020000);
-  auto gload = [&](u32x4_t (&v)[NG], int& sl, int t) {  // tile t <= tl: thread's chunks tid + 256 i
+  unsigned voff[NL];   // chunk tid + NT i of a tile (one past its end: out of range, loads nothing)
+  int loff[NL];
 #pragma unroll
-    for (int i = 0; i < NG; ++i)
-      v[i] = __builtin_amdgcn_raw_buffer_load_b128(rsx, tid * 16 + i * 4096, t * TB, 2);  // non-temporal
+  for (int i = 0; i < NL; ++i) {
+    const int idx = tid + NT * i, r = idx / CPR, c = idx % CPR;
+    voff[i] = idx < 16 * CPR ? idx * 16u : 0x7ffffff0u;
+    loff[i] = r * RB + ((c ^ (r & 15)) << 4);
+  }
+  auto gload = [&](u32x4_t (&v)[NL], int& sl, int t) {  // tile t <= tl
+#pragma unroll
+    for (int i = 0; i < NL; ++i)
+      v[i] = __builtin_amdgcn_raw_buffer_load_b128(rsx, voff[i], t * TB, 2);  // non-temporal
     sl = __builtin_amdgcn_raw_buffer_load_b32(rss, fr * 4, t * 64, 0);
   };
-  auto lstore = [&](const u32x4_t (&v)[NG], int buf) {
+  auto lstore = [&](const u32x4_t (&v)[NL], int buf) {
 #pragma unroll
-    for (int i = 0; i < NG; ++i) {
-      const int idx = tid + 256 * i, r = idx / CPR, c = idx % CPR;
-      *(u32x4_t*)(&sX[buf][r * RB + ((c ^ (r & 15)) << 4)]) = v[i];
-    }
+    for (int i = 0; i < NL; ++i)
+      if ((i + 1) * NT <= 16 * CPR || tid + NT * i < 16 * CPR) *(u32x4_t*)(&sX[buf][loff[i]]) = v[i];
   };
   int xo[4];  // where chunk 4 kk + fg of row fr is: the swizzle only touches the chunk's low four bits
 #pragma unroll
   for (int j = 0; j < 4; ++j) xo[j] = fr * RB + (((j * 4 + fg) ^ fr) << 4);
   __syncthreads();  // the lists' initial values (before any load is in flight: this drains them)
-  u32x4_t ring[TD_PF][NG];
+  u32x4_t ring[TD_PF][NL];
   int slot[TD_PF];
 #pragma unroll
   for (int u = 0; u < TD_PF; ++u) {
@@ -465,25 +466,15 @@ topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict_
       // barrier (__syncthreads() would drain the loads in flight)
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
-      f32x4_t acc[QB];
+      f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < QB; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kk = 0; kk < NK; ++kk) {
-        const bf16x8_t a = *(const bf16x8_t*)(&sX[buf][xo[kk & 3] + (kk >> 2) * 256]);
-#pragma unroll
-        for (int j = 0; j < QB; ++j) acc[j] = mfma16(a, bq[j][kk], acc[j]);
-      }
-#pragma unroll
-      for (int j = 0; j < QB; ++j)
-        st[j].tile(acc[j], rbeg + t * 16 + fg * 4, rend, qok[j], thr, sl, bitmap, W, qbase[j] + fr);
+      for (int kk = 0; kk < NK; ++kk)
+        acc = mfma16(*(const bf16x8_t*)(&sX[buf][xo[kk & 3] + (kk >> 2) * 256]), bq[kk], acc);
+      st.tile(acc, rbeg + t * 16 + fg * 4, rend, qok, thr, sl, bitmap, W, qbase + fr);
     }
   }
-#pragma unroll
-  for (int j = 0; j < QB; ++j) {
-    st[j].finish();
-    st[j].store(max(0, min(16, Q - qbase[j])), ((size_t)rb * Q + qbase[j]) * K, out_s, out_i);
-  }
+  st.finish();
+  st.store(nq, ((size_t)rb * Q + qbase) * K, out_s, out_i);
 }
 
 // A wave's unsorted top-K list in LDS: cs / ci hold TL_SL slots, [0, K) the list, the rest room for what is
@@ -762,18 +753,18 @@ DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slot
   if (parts * nqg > 0x7fffffffL) return (int)hipErrorInvalidValue;
   float* cs = (float*)ws;
   int* ci = (int*)(cs + (size_t)parts * Q * K);
-#define TDQ(NG, QB)                                                                                     \
-  topk_dense_mq_kernel<NG, QB><<<(int)parts * nqg, 256, 0, s>>>((const bf16_t*)X, N, (const int*)slots,  \
-      (const bf16_t*)Qv, Q, (const unsigned*)bitmap, W, thr, K, rpb, nqg, cs, ci)
+#define TDQ(NG, NW)                                                                                     \
+  topk_dense_mq_kernel<NG, NW><<<(int)parts * nqg, 64 * NW, 0, s>>>((const bf16_t*)X, N,                \
+      (const int*)slots, (const bf16_t*)Qv, Q, (const unsigned*)bitmap, W, thr, K, rpb, nqg, cs, ci)
 #define TDS(NG)                                                                                         \
   do {                                                                                                  \
     if (Q <= 16)                                                                                        \
       topk_dense_stream_kernel<NG><<<(int)parts, 256, 0, s>>>((const bf16_t*)X, N, (const int*)slots,   \
           (const bf16_t*)Qv, Q, (const unsigned*)bitmap, W, thr, K, rows_per_wave, 1, cs, ci);           \
     else if (Q <= 64)                                                                                   \
-      TDQ(NG, 1);                                                                                       \
+      TDQ(NG, 4);                                                                                       \
     else                                                                                                \
-      TDQ(NG, 2);                                                                                       \
+      TDQ(NG, 8);                                                                                       \
   } while (0)
   switch (d) {
     case 384: TDS(3); break;
