@@ -192,8 +192,27 @@ __device__ __forceinline__ float block_max(float v, float* red) {
   return t;
 }
 
+// x Phi(x) = max(x, 0) - |x|/2 erfc(|x| / sqrt 2), with erfc(z) = t Q(t) exp(-z^2), t = 1 / (1 + 0.3 z): Q is a
+// polynomial of degree 8 fitted to erfcx(z) / t over 0 <= z <= 14 by reweighted least squares (relative error 4e-8; in
+// fp32 2.4e-7 absolute and 2e-6 relative at worst over |x| <= 6, against 4.4e-7 and a cancelled tail of
+// x/2 (1 + erff)). 18 instructions, two of them transcendental; erff evaluates both of its branches where a wave's
+// lanes differ. Beyond |x| = 20 the term is 0 (-inf gives 0, NaN stays). Bound by the vector ALU: an instruction
+// takes a SIMD 4 cycles for a wave, a transcendental one 16. A 24105 x 4096 x 1024 fp16 product with it in the epilogue:
+// 249 -> 239 us.
 __device__ __forceinline__ float gelu_erf(float x) {
-  return 0.5f * x * (1.f + erff(x * 0.70710678118654752f));
+  const float a = fminf(fabsf(x), 20.f);
+  const float t = __builtin_amdgcn_rcpf(fmaf(a, 0.212132034f, 1.f));
+  float q = -0.0631891487f;
+  q = fmaf(q, t, 0.235351475f);
+  q = fmaf(q, t, -0.241223139f);
+  q = fmaf(q, t, 0.257284522f);
+  q = fmaf(q, t, -0.0361995057f);
+  q = fmaf(q, t, 0.102854722f);
+  q = fmaf(q, t, 0.0753173695f);
+  q = fmaf(q, t, 0.0852007243f);
+  q = fmaf(q, t, 0.0846030018f);
+  const float e = __builtin_amdgcn_exp2f(a * a * -0.721347520f);
+  return fmaf(-(q * t), a * e, x < 0.f ? 0.f : x);
 }
 
 // x * sigmoid(x) with the hardware reciprocal (1 ulp) instead of an IEEE division (a 10-instruction

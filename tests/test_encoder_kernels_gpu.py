@@ -51,3 +51,22 @@ def test_bert_embed_rows(T, D, dtype):
         want = torch.nn.functional.layer_norm(e, (D,), g.double(), b.double(), 1e-12)
         got = f(ids, ps, types, word, pos, typ, g, b, 1e-12)
         assert bool(((got.double() - want).abs() <= ulp * want.abs() + 1e-5 * (1 + want.abs())).all())
+
+
+@pytest.mark.parametrize("dtype,M,Kd", [(torch.bfloat16, 16, 256), (torch.bfloat16, 300, 128), (torch.float16, 300, 128)])
+def test_gelu_epilogue(dtype, M, Kd):
+    """The activation alone (an identity product): over its curve, its tails, infinities and NaN."""
+    w = torch.eye(Kd, device=DEV).to(dtype)
+    x = torch.linspace(-9, 9, M * Kd, device=DEV).view(M, Kd).to(dtype)
+    zero = torch.zeros(Kd, dtype=dtype, device=DEV)
+    f = K.gemm_f16 if dtype == torch.float16 else K.gemm
+    got = f(x, w, bias=zero, epi=K.EPI_GELU)
+    want = torch.nn.functional.gelu(x.double())
+    # half a unit in the last place of the result's type; 2e-6 relative and 2.4e-7 absolute before the rounding
+    ulp, tiny = (2.0 ** -11, 2.0 ** -25) if dtype == torch.float16 else (2.0 ** -8, 0.0)
+    assert bool(((got.double() - want).abs() <= (ulp + 2e-6) * want.abs() + 2.4e-7 + tiny).all())
+    big = 6e4 if dtype == torch.float16 else 3e38
+    bias = zero.clone()
+    bias[:5] = torch.tensor([math.inf, -math.inf, math.nan, big, -big])
+    got = f(torch.zeros_like(x), w, bias=bias, epi=K.EPI_GELU)[0]
+    assert got[0] == math.inf and bool(got[2].isnan()) and got[3] == bias[3] and got[4] == 0 and bool((got[5:] == 0).all())
