@@ -34,6 +34,10 @@
 //  * PERSIST: one workgroup per CU walks tile ids b, b + G, ... (G a multiple of 8: each id stays on
 //    the workgroup's XCD); the staged rows go to registers, then the next tile's prologue DMA is
 //    issued before this tile's stores (profiles/r5/gemm_persist/: +0.3..1 %, not for EPI_ROPE).
+//  * Tail: the tiles behind the last whole round of the chip (all of them, when they fill none) are each cut along K
+//    for tail_s workgroups, as many as the chip has room for. A workgroup leaves its fp32 partial in tail_ws, counts
+//    itself in on a counter, and the second of two to come adds the other's to its own, pair by pair in a fixed tree (so
+//    the result does not depend on who came when); who is left runs the epilogue. Nothing waits: no workgroup depends on another one running.
 #include "gemm.h"
 
 #include <cstdlib>
@@ -45,6 +49,7 @@ namespace {
 constexpr int BN = 256;
 constexpr int HALF_B = 16384;                // B half-tile: 128 rows x 64 bf16
 constexpr int SROW = 64 * 2 + 16;            // epilogue staging row stride (bytes)
+constexpr int TAIL_SKEW = 3;                 // K-tiles moved from an odd slice of a tail tile to the even one before it
 }  // namespace
 
 template <int N>
@@ -52,10 +57,19 @@ __device__ __forceinline__ void vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// The lane id, worked out anew at every call (the compiler cannot see that it is the same value): what is derived from
+// it stays local instead of living across the tile loop's registers, which have no room for it.
+__device__ __forceinline__ int fresh_lane() {
+  int z = 0;
+  asm volatile("" : "+s"(z));
+  return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, z));
+}
+
 template <int EPI, int BM, typename T = BF16T, bool PERSIST = false>
 __global__ void __launch_bounds__(512)
 gemm8p_kernel(GemmArgs p) {
   static_assert(BM == 256 || BM == 128, "BM");
+  constexpr bool TAIL = PERSIST && EPI != EPI_GELU;  // (beside the activation's registers the tail's spill)
   constexpr int HALF_A = BM / 2 * 128;       // A half-tile: BM/2 rows x 64 bf16
   constexpr int OFF_A0 = 0, OFF_A1 = HALF_A, OFF_B0 = 2 * HALF_A, OFF_B1 = 2 * HALF_A + HALF_B;
   constexpr int BUF = 2 * HALF_A + 2 * HALF_B;
@@ -85,7 +99,33 @@ gemm8p_kernel(GemmArgs p) {
     m0_ = (first_m + tin % gsz) * BM;
     n0_ = (tin / gsz) * BN;
   };
-  int id = blockIdx.x, m0, n0;
+  // the unit behind id: PERSIST's next whole tile, then this workgroup's slice of a tail tile, if it has one. (Slices
+  // of a tile are TR workgroups apart, TR a multiple of 8: the tile ids keep the XCDs that xcd_remap gives them.)
+  const int nkt = p.K / 64, full = TAIL && p.tail_s > 1 ? ntiles / (int)GEMM_TAIL_WGS * (int)GEMM_TAIL_WGS : ntiles;
+  const int rest = ntiles - full, TR = (rest + 7) & ~7;
+  int id = blockIdx.x, m0, n0, kb = 0, nk = nkt;  // nk >= 2 (host-checked)
+  [[maybe_unused]] bool tail = false;
+  // this workgroup's tail tile and, from bit 16 on, its slice; -1: none (worked out here, in one register: the division
+  // does not fit beside the epilogue's)
+  [[maybe_unused]] int unit = -1;
+  if constexpr (TAIL) {
+    const int t = blockIdx.x % max(TR, 1), sl = blockIdx.x / max(TR, 1);
+    if (p.tail_s > 1 && t < rest && sl < p.tail_s) unit = t | sl << 16;
+    unit = __builtin_amdgcn_readfirstlane(unit);
+  }
+  auto to_tail = [&]() __attribute__((always_inline)) {  // false: no slice for this workgroup
+    if (unit < 0) return false;
+    const int sl = unit >> 16, lg = __builtin_ctz(p.tail_s);
+    // (an even slice has a few K-tiles more than the odd one that it meets first, see the meeting)
+    const int skew = min(TAIL_SKEW, nkt >> lg >> 2);
+    id = full + (unit & 0xffff);
+    kb = (sl * nkt >> lg) + (sl & 1) * skew;
+    nk = ((sl + 1) * nkt >> lg) + (~sl & 1) * skew - kb;
+    tail = true;
+    return true;
+  };
+  if constexpr (TAIL)
+    if (full == 0 && !to_tail()) return;
   tile_of(id, m0, n0);
 
   // ---- LDS-DMA sources: buffer resources at the tile's first A row / W row; wave w fills rows
@@ -94,13 +134,12 @@ gemm8p_kernel(GemmArgs p) {
   //      outputs that are never stored.
   __amdgpu_buffer_rsrc_t rsa, rsw;
   unsigned aoffs[2][2], boffs[2][2];  // (fixed extents: a template-dependent array extent in a builtin argument makes hipcc's host pass drop the launch stub)
-  auto sources = [&](int m0_, int n0_) __attribute__((always_inline)) {
-    int sl = lane;  // (laundered like the epilogue's lane indices: recomputed per tile, not hoisted)
-    if constexpr (PERSIST) asm volatile("" : "+v"(sl));
+  auto sources = [&](int m0_, int n0_, int kb_) __attribute__((always_inline)) {  // kb_: the first K-tile
+    const int sl = PERSIST ? fresh_lane() : lane;
     rsa = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)((const char*)p.A + (size_t)m0_ * p.lda * 2), (short)0, 0x7ffffff0, 0x00020000);
+        (void*)((const char*)p.A + (size_t)m0_ * p.lda * 2 + kb_ * 128), (short)0, 0x7ffffff0, 0x00020000);
     rsw = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)((const char*)p.W + (size_t)n0_ * p.K * 2), (short)0, 0x7ffffff0, 0x00020000);
+        (void*)((const char*)p.W + (size_t)n0_ * p.K * 2 + kb_ * 128), (short)0, 0x7ffffff0, 0x00020000);
 #pragma unroll
     for (int j = 0; j < NA; ++j) {
       const int r = (wid * NA + j) * 8 + (sl >> 3);
@@ -221,8 +260,6 @@ gemm8p_kernel(GemmArgs p) {
   };
   using T_ = std::true_type;
   using F_ = std::false_type;
-  const int nk = p.K / 64;  // >= 2 (host-checked)
-
   constexpr bool SW = (EPI == EPI_SWIGLU);
   constexpr int HC = SW ? 16 : 32;   // staged columns per jh half (one contiguous global run)
   constexpr int CPR = 2 * HC / 8;    // 16-B chunks per staged row
@@ -237,7 +274,7 @@ gemm8p_kernel(GemmArgs p) {
   using X0 = std::integral_constant<int, 0>;
   using XN = std::integral_constant<int, XS>;
 
-  sources(m0, n0);
+  sources(m0, n0, kb);
   prologue();
   bool first = true;
   for (;;) {
@@ -269,11 +306,60 @@ gemm8p_kernel(GemmArgs p) {
     if (!wg) bar();  // re-align the groups
     __syncthreads();
 
-    // lane-derived epilogue indices from a copy of the lane id the compiler cannot see through, so
-    // they are recomputed here rather than hoisted out of the tile loop (live across the K-loop
-    // they pushed a persistent instance past 256 VGPRs into scratch)
-    int el = lane;
-    if constexpr (PERSIST) asm volatile("" : "+v"(el));
+    if constexpr (TAIL) {
+      if (tail) {
+        // Slices meet in pairs, sums of two in pairs again: at each meeting the first to come leaves its sum and goes,
+        // the second adds that to its own (a + b whoever it is). Fragment f of thread tid is at [f][tid], 16 B, moved
+        // past the XCDs' L2s (sc1) to where all of them see it: no fence has to write back and invalidate a whole L2
+        // (plain stores between __threadfence()s cost 100 us a launch, a last workgroup that adds up all slices 50 for 8).
+        constexpr int NF = 8 * MI, NV = 8;
+        const int t = unit & 0xffff;
+        const int ft = wid * 64 + fresh_lane();
+        const unsigned at = ft * 16u;
+        const __amdgpu_buffer_rsrc_t rst =
+            __builtin_amdgcn_make_buffer_rsrc((void*)p.tail_ws, (short)0, (int)(GEMM_TAIL_WGS * 65536 * 4), 0x00020000);
+        int node = t * 8, half = p.tail_s / 2;  // the level's first counter, its meetings
+        for (int sl = unit >> 16, level = 0; half > 0; ++level, sl >>= 1, node += half, half >>= 1) {
+          const unsigned own = (t * p.tail_s + (sl << level)) * (unsigned)(NF * 8192);
+          const unsigned other = (t * p.tail_s + ((sl ^ 1) << level)) * (unsigned)(NF * 8192);
+          // the even slice is longer: mostly the odd one's sum is there when it comes, and its own need not be written
+          int* cnt = p.tail_cnt + node + (sl >> 1);
+          if (ft == 0) *(int*)smem = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __syncthreads();
+          bool second = *(volatile int*)smem != 0;
+          if (!second) {
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+              __builtin_amdgcn_raw_buffer_store_b128(
+                  __builtin_bit_cast(u32x4_t, acc[f / (4 * MI)][f / (2 * MI) % 2][f / 2 % MI][f % 2]), rst,
+                  at + f * 8192, own, 16);
+            vmcnt<0>();  // this wave's stores are done; then every wave's
+            __syncthreads();
+            if (ft == 0)
+              *(int*)smem = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            second = *(volatile int*)smem != 0;
+            if (!second) return;
+          }
+          if (ft == 0) *cnt = 0;
+#pragma unroll
+          for (int f0 = 0; f0 < NF; f0 += NV) {
+            u32x4_t v[NV];
+#pragma unroll
+            for (int f = 0; f < NV; ++f)
+              v[f] = __builtin_amdgcn_raw_buffer_load_b128(rst, at + (f0 + f) * 8192, other, 16);
+#pragma unroll
+            for (int f = 0; f < NV; ++f) {
+              const int g = f0 + f;
+              acc[g / (4 * MI)][g / (2 * MI) % 2][g / 2 % MI][g % 2] += __builtin_bit_cast(f32x4_t, v[f]);
+            }
+          }
+          __syncthreads();  // (smem is written again)
+        }
+      }
+    }
+
+    const int el = PERSIST ? fresh_lane() : lane;
     const int efr = el & 15, efg = el >> 4;
     const int ch = el % CPR;
     const int jh = ch / (HC / 8);
@@ -387,15 +473,18 @@ gemm8p_kernel(GemmArgs p) {
     if constexpr (XS > 0)
       rsc = __builtin_amdgcn_make_buffer_rsrc((void*)(p.C + (size_t)m0 * p.ldc), (short)0,
                                               (int)min((long long)(p.M - m0) * p.ldc * 2, 0x7ffffff0ll), 0x00020000);
-    const int nid = id + (int)gridDim.x;
-    const bool more = PERSIST && nid < ntiles;
-    int nm0 = 0, nn0 = 0;
+    [[maybe_unused]] const int om0 = m0;  // of the tile that is stored below
+    bool more = false;
     if constexpr (PERSIST) {
       lgkm0();
       bar();  // every wave holds its staged rows: both operand buffers are free
+      if (!tail) {
+        id += (int)gridDim.x;
+        more = id < full || (TAIL && to_tail());
+      }
       if (more) {
-        tile_of(nid, nm0, nn0);
-        sources(nm0, nn0);
+        tile_of(id, m0, n0);
+        sources(m0, n0, kb);
         prologue();
       }
     }
@@ -456,7 +545,7 @@ gemm8p_kernel(GemmArgs p) {
           if constexpr (XS > 0) {
             // exactly one store instruction per row, whatever the row / column (the counted waits
             // of the next tile's K-tile 0 rely on it): out-of-range ones land past num_records
-            const unsigned off = col_ok ? (unsigned)((gm - m0) * p.ldc + gcol) * 2u : 0x80000000u;
+            const unsigned off = col_ok ? (unsigned)((gm - om0) * p.ldc + gcol) * 2u : 0x80000000u;
             __builtin_amdgcn_raw_buffer_store_b128(v, rsc, off, 0, 0);
           } else {
             *(u32x4_t*)(p.C + (size_t)gm * p.ldc + gcol) = v;
@@ -465,7 +554,6 @@ gemm8p_kernel(GemmArgs p) {
       }
     }
     if (!more) break;
-    id = nid; m0 = nm0; n0 = nn0;
   }
 #undef ISSUE_A
 #undef ISSUE_B
@@ -508,12 +596,47 @@ DA_EXPORT int da_gemm8p_persist(int on) {
   return prev;
 }
 
+// What the last round takes with `sl` workgroups per tile (1: whole tiles), in hundredths of a K-tile of bm rows: the
+// longer slice's K-tiles, and for each meeting what writing and reading the partials was measured to take, which grows
+// with the workgroups that write at once, more where the last whole round's stores are still under way. 5 % on top: a
+// close call stays whole.
+//   7067 x 3072 x 3072 / 8192 (1.31 rounds, bf16): 125 -> 111 / 296 -> 259 us   24105 x 1024 x 4096 (1.48, fp16): 190 -> 171
+//   1000 x 4096 x 4096 / 14336 (0.25): 48 -> 36 / 153 -> 101                   3618 x 320 x 8192 (0.12): 84 -> 39
+//   left whole: 24105 x 1024 x 1024 (59, cut: 71), 24105 x 3072 x 1024 (148, cut: 153), 2000 x 3072 x 3072 (40, cut: 42)
+static long tail_cost(int ntiles, int nk, int bm, int sl) {
+  if (sl == 1) return nk * 100L;
+  const bool behind = ntiles > (int)GEMM_TAIL_WGS;
+  long c = ((nk + sl - 1) / sl + min(TAIL_SKEW, nk / sl / 4)) * 100L;
+  for (int wgs = ntiles % (int)GEMM_TAIL_WGS * sl; sl > 1; sl /= 2, wgs /= 2)
+    c += (behind ? 500 + 1500L * wgs / 256 : 700 + 200L * wgs / 256) * (bm == 256 ? 10 : 7) / 10;
+  return c * 105 / 100;
+}
+
+// Workgroups per tail tile: 1, or 2, 4 or 8 where the chip has room for them beside each other, they have at least 4
+// K-tiles each, and that is the fastest.
+static int tail_slices(int ntiles, int nk, int bm) {
+  const int G = (int)GEMM_TAIL_WGS, rest = ntiles % G;
+  int best = 1;
+  if (num_cus() < G || rest == 0) return best;
+  for (int sl = 2; sl <= 8 && sl * ((rest + 7) & ~7) <= G && nk / sl >= 4; sl *= 2)
+    if (tail_cost(ntiles, nk, bm, sl) < tail_cost(ntiles, nk, bm, best)) best = sl;
+  return best;
+}
+
 template <int EPI, int BM, typename T>
-static void launch8p_epi(const GemmArgs& a, int ntiles, hipStream_t s) {
+static void launch8p_epi(const GemmArgs& a0, int ntiles, hipStream_t s) {
+  GemmArgs a = a0;
   const int cus = num_cus();
   // (not EPI_ROPE: its per-row positions / slots / cos-sin next to the tile loop's state spill past
   // 256 VGPRs, and the persistent QKV projection measured 4 % slower, profiles/r5/gemm_persist/)
   if constexpr (EPI != EPI_ROPE) {
+    a.tail_s = EPI != EPI_GELU && persist_on() && a.tail_ws ? tail_slices(ntiles, a.K / 64, BM) : 1;
+    const int rest = ntiles % (int)GEMM_TAIL_WGS;
+    if (a.tail_s > 1) {
+      const int grid = ntiles >= (int)GEMM_TAIL_WGS ? (int)GEMM_TAIL_WGS : a.tail_s * ((rest + 7) & ~7);
+      gemm8p_kernel<EPI, BM, T, true><<<dim3(grid), dim3(512), 0, s>>>(a);
+      return;
+    }
     if (persist_on() && ntiles > cus && cus >= 8) {
       gemm8p_kernel<EPI, BM, T, true><<<dim3(cus & ~7), dim3(512), 0, s>>>(a);
       return;
@@ -557,12 +680,15 @@ static int launch8p(const GemmArgs& a0, int epi, hipStream_t s) {
 // 252 128-row tiles in one wave instead of 132 256-row tiles on half the chip; QA-sized chunks
 // (M ~ 64k) keep 256 (the round-3 rule, 256 rows once the 256-row grid reached half the chip,
 // measured 65.5 vs 74.9 us per O projection at M ~ 2.6k: profiles/r4/bm_rule/).
-int gemm8p_pick_bm(int M, int N) {
-  const long ntn = (N + 255) / 256;
-  const long t256 = (long)((M + 255) / 256) * ntn, t128 = (long)((M + 127) / 128) * ntn;
-  const int cus = num_cus();
-  const long w256 = (t256 + cus - 1) / cus, w128 = (t128 + cus - 1) / cus;
-  return w128 * 72 < w256 * 100 ? 128 : 256;
+// A tail (tail_slices) costs its slices' K-tiles and meetings, and has to be 5 % better than the other height.
+int gemm8p_pick_bm(int M, int N, int K, bool tail) {
+  const int ntn = (N + 255) / 256, cus = num_cus(), nk = K / 64;
+  auto cost = [&](int bm, int per_ktile) {
+    const long t = (long)((M + bm - 1) / bm) * ntn;
+    const int s = tail && t < 0x7fffffff ? tail_slices((int)t, nk, bm) : 1;
+    return ((t - 1) / cus * nk * 100 + tail_cost((int)t, nk, bm, s)) * per_ktile * (s > 1 ? 105 : 100);
+  };
+  return cost(128, 72) < cost(256, 100) ? 128 : 256;
 }
 
 // epi + 100: the same kernel on fp16 operands / output (v_mfma_f32_16x16x32_f16)
@@ -577,7 +703,8 @@ int launch_gemm8p(const GemmArgs& a, int epi, hipStream_t s, int bm) {
 // resid fp16, fp32 accumulation; epi NONE / BIAS / GELU / RESID. Every M on the phase-split tile
 // (128-row tiles below half a chip of 256-row ones): the fp16 path has no decode-sized tiles.
 DA_EXPORT int da_gemm_f16(const void* A, int lda, const void* W, void* C, int ldc, const void* bias,
-                          const void* resid, int ldr, int M, int N, int K, int epi, void* stream) {
+                          const void* resid, int ldr, int M, int N, int K, int epi, void* tail_ws, void* tail_cnt,
+                          void* stream) {
   if (M < 1 || K % 64 || K < 128 || N % 8 || lda % 8 || ldc % 8) return (int)hipErrorInvalidValue;
   if (epi != EPI_NONE && epi != EPI_BIAS && epi != EPI_GELU && epi != EPI_RESID) return (int)hipErrorInvalidValue;
   if (epi == EPI_RESID && (!resid || ldr % 8)) return (int)hipErrorInvalidValue;
@@ -585,5 +712,6 @@ DA_EXPORT int da_gemm_f16(const void* A, int lda, const void* W, void* C, int ld
   a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = (bf16_t*)C;
   a.bias = (const bf16_t*)bias; a.resid = (const bf16_t*)resid;
   a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc; a.ldr = ldr; a.k_per_split = K;
-  return launch_gemm8p(a, 100 + epi, (hipStream_t)stream, gemm8p_pick_bm(M, N));
+  if (tail_ws && tail_cnt && epi != EPI_GELU) { a.tail_ws = (float*)tail_ws; a.tail_cnt = (int*)tail_cnt; }
+  return launch_gemm8p(a, 100 + epi, (hipStream_t)stream, gemm8p_pick_bm(M, N, K, a.tail_ws != nullptr));
 }

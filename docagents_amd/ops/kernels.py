@@ -34,7 +34,7 @@ c_void_p, c_int, c_float, c_uint, c_size_t = (ctypes.c_void_p, ctypes.c_int, cty
 
 _SIGS = {
     "da_gemm_bf16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int,
-                     c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p],
+                     c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p],
     "da_gemm_rope": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int] + [c_void_p] * 5
                     + [c_int] * 5 + [c_void_p],
     "da_gemm_fp8": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int,
@@ -87,7 +87,7 @@ _SIGS = {
     "da_gemm8p_persist": [c_int],
     "da_gemm4w_variant": [c_int],
     "da_gemm_f16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
-                    c_void_p],
+                    c_void_p, c_void_p, c_void_p],
     "da_flash_attn_f16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int,
                           c_int, c_int, c_float, c_void_p, c_int, c_void_p],
     "da_layernorm_f16": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
@@ -232,6 +232,30 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
     return buf
 
 
+# Scratch of the prefill products' last round (csrc/gemm8p.hip, "Tail"): 256 workgroups' fp32 partials and their tiles'
+# counters, 64 MB, per stream: streams run products beside each other. At most TAIL_STREAMS of them per device have one;
+# never given back (the caching allocator would hand the memory to kernels that may still run beside it).
+TAIL_STREAMS = 8
+_TAIL: dict = {}
+
+
+def _gemm_tail(device, stream: int):
+    """(partials, counters) of a stream, (None, None): this product keeps its tiles whole. Under capture too: a graph
+    may be replayed on another stream, beside the one that it was recorded on."""
+    if torch.cuda.is_current_stream_capturing():
+        return None, None
+    key = (device.index, stream)
+    bufs = _TAIL.get(key)
+    if bufs is None:
+        with _LOCK:
+            bufs = _TAIL.get(key)
+            if bufs is None and sum(k[0] == device.index for k in _TAIL) >= TAIL_STREAMS:
+                return None, None
+            bufs = _TAIL[key] = bufs or (torch.empty(256 * 256 * 256, dtype=torch.float32, device=device),
+                                         torch.zeros(256 * 8, dtype=torch.int32, device=device))
+    return _ptr(bufs[0]), _ptr(bufs[1])
+
+
 def gemv_fusable(M: int, N: int, K: int, epi: int = EPI_NONE) -> bool:
     """True when gemm() runs the batch-1 GEMV (which can also fuse the input RMSNorm)."""
     return M == 1 and K % 512 == 0 and N % 4 == 0 and (epi not in GATED or N % 32 == 0)
@@ -287,8 +311,10 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
     ws = None
     if splits > 1:
         ws = _workspace(splits * M * N * 4, a.device)
+    stream = torch.cuda.current_stream().cuda_stream
+    tail = _gemm_tail(a.device, stream) if M >= 256 else (None, None)
     rc = lib().da_gemm_bf16(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
-                            M, N, K, epi, tile, splits, _ptr(ws), _ptr(gamma), float(eps), _stream())
+                            M, N, K, epi, tile, splits, _ptr(ws), _ptr(gamma), float(eps), *tail, c_void_p(stream))
     _check(rc, "gemm")
     return out
 
@@ -1097,8 +1123,10 @@ def gemm_f16(a, w, bias=None, epi: int = EPI_NONE, resid=None, out=None) -> torc
     if out is None:
         out = torch.empty((M, N), dtype=torch.float16, device=a.device)
     _req(out.dtype == torch.float16 and out.shape == (M, N) and out.stride(1) == 1 and out.stride(0) % 8 == 0, "out")
+    stream = torch.cuda.current_stream().cuda_stream
+    tail = _gemm_tail(a.device, stream) if M >= 256 else (None, None)
     _check(lib().da_gemm_f16(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
-                             M, N, K, epi, _stream()), "gemm_f16")
+                             M, N, K, epi, *tail, c_void_p(stream)), "gemm_f16")
     return out
 
 
