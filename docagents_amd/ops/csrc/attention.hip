@@ -786,8 +786,8 @@ __device__ __forceinline__ int dec_chunk(int L, int nsplit, int chunk_arg) {
 
 __device__ __forceinline__ void dec_store(float o, float M, float ls, int b, int h, int d, int H, int nsplit,
                                           int split, int D, float* po, float* pm, float* pl, bf16_t* out,
-                                          int ldo) {
-  if (nsplit == 1) {
+                                          int ldo, int act) {
+  if (act == 1) {
     out[(size_t)b * ldo + h * D + d] = f2bf(ls > 0.f ? o / ls : 0.f);
     return;
   }
@@ -802,8 +802,9 @@ __device__ __forceinline__ void dec_store(float o, float M, float ls, int b, int
 // the partials from L2 (agent-scope loads: past its L1) — L2 round trips instead of uncached ones.
 template <int D, int G, bool XC = false>
 __device__ __forceinline__ void dec_finish(const float* po, const float* pm, const float* pl, int H, int Hkv,
-                                           int nsplit, int b, int hk, int* cnt, bf16_t* out, int ldo, int* s_last) {
-  if (nsplit == 1 || cnt == nullptr) return;  // no counters: the host launches decode_combine_kernel
+                                           int nsplit, int b, int hk, int* cnt, bf16_t* out, int ldo, int* s_last,
+                                           int act) {
+  if (act == 1 || cnt == nullptr) return;  // no counters: the host launches decode_combine_kernel
   const int tid = threadIdx.x;
   // Partials and tickets live in UNCACHED memory (da_malloc_uncached: MTYPE UC, L2 bypassed), so
   // device-wide visibility needs only this workgroup's stores to have completed — no
@@ -814,7 +815,7 @@ __device__ __forceinline__ void dec_finish(const float* po, const float* pm, con
   if (tid == 0) {
     int* c = &cnt[b * Hkv + hk];
     const int old = XC ? __hip_atomic_fetch_add(c, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : atomicAdd(c, 1);
-    *s_last = old == nsplit - 1;
+    *s_last = old == act - 1;
     if (*s_last) {
       if constexpr (XC) __hip_atomic_store(c, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       else *c = 0;
@@ -833,11 +834,11 @@ __device__ __forceinline__ void dec_finish(const float* po, const float* pm, con
     const int g = i / D, d = i % D, h = hk * G + g;
     const size_t base = ((size_t)b * H + h) * nsplit;
     float M = -INFINITY, lsum = 0.f, acc = 0.f;
-    for (int s0 = 0; s0 < nsplit; s0 += 8) {
+    for (int s0 = 0; s0 < act; s0 += 8) {
       float ms[8], ls[8], os[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int s = min(s0 + j, nsplit - 1);
+        const int s = min(s0 + j, act - 1);
         ms[j] = ld(pm + base + s);
         ls[j] = ld(pl + base + s);
         os[j] = ld(po + (base + s) * D + d);
@@ -845,14 +846,14 @@ __device__ __forceinline__ void dec_finish(const float* po, const float* pm, con
       float mx = M;
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        if (s0 + j < nsplit) mx = fmaxf(mx, ms[j]);
+        if (s0 + j < act) mx = fmaxf(mx, ms[j]);
       const float mu = (mx == -INFINITY) ? 0.f : mx;
       const float r = (M == -INFINITY) ? 0.f : exp2f(M - mu);
       lsum *= r;
       acc *= r;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        if (s0 + j >= nsplit) continue;
+        if (s0 + j >= act) continue;
         const float f = exp2f(ms[j] - mu);
         lsum += ls[j] * f;
         acc += os[j] * f;
@@ -1226,10 +1227,10 @@ decode_attn_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __restri
       o += svn[d] * f;
       ls += f;
     }
-    dec_store(o, M, ls, b, hk * G + g, d, H, nsplit, split, D, po, pm, pl, out, ldo);
+    dec_store(o, M, ls, b, hk * G + g, d, H, nsplit, split, D, po, pm, pl, out, ldo, nsplit);
   }
   __shared__ int s_last;
-  dec_finish<D, G, XC>(po, pm, pl, H, Hkv, nsplit, b, hk, cnt, out, ldo, &s_last);
+  dec_finish<D, G, XC>(po, pm, pl, H, Hkv, nsplit, b, hk, cnt, out, ldo, &s_last, nsplit);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1246,6 +1247,10 @@ decode_attn_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __restri
 //                         is a contiguous [64 x D] block of the cache, so it is copied by LDS-DMA
 //                         (global_load_lds, 1 KiB per wave-instruction) with an XOR chunk swizzle
 //                         on the source address that makes the transposed reads conflict-free.
+// by_len: a row is split by its own length, and splits are the slowest grid dimension: as the fastest one, the
+// workgroups of a launch with two splits whose rows need one only were all on the even XCDs (64 rows of 2048 keys: 147 us
+// against 86). A workgroup of a split past the row's keys ends at once. Tried and slower: two tiles in flight per wave
+// (hipcc drains the DMA before the transposed reads, and twice the LDS leaves one workgroup per CU).
 template <int D>
 __device__ __forceinline__ int vswz(int r) {
   return D == 128 ? ((r & 7) << 1) : (((r >> 1) & 3) << 1);
@@ -1258,7 +1263,7 @@ decode_attn_gqa_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __re
                    const int* __restrict__ pre,
                        int H, int Hkv, int max_seq, int chunk_max, int nsplit, float scale_log2e,
                        float* __restrict__ po, float* __restrict__ pm, float* __restrict__ pl,
-                       bf16_t* __restrict__ out, int ldo, int* __restrict__ cnt) {
+                       bf16_t* __restrict__ out, int ldo, int* __restrict__ cnt, int by_len) {
   static_assert(D == 64 || D == 128, "GQA MFMA decode supports head dims 64 and 128");
   constexpr int KT = 64, NDS = D / 32, NDT = D / 16, NS = D / 8;   // d-steps (S), d-tiles (O), 16-B chunks/row
   constexpr int VBYTES = KT * D * 2, NDMA = VBYTES / 1024;
@@ -1267,10 +1272,14 @@ decode_attn_gqa_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __re
   __shared__ __attribute__((aligned(16))) char sv[4 * VBYTES];
   __shared__ float swm[4][16], swl[4][16];
 
-  const int split = blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
+  const int hk = by_len ? blockIdx.x : blockIdx.y, b = by_len ? blockIdx.y : blockIdx.z;
+  const int split = by_len ? blockIdx.z : blockIdx.x;
   const int L = lens[b];
   DA_ASSERT(L >= 0 && L <= max_seq && slot[b] >= 0);
-  const int chunk = dec_chunk(L, nsplit, chunk_max);
+  // by_len: a row's keys over as many splits as hold chunk_max of them each, evenly; the others have nothing to do
+  const int act = by_len && cnt ? min(nsplit, max(1, (L + chunk_max - 1) / chunk_max)) : nsplit;
+  if (split >= act) return;
+  const int chunk = dec_chunk(L, act, chunk_max);
   const int kstart = split * chunk;
   const int kend = min(L, kstart + chunk);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -1395,10 +1404,10 @@ decode_attn_gqa_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __re
       o += so[(ww * 16 + g) * D + d] * f;
       ls += swl[ww][g] * f;
     }
-    dec_store(o, M, ls, b, hk * G + g, d, H, nsplit, split, D, po, pm, pl, out, ldo);
+    dec_store(o, M, ls, b, hk * G + g, d, H, nsplit, split, D, po, pm, pl, out, ldo, act);
   }
   __shared__ int s_last;
-  dec_finish<D, G>(po, pm, pl, H, Hkv, nsplit, b, hk, cnt, out, ldo, &s_last);
+  dec_finish<D, G>(po, pm, pl, H, Hkv, nsplit, b, hk, cnt, out, ldo, &s_last, act);
 }
 
 // MHA decode attention on MFMA for few (row, kv head) pairs (batch 1..: the p50 path). The VALU
@@ -1624,10 +1633,10 @@ decode_attn_mfma1_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __
       o += svn[d] * f;
       ls += f;
     }
-    dec_store(o, M, ls, b, hk, d, H, nsplit, split, D, po, pm, pl, out, ldo);
+    dec_store(o, M, ls, b, hk, d, H, nsplit, split, D, po, pm, pl, out, ldo, nsplit);
   }
   __shared__ int s_last;
-  dec_finish<D, 1, XC>(po, pm, pl, H, Hkv, nsplit, b, hk, cnt, out, ldo, &s_last);
+  dec_finish<D, 1, XC>(po, pm, pl, H, Hkv, nsplit, b, hk, cnt, out, ldo, &s_last, nsplit);
 }
 
 template <int D>
@@ -1682,6 +1691,8 @@ static int launch_decode(int G, dim3 grid, hipStream_t s, const bf16_t* q, int l
                          const bf16_t* vc, const int* lens, const int* slot, const int* pre, int H, int Hkv, int max_seq, int chunk,
                          int nsplit, float sl2e, float* po, float* pm, float* pl, bf16_t* out, int ldo,
                          int* cnt, DecRope rope, int xc) {
+  const int by_len = xc >> 1;  // GQA on MFMA: splits by the row's length (bit 1)
+  xc &= 1;
   static int mfma1 = -1;
   if (mfma1 < 0) {
     const char* e = getenv("DA_DECODE_MFMA1");
@@ -1708,10 +1719,11 @@ static int launch_decode(int G, dim3 grid, hipStream_t s, const bf16_t* q, int l
   }
   if (rope.cs) return (int)hipErrorInvalidValue;  // fused RoPE: MHA kernel only
   if constexpr (D == 64 || D == 128) {
+    const dim3 grid_g = by_len ? dim3(Hkv, grid.z, nsplit) : grid;
     switch (G) {
-      case 2: decode_attn_gqa_kernel<D, 2><<<grid, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt); break;
-      case 4: decode_attn_gqa_kernel<D, 4><<<grid, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt); break;
-      case 8: decode_attn_gqa_kernel<D, 8><<<grid, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt); break;
+      case 2: decode_attn_gqa_kernel<D, 2><<<grid_g, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt, by_len); break;
+      case 4: decode_attn_gqa_kernel<D, 4><<<grid_g, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt, by_len); break;
+      case 8: decode_attn_gqa_kernel<D, 8><<<grid_g, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt, by_len); break;
       default: return (int)hipErrorInvalidValue;
     }
     return (int)hipGetLastError();

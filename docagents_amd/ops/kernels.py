@@ -737,16 +737,30 @@ def _uncached(tag: str, nbytes: int, device) -> _RawBuf:
     return bufs[-1]
 
 
-def _decode_split(B: int, Hkv: int, max_len: int, chunk: int):
+def _decode_split(B: int, Hkv: int, max_len: int, chunk: int, by_len: bool = False):
     """(chunk, nsplit) of a decode-attention launch (static for a captured graph: from max_len)."""
+    want = max_len * B * Hkv
+    if chunk <= 0 and by_len:
+        # splits by a row's own length: merging costs a split 10 us and more, and a second workgroup on a CU slows the
+        # first: 340 workgroups if every row were full (rows are half that on average), whole rows from 192 on
+        chunk = max_len if B * Hkv >= 192 else max(512, math.ceil(want / 340 / 256) * 256)
     if chunk <= 0:
         # measured on MI355X (profiles/decode_attn_chunks_r1.txt): per-workgroup overhead dominates
         # small chunks; aim for ~768 workgroups, 512..4096 keys each
-        want = max_len * B * Hkv / 768
         chunk = 512
-        while chunk < want and chunk < 4096:
+        while chunk < want / 768 and chunk < 4096:
             chunk *= 2
+    chunk = math.ceil(chunk / 64) * 64
     return chunk, max(1, math.ceil(max_len / chunk))
+
+
+def _decode_by_len(B: int, H: int, Hkv: int, D: int, max_len: int) -> bool:
+    """Few grouped-query (row, head) pairs are split by the rows' own length, not over every split of the launch: below 320
+    pairs with a cache of up to 4096 keys, below 128 with a longer one. 8 KV heads x 128, rows of 500 - 3000 of 4096: 8 /
+    16 / 32 rows 29.5 / 39.4 / 64.1 -> 25.0 / 33.2 / 55.2 us, 33 rows of 100 - 400: 26.5 -> 17.0; of 1000 - 8000 of 8192:
+    4 / 8 / 12 rows 29.5 / 42.2 / 56.9 -> 24.5 / 36.9 / 49.1. Beyond, the even splits are as good or better (48 rows of
+    500 - 3000: 86 against 93; 16 rows of 1000 - 8000: 72 against 77)."""
+    return H != Hkv and D in (64, 128) and B * Hkv < (320 if max_len <= 4096 else 128)
 
 
 # Same-XCD split exchange of the batch-1..small-batch MHA decode attention (attention.hip, VAR bit 3):
@@ -824,8 +838,9 @@ def decode_attn(q, k_cache, v_cache, lens, slot, H, Hkv, D, max_len: int, chunk:
     [B, (H + 2 Hkv) D]; the kernel applies RoPE to q and the new token's k and writes that token's
     k / v into the cache at pos (== lens - 1) — the decode step's rope_cache launch folded in."""
     cs, ps = _decode_checks(q, k_cache, v_cache, lens, slot, H, Hkv, D, max_len, pre, rope)
-    chunk, nsplit = _decode_split(q.shape[0], Hkv, max_len, chunk)
     B = q.shape[0]
+    by_len = _decode_by_len(B, H, Hkv, D, max_len)
+    chunk, nsplit = _decode_split(B, Hkv, max_len, chunk, by_len)
     ws = _workspace(B * H * nsplit * (D + 2) * 4, q.device)
     if out is None:
         out = torch.empty((B, H * D), dtype=torch.bfloat16, device=q.device)
@@ -841,7 +856,7 @@ def decode_attn(q, k_cache, v_cache, lens, slot, H, Hkv, D, max_len: int, chunk:
             ws = _uncached("decode_ws", B * H * nsplit * (D + 2) * 4, q.device)
     _check(lib().da_decode_attn(_ptr(q), q.stride(0), _ptr(k_cache), _ptr(v_cache), _ptr(lens), _ptr(slot), _ptr(pre), B, H,
                                 Hkv, D, k_cache.shape[2], chunk, nsplit, float(scale), _ptr(ws), _ptr(out), out.stride(0),
-                                _ptr(cnt), _ptr(cs), _ptr(ps), xc, _stream()), "decode_attn")
+                                _ptr(cnt), _ptr(cs), _ptr(ps), xc | 2 * by_len, _stream()), "decode_attn")
     return out
 
 

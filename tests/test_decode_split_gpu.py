@@ -1,0 +1,37 @@
+"""Grouped-query decode attention with splits by the rows' own length, against fp32."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from docagents_amd.ops import kernels as K  # noqa: E402
+from docagents_amd.ops import reference as R  # noqa: E402
+
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("H,Hkv,D", [(8, 2, 128), (16, 8, 64), (8, 1, 128)])
+@pytest.mark.parametrize("chunk", [0, 64, 512, 640])
+def test_rows_of_every_length(H, Hkv, D, chunk, monkeypatch):
+    """One key, a split exactly full and one key more, the whole cache; with the merge in the kernel and by itself; the
+    tickets are back at zero for the launches that follow; a shared head in another slot."""
+    torch.manual_seed(H + chunk)
+    S, lens = 1300, [1, 63, 64, 65, 512, 513, 640, 641, 1024, 1025, 1300]
+    B = len(lens)
+    kc, vc = ((torch.randn(B + 1, Hkv, S, D, device=DEV)).bfloat16() for _ in range(2))
+    q = torch.randn(B, H * D, device=DEV).bfloat16()
+    lt = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    slot = torch.randperm(B, device=DEV).int()
+    pre = torch.zeros(B, 2, dtype=torch.int32, device=DEV)
+    pre[4:, 0], pre[4:, 1] = 64, B
+    kx, vx = kc.clone(), vc.clone()
+    for b in range(4, B):
+        kx[slot[b], :, :64], vx[slot[b], :, :64] = kc[B, :, :64], vc[B, :, :64]
+    for p, k, v in ((None, kc, vc), (pre, kx, vx)):
+        want = R.decode_attn(q, k, v, lt, slot, H, Hkv, D).float()
+        for fused in (True, False):
+            monkeypatch.setattr(K, "_FUSED_COMBINE", fused)
+            for _ in range(3):
+                got = K.decode_attn(q, kc, vc, lt, slot, H, Hkv, D, max_len=S, chunk=chunk, pre=p).float()
+                # weights and result are rounded to bf16: 2^-8 of values of about 1 each
+                assert bool(((got - want).abs() <= 2.0 ** -7 * (1 + want.abs())).all())
