@@ -312,7 +312,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
     if splits > 1:
         ws = _workspace(splits * M * N * 4, a.device)
     stream = torch.cuda.current_stream().cuda_stream
-    tail = _gemm_tail(a.device, stream) if M >= 256 else (None, None)
+    tail = _gemm_tail(a.device, stream) if M >= 640 or tile else (None, None)  # (gemm8p's rows)
     rc = lib().da_gemm_bf16(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
                             M, N, K, epi, tile, splits, _ptr(ws), _ptr(gamma), float(eps), *tail, c_void_p(stream))
     _check(rc, "gemm")
