@@ -227,6 +227,179 @@ gemm_bf16_kernel(GemmArgs p) {
   }
 }
 
+// ------------------------------------------------------------------------------------------
+// Weight-streaming product (33..639 rows: decoding, short prompts): 64 x 128 tiles, four waves of 64 rows x 32 columns, for
+// up to 64 rows; 128 x 128 with eight above. K in stages of 64.
+//  * A stage (8 or 16 KB of A, 16 KB of W) arrives by LDS-DMA in a ring of 6 or 5 stages, so 80 or 64 KB of W are on
+//    their way per CU whatever the registers hold. (Staged through registers, four in flight and a ds_write each:
+//    3.6 - 4.3 TB/s.)
+//  * One workgroup per CU walks units (tile, K split) b, b + G, ...; the ring runs on across units, so the next one's
+//    weights are on their way during this one's epilogue. Past the last unit the pieces are issued against an empty
+//    resource (no traffic): the counted waits stay the same to the end.
+//  * W is the MFMA's A operand, so a lane holds 4 consecutive columns of a row and stores them without staging.
+//  * nrm: the rows of A are the raw residual stream, and the result's rows are scaled by rsqrt(sum of the parts'
+//    squares / norm_k + eps) (gemm_dk.hip).
+// Bound by HBM where tiles cover the CUs: 64 x 28672 x 4096 (235 MB, no split) 48 us (4.9 TB/s) vs 62 with two splits and
+// their reduce before; 64 x 128256 x 4096 191 (5.5 TB/s) vs 248. Above 128 rows by the stage's turn-around on one CU
+// (0.56 us; with four waves 0.7): 200 x 28672 x 4096 79 vs 99, 256 x 4096 x 14336 50 vs 62, 512 x 6144 x 4096 41 vs 53.
+struct WsNorm {
+  const float* ssq;  // [parts][64]; null: none
+  int parts, norm_k;
+  float eps;
+};
+
+template <int BM, int EPI, bool NT>
+__global__ void __launch_bounds__(BM * 4)
+gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
+  constexpr int BN = 128, A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128;
+  constexpr int WS_ST = BM == 64 ? 6 : 5;
+  constexpr int PW = 256 / BM;  // LDS-DMA instructions of a wave per stage: 2 of A, PW of W
+  typedef __attribute__((address_space(3))) void* lds_ptr_t;
+  __shared__ __attribute__((aligned(16))) char smem[WS_ST * STAGE];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 15, fg = lane >> 4;
+  const int ntm = (p.M + BM - 1) / BM, ntn = (p.N + BN - 1) / BN, units = ntm * ntn * splits;
+  const int nk = p.k_per_split / 64, G = gridDim.x;
+  const int mine = (units - (int)blockIdx.x + G - 1) / G;  // units of this workgroup (>= 1)
+
+  // unit -> (first row, first column, split); row blocks of one W tile are neighbours on one XCD
+  auto unit_of = [&](int i, int& m0, int& n0, int& sp) __attribute__((always_inline)) {
+    const int t = xcd_remap((int)blockIdx.x + i * G, units);
+    m0 = t % ntm * BM;
+    n0 = t / ntm % ntn * BN;
+    sp = t / (ntm * ntn);
+  };
+
+  // ---- the ring's writing side: stage `ik` of unit `iu` is next ----
+  __amdgpu_buffer_rsrc_t ra, rw;
+  unsigned ao[2], wo[4];  // row w * 16 + j * 8 + lane / 8 of A (w * 8 * PW + ... of W), 16-B chunk swizzled by (row >> 1) & 7
+  int iu = 0, ik = 0, slot = 0;
+  auto open = [&]() __attribute__((always_inline)) {  // resources and offsets of unit iu
+    int m0, n0, sp;
+    unit_of(iu, m0, n0, sp);
+    const int n = iu < mine ? 0x7ffffff0 : 0;
+    ra = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)((const char*)p.A + (size_t)m0 * p.lda * 2 + (size_t)sp * p.k_per_split * 2), (short)0, n, 0x00020000);
+    rw = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)((const char*)p.W + (size_t)n0 * p.K * 2 + (size_t)sp * p.k_per_split * 2), (short)0, n, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int r = w * 16 + j * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+      ao[j] = (unsigned)(min(m0 + r, p.M - 1) - m0) * (unsigned)(p.lda * 2) + c * 16;
+    }
+#pragma unroll
+    for (int j = 0; j < PW; ++j) {
+      const int r = w * 8 * PW + j * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+      wo[j] = (unsigned)(min(n0 + r, p.N - 1) - n0) * (unsigned)(p.K * 2) + c * 16;
+    }
+  };
+  auto issue = [&]() __attribute__((always_inline)) {
+    char* base = smem + slot * STAGE;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(base + (w * 2 + j) * 1024), 16, ao[j], ik * 128, 0, 0);
+#pragma unroll
+    for (int j = 0; j < PW; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t)(base + A_BYTES + (w * PW + j) * 1024), 16, wo[j], ik * 128, 0,
+                                               NT ? 2 : 0);
+    slot = slot + 1 == WS_ST ? 0 : slot + 1;
+    if (++ik == nk) {
+      ik = 0;
+      ++iu;
+      open();
+    }
+  };
+  open();
+#pragma unroll 1
+  for (int i = 0; i < WS_ST - 1; ++i) issue();
+
+  int rd = 0;  // the slot that is read next
+  const int sw = (fr >> 1) & 7;
+  for (int u = 0; u < mine; ++u) {
+    int m0, n0, sp;
+    unit_of(u, m0, n0, sp);
+    f32x4_t acc[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int kt = 0; kt < nk; ++kt) {
+      // this wave's pieces of the stage are in; after the barrier everyone's, and the slot before it has been read
+      if constexpr (BM == 64)
+        asm volatile("s_waitcnt vmcnt(24) lgkmcnt(0)" ::: "memory");  // 6 * (6 - 2)
+      else
+        asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)" ::: "memory");  // 4 * (5 - 2)
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      issue();
+      const char* sa = smem + rd * STAGE + (w >> 2) * 64 * 128;
+      const char* sb = smem + rd * STAGE + A_BYTES + (w & 3) * 32 * 128;
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        const int c = ((kk * 4 + fg) ^ sw) << 4;
+        bf16x8_t af[4], wf[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) wf[j] = *(const bf16x8_t*)(sb + (j * 16 + fr) * 128 + c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) af[i] = *(const bf16x8_t*)(sa + (i * 16 + fr) * 128 + c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = mfma16(wf[j], af[i], acc[i][j]);
+      }
+      rd = rd + 1 == WS_ST ? 0 : rd + 1;
+    }
+    // ---- row m0 (+ 64) + 16 i + fr, columns col + 16 j + 4 fg .. + 3 ----
+    const int col = n0 + (w & 3) * 32 + 4 * fg;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = m0 + (w >> 2) * 64 + i * 16 + fr;
+      if (m >= p.M) continue;
+      float inv = 1.f;
+      if (nrm.ssq) inv = rsqrtf(sum_strided(nrm.ssq + m, nrm.parts, 64) / nrm.norm_k + nrm.eps);
+      if constexpr (EPI == EPI_SWIGLU) {
+        const int oc = n0 / 2 + (w & 3) * 16 + 4 * fg;
+        if (oc >= p.N / 2) continue;
+        float v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          v[q] = gate_act(fmaf(acc[i][0][q], inv, p.bias ? bf2f(p.bias[col + q]) : 0.f), p.relu) *
+                 fmaf(acc[i][1][q], inv, p.bias ? bf2f(p.bias[col + 16 + q]) : 0.f);
+        *(u32x2_t*)(p.C + (size_t)m * p.ldc + oc) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+      } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int gn = col + 16 * j;
+          if (gn >= p.N) continue;
+          if constexpr (EPI == EPI_PARTIAL) {
+            *(f32x4_t*)(p.ws + ((size_t)sp * p.M + m) * p.N + gn) = acc[i][j];
+          } else {
+            float v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = fmaf(acc[i][j][q], inv, p.bias ? bf2f(p.bias[gn + q]) : 0.f);
+            if constexpr (EPI == EPI_GELU) {
+#pragma unroll
+              for (int q = 0; q < 4; ++q) v[q] = gelu_erf(v[q]);
+            }
+            if constexpr (EPI == EPI_RESID) {
+              const u32x2_t r = *(const u32x2_t*)(p.resid + (size_t)m * p.ldr + gn);
+#pragma unroll
+              for (int q = 0; q < 2; ++q) {
+                v[2 * q] += bf2f((bf16_t)(r[q] & 0xffff));
+                v[2 * q + 1] += bf2f((bf16_t)(r[q] >> 16));
+              }
+            }
+            *(u32x2_t*)(p.C + (size_t)m * p.ldc + gn) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+          }
+        }
+      }
+    }
+  }
+  // the pieces issued past the end write zeros into LDS: in before the workgroup (and its LDS) goes
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // Split-K reduction + epilogue. One thread per 8 output elements (16-B stores).
 // ssq_in (nullable): deferred RMSNorm of the product's rows — the A rows were the raw residual
 // stream, so by linearity out[m, :] = inv[m] * (A W^T)[m, :], inv[m] = rsqrt(sum_p ssq_in[p][m] /
@@ -476,10 +649,40 @@ static int launch_tile(const GemmArgs& a, int epi, int splits, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-// Decode tiles (64x128 / 32x128): 4 k-tiles in flight per workgroup (register prefetch depth 4;
-// 1 / 2 / 8 measured slower, profiles/decode_gemm_prefetch_sweep_r1.jsonl).
+template <int BM, bool NT>
+static int launch_ws_tile(const GemmArgs& a, int epi, int splits, const WsNorm& nrm, hipStream_t s) {
+  const long units = (long)((a.M + BM - 1) / BM) * ((a.N + 127) / 128) * splits;
+  if (units > 0x7fffffffL || a.k_per_split % 64 || a.k_per_split < 64) return (int)hipErrorInvalidValue;
+  const dim3 grid((unsigned)min(units, 256L)), block(BM * 4);
+#define WS_LAUNCH(E) gemm_ws_kernel<BM, E, NT><<<grid, block, 0, s>>>(a, nrm, splits)
+  switch (splits > 1 ? (int)EPI_PARTIAL : epi) {
+    case EPI_NONE: WS_LAUNCH(EPI_NONE); break;
+    case EPI_BIAS: WS_LAUNCH(EPI_BIAS); break;
+    case EPI_GELU: WS_LAUNCH(EPI_GELU); break;
+    case EPI_SWIGLU: WS_LAUNCH(EPI_SWIGLU); break;
+    case EPI_RESID: WS_LAUNCH(EPI_RESID); break;
+    case EPI_PARTIAL: WS_LAUNCH(EPI_PARTIAL); break;
+    default: return (int)hipErrorInvalidValue;
+  }
+#undef WS_LAUNCH
+  return (int)hipGetLastError();
+}
+
+// W is read once where there is one row block only: not worth a place in the caches then.
+static int launch_ws(const GemmArgs& a, int epi, int splits, const WsNorm& nrm, hipStream_t s) {
+  if (a.M <= 64) return launch_ws_tile<64, true>(a, epi, splits, nrm, s);
+  if (a.M <= 128) return launch_ws_tile<128, true>(a, epi, splits, nrm, s);
+  return launch_ws_tile<128, false>(a, epi, splits, nrm, s);
+}
+
+// Its offsets into a tile's rows are 32 bits wide.
+static bool ws_spans(const GemmArgs& a) { return (size_t)max(a.K, a.lda) * 256 < 0x7ffffff0ull; }
+
+// Decode tiles: the streaming kernel (64x128 / 128x128); 32x128, and 64x128 for rows too long for it, with 4 k-tiles in flight per workgroup (register prefetch depth
+// 4; 1 / 2 / 8 measured slower, profiles/decode_gemm_prefetch_sweep_r1.jsonl).
 template <int BM, int BN>
 static int launch_decode_tile(const GemmArgs& a, int epi, int splits, hipStream_t s) {
+  if (BM == 64 && ws_spans(a)) return launch_ws(a, epi, splits, WsNorm{}, s);
   return launch_tile<BM, BN, 1, 4, 4>(a, epi, splits, s);
 }
 
@@ -589,17 +792,17 @@ splitk_reduce_resid_ssq(const float* __restrict__ ws, int splits, int M, int N, 
   if (lane == 0) ssq_out[(size_t)blockIdx.x * 64 + m] = sq;
 }
 
-// gemm_dk's contract (DkArgs semantics, csrc/gemm_dk.hip) for 33..64 rows on the 64x128 split-K
+// gemm_dk's contract (DkArgs semantics, csrc/gemm_dk.hip) for 33..64 rows on the 64x128 streaming
 // tiles: epi NONE / BIAS / SWIGLU with an optional deferred norm of A's rows (ssq_in: the raw
-// residual stream as A, the row scale applied in the reduce), or EPI_RESID with optional per-part
-// sums of squares out (ssq_out: [N / 512][64]). splits >= 2 whenever a reduce is needed; ws holds
+// residual stream as A, the row scale applied in the reduce, or without splits in the epilogue), or EPI_RESID with optional per-part
+// sums of squares out (ssq_out: [N / 512][64]). splits 1: no reduce (not with ssq_out); else ws holds
 // splits * M * N floats.
 DA_EXPORT int da_gemm_dk_splitk(const void* A, int lda, const void* W, void* C, int ldc, const void* bias,
                                 const void* resid, int ldr, int M, int N, int K, int epi, const float* ssq_in,
                                 int ssq_parts, int norm_k, float eps, float* ssq_out, void* ws, int splits,
                                 void* stream) {
   hipStream_t s = (hipStream_t)stream;
-  if (M < 1 || M > 64 || K % 64 || N % 16 || lda % 8 || ldc % 8 || !ws || splits < 2 || (K / 64) % splits)
+  if (M < 1 || M > 64 || K % 64 || N % 16 || lda % 8 || ldc % 8 || (splits > 1 && !ws) || splits < 1 || (K / 64) % splits)
     return (int)hipErrorInvalidValue;
   const int relu = epi == EPI_REGLU;
   if (relu) epi = EPI_SWIGLU;
@@ -612,6 +815,11 @@ DA_EXPORT int da_gemm_dk_splitk(const void* A, int lda, const void* W, void* C, 
   a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = (bf16_t*)C;
   a.ws = (float*)ws;
   a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc; a.ldr = ldr; a.k_per_split = K / splits;
+  if (splits == 1) {  // wide products: the epilogue in the same launch
+    if (ssq_out || !ws_spans(a)) return (int)hipErrorInvalidValue;
+    a.bias = (const bf16_t*)bias; a.resid = (const bf16_t*)resid; a.relu = relu;
+    return launch_ws(a, epi, 1, WsNorm{ssq_in, ssq_parts, norm_k, eps}, s);
+  }
   const int err = launch_decode_tile<64, 128>(a, EPI_PARTIAL, splits, s);
   if (err) return err;
   if (epi == EPI_RESID && ssq_out) {
@@ -663,7 +871,7 @@ DA_EXPORT int da_gemm_rope(const void* A, int lda, const void* W, void* C, int l
 }
 
 // Tile selection: big tiles when the grid fills 256 CUs, skinny tiles (+ split-K) for decode-sized M.
-// tile: 0 = auto, 1 = 128x128, 2 = 64x128, 3 = 32x128, 4 / 7 = 256x256 phase-split (gemm8p),
+// tile: 0 = auto, 1 = 128x128, 2 = weight-streaming 64x128 / 128x128, 3 = 32x128, 4 / 7 = 256x256 phase-split (gemm8p),
 // 6 = GEMV (M = 1), 8 = 128x128 PF4, 9 = 128x64 PF4, 10 = 128x256 phase-split (gemm8p),
 // 13 = 256x256 four-wave (gemm4w).
 DA_EXPORT int da_gemm_bf16(const void* A, int lda, const void* W, void* C, int ldc,
@@ -686,9 +894,8 @@ DA_EXPORT int da_gemm_bf16(const void* A, int lda, const void* W, void* C, int l
   if (tail_ws && tail_cnt && epi != EPI_GELU) { a.tail_ws = (float*)tail_ws; a.tail_cnt = (int*)tail_cnt; }
   if ((rms_gamma || rms_eps > 0.f) && tile != 6) return (int)hipErrorInvalidValue;  // fused RMSNorm: GEMV only
   if (tile == 0) {
-    // decode-sized M: 32x128 / 64x128 weight-streaming tiles (+ split-K, chosen by the caller);
-    // 65..639 rows: the 64x128 tile over ceil(M/64) row blocks; from 640 rows the phase-split
-    // kernel with the row-tile height of fewer workgroup waves (gemm8p_pick_bm; 32-layer Phi-3
+    // decode-sized M: 32x128 / weight-streaming tiles (+ split-K, chosen by the caller), to 639 rows;
+    // from 640 rows the phase-split kernel with the row-tile height of fewer workgroup waves (gemm8p_pick_bm; 32-layer Phi-3
     // chain and single-GEMM sweeps: bench/midm_chain.py, bench/gemm_ab.py, profiles/r2, r3)
     if (M <= 32) tile = 3;
     else if (M < 640 || splits > 1) tile = 2;

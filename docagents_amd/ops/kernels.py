@@ -323,10 +323,10 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
 # workgroup and summed through LDS, no split-K partials, no reduce launch). False: the 64x128 /
 # 32x128 tiles + split-K + reduce (bench/ab_arms.py DA_DECODE_DK=0).
 DECODE_DK = True
-# 33..64 rows keep the gemm_dk layer structure (norms deferred into the consumer) on the split-K
+# 33..64 rows keep the gemm_dk layer structure (norms deferred into the consumer) on the streaming
 # tiles: the narrow dk tiles re-read the activation block once per 16-64 weight rows there
 # (bench/midm_chain.py, profiles/r3/dk/), so gemm_dk() routes those rows to da_gemm_dk_splitk
-# (reduce + residual + row sums of squares; the consumer's reduce applies the row scale)
+# (reduce + residual + row sums of squares; the consumer's reduce or epilogue applies the row scale)
 DK_MAX_M = 64
 DK_SPLITK_ABOVE = 32
 
@@ -341,13 +341,16 @@ def _dk_splitk(M: int, N: int) -> bool:
     return DK_SPLITK_ABOVE < M <= 64 and N % 512 == 0
 
 
-def _dk_splits(N: int, K: int) -> int:
+def _dk_splits(N: int, K: int, reduce: bool = False) -> int:
     """Split-K of the 33..64-row route (64x128 tiles): the largest of 2, 3, 4, 6, 8, 12, 16 that keeps
-    the grid within one round of 256 workgroups and >= 4 K-steps of 64 per split; at least 2 (the
-    reduce carries the epilogue). 3 is the point of this list: the Phi-3 QKV projection (72 tiles)
-    18.7 us at 3 splits vs 21.8 at 2 and 25.7 at 4 (bench/splitk_m64.py, profiles/r3/splitk_m64.txt)."""
+    the grid within one round of 256 workgroups and >= 4 K-steps of 64 per split. 3 is the point of this
+    list: the Phi-3 QKV projection (72 tiles) 18.7 us at 3 splits vs 21.8 at 2 and 25.7 at 4
+    (bench/splitk_m64.py, profiles/r3/splitk_m64.txt). None above 128 tiles: the streaming tile reaches
+    HBM's rate on that many CUs without, and the reduce launch goes (64 rows, N = 17920, K = 5120: 49 us
+    vs 59 at 2; 28672 x 4096: 48 vs 60; 128256 x 4096: 191 vs 232; below the line 48 rows, 16384 x 3072:
+    26.5 at 2 vs 29.6). reduce: at least 2 (row sums of squares are written there)."""
     tiles, ks = (N + 127) // 128, K // 64
-    best = 2
+    best = 2 if reduce else 1
     for s in (2, 3, 4, 6, 8, 12, 16):
         if ks % s == 0 and ks // s >= 4 and tiles * s <= 256:
             best = s
@@ -390,8 +393,9 @@ def gemm_dk(a, w, epi: int = EPI_NONE, bias=None, resid=None, out=None, norm_in=
         _req(epi == EPI_RESID and ssq_out.dtype == torch.float32 and ssq_out.is_contiguous()
              and ssq_out.numel() >= dk_parts(N, M) * 64, "bad ssq_out")
     if _dk_splitk(M, N) or (DK_SPLITK_ABOVE < M <= 64 and ssq_out is None):
-        splits = _dk_splits(N, K)
-        ws = _workspace(splits * M * N * 4, a.device)
+        # (rows too long for the unsplit tile's 32-bit offsets: the reduce carries the epilogue)
+        splits = _dk_splits(N, K, ssq_out is not None or max(K, a.stride(0)) >= 1 << 22)
+        ws = _workspace(splits * M * N * 4, a.device) if splits > 1 else None
         _check(lib().da_gemm_dk_splitk(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid),
                                        ldr, M, N, K, epi, _ptr(ssq), parts, K, float(eps), _ptr(ssq_out), _ptr(ws),
                                        splits, _stream()), "gemm_dk_splitk")
@@ -513,16 +517,15 @@ def gemm_resid_norm(a, w, resid, gamma, eps: float, out=None, h_out=None, bias=N
 
 
 def _decode_tile(M: int, N: int = 0) -> int:
-    """Decode-sized M: 32x128 tiles up to 32 rows, 64x128 to 64; 65..128 rows (a batch-128 decode
-    step): N >= 8192 (QKV, gate/up, LM head: >= 128 weight tiles) the 64x128 tile over the two row
-    blocks without split-K, else one 128x64 weight-streaming tile per 64 weight rows with split-K
-    (profiles/r5/midm/decode_gemm_sweep_m128.txt, weights cold: QKV 28.0 vs 33.5 us, gate/up 30.5 vs
-    47.4 us at 128 rows vs the 128x64 tile at split 4; O / down best on the 128x64 tile at split 4);
-    129..639 rows the 64x128 tile over ceil(M/64) row blocks."""
+    """Decode-sized M: 32x128 tiles up to 32 rows, else the weight-streaming tile (64x128 to 64 rows,
+    128x128 above; csrc/gemm.hip). 65..128 rows have it only for N >= 20480 (gate/up, LM head), where its
+    tiles cover most of the CUs: one 128x64 register-staged tile per 64 weight rows otherwise (weights
+    cold: 80 x 28672 x 4096 48.5 vs 58 us, 128 x 128256 x 4096 230 vs 255, but 100 x 12288 x 3072 29 vs
+    27 and 128 x 4096 x 4096 21 vs 18)."""
     if M <= 32:
         return 3
     if 64 < M <= 128:
-        return 2 if N >= 8192 else 9
+        return 2 if N >= 20480 else 9
     return 2
 
 
@@ -543,14 +546,17 @@ def _auto_splits(M: int, N: int, K: int) -> int:
         while s > 1 and (ksteps % s or ksteps // s < 4):
             s //= 2
         return s
+    if M > 128:
+        # rounds of the 128x128 tile (0.56 us a K-step of 64) + the reduce (a launch, and its partials out and in at
+        # 4 TB/s): 600 x 4096 x 14336 113 us at 4 splits vs 125 at 1 and 135 at 2; 256 x 4096 x 14336 50 at 4 vs 54
+        # at 8 and 78 at 2; 200 x 28672 x 4096 79 at 1 vs 96 at 2; 200 x 3072 x 8192 29 at 4 vs 32 at 8
+        tiles = math.ceil(M / 128) * math.ceil(N / 128)
+        cost = {s: math.ceil(tiles * s / 256) * (ksteps // s) * 0.56 + (4 + s * M * N * 2e-6 if s > 1 else 0)
+                for s in (1, 2, 4, 8) if ksteps % s == 0 and (s == 1 or ksteps // s >= 4)}
+        return min(cost, key=cost.get)
     tiles = math.ceil(M / (32 if _decode_tile(M) == 3 else 64)) * math.ceil(N / 128)
-    # 65..639 rows run the 64x128 tile over ceil(M/64) row blocks (the row blocks of one weight tile
-    # share it through L2): up to 4 workgroups per CU below 256 rows, 2.5 from 256 (32-layer Phi-3
-    # chain, bench/midm_chain.py, profiles/r2/midm_chain.txt: split 4 best at M = 65 / 128, 2 at 192 /
-    # 256, 1 from 384)
-    cap = 256 if M <= 64 else (1024 if M < 256 else 640)
     s = 1
-    while tiles * s * 2 <= cap and ksteps % (s * 2) == 0 and ksteps // (s * 2) >= 4:
+    while tiles * s * 2 <= 256 and ksteps % (s * 2) == 0 and ksteps // (s * 2) >= 4:
         s *= 2
     return s
 

@@ -1,0 +1,62 @@
+"""The weight-streaming 64x128 tile (33..639 rows): every epilogue, K split and ragged edge against 64-bit products."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from docagents_amd.ops import kernels as K
+
+U = 2.0 ** -8  # a bf16 rounding
+
+
+def _operands(M, N, Kd, lda=0):
+    g = torch.Generator(device="cuda").manual_seed(M * 7 + N)
+    full = torch.randn(M, lda or Kd, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(N, Kd, device="cuda", generator=g) * Kd ** -0.5).bfloat16()
+    bias = torch.randn(N, device="cuda", generator=g).bfloat16()
+    return full[:, :Kd], w, bias, g
+
+
+def _swiglu(x):
+    M, N = x.shape
+    x = x.view(M, N // 32, 2, 16)
+    return (torch.nn.functional.silu(x[:, :, 0]) * x[:, :, 1]).reshape(M, N // 2)
+
+
+# (rows, columns, K, K splits): one K step (fewer than the ring's stages), the ring's length and one more, a last row
+# and column tile that are not full, more tiles than workgroups (257 and several rounds of them), several row blocks
+@pytest.mark.parametrize("M,N,Kd,splits", [(33, 128, 64, 1), (64, 136, 64 * 6, 1), (63, 96, 64 * 7, 1), (64, 128 * 257, 128, 1),
+                                           (65, 32, 128, 2), (200, 128 * 200 + 32, 192, 1), (64, 4096, 2048, 8),
+                                           (129, 160, 64 * 12, 4), (639, 1024, 512, 1)])
+@pytest.mark.parametrize("epi", ["none", "bias", "gelu", "swiglu", "resid"])
+def test_stream_tile(M, N, Kd, splits, epi):
+    if epi == "swiglu" and N % 32:
+        N += 32 - N % 32
+    a, w, bias, g = _operands(M, N, Kd, Kd + 64)
+    code = {"none": K.EPI_NONE, "bias": K.EPI_BIAS, "gelu": K.EPI_GELU, "swiglu": K.EPI_SWIGLU, "resid": K.EPI_RESID}[epi]
+    resid = torch.randn(M, N, device="cuda", generator=g).bfloat16() if epi == "resid" else None
+    b = None if epi == "none" else bias
+    got = K.gemm(a, w, b, epi=code, resid=resid, tile=2, splits=splits).double()
+    ref = a.double() @ w.double().T + (0 if b is None else b.double())
+    ref = {"gelu": torch.nn.functional.gelu, "swiglu": _swiglu}.get(epi, lambda x: x)(ref)
+    if resid is not None:
+        ref = ref + resid.double()
+    # one rounding of the result, and fp32 sums of Kd products of size ~Kd^-1/2 (times the other gated factor: < 8)
+    tol = U * ref.abs() + 8 * Kd * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T).max()
+    assert ((got - ref).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("M,N,Kd", [(33, 128 * 128, 512), (64, 128 * 129, 512), (48, 128 * 224 + 32, 256)])
+@pytest.mark.parametrize("epi", ["none", "swiglu"])
+def test_row_norm_without_splits(M, N, Kd, epi):
+    """Wide products of 33..64 rows: the rows' scale in the epilogue (no partials), either side of the rule's line."""
+    a, w, bias, g = _operands(M, N, Kd)
+    parts = 3
+    ssq = torch.rand(parts, 64, device="cuda", generator=g) * Kd / parts * 2
+    got = K.gemm_dk(a, w, epi=K.EPI_SWIGLU if epi == "swiglu" else K.EPI_NONE, norm_in=(ssq, parts, 1e-5)).double()
+    inv = (ssq[:, :M].double().sum(0) / Kd + 1e-5).rsqrt()[:, None]
+    ref = (a.double() @ w.double().T) * inv
+    mag = ((a.double().abs() @ w.double().abs().T) * inv).max()
+    ref = _swiglu(ref) if epi == "swiglu" else ref
+    assert ((got - ref).abs() <= U * ref.abs() + 8 * Kd * 2.0 ** -24 * mag).all()
