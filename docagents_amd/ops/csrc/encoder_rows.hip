@@ -1,0 +1,230 @@
+// Encoder products for few rows (a question: <= 64 tokens), with the LayerNorms between them inside: five launches a layer.
+//
+//   C[M, N] = epi(LN(A)[M, K] . W[N, K]^T + bias)      epi: none / GELU
+//   C[M, N] = A . W^T + bias + LN(R)                   and the row statistics that the next LN needs
+//
+// A post-norm layer's LayerNorm sits between two products and its output is read twice, as the next product's operand and
+// as the residual after it. Here no launch writes it: the product that makes the sum y also writes, for each row and 16
+// columns, their mean and sum of squared deviations; its readers merge those (K / 16 pairs a row: the pairwise variance
+// formula of Chan, Golub and LeVeque, no cancellation) and normalise y as they load it, rounded to bf16 like the row that
+// the layernorm kernel stores.
+//
+// What bounds it is latency: 12 layers' 170 MB are 35 us at HBM's rate, a launch is 4 - 5. So a workgroup is a strip of
+// 16 columns (48 - 256 of them) whose up to 16 waves share K in units of 64, operands go from global memory straight to
+// the MFMA, everything that a wave needs is requested before the first wait (the statistics first: they are merged while
+// the weights are on their way), and the waves' sums meet in LDS once.
+// 32 rows of 12 layers of 768 x 3072 columns: 4.8 us (K = 768), 5.9 (a norm on A), 6.9 (and GELU) and 8.5 (K = 3072) a
+// launch, the question 485 -> 403 us; a dk product, a norm, or a split-K product with its reduce took 5.2 / 7.1, 4.6 and
+// 9.7.
+#include "gemm.h"
+
+struct EncRowsArgs {
+  const bf16_t *A, *W, *bias, *resid;
+  bf16_t* C;
+  const float* st;        // [64 rows][64 parts] (mean, squared deviations) of the rows that are normalised; null: none are
+  const bf16_t *g, *b;    // gain and shift of that norm
+  float* st_out;          // RESID: the same of the rows of C, a part per 16 columns
+  int M, N, K, lda, ldc, ldr, parts;
+  float eps;
+};
+
+// PFU: units of 64 k that a wave has in flight
+template <int FM, bool LNA, int EPI, int PFU>
+__global__ void __launch_bounds__(1024)
+enc_rows_kernel(EncRowsArgs p) {
+  constexpr int ROWS = FM * 16, SLD = 20;
+  __shared__ __attribute__((aligned(16))) float red[16][ROWS][SLD];
+  __shared__ float smean[ROWS], srstd[ROWS];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
+  const int fr = lane & 15, fg = lane >> 4;
+  const int n0 = blockIdx.x * 16, units = p.K / 64;
+  {  // this block's rows
+    const int m0 = blockIdx.y * ROWS;
+    p.M -= m0;
+    p.A += (size_t)m0 * p.lda;
+    p.C += (size_t)m0 * p.ldc;
+    if (p.resid) p.resid += (size_t)m0 * p.ldr;
+    if (p.st) p.st += m0 * 128;
+    if (p.st_out) p.st_out += m0 * 128;
+  }
+
+  // ---- requests: statistics (16 lanes a row, 4 parts each) and the epilogue's operands, then the product's ----
+  const int sl = lane & 15;
+  f32x4_t s0, s1;
+  auto stats_load = [&](int r) __attribute__((always_inline)) {
+    const f32x4_t* q = (const f32x4_t*)(p.st + (size_t)min(r, p.M - 1) * 128 + sl * 8);
+    s0 = q[0];
+    s1 = q[1];
+  };
+  auto stats_merge = [&](int r) __attribute__((always_inline)) {
+    const float mean[4] = {s0[0], s0[2], s1[0], s1[2]}, dev[4] = {s0[1], s0[3], s1[1], s1[3]};
+    float a = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) a += sl * 4 + e < p.parts ? mean[e] : 0.f;
+#pragma unroll
+    for (int x = 8; x; x >>= 1) a += __shfl_xor(a, x, 64);
+    const float m = a / p.parts;
+    float v = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v += sl * 4 + e < p.parts ? fmaf(16.f * (mean[e] - m), mean[e] - m, dev[e]) : 0.f;
+#pragma unroll
+    for (int x = 8; x; x >>= 1) v += __shfl_xor(v, x, 64);
+    if (sl == 0 && r < ROWS) {
+      smean[r] = m;
+      srstd[r] = rsqrtf(v / (16 * p.parts) + p.eps);
+    }
+  };
+  if (p.st) stats_load(4 * w + fg);
+  const int om = tid >> 2, oc = n0 + 4 * (tid & 3);  // the output row and columns of this thread (tid < 4 * ROWS)
+  const bool out = om < p.M && tid < 4 * ROWS;
+  u32x2_t ob{0, 0}, orr{0, 0}, og{0, 0}, obb{0, 0};
+  if (out) {
+    if (p.bias) ob = *(const u32x2_t*)(p.bias + oc);
+    if constexpr (EPI == EPI_RESID) {
+      orr = *(const u32x2_t*)(p.resid + (size_t)om * p.ldr + oc);
+      if (p.st && FM < 4) {
+        og = *(const u32x2_t*)(p.g + oc);
+        obb = *(const u32x2_t*)(p.b + oc);
+      }
+    }
+  }
+  asm volatile("" ::: "memory");
+  bf16x8_t wf[PFU][2], af[PFU][2][FM], gf[2], bf[2];
+  auto load = [&](int u0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < PFU; ++j) {
+      const int k = min(u0 + nw * j, units - 1) * 64 + fg * 8;  // (past the end: the last unit again, not used)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) wf[j][h] = *(const bf16x8_t*)(p.W + (size_t)(n0 + fr) * p.K + k + 32 * h);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+          af[j][h][i] = *(const bf16x8_t*)(p.A + (size_t)min(16 * i + fr, p.M - 1) * p.lda + k + 32 * h);
+      if constexpr (LNA) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          gf[h] = *(const bf16x8_t*)(p.g + k + 32 * h);
+          bf[h] = *(const bf16x8_t*)(p.b + k + 32 * h);
+        }
+      }
+    }
+  };
+  load(w);
+  if (p.st) {
+    asm volatile("" ::: "memory");
+    stats_merge(4 * w + fg);
+    for (int r = 4 * (w + nw) + fg; r - fg < ROWS; r += 4 * nw) {
+      stats_load(r);
+      stats_merge(r);
+    }
+    __syncthreads();
+  }
+  f32x4_t acc[FM];
+#pragma unroll
+  for (int i = 0; i < FM; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int u0 = w;;) {
+#pragma unroll
+    for (int j = 0; j < PFU; ++j) {
+      if (u0 + nw * j >= units) continue;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+          bf16x8_t a = af[j][h][i];
+          if constexpr (LNA) {
+            const float mean = smean[16 * i + fr], rstd = srstd[16 * i + fr];
+            u32x4_t y;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              y[e] = pack_bf2(fmaf((bf2f((bf16_t)a[2 * e]) - mean) * rstd, bf2f((bf16_t)gf[h][2 * e]), bf2f((bf16_t)bf[h][2 * e])),
+                              fmaf((bf2f((bf16_t)a[2 * e + 1]) - mean) * rstd, bf2f((bf16_t)gf[h][2 * e + 1]),
+                                   bf2f((bf16_t)bf[h][2 * e + 1])));
+            a = __builtin_bit_cast(bf16x8_t, y);
+          }
+          acc[i] = mfma16(wf[j][h], a, acc[i]);  // (W first: a lane has 4 columns of a row)
+        }
+    }
+    u0 += nw * PFU;
+    if (u0 >= units) break;
+    load(u0);
+  }
+#pragma unroll
+  for (int i = 0; i < FM; ++i) *(f32x4_t*)&red[w][16 * i + fr][4 * fg] = acc[i];
+  __syncthreads();
+  if (tid >= 4 * ROWS) return;  // (whole waves)
+  if (EPI == EPI_RESID && FM == 4 && out && p.st) {  // (no registers for them before)
+    og = *(const u32x2_t*)(p.g + oc);
+    obb = *(const u32x2_t*)(p.b + oc);
+  }
+  f32x4_t v = *(const f32x4_t*)&red[0][om][4 * (tid & 3)];
+  for (int x = 1; x < nw; ++x) v += *(const f32x4_t*)&red[x][om][4 * (tid & 3)];
+  float y[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    auto half = [&](const u32x2_t& q) { return bf2f((bf16_t)(e & 1 ? q[e >> 1] >> 16 : q[e >> 1] & 0xffff)); };
+    y[e] = v[e] + half(ob);
+    if constexpr (EPI == EPI_GELU) y[e] = gelu_erf(y[e]);
+    if constexpr (EPI == EPI_RESID) {
+      float r = half(orr);
+      if (p.st) r = bf2f(f2bf(fmaf((r - smean[om]) * srstd[om], half(og), half(obb))));
+      y[e] += r;
+    }
+  }
+  const u32x2_t o{pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3])};
+  if (out) *(u32x2_t*)(p.C + (size_t)om * p.ldc + oc) = o;
+  if constexpr (EPI == EPI_RESID) {  // of the values as stored
+    float q[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q[e] = bf2f((bf16_t)(e & 1 ? o[e >> 1] >> 16 : o[e >> 1] & 0xffff));
+    float s = (q[0] + q[1]) + (q[2] + q[3]);
+    s += __shfl_xor(s, 1, 64);
+    s += __shfl_xor(s, 2, 64);
+    const float m = s * (1.f / 16.f);
+    float d = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) d = fmaf(q[e] - m, q[e] - m, d);
+    d += __shfl_xor(d, 1, 64);
+    d += __shfl_xor(d, 2, 64);
+    if (out && (tid & 3) == 0) *(float2*)(p.st_out + (size_t)om * 128 + blockIdx.x * 2) = float2{m, d};
+  }
+}
+
+template <int FM>
+static int enc_rows_launch(const EncRowsArgs& a, int epi, hipStream_t s) {
+  // as many waves as share the units of 64 k evenly, up to 16; at least FM (4 threads an output row)
+  const int units = a.K / 64, per = (units + 15) / 16;
+  const dim3 grid(a.N / 16, (a.M + FM * 16 - 1) / (FM * 16)), block(max((units + per - 1) / per, FM) * 64);
+#define ENC_ROWS(LNA, E, PFU) enc_rows_kernel<FM, LNA, E, PFU><<<grid, block, 0, s>>>(a)
+  if (epi == EPI_RESID) {  // (a unit past the end costs what one within it does)
+    if (per == 1) ENC_ROWS(false, EPI_RESID, 1);
+    else if (per == 2 || FM == 4 || (FM == 2 && per != 3)) ENC_ROWS(false, EPI_RESID, 2);
+    else if (per == 3) ENC_ROWS(false, EPI_RESID, FM == 4 ? 2 : 3);
+    else ENC_ROWS(false, EPI_RESID, FM == 1 ? 4 : 2);
+  }
+  else if (epi == EPI_GELU && a.st) ENC_ROWS(true, EPI_GELU, 1);
+  else if (epi == EPI_BIAS && a.st) ENC_ROWS(true, EPI_BIAS, 1);
+  else if (epi == EPI_BIAS) ENC_ROWS(false, EPI_BIAS, 1);
+  else return (int)hipErrorInvalidValue;
+#undef ENC_ROWS
+  return (int)hipGetLastError();
+}
+
+// epi BIAS / GELU (st: the norm of A's rows, over K columns; GELU only with it) / RESID (st: the norm of resid's rows,
+// over N columns; st_out is written). 1 <= M <= 64, K % 64 == 0, N % 16 == 0, a normed width of at most 1024.
+DA_EXPORT int da_enc_rows(const void* A, int lda, const void* W, void* C, int ldc, const void* bias, const void* resid,
+                         int ldr, int M, int N, int K, int epi, const float* st, const void* g, const void* b, float eps,
+                         float* st_out, void* stream) {
+  const int width = epi == EPI_RESID ? N : K;
+  if (M < 1 || M > 64 || K < 64 || K % 64 || N < 16 || N % 16 || lda % 8 || ldc % 4 || (st && (!g || !b || width > 1024 || width % 16)))
+    return (int)hipErrorInvalidValue;
+  if (epi == EPI_RESID && (!resid || ldr % 4 || !st_out || N > 1024)) return (int)hipErrorInvalidValue;
+  EncRowsArgs a{(const bf16_t*)A, (const bf16_t*)W, (const bf16_t*)bias, (const bf16_t*)resid, (bf16_t*)C, st,
+                (const bf16_t*)g, (const bf16_t*)b, st_out, M, N, K, lda, ldc, ldr, width / 16, eps};
+  hipStream_t s = (hipStream_t)stream;
+  // the smallest row blocks whose workgroups still fit the CUs in one round: a CU's share of A is what it waits for
+  // (K = 3072, 32 rows: 8.5 us in two blocks, 10.9 in one; 144 and 192 strips in two blocks 6.6 and 7.3 vs 5.9 and 6.9)
+  const int strips = N / 16, blocks = (M + 15) / 16;
+  if (strips * blocks <= 256) return enc_rows_launch<1>(a, epi, s);
+  return M <= 32 || strips * ((blocks + 1) / 2) <= 256 ? enc_rows_launch<2>(a, epi, s) : enc_rows_launch<4>(a, epi, s);
+}

@@ -60,6 +60,8 @@ _SIGS = {
     "da_gemm_dk": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                    c_int, c_void_p, c_int, c_int, c_float, c_void_p, c_void_p],
     "da_gemm_dk_parts": [c_int],
+    "da_enc_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5
+                  + [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p],
     "da_gemm_dk_splitk": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                           c_int, c_void_p, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_void_p],
     "da_decode_attn": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
@@ -402,6 +404,37 @@ def gemm_dk(a, w, epi: int = EPI_NONE, bias=None, resid=None, out=None, norm_in=
         return out
     _check(lib().da_gemm_dk(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
                             M, N, K, epi, _ptr(ssq), parts, K, float(eps), _ptr(ssq_out), _stream()), "gemm_dk")
+    return out
+
+
+def gemm_ln_fit(M: int, hidden: int, ffn: int) -> bool:
+    """Whether an encoder layer's products take ``gemm_ln`` (csrc/encoder_rows.hip)."""
+    return 1 <= M <= 64 and hidden % 64 == 0 and ffn % 64 == 0 and hidden <= 1024
+
+
+def gemm_ln(a, w, bias, epi: int = EPI_BIAS, norm=None, resid=None, st_out=None):
+    """Products of up to 64 rows between LayerNorms. norm = (st, g, b, eps): the rows of ``a`` (EPI_BIAS, EPI_GELU) or
+    of ``resid`` (EPI_RESID) are sums whose LayerNorm is taken here, by the statistics st (fp32 [64, 64, 2]) that the
+    EPI_RESID product which made them wrote as its ``st_out``."""
+    _bf16_cuda(a, "a"); _bf16_cuda(w, "w"); _bf16_cuda(bias, "bias")
+    M, K = a.shape
+    N = w.shape[0]
+    _req(gemm_ln_fit(M, K if epi != EPI_RESID else N, N if epi != EPI_RESID else K) and w.shape[1] == K
+         and bias.shape == (N,), f"gemm_ln shape M={M} N={N} K={K}")
+    _req(a.stride(1) == 1 and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.is_contiguous()
+         and w.data_ptr() % 16 == 0, "gemm_ln layout")
+    _req(epi == EPI_BIAS or (epi == EPI_GELU and norm is not None) or (epi == EPI_RESID and st_out is not None),
+         "gemm_ln epilogue")
+    st, g, b, eps = norm or (None, None, None, 0.0)
+    for t in (st, st_out):
+        _req(t is None or (t.dtype == torch.float32 and t.shape == (64, 64, 2) and t.is_contiguous()), "bad statistics")
+    if epi == EPI_RESID:
+        _bf16_cuda(resid, "resid")
+        _req(resid.shape == (M, N) and resid.stride(1) == 1 and resid.stride(0) % 8 == 0, "bad resid")
+    out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
+    _check(lib().da_enc_rows(_ptr(a), a.stride(0), _ptr(w), _ptr(out), N, _ptr(bias), _ptr(resid),
+                            0 if resid is None else resid.stride(0), M, N, K, epi, _ptr(st), _ptr(g), _ptr(b), float(eps),
+                            _ptr(st_out), _stream()), "gemm_ln")
     return out
 
 

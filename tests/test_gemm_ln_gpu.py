@@ -1,0 +1,50 @@
+"""Encoder products of up to 64 rows with the LayerNorms inside, against 64-bit arithmetic at the edges of their ranges."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from docagents_amd.ops import kernels as K
+
+U = 2.0 ** -8  # a bf16 rounding
+
+
+# (rows, hidden, ffn): each row tile's edges; one unit of K a wave, fewer units than waves that store, two groups of units
+@pytest.mark.parametrize("M,h,f", [(1, 768, 3072), (16, 128, 256), (17, 384, 1536), (32, 1024, 4096), (33, 768, 3072),
+                                   (64, 64, 64), (64, 1024, 4096), (20, 960, 64 * 33)])
+def test_gemm_ln(M, h, f):
+    g = torch.Generator(device="cuda").manual_seed(M + h)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    a, resid = r(M, h).bfloat16(), (3 * r(M, h) + 40).bfloat16()  # a mean far from zero: no cancellation allowed
+    wo, w1, w2, wq = (r(h, h) * h ** -0.5).bfloat16(), (r(f, h) * h ** -0.5).bfloat16(), (r(h, f) * f ** -0.5).bfloat16(), \
+        (r(3 * h, h) * h ** -0.5).bfloat16()
+    bo, b1, bq, lg, lb = (r(n).bfloat16() for n in (h, f, 3 * h, h, h))
+    st, st2 = torch.full((2, 64, 64, 2), float("nan"), device="cuda")  # (what a part does not write is not read)
+    d = lambda t: t.double()  # noqa: E731
+
+    def close(got, ref, a_, w_, slack=0.0):
+        # one rounding of the result, fp32 sums (with a margin), and what the operands' own roundings allow
+        tol = U * ref.abs() + 8 * w_.shape[1] * 2.0 ** -24 * (d(a_).abs() @ d(w_).abs().T).max() + slack
+        assert ((d(got) - ref).abs() <= tol).all(), float(((d(got) - ref).abs() / tol).max())
+
+    y = K.gemm_ln(a, wo, bo, K.EPI_RESID, resid=resid, st_out=st)
+    close(y, d(a) @ d(wo).T + d(bo) + d(resid), a, wo)
+    n = torch.nn.functional.layer_norm(d(y), (h,), d(lg), d(lb), 1e-12)
+    norm = (st, lg, lb, 1e-12)
+    nb = n.bfloat16()  # differs from the kernel's by an ulp where fp32 rounds the other way: an operand's rounding each
+    def flips(w):
+        return (U * nb.double().abs()).square() @ d(w).square().T  # (their sum's variance, if all of them did)
+    z = K.gemm_ln(y, wq, bq, norm=norm)
+    close(z, d(nb) @ d(wq).T + d(bq), nb, wq, flips(wq).sqrt())
+    u = d(nb) @ d(w1).T + d(b1)
+    x = K.gemm_ln(y, w1, b1, K.EPI_GELU, norm=norm)
+    close(x, torch.nn.functional.gelu(u), nb, w1, 1.2 * flips(w1).sqrt())
+    x2 = K.gemm_ln(x, w2, bo, K.EPI_RESID, norm=norm, resid=y, st_out=st2)
+    close(x2, d(x) @ d(w2).T + d(bo) + d(nb), x, w2, U * n.abs())
+    # the statistics: each part's own, of the stored values
+    parts = d(x2).view(M, h // 16, 16)
+    mean = parts.mean(-1)
+    assert torch.allclose(d(st2[:M, :h // 16, 0]), mean, rtol=0, atol=2.0 ** -22 * float(parts.abs().max()))
+    dev = (parts - mean[..., None]).square().sum(-1)
+    assert torch.allclose(d(st2[:M, :h // 16, 1]), dev, rtol=1e-5, atol=1e-5 * float(dev.max()))
