@@ -132,7 +132,7 @@ class BertEncoder:
         if q8:
             x, *xq = x
         elif o.gemm_ln_fit(x.shape[0], h, c.ffn):
-            return self._layers_few_rows(x, cu_seqlens, max_seqlen)
+            return self._layers_few_rows(x, cu_seqlens, max_seqlen, o.flash_attn_varlen, o.layernorm)
         for L in w["layers"]:
             qkv = self._linear(x, L, "wqkv", L["bqkv"], EPI_BIAS, xq=xq)
             a = o.flash_attn_varlen(qkv[:, :h], qkv[:, h:2 * h], qkv[:, 2 * h:], cu_seqlens, max_seqlen, nh, nh, hd,
@@ -148,7 +148,7 @@ class BertEncoder:
                 x, *xq = x
         return x
 
-    def _layers_few_rows(self, x, cu_seqlens, max_seqlen):
+    def _layers_few_rows(self, x, cu_seqlens, max_seqlen, attn, layernorm):
         """The layers of a short text: the LayerNorms ride in the products around them, and between layers the residual
         is the sum y that the next norm reads, with its row statistics (only the last norm is a launch)."""
         c, o = self.cfg, self.ops
@@ -157,20 +157,21 @@ class BertEncoder:
         norm = None
         for L in self.w["layers"]:
             qkv = o.gemm_ln(x, L["wqkv"], L["bqkv"], norm=norm)
-            a = o.flash_attn_varlen(qkv[:, :h], qkv[:, h:2 * h], qkv[:, 2 * h:], cu_seqlens, max_seqlen, nh, nh, hd,
-                                    causal=False)
+            a = attn(qkv[:, :h], qkv[:, h:2 * h], qkv[:, 2 * h:], cu_seqlens, max_seqlen, nh, nh, hd, causal=False)
             y = o.gemm_ln(a, L["wo"], L["bo"], EPI_RESID, norm=norm, resid=x, st_out=st1)
             norm = (st1, L["ln1_g"], L["ln1_b"], c.eps)
             f = o.gemm_ln(y, L["w1"], L["b1"], EPI_GELU, norm=norm)
             x = o.gemm_ln(f, L["w2"], L["b2"], EPI_RESID, norm=norm, resid=y, st_out=st2)
             norm = (st2, L["ln2_g"], L["ln2_b"], c.eps)
-        return x if norm is None else o.layernorm(x, *norm[1:])
+        return x if norm is None else layernorm(x, *norm[1:])
 
     def _forward_f16(self, ids, positions, cu_seqlens, max_seqlen):
         c, o, w = self.cfg, self.ops, self.w
         h, nh, hd = c.hidden, c.heads, c.head_dim
         x = o.bert_embed_ln_f16(ids, positions, None, w["word"], w["pos"], w["type"], w["emb_ln_g"], w["emb_ln_b"],
                                 c.eps)
+        if o.gemm_ln_fit(x.shape[0], h, c.ffn):
+            return self._layers_few_rows(x, cu_seqlens, max_seqlen, o.flash_attn_f16, o.layernorm_f16)
         for L in w["layers"]:
             qkv = o.gemm_f16(x, L["wqkv"], bias=L["bqkv"], epi=EPI_BIAS)
             a = o.flash_attn_f16(qkv[:, :h], qkv[:, h:2 * h], qkv[:, 2 * h:], cu_seqlens, max_seqlen, nh, nh, hd)

@@ -29,7 +29,7 @@ struct EncRowsArgs {
 };
 
 // PFU: units of 64 k that a wave has in flight
-template <int FM, bool LNA, int EPI, int PFU>
+template <typename T, int FM, bool LNA, int EPI, int PFU>
 __global__ void __launch_bounds__(1024)
 enc_rows_kernel(EncRowsArgs p) {
   constexpr int ROWS = FM * 16, SLD = 20;
@@ -137,12 +137,12 @@ enc_rows_kernel(EncRowsArgs p) {
             u32x4_t y;
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-              y[e] = pack_bf2(fmaf((bf2f((bf16_t)a[2 * e]) - mean) * rstd, bf2f((bf16_t)gf[h][2 * e]), bf2f((bf16_t)bf[h][2 * e])),
-                              fmaf((bf2f((bf16_t)a[2 * e + 1]) - mean) * rstd, bf2f((bf16_t)gf[h][2 * e + 1]),
-                                   bf2f((bf16_t)bf[h][2 * e + 1])));
+              y[e] = T::pack2(fmaf((T::to_f((bf16_t)a[2 * e]) - mean) * rstd, T::to_f((bf16_t)gf[h][2 * e]), T::to_f((bf16_t)bf[h][2 * e])),
+                              fmaf((T::to_f((bf16_t)a[2 * e + 1]) - mean) * rstd, T::to_f((bf16_t)gf[h][2 * e + 1]),
+                                   T::to_f((bf16_t)bf[h][2 * e + 1])));
             a = __builtin_bit_cast(bf16x8_t, y);
           }
-          acc[i] = mfma16(wf[j][h], a, acc[i]);  // (W first: a lane has 4 columns of a row)
+          acc[i] = T::mma16(wf[j][h], a, acc[i]);  // (W first: a lane has 4 columns of a row)
         }
     }
     u0 += nw * PFU;
@@ -162,21 +162,21 @@ enc_rows_kernel(EncRowsArgs p) {
   float y[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    auto half = [&](const u32x2_t& q) { return bf2f((bf16_t)(e & 1 ? q[e >> 1] >> 16 : q[e >> 1] & 0xffff)); };
+    auto half = [&](const u32x2_t& q) { return T::to_f((bf16_t)(e & 1 ? q[e >> 1] >> 16 : q[e >> 1] & 0xffff)); };
     y[e] = v[e] + half(ob);
     if constexpr (EPI == EPI_GELU) y[e] = gelu_erf(y[e]);
     if constexpr (EPI == EPI_RESID) {
       float r = half(orr);
-      if (p.st) r = bf2f(f2bf(fmaf((r - smean[om]) * srstd[om], half(og), half(obb))));
+      if (p.st) r = T::to_f(T::from_f(fmaf((r - smean[om]) * srstd[om], half(og), half(obb))));
       y[e] += r;
     }
   }
-  const u32x2_t o{pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3])};
+  const u32x2_t o{T::pack2(y[0], y[1]), T::pack2(y[2], y[3])};
   if (out) *(u32x2_t*)(p.C + (size_t)om * p.ldc + oc) = o;
   if constexpr (EPI == EPI_RESID) {  // of the values as stored
     float q[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) q[e] = bf2f((bf16_t)(e & 1 ? o[e >> 1] >> 16 : o[e >> 1] & 0xffff));
+    for (int e = 0; e < 4; ++e) q[e] = T::to_f((bf16_t)(e & 1 ? o[e >> 1] >> 16 : o[e >> 1] & 0xffff));
     float s = (q[0] + q[1]) + (q[2] + q[3]);
     s += __shfl_xor(s, 1, 64);
     s += __shfl_xor(s, 2, 64);
@@ -190,12 +190,12 @@ enc_rows_kernel(EncRowsArgs p) {
   }
 }
 
-template <int FM>
+template <typename T, int FM>
 static int enc_rows_launch(const EncRowsArgs& a, int epi, hipStream_t s) {
   // as many waves as share the units of 64 k evenly, up to 16; at least FM (4 threads an output row)
   const int units = a.K / 64, per = (units + 15) / 16;
   const dim3 grid(a.N / 16, (a.M + FM * 16 - 1) / (FM * 16)), block(max((units + per - 1) / per, FM) * 64);
-#define ENC_ROWS(LNA, E, PFU) enc_rows_kernel<FM, LNA, E, PFU><<<grid, block, 0, s>>>(a)
+#define ENC_ROWS(LNA, E, PFU) enc_rows_kernel<T, FM, LNA, E, PFU><<<grid, block, 0, s>>>(a)
   if (epi == EPI_RESID) {  // (a unit past the end costs what one within it does)
     if (per == 1) ENC_ROWS(false, EPI_RESID, 1);
     else if (per == 2 || FM == 4 || (FM == 2 && per != 3)) ENC_ROWS(false, EPI_RESID, 2);
@@ -210,11 +210,20 @@ static int enc_rows_launch(const EncRowsArgs& a, int epi, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
+template <typename T>
+static int enc_rows_rows(const EncRowsArgs& a, int epi, hipStream_t s) {
+  // the smallest row blocks whose workgroups still fit the CUs in one round: a CU's share of A is what it waits for
+  // (K = 3072, 32 rows: 8.5 us in two blocks, 10.9 in one; 144 and 192 strips in two blocks 6.6 and 7.3 vs 5.9 and 6.9)
+  const int strips = a.N / 16, blocks = (a.M + 15) / 16;
+  if (strips * blocks <= 256) return enc_rows_launch<T, 1>(a, epi, s);
+  return a.M <= 32 || strips * ((blocks + 1) / 2) <= 256 ? enc_rows_launch<T, 2>(a, epi, s) : enc_rows_launch<T, 4>(a, epi, s);
+}
+
 // epi BIAS / GELU (st: the norm of A's rows, over K columns; GELU only with it) / RESID (st: the norm of resid's rows,
-// over N columns; st_out is written). 1 <= M <= 64, K % 64 == 0, N % 16 == 0, a normed width of at most 1024.
+// over N columns; st_out is written). 1 <= M <= 64, K % 64 == 0, N % 16 == 0, a normed width of at most 1024; bf16 or fp16 throughout.
 DA_EXPORT int da_enc_rows(const void* A, int lda, const void* W, void* C, int ldc, const void* bias, const void* resid,
                          int ldr, int M, int N, int K, int epi, const float* st, const void* g, const void* b, float eps,
-                         float* st_out, void* stream) {
+                         float* st_out, int f16, void* stream) {
   const int width = epi == EPI_RESID ? N : K;
   if (M < 1 || M > 64 || K < 64 || K % 64 || N < 16 || N % 16 || lda % 8 || ldc % 4 || (st && (!g || !b || width > 1024 || width % 16)))
     return (int)hipErrorInvalidValue;
@@ -222,9 +231,5 @@ DA_EXPORT int da_enc_rows(const void* A, int lda, const void* W, void* C, int ld
   EncRowsArgs a{(const bf16_t*)A, (const bf16_t*)W, (const bf16_t*)bias, (const bf16_t*)resid, (bf16_t*)C, st,
                 (const bf16_t*)g, (const bf16_t*)b, st_out, M, N, K, lda, ldc, ldr, width / 16, eps};
   hipStream_t s = (hipStream_t)stream;
-  // the smallest row blocks whose workgroups still fit the CUs in one round: a CU's share of A is what it waits for
-  // (K = 3072, 32 rows: 8.5 us in two blocks, 10.9 in one; 144 and 192 strips in two blocks 6.6 and 7.3 vs 5.9 and 6.9)
-  const int strips = N / 16, blocks = (M + 15) / 16;
-  if (strips * blocks <= 256) return enc_rows_launch<1>(a, epi, s);
-  return M <= 32 || strips * ((blocks + 1) / 2) <= 256 ? enc_rows_launch<2>(a, epi, s) : enc_rows_launch<4>(a, epi, s);
+  return f16 ? enc_rows_rows<F16T>(a, epi, s) : enc_rows_rows<BF16T>(a, epi, s);
 }

@@ -61,7 +61,7 @@ _SIGS = {
                    c_int, c_void_p, c_int, c_int, c_float, c_void_p, c_void_p],
     "da_gemm_dk_parts": [c_int],
     "da_enc_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5
-                  + [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p],
+                  + [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_void_p],
     "da_gemm_dk_splitk": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                           c_int, c_void_p, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_void_p],
     "da_decode_attn": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
@@ -413,10 +413,12 @@ def gemm_ln_fit(M: int, hidden: int, ffn: int) -> bool:
 
 
 def gemm_ln(a, w, bias, epi: int = EPI_BIAS, norm=None, resid=None, st_out=None):
-    """Products of up to 64 rows between LayerNorms. norm = (st, g, b, eps): the rows of ``a`` (EPI_BIAS, EPI_GELU) or
+    """bf16 or fp16 products of up to 64 rows between LayerNorms. norm = (st, g, b, eps): the rows of ``a`` (EPI_BIAS, EPI_GELU) or
     of ``resid`` (EPI_RESID) are sums whose LayerNorm is taken here, by the statistics st (fp32 [64, 64, 2]) that the
     EPI_RESID product which made them wrote as its ``st_out``."""
-    _bf16_cuda(a, "a"); _bf16_cuda(w, "w"); _bf16_cuda(bias, "bias")
+    f16 = a.dtype == torch.float16
+    is_cuda = _f16_cuda if f16 else _bf16_cuda
+    is_cuda(a, "a"); is_cuda(w, "w"); is_cuda(bias, "bias")
     M, K = a.shape
     N = w.shape[0]
     _req(gemm_ln_fit(M, K if epi != EPI_RESID else N, N if epi != EPI_RESID else K) and w.shape[1] == K
@@ -429,12 +431,12 @@ def gemm_ln(a, w, bias, epi: int = EPI_BIAS, norm=None, resid=None, st_out=None)
     for t in (st, st_out):
         _req(t is None or (t.dtype == torch.float32 and t.shape == (64, 64, 2) and t.is_contiguous()), "bad statistics")
     if epi == EPI_RESID:
-        _bf16_cuda(resid, "resid")
+        is_cuda(resid, "resid")
         _req(resid.shape == (M, N) and resid.stride(1) == 1 and resid.stride(0) % 8 == 0, "bad resid")
-    out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
+    out = torch.empty((M, N), dtype=a.dtype, device=a.device)
     _check(lib().da_enc_rows(_ptr(a), a.stride(0), _ptr(w), _ptr(out), N, _ptr(bias), _ptr(resid),
                             0 if resid is None else resid.stride(0), M, N, K, epi, _ptr(st), _ptr(g), _ptr(b), float(eps),
-                            _ptr(st_out), _stream()), "gemm_ln")
+                            _ptr(st_out), f16, _stream()), "gemm_ln")
     return out
 
 

@@ -7,19 +7,18 @@ pytestmark = pytest.mark.gpu
 if torch.cuda.is_available():
     from docagents_amd.ops import kernels as K
 
-U = 2.0 ** -8  # a bf16 rounding
-
-
 # (rows, hidden, ffn): each row tile's edges; one unit of K a wave, fewer units than waves that store, two groups of units
 @pytest.mark.parametrize("M,h,f", [(1, 768, 3072), (16, 128, 256), (17, 384, 1536), (32, 1024, 4096), (33, 768, 3072),
                                    (64, 64, 64), (64, 1024, 4096), (20, 960, 64 * 33)])
-def test_gemm_ln(M, h, f):
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_gemm_ln(M, h, f, dt):
+    U = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11  # a rounding of the type
     g = torch.Generator(device="cuda").manual_seed(M + h)
     r = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
-    a, resid = r(M, h).bfloat16(), (3 * r(M, h) + 40).bfloat16()  # a mean far from zero: no cancellation allowed
-    wo, w1, w2, wq = (r(h, h) * h ** -0.5).bfloat16(), (r(f, h) * h ** -0.5).bfloat16(), (r(h, f) * f ** -0.5).bfloat16(), \
-        (r(3 * h, h) * h ** -0.5).bfloat16()
-    bo, b1, bq, lg, lb = (r(n).bfloat16() for n in (h, f, 3 * h, h, h))
+    a, resid = r(M, h).to(dt), (3 * r(M, h) + 40).to(dt)  # a mean far from zero: no cancellation allowed
+    wo, w1, w2, wq = (r(h, h) * h ** -0.5).to(dt), (r(f, h) * h ** -0.5).to(dt), (r(h, f) * f ** -0.5).to(dt), \
+        (r(3 * h, h) * h ** -0.5).to(dt)
+    bo, b1, bq, lg, lb = (r(n).to(dt) for n in (h, f, 3 * h, h, h))
     st, st2 = torch.full((2, 64, 64, 2), float("nan"), device="cuda")  # (what a part does not write is not read)
     d = lambda t: t.double()  # noqa: E731
 
@@ -32,7 +31,7 @@ def test_gemm_ln(M, h, f):
     close(y, d(a) @ d(wo).T + d(bo) + d(resid), a, wo)
     n = torch.nn.functional.layer_norm(d(y), (h,), d(lg), d(lb), 1e-12)
     norm = (st, lg, lb, 1e-12)
-    nb = n.bfloat16()  # differs from the kernel's by an ulp where fp32 rounds the other way: an operand's rounding each
+    nb = n.to(dt)  # differs from the kernel's by an ulp where fp32 rounds the other way: an operand's rounding each
     def flips(w):
         return (U * nb.double().abs()).square() @ d(w).square().T  # (their sum's variance, if all of them did)
     z = K.gemm_ln(y, wq, bq, norm=norm)
