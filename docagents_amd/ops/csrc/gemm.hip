@@ -229,9 +229,10 @@ gemm_bf16_kernel(GemmArgs p) {
 
 // ------------------------------------------------------------------------------------------
 // Weight-streaming product (33..639 rows: decoding, short prompts): 64 x 128 tiles, four waves of 64 rows x 32 columns, for
-// up to 64 rows; 128 x 128 with eight above. K in stages of 64.
-//  * A stage (8 or 16 KB of A, 16 KB of W) arrives by LDS-DMA in a ring of 6 or 5 stages, so 80 or 64 KB of W are on
-//    their way per CU whatever the registers hold. (Staged through registers, four in flight and a ds_write each:
+// up to 64 rows; 64 x 64 (32 x 32 a wave) where only those fill the CUs without splits; 128 x 128 with eight waves above 64
+// rows. K in stages of 64.
+//  * A stage (8 or 16 KB of A, 8 or 16 KB of W) arrives by LDS-DMA in a ring of 5, 6 or 10 stages, so 64 - 80 KB of W are
+//    on their way per CU whatever the registers hold. (Staged through registers, four in flight and a ds_write each:
 //    3.6 - 4.3 TB/s.)
 //  * One workgroup per CU walks units (tile, K split) b, b + G, ...; the ring runs on across units, so the next one's
 //    weights are on their way during this one's epilogue. Past the last unit the pieces are issued against an empty
@@ -240,7 +241,8 @@ gemm_bf16_kernel(GemmArgs p) {
 //  * nrm: the rows of A are the raw residual stream, and the result's rows are scaled by rsqrt(sum of the parts'
 //    squares / norm_k + eps) (gemm_dk.hip).
 // Bound by HBM where tiles cover the CUs: 64 x 28672 x 4096 (235 MB, no split) 48 us (4.9 TB/s) vs 62 with two splits and
-// their reduce before; 64 x 128256 x 4096 191 (5.5 TB/s) vs 248. Above 128 rows by the stage's turn-around on one CU
+// their reduce before; 64 x 128256 x 4096 191 (5.5 TB/s) vs 248;
+// 64 x 12672 x 4096 29 in 64 x 64 tiles, 33 in two splits of 64 x 128. Above 128 rows by the stage's turn-around on one CU
 // (0.56 us; with four waves 0.7): 200 x 28672 x 4096 79 vs 99, 256 x 4096 x 14336 50 vs 62, 512 x 6144 x 4096 41 vs 53.
 struct WsNorm {
   const float* ssq;  // [parts][64]; null: none
@@ -248,12 +250,14 @@ struct WsNorm {
   float eps;
 };
 
-template <int BM, int EPI, bool NT>
+template <int BM, int BN, int EPI, bool NT>
 __global__ void __launch_bounds__(BM * 4)
 gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
-  constexpr int BN = 128, A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128;
-  constexpr int WS_ST = BM == 64 ? 6 : 5;
-  constexpr int PW = 256 / BM;  // LDS-DMA instructions of a wave per stage: 2 of A, PW of W
+  constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128;
+  constexpr int WS_ST = BM == 128 ? 5 : BN == 128 ? 6 : 10;
+  constexpr int PW = 2 * BN / BM;   // LDS-DMA instructions of a wave per stage: 2 of A, PW of W
+  constexpr int WN = BN / 32;       // waves along N (32 columns each)
+  constexpr int FM = BN == 64 ? 2 : 4, WROWS = FM * 16;  // row fragments and rows of a wave
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   __shared__ __attribute__((aligned(16))) char smem[WS_ST * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -318,14 +322,16 @@ gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
   for (int u = 0; u < mine; ++u) {
     int m0, n0, sp;
     unit_of(u, m0, n0, sp);
-    f32x4_t acc[4][2];
+    f32x4_t acc[FM][2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     for (int kt = 0; kt < nk; ++kt) {
       // this wave's pieces of the stage are in; after the barrier everyone's, and the slot before it has been read
-      if constexpr (BM == 64)
+      if constexpr (BN == 64)
+        asm volatile("s_waitcnt vmcnt(32) lgkmcnt(0)" ::: "memory");  // 4 * (10 - 2)
+      else if constexpr (BM == 64)
         asm volatile("s_waitcnt vmcnt(24) lgkmcnt(0)" ::: "memory");  // 6 * (6 - 2)
       else
         asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)" ::: "memory");  // 4 * (5 - 2)
@@ -333,33 +339,33 @@ gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
       issue();
-      const char* sa = smem + rd * STAGE + (w >> 2) * 64 * 128;
-      const char* sb = smem + rd * STAGE + A_BYTES + (w & 3) * 32 * 128;
+      const char* sa = smem + rd * STAGE + (w / WN) * WROWS * 128;
+      const char* sb = smem + rd * STAGE + A_BYTES + (w % WN) * 32 * 128;
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
         const int c = ((kk * 4 + fg) ^ sw) << 4;
-        bf16x8_t af[4], wf[2];
+        bf16x8_t af[FM], wf[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) wf[j] = *(const bf16x8_t*)(sb + (j * 16 + fr) * 128 + c);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) af[i] = *(const bf16x8_t*)(sa + (i * 16 + fr) * 128 + c);
+        for (int i = 0; i < FM; ++i) af[i] = *(const bf16x8_t*)(sa + (i * 16 + fr) * 128 + c);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
           for (int j = 0; j < 2; ++j) acc[i][j] = mfma16(wf[j], af[i], acc[i][j]);
       }
       rd = rd + 1 == WS_ST ? 0 : rd + 1;
     }
-    // ---- row m0 (+ 64) + 16 i + fr, columns col + 16 j + 4 fg .. + 3 ----
-    const int col = n0 + (w & 3) * 32 + 4 * fg;
+    // ---- row m0 (+ WROWS) + 16 i + fr, columns col + 16 j + 4 fg .. + 3 ----
+    const int col = n0 + (w % WN) * 32 + 4 * fg;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = m0 + (w >> 2) * 64 + i * 16 + fr;
+    for (int i = 0; i < FM; ++i) {
+      const int m = m0 + (w / WN) * WROWS + i * 16 + fr;
       if (m >= p.M) continue;
       float inv = 1.f;
       if (nrm.ssq) inv = rsqrtf(sum_strided(nrm.ssq + m, nrm.parts, 64) / nrm.norm_k + nrm.eps);
       if constexpr (EPI == EPI_SWIGLU) {
-        const int oc = n0 / 2 + (w & 3) * 16 + 4 * fg;
+        const int oc = n0 / 2 + (w % WN) * 16 + 4 * fg;
         if (oc >= p.N / 2) continue;
         float v[4];
 #pragma unroll
@@ -649,12 +655,12 @@ static int launch_tile(const GemmArgs& a, int epi, int splits, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-template <int BM, bool NT>
+template <int BM, int BN, bool NT>
 static int launch_ws_tile(const GemmArgs& a, int epi, int splits, const WsNorm& nrm, hipStream_t s) {
-  const long units = (long)((a.M + BM - 1) / BM) * ((a.N + 127) / 128) * splits;
+  const long units = (long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN) * splits;
   if (units > 0x7fffffffL || a.k_per_split % 64 || a.k_per_split < 64) return (int)hipErrorInvalidValue;
   const dim3 grid((unsigned)min(units, 256L)), block(BM * 4);
-#define WS_LAUNCH(E) gemm_ws_kernel<BM, E, NT><<<grid, block, 0, s>>>(a, nrm, splits)
+#define WS_LAUNCH(E) gemm_ws_kernel<BM, BN, E, NT><<<grid, block, 0, s>>>(a, nrm, splits)
   switch (splits > 1 ? (int)EPI_PARTIAL : epi) {
     case EPI_NONE: WS_LAUNCH(EPI_NONE); break;
     case EPI_BIAS: WS_LAUNCH(EPI_BIAS); break;
@@ -668,11 +674,15 @@ static int launch_ws_tile(const GemmArgs& a, int epi, int splits, const WsNorm& 
   return (int)hipGetLastError();
 }
 
+// 64 x 64 tiles: (8192, 16384] columns without splits (_dk_splits, _auto_splits). Narrower products have to be split either
+// way, and the wider tile then moves less of A: 64 x 8192 x 4096 22.8 us at four splits vs 24.0 at two of 64 x 64.
 // W is read once where there is one row block only: not worth a place in the caches then.
 static int launch_ws(const GemmArgs& a, int epi, int splits, const WsNorm& nrm, hipStream_t s) {
-  if (a.M <= 64) return launch_ws_tile<64, true>(a, epi, splits, nrm, s);
-  if (a.M <= 128) return launch_ws_tile<128, true>(a, epi, splits, nrm, s);
-  return launch_ws_tile<128, false>(a, epi, splits, nrm, s);
+  if (a.M <= 64)
+    return splits == 1 && a.N <= 16384 ? launch_ws_tile<64, 64, true>(a, epi, splits, nrm, s)
+                                       : launch_ws_tile<64, 128, true>(a, epi, splits, nrm, s);
+  if (a.M <= 128) return launch_ws_tile<128, 128, true>(a, epi, splits, nrm, s);
+  return launch_ws_tile<128, 128, false>(a, epi, splits, nrm, s);
 }
 
 // Its offsets into a tile's rows are 32 bits wide.

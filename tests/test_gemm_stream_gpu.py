@@ -26,7 +26,7 @@ def _swiglu(x):
 
 # (rows, columns, K, K splits): one K step (fewer than the ring's stages), the ring's length and one more, a last row
 # and column tile that are not full, more tiles than workgroups (257 and several rounds of them), several row blocks
-@pytest.mark.parametrize("M,N,Kd,splits", [(33, 128, 64, 1), (64, 136, 64 * 6, 1), (63, 96, 64 * 7, 1), (64, 128 * 257, 128, 1),
+@pytest.mark.parametrize("M,N,Kd,splits", [(33, 128, 64, 1), (64, 136, 64 * 10, 1), (63, 96, 64 * 11, 1), (50, 16384 + 40, 64 * 7, 1), (64, 128 * 257, 128, 1),
                                            (65, 32, 128, 2), (200, 128 * 200 + 32, 192, 1), (64, 4096, 2048, 8),
                                            (129, 160, 64 * 12, 4), (639, 1024, 512, 1)])
 @pytest.mark.parametrize("epi", ["none", "bias", "gelu", "swiglu", "resid"])
@@ -47,7 +47,7 @@ def test_stream_tile(M, N, Kd, splits, epi):
     assert ((got - ref).abs() <= tol).all()
 
 
-@pytest.mark.parametrize("M,N,Kd", [(33, 128 * 128, 512), (64, 128 * 129, 512), (48, 128 * 224 + 32, 256)])
+@pytest.mark.parametrize("M,N,Kd", [(33, 8192, 512), (64, 8192 + 32, 512), (40, 16384, 256), (48, 128 * 224 + 32, 256)])
 @pytest.mark.parametrize("epi", ["none", "swiglu"])
 def test_row_norm_without_splits(M, N, Kd, epi):
     """Wide products of 33..64 rows: the rows' scale in the epilogue (no partials), either side of the rule's line."""
