@@ -72,10 +72,11 @@ def _meta(m: SeqBatch):
     return [_ptr(m.cu), _ptr(m.slot), _ptr(m.pos0), _ptr(m.seq), m.T, m.B]
 
 
-def _scratch(m: SeqBatch, waves: int, fill: int, device, *shapes):
+def _scratch(m: SeqBatch, waves: int, fill: int, device, *shapes, deep: int = 1):
     """Arguments of a chunked recurrence: fp32 scratch [chunks + B, *shape] each, the chunk list, its length and
     the chunk length (no scratch and no chunks where the portions are walked from end to end)."""
-    n = m.chunk_len(waves, fill)
+    # (deep: chunks that fill the chip that many times, where the portions alone do not fill it once)
+    n = m.chunk_len(waves, fill) and m.chunk_len(waves, fill * deep)
     if n == 0:
         return [], [None] * len(shapes) + [None, None, 0, 0]
     ck, base, tot = m.chunks(n)
@@ -285,7 +286,10 @@ def selective_scan(x, dt, bc, off_b: int, off_c: int, z, A, D, state, conv_x, co
     _req(x.shape == (m.T, C) and z.shape == (m.T, C) and state.shape[1:] == (C, N) and N <= 512
          and max(off_b, off_c) + N <= bc.shape[1] and bc.shape[0] == m.T, "selective_scan shapes")
     y = torch.empty((m.T, C), dtype=x.dtype, device=x.device)
-    ws, chunk = _scratch(m, C * -(-N // 8) // 64, 2048, x.device, (C, N), (C,))
+    # (four times over: a CU has 8 - 9 chunks instead of 2 or 3, so neither a last round of workgroups is nearly empty nor
+    # are two waves a SIMD left to hide the exponentials: 2048 + 1570 tokens, 8192 x 16 states, 217 us in chunks of 128 vs
+    # 304 of 448; 700 tokens 68 in chunks of 64 vs 91 of 128; 5981 tokens in 5 portions 350 of 192 vs 495 of 704)
+    ws, chunk = _scratch(m, C * -(-N // 8) // 64, 2048, x.device, (C, N), (C,), deep=4)
     _check(lib().da_selective_scan(_ptr(x), x.stride(0), _ptr(dt), C, _ptr(bc), bc.stride(0), off_b, off_c, _ptr(z),
                                    z.stride(0), _ptr(A), _ptr(D), _ptr(state), _ptr(y), C, C, N,
                                    *_conv_args(conv_x, conv_state, C, x.dtype, m), *chunk, m.max_len, *_meta(m), f32,
