@@ -585,11 +585,14 @@ def _auto_splits(M: int, N: int, K: int) -> int:
         return s
     if M > 128:
         # rounds of the 128x128 tile (0.56 us a K-step of 64) + the reduce (a launch, and its partials out and in at
-        # 4 TB/s): 600 x 4096 x 14336 113 us at 4 splits vs 125 at 1 and 135 at 2; 256 x 4096 x 14336 50 at 4 vs 54
-        # at 8 and 78 at 2; 200 x 28672 x 4096 79 at 1 vs 96 at 2; 200 x 3072 x 8192 29 at 4 vs 32 at 8
+        # 4 TB/s): 256 x 4096 x 14336 50 us at 4 splits vs 78 at 2; 200 x 28672 x 4096 79 at 1 vs 96 at 2; 200 x 3072 x
+        # 8192 29 at 4 vs 32 at 8. At most 1024 64x128 blocks of partials below 256 rows and 640 from there: a prefill
+        # must not outgrow the workspace that captured decode steps point at
+        blocks = math.ceil(M / 64) * math.ceil(N / 128)
         tiles = math.ceil(M / 128) * math.ceil(N / 128)
         cost = {s: math.ceil(tiles * s / 256) * (ksteps // s) * 0.56 + (4 + s * M * N * 2e-6 if s > 1 else 0)
-                for s in (1, 2, 4, 8) if ksteps % s == 0 and (s == 1 or ksteps // s >= 4)}
+                for s in (1, 2, 4, 8) if s == 1 or (ksteps % s == 0 and ksteps // s >= 4
+                                                    and blocks * s <= (1024 if M < 256 else 640))}
         return min(cost, key=cost.get)
     if M > 32 and N > 8192:  # (see _dk_splits)
         return 1
