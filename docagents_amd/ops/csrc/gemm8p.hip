@@ -691,6 +691,15 @@ int gemm8p_pick_bm(int M, int N, int K, bool tail) {
   return cost(128, 72) < cost(256, 100) ? 128 : 256;
 }
 
+// Whether a product that is handed scratch (tail_ws, tail_cnt) uses it: its counters have to be zero then. tile: 0, or
+// the row-tile height's code (4 / 7: 256, 10: 128).
+DA_EXPORT int da_gemm_tail_used(int M, int N, int K, int epi, int tile) {
+  if (epi == EPI_GELU || epi == EPI_ROPE || K < 128 || !persist_on()) return 0;
+  const int bm = tile == 10 ? 128 : tile ? 256 : gemm8p_pick_bm(M, N, K, true);
+  const long nt = (long)((M + bm - 1) / bm) * ((N + BN - 1) / BN);
+  return nt < 0x7fffffff && tail_slices((int)nt, K / 64, bm) > 1;
+}
+
 // epi + 100: the same kernel on fp16 operands / output (v_mfma_f32_16x16x32_f16)
 int launch_gemm8p(const GemmArgs& a, int epi, hipStream_t s, int bm) {
   if (a.K < 128 || a.K % 64) return (int)hipErrorInvalidValue;

@@ -62,6 +62,7 @@ _SIGS = {
     "da_gemm_dk_parts": [c_int],
     "da_enc_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5
                   + [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_void_p],
+    "da_gemm_tail_used": [c_int] * 5,
     "da_gemm_dk_splitk": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                           c_int, c_void_p, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_void_p],
     "da_decode_attn": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
@@ -235,27 +236,29 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
 
 
 # Scratch of the prefill products' last round (csrc/gemm8p.hip, "Tail"): 256 workgroups' fp32 partials and their tiles'
-# counters, 64 MB, per stream: streams run products beside each other. At most TAIL_STREAMS of them per device have one;
-# never given back (the caching allocator would hand the memory to kernels that may still run beside it).
+# counters, 64 MB, per stream: streams run products beside each other. At most TAIL_STREAMS of them per device keep one
+# (never given back: the caching allocator would hand the memory to kernels that may still run beside it).
 TAIL_STREAMS = 8
 _TAIL: dict = {}
 
 
-def _gemm_tail(device, stream: int):
-    """(partials, counters) of a stream, (None, None): this product keeps its tiles whole. Under capture too: a graph
-    may be replayed on another stream, beside the one that it was recorded on."""
-    if torch.cuda.is_current_stream_capturing():
-        return None, None
-    key = (device.index, stream)
-    bufs = _TAIL.get(key)
-    if bufs is None:
-        with _LOCK:
-            bufs = _TAIL.get(key)
-            if bufs is None and sum(k[0] == device.index for k in _TAIL) >= TAIL_STREAMS:
-                return None, None
-            bufs = _TAIL[key] = bufs or (torch.empty(256 * 256 * 256, dtype=torch.float32, device=device),
+def _gemm_tail(device, stream: int, M: int, N: int, K: int, epi: int, tile: int = 0):
+    """(partials, counters) for a product on the current stream ``stream``; the caller holds them until it is launched.
+    Streams beyond TAIL_STREAMS and captured products (a graph may be replayed on another stream) have them for the one
+    call, the counters cleared by a launch: the sums are the same everywhere, in the same order."""
+    if not torch.cuda.is_current_stream_capturing():
+        key = (device.index, stream)
+        bufs = _TAIL.get(key)
+        if bufs is None:
+            with _LOCK:
+                bufs = _TAIL.get(key)
+                if bufs is None and sum(k[0] == device.index for k in _TAIL) < TAIL_STREAMS:
+                    bufs = _TAIL[key] = (torch.empty(256 * 256 * 256, dtype=torch.float32, device=device),
                                          torch.zeros(256 * 8, dtype=torch.int32, device=device))
-    return _ptr(bufs[0]), _ptr(bufs[1])
+        if bufs is not None:
+            return bufs
+    make = torch.zeros if lib().da_gemm_tail_used(M, N, K, epi, tile) else torch.empty
+    return torch.empty(256 * 256 * 256, dtype=torch.float32, device=device), make(256 * 8, dtype=torch.int32, device=device)
 
 
 def gemv_fusable(M: int, N: int, K: int, epi: int = EPI_NONE) -> bool:
@@ -314,9 +317,10 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
     if splits > 1:
         ws = _workspace(splits * M * N * 4, a.device)
     stream = torch.cuda.current_stream().cuda_stream
-    tail = _gemm_tail(a.device, stream) if M >= 640 or tile else (None, None)  # (gemm8p's rows)
+    # (gemm8p's rows and tiles)
+    tail = _gemm_tail(a.device, stream, M, N, K, epi, tile) if tile in (4, 7, 10) or (tile == 0 and M >= 640) else (None, None)
     rc = lib().da_gemm_bf16(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
-                            M, N, K, epi, tile, splits, _ptr(ws), _ptr(gamma), float(eps), *tail, c_void_p(stream))
+                            M, N, K, epi, tile, splits, _ptr(ws), _ptr(gamma), float(eps), *map(_ptr, tail), c_void_p(stream))
     _check(rc, "gemm")
     return out
 
@@ -1187,9 +1191,9 @@ def gemm_f16(a, w, bias=None, epi: int = EPI_NONE, resid=None, out=None) -> torc
         out = torch.empty((M, N), dtype=torch.float16, device=a.device)
     _req(out.dtype == torch.float16 and out.shape == (M, N) and out.stride(1) == 1 and out.stride(0) % 8 == 0, "out")
     stream = torch.cuda.current_stream().cuda_stream
-    tail = _gemm_tail(a.device, stream) if M >= 256 else (None, None)
+    tail = _gemm_tail(a.device, stream, M, N, K, epi) if M >= 256 else (None, None)
     _check(lib().da_gemm_f16(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
-                             M, N, K, epi, *tail, c_void_p(stream)), "gemm_f16")
+                             M, N, K, epi, *map(_ptr, tail), c_void_p(stream)), "gemm_f16")
     return out
 
 

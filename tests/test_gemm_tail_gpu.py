@@ -64,9 +64,11 @@ def test_tail_f16(M, N, Kd, monkeypatch):
 
 
 def test_tail_streams():
-    """Products beside each other on several streams, more of them than have scratch of their own."""
+    """Products beside each other on several streams, more of them than keep scratch, and captured ones: the same bits."""
     a, w, _, _ = _operands(700, 768, 2048, torch.bfloat16, 1)
     want = a.double() @ w.double().T
+    first = K.gemm(a, w, tile=7)
+    assert float((first.double() - want).norm() / want.norm()) < 2.0 ** -8
     streams = [torch.cuda.Stream() for _ in range(K.TAIL_STREAMS + 2)]
     torch.cuda.synchronize()
     out = []
@@ -75,5 +77,15 @@ def test_tail_streams():
             with torch.cuda.stream(s):
                 out.append(K.gemm(a, w, tile=7))
     torch.cuda.synchronize()
-    assert max(float((x.double() - want).norm() / want.norm()) for x in out) < 2.0 ** -8
+    assert all(torch.equal(x, first) for x in out)
     assert len(K._TAIL) <= K.TAIL_STREAMS
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = [K.gemm(a, w, tile=7) for _ in range(2)]
+    for _ in range(3):
+        for x in captured:
+            x.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, first) for x in captured)
+        assert torch.equal(K.gemm(a, w, tile=7), first)
