@@ -1247,10 +1247,11 @@ decode_attn_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __restri
 //                         is a contiguous [64 x D] block of the cache, so it is copied by LDS-DMA
 //                         (global_load_lds, 1 KiB per wave-instruction) with an XOR chunk swizzle
 //                         on the source address that makes the transposed reads conflict-free.
-// by_len: a row is split by its own length, and splits are the slowest grid dimension: as the fastest one, the
-// workgroups of a launch with two splits whose rows need one only were all on the even XCDs (64 rows of 2048 keys: 147 us
-// against 86). A workgroup of a split past the row's keys ends at once. Tried and slower: two tiles in flight per wave
-// (hipcc drains the DMA before the transposed reads, and twice the LDS leaves one workgroup per CU).
+// by_len: a row takes at most as many splits as hold chunk_max keys each (256: a split's merge costs what reading 100 - 200
+// keys does), and splits are the slowest grid dimension: as the fastest one, the workgroups of a launch with two splits
+// whose rows need one only were all on the even XCDs (64 rows of 2048 keys: 147 us against 86). A workgroup of a split
+// past the row's keys ends at once. Tried and slower: two tiles in flight per wave (hipcc drains the DMA before the
+// transposed reads, and twice the LDS leaves one workgroup per CU).
 template <int D>
 __device__ __forceinline__ int vswz(int r) {
   return D == 128 ? ((r & 7) << 1) : (((r >> 1) & 3) << 1);
@@ -1276,10 +1277,10 @@ decode_attn_gqa_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __re
   const int split = by_len ? blockIdx.z : blockIdx.x;
   const int L = lens[b];
   DA_ASSERT(L >= 0 && L <= max_seq && slot[b] >= 0);
-  // by_len: a row's keys over as many splits as hold chunk_max of them each, evenly; the others have nothing to do
+  // by_len: a row's keys evenly over as many splits as hold chunk_max of them each; the others have nothing to do
   const int act = by_len && cnt ? min(nsplit, max(1, (L + chunk_max - 1) / chunk_max)) : nsplit;
   if (split >= act) return;
-  const int chunk = dec_chunk(L, act, chunk_max);
+  const int chunk = dec_chunk(L, act, by_len ? 0x7fffffff : chunk_max);
   const int kstart = split * chunk;
   const int kend = min(L, kstart + chunk);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;

@@ -789,30 +789,41 @@ def _uncached(tag: str, nbytes: int, device) -> _RawBuf:
     return bufs[-1]
 
 
-def _decode_split(B: int, Hkv: int, max_len: int, chunk: int, by_len: bool = False):
+def _decode_split(B: int, Hkv: int, max_len: int, chunk: int):
     """(chunk, nsplit) of a decode-attention launch (static for a captured graph: from max_len)."""
-    want = max_len * B * Hkv
-    if chunk <= 0 and by_len:
-        # splits by a row's own length: merging costs a split 10 us and more, and a second workgroup on a CU slows the
-        # first: 340 workgroups if every row were full (rows are half that on average), whole rows from 192 on
-        chunk = max_len if B * Hkv >= 192 else max(512, math.ceil(want / 340 / 256) * 256)
     if chunk <= 0:
         # measured on MI355X (profiles/decode_attn_chunks_r1.txt): per-workgroup overhead dominates
         # small chunks; aim for ~768 workgroups, 512..4096 keys each
+        want = max_len * B * Hkv / 768
         chunk = 512
-        while chunk < want / 768 and chunk < 4096:
+        while chunk < want and chunk < 4096:
             chunk *= 2
-    chunk = math.ceil(chunk / 64) * 64
     return chunk, max(1, math.ceil(max_len / chunk))
 
 
-def _decode_by_len(B: int, H: int, Hkv: int, D: int, max_len: int) -> bool:
-    """Few grouped-query (row, head) pairs are split by the rows' own length, not over every split of the launch: below 320
-    pairs with a cache of up to 4096 keys, below 128 with a longer one. 8 KV heads x 128, rows of 500 - 3000 of 4096: 8 /
-    16 / 32 rows 29.5 / 39.4 / 64.1 -> 25.0 / 33.2 / 55.2 us, 33 rows of 100 - 400: 26.5 -> 17.0; of 1000 - 8000 of 8192:
-    4 / 8 / 12 rows 29.5 / 42.2 / 56.9 -> 24.5 / 36.9 / 49.1. Beyond, the even splits are as good or better (48 rows of
-    500 - 3000: 86 against 93; 16 rows of 1000 - 8000: 72 against 77)."""
-    return H != Hkv and D in (64, 128) and B * Hkv < (320 if max_len <= 4096 else 128)
+BY_LEN_KEYS = 256
+
+
+def _gqa_split(B: int, Hkv: int, max_len: int):
+    """(chunk, nsplit, by_len) of a grouped-query launch (head dims 64 and 128) whose caller names no chunk. by_len: a row's
+    keys over as many of the nsplit splits as hold ``chunk`` of them each; else over all of them. Measured over 16 query
+    heads on 2 KV heads x 64, 32 on 4 and on 8 x 128, 1 - 64 rows in caches of 1024 - 16384 keys, all rows of a length or
+    mixed:
+      * 192 - 256 (row, head) pairs in up to 2048 keys: whole rows, a workgroup per CU (8 heads, 24 - 32 rows of 100 - 750
+        of 1024: 24 - 28 -> 18 - 19 us; of 250 - 1500 of 2048: 37 - 42 -> 31 - 32; one full row among short ones loses
+        up to 1.5x). In 4096 keys the gain is 3 - 13 % and the loss 1.65x: not there.
+      * the even splits are of 512 keys and more than one round of workgroups, or the cache is up to 1024 or from 8192
+        keys long: by the row's length (8 heads, 8 rows of 1024 in 4096: 21.9 -> 14.5; 4 rows of 2000 in 8192: 26.5 ->
+        15.1, of 4000 30.5 -> 26.5; 12 rows of 500 in 2048: 21.2 -> 13.6, full 33.5 -> 32.3; half the rows full and half
+        short loses up to 1.17x). Even splits of 1024 keys gain 4 % by it and lose up to 1.5x.
+      * else even: a launch that leaves CUs idle is the faster the more splits it has (one row of 1024 in 4096: 10.9 us
+        even, 12.1 by length)."""
+    if 192 <= B * Hkv <= 256 and max_len <= 2048:
+        return math.ceil(max_len / 64) * 64, 1, False
+    chunk, nsplit = _decode_split(B, Hkv, max_len, 0)
+    if chunk == 512 and nsplit > 1 and (B * Hkv * nsplit > 256 or not 1024 < max_len < 8192):
+        return BY_LEN_KEYS, nsplit, True
+    return chunk, nsplit, False
 
 
 # Same-XCD split exchange of the batch-1..small-batch MHA decode attention (attention.hip, VAR bit 3):
@@ -891,8 +902,10 @@ def decode_attn(q, k_cache, v_cache, lens, slot, H, Hkv, D, max_len: int, chunk:
     k / v into the cache at pos (== lens - 1) — the decode step's rope_cache launch folded in."""
     cs, ps = _decode_checks(q, k_cache, v_cache, lens, slot, H, Hkv, D, max_len, pre, rope)
     B = q.shape[0]
-    by_len = _decode_by_len(B, H, Hkv, D, max_len)
-    chunk, nsplit = _decode_split(B, Hkv, max_len, chunk, by_len)
+    if chunk <= 0 and H != Hkv and D in (64, 128):
+        chunk, nsplit, by_len = _gqa_split(B, Hkv, max_len)
+    else:
+        (chunk, nsplit), by_len = _decode_split(B, Hkv, max_len, chunk), False
     ws = _workspace(B * H * nsplit * (D + 2) * 4, q.device)
     if out is None:
         out = torch.empty((B, H * D), dtype=torch.bfloat16, device=q.device)

@@ -35,3 +35,25 @@ def test_rows_of_every_length(H, Hkv, D, chunk, monkeypatch):
                 got = K.decode_attn(q, kc, vc, lt, slot, H, Hkv, D, max_len=S, chunk=chunk, pre=p).float()
                 # weights and result are rounded to bf16: 2^-8 of values of about 1 each
                 assert bool(((got - want).abs() <= 2.0 ** -7 * (1 + want.abs())).all())
+
+
+@pytest.mark.parametrize("H,Hkv,D,B,S,route", [
+    (8, 2, 128, 11, 1000, "by_len"), (8, 1, 64, 11, 8200, "by_len"), (16, 8, 64, 11, 1500, "by_len"),
+    (16, 8, 128, 24, 333, "rows"), (32, 8, 64, 32, 1027, "rows"), (8, 4, 128, 11, 1300, "even"),
+])
+def test_automatic_split(H, Hkv, D, B, S, route, monkeypatch):
+    """Rows at the edges of a split's 256 keys, one key, the whole cache; splits past a row's keys do nothing."""
+    torch.manual_seed(S)
+    chunk, nsplit, by_len = K._gqa_split(B, Hkv, S)
+    assert route == ("by_len" if by_len else "rows" if nsplit == 1 else "even")
+    lens = ([1, 64, 255, 256, 257, 300, 511, 512, 513, S - 1, S] * 3)[:B]
+    lens = [min(n, S) for n in lens]
+    kc, vc = (torch.randn(B, Hkv, S, D, device=DEV).bfloat16() for _ in range(2))
+    q = torch.randn(B, H * D, device=DEV).bfloat16()
+    lt, slot = torch.tensor(lens, dtype=torch.int32, device=DEV), torch.randperm(B, device=DEV).int()
+    want = R.decode_attn(q, kc, vc, lt, slot, H, Hkv, D).float()
+    for fused in (True, False):
+        monkeypatch.setattr(K, "_FUSED_COMBINE", fused)
+        for _ in range(2):
+            got = K.decode_attn(q, kc, vc, lt, slot, H, Hkv, D, max_len=S).float()
+            assert bool(((got - want).abs() <= 2.0 ** -7 * (1 + want.abs())).all())
