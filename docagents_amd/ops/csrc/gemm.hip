@@ -685,14 +685,22 @@ static int launch_ws(const GemmArgs& a, int epi, int splits, const WsNorm& nrm, 
   return launch_ws_tile<128, 128, false>(a, epi, splits, nrm, s);
 }
 
-// Its offsets into a tile's rows are 32 bits wide.
-static bool ws_spans(const GemmArgs& a) { return (size_t)max(a.K, a.lda) * 256 < 0x7ffffff0ull; }
+// The streaming kernel's offsets into a tile's rows are 32 bits wide (_dk_splits draws the same line).
+static bool ws_spans(const GemmArgs& a) { return max(a.K, a.lda) < 1 << 22; }
 
-// Decode tiles: the streaming kernel (64x128 / 128x128); 32x128, and 64x128 for rows too long for it, with 4 k-tiles in flight per workgroup (register prefetch depth
-// 4; 1 / 2 / 8 measured slower, profiles/decode_gemm_prefetch_sweep_r1.jsonl).
+// Filling the ring and draining it costs the streaming kernel a microsecond, which K splits of fewer than 28 stages of up
+// to 64 rows do not win back from the register-staged 64x128 tile with 4 k-tiles in flight (depth 1 / 2 / 8 measured slower,
+// profiles/decode_gemm_prefetch_sweep_r1.jsonl): with their reduce, 64 rows, register / streaming us: 768 x 768 8.3 / 9.7
+// (6 stages), 8192 x 2048 15.7 / 17.7 (8), 3072 x 8192 18.5 / 19.4 (16), 4096 x 14336 29.4 / 29.3 (28), 8192 x 14336 48.4 /
+// 46.5 (56). Unsplit products are faster on the ring at every length (64 x 12288 x 768 9.9 / 9.3).
+static bool ws_pays(const GemmArgs& a, int splits) {
+  return ws_spans(a) && (a.M > 64 || splits == 1 || a.k_per_split >= 28 * 64);
+}
+
+// Decode tiles: 64x128 by the rule above, else 4 k-tiles in flight per workgroup.
 template <int BM, int BN>
 static int launch_decode_tile(const GemmArgs& a, int epi, int splits, hipStream_t s) {
-  if (BM == 64 && ws_spans(a)) return launch_ws(a, epi, splits, WsNorm{}, s);
+  if (BM == 64 && ws_pays(a, splits)) return launch_ws(a, epi, splits, WsNorm{}, s);
   return launch_tile<BM, BN, 1, 4, 4>(a, epi, splits, s);
 }
 

@@ -351,13 +351,15 @@ def _dk_splits(N: int, K: int, reduce: bool = False) -> int:
     """Split-K of the 33..64-row route (64x128 tiles): the largest of 2, 3, 4, 6, 8, 12, 16 that keeps
     the grid within one round of 256 workgroups and >= 4 K-steps of 64 per split. 3 is the point of this
     list: the Phi-3 QKV projection (72 tiles) 18.7 us at 3 splits vs 21.8 at 2 and 25.7 at 4
-    (bench/splitk_m64.py, profiles/r3/splitk_m64.txt). None above N = 8192: the streaming tile (64 wide
-    to N = 16384) reaches HBM's rate on the CUs that it fills without, and the reduce launch goes (64 rows,
-    N = 17920, K = 5120: 49 us vs 59 at 2; 28672 x 4096: 48 vs 60; 12672 x 4096: 29 vs 33; 9216 x 3072:
-    21.2 vs 23.1 at 3; below the line 8192 x 4096: 25.0 vs 22.8 at 4). reduce: at least 2 (row sums of squares are written there)."""
+    (bench/splitk_m64.py, profiles/r3/splitk_m64.txt). None above N = 8192 (to K = 8192): the streaming
+    tile (64 wide to N = 16384) reaches HBM's rate on the CUs that it fills without, and the reduce launch
+    goes (64 rows, N = 17920, K = 5120: 49 us vs 59 at 2; 28672 x 4096: 48 vs 60; 12672 x 4096: 29 vs 33;
+    9216 x 3072: 21.2 vs 23.1 at 3; below the line 8192 x 4096: 25.0 vs 22.8 at 4); with a longer K two
+    128-wide splits move half of A and are faster (12288 x 8192: 45.1 vs 47.2 at 2, x 14336: 86.6 vs 71.7).
+    reduce: at least 2 (row sums of squares are written there)."""
     tiles, ks = (N + 127) // 128, K // 64
     best = 2 if reduce else 1
-    if not reduce and N > 8192:
+    if not reduce and N > 8192 and K <= 8192:
         return 1
     for s in (2, 3, 4, 6, 8, 12, 16):
         if ks % s == 0 and ks // s >= 4 and tiles * s <= 256:
@@ -598,7 +600,7 @@ def _auto_splits(M: int, N: int, K: int) -> int:
                 for s in (1, 2, 4, 8) if s == 1 or (ksteps % s == 0 and ksteps // s >= 4
                                                     and blocks * s <= (1024 if M < 256 else 640))}
         return min(cost, key=cost.get)
-    if M > 32 and N > 8192:  # (see _dk_splits)
+    if M > 32 and N > 8192 and K <= 8192:  # (see _dk_splits)
         return 1
     tiles = math.ceil(N / 128)
     s = 1

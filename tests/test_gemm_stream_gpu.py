@@ -60,3 +60,29 @@ def test_row_norm_without_splits(M, N, Kd, epi):
     mag = ((a.double().abs() @ w.double().abs().T) * inv).max()
     ref = _swiglu(ref) if epi == "swiglu" else ref
     assert ((got - ref).abs() <= U * ref.abs() + 8 * Kd * 2.0 ** -24 * mag).all()
+
+
+@pytest.mark.parametrize("M,N,stages,splits", [(64, 136, 27, 2), (64, 136, 28, 2), (33, 4096 + 8, 28, 3), (48, 320, 4, 32)])
+def test_split_products_either_side_of_the_ring(M, N, stages, splits):
+    """K splits of up to 64 rows: 28 stages are the first on the ring, shorter ones are staged through registers."""
+    Kd = 64 * stages * splits
+    a, w, bias, g = _operands(M, N, Kd, Kd + 64)
+    resid = torch.randn(M, N, device="cuda", generator=g).bfloat16()
+    got = K.gemm(a, w, bias, epi=K.EPI_RESID, resid=resid, tile=2, splits=splits).double()
+    ref = a.double() @ w.double().T + bias.double() + resid.double()
+    tol = U * ref.abs() + 8 * Kd * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T).max()
+    assert ((got - ref).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("Kd", [8192, 8192 + 256])
+def test_wide_long_products(Kd):
+    """More than 8192 columns: whole to K = 8192, in splits from there."""
+    M, N = 40, 8192 + 64
+    assert (K._dk_splits(N, Kd) == 1) == (Kd <= 8192) == (K._auto_splits(M, N, Kd) == 1)
+    a, w, bias, g = _operands(M, N, Kd)
+    ssq = torch.rand(3, 64, device="cuda", generator=g) * Kd / 3 * 2
+    got = K.gemm_dk(a, w, epi=K.EPI_SWIGLU, norm_in=(ssq, 3, 1e-5)).double()
+    inv = (ssq[:, :M].double().sum(0) / Kd + 1e-5).rsqrt()[:, None]
+    ref = _swiglu((a.double() @ w.double().T) * inv)
+    mag = ((a.double().abs() @ w.double().abs().T) * inv).max()
+    assert ((got - ref).abs() <= U * ref.abs() + 8 * Kd * 2.0 ** -24 * mag).all()
