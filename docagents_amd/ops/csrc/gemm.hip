@@ -890,7 +890,7 @@ DA_EXPORT int da_gemm_rope(const void* A, int lda, const void* W, void* C, int l
 
 // Tile selection: big tiles when the grid fills 256 CUs, skinny tiles (+ split-K) for decode-sized M.
 // tile: 0 = auto, 1 = 128x128, 2 = weight-streaming 64x128 / 128x128, 3 = 32x128, 4 / 7 = 256x256 phase-split (gemm8p),
-// 6 = GEMV (M = 1), 8 = 128x128 PF4, 9 = 128x64 PF4, 10 = 128x256 phase-split (gemm8p),
+// 6 = GEMV (M = 1), 8 = 128x128 PF4, 9 = 128x64 PF4, 10 = 128x256 phase-split (gemm8p), 11 = 64x128 PF4,
 // 13 = 256x256 four-wave (gemm4w).
 DA_EXPORT int da_gemm_bf16(const void* A, int lda, const void* W, void* C, int ldc,
                            const void* bias, const void* resid, int ldr,
@@ -936,6 +936,7 @@ DA_EXPORT int da_gemm_bf16(const void* A, int lda, const void* W, void* C, int l
     case 3: err = launch_decode_tile<32, 128>(a, epi, splits, s); break;
     case 8: err = launch_tile<128, 128, 2, 2, 4>(a, epi, splits, s); break;   // mid-M weight streaming
     case 9: err = launch_tile<128, 64, 2, 2, 4>(a, epi, splits, s); break;
+    case 11: err = launch_tile<64, 128, 1, 4, 4>(a, epi, splits, s); break;
     default: return (int)hipErrorInvalidValue;
   }
   if (err || splits == 1) return err;

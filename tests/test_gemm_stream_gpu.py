@@ -86,3 +86,22 @@ def test_wide_long_products(Kd):
     ref = _swiglu((a.double() @ w.double().T) * inv)
     mag = ((a.double().abs() @ w.double().abs().T) * inv).max()
     assert ((got - ref).abs() <= U * ref.abs() + 8 * Kd * 2.0 ** -24 * mag).all()
+
+
+@pytest.mark.parametrize("M,N,Kd", [(300, 12288, 256), (129, 320, 4096), (449, 1160, 64), (639, 3072, 512), (200, 2304, 8192), (130, 3072 + 8, 8192)])
+@pytest.mark.parametrize("epi", ["none", "gelu", "swiglu", "resid"])
+def test_mid_rows(M, N, Kd, epi):
+    """129..639 rows as the rule has them: either tile, whole and in splits."""
+    if epi == "swiglu" and N % 32:
+        N += 32 - N % 32
+    a, w, bias, g = _operands(M, N, Kd)
+    code = {"none": K.EPI_NONE, "gelu": K.EPI_GELU, "swiglu": K.EPI_SWIGLU, "resid": K.EPI_RESID}[epi]
+    resid = torch.randn(M, N, device="cuda", generator=g).bfloat16() if epi == "resid" else None
+    b = None if epi == "none" else bias
+    got = K.gemm(a, w, b, epi=code, resid=resid).double()
+    ref = a.double() @ w.double().T + (0 if b is None else b.double())
+    ref = {"gelu": torch.nn.functional.gelu, "swiglu": _swiglu}.get(epi, lambda x: x)(ref)
+    if resid is not None:
+        ref = ref + resid.double()
+    tol = U * ref.abs() + 8 * Kd * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T).max()
+    assert ((got - ref).abs() <= tol).all()
