@@ -65,11 +65,11 @@ __device__ __forceinline__ int fresh_lane() {
   return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, z));
 }
 
-template <int EPI, int BM, typename T = BF16T, bool PERSIST = false>
+template <int EPI, int BM, typename T = BF16T, bool PERSIST = false, bool TAIL = false>
 __global__ void __launch_bounds__(512)
 gemm8p_kernel(GemmArgs p) {
   static_assert(BM == 256 || BM == 128, "BM");
-  constexpr bool TAIL = PERSIST && EPI != EPI_GELU;  // (beside the activation's registers the tail's spill)
+  static_assert(!TAIL || (PERSIST && EPI != EPI_GELU), "TAIL");  // (beside the activation's registers the tail's spill)
   constexpr int HALF_A = BM / 2 * 128;       // A half-tile: BM/2 rows x 64 bf16
   constexpr int OFF_A0 = 0, OFF_A1 = HALF_A, OFF_B0 = 2 * HALF_A, OFF_B1 = 2 * HALF_A + HALF_B;
   constexpr int BUF = 2 * HALF_A + 2 * HALF_B;
@@ -101,7 +101,7 @@ gemm8p_kernel(GemmArgs p) {
   };
   // the unit behind id: PERSIST's next whole tile, then this workgroup's slice of a tail tile, if it has one. (Slices
   // of a tile are TR workgroups apart, TR a multiple of 8: the tile ids keep the XCDs that xcd_remap gives them.)
-  const int nkt = p.K / 64, full = TAIL && p.tail_s > 1 ? ntiles / (int)GEMM_TAIL_WGS * (int)GEMM_TAIL_WGS : ntiles;
+  const int nkt = p.K / 64, full = TAIL ? ntiles / (int)GEMM_TAIL_WGS * (int)GEMM_TAIL_WGS : ntiles;
   const int rest = ntiles - full, TR = (rest + 7) & ~7;
   int id = blockIdx.x, m0, n0, kb = 0, nk = nkt;  // nk >= 2 (host-checked)
   [[maybe_unused]] bool tail = false;
@@ -110,7 +110,7 @@ gemm8p_kernel(GemmArgs p) {
   [[maybe_unused]] int unit = -1;
   if constexpr (TAIL) {
     const int t = blockIdx.x % max(TR, 1), sl = blockIdx.x / max(TR, 1);
-    if (p.tail_s > 1 && t < rest && sl < p.tail_s) unit = t | sl << 16;
+    if (t < rest && sl < p.tail_s) unit = t | sl << 16;
     unit = __builtin_amdgcn_readfirstlane(unit);
   }
   auto to_tail = [&]() __attribute__((always_inline)) {  // false: no slice for this workgroup
@@ -630,12 +630,14 @@ static void launch8p_epi(const GemmArgs& a0, int ntiles, hipStream_t s) {
   // (not EPI_ROPE: its per-row positions / slots / cos-sin next to the tile loop's state spill past
   // 256 VGPRs, and the persistent QKV projection measured 4 % slower, profiles/r5/gemm_persist/)
   if constexpr (EPI != EPI_ROPE) {
-    a.tail_s = EPI != EPI_GELU && persist_on() && a.tail_ws ? tail_slices(ntiles, a.K / 64, BM) : 1;
-    const int rest = ntiles % (int)GEMM_TAIL_WGS;
-    if (a.tail_s > 1) {
-      const int grid = ntiles >= (int)GEMM_TAIL_WGS ? (int)GEMM_TAIL_WGS : a.tail_s * ((rest + 7) & ~7);
-      gemm8p_kernel<EPI, BM, T, true><<<dim3(grid), dim3(512), 0, s>>>(a);
-      return;
+    if constexpr (EPI != EPI_GELU) {
+      a.tail_s = persist_on() && a.tail_ws ? tail_slices(ntiles, a.K / 64, BM) : 1;
+      const int rest = ntiles % (int)GEMM_TAIL_WGS;
+      if (a.tail_s > 1) {
+        const int grid = ntiles >= (int)GEMM_TAIL_WGS ? (int)GEMM_TAIL_WGS : a.tail_s * ((rest + 7) & ~7);
+        gemm8p_kernel<EPI, BM, T, true, true><<<dim3(grid), dim3(512), 0, s>>>(a);
+        return;
+      }
     }
     if (persist_on() && ntiles > cus && cus >= 8) {
       gemm8p_kernel<EPI, BM, T, true><<<dim3(cus & ~7), dim3(512), 0, s>>>(a);

@@ -106,3 +106,13 @@ def test_serial_load_detector_catches_the_round_trip_loop():
                + "\ts_cbranch_scc1 .LBB0_10\n")
     assert _serial_load_loops("_Zk:\n" + serial) == [".LBB0_10"]
     assert _serial_load_loops("_Zk:\n" + batched) == []
+
+
+def test_whole_tile_products_carry_no_shared_round(tmp_path):
+    """The persistent prefill products whose tiles fill the chip's rounds keep their scalars in registers: what the shared
+    last round needs (24 - 34 spilled scalars when it was compiled into every instance) is in instances of its own."""
+    asm = _asm("gemm8p.hip", tmp_path)
+    spills = {m.group(1): int(m.group(2)) for m in re.finditer(
+        r"\.name:\s+(\S+)\n(?:(?!\.name:).)*?\.sgpr_spill_count:\s+(\d+)", asm, re.S)}
+    whole = {n: c for n, c in spills.items() if re.match(r"_Z13gemm8p_kernelILi[0134]ELi(128|256)E\d*B?F16TLb1ELb0E", n)}
+    assert len(whole) == 14 and max(whole.values()) <= 6, whole
