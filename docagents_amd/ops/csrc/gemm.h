@@ -31,13 +31,13 @@ struct GemmArgs {
   RopeArgs rope;                     // EPI_ROPE only
   int relu;   // EPI_SWIGLU: the gate's activation is relu, not silu
   int group;  // gemm8p: row tiles per grouped-M band of the tile order (0: the default, 4)
-  // gemm8p, tiles that do not fill a round of the chip: `tail_s` workgroups share the K of each (1: whole tiles only; not EPI_GELU),
-  // with fp32 partials in tail_ws and 8 counters per tile in tail_cnt (zero between launches)
+  // gemm8p, tiles that do not fill a round of the chip: `tail_s` workgroups share the K of each (1: whole tiles only),
+  // with fp32 partials in tail_ws (a tile for each) and 8 counters per tile in tail_cnt (zero between launches)
   float* tail_ws; int* tail_cnt;
   int tail_s;
 };
 
-// of a round; tail_ws holds a 256 x 256 fp32 partial for each
+// of a round
 constexpr size_t GEMM_TAIL_WGS = 256;
 
 // 256x256 fp8 tile (gemm256.hip): A and W hold OCP e4m3 bytes (lda / K in elements = bytes),
@@ -48,4 +48,4 @@ int launch_gemm8p(const GemmArgs& a, int epi, hipStream_t s, int bm = 256);
 // four-wave 256x256 kernel (gemm4w.hip, 128x128 per wave; the tile-13 A/B arm), bf16, no EPI_ROPE
 int launch_gemm4w(const GemmArgs& a, int epi, hipStream_t s);
 // row-tile height (128 / 256) for a non-RoPE prefill product of M x N (gemm8p.hip)
-int gemm8p_pick_bm(int M, int N, int K, bool tail);
+int gemm8p_pick_bm(int M, int N, int K, int epi);

@@ -909,7 +909,7 @@ DA_EXPORT int da_gemm_bf16(const void* A, int lda, const void* W, void* C, int l
   a.bias = (const bf16_t*)bias; a.resid = (const bf16_t*)resid; a.ws = (float*)ws;
   a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc; a.ldr = ldr; a.k_per_split = K / splits;
   a.gamma = (const bf16_t*)rms_gamma; a.eps = rms_eps; a.relu = relu;
-  if (tail_ws && tail_cnt && epi != EPI_GELU) { a.tail_ws = (float*)tail_ws; a.tail_cnt = (int*)tail_cnt; }
+  if (tail_ws && tail_cnt) { a.tail_ws = (float*)tail_ws; a.tail_cnt = (int*)tail_cnt; }
   if ((rms_gamma || rms_eps > 0.f) && tile != 6) return (int)hipErrorInvalidValue;  // fused RMSNorm: GEMV only
   if (tile == 0) {
     // decode-sized M: 32x128 / weight-streaming tiles (+ split-K, chosen by the caller), to 639 rows;
@@ -918,7 +918,7 @@ DA_EXPORT int da_gemm_bf16(const void* A, int lda, const void* W, void* C, int l
     if (M <= 32) tile = 3;
     else if (M < 640 || splits > 1) tile = 2;
     else if (K < 128) tile = 1;
-    else tile = gemm8p_pick_bm(M, N, K, a.tail_ws != nullptr) == 256 ? 7 : 10;
+    else tile = gemm8p_pick_bm(M, N, K, epi) == 256 ? 7 : 10;
   }
   if (tile == 4 || tile == 7 || tile == 10) {
     if (splits != 1 || K < 128) return (int)hipErrorInvalidValue;

@@ -34,8 +34,9 @@
 //  * PERSIST: one workgroup per CU walks tile ids b, b + G, ... (G a multiple of 8: each id stays on
 //    the workgroup's XCD); the staged rows go to registers, then the next tile's prologue DMA is
 //    issued before this tile's stores (profiles/r5/gemm_persist/: +0.3..1 %, not for EPI_ROPE).
-//  * Tail: the tiles behind the last whole round of the chip (all of them, when they fill none) are each cut along K
-//    for tail_s workgroups, as many as the chip has room for. A workgroup leaves its fp32 partial in tail_ws, counts
+//  * TAIL: the tiles behind the last whole round of the chip (all of them, when they fill none) are each cut along K
+//    for tail_s workgroups: 2, 4 or 8 of those that fit beside each other, with at least 4 K-tiles each, by the lowest
+//    estimate (tail_slices; a product for which none is below whole tiles is not cut). A workgroup leaves its fp32 partial in tail_ws, counts
 //    itself in on a counter, and the second of two to come adds the other's to its own, pair by pair in a fixed tree (so
 //    the result does not depend on who came when); who is left runs the epilogue. Nothing waits: no workgroup depends on another one running.
 #include "gemm.h"
@@ -317,7 +318,7 @@ gemm8p_kernel(GemmArgs p) {
         const int ft = wid * 64 + fresh_lane();
         const unsigned at = ft * 16u;
         const __amdgpu_buffer_rsrc_t rst =
-            __builtin_amdgcn_make_buffer_rsrc((void*)p.tail_ws, (short)0, (int)(GEMM_TAIL_WGS * 65536 * 4), 0x00020000);
+            __builtin_amdgcn_make_buffer_rsrc((void*)p.tail_ws, (short)0, rest * p.tail_s * NF * 8192, 0x00020000);
         int node = t * 8, half = p.tail_s / 2;  // the level's first counter, its meetings
         for (int sl = unit >> 16, level = 0; half > 0; ++level, sl >>= 1, node += half, half >>= 1) {
           const unsigned own = (t * p.tail_s + (sl << level)) * (unsigned)(NF * 8192);
@@ -589,12 +590,16 @@ static bool persist_on() {
 }
 
 // on = 0 / 1 sets the persistent tile loop off / on for later launches, -1 only queries; returns
-// the previous setting (tests run one product both ways and compare bit for bit)
+// the previous setting (tests run one product both ways: bit for bit the same where no round is shared, which only the
+// persistent form does)
 DA_EXPORT int da_gemm8p_persist(int on) {
   const int prev = persist_on() ? 1 : 0;
   if (on == 0 || on == 1) g_persist = on;
   return prev;
 }
+
+// (GELU's registers and RoPE's per-row state leave the tail's no room)
+static bool tail_allowed(int epi) { return epi != EPI_GELU && epi != EPI_ROPE && persist_on(); }
 
 // What the last round takes with `sl` workgroups per tile (1: whole tiles), in hundredths of a K-tile of bm rows: the
 // longer slice's K-tiles, and for each meeting what writing and reading the partials was measured to take, which grows
@@ -631,7 +636,7 @@ static void launch8p_epi(const GemmArgs& a0, int ntiles, hipStream_t s) {
   // 256 VGPRs, and the persistent QKV projection measured 4 % slower, profiles/r5/gemm_persist/)
   if constexpr (EPI != EPI_ROPE) {
     if constexpr (EPI != EPI_GELU) {
-      a.tail_s = persist_on() && a.tail_ws ? tail_slices(ntiles, a.K / 64, BM) : 1;
+      a.tail_s = tail_allowed(EPI) && a.tail_ws ? tail_slices(ntiles, a.K / 64, BM) : 1;
       const int rest = ntiles % (int)GEMM_TAIL_WGS;
       if (a.tail_s > 1) {
         const int grid = ntiles >= (int)GEMM_TAIL_WGS ? (int)GEMM_TAIL_WGS : a.tail_s * ((rest + 7) & ~7);
@@ -683,7 +688,8 @@ static int launch8p(const GemmArgs& a0, int epi, hipStream_t s) {
 // (M ~ 64k) keep 256 (the round-3 rule, 256 rows once the 256-row grid reached half the chip,
 // measured 65.5 vs 74.9 us per O projection at M ~ 2.6k: profiles/r4/bm_rule/).
 // A tail (tail_slices) costs its slices' K-tiles and meetings, and has to be 5 % better than the other height.
-int gemm8p_pick_bm(int M, int N, int K, bool tail) {
+int gemm8p_pick_bm(int M, int N, int K, int epi) {
+  const bool tail = tail_allowed(epi);
   const int ntn = (N + 255) / 256, cus = num_cus(), nk = K / 64;
   auto cost = [&](int bm, int per_ktile) {
     const long t = (long)((M + bm - 1) / bm) * ntn;
@@ -693,13 +699,22 @@ int gemm8p_pick_bm(int M, int N, int K, bool tail) {
   return cost(128, 72) < cost(256, 100) ? 128 : 256;
 }
 
-// Whether a product that is handed scratch (tail_ws, tail_cnt) uses it: its counters have to be zero then. tile: 0, or
-// the row-tile height's code (4 / 7: 256, 10: 128).
-DA_EXPORT int da_gemm_tail_used(int M, int N, int K, int epi, int tile) {
-  if (epi == EPI_GELU || epi == EPI_ROPE || K < 128 || !persist_on()) return 0;
-  const int bm = tile == 10 ? 128 : tile ? 256 : gemm8p_pick_bm(M, N, K, true);
+// Bytes of partials that a product's shared last round needs (tail_ws; tail_cnt holds 256 * 8 counters), 0: it has none
+// and takes no scratch. tile: 0, or the row-tile height's code (4 / 7: 256, 10: 128).
+DA_EXPORT size_t da_gemm_tail_ws(int M, int N, int K, int epi, int tile) {
+  if (M < 1 || N < 1 || K < 128 || !tail_allowed(epi)) return 0;
+  const int bm = tile == 10 ? 128 : tile ? 256 : gemm8p_pick_bm(M, N, K, epi);
   const long nt = (long)((M + bm - 1) / bm) * ((N + BN - 1) / BN);
-  return nt < 0x7fffffff && tail_slices((int)nt, K / 64, bm) > 1;
+  const int s = nt < 0x7fffffff ? tail_slices((int)nt, K / 64, bm) : 1;
+  return s > 1 ? (size_t)(nt % (long)GEMM_TAIL_WGS) * s * bm * BN * 4 : 0;
+}
+
+// Which capture a stream is in (0: none).
+DA_EXPORT size_t da_gemm_capture_id(void* stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo((hipStream_t)stream, &st, &id) != hipSuccess) return 0;
+  return st == hipStreamCaptureStatusActive ? (size_t)id : 0;
 }
 
 // epi + 100: the same kernel on fp16 operands / output (v_mfma_f32_16x16x32_f16)
@@ -723,6 +738,6 @@ DA_EXPORT int da_gemm_f16(const void* A, int lda, const void* W, void* C, int ld
   a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = (bf16_t*)C;
   a.bias = (const bf16_t*)bias; a.resid = (const bf16_t*)resid;
   a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc; a.ldr = ldr; a.k_per_split = K;
-  if (tail_ws && tail_cnt && epi != EPI_GELU) { a.tail_ws = (float*)tail_ws; a.tail_cnt = (int*)tail_cnt; }
-  return launch_gemm8p(a, 100 + epi, (hipStream_t)stream, gemm8p_pick_bm(M, N, K, a.tail_ws != nullptr));
+  if (tail_ws && tail_cnt) { a.tail_ws = (float*)tail_ws; a.tail_cnt = (int*)tail_cnt; }
+  return launch_gemm8p(a, 100 + epi, (hipStream_t)stream, gemm8p_pick_bm(M, N, K, epi));
 }

@@ -62,7 +62,8 @@ _SIGS = {
     "da_gemm_dk_parts": [c_int],
     "da_enc_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5
                   + [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_void_p],
-    "da_gemm_tail_used": [c_int] * 5,
+    "da_gemm_tail_ws": [c_int] * 5,
+    "da_gemm_capture_id": [c_void_p],
     "da_gemm_dk_splitk": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                           c_int, c_void_p, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_void_p],
     "da_decode_attn": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
@@ -153,7 +154,7 @@ def load_part(part: str) -> None:
             if _part_of(name) == part:
                 fn = getattr(L, name)
                 fn.argtypes = argt
-                fn.restype = c_size_t if name.endswith("_ws") else c_int
+                fn.restype = c_size_t if name.endswith(("_ws", "_capture_id")) else c_int
                 _LIB.__dict__[name] = fn
         _LOADED[part] = L
 
@@ -235,30 +236,41 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
     return buf
 
 
-# Scratch of the prefill products' last round (csrc/gemm8p.hip, "Tail"): 256 workgroups' fp32 partials and their tiles'
-# counters, 64 MB, per stream: streams run products beside each other. At most TAIL_STREAMS of them per device keep one
-# (never given back: the caching allocator would hand the memory to kernels that may still run beside it).
-TAIL_STREAMS = 8
-_TAIL: dict = {}
+# The prefill products' shared last round (csrc/gemm8p.hip, TAIL) needs fp32 partials, up to 64 MB, and its tiles' counters,
+# 8 KB that are zero between launches. The partials are the call's own: the caching allocator hands a stream the same block
+# for each product and has it back in between. The counters stay, so that no launch has to clear them: a set per stream
+# (streams run products beside each other) for the TAIL_STREAMS latest streams, and in a capture one per capture and
+# stream, cleared by a node in front of its first such product.
+TAIL_STREAMS = 32
+TAIL_MIN_K = 768  # no round of a shorter product is shared (csrc/gemm8p.hip, tail_cost)
+_TAIL: dict = {}  # (device, stream) -> counters, oldest first
+_TAIL_CAPTURED: dict = {}  # (device, stream) -> (capture, counters): kept until the stream's next capture
 
 
 def _gemm_tail(device, stream: int, M: int, N: int, K: int, epi: int, tile: int = 0):
-    """(partials, counters) for a product on the current stream ``stream``; the caller holds them until it is launched.
-    Streams beyond TAIL_STREAMS and captured products (a graph may be replayed on another stream) have them for the one
-    call, the counters cleared by a launch: the sums are the same everywhere, in the same order."""
-    if not torch.cuda.is_current_stream_capturing():
-        key = (device.index, stream)
-        bufs = _TAIL.get(key)
-        if bufs is None:
-            with _LOCK:
-                bufs = _TAIL.get(key)
-                if bufs is None and sum(k[0] == device.index for k in _TAIL) < TAIL_STREAMS:
-                    bufs = _TAIL[key] = (torch.empty(256 * 256 * 256, dtype=torch.float32, device=device),
-                                         torch.zeros(256 * 8, dtype=torch.int32, device=device))
-        if bufs is not None:
-            return bufs
-    make = torch.zeros if lib().da_gemm_tail_used(M, N, K, epi, tile) else torch.empty
-    return torch.empty(256 * 256 * 256, dtype=torch.float32, device=device), make(256 * 8, dtype=torch.int32, device=device)
+    """(partials, counters) of a product on the current stream ``stream`` whose last round is shared, (None, None) of
+    others; the caller holds them until it is launched. A set of counters that makes room for another stream's goes back to
+    the allocator, which keeps it for the stream that used it: in order."""
+    nbytes = lib().da_gemm_tail_ws(M, N, K, epi, tile) if K >= TAIL_MIN_K else 0
+    if not nbytes:
+        return None, None
+    part = torch.empty(nbytes // 4, dtype=torch.float32, device=device)
+    key = (device.index, stream)
+    if torch.cuda.is_current_stream_capturing():
+        capture = lib().da_gemm_capture_id(stream)
+        had, cnt = _TAIL_CAPTURED.get(key, (0, None))
+        if had != capture:
+            cnt = torch.zeros(256 * 8, dtype=torch.int32, device=device)
+            _TAIL_CAPTURED[key] = capture, cnt
+        return part, cnt
+    cnt = _TAIL.get(key)
+    if cnt is None:
+        cnt = torch.zeros(256 * 8, dtype=torch.int32, device=device)
+        with _LOCK:
+            cnt = _TAIL.setdefault(key, cnt)
+            while len(_TAIL) > TAIL_STREAMS:
+                del _TAIL[next(iter(_TAIL))]
+    return part, cnt
 
 
 def gemv_fusable(M: int, N: int, K: int, epi: int = EPI_NONE) -> bool:

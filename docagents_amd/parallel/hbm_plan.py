@@ -12,6 +12,9 @@ Every term is the allocation the code makes, by the formula it makes it with:
   decode workspace    ``Generator.workspace_bytes`` (split-K / split-KV partials)
   prefill transient   one ``max_prefill_tokens`` chunk of activations (x, h, qkv, attention out,
                       gate/up out) — freed between chunks, counted once
+  product partials    the shared last round of the prefill products (``kernels._gemm_tail``): at most
+                      TAIL_BYTES for each stream that runs them (answers, summaries, the embedder's
+                      two lanes)
   index shard         ``FlatIndex``: rows x (dim bf16 + slot int32 + id int64), built at exactly ``rows``;
                       with ingest the first add grows it 1.5x and the copy holds old + new: +1.5x in
                       the headline, +0.5x after it (config 4 at 1.25M x 1024 peaked 3.3 GB over a
@@ -38,6 +41,8 @@ HBM_BYTES = 288 * GB
 PLAN_LIMIT_BYTES = 270 * GB  # what a phase may hold: the rest is the runtime, RCCL and fragmentation
 MAX_PREFILL_TOKENS = 65536   # Generator.max_prefill_tokens default
 RUNTIME_BYTES = 2 * GB       # graph pools, tables, small buffers, allocator rounding (every phase)
+TAIL_BYTES = 256 * 256 * 256 * 4 + 8192  # 256 workgroups' fp32 partials and their tiles' counters
+TAIL_LANES = 4               # streams that run prefill products
 TP70B_BATCHES = (1, 16)      # tp_decode_70b: decode batches timed
 TP70B_WORLD = 8              # tp_decode_70b runs at N = 8 (Llama-3-70B TP=8)
 
@@ -132,6 +137,7 @@ def bench_plan(a: BenchArgs, world: int, release_engine_kv: bool = True) -> dict
         "encoder": encoder_bytes(enc, a.enc_dtype),
         "decoder_weights": decoder_weight_bytes(dec, tp),
         "index": index_bytes(a.index_rows, enc.hidden),
+        "product_partials": TAIL_LANES * TAIL_BYTES,
     }
     engine_kv = kv_bytes(dec, slots, eng_seq, tp)
     phases: dict = {}

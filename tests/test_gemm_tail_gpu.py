@@ -89,3 +89,89 @@ def test_tail_streams():
         torch.cuda.synchronize()
         assert all(torch.equal(x, first) for x in captured)
         assert torch.equal(K.gemm(a, w, tile=7), first)
+
+
+# (M, N, K, tile height's code) -> tiles behind the whole rounds, slices of each; None: left whole
+@pytest.mark.parametrize("M,N,Kd,tile,cut", [
+    (700, 768, 2048, 7, (9, 4)), (256, 256, 4096, 7, (1, 8)), (1000, 768, 8192, 7, (12, 8)), (6244, 3072, 2048, 7, (44, 2)),
+    (700, 776, 64 * 33, 7, (12, 4)), (1000, 520, 2048, 10, (24, 4)), (700, 768, 1024, 7, None), (4096, 4096, 1024, 7, None)])
+@pytest.mark.parametrize("epi", [K.EPI_NONE, K.EPI_GELU, K.EPI_RESID, K.EPI_SWIGLU])
+def test_which_rounds_are_cut(M, N, Kd, tile, cut, epi):
+    """A product takes scratch for as many partials as it leaves, and none where its tiles stay whole. GELU's always do."""
+    height = 128 if tile == 10 else 256
+    want = 0 if cut is None or epi == K.EPI_GELU else cut[0] * cut[1] * height * 256 * 4
+    assert K.lib().da_gemm_tail_ws(M, N, Kd, epi, tile) == want
+    if epi == K.EPI_SWIGLU and N % 32:
+        return
+    a, w, _, resid = _operands(M, N, Kd, torch.bfloat16, M)
+    stream = torch.cuda.current_stream().cuda_stream
+    part, cnt = K._gemm_tail(a.device, stream, M, N, Kd, epi, tile)
+    assert (part is None and cnt is None) if not want else part.numel() * 4 == want
+    got = K.gemm(a, w, epi=epi, tile=tile, resid=resid if epi == K.EPI_RESID else None)
+    if cnt is not None:
+        assert int(cnt.abs().max()) == 0  # back at zero
+    if epi == K.EPI_NONE:
+        ref = a.double() @ w.double().T
+        assert float((got.double() - ref).norm() / ref.norm()) < 2.0 ** -8
+
+
+def test_short_products_are_never_cut():
+    for Kd in range(128, K.TAIL_MIN_K, 64):
+        for M in (256, 700, 1000, 2720, 2797, 3000, 5415, 6244, 24105):
+            for N in (256, 768, 1024, 2304, 3072, 4096):
+                for tile in (0, 7, 10):
+                    assert K.lib().da_gemm_tail_ws(M, N, Kd, K.EPI_NONE, tile) == 0
+
+
+def test_scratch_is_given_back():
+    """Neither a stream that runs a product once nor a whole product keeps partials; a capture has one set of counters,
+    cleared once, and they are its own."""
+    a, w, _, _ = _operands(700, 768, 2048, torch.bfloat16, 3)
+    nbytes = K.lib().da_gemm_tail_ws(700, 768, 2048, K.EPI_NONE, 7)
+    assert nbytes == 9 * 4 * 256 * 256 * 4
+    out = torch.empty(700, 768, dtype=torch.bfloat16, device=DEV)
+    first = K.gemm(a, w, tile=7)
+    streams = [torch.cuda.Stream() for _ in range(6)]
+    torch.cuda.synchronize()
+    held = torch.cuda.memory_allocated()
+    for s in streams:
+        with torch.cuda.stream(s):
+            K.gemm(a, w, tile=7, out=out)
+        torch.cuda.synchronize()
+    assert torch.cuda.memory_allocated() - held <= 6 * 256 * 8 * 4
+    assert torch.equal(out, first)
+    side = torch.cuda.Stream()
+    graphs = []
+    for n in (3, 2):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side):
+            ys = [K.gemm(a, w, tile=7) for _ in range(n)]
+            cnt = K._TAIL_CAPTURED[torch.device(DEV, 0).index, side.cuda_stream][1]
+        graphs.append((g, ys, cnt))
+    assert graphs[0][2] is not graphs[1][2]
+    for _ in range(3):
+        for g, ys, cnt in graphs:
+            cnt.fill_(1)  # (whatever lies there: the graph's own node clears it)
+            for y in ys:
+                y.zero_()
+            g.replay()
+            K.gemm(a, w, tile=7, out=out)
+            torch.cuda.synchronize()
+            assert all(torch.equal(y, first) for y in ys) and torch.equal(out, first)
+
+
+def test_more_streams_than_counters(monkeypatch):
+    """Counters that make room for another stream's while their product may still run."""
+    monkeypatch.setattr(K, "TAIL_STREAMS", 2)
+    monkeypatch.setattr(K, "_TAIL", {})
+    a, w, _, _ = _operands(700, 768, 2048, torch.bfloat16, 4)
+    first = K.gemm(a, w, tile=7)
+    streams = [torch.cuda.Stream() for _ in range(5)]
+    torch.cuda.synchronize()
+    out = []
+    for _ in range(6):
+        for s in streams:
+            with torch.cuda.stream(s):
+                out.append(K.gemm(a, w, tile=7))
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, first) for x in out) and len(K._TAIL) == 2

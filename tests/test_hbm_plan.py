@@ -76,3 +76,9 @@ def test_index_growth_and_runtime_cover_the_measured_config4_peak():
     assert HP.check(HP.bench_plan(a, 1)) == []
     q = HP.bench_plan(HP.BenchArgs(enc="bge-large", enc_dtype="fp16", index_rows=1_250_000, ingest=False), 1)
     assert "index_growth" not in q["headline"]
+
+
+def test_every_phase_counts_the_products_partials():
+    """The shared last round of the prefill products takes up to 64 MB a stream, whatever the phase."""
+    for phase in HP.bench_plan(HP.BenchArgs(), 8).values():
+        assert phase["product_partials"] == HP.TAIL_LANES * (256 * 256 * 256 * 4 + 256 * 8 * 4)
