@@ -108,13 +108,17 @@ class FlatIndex:
         ids[:self.n] = self.ids[:self.n]
         ids_t = torch.zeros(new, dtype=torch.int64, device=self.device)
         ids_t[:self.n] = self.ids_t[:self.n]
-        if self.device.type == "cuda":
-            # the copies above read the old buffers on this stream: the allocator must not hand
-            # them out again (to an allocation on their own stream) before those copies ran
-            st = torch.cuda.current_stream(self.device)
-            for old in (self.X, self.slots_t, self.ids_t):
-                old.record_stream(st)
+        self._retire(self.X, self.slots_t, self.ids_t)  # (the copies above read them on this stream)
         self.X, self.slots_t, self.ids, self.ids_t = X, s, ids, ids_t
+
+    def _retire(self, *old) -> None:
+        """Tensors that a write replaces: the allocator must not hand them out again (to an allocation on their own stream)
+        before what this stream has read of them, and the reads that it waited for, have run."""
+        if self.device.type == "cuda":
+            st = torch.cuda.current_stream(self.device)
+            for t in old:
+                if t is not None:
+                    t.record_stream(st)
 
     def doc_slot(self, doc_id: str) -> int:
         e = self.docs.get(doc_id)

@@ -40,6 +40,7 @@ class IVFFlatIndex(FlatIndex):
         self.most_rows = None   # np int64 [lists + 1]: rows of the p longest lists together
 
     def _set_lists(self, list_off: np.ndarray) -> None:
+        self._retire(self.list_off_t)  # (searches on other streams may still walk it)
         self.list_off = list_off
         self.list_off_t = h2d(list_off.astype(np.int32), self.device)
         self.most_rows = np.concatenate([[0], np.cumsum(np.sort(np.diff(list_off))[::-1])])
@@ -76,6 +77,7 @@ class IVFFlatIndex(FlatIndex):
                 Xs = X.index_select(0, torch.from_numpy(rng.choice(n, sample, replace=False)).to(self.device))
             else:
                 Xs = X
+            self._retire(self.centroids)
             self.centroids = self._kmeans(Xs.contiguous(), iters)
             self._build_lists()
             return True
