@@ -1181,7 +1181,7 @@ def gather_ids(rows, ids):
     _req(rows.is_cuda, "rows must be on GPU")
     _req(ids.is_cuda and ids.dtype == torch.int64 and ids.is_contiguous() and ids.dim() == 1, "ids must be int64 [N]")
     if rows.dtype != torch.int32:
-        rows = rows.clamp(-1, 2**31 - 1).int()
+        rows = rows.long().clamp(-1, 2**31 - 1).int()
     rows = rows.contiguous()
     out = torch.empty(rows.shape, dtype=torch.int64, device=rows.device)
     _check(lib().da_gather_ids(_ptr(rows), rows.numel(), _ptr(ids), ids.numel(), _ptr(out), _stream()), "gather_ids")
