@@ -445,14 +445,19 @@ def gemm_ln(a, w, bias, epi: int = EPI_BIAS, norm=None, resid=None, st_out=None)
     M, K = a.shape
     N = w.shape[0]
     _req(gemm_ln_fit(M, K if epi != EPI_RESID else N, N if epi != EPI_RESID else K) and w.shape[1] == K
-         and bias.shape == (N,), f"gemm_ln shape M={M} N={N} K={K}")
+         and bias.shape == (N,) and bias.is_contiguous(), f"gemm_ln shape M={M} N={N} K={K}")
     _req(a.stride(1) == 1 and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.is_contiguous()
          and w.data_ptr() % 16 == 0, "gemm_ln layout")
     _req(epi == EPI_BIAS or (epi == EPI_GELU and norm is not None) or (epi == EPI_RESID and st_out is not None),
          "gemm_ln epilogue")
     st, g, b, eps = norm or (None, None, None, 0.0)
     for t in (st, st_out):
-        _req(t is None or (t.dtype == torch.float32 and t.shape == (64, 64, 2) and t.is_contiguous()), "bad statistics")
+        _req(t is None or (t.is_cuda and t.dtype == torch.float32 and t.shape == (64, 64, 2) and t.is_contiguous()),
+             "bad statistics")
+    if norm is not None:
+        for t in (g, b):
+            is_cuda(t, "norm")
+            _req(t.shape == (N if epi == EPI_RESID else K,) and t.is_contiguous(), "norm must be [columns]")
     if epi == EPI_RESID:
         is_cuda(resid, "resid")
         _req(resid.shape == (M, N) and resid.stride(1) == 1 and resid.stride(0) % 8 == 0, "bad resid")

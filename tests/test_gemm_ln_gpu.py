@@ -47,3 +47,20 @@ def test_gemm_ln(M, h, f, dt):
     assert torch.allclose(d(st2[:M, :h // 16, 0]), mean, rtol=0, atol=2.0 ** -22 * float(parts.abs().max()))
     dev = (parts - mean[..., None]).square().sum(-1)
     assert torch.allclose(d(st2[:M, :h // 16, 1]), dev, rtol=1e-5, atol=1e-5 * float(dev.max()))
+
+
+def test_what_the_product_refuses():
+    """Operands that the kernel would read at other places than the caller's."""
+    M, h = 8, 128
+    t = lambda *s: torch.ones(s, device="cuda", dtype=torch.bfloat16)  # noqa: E731
+    a, w, b, v = t(M, h), t(h, h), t(h), t(h)
+    st, st2 = torch.zeros((2, 64, 64, 2), device="cuda")
+    K.gemm_ln(a, w, b, norm=(st, v, v, 1e-5))
+    for bias, norm in [(t(2 * h)[::2], None), (b, (st, t(2 * h)[::2], v, 1e-5)), (b, (st, v, t(h // 2), 1e-5)),
+                       (b, (st, v.float(), v, 1e-5)), (b, (st.cpu(), v, v, 1e-5)), (b, (st[:32], v, v, 1e-5))]:
+        with pytest.raises(ValueError):
+            K.gemm_ln(a, w, bias, norm=norm)
+        with pytest.raises(ValueError):
+            K.gemm_ln(a, w, bias, K.EPI_RESID, norm=norm, resid=a, st_out=st2)
+    with pytest.raises(ValueError):
+        K.gemm_ln(a, w, b, K.EPI_RESID, resid=a, st_out=st2[:, :32])
