@@ -1158,10 +1158,12 @@ def _ranges(X, Qv, ranges, range_off, lists, K, thr, max_rows, slots, bitmap, ro
         _req(slots is not None, "bitmap needs slots")
         _req(bitmap.dtype == torch.int32 and bitmap.shape[0] == Q, "bitmap")
         W = bitmap.shape[1]
-    splits = max(1, math.ceil(max_rows / rows_per_split))
-    ws = _workspace(splits * Q * K * 8, X.device)
     out_s = torch.empty((Q, K), dtype=torch.float32, device=X.device)
     out_i = torch.empty((Q, K), dtype=torch.int32, device=X.device)
+    if Q == 0:
+        return out_s, out_i
+    splits = max(1, math.ceil(max_rows / rows_per_split))
+    ws = _workspace(splits * Q * K * 8, X.device)
     _check(lib().da_topk_ranges(_ptr(X), d, _ptr(slots), _ptr(Qv), Q, _ptr(ranges), _ptr(range_off), _ptr(lists),
                                 0 if lists is None else lists.shape[1], _ptr(bitmap),
                                 W, float(thr), K, splits, rows_per_split, _ptr(ws), _ptr(out_s), _ptr(out_i),

@@ -28,3 +28,91 @@ def test_gather_ids(dtype):
     assert K.gather_ids(rt, ids[:0]).tolist() == [-1] * len(rows)
     assert K.gather_ids(rt[:0], ids).shape == (0,)
     assert K.gather_ids(torch.arange(1000, dtype=torch.int32, device=DEV), ids).tolist() == ids.tolist() + [-1] * 700
+
+
+LENGTHS = [0, 1, 64, 65, 4200, 0, 130, 63, 700, 1]
+
+
+def _check(s, i, dots, named, Kk, tol):
+    """Scores and rows of one query against every row that it names (dots: 64-bit scores)."""
+    named = torch.tensor(named, dtype=torch.long)
+    want = dots[named].sort(descending=True).values[:Kk]
+    n = len(want)
+    assert i[n:].tolist() == [-1] * (Kk - n) and bool((s[n:] == -float("inf")).all())
+    got = i[:n].long()
+    assert got.unique().numel() == n and bool(torch.isin(got, named).all())
+    assert torch.allclose(s[:n].double(), want, rtol=0, atol=tol)
+    assert torch.allclose(s[:n].double(), dots[got], rtol=0, atol=tol)
+
+
+@pytest.mark.parametrize("d,Kk", [(128, 5), (768, 32), (1024, 1)])
+@pytest.mark.parametrize("mean_rows", [1, 500, 5300])
+def test_topk_lists(d, Kk, mean_rows):
+    """Empty lists, lists of a step of the kernel and one row more, one much longer than all others, places that name no
+    list, queries of different lists and of none, splits that end inside a later list; with removed rows and a filter; the
+    expected count of rows, which only shapes the launch, wrong by far in both directions."""
+    torch.manual_seed(d + mean_rows)
+    off = torch.tensor([0] + LENGTHS).cumsum(0)
+    N = int(off[-1])
+    X = torch.nn.functional.normalize(torch.randn(N, d, device=DEV), dim=-1).bfloat16()
+    lists = [[0, 1, 2, 3], [4, -1, 6, 8], [-1, -1, -1, -1], [9, 3, 4, 7], [-1, 5, 0, -1], [8, 4, 2, 6], [1, -1, 9, -1]]
+    Q = len(lists)
+    Qv = torch.nn.functional.normalize(torch.randn(Q, d, device=DEV), dim=-1).bfloat16()
+    lt, ot = torch.tensor(lists, dtype=torch.int32, device=DEV), off.int().to(DEV)
+    max_rows = int(sum(sorted(LENGTHS)[-4:]))
+    slots = (torch.arange(N, device=DEV, dtype=torch.int32) // 4).contiguous()
+    slots[::5] = -1
+    bitmap = torch.randint(-2 ** 31, 2 ** 31 - 1, (Q, N // 128 + 1), device=DEV, dtype=torch.int32)
+    dots = Qv.double().cpu() @ X.double().cpu().T
+    sc, bc = slots.long().cpu(), bitmap.cpu()
+    for sl, bm in ((None, None), (slots, None), (slots, bitmap)):
+        s, i = K.topk_lists(X, Qv, lt, ot, Kk, -1.0, mean_rows=mean_rows, max_rows=max_rows, slots=sl, bitmap=bm)
+        for q in range(Q):
+            named = [r for x in lists[q] if x >= 0 for r in range(int(off[x]), int(off[x + 1]))]
+            if sl is not None:
+                named = [r for r in named if sc[r] >= 0]
+            if bm is not None:
+                named = [r for r in named if (int(bc[q, sc[r] >> 5]) >> (int(sc[r]) & 31)) & 1]
+            _check(s[q].cpu(), i[q].cpu(), dots[q], named, Kk, d * 2.0 ** -23)
+    s, i = K.topk_lists(X, Qv[:0], lt[:0], ot, Kk, -1.0, mean_rows=mean_rows, max_rows=max_rows)
+    assert s.shape == i.shape == (0, Kk)
+
+
+@pytest.mark.parametrize("probes", [1, 33, 200])
+def test_many_lists(probes):
+    """More lists named than a wave has lanes; every list empty but one; a threshold that most rows miss."""
+    torch.manual_seed(probes)
+    L, d, Q, Kk = 400, 384, 5, 7
+    n = torch.randint(0, 90, (L,))
+    off = torch.cat([torch.zeros(1, dtype=torch.long), n.cumsum(0)])
+    N = int(off[-1])
+    X = torch.nn.functional.normalize(torch.randn(N, d, device=DEV), dim=-1).bfloat16()
+    Qv = torch.nn.functional.normalize(torch.randn(Q, d, device=DEV), dim=-1).bfloat16()
+    lt = torch.stack([torch.randperm(L)[:probes] for _ in range(Q)]).int()
+    dots = Qv.double().cpu() @ X.double().cpu().T
+    longest = int(n.sort(descending=True).values[:probes].sum())
+    for thr in (-1.0, 0.1):
+        s, i = K.topk_lists(X, Qv, lt.to(DEV), off.int().to(DEV), Kk, thr, mean_rows=-(-probes * N // L), max_rows=longest)
+        for q in range(Q):
+            named = [r for x in lt[q].tolist() for r in range(int(off[x]), int(off[x + 1])) if dots[q, r] >= thr]
+            _check(s[q].cpu(), i[q].cpu(), dots[q], named, Kk, d * 2.0 ** -23)
+    one = torch.zeros(L + 1, dtype=torch.long)
+    one[L // 2 + 1:] = N
+    s, i = K.topk_lists(X, Qv, lt.to(DEV), one.int().to(DEV), Kk, -1.0, mean_rows=1, max_rows=N)
+    for q in range(Q):
+        _check(s[q].cpu(), i[q].cpu(), dots[q], list(range(N)) if L // 2 in lt[q].tolist() else [], Kk, d * 2.0 ** -23)
+
+
+def test_index_without_questions():
+    """A batch that holds no question, before and after training, with rows added since and with a filter."""
+    from docagents_amd.index import make_index
+    index = make_index("ivfflat", 384, DEV, lists=4, probes=2)
+    g = torch.Generator().manual_seed(1)
+    for n in (40, 5):
+        x = torch.nn.functional.normalize(torch.randn(n, 384, generator=g), dim=-1)
+        index.add(f"d{n}", torch.arange(n).numpy(), x)
+        if n == 40:
+            assert index.train(iters=1)
+        for filters in (None, []):
+            s, i = index.search(torch.empty(0, 384, device=DEV), 3, -1.0, filters)
+            assert s.shape == i.shape == (0, 3)
