@@ -17,11 +17,12 @@ def _operands(M, N, Kd, dtype, seed):
     return a, w, bias, torch.randn(M, N, device=DEV, generator=g).to(dtype)
 
 
-# tiles of 256 x 256: fewer than a round (9 in 4 slices, 1 in 8), a round and some (300, 5 slices), slices of unequal
-# length (33 K-tiles in 4), a last row and column tile that are not full; tiles of 128 rows; exactly a round (whole)
-@pytest.mark.parametrize("M,N,Kd,tile", [(700, 768, 1024, 7), (256, 256, 4096, 7), (6244, 3072, 2048, 7),
+# tiles of 256 x 256: fewer than a round (9 in 4 slices, 1 and 12 in 8), a round and some (300, the last 44 in 2), slices of
+# unequal length (33 K-tiles in 4), a last row and column tile that are not full; tiles of 128 rows; too short to be cut and
+# exactly a round (whole)
+@pytest.mark.parametrize("M,N,Kd,tile", [(700, 768, 2048, 7), (256, 256, 4096, 7), (1000, 768, 8192, 7), (6244, 3072, 2048, 7),
                                          (700, 776, 64 * 33, 7), (1000, 520, 2048, 10), (6400, 3072, 2048, 10),
-                                         (4096, 4096, 1024, 7)])
+                                         (700, 768, 1024, 7), (4096, 4096, 1024, 7)])
 @pytest.mark.parametrize("epi", [K.EPI_NONE, K.EPI_BIAS, K.EPI_GELU, K.EPI_RESID, K.EPI_SWIGLU])
 def test_tail(M, N, Kd, tile, epi, monkeypatch):
     a, w, bias, resid = _operands(M, N, Kd, torch.bfloat16, M + N)
@@ -29,6 +30,8 @@ def test_tail(M, N, Kd, tile, epi, monkeypatch):
         pytest.skip("gated products need whole groups")
     kw = dict(epi=epi, tile=tile, bias=None if epi in (K.EPI_NONE, K.EPI_SWIGLU) else bias,
               resid=resid if epi == K.EPI_RESID else None)
+    cut = K.lib().da_gemm_tail_ws(M, N, Kd, epi, tile) > 0
+    assert cut == (epi != K.EPI_GELU and Kd > 1024)  # (else both sides below are one kernel)
     got = K.gemm(a, w, **kw)
     again = [K.gemm(a, w, **kw) for _ in range(3)]  # the counters are back at zero, the sums in one order
     assert all(torch.equal(got, x) for x in again)
@@ -51,6 +54,7 @@ def test_tail(M, N, Kd, tile, epi, monkeypatch):
 
 @pytest.mark.parametrize("M,N,Kd", [(3000, 1024, 4096), (24105, 1024, 4096)])
 def test_tail_f16(M, N, Kd, monkeypatch):
+    assert K.lib().da_gemm_tail_ws(M, N, Kd, K.EPI_RESID, 0) > 0
     a, w, bias, resid = _operands(M, N, Kd, torch.float16, M)
     got = K.gemm_f16(a, w, bias=bias, epi=K.EPI_RESID, resid=resid)
     with monkeypatch.context() as m:

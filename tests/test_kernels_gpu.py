@@ -111,7 +111,8 @@ def test_gemm4w_tile(M, N, Kd, epi):
 def test_gemm8p_persistent(M, N, Kd, epi, tile):
     """More tiles than CUs: the persistent tile loop (workgroups running 1-3 tiles each, ragged M / N;
     K = 128 / 192 / 256 / 3072: every K-loop shape of the first K-tile whose counted waits let the
-    previous tile's stores fly) vs the fp32 reference, and bit-identical to one workgroup per tile."""
+    previous tile's stores fly) vs the fp32 reference, and bit-identical to one workgroup per tile (none
+    of these shares its last round along K, which only the persistent form does)."""
     torch.manual_seed(M + N + epi + tile)
     if epi == K.EPI_SWIGLU:
         N = (N // 32) * 32
@@ -119,6 +120,7 @@ def test_gemm8p_persistent(M, N, Kd, epi, tile):
     bias = _rand(N) if epi in (K.EPI_BIAS, K.EPI_GELU, K.EPI_RESID) else None
     resid = _rand(M, N) if epi == K.EPI_RESID else None
     prev = K.gemm8p_persist(1)
+    assert K.lib().da_gemm_tail_ws(M, N, Kd, epi, tile) == 0
     try:
         got = K.gemm(a, w, bias=bias, epi=epi, resid=resid, tile=tile, splits=1)
         K.gemm8p_persist(0)
