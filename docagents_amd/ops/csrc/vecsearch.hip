@@ -555,8 +555,34 @@ topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ 
   const int pbeg = split * rows_per_split, pend = pbeg + rows_per_split;
   __syncthreads();
   // walk the concatenated ranges; position p counts rows across this query's ranges
-  int pos = 0, buf = 0;
-  for (int r = rb; r < re; ++r) {
+  int pos = 0, buf = 0, r0 = rb;
+  if (pbeg > 0 && re - rb > 16) {
+    // to the range that this split begins in: 64 lengths a step and their sums (one range after another, each a load of its
+    // own that the next waits for, the last of 250 splits took 0.3 us for each of 2000 ranges)
+    for (; r0 < re; r0 += 64) {
+      const int r = min(r0 + lane, re - 1), l = lists ? lists[r] : 0;
+      const bool in = r0 + lane < re && l >= 0;
+      const int at = !in ? 0 : lists ? l : 2 * r;
+      const int len = ranges[at + 1] - ranges[at];
+      int sum = in ? len : 0;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int below = __shfl_up(sum, o, 64);
+        sum += lane >= o ? below : 0;
+      }
+      const unsigned long long past = __ballot(pos + sum > pbeg);
+      if (past) {
+        const int first = __builtin_ctzll(past);
+        pos += first ? __shfl(sum, first - 1, 64) : 0;
+        r0 += first;
+        break;
+      }
+      pos += __shfl(sum, 63, 64);
+    }
+    r0 = __builtin_amdgcn_readfirstlane(r0);
+    pos = __builtin_amdgcn_readfirstlane(pos);
+  }
+  for (int r = r0; r < re; ++r) {
     const int l = lists ? lists[r] : 0;
     if (l < 0) continue;
     const int s0 = ranges[lists ? l : 2 * r], s1 = ranges[lists ? l + 1 : 2 * r + 1];

@@ -103,6 +103,37 @@ def test_many_lists(probes):
         _check(s[q].cpu(), i[q].cpu(), dots[q], list(range(N)) if L // 2 in lt[q].tolist() else [], Kk, d * 2.0 ** -23)
 
 
+@pytest.mark.parametrize("count", [16, 17, 63, 64, 65, 128, 1000])
+@pytest.mark.parametrize("by_list", [False, True])
+def test_splits_that_begin_behind_many_ranges(count, by_list):
+    """A query's later splits find the range that they begin in by sums over 64 ranges a step: empty ranges, ranges that
+    end where a split begins, places that name no list, a query without rows beside ones with many."""
+    torch.manual_seed(count)
+    d, Q, Kk = 256, 3, 32
+    n = torch.randint(0, 12, (Q, count))
+    n[0, ::3] = 64  # (splits of 64 rows: some begin exactly at a range)
+    n[1, count // 2:] = 0
+    n[2] = 0
+    N = int(n.sum())
+    off = torch.cat([torch.zeros(1, dtype=torch.long), n.flatten().cumsum(0)])
+    X = torch.nn.functional.normalize(torch.randn(N, d, device=DEV), dim=-1).bfloat16()
+    Qv = torch.nn.functional.normalize(torch.randn(Q, d, device=DEV), dim=-1).bfloat16()
+    order = torch.stack([torch.randperm(count) for _ in range(Q)])
+    lists = torch.gather(torch.arange(Q * count).view(Q, count), 1, order)
+    most = int(n.sum(1).max())
+    if by_list:
+        lists[torch.rand(Q, count) < 0.2] = -1
+        s, i = K.topk_lists(X, Qv, lists.int().to(DEV), off.int().to(DEV), Kk, -1.0, mean_rows=1, max_rows=most)
+    else:
+        ranges = torch.stack([off[lists], off[lists + 1]], -1).view(-1, 2).int().to(DEV)
+        ro = (torch.arange(Q + 1) * count).int().to(DEV)
+        s, i = K.topk_ranges(X, Qv, ranges, ro, Kk, -1.0, max_rows=most, rows_per_split=64)
+    dots = Qv.double().cpu() @ X.double().cpu().T
+    for q in range(Q):
+        named = [r for x in lists[q].tolist() if x >= 0 for r in range(int(off[x]), int(off[x + 1]))]
+        _check(s[q].cpu(), i[q].cpu(), dots[q], named, Kk, d * 2.0 ** -23)
+
+
 def test_index_without_questions():
     """A batch that holds no question, before and after training, with rows added since and with a filter."""
     from docagents_amd.index import make_index
