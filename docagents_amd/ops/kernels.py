@@ -1078,6 +1078,15 @@ def sample_finalize(gathered, ranks: int, out_tok=None, out_lp=None, conf=None, 
 
 
 # --------------------------------------------------------------------------- vector search
+def _scan_rows(N: int) -> int:
+    """Rows of a wave in the streaming scan of up to 16 queries: 16 waves a CU over the chip (256 CUs), but at least 64 rows
+    each, with 256 workgroups of 4 waves where that leaves CUs idle (one tile of 16 rows each at least: a few hundred
+    centroids). More workgroups than CUs for less each are slower, us in 16 / 32 / 64 rows: 60000 x 1024, one query, 74.8 /
+    56.2 / 45.7 (16 queries 197 / 127 / 126); 30000 42.7 / 33.5 / 40.1; 16000 28.0 / 30.4 / 38.8; 512 x 384 15.1 / 16.9 / 20.5."""
+    tiles = lambda waves: math.ceil(N / waves / 16) * 16  # noqa: E731
+    return max(min(tiles(256 * 4), 64), tiles(256 * 16), 16)
+
+
 def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_block: int | None = None):
     """Exact top-K of Qv @ X^T per query with threshold and optional doc-slot bitmap [Q, W] int32."""
     _bf16_cuda(X, "X"); _bf16_cuda(Qv, "Qv")
@@ -1095,9 +1104,8 @@ def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_bloc
         W = bitmap.shape[1]
     if d in (384, 768, 1024) and rows_per_block is None and N > 0 and Q <= 256:
         # the streaming scan (search-sized batches over a big shard; k-means assignment, with the
-        # rows as the queries, keeps the query-major tiles below): ~16 waves of rows per CU over
-        # the chip (256 CUs), one tile of 16 rows each at least (a few hundred centroids)
-        rpw = max(16, math.ceil(N / (256 * 16) / 16) * 16)
+        # rows as the queries, keeps the query-major tiles below)
+        rpw = _scan_rows(N)
         ws = _workspace(int(lib().da_topk_stream_ws(N, Q, K, rpw)), X.device)
         out_s = torch.empty((Q, K), dtype=torch.float32, device=X.device)
         out_i = torch.empty((Q, K), dtype=torch.int32, device=X.device)
