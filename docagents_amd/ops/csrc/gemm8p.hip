@@ -35,7 +35,7 @@
 //    the workgroup's XCD); the staged rows go to registers, then the next tile's prologue DMA is
 //    issued before this tile's stores (profiles/r5/gemm_persist/: +0.3..1 %, not for EPI_ROPE).
 //  * TAIL: the tiles behind the last whole round of the chip (all of them, when they fill none) are each cut along K
-//    for tail_s workgroups: 2, 4 or 8 of those that fit beside each other, with at least 4 K-tiles each, by the lowest
+//    for tail_s workgroups: 2, 4 or 8 of those that fit beside each other, with at least 8 K-tiles each, by the lowest
 //    estimate (tail_slices; a product for which none is below whole tiles is not cut). A workgroup leaves its fp32 partial in tail_ws, counts
 //    itself in on a counter, and the second of two to come adds the other's to its own, pair by pair in a fixed tree (so
 //    the result does not depend on who came when); who is left runs the epilogue. Nothing waits: no workgroup depends on another one running.
@@ -603,27 +603,29 @@ static bool tail_allowed(int epi) { return epi != EPI_GELU && epi != EPI_ROPE &&
 
 // What the last round takes with `sl` workgroups per tile (1: whole tiles), in hundredths of a K-tile of bm rows: the
 // longer slice's K-tiles, and for each meeting what writing and reading the partials was measured to take, which grows
-// with the workgroups that write at once, more where the last whole round's stores are still under way. 5 % on top: a
-// close call stays whole.
+// with the workgroups that write at once. At the first the odd slice's sum is mostly there and one of the two is written;
+// at later ones nothing keeps the two apart. 2 % on top: a close call stays whole. From 4 to 384 tiles of both heights with
+// 16 - 128 K-tiles, uncut and in 2, 4 and 8 slices: the choice takes 1.003 times the fastest on average, 1.09 at worst, and
+// one of 228 is above uncut (1.04: 112 tiles of 256 rows, K 2048, where tiles of 128 rows are the choice anyway).
 //   7067 x 3072 x 3072 / 8192 (1.31 rounds, bf16): 125 -> 111 / 296 -> 259 us   24105 x 1024 x 4096 (1.48, fp16): 190 -> 171
 //   1000 x 4096 x 4096 / 14336 (0.25): 48 -> 36 / 153 -> 101                   3618 x 320 x 8192 (0.12): 84 -> 39
-//   left whole: 24105 x 1024 x 1024 (59, cut: 71), 24105 x 3072 x 1024 (148, cut: 153), 2000 x 3072 x 3072 (40, cut: 42)
+//   58 tiles of 128 rows, K 1536: 21.7 uncut, 19.1 in two, 23.0 in four        24105 x 1024 x 1024: 59 uncut, 71 in two
 static long tail_cost(int ntiles, int nk, int bm, int sl) {
   if (sl == 1) return nk * 100L;
-  const bool behind = ntiles > (int)GEMM_TAIL_WGS;
   long c = ((nk + sl - 1) / sl + min(TAIL_SKEW, nk / sl / 4)) * 100L;
-  for (int wgs = ntiles % (int)GEMM_TAIL_WGS * sl; sl > 1; sl /= 2, wgs /= 2)
-    c += (behind ? 500 + 1500L * wgs / 256 : 700 + 200L * wgs / 256) * (bm == 256 ? 10 : 7) / 10;
-  return c * 105 / 100;
+  bool first = true;
+  for (int wgs = ntiles % (int)GEMM_TAIL_WGS * sl; sl > 1; sl /= 2, wgs /= 2, first = false)
+    c += (first ? 550 + 750L * wgs / 256 : 800 + 1150L * wgs / 256) * (bm == 256 ? 10 : 7) / 10;
+  return c * 102 / 100;
 }
 
-// Workgroups per tail tile: 1, or 2, 4 or 8 where the chip has room for them beside each other, they have at least 4
-// K-tiles each, and that is the fastest.
+// Workgroups per tail tile: 1, or 2, 4 or 8 where the chip has room for them beside each other, they have at least 8
+// K-tiles each (fewer were never the fastest), and that is the fastest.
 static int tail_slices(int ntiles, int nk, int bm) {
   const int G = (int)GEMM_TAIL_WGS, rest = ntiles % G;
   int best = 1;
   if (num_cus() < G || rest == 0) return best;
-  for (int sl = 2; sl <= 8 && sl * ((rest + 7) & ~7) <= G && nk / sl >= 4; sl *= 2)
+  for (int sl = 2; sl <= 8 && sl * ((rest + 7) & ~7) <= G && nk / sl >= 8; sl *= 2)
     if (tail_cost(ntiles, nk, bm, sl) < tail_cost(ntiles, nk, bm, best)) best = sl;
   return best;
 }

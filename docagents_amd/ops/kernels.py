@@ -242,7 +242,7 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
 # (streams run products beside each other) for the TAIL_STREAMS latest streams, and in a capture one per capture and
 # stream, cleared by a node in front of its first such product.
 TAIL_STREAMS = 32
-TAIL_MIN_K = 768  # no round of a shorter product is shared (csrc/gemm8p.hip, tail_cost)
+TAIL_MIN_K = 1024  # no round of a shorter product is shared (csrc/gemm8p.hip, tail_slices)
 _TAIL: dict = {}  # (device, stream) -> counters, oldest first
 _TAIL_CAPTURED: dict = {}  # (device, stream) -> (capture, counters): kept until the stream's next capture
 

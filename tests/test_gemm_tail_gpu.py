@@ -17,12 +17,13 @@ def _operands(M, N, Kd, dtype, seed):
     return a, w, bias, torch.randn(M, N, device=DEV, generator=g).to(dtype)
 
 
-# tiles of 256 x 256: fewer than a round (9 in 4 slices, 1 and 12 in 8), a round and some (300, the last 44 in 2), slices of
-# unequal length (33 K-tiles in 4), a last row and column tile that are not full; tiles of 128 rows; too short to be cut and
-# exactly a round (whole)
-@pytest.mark.parametrize("M,N,Kd,tile", [(700, 768, 2048, 7), (256, 256, 4096, 7), (1000, 768, 8192, 7), (6244, 3072, 2048, 7),
-                                         (700, 776, 64 * 33, 7), (1000, 520, 2048, 10), (6400, 3072, 2048, 10),
-                                         (700, 768, 1024, 7), (4096, 4096, 1024, 7)])
+# tiles of 256 x 256: fewer than a round (9 in 2 and 4 slices, 1 and 12 in 8), a round and some (300, the last 44 in 2),
+# slices of unequal length (33 K-tiles in 2, 65 in 4), a last row and column tile that are not full; tiles of 128 rows; too
+# short to be cut and exactly a round (whole)
+@pytest.mark.parametrize("M,N,Kd,tile", [(700, 768, 2048, 7), (700, 768, 4096, 7), (256, 256, 4096, 7), (1000, 768, 8192, 7),
+                                         (6244, 3072, 2048, 7), (700, 776, 64 * 33, 7), (700, 776, 64 * 65, 7),
+                                         (1000, 520, 2048, 10), (6400, 3072, 2048, 10), (700, 768, 1024, 7),
+                                         (4096, 4096, 1024, 7)])
 @pytest.mark.parametrize("epi", [K.EPI_NONE, K.EPI_BIAS, K.EPI_GELU, K.EPI_RESID, K.EPI_SWIGLU])
 def test_tail(M, N, Kd, tile, epi, monkeypatch):
     a, w, bias, resid = _operands(M, N, Kd, torch.bfloat16, M + N)
@@ -97,8 +98,12 @@ def test_tail_streams():
 
 # (M, N, K, tile height's code) -> tiles behind the whole rounds, slices of each; None: left whole
 @pytest.mark.parametrize("M,N,Kd,tile,cut", [
-    (700, 768, 2048, 7, (9, 4)), (256, 256, 4096, 7, (1, 8)), (1000, 768, 8192, 7, (12, 8)), (6244, 3072, 2048, 7, (44, 2)),
-    (700, 776, 64 * 33, 7, (12, 4)), (1000, 520, 2048, 10, (24, 4)), (700, 768, 1024, 7, None), (4096, 4096, 1024, 7, None)])
+    (700, 768, 2048, 7, (9, 2)), (700, 768, 4096, 7, (9, 4)), (256, 256, 4096, 7, (1, 8)), (1000, 768, 8192, 7, (12, 8)),
+    (6244, 3072, 2048, 7, (44, 2)), (700, 776, 64 * 33, 7, (12, 2)), (700, 776, 64 * 65, 7, (12, 4)),
+    (1000, 520, 2048, 10, (24, 4)), (700, 768, 1024, 7, None), (4096, 4096, 1024, 7, None),
+    # four slices of few K-tiles that fill the chip are slower than two, and than none
+    (3675, 512, 1536, 10, (58, 2)), (3675, 512, 2048, 10, (58, 2)), (8000, 512, 1536, 10, None),
+    (700, 768, 1472, 7, (9, 2))])
 @pytest.mark.parametrize("epi", [K.EPI_NONE, K.EPI_GELU, K.EPI_RESID, K.EPI_SWIGLU])
 def test_which_rounds_are_cut(M, N, Kd, tile, cut, epi):
     """A product takes scratch for as many partials as it leaves, and none where its tiles stay whole. GELU's always do."""
@@ -132,7 +137,7 @@ def test_scratch_is_given_back():
     cleared once, and they are its own."""
     a, w, _, _ = _operands(700, 768, 2048, torch.bfloat16, 3)
     nbytes = K.lib().da_gemm_tail_ws(700, 768, 2048, K.EPI_NONE, 7)
-    assert nbytes == 9 * 4 * 256 * 256 * 4
+    assert nbytes == 9 * 2 * 256 * 256 * 4
     out = torch.empty(700, 768, dtype=torch.bfloat16, device=DEV)
     first = K.gemm(a, w, tile=7)
     streams = [torch.cuda.Stream() for _ in range(6)]
