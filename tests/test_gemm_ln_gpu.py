@@ -64,3 +64,27 @@ def test_what_the_product_refuses():
             K.gemm_ln(a, w, bias, K.EPI_RESID, norm=norm, resid=a, st_out=st2)
     with pytest.raises(ValueError):
         K.gemm_ln(a, w, b, K.EPI_RESID, resid=a, st_out=st2[:, :32])
+
+
+@pytest.mark.parametrize("h,f,one", [(1024, 4096, False), (1024, 2048, True), (768, 3072, True)])
+def test_which_short_texts_take_it(h, f, one, monkeypatch):
+    """Up to 64 tokens do, but one token of a wide encoder has matrix-vector products; both agree."""
+    from docagents_amd.models.bert import BertEncoder
+    from docagents_amd.models.configs import EncoderConfig
+    enc = BertEncoder(EncoderConfig("e", vocab=100, hidden=h, layers=2, heads=h // 64, ffn=f), "cuda")
+    calls, real = [], K.gemm_ln
+    monkeypatch.setattr(K, "gemm_ln", lambda *a, **kw: calls.append(1) or real(*a, **kw))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    for T, few in ((1, one), (2, True), (64, True), (65, False)):
+        calls.clear()
+        args = i32([7] * T), i32(list(range(T))), i32([0, T]), T
+        got = enc.forward(*args).double()
+        assert len(calls) == (8 if few else 0)
+        if T == 1:
+            with monkeypatch.context() as m:
+                m.setattr(BertEncoder, "_one_row", lambda self, rows: one)  # the other way
+                if one:
+                    m.setattr(K, "gemm_ln_fit", lambda *a: False)
+                want = enc.forward(*args).double()
+            # bf16 roundings of two layers: each of about a dozen adds 2^-9 of values of about 1
+            assert float((got - want).norm() / want.norm()) < 12 * 2.0 ** -9
