@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 import math
 import os
 import threading
@@ -18,6 +19,9 @@ from pathlib import Path
 import torch
 
 _LOCK = threading.Lock()
+# What the rules below choose for a shape, looked up instead of worked out for each product of each layer (2 us each, which
+# an encoder's layers that are launched one by one wait for)
+_rule = functools.lru_cache(maxsize=4096)
 # DA_KERNELS_DEBUG=1: the -DDA_DEBUG build (device asserts: bounds / shape preconditions inside the
 # kernels; python -m docagents_amd.ops.build --debug) instead of the -O3 library
 _DEBUG = os.environ.get("DA_KERNELS_DEBUG", "0") == "1"
@@ -247,11 +251,16 @@ _TAIL: dict = {}  # (device, stream) -> counters, oldest first
 _TAIL_CAPTURED: dict = {}  # (device, stream) -> (capture, counters): kept until the stream's next capture
 
 
+@_rule
+def _tail_bytes(M: int, N: int, K: int, epi: int, tile: int) -> int:
+    return lib().da_gemm_tail_ws(M, N, K, epi, tile)
+
+
 def _gemm_tail(device, stream: int, M: int, N: int, K: int, epi: int, tile: int = 0):
     """(partials, counters) of a product on the current stream ``stream`` whose last round is shared, (None, None) of
     others; the caller holds them until it is launched. A set of counters that makes room for another stream's goes back to
     the allocator, which keeps it for the stream that used it: in order."""
-    nbytes = lib().da_gemm_tail_ws(M, N, K, epi, tile) if K >= TAIL_MIN_K else 0
+    nbytes = _tail_bytes(M, N, K, epi, tile) if K >= TAIL_MIN_K else 0
     if not nbytes:
         return None, None
     part = torch.empty(nbytes // 4, dtype=torch.float32, device=device)
@@ -362,6 +371,7 @@ def _dk_splitk(M: int, N: int) -> bool:
     return DK_SPLITK_ABOVE < M <= 64 and N % 512 == 0
 
 
+@_rule
 def _dk_splits(N: int, K: int, reduce: bool = False) -> int:
     """Split-K of the 33..64-row route (64x128 tiles): the largest of 2, 3, 4, 6, 8, 12, 16 that keeps
     the grid within one round of 256 workgroups and >= 4 K-steps of 64 per split. 3 is the point of this
@@ -592,6 +602,7 @@ def _decode_tile(M: int, N: int = 0) -> int:
     return 2
 
 
+@_rule
 def _auto_splits(M: int, N: int, K: int) -> int:
     """Split-K for decode-sized M. Up to 64 rows (without the exceptions below): the largest power of two
     keeping <= 256 workgroups (one per CU) and >= 4 K-steps per split. With 4 k-tiles in flight per
@@ -636,6 +647,7 @@ def _mid_stream(M: int, N: int, K: int):
                if s == 1 or (ksteps % s == 0 and ksteps // s >= 4 and s <= most))
 
 
+@_rule
 def _mid_tile(M: int, N: int, K: int):
     """(tile, splits) of a product of 129..639 rows: the 128x128 streaming tile (2), or the register-staged 64x128 one (11)
     over ceil(M / 64) row blocks with up to 4 workgroups a CU below 256 rows and 2.5 from there (32-layer Phi-3 chain,
@@ -851,6 +863,7 @@ def _decode_split(B: int, Hkv: int, max_len: int, chunk: int):
 BY_LEN_KEYS = 256
 
 
+@_rule
 def _gqa_split(B: int, Hkv: int, max_len: int):
     """(chunk, nsplit, by_len) of a grouped-query launch (head dims 64 and 128) whose caller names no chunk. by_len: a row's
     keys over as many of the nsplit splits as hold ``chunk`` of them each; else over all of them. Measured over 16 query
@@ -1227,6 +1240,7 @@ def spin(us: int, device=None) -> None:
 def gemm8p_persist(on: int = -1) -> int:
     """Persistent tile loop of the prefill GEMM (one workgroup per CU walking its XCD's tiles) on
     (1) / off (0) for later launches; -1 only queries. Returns the previous setting."""
+    _tail_bytes.cache_clear()
     return int(lib().da_gemm8p_persist(int(on)))
 
 
