@@ -609,7 +609,7 @@ static bool tail_allowed(int epi) { return epi != EPI_GELU && epi != EPI_ROPE &&
 // one of 228 is above uncut (1.04: 112 tiles of 256 rows, K 2048, where tiles of 128 rows are the choice anyway).
 //   7067 x 3072 x 3072 / 8192 (1.31 rounds, bf16): 125 -> 111 / 296 -> 259 us   24105 x 1024 x 4096 (1.48, fp16): 190 -> 171
 //   1000 x 4096 x 4096 / 14336 (0.25): 48 -> 36 / 153 -> 101                   3618 x 320 x 8192 (0.12): 84 -> 39
-//   58 tiles of 128 rows, K 1536: 21.7 uncut, 19.1 in two, 23.0 in four        24105 x 1024 x 1024: 59 uncut, 71 in two
+//   58 tiles of 128 rows, K 2048: 26.4 uncut, 21.5 in two, 24.8 in four        24105 x 1024 x 1024: 59 uncut, 71 in two
 static long tail_cost(int ntiles, int nk, int bm, int sl) {
   if (sl == 1) return nk * 100L;
   long c = ((nk + sl - 1) / sl + min(TAIL_SKEW, nk / sl / 4)) * 100L;
@@ -620,13 +620,15 @@ static long tail_cost(int ntiles, int nk, int bm, int sl) {
 }
 
 // Workgroups per tail tile: 1, or 2, 4 or 8 where the chip has room for them beside each other, they have at least 8
-// K-tiles each (fewer were never the fastest), and that is the fastest.
+// K-tiles each (fewer were never the fastest), and that is the fastest. Within one round by at least 5 K-tiles (3 - 4 us):
+// taking the partials from the allocator is 3 us of the host's time, which a small model's launches wait for (12 layers of
+// 384 x 1536, 3058 rows: 1255 us whole, 1294 in two slices though each product is 2.5 us shorter on the GPU).
 static int tail_slices(int ntiles, int nk, int bm) {
   const int G = (int)GEMM_TAIL_WGS, rest = ntiles % G;
   int best = 1;
   if (num_cus() < G || rest == 0) return best;
   for (int sl = 2; sl <= 8 && sl * ((rest + 7) & ~7) <= G && nk / sl >= 8; sl *= 2)
-    if (tail_cost(ntiles, nk, bm, sl) < tail_cost(ntiles, nk, bm, best)) best = sl;
+    if (tail_cost(ntiles, nk, bm, sl) + (best == 1 && ntiles < G ? 500 : 0) < tail_cost(ntiles, nk, bm, best)) best = sl;
   return best;
 }
 
