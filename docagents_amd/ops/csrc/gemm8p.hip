@@ -620,15 +620,16 @@ static long tail_cost(int ntiles, int nk, int bm, int sl) {
 }
 
 // Workgroups per tail tile: 1, or 2, 4 or 8 where the chip has room for them beside each other, they have at least 8
-// K-tiles each (fewer were never the fastest), and that is the fastest. Within one round by at least 5 K-tiles (3 - 4 us):
-// taking the partials from the allocator is 3 us of the host's time, which a small model's launches wait for (12 layers of
-// 384 x 1536, 3058 rows: 1255 us whole, 1294 in two slices though each product is 2.5 us shorter on the GPU).
+// K-tiles each (fewer were never the fastest), and that is the fastest. Within one round from 28 K-tiles on: taking the
+// partials from the allocator is 3 us of the host's time, which a small model's launches wait for. 12 layers with a
+// 384 x 1536 product, 3058 rows, launched one by one: 1255 us whole, 1294 in two slices, though on the GPU each is 22 us
+// whole and 19 in two; from K = 2048 a cut saves 4 - 6 us.
 static int tail_slices(int ntiles, int nk, int bm) {
   const int G = (int)GEMM_TAIL_WGS, rest = ntiles % G;
   int best = 1;
-  if (num_cus() < G || rest == 0) return best;
+  if (num_cus() < G || rest == 0 || (ntiles < G && nk < 28)) return best;
   for (int sl = 2; sl <= 8 && sl * ((rest + 7) & ~7) <= G && nk / sl >= 8; sl *= 2)
-    if (tail_cost(ntiles, nk, bm, sl) + (best == 1 && ntiles < G ? 500 : 0) < tail_cost(ntiles, nk, bm, best)) best = sl;
+    if (tail_cost(ntiles, nk, bm, sl) < tail_cost(ntiles, nk, bm, best)) best = sl;
   return best;
 }
 

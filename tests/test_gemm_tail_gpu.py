@@ -101,8 +101,8 @@ def test_tail_streams():
     (700, 768, 2048, 7, (9, 2)), (700, 768, 4096, 7, (9, 4)), (256, 256, 4096, 7, (1, 8)), (1000, 768, 8192, 7, (12, 8)),
     (6244, 3072, 2048, 7, (44, 2)), (700, 776, 64 * 33, 7, (12, 2)), (700, 776, 64 * 65, 7, (12, 4)),
     (1000, 520, 2048, 10, (24, 4)), (700, 768, 1024, 7, None), (4096, 4096, 1024, 7, None),
-    # within one round a cut has to be worth the allocation: 5 K-tiles; slices that fill the chip are slower in four than in two
-    (3675, 512, 1536, 10, None), (3675, 512, 2048, 10, (58, 2)), (700, 768, 1600, 10, None), (700, 768, 1664, 10, (18, 2))])
+    # within one round a cut has to be worth its allocation: from 28 K-tiles; slices that fill the chip are slower in four
+    (3675, 512, 1536, 10, None), (3675, 512, 2048, 10, (58, 2)), (700, 768, 1728, 10, None), (700, 768, 1792, 10, (18, 2))])
 @pytest.mark.parametrize("epi", [K.EPI_NONE, K.EPI_GELU, K.EPI_RESID, K.EPI_SWIGLU])
 def test_which_rounds_are_cut(M, N, Kd, tile, cut, epi):
     """A product takes scratch for as many partials as it leaves, and none where its tiles stay whole. GELU's always do."""
