@@ -688,19 +688,21 @@ static int launch_ws(const GemmArgs& a, int epi, int splits, const WsNorm& nrm, 
 // The streaming kernel's offsets into a tile's rows are 32 bits wide (_dk_splits draws the same line).
 static bool ws_spans(const GemmArgs& a) { return max(a.K, a.lda) < 1 << 22; }
 
-// Filling the ring and draining it costs the streaming kernel a microsecond, which K splits of fewer than 28 stages of up
-// to 64 rows do not win back from the register-staged 64x128 tile with 4 k-tiles in flight (depth 1 / 2 / 8 measured slower,
-// profiles/decode_gemm_prefetch_sweep_r1.jsonl): with their reduce, 64 rows, register / streaming us: 768 x 768 8.3 / 9.7
-// (6 stages), 8192 x 2048 15.7 / 17.7 (8), 3072 x 8192 18.5 / 19.4 (16), 4096 x 14336 29.4 / 29.3 (28), 8192 x 14336 48.4 /
-// 46.5 (56). Unsplit products are faster on the ring at every length (64 x 12288 x 768 9.9 / 9.3).
-static bool ws_pays(const GemmArgs& a, int splits) {
-  return ws_spans(a) && (a.M > 64 || splits == 1 || a.k_per_split >= 28 * 64);
+// K splits of up to 64 rows: the ring costs a microsecond to fill and drain, and a reduce behind it 1 - 2 more than behind
+// the register-staged 64x128 tile with 4 k-tiles in flight (depth 1 / 2 / 8 measured slower,
+// profiles/decode_gemm_prefetch_sweep_r1.jsonl). 64 rows, weights from HBM, register / ring us, with the reduce: 768 x 768
+// 10.4 / 10.2 (6 stages), 8192 x 2048 16.2 / 18.0 (8), 8192 x 4096 22.3 / 23.3 (16), 3072 x 8192 18.6 / 19.3 (16), 5120 x
+// 5120 22.9 / 20.8 (20), 4096 x 14336 31.3 / 30.3 (28). Partials that the next kernel sums (`stages` 6): 1024 x 1024 6.4 / 6.9
+// (4), 3072 x 3072 9.5 / 9.4 (6), 4096 x 4096 12.5 / 11.8 (8), 6272 x 4096 15.9 / 15.0 (16). Unsplit products are faster on
+// the ring at every length (64 x 12288 x 768 9.9 / 9.3).
+static bool ws_pays(const GemmArgs& a, int splits, int stages) {
+  return ws_spans(a) && (a.M > 64 || splits == 1 || a.k_per_split >= stages * 64);
 }
 
 // Decode tiles: 64x128 by the rule above, else 4 k-tiles in flight per workgroup.
 template <int BM, int BN>
-static int launch_decode_tile(const GemmArgs& a, int epi, int splits, hipStream_t s) {
-  if (BM == 64 && ws_pays(a, splits)) return launch_ws(a, epi, splits, WsNorm{}, s);
+static int launch_decode_tile(const GemmArgs& a, int epi, int splits, hipStream_t s, int stages = 20) {
+  if (BM == 64 && ws_pays(a, splits, stages)) return launch_ws(a, epi, splits, WsNorm{}, s);
   return launch_tile<BM, BN, 1, 4, 4>(a, epi, splits, s);
 }
 
@@ -864,7 +866,7 @@ DA_EXPORT int da_gemm_partials(const void* A, int lda, const void* W, int M, int
   a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = N; a.k_per_split = K / splits;
   hipStream_t s = (hipStream_t)stream;
   switch (tile) {
-    case 2: return launch_decode_tile<64, 128>(a, EPI_PARTIAL, splits, s);
+    case 2: return launch_decode_tile<64, 128>(a, EPI_PARTIAL, splits, s, 6);
     case 3: return launch_decode_tile<32, 128>(a, EPI_PARTIAL, splits, s);
     case 9: return launch_tile<128, 64, 2, 2, 4>(a, EPI_PARTIAL, splits, s);
     default: return (int)hipErrorInvalidValue;

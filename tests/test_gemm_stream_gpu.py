@@ -62,9 +62,9 @@ def test_row_norm_without_splits(M, N, Kd, epi):
     assert ((got - ref).abs() <= U * ref.abs() + 8 * Kd * 2.0 ** -24 * mag).all()
 
 
-@pytest.mark.parametrize("M,N,stages,splits", [(64, 136, 27, 2), (64, 136, 28, 2), (33, 4096 + 8, 28, 3), (48, 320, 4, 32)])
+@pytest.mark.parametrize("M,N,stages,splits", [(64, 136, 19, 2), (64, 136, 20, 2), (33, 4096 + 8, 28, 3), (48, 320, 4, 32)])
 def test_split_products_either_side_of_the_ring(M, N, stages, splits):
-    """K splits of up to 64 rows: 28 stages are the first on the ring, shorter ones are staged through registers."""
+    """K splits of up to 64 rows: 20 stages are the first on the ring, shorter ones are staged through registers."""
     Kd = 64 * stages * splits
     a, w, bias, g = _operands(M, N, Kd, Kd + 64)
     resid = torch.randn(M, N, device="cuda", generator=g).bfloat16()
@@ -72,6 +72,18 @@ def test_split_products_either_side_of_the_ring(M, N, stages, splits):
     ref = a.double() @ w.double().T + bias.double() + resid.double()
     tol = U * ref.abs() + 8 * Kd * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T).max()
     assert ((got - ref).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("M,N,stages,splits", [(64, 136, 5, 3), (64, 136, 6, 3), (33, 328, 7, 4)])
+def test_partials_either_side_of_the_ring(M, N, stages, splits):
+    """Partials that no reduce follows: 6 stages are the first on the ring."""
+    Kd = 64 * stages * splits
+    a, w, _, _ = _operands(M, N, Kd, Kd + 64)
+    ws = torch.empty(splits, M, N, device="cuda")
+    K._check(K.lib().da_gemm_partials(K._ptr(a), a.stride(0), K._ptr(w), M, N, Kd, 2, splits, K._ptr(ws), K._stream()), "partials")
+    for i, (x, y) in enumerate(zip(a.double().split(64 * stages, 1), w.double().split(64 * stages, 1))):
+        tol = 8 * stages * 64 * 2.0 ** -24 * (x.abs() @ y.abs().T).max()
+        assert ((ws[i].double() - x @ y.T).abs() <= tol).all()
 
 
 @pytest.mark.parametrize("Kd", [8192, 8192 + 256])
