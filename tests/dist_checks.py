@@ -1,5 +1,5 @@
 """Multi-process correctness checks for the distributed paths (test harness: run with gloo on CPU,
-or with GPU ranks through gpurun). Each ``check_*`` is a ``torch.multiprocessing.spawn`` target;
+or with GPU ranks). Each ``check_*`` is a ``torch.multiprocessing.spawn`` target;
 rank 0 writes a JSON verdict to ``out_path``. Imported by the tests as ``dist_checks`` (tests/ is on
 sys.path under pytest, and spawned children inherit it).
 
