@@ -15,6 +15,8 @@
 //  * split-K writes fp32 partials; gemm_splitk_reduce applies the same epilogue.
 #include "gemm.h"
 
+#include <type_traits>
+
 template <int BM, int BN, int WM, int WN, int EPI, int PF = 1>
 __global__ void __launch_bounds__(256)
 gemm_bf16_kernel(GemmArgs p) {
@@ -228,39 +230,46 @@ gemm_bf16_kernel(GemmArgs p) {
 }
 
 // ------------------------------------------------------------------------------------------
-// Weight-streaming product (33..639 rows: decoding, short prompts): 64 x 128 tiles, four waves of 64 rows x 32 columns, for
-// up to 64 rows; 64 x 64 (32 x 32 a wave) where only those fill the CUs without splits; 128 x 128 with eight waves above 64
-// rows. K in stages of 64.
-//  * A stage (8 or 16 KB of A, 8 or 16 KB of W) arrives by LDS-DMA in a ring of 5, 6 or 10 stages, so 64 - 80 KB of W are
-//    on their way per CU whatever the registers hold. (Staged through registers, four in flight and a ds_write each:
-//    3.6 - 4.3 TB/s.)
+// Weight-streaming product (33 rows to some 1000: decoding, short prompts, short texts; bf16, and fp16 for the encoders).
+// K in stages of 64; tiles of 64 x 128, 64 x 64, 128 x 64, 128 x 128 and 192 x 128, four or eight waves.
+//  * A stage (8 - 24 KB of A, 8 or 16 KB of W) arrives by LDS-DMA in a ring that fills LDS. What a CU can have on its way
+//    beyond the L2 is 32 KB whatever is asked for (57 GB/s from HBM or the last-level cache, 142 GB/s from L2; loads into
+//    registers the same), and A's pieces wait in that queue behind W's, so the tile's bytes per product bound it, not the
+//    ring's depth.
+//  * A stage's two halves of 32 are read from LDS one ahead of the MFMAs, across the barrier, and the next stage's LDS-DMA
+//    instructions lie between the MFMAs (16 address cycles each: behind the barrier, all together, every wave's MFMAs waited
+//    for them). 1024 x 1024 x 4096 in 128 x 128 tiles 37 -> 31 (halves) -> 26 us (pieces), 256 x 4096 x 1024 in 64 x 64 8.4 -> 7.6.
 //  * One workgroup per CU walks units (tile, K split) b, b + G, ...; the ring runs on across units, so the next one's
 //    weights are on their way during this one's epilogue. Past the last unit the pieces are issued against an empty
 //    resource (no traffic): the counted waits stay the same to the end.
+//  * NT, one row block (W is read once): a tile of columns begins at a K-step of its own (its number, round K). Workgroups that
+//    all read the same columns of rows a power of two apart ask the same few channels at a time: 64 x 28672 x 4096 46.6 ->
+//    40.3 us (5.8 TB/s; a kernel that only loads that much takes 38), 64 x 128256 x 4096 197 -> 189. The order of a sum depends
+//    on its column only. With more row blocks it gained nothing, and sums are in the phase-split kernel's order.
 //  * W is the MFMA's A operand, so a lane holds 4 consecutive columns of a row and stores them without staging.
 //  * nrm: the rows of A are the raw residual stream, and the result's rows are scaled by rsqrt(sum of the parts'
 //    squares / norm_k + eps) (gemm_dk.hip).
-// Bound by HBM where tiles cover the CUs: 64 x 28672 x 4096 (235 MB, no split) 48 us (4.9 TB/s) vs 62 with two splits and
-// their reduce before; 64 x 128256 x 4096 191 (5.5 TB/s) vs 248;
-// 64 x 12672 x 4096 29 in 64 x 64 tiles, 33 in two splits of 64 x 128. Above 128 rows by the stage's turn-around on one CU
-// (0.56 us; with four waves 0.7): 200 x 28672 x 4096 79 vs 99, 256 x 4096 x 14336 50 vs 62, 512 x 6144 x 4096 41 vs 53.
+constexpr int WS_LDS = 160 * 1024;
+
 struct WsNorm {
   const float* ssq;  // [parts][64]; null: none
   int parts, norm_k;
   float eps;
 };
 
-template <int BM, int BN, int EPI, bool NT>
-__global__ void __launch_bounds__(BM * 4)
+template <int BM, int BN, int WGM, int WGN, int EPI, bool NT, typename T>
+__global__ void __launch_bounds__(64 * WGM * WGN)
 gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
-  constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128;
-  constexpr int WS_ST = BM == 128 ? 5 : BN == 128 ? 6 : 10;
-  constexpr int PW = 2 * BN / BM;   // LDS-DMA instructions of a wave per stage: 2 of A, PW of W
-  constexpr int WN = BN / 32;       // waves along N (32 columns each)
-  constexpr int FM = BN == 64 ? 2 : 4, WROWS = FM * 16;  // row fragments and rows of a wave
+  constexpr int NW = WGM * WGN, A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128;
+  constexpr int ST = WS_LDS / STAGE < 10 ? WS_LDS / STAGE : 10;  // stages of the ring
+  constexpr int PA = BM / 8 / NW, PW = BN / 8 / NW;  // LDS-DMA instructions of a wave per stage
+  constexpr int P = PA + PW, PH = P / 2;  // of them beside a stage's first half
+  constexpr int FM = BM / WGM / 16, FN = BN / WGN / 16, WROWS = FM * 16, WCOLS = FN * 16;
+  static_assert(PA >= 1 && PA <= 4 && PW >= 1 && PW <= 4 && FN % 2 == 0 && ST >= 3 && P * (ST - 2) < 64, "tile");
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
-  __shared__ __attribute__((aligned(16))) char smem[WS_ST * STAGE];
+  __shared__ __attribute__((aligned(16))) char smem[ST * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = w / WGN, wn = w % WGN;
   const int fr = lane & 15, fg = lane >> 4;
   const int ntm = (p.M + BM - 1) / BM, ntn = (p.N + BN - 1) / BN, units = ntm * ntn * splits;
   const int nk = p.k_per_split / 64, G = gridDim.x;
@@ -276,19 +285,20 @@ gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
 
   // ---- the ring's writing side: stage `ik` of unit `iu` is next ----
   __amdgpu_buffer_rsrc_t ra, rw;
-  unsigned ao[2], wo[4];  // row w * 16 + j * 8 + lane / 8 of A (w * 8 * PW + ... of W), 16-B chunk swizzled by (row >> 1) & 7
-  int iu = 0, ik = 0, slot = 0;
+  unsigned ao[4], wo[4];  // row w * 8 * PA + j * 8 + lane / 8 of A (PW: of W), 16-B chunk swizzled by (row >> 1) & 7
+  int iu = 0, ik = 0, pos = 0, slot = 0;  // pos: the K-step that stage ik holds
   auto open = [&]() __attribute__((always_inline)) {  // resources and offsets of unit iu
     int m0, n0, sp;
     unit_of(iu, m0, n0, sp);
+    pos = NT ? n0 / BN % nk : 0;
     const int n = iu < mine ? 0x7ffffff0 : 0;
     ra = __builtin_amdgcn_make_buffer_rsrc(
         (void*)((const char*)p.A + (size_t)m0 * p.lda * 2 + (size_t)sp * p.k_per_split * 2), (short)0, n, 0x00020000);
     rw = __builtin_amdgcn_make_buffer_rsrc(
         (void*)((const char*)p.W + (size_t)n0 * p.K * 2 + (size_t)sp * p.k_per_split * 2), (short)0, n, 0x00020000);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int r = w * 16 + j * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+    for (int j = 0; j < PA; ++j) {
+      const int r = w * 8 * PA + j * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
       ao[j] = (unsigned)(min(m0 + r, p.M - 1) - m0) * (unsigned)(p.lda * 2) + c * 16;
     }
 #pragma unroll
@@ -297,85 +307,114 @@ gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
       wo[j] = (unsigned)(min(n0 + r, p.N - 1) - n0) * (unsigned)(p.K * 2) + c * 16;
     }
   };
-  auto issue = [&]() __attribute__((always_inline)) {
+  auto piece = [&](int j) __attribute__((always_inline)) {  // the wave's j-th of PA + PW instructions of a stage
     char* base = smem + slot * STAGE;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(base + (w * 2 + j) * 1024), 16, ao[j], ik * 128, 0, 0);
-#pragma unroll
-    for (int j = 0; j < PW; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t)(base + A_BYTES + (w * PW + j) * 1024), 16, wo[j], ik * 128, 0,
-                                               NT ? 2 : 0);
-    slot = slot + 1 == WS_ST ? 0 : slot + 1;
+    if (j < PA)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(base + (w * PA + j) * 1024), 16, ao[j & 3], pos * 128, 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t)(base + A_BYTES + (w * PW + j - PA) * 1024), 16, wo[(j - PA) & 3],
+                                               pos * 128, 0, NT ? 2 : 0);
+  };
+  auto next_stage = [&]() __attribute__((always_inline)) {
+    slot = slot + 1 == ST ? 0 : slot + 1;
+    pos = pos + 1 == nk ? 0 : pos + 1;
     if (++ik == nk) {
       ik = 0;
       ++iu;
       open();
     }
   };
+  // this wave's pieces of the stage that is read next are in (newer ones: ST - 3 whole stages and PH pieces); after the
+  // barrier everyone's are, and what was read before it may be written
+  auto landed = [&](auto newer) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(newer)::value) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
   open();
 #pragma unroll 1
-  for (int i = 0; i < WS_ST - 1; ++i) issue();
+  for (int i = 0; i < ST - 1; ++i) {
+#pragma unroll
+    for (int j = 0; j < P; ++j) piece(j);
+    next_stage();
+  }
 
   int rd = 0;  // the slot that is read next
   const int sw = (fr >> 1) & 7;
-  for (int u = 0; u < mine; ++u) {
-    int m0, n0, sp;
-    unit_of(u, m0, n0, sp);
-    f32x4_t acc[FM][2];
+  const int co[2] = {(fg ^ sw) << 4, ((4 + fg) ^ sw) << 4};
+  bf16x8_t af[2][FM], wf[2][FN];  // fragments of a stage's halves: one is read while the other is multiplied
+  auto read = [&](auto half) __attribute__((always_inline)) {
+    constexpr int H = decltype(half)::value;
+    const char* sa = smem + rd * STAGE + wm * WROWS * 128 + fr * 128 + co[H];
+    const char* sb = smem + rd * STAGE + A_BYTES + wn * WCOLS * 128 + fr * 128 + co[H];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) wf[H][j] = *(const bf16x8_t*)(sb + j * 2048);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) af[H][i] = *(const bf16x8_t*)(sa + i * 2048);
+  };
+  f32x4_t acc[FM][FN];
+  // MFMAs of a half with pieces of the next stage between them (together at the barrier the waves would wait for the
+  // address unit, 16 cycles an instruction, with their MFMAs behind them)
+  auto multiply = [&](auto half) __attribute__((always_inline)) {
+    constexpr int H = decltype(half)::value, J0 = H ? PH : 0, NJ = H ? P - PH : PH;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int kt = 0; kt < nk; ++kt) {
-      // this wave's pieces of the stage are in; after the barrier everyone's, and the slot before it has been read
-      if constexpr (BN == 64)
-        asm volatile("s_waitcnt vmcnt(32) lgkmcnt(0)" ::: "memory");  // 4 * (10 - 2)
-      else if constexpr (BM == 64)
-        asm volatile("s_waitcnt vmcnt(24) lgkmcnt(0)" ::: "memory");  // 6 * (6 - 2)
-      else
-        asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)" ::: "memory");  // 4 * (5 - 2)
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      issue();
-      const char* sa = smem + rd * STAGE + (w / WN) * WROWS * 128;
-      const char* sb = smem + rd * STAGE + A_BYTES + (w % WN) * 32 * 128;
+      for (int j = 0; j < FN; ++j) {
+        acc[i][j] = T::mma16(wf[H][j], af[H][i], acc[i][j]);
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        const int c = ((kk * 4 + fg) ^ sw) << 4;
-        bf16x8_t af[FM], wf[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) wf[j] = *(const bf16x8_t*)(sb + (j * 16 + fr) * 128 + c);
-#pragma unroll
-        for (int i = 0; i < FM; ++i) af[i] = *(const bf16x8_t*)(sa + (i * 16 + fr) * 128 + c);
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = mfma16(wf[j], af[i], acc[i][j]);
+        for (int q = 0; q < NJ; ++q)
+          if (i * FN + j == (q + 1) * FM * FN / (NJ + 1) - 1 + (NJ + 1 > FM * FN)) {
+            __builtin_amdgcn_sched_barrier(0);
+            piece(J0 + q);
+            __builtin_amdgcn_sched_barrier(0);
+          }
       }
-      rd = rd + 1 == WS_ST ? 0 : rd + 1;
+  };
+  using H0 = std::integral_constant<int, 0>;
+  using H1 = std::integral_constant<int, 1>;
+  landed(std::integral_constant<int, P * (ST - 2)>{});  // stage 0
+  read(H0{});
+  for (int u = 0; u < mine; ++u) {
+    int m0, n0, sp;
+    unit_of(u, m0, n0, sp);
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int kt = 0; kt < nk; ++kt) {
+      read(H1{});
+      multiply(H0{});
+      rd = rd + 1 == ST ? 0 : rd + 1;
+      landed(std::integral_constant<int, P * (ST - 3) + PH>{});
+      read(H0{});
+      multiply(H1{});
+      next_stage();
     }
-    // ---- row m0 (+ WROWS) + 16 i + fr, columns col + 16 j + 4 fg .. + 3 ----
-    const int col = n0 + (w % WN) * 32 + 4 * fg;
+    // ---- row m0 + WROWS wm + 16 i + fr, columns col + 16 j + 4 fg .. + 3 ----
+    const int col = n0 + wn * WCOLS + 4 * fg;
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-      const int m = m0 + (w / WN) * WROWS + i * 16 + fr;
+      const int m = m0 + wm * WROWS + i * 16 + fr;
       if (m >= p.M) continue;
       float inv = 1.f;
       if (nrm.ssq) inv = rsqrtf(sum_strided(nrm.ssq + m, nrm.parts, 64) / nrm.norm_k + nrm.eps);
       if constexpr (EPI == EPI_SWIGLU) {
-        const int oc = n0 / 2 + (w % WN) * 16 + 4 * fg;
-        if (oc >= p.N / 2) continue;
-        float v[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          v[q] = gate_act(fmaf(acc[i][0][q], inv, p.bias ? bf2f(p.bias[col + q]) : 0.f), p.relu) *
-                 fmaf(acc[i][1][q], inv, p.bias ? bf2f(p.bias[col + 16 + q]) : 0.f);
-        *(u32x2_t*)(p.C + (size_t)m * p.ldc + oc) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+        for (int j = 0; j < FN; j += 2) {
+          const int oc = n0 / 2 + wn * (WCOLS / 2) + j * 8 + 4 * fg, gc = col + 16 * j;
+          if (oc >= p.N / 2) continue;
+          float v[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            v[q] = gate_act(fmaf(acc[i][j][q], inv, p.bias ? T::to_f(p.bias[gc + q]) : 0.f), p.relu) *
+                   fmaf(acc[i][j + 1][q], inv, p.bias ? T::to_f(p.bias[gc + 16 + q]) : 0.f);
+          *(u32x2_t*)(p.C + (size_t)m * p.ldc + oc) = u32x2_t{T::pack2(v[0], v[1]), T::pack2(v[2], v[3])};
+        }
       } else {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < FN; ++j) {
           const int gn = col + 16 * j;
           if (gn >= p.N) continue;
           if constexpr (EPI == EPI_PARTIAL) {
@@ -383,7 +422,7 @@ gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
           } else {
             float v[4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) v[q] = fmaf(acc[i][j][q], inv, p.bias ? bf2f(p.bias[gn + q]) : 0.f);
+            for (int q = 0; q < 4; ++q) v[q] = fmaf(acc[i][j][q], inv, p.bias ? T::to_f(p.bias[gn + q]) : 0.f);
             if constexpr (EPI == EPI_GELU) {
 #pragma unroll
               for (int q = 0; q < 4; ++q) v[q] = gelu_erf(v[q]);
@@ -392,11 +431,11 @@ gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
               const u32x2_t r = *(const u32x2_t*)(p.resid + (size_t)m * p.ldr + gn);
 #pragma unroll
               for (int q = 0; q < 2; ++q) {
-                v[2 * q] += bf2f((bf16_t)(r[q] & 0xffff));
-                v[2 * q + 1] += bf2f((bf16_t)(r[q] >> 16));
+                v[2 * q] += T::to_f((bf16_t)(r[q] & 0xffff));
+                v[2 * q + 1] += T::to_f((bf16_t)(r[q] >> 16));
               }
             }
-            *(u32x2_t*)(p.C + (size_t)m * p.ldc + gn) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+            *(u32x2_t*)(p.C + (size_t)m * p.ldc + gn) = u32x2_t{T::pack2(v[0], v[1]), T::pack2(v[2], v[3])};
           }
         }
       }
@@ -410,6 +449,7 @@ gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
 // ssq_in (nullable): deferred RMSNorm of the product's rows — the A rows were the raw residual
 // stream, so by linearity out[m, :] = inv[m] * (A W^T)[m, :], inv[m] = rsqrt(sum_p ssq_in[p][m] /
 // norm_k + eps) over the producer's `parts` row sums ([parts][64] floats; gains folded into W).
+template <typename T = BF16T>
 __global__ void __launch_bounds__(256)
 gemm_splitk_reduce(const float* __restrict__ ws, int splits, int M, int N, int epi,
                    const bf16_t* __restrict__ bias, const bf16_t* __restrict__ resid, int ldr,
@@ -434,15 +474,15 @@ gemm_splitk_reduce(const float* __restrict__ ws, int splits, int M, int N, int e
       sum_rows8(ws + (size_t)m * N + gc + 16, splits, (size_t)M * N, u);
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        v[e] = gate_act(fmaf(g[e], inv, bias ? bf2f(bias[gc + e]) : 0.f), relu) *
-               fmaf(u[e], inv, bias ? bf2f(bias[gc + 16 + e]) : 0.f);
+        v[e] = gate_act(fmaf(g[e], inv, bias ? T::to_f(bias[gc + e]) : 0.f), relu) *
+               fmaf(u[e], inv, bias ? T::to_f(bias[gc + 16 + e]) : 0.f);
     } else {
       sum_rows8(ws + (size_t)m * N + oc, splits, (size_t)M * N, v);
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] *= inv;
       if (bias) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] += bf2f(bias[oc + e]);
+        for (int e = 0; e < 8; ++e) v[e] += T::to_f(bias[oc + e]);
       }
       if (epi == EPI_GELU) {
 #pragma unroll
@@ -450,11 +490,11 @@ gemm_splitk_reduce(const float* __restrict__ ws, int splits, int M, int N, int e
       }
       if (epi == EPI_RESID) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] += bf2f(resid[(size_t)m * ldr + oc + e]);
+        for (int e = 0; e < 8; ++e) v[e] += T::to_f(resid[(size_t)m * ldr + oc + e]);
       }
     }
     *(u32x4_t*)(C + (size_t)m * ldc + oc) =
-        u32x4_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]), pack_bf2(v[4], v[5]), pack_bf2(v[6], v[7])};
+        u32x4_t{T::pack2(v[0], v[1]), T::pack2(v[2], v[3]), T::pack2(v[4], v[5]), T::pack2(v[6], v[7])};
   }
 }
 
@@ -655,17 +695,20 @@ static int launch_tile(const GemmArgs& a, int epi, int splits, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-template <int BM, int BN, bool NT>
+template <int BM, int BN, int WGM, int WGN, bool NT, typename T = BF16T>
 static int launch_ws_tile(const GemmArgs& a, int epi, int splits, const WsNorm& nrm, hipStream_t s) {
   const long units = (long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN) * splits;
   if (units > 0x7fffffffL || a.k_per_split % 64 || a.k_per_split < 64) return (int)hipErrorInvalidValue;
-  const dim3 grid((unsigned)min(units, 256L)), block(BM * 4);
-#define WS_LAUNCH(E) gemm_ws_kernel<BM, BN, E, NT><<<grid, block, 0, s>>>(a, nrm, splits)
+  const dim3 grid((unsigned)min(units, 256L)), block(64 * WGM * WGN);
+#define WS_LAUNCH(E) gemm_ws_kernel<BM, BN, WGM, WGN, E, NT, T><<<grid, block, 0, s>>>(a, nrm, splits)
   switch (splits > 1 ? (int)EPI_PARTIAL : epi) {
     case EPI_NONE: WS_LAUNCH(EPI_NONE); break;
     case EPI_BIAS: WS_LAUNCH(EPI_BIAS); break;
     case EPI_GELU: WS_LAUNCH(EPI_GELU); break;
-    case EPI_SWIGLU: WS_LAUNCH(EPI_SWIGLU); break;
+    case EPI_SWIGLU:
+      if constexpr (T::kF16) return (int)hipErrorInvalidValue;
+      else WS_LAUNCH(EPI_SWIGLU);
+      break;
     case EPI_RESID: WS_LAUNCH(EPI_RESID); break;
     case EPI_PARTIAL: WS_LAUNCH(EPI_PARTIAL); break;
     default: return (int)hipErrorInvalidValue;
@@ -675,34 +718,52 @@ static int launch_ws_tile(const GemmArgs& a, int epi, int splits, const WsNorm& 
 }
 
 // 64 x 64 tiles: (8192, 16384] columns without splits (_dk_splits, _auto_splits). Narrower products have to be split either
-// way, and the wider tile then moves less of A: 64 x 8192 x 4096 22.8 us at four splits vs 24.0 at two of 64 x 64.
+// way, and the wider tile then moves less of A: 64 x 8192 x 4096 22.8 us at four splits vs 24.0 at two of 64 x 64. Splits are
+// short, and eight waves fill and drain faster: with the reduce, 64 x 4096 x 4096 14.4 us vs 15.8 with four (8 splits), x 14336
+// 28.5 / 30.2, 64 x 6144 x 4096 18.2 / 18.9 (4); unsplit 64 x 28672 x 4096 42.9 / 40.3.
 // W is read once where there is one row block only: not worth a place in the caches then.
 static int launch_ws(const GemmArgs& a, int epi, int splits, const WsNorm& nrm, hipStream_t s) {
-  if (a.M <= 64)
-    return splits == 1 && a.N <= 16384 ? launch_ws_tile<64, 64, true>(a, epi, splits, nrm, s)
-                                       : launch_ws_tile<64, 128, true>(a, epi, splits, nrm, s);
-  if (a.M <= 128) return launch_ws_tile<128, 128, true>(a, epi, splits, nrm, s);
-  return launch_ws_tile<128, 128, false>(a, epi, splits, nrm, s);
+  if (a.M <= 64) {
+    if (splits > 1) return launch_ws_tile<64, 128, 2, 4, true>(a, epi, splits, nrm, s);
+    return a.N <= 16384 ? launch_ws_tile<64, 64, 2, 2, true>(a, epi, splits, nrm, s)
+                        : launch_ws_tile<64, 128, 1, 4, true>(a, epi, splits, nrm, s);
+  }
+  return a.M <= 128 ? launch_ws_tile<128, 128, 2, 4, true>(a, epi, splits, nrm, s)
+                    : launch_ws_tile<128, 128, 2, 4, false>(a, epi, splits, nrm, s);
 }
 
 // The streaming kernel's offsets into a tile's rows are 32 bits wide (_dk_splits draws the same line).
 static bool ws_spans(const GemmArgs& a) { return max(a.K, a.lda) < 1 << 22; }
 
-// K splits of up to 64 rows: the ring costs a microsecond to fill and drain, and a reduce behind it 1 - 2 more than behind
-// the register-staged 64x128 tile with 4 k-tiles in flight (depth 1 / 2 / 8 measured slower,
-// profiles/decode_gemm_prefetch_sweep_r1.jsonl). 64 rows, weights from HBM, register / ring us, with the reduce: 768 x 768
-// 10.4 / 10.2 (6 stages), 8192 x 2048 16.2 / 18.0 (8), 8192 x 4096 22.3 / 23.3 (16), 3072 x 8192 18.6 / 19.3 (16), 5120 x
-// 5120 22.9 / 20.8 (20), 4096 x 14336 31.3 / 30.3 (28). Partials that the next kernel sums (`stages` 6): 1024 x 1024 6.4 / 6.9
-// (4), 3072 x 3072 9.5 / 9.4 (6), 4096 x 4096 12.5 / 11.8 (8), 6272 x 4096 15.9 / 15.0 (16). Unsplit products are faster on
-// the ring at every length (64 x 12288 x 768 9.9 / 9.3).
-static bool ws_pays(const GemmArgs& a, int splits, int stages) {
-  return ws_spans(a) && (a.M > 64 || splits == 1 || a.k_per_split >= stages * 64);
+// The tiles of more than 64 rows (kernels.py, _row_tile): 14 = 128x128, 15 = 128x64, 16 = 64x64, 17 = 64x128, 18 = 192x128.
+template <typename T>
+static int launch_ws_rows(const GemmArgs& a, int epi, int tile, int splits, hipStream_t s) {
+  if (!ws_spans(a)) return (int)hipErrorInvalidValue;
+  switch (tile) {
+    case 14:
+      return a.M <= 128 ? launch_ws_tile<128, 128, 2, 4, true, T>(a, epi, splits, WsNorm{}, s)
+                        : launch_ws_tile<128, 128, 2, 4, false, T>(a, epi, splits, WsNorm{}, s);
+    case 15: return launch_ws_tile<128, 64, 4, 2, false, T>(a, epi, splits, WsNorm{}, s);
+    case 16: return launch_ws_tile<64, 64, 2, 2, false, T>(a, epi, splits, WsNorm{}, s);
+    case 17: return launch_ws_tile<64, 128, 2, 4, false, T>(a, epi, splits, WsNorm{}, s);
+    case 18: return launch_ws_tile<192, 128, 4, 2, false, T>(a, epi, splits, WsNorm{}, s);
+    default: return (int)hipErrorInvalidValue;
+  }
+}
+
+// K splits of up to 64 rows: the ring's fill and drain cost what four stages gain over the register-staged 64x128 tile with 4
+// k-tiles in flight. 64 rows, weights from HBM, register / ring us, with the reduce: 768 x 768 8.0 / 8.6 (3 stages a split), 1024
+// x 1024 8.7 / 9.1 (4), 768 x 3072 10.2 / 9.8 (6), 3072 x 3072 14.5 / 13.6 (6), 4096 x 4096 15.6 / 14.5 (8), 6144 x 4096 18.8 /
+// 17.2 (16), 5120 x 5120 22.9 / 20.6 (20), 4096 x 14336 29.7 / 28.3 (28). Unsplit products are faster on the ring at every
+// length (64 x 12288 x 768 9.9 / 9.3).
+static bool ws_pays(const GemmArgs& a, int splits) {
+  return ws_spans(a) && (a.M > 64 || splits == 1 || a.k_per_split >= 6 * 64);
 }
 
 // Decode tiles: 64x128 by the rule above, else 4 k-tiles in flight per workgroup.
 template <int BM, int BN>
-static int launch_decode_tile(const GemmArgs& a, int epi, int splits, hipStream_t s, int stages = 20) {
-  if (BM == 64 && ws_pays(a, splits, stages)) return launch_ws(a, epi, splits, WsNorm{}, s);
+static int launch_decode_tile(const GemmArgs& a, int epi, int splits, hipStream_t s) {
+  if (BM == 64 && ws_pays(a, splits)) return launch_ws(a, epi, splits, WsNorm{}, s);
   return launch_tile<BM, BN, 1, 4, 4>(a, epi, splits, s);
 }
 
@@ -850,7 +911,7 @@ DA_EXPORT int da_gemm_dk_splitk(const void* A, int lda, const void* W, void* C, 
   const int nout = (epi == EPI_SWIGLU) ? N / 2 : N;
   const size_t work = (size_t)M * (nout / 8);
   const int blocks = (int)((work + 255) / 256);
-  gemm_splitk_reduce<<<blocks, 256, 0, s>>>((const float*)ws, splits, M, N, epi, (const bf16_t*)bias,
+  gemm_splitk_reduce<BF16T><<<blocks, 256, 0, s>>>((const float*)ws, splits, M, N, epi, (const bf16_t*)bias,
                                              (const bf16_t*)resid, ldr, (bf16_t*)C, ldc, ssq_in, ssq_parts, norm_k,
                                              eps, relu);
   DA_LAUNCH_CHECK();
@@ -866,7 +927,7 @@ DA_EXPORT int da_gemm_partials(const void* A, int lda, const void* W, int M, int
   a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = N; a.k_per_split = K / splits;
   hipStream_t s = (hipStream_t)stream;
   switch (tile) {
-    case 2: return launch_decode_tile<64, 128>(a, EPI_PARTIAL, splits, s, 6);
+    case 2: return launch_decode_tile<64, 128>(a, EPI_PARTIAL, splits, s);
     case 3: return launch_decode_tile<32, 128>(a, EPI_PARTIAL, splits, s);
     case 9: return launch_tile<128, 64, 2, 2, 4>(a, EPI_PARTIAL, splits, s);
     default: return (int)hipErrorInvalidValue;
@@ -893,7 +954,7 @@ DA_EXPORT int da_gemm_rope(const void* A, int lda, const void* W, void* C, int l
 // Tile selection: big tiles when the grid fills 256 CUs, skinny tiles (+ split-K) for decode-sized M.
 // tile: 0 = auto, 1 = 128x128, 2 = weight-streaming 64x128 / 128x128, 3 = 32x128, 4 / 7 = 256x256 phase-split (gemm8p),
 // 6 = GEMV (M = 1), 8 = 128x128 PF4, 9 = 128x64 PF4, 10 = 128x256 phase-split (gemm8p), 11 = 64x128 PF4,
-// 13 = 256x256 four-wave (gemm4w).
+// 13 = 256x256 four-wave (gemm4w), 14 - 18 = weight-streaming 128x128, 128x64, 64x64, 64x128, 192x128 (launch_ws_rows).
 DA_EXPORT int da_gemm_bf16(const void* A, int lda, const void* W, void* C, int ldc,
                            const void* bias, const void* resid, int ldr,
                            int M, int N, int K, int epi, int tile, int splits, void* ws,
@@ -939,6 +1000,7 @@ DA_EXPORT int da_gemm_bf16(const void* A, int lda, const void* W, void* C, int l
     case 8: err = launch_tile<128, 128, 2, 2, 4>(a, epi, splits, s); break;   // mid-M weight streaming
     case 9: err = launch_tile<128, 64, 2, 2, 4>(a, epi, splits, s); break;
     case 11: err = launch_tile<64, 128, 1, 4, 4>(a, epi, splits, s); break;
+    case 14: case 15: case 16: case 17: case 18: err = launch_ws_rows<BF16T>(a, epi, tile, splits, s); break;
     default: return (int)hipErrorInvalidValue;
   }
   if (err || splits == 1) return err;
@@ -946,7 +1008,35 @@ DA_EXPORT int da_gemm_bf16(const void* A, int lda, const void* W, void* C, int l
   const size_t work = (size_t)M * (nout / 8);
   int blocks = (int)((work + 255) / 256);
   if (blocks > 4096) blocks = 4096;
-  gemm_splitk_reduce<<<blocks, 256, 0, s>>>((const float*)ws, splits, M, N, epi, a.bias, a.resid, ldr,
+  gemm_splitk_reduce<BF16T><<<blocks, 256, 0, s>>>((const float*)ws, splits, M, N, epi, a.bias, a.resid, ldr,
                                              a.C, ldc, nullptr, 0, 1, 0.f, relu);
+  DA_LAUNCH_CHECK();
+}
+
+// fp16 product for the encoder's DTYPE=fp16 path: C = epi(A W^T), A [M, K] / W [N, K] / C / bias / resid fp16, fp32
+// accumulation; epi NONE / BIAS / GELU / RESID. tile: 0 = the phase-split kernel with the row-tile height of fewer workgroup
+// waves, 7 / 10 = that with 256 / 128 rows, 14 - 18 as da_gemm_bf16.
+DA_EXPORT int da_gemm_f16(const void* A, int lda, const void* W, void* C, int ldc, const void* bias,
+                          const void* resid, int ldr, int M, int N, int K, int epi, int tile, int splits, void* ws,
+                          void* tail_ws, void* tail_cnt, void* stream) {
+  hipStream_t s = (hipStream_t)stream;
+  if (M < 1 || K % 64 || K < 128 || N % 8 || lda % 8 || ldc % 8) return (int)hipErrorInvalidValue;
+  if (epi != EPI_NONE && epi != EPI_BIAS && epi != EPI_GELU && epi != EPI_RESID) return (int)hipErrorInvalidValue;
+  if (epi == EPI_RESID && (!resid || ldr % 8)) return (int)hipErrorInvalidValue;
+  if (splits < 1 || (K / 64) % splits || (splits > 1 && !ws)) return (int)hipErrorInvalidValue;
+  GemmArgs a{};
+  a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = (bf16_t*)C; a.ws = (float*)ws;
+  a.bias = (const bf16_t*)bias; a.resid = (const bf16_t*)resid;
+  a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc; a.ldr = ldr; a.k_per_split = K / splits;
+  if (tile == 0 || tile == 7 || tile == 10) {
+    if (splits != 1) return (int)hipErrorInvalidValue;
+    if (tail_ws && tail_cnt) { a.tail_ws = (float*)tail_ws; a.tail_cnt = (int*)tail_cnt; }
+    return launch_gemm8p(a, 100 + epi, s, tile == 7 ? 256 : tile == 10 ? 128 : gemm8p_pick_bm(M, N, K, epi));
+  }
+  const int err = launch_ws_rows<F16T>(a, epi, tile, splits, s);
+  if (err || splits == 1) return err;
+  const int blocks = (int)min(((size_t)M * (N / 8) + 255) / 256, (size_t)4096);
+  gemm_splitk_reduce<F16T><<<blocks, 256, 0, s>>>((const float*)ws, splits, M, N, epi, a.bias, a.resid, ldr, a.C, ldc, nullptr,
+                                                  0, 1, 0.f, 0);
   DA_LAUNCH_CHECK();
 }

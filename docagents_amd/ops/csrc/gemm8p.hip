@@ -714,6 +714,16 @@ DA_EXPORT size_t da_gemm_tail_ws(int M, int N, int K, int epi, int tile) {
   return s > 1 ? (size_t)(nt % (long)GEMM_TAIL_WGS) * s * bm * BN * 4 : 0;
 }
 
+// What a product takes, in hundredths of a K-tile's time: whole rounds, and the last one as it would be shared out. tile: the
+// row-tile height's code (10: 128, else 256).
+DA_EXPORT int da_gemm8p_ksteps(int M, int N, int K, int epi, int tile) {
+  const int bm = tile == 10 ? 128 : 256, nk = K / 64;
+  const long t = (long)((M + bm - 1) / bm) * ((N + BN - 1) / BN);
+  if (t < 1 || t >= 0x7fffffff) return 0x7fffffff;
+  const long c = (t - 1) / num_cus() * nk * 100 + tail_cost((int)t, nk, bm, tail_allowed(epi) ? tail_slices((int)t, nk, bm) : 1);
+  return (int)min(c, 0x7fffffffL);
+}
+
 // Which capture a stream is in (0: none).
 DA_EXPORT size_t da_gemm_capture_id(void* stream) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -728,21 +738,4 @@ int launch_gemm8p(const GemmArgs& a, int epi, hipStream_t s, int bm) {
   // buffer resources span the tile's rows from its first one (num_records < 2 GiB)
   if ((size_t)bm * a.lda * 2 >= 0x7ffffff0ull || (size_t)256 * a.K * 2 >= 0x7ffffff0ull) return (int)hipErrorInvalidValue;
   return bm == 128 ? launch8p<128>(a, epi, s) : launch8p<256>(a, epi, s);
-}
-
-// fp16 GEMM for the encoder's DTYPE=fp16 path: C = epi(A W^T), A [M, K] / W [N, K] / C / bias /
-// resid fp16, fp32 accumulation; epi NONE / BIAS / GELU / RESID. Every M on the phase-split tile
-// (128-row tiles below half a chip of 256-row ones): the fp16 path has no decode-sized tiles.
-DA_EXPORT int da_gemm_f16(const void* A, int lda, const void* W, void* C, int ldc, const void* bias,
-                          const void* resid, int ldr, int M, int N, int K, int epi, void* tail_ws, void* tail_cnt,
-                          void* stream) {
-  if (M < 1 || K % 64 || K < 128 || N % 8 || lda % 8 || ldc % 8) return (int)hipErrorInvalidValue;
-  if (epi != EPI_NONE && epi != EPI_BIAS && epi != EPI_GELU && epi != EPI_RESID) return (int)hipErrorInvalidValue;
-  if (epi == EPI_RESID && (!resid || ldr % 8)) return (int)hipErrorInvalidValue;
-  GemmArgs a{};
-  a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = (bf16_t*)C;
-  a.bias = (const bf16_t*)bias; a.resid = (const bf16_t*)resid;
-  a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc; a.ldr = ldr; a.k_per_split = K;
-  if (tail_ws && tail_cnt) { a.tail_ws = (float*)tail_ws; a.tail_cnt = (int*)tail_cnt; }
-  return launch_gemm8p(a, 100 + epi, (hipStream_t)stream, gemm8p_pick_bm(M, N, K, epi));
 }

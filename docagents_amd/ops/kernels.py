@@ -67,6 +67,7 @@ _SIGS = {
     "da_enc_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5
                   + [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_void_p],
     "da_gemm_tail_ws": [c_int] * 5,
+    "da_gemm8p_ksteps": [c_int] * 5,
     "da_gemm_capture_id": [c_void_p],
     "da_gemm_dk_splitk": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                           c_int, c_void_p, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_void_p],
@@ -95,7 +96,7 @@ _SIGS = {
     "da_gemm8p_persist": [c_int],
     "da_gemm4w_variant": [c_int],
     "da_gemm_f16": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
-                    c_void_p, c_void_p, c_void_p],
+                    c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
     "da_flash_attn_f16": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int,
                           c_int, c_int, c_float, c_void_p, c_int, c_void_p],
     "da_layernorm_f16": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
@@ -282,6 +283,11 @@ def _gemm_tail(device, stream: int, M: int, N: int, K: int, epi: int, tile: int 
     return part, cnt
 
 
+def _call_partials(splits: int, M: int, N: int, device):
+    """A product's K-split partials as the call's own (the workspace of a role is one stream's): None if whole."""
+    return torch.empty(splits * M * N, dtype=torch.float32, device=device) if splits > 1 else None
+
+
 def gemv_fusable(M: int, N: int, K: int, epi: int = EPI_NONE) -> bool:
     """True when gemm() runs the batch-1 GEMV (which can also fuse the input RMSNorm)."""
     return M == 1 and K % 512 == 0 and N % 4 == 0 and (epi not in GATED or N % 32 == 0)
@@ -330,15 +336,18 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
         _req(eps > 0, "fused RMSNorm needs eps > 0")
         if gamma is not None:
             _bf16_cuda(gamma, "gamma"); _req(gamma.numel() == K, "gamma must be [K]")
+    ws = None
     if splits <= 0:
-        if tile == 0 and 128 < M < 640:
+        if tile == 0 and 64 < M < ROW_TILES_BELOW and max(K, a.stride(0)) < 1 << 22:
+            tile, splits = _row_tile(M, N, K, epi)
+            ws = _call_partials(splits, M, N, a.device)
+        elif tile == 0 and 128 < M < 640:
             tile, splits = _mid_tile(M, N, K)
         else:
             if tile == 0 and M < 640:
                 tile = _decode_tile(M, N)
             splits = _auto_splits(M, N, K) if tile in (0, 2, 3) or (tile == 9 and M <= 128) else 1
-    ws = None
-    if splits > 1:
+    if splits > 1 and ws is None:
         ws = _workspace(splits * M * N * 4, a.device)
     stream = torch.cuda.current_stream().cuda_stream
     # (gemm8p's rows and tiles)
@@ -488,7 +497,7 @@ def gemm_rope(a, w, pos, cos_sin, H: int, Hkv: int, D: int, slot, k_cache, v_cac
               kv_out: bool = True) -> torch.Tensor:
     """Prefill QKV projection: qkv = a @ w^T with RoPE applied to the q / k heads and the token's
     k / v written to the KV cache (cache [slots, Hkv, max_seq, D]) — one kernel (gemm8p EPI_ROPE)
-    from 256 rows; shorter prefills run gemm + rope_cache (identical roundings). kv_out=False: the
+    from 256 rows on, but where ``_rope_apart``; those and shorter prefills run gemm + rope_cache (identical roundings). kv_out=False: the
     k / v columns of the result may be left unwritten (the attention reads the cache; see
     flash_attn_varlen kv_cache) — only the q columns are defined."""
     _bf16_cuda(a, "a"); _bf16_cuda(w, "w"); _i32(pos, "pos"); _i32(slot, "slot")
@@ -499,7 +508,8 @@ def gemm_rope(a, w, pos, cos_sin, H: int, Hkv: int, D: int, slot, k_cache, v_cac
     _req(cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and cos_sin.shape[1] == D // 2, "cos_sin")
     _req(k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.shape == v_cache.shape
          and k_cache.dim() == 4 and k_cache.shape[1] == Hkv and k_cache.shape[3] == D, "caches")
-    if M < 256 or K % 64 or K < 128 or a.stride(1) != 1 or a.stride(0) % 8 or not w.is_contiguous():
+    plain = K % 64 == 0 and K >= 128 and a.stride(1) == 1 and a.stride(0) % 8 == 0 and w.is_contiguous()
+    if M < 256 or not plain or (a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and _rope_apart(M, N, K)):
         qkv = gemm(a, w, out=out)
         return rope_cache(qkv, pos, cos_sin, H, Hkv, D, slot=slot, k_cache=k_cache, v_cache=v_cache)
     if out is None:
@@ -629,6 +639,69 @@ def _auto_splits(M: int, N: int, K: int) -> int:
     while tiles * s * 2 <= 256 and ksteps % (s * 2) == 0 and ksteps // (s * 2) >= 4:
         s *= 2
     return s
+
+
+# Weight-streaming tiles of more than 64 rows (csrc/gemm.hip): code -> rows, columns, and what a product takes on them in us:
+# the first round's fill and drain, a K-step of 64 of a round, each further round, a reduce and its partials per million
+# values, and a unit's K-step on 1/256 of the chip (what all of them load). Phase-split kernel (csrc/gemm8p.hip): code ->
+# rows, fill, a K-step of 256 columns, the same on 1/256 of the chip. Fitted to 598 products of 65 - 1200 rows (projections,
+# feed-forwards and encoder layers 384 - 4096 wide, weights cold; a median of 5 % off): the choice takes 1.008 times the
+# fastest tile on average and at worst 1.2, and 0.81 times the rules before it (25 up to 1.1 times as long, near ties).
+_ROW_TILES = {14: (128, 128, 8.46, 0.38, -0.06, -0.22, 1.9, 0.14), 15: (128, 64, 5.96, 0.25, 0.83, 1.35, 1.96, 0.1),
+              16: (64, 64, 5.82, 0.16, 1.66, 2.54, 1.26, 0.08), 17: (64, 128, 5.79, 0.26, 0.72, 1.61, 1.78, 0.13),
+              18: (192, 128, 11.58, 0.46, -0.59, -2.04, 1.81, 0.16)}
+_PHASE_TILES = {7: (256, 10.76, 0.67, 0.64), 10: (128, 7.11, 0.55, 0.37)}
+ROW_TILES_BELOW = 1280
+
+
+def _stream_us(M: int, N: int, K: int):
+    """(us, tile, splits) of a product on the fastest weight-streaming tile. Splits: below 8192 columns (wider products
+    cover the CUs), 4 K-steps at least, two rounds of units at most, and 32 MB of partials below 256 rows, 20 MB from there."""
+    ksteps, best = K // 64, None
+    most = (1024 if M < 256 else 640) // (math.ceil(M / 64) * math.ceil(N / 128))
+    for t, (bm, bn, fill, step, again, reduce, part, load) in _ROW_TILES.items():
+        tiles = math.ceil(M / bm) * math.ceil(N / bn)
+        for s in (1, 2, 4, 8):
+            if s > 1 and (N >= 8192 or ksteps % s or ksteps // s < 4 or tiles * s > 520 or s > most):
+                continue
+            rounds, nk = math.ceil(tiles * s / 256), ksteps // s
+            us = fill + rounds * nk * step + (rounds - 1) * again + tiles * s * nk * load / 256
+            if s > 1:
+                us = 1.06 * (us + reduce + part * s * M * N * 1e-6)  # (a close call stays whole)
+            if best is None or us < best[0]:
+                best = us, t, s
+    return best
+
+
+def _phase_us(M: int, N: int, K: int, epi: int, tile: int) -> float:
+    """us of a product on the phase-split kernel, its last round shared where that kernel shares it."""
+    rows, fill, step, load = _PHASE_TILES[tile]
+    tiles = math.ceil(M / rows) * math.ceil(N / 256)
+    return fill + step * lib().da_gemm8p_ksteps(M, N, K, epi, tile) / 100 + load * tiles * (K // 64) / 256
+
+
+@_rule
+def _row_tile(M: int, N: int, K: int, epi: int = EPI_NONE, f16: bool = False):
+    """(tile, splits) of a product of 65 rows to ROW_TILES_BELOW: the fastest by estimate (``_ROW_TILES``). From 640 rows on
+    the phase-split kernel picks its own row height, and keeps what is within 3 %. Below, bf16 residuals are added to the
+    fp32 sums only (that kernel rounds the product first)."""
+    us, tile, splits = _stream_us(M, N, K)
+    if K < 128 or (epi == EPI_RESID and M < 640 and not f16):
+        return tile, splits
+    phase = min((_phase_us(M, N, K, epi, t), t) for t in _PHASE_TILES)
+    if us < phase[0] * (0.97 if M >= 640 else 1):
+        return tile, splits
+    return (0 if M >= 640 else phase[1]), 1
+
+
+@_rule
+def _rope_apart(M: int, N: int, K: int) -> bool:
+    """A QKV projection of 256 rows and more as a weight-streaming product and rope_cache behind it (which reads and writes
+    the result once more; the rotation costs the phase-split kernel 4 us): 432 x 6144 x 4096 54 -> 39 us, 300 x 9216 x 3072 46 -> 34,
+    where 128x256 tiles leave CUs idle; 800 x 6144 x 4096 50 / 54 stays."""
+    tiles = math.ceil(M / 256) * math.ceil(N / 256)
+    return M < ROW_TILES_BELOW and (_stream_us(M, N, K)[0] + 4 + M * N * 1e-6
+                                    < 0.97 * (_phase_us(M, N, K, EPI_ROPE, 7 if tiles >= 256 else 10) + 4))
 
 
 def _reduce_us(M: int, N: int, splits: int) -> float:
@@ -1275,9 +1348,11 @@ def gemm_f16(a, w, bias=None, epi: int = EPI_NONE, resid=None, out=None) -> torc
         out = torch.empty((M, N), dtype=torch.float16, device=a.device)
     _req(out.dtype == torch.float16 and out.shape == (M, N) and out.stride(1) == 1 and out.stride(0) % 8 == 0, "out")
     stream = torch.cuda.current_stream().cuda_stream
-    tail = _gemm_tail(a.device, stream, M, N, K, epi) if M >= 256 else (None, None)
+    tile, splits = _row_tile(M, N, K, epi, True) if M < ROW_TILES_BELOW and max(K, a.stride(0)) < 1 << 22 else (0, 1)
+    ws = _call_partials(splits, M, N, a.device)
+    tail = _gemm_tail(a.device, stream, M, N, K, epi, tile) if tile in (7, 10) or (tile == 0 and M >= 256) else (None, None)
     _check(lib().da_gemm_f16(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
-                             M, N, K, epi, *map(_ptr, tail), c_void_p(stream)), "gemm_f16")
+                             M, N, K, epi, tile, splits, _ptr(ws), *map(_ptr, tail), c_void_p(stream)), "gemm_f16")
     return out
 
 

@@ -1,0 +1,27 @@
+"""Which weight-streaming tile and how many K splits products of 65 rows to some 1000 take."""
+import pytest
+
+from docagents_amd.ops import kernels as K
+
+
+@pytest.mark.parametrize("M,N,Kd,epi,want", [(80, 4096, 1024, K.EPI_GELU, (16, 1)), (80, 28672, 4096, K.EPI_SWIGLU, (14, 1)),
+                                             (200, 28672, 4096, K.EPI_SWIGLU, None), (512, 28672, 4096, K.EPI_SWIGLU, (7, 1)),
+                                             (300, 16384, 3072, K.EPI_SWIGLU, (18, 1)), (900, 768, 3072, K.EPI_RESID, (16, 1)),
+                                             (1000, 28672, 4096, K.EPI_SWIGLU, (0, 1)), (500, 4096, 14336, K.EPI_NONE, (10, 1))])
+def test_tiles(M, N, Kd, epi, want):
+    got = K._row_tile(M, N, Kd, epi)
+    assert want is None or got == want
+    assert got[0] in (0, 7, 10, *K._ROW_TILES)
+
+
+@pytest.mark.parametrize("M", [65, 128, 129, 255, 256, 639, 640, 1279])
+@pytest.mark.parametrize("N", [8, 320, 768, 3072, 8184, 8192, 28672])
+@pytest.mark.parametrize("Kd", [64, 128, 768, 4096, 14336])
+def test_splits(M, N, Kd):
+    """Splits divide K, keep four K-steps each, and their partials stay within 32 MB below 256 rows and 20 MB from there."""
+    for f16 in (False, True):
+        tile, splits = K._row_tile(M, N, Kd, K.EPI_RESID, f16)
+        assert (Kd // 64) % splits == 0 and (splits == 1 or Kd // 64 // splits >= 4)
+        assert splits == 1 or splits * M * N * 4 <= (32 if M < 256 else 20) << 20
+        # a bf16 residual is added to the fp32 sums below 640 rows
+        assert f16 or M >= 640 or tile in K._ROW_TILES
