@@ -1238,44 +1238,71 @@ decode_attn_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __restri
 // Llama-3-70B at TP=8 G=8). The G queries of a KV head form the N=16 side of
 // v_mfma_f32_16x16x32_bf16 (zero-padded), so K and V are read once per KV head instead of being
 // multiplied against each query on the VALU (the G >= 2 path of decode_attn_kernel is VALU-bound).
-// Per wave and 64-key tile:
-//   S^T[key][g] = K·Q^T : A = K rows straight from HBM into registers (non-temporal 16-B loads),
-//                         B = Q^T (registers, loaded once);
-//   softmax over the 64 keys of each query column: 16 values per lane + two cross-lane steps;
-//   O^T[d][g] += V^T·P^T : B = P^T from the S^T registers (k index permuted), A = V^T read from the
-//                         wave's private LDS copy of the V tile with ds_read_b64_tr_b16. The V tile
-//                         is a contiguous [64 x D] block of the cache, so it is copied by LDS-DMA
-//                         (global_load_lds, 1 KiB per wave-instruction) with an XOR chunk swizzle
-//                         on the source address that makes the transposed reads conflict-free.
+// Per wave and 32-key tile:
+//   S^T[key][g] = K·Q^T : A = K rows from the wave's private LDS ring, B = Q^T (registers, loaded once);
+//   softmax over the 32 keys of each query column: 8 values per lane + two cross-lane steps;
+//   O^T[d][g] += V^T·P^T : B = P^T from the S^T registers (k index permuted), A = V^T read with ds_read_b64_tr_b16.
+// K and V tiles are contiguous [32 x D] blocks of the cache, copied by LDS-DMA (1 KiB per wave instruction) with an XOR
+// chunk swizzle on the source address that makes both reads conflict-free. A tile's place is filled again as soon as its
+// fragments are in registers, so a wave's next K tile is on its way beside the softmax and V's beside the next scores (D = 64:
+// another tile more): counted waits, no barrier; rows past the end are out of the resource's range (zeros, no traffic).
+// Bound by HBM and by what a CU can have on its way (some 256 requests, whatever is asked for): K rows loaded straight into A
+// registers were requests of 64 B (four lanes a row), and a workgroup got 31 GB/s of the 57 that whole rows give it. 64 rows of
+// 900 - 3100 keys, 8 heads x 128: 112 -> 87 us (6.0 TB/s), all of 2000 89 -> 83, 33 rows 66 -> 52, 8 of 4000 among 56 of 300
+// 70 -> 55. Two stages for D = 128 leave one workgroup per CU, whose start and end nothing covers: 89, 90, 54, 55.
 // by_len: a row takes at most as many splits as hold chunk_max keys each (256: a split's merge costs what reading 100 - 200
 // keys does), and splits are the slowest grid dimension: as the fastest one, the workgroups of a launch with two splits
 // whose rows need one only were all on the even XCDs (64 rows of 2048 keys: 147 us against 86). A workgroup of a split
-// past the row's keys ends at once. Tried and slower: two tiles in flight per wave (hipcc drains the DMA before the
-// transposed reads, and twice the LDS leaves one workgroup per CU).
+// past the row's keys ends at once.
+// pair_rows: whole rows, up to 64 of them, two workgroups per CU: paired_row (91 -> 87 us in the first case above).
 template <int D>
 __device__ __forceinline__ int vswz(int r) {
   return D == 128 ? ((r & 7) << 1) : (((r >> 1) & 3) << 1);
 }
+template <int D>
+__device__ __forceinline__ int kswz(int r) {
+  return D == 128 ? r & 15 : (r >> 1) & 7;
+}
+
+// The row that workgroup row z of B <= 64 takes, and its keys: the `round` longest first (a workgroup per CU), then from the
+// shortest on, so that the second workgroup of a CU with a long row has a short one; as they come where none is 512 keys off
+// the first (the ranks take 1 us).
+__device__ __forceinline__ int paired_row(const int* __restrict__ lens, int B, int z, int round, int& L) {
+  const int lane = threadIdx.x & 63;
+  const int len = lane < B ? lens[lane] : -1;
+  int row = z;
+  if (__ballot(lane < B && abs(len - __builtin_amdgcn_readfirstlane(len)) > 512)) {
+    int rank = 0;
+    for (int j = 0; j < B; ++j) {
+      const int o = __builtin_amdgcn_readlane(len, j);
+      rank += o > len || (o == len && j < lane);
+    }
+    row = __builtin_ctzll(__ballot(lane < B && rank == (z < round ? z : B - 1 - (z - round))));
+  }
+  L = __builtin_amdgcn_readlane(len, row);
+  return row;
+}
 
 template <int D, int G>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 2)
 decode_attn_gqa_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __restrict__ kc,
                        const bf16_t* __restrict__ vc, const int* __restrict__ lens, const int* __restrict__ slot,
                    const int* __restrict__ pre,
                        int H, int Hkv, int max_seq, int chunk_max, int nsplit, float scale_log2e,
                        float* __restrict__ po, float* __restrict__ pm, float* __restrict__ pl,
-                       bf16_t* __restrict__ out, int ldo, int* __restrict__ cnt, int by_len) {
+                       bf16_t* __restrict__ out, int ldo, int* __restrict__ cnt, int by_len, int pair_rows) {
   static_assert(D == 64 || D == 128, "GQA MFMA decode supports head dims 64 and 128");
-  constexpr int KT = 64, NDS = D / 32, NDT = D / 16, NS = D / 8;   // d-steps (S), d-tiles (O), 16-B chunks/row
-  constexpr int VBYTES = KT * D * 2, NDMA = VBYTES / 1024;
+  constexpr int KT = 32, NDS = D / 32, NDT = D / 16, NS = D / 8;   // d-steps (S), d-tiles (O), 16-B chunks/row
+  constexpr int TB = KT * D * 2, ND = TB / 1024, ST = D == 128 ? 1 : 2;  // bytes and DMA instructions of a tile, stages
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
-  typedef __attribute__((address_space(1))) const void* gptr_t;
-  __shared__ __attribute__((aligned(16))) char sv[4 * VBYTES];
-  __shared__ float swm[4][16], swl[4][16];
+  __shared__ __attribute__((aligned(16))) char ring[4 * ST * 2 * TB + 2 * 4 * 16 * 4 + 16];
+  float (*swm)[16] = (float (*)[16])(ring + 4 * ST * 2 * TB), (*swl)[16] = swm + 4;
 
-  const int hk = by_len ? blockIdx.x : blockIdx.y, b = by_len ? blockIdx.y : blockIdx.z;
+  const int hk = by_len ? blockIdx.x : blockIdx.y;
   const int split = by_len ? blockIdx.z : blockIdx.x;
-  const int L = lens[b];
+  int b = by_len ? blockIdx.y : blockIdx.z, L;
+  if (pair_rows) b = paired_row(lens, gridDim.z, b, pair_rows, L);
+  else L = __builtin_amdgcn_readfirstlane(lens[b]);  // (uniform, for the DMA's resources)
   DA_ASSERT(L >= 0 && L <= max_seq && slot[b] >= 0);
   // by_len: a row's keys evenly over as many splits as hold chunk_max of them each; the others have nothing to do
   const int act = by_len && cnt ? min(nsplit, max(1, (L + chunk_max - 1) / chunk_max)) : nsplit;
@@ -1283,13 +1310,13 @@ decode_attn_gqa_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __re
   const int chunk = dec_chunk(L, act, by_len ? 0x7fffffff : chunk_max);
   const int kstart = split * chunk;
   const int kend = min(L, kstart + chunk);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fg = lane >> 4;
-  const size_t cbase = ((size_t)slot[b] * Hkv + hk) * (size_t)max_seq * D;
-  const int P = pre ? pre[2 * b] : 0;  // shared-prefix keys [0, P) live in slot pre[2b + 1]
-  const size_t pbase = P ? ((size_t)pre[2 * b + 1] * Hkv + hk) * (size_t)max_seq * D : cbase;
+  const size_t cbase = ((size_t)__builtin_amdgcn_readfirstlane(slot[b]) * Hkv + hk) * (size_t)max_seq * D;
+  const int P = pre ? __builtin_amdgcn_readfirstlane(pre[2 * b]) : 0;  // shared-prefix keys [0, P) live in slot pre[2b + 1]
+  const size_t pbase = P ? ((size_t)__builtin_amdgcn_readfirstlane(pre[2 * b + 1]) * Hkv + hk) * (size_t)max_seq * D : cbase;
   DA_ASSERT(P % 64 == 0 && P <= L);
-  char* myv = sv + w * VBYTES;
+  char* mine = ring + w * (ST * 2 * TB);
 
   bf16x8_t qf[NDS];
 #pragma unroll
@@ -1297,98 +1324,127 @@ decode_attn_gqa_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __re
     if (fr < G) qf[ds] = *(const bf16x8_t*)(q + (size_t)b * ldq + (hk * G + fr) * D + ds * 32 + fg * 8);
     else qf[ds] = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
   }
+  // DMA sources within a tile: 1 KiB instruction i covers rows of D elements, chunk position sl holds chunk sl ^ swizzle
+  unsigned ko[8], vo[8];
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    const int p = i * 64 + lane, row = p / NS, sl = p % NS;
+    ko[i] = (unsigned)(row * D * 2 + ((sl ^ kswz<D>(row)) << 4));
+    vo[i] = (unsigned)(row * D * 2 + ((sl ^ vswz<D>(row)) << 4));
+  }
+  auto issue = [&](const bf16_t* cache, const unsigned (&off)[8], int t0, char* dst) __attribute__((always_inline)) {
+    // the tile from key t0 on (none past kend)
+    const int n = __builtin_amdgcn_readfirstlane(max(0, min(KT, kend - t0))) * D * 2;  // (uniform: no loop over resources)
+    const size_t at = (t0 < P ? pbase : cbase) + (size_t)t0 * D;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(cache + at), (short)0, n, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < ND; ++i)  // aux 2 = nt (read once per step; see decode_attn_mfma1_kernel)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(dst + i * 1024), 16, off[i & 7], 0, 0, 2);
+  };
+  // the oldest K or V tile of the ring is in: the 2 ST - 1 issued after it may be on their way
+  auto landed = [&]() __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ND * (2 * ST - 1)) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // transposed V reads: the lane's row, its half of a 16-B chunk and the odd chunk; the row's swizzle of chunk pairs
+  const int vr = 4 * fg + (fr >> 2), vx = vswz<D>(vr) >> 1;
+  const unsigned vrow = vr * (D * 2) + ((fr & 3) >> 1) * 16 + (fr & 1) * 8;
   f32x4_t oacc[NDT];
 #pragma unroll
   for (int i = 0; i < NDT; ++i) oacc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_part = 0.f;
 
+#pragma unroll
+  for (int i = 0; i < ST; ++i) {
+    issue(kc, ko, kstart + (w + 4 * i) * KT, mine + i * 2 * TB);
+    issue(vc, vo, kstart + (w + 4 * i) * KT, mine + i * 2 * TB + TB);
+  }
+#pragma unroll
+  for (int ds = 0; ds < NDS; ++ds) asm volatile("" : "+v"(qf[ds]));  // (waited for here, the tiles on their way)
+  int stage = 0;
   for (int t0 = kstart + w * KT; t0 < kend; t0 += 4 * KT) {
-    const int nk = min(KT, kend - t0);
-    const bool shared = t0 < P;
-    const bf16_t* kb = kc + (shared ? pbase : cbase) + (size_t)t0 * D;
-    const bf16_t* vb = vc + (shared ? pbase : cbase) + (size_t)t0 * D;
-    // ---- K straight to registers (A operand rows = keys), then the V tile by LDS-DMA ----
-    u32x4_t kr[4][NDS];
+    char* kt = mine + stage * 2 * TB;
+    char* vt = kt + TB;
+    // ---- S^T = K Q^T; the K tile's place is free once it is in registers ----
+    landed();
+    bf16x8_t kf[2][NDS];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int ds = 0; ds < NDS; ++ds) {
-        const int key = min(16 * t + fr, nk - 1);
-        const u32x4_t* src = (const u32x4_t*)(kb + (size_t)key * D + ds * 32 + fg * 8);
-        kr[t][ds] = __builtin_nontemporal_load(src);
-      }
+      for (int ds = 0; ds < NDS; ++ds)
+        kf[t][ds] = *(const bf16x8_t*)(kt + (16 * t + fr) * (D * 2) + (((4 * ds + fg) ^ kswz<D>(16 * t + fr)) << 4));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    issue(kc, ko, t0 + 4 * ST * KT, kt);
+    f32x4_t sacc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int i = 0; i < NDMA; ++i) {
-      const int P = i * 64 + lane, row = P / NS, sl = P % NS;
-      const int c = sl ^ vswz<D>(row);
-      const int key = min(row, nk - 1);
-      // aux 2 = nt (read once per step; see decode_attn_mfma1_kernel)
-      __builtin_amdgcn_global_load_lds((gptr_t)(vb + (size_t)key * D + c * 8), (lds_ptr_t)(myv + i * 1024), 16, 0, 2);
-    }
-    // ---- S^T = K Q^T ----
-    f32x4_t sacc[4];
+    for (int ds = 0; ds < NDS; ++ds)
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      sacc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ds = 0; ds < NDS; ++ds) sacc[t] = mfma16(__builtin_bit_cast(bf16x8_t, kr[t][ds]), qf[ds], sacc[t]);
-    }
+      for (int t = 0; t < 2; ++t) sacc[t] = mfma16(kf[t][ds], qf[ds], sacc[t]);
     float mx = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int key = 16 * t + 4 * fg + i;
-        const float sc = key < nk ? sacc[t][i] * scale_log2e : -INFINITY;
+        const float sc = t0 + 16 * t + 4 * fg + i < kend ? sacc[t][i] * scale_log2e : -INFINITY;
         sacc[t][i] = sc;
         mx = fmaxf(mx, sc);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = max_xhalf(mx);
-    const float m_new = fmaxf(m_run, mx);
-    const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-    const float alpha = exp2f(m_run - m_use);
-    m_run = m_new;
-    float psum = 0.f;
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+    mx = max_xhalf(fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1])));
+    if (__ballot(mx > m_run)) {  // (a new maximum is rare after the first tiles)
+      const float m_new = fmaxf(m_run, mx);
+      const float alpha = exp2f(m_run - (m_new == -INFINITY ? 0.f : m_new));
+      m_run = m_new;
+      l_part *= alpha;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+      for (int i = 0; i < NDT; ++i) oacc[i] *= alpha;
+    }
+    const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float p = __builtin_amdgcn_exp2f(sacc[t][i] - m_use);
         sacc[t][i] = p;
-        psum += p;
+        l_part += p;
       }
-    l_part = l_part * alpha + psum;
+    // ---- O^T += V^T P^T: slot j -> key 16(j>>2) + 4fg + (j&3) ----
+    const u32x4_t pw = u32x4_t{pack_bf2(sacc[0][0], sacc[0][1]), pack_bf2(sacc[0][2], sacc[0][3]),
+                               pack_bf2(sacc[1][0], sacc[1][1]), pack_bf2(sacc[1][2], sacc[1][3])};
+    const bf16x8_t pb = __builtin_bit_cast(bf16x8_t, pw);
+    // (row 4 fg + fr / 4 and the one 16 on, whose swizzle is the same; with the builtin hipcc drains the DMA first)
+    landed();
+    const unsigned va0 = (unsigned)(size_t)(lds_ptr_t)vt + vrow;
+    s16x4_t v[2][8];
 #pragma unroll
-    for (int i = 0; i < NDT; ++i) oacc[i] *= alpha;
-    // ---- O^T += V^T P^T: k-step c covers keys 32c..32c+31; slot j -> key 32c + 16(j>>2) + 4fg + (j&3) ----
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's V DMA landed (wave-private LDS)
+    for (int h = 0; h < NDT / 4; ++h) {
+      const int dt = 4 * h;
+      asm volatile("ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %8 offset:%12\n\t"
+                   "ds_read_b64_tr_b16 %2, %9\n\tds_read_b64_tr_b16 %3, %9 offset:%12\n\t"
+                   "ds_read_b64_tr_b16 %4, %10\n\tds_read_b64_tr_b16 %5, %10 offset:%12\n\t"
+                   "ds_read_b64_tr_b16 %6, %11\n\tds_read_b64_tr_b16 %7, %11 offset:%12\n\ts_waitcnt lgkmcnt(0)"
+                   : "=&v"(v[h][0]), "=&v"(v[h][1]), "=&v"(v[h][2]), "=&v"(v[h][3]), "=&v"(v[h][4]), "=&v"(v[h][5]),
+                     "=&v"(v[h][6]), "=&v"(v[h][7])
+                   : "v"(va0 + ((dt ^ vx) << 5)), "v"(va0 + (((dt + 1) ^ vx) << 5)), "v"(va0 + (((dt + 2) ^ vx) << 5)),
+                     "v"(va0 + (((dt + 3) ^ vx) << 5)), "n"(16 * D * 2)
+                   : "memory");
+      if (h == NDT / 4 - 1) issue(vc, vo, t0 + 4 * ST * KT, vt);
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const u32x4_t pw = u32x4_t{pack_bf2(sacc[2 * c][0], sacc[2 * c][1]), pack_bf2(sacc[2 * c][2], sacc[2 * c][3]),
-                                 pack_bf2(sacc[2 * c + 1][0], sacc[2 * c + 1][1]),
-                                 pack_bf2(sacc[2 * c + 1][2], sacc[2 * c + 1][3])};
-      const bf16x8_t pb = __builtin_bit_cast(bf16x8_t, pw);
-      const int q4 = fr >> 2, p4 = fr & 3;
-#pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) {
-        const int col = dt * 16 + 4 * p4;                      // 4 columns of this lane's address
-        const int r0 = 32 * c + 4 * fg + q4, r1 = r0 + 16;
-        const s16x4_t lo = lds_read_tr16(myv + r0 * (D * 2) + (((col >> 3) ^ vswz<D>(r0)) << 4) + (col & 7) * 2);
-        const s16x4_t hi = lds_read_tr16(myv + r1 * (D * 2) + (((col >> 3) ^ vswz<D>(r1)) << 4) + (col & 7) * 2);
-        const bf16x8_t va = bf16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        oacc[dt] = mfma16(va, pb, oacc[dt]);
+      for (int j = 0; j < 4; ++j) {
+        const s16x4_t lo = v[h][2 * j], hi = v[h][2 * j + 1];
+        oacc[dt + j] = mfma16(bf16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, pb, oacc[dt + j]);
       }
     }
-    // the next tile's DMA rewrites this wave's V region: finish the tr-reads first
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    stage = stage + 1 == ST ? 0 : stage + 1;
   }
   // ---- merge the 4 waves: per-query (m, l) and O^T partials through LDS ----
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (pieces past the end write zeros)
   float l_tot = l_part + __shfl_xor(l_part, 16, 64);
   l_tot = sum_xhalf(l_tot);
   if (fg == 0) { swm[w][fr] = m_run; swl[w][fr] = l_tot; }
-  __syncthreads();  // every wave is done with its V region
-  float* so = (float*)sv;  // [4][16][D]
+  __syncthreads();  // every wave is done with its ring
+  float* so = (float*)ring;  // [4][16][D]
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
@@ -1407,8 +1463,7 @@ decode_attn_gqa_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __re
     }
     dec_store(o, M, ls, b, hk * G + g, d, H, nsplit, split, D, po, pm, pl, out, ldo, act);
   }
-  __shared__ int s_last;
-  dec_finish<D, G>(po, pm, pl, H, Hkv, nsplit, b, hk, cnt, out, ldo, &s_last, act);
+  dec_finish<D, G>(po, pm, pl, H, Hkv, nsplit, b, hk, cnt, out, ldo, (int*)(swl + 4), act);
 }
 
 // MHA decode attention on MFMA for few (row, kv head) pairs (batch 1..: the p50 path). The VALU
@@ -1721,10 +1776,11 @@ static int launch_decode(int G, dim3 grid, hipStream_t s, const bf16_t* q, int l
   if (rope.cs) return (int)hipErrorInvalidValue;  // fused RoPE: MHA kernel only
   if constexpr (D == 64 || D == 128) {
     const dim3 grid_g = by_len ? dim3(Hkv, grid.z, nsplit) : grid;
+    const int pair_rows = nsplit == 1 && !by_len && grid.z <= 64 && Hkv * grid.z > 256 ? 256 / Hkv : 0;
     switch (G) {
-      case 2: decode_attn_gqa_kernel<D, 2><<<grid_g, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt, by_len); break;
-      case 4: decode_attn_gqa_kernel<D, 4><<<grid_g, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt, by_len); break;
-      case 8: decode_attn_gqa_kernel<D, 8><<<grid_g, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt, by_len); break;
+      case 2: decode_attn_gqa_kernel<D, 2><<<grid_g, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt, by_len, pair_rows); break;
+      case 4: decode_attn_gqa_kernel<D, 4><<<grid_g, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt, by_len, pair_rows); break;
+      case 8: decode_attn_gqa_kernel<D, 8><<<grid_g, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt, by_len, pair_rows); break;
       default: return (int)hipErrorInvalidValue;
     }
     return (int)hipGetLastError();

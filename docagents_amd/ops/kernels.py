@@ -698,7 +698,7 @@ def _row_tile(M: int, N: int, K: int, epi: int = EPI_NONE, f16: bool = False):
 def _rope_apart(M: int, N: int, K: int) -> bool:
     """A QKV projection of 256 rows and more as a weight-streaming product and rope_cache behind it (which reads and writes
     the result once more; the rotation costs the phase-split kernel 4 us): 432 x 6144 x 4096 54 -> 39 us, 300 x 9216 x 3072 46 -> 34,
-    where 128x256 tiles leave CUs idle; 800 x 6144 x 4096 50 / 54 stays."""
+    800 x 6144 x 4096 54 -> 50, where 128x256 tiles leave CUs idle."""
     tiles = math.ceil(M / 256) * math.ceil(N / 256)
     return M < ROW_TILES_BELOW and (_stream_us(M, N, K)[0] + 4 + M * N * 1e-6
                                     < 0.97 * (_phase_us(M, N, K, EPI_ROPE, 7 if tiles >= 256 else 10) + 4))

@@ -1,0 +1,51 @@
+"""Grouped-query decode attention: whole rows paired by length, tiles of 32 keys and their ends, against 64-bit attention."""
+import random
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from docagents_amd.ops import kernels as K
+
+
+def _attention(q, kc, vc, lens, slot, H, Hkv, D, pre):
+    out = []
+    for b, n in enumerate(lens):
+        k, v = kc[slot[b], :, :n].double(), vc[slot[b], :, :n].double()
+        if pre and pre[0]:
+            k, v = k.clone(), v.clone()
+            k[:, :pre[0]], v[:, :pre[0]] = kc[pre[1], :, :pre[0]].double(), vc[pre[1], :, :pre[0]].double()
+        s = (q[b].double().view(Hkv, H // Hkv, D) @ k.transpose(1, 2)) * D ** -0.5
+        out.append((torch.softmax(s, -1) @ v).reshape(-1))
+    return torch.stack(out)
+
+
+def _lens(kind, B, S):
+    r = random.Random(B * 31 + S)
+    if kind == "edges":
+        return [(1, 31, 32, 33, 63, 64, 65, 127, 128, 129, S - 1, S)[i % 12] for i in range(B)]
+    if kind == "equal":
+        return [S // 2 + i % 7 for i in range(B)]
+    return [r.randint(1, S) for _ in range(B)]
+
+
+# more and fewer row-and-head pairs than CUs, one row a round, the most rows that are paired and one more
+@pytest.mark.parametrize("B,Hkv,G,D,S", [(33, 8, 4, 128, 2112), (64, 8, 2, 128, 4096), (65, 8, 4, 128, 2112), (64, 4, 8, 64, 2112),
+                                         (40, 8, 2, 64, 2112), (3, 2, 4, 64, 512), (5, 8, 8, 128, 1024)])
+@pytest.mark.parametrize("kind", ["edges", "equal", "ragged"])
+@pytest.mark.parametrize("prefix", [0, 64])
+def test_rows(B, Hkv, G, D, S, kind, prefix):
+    H, g = Hkv * G, torch.Generator(device="cuda").manual_seed(B + D)
+    lens = [max(n, prefix + 1) for n in _lens(kind, B, S)]
+    kc, vc = (torch.randn(B + 1, Hkv, S, D, device="cuda", generator=g).bfloat16() for _ in range(2))
+    q = torch.randn(B, H * D, device="cuda", generator=g).bfloat16()
+    slot = random.Random(1).sample(range(B), B)
+    to = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    pre = to([[prefix, B]] * B) if prefix else None
+    got = K.decode_attn(q, kc, vc, to(lens), to(slot), H, Hkv, D, S, pre=pre)
+    want = _attention(q, kc, vc, lens, slot, H, Hkv, D, (prefix, B))
+    # weights and the result are rounded to bf16; the values are within 6 of zero
+    assert (got.double() - want).abs().max() <= 2.0 ** -8 * (want.abs().max() + 6)
+    assert torch.equal(K.decode_attn(q, kc, vc, to(lens), to(slot), H, Hkv, D, S, pre=pre), got)
