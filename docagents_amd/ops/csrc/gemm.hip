@@ -230,8 +230,8 @@ gemm_bf16_kernel(GemmArgs p) {
 }
 
 // ------------------------------------------------------------------------------------------
-// Weight-streaming product (33 rows to some 1000: decoding, short prompts, short texts; bf16, and fp16 for the encoders).
-// K in stages of 64; tiles of 64 x 128, 64 x 64, 128 x 64, 128 x 128 and 192 x 128, four or eight waves.
+// Weight-streaming product (2 rows to some 1000: decoding, short prompts, short texts; bf16, and fp16 for the encoders).
+// K in stages of 64; tiles of 32 x 64, 32 x 128, 64 x 128, 64 x 64, 128 x 64, 128 x 128 and 192 x 128, four or eight waves.
 //  * A stage (8 - 24 KB of A, 8 or 16 KB of W) arrives by LDS-DMA in a ring that fills LDS. What a CU can have on its way
 //    beyond the L2 is 32 KB whatever is asked for (57 GB/s from HBM or the last-level cache, 142 GB/s from L2; loads into
 //    registers the same), and A's pieces wait in that queue behind W's, so the tile's bytes per product bound it, not the
@@ -248,7 +248,7 @@ gemm_bf16_kernel(GemmArgs p) {
 //    on its column only. With more row blocks it gained nothing, and sums are in the phase-split kernel's order.
 //  * W is the MFMA's A operand, so a lane holds 4 consecutive columns of a row and stores them without staging.
 //  * nrm: the rows of A are the raw residual stream, and the result's rows are scaled by rsqrt(sum of the parts'
-//    squares / norm_k + eps) (gemm_dk.hip).
+//    squares / norm_k + eps) (gemm_dk.hip); the parts are added up while the first stages are on their way.
 constexpr int WS_LDS = 160 * 1024;
 
 struct WsNorm {
@@ -261,13 +261,15 @@ template <int BM, int BN, int WGM, int WGN, int EPI, bool NT, typename T>
 __global__ void __launch_bounds__(64 * WGM * WGN)
 gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
   constexpr int NW = WGM * WGN, A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128;
-  constexpr int ST = WS_LDS / STAGE < 10 ? WS_LDS / STAGE : 10;  // stages of the ring
+  constexpr bool NORM = BM <= 64 && EPI != EPI_PARTIAL;
+  constexpr int SCALES = NORM ? (NW + 1) * BM * 4 : 0;                 // the rows' scales, and each wave's part of the sums
+  constexpr int ST = (WS_LDS - SCALES) / STAGE < 10 ? (WS_LDS - SCALES) / STAGE : 10;  // stages of the ring
   constexpr int PA = BM / 8 / NW, PW = BN / 8 / NW;  // LDS-DMA instructions of a wave per stage
   constexpr int P = PA + PW, PH = P / 2;  // of them beside a stage's first half
   constexpr int FM = BM / WGM / 16, FN = BN / WGN / 16, WROWS = FM * 16, WCOLS = FN * 16;
   static_assert(PA >= 1 && PA <= 4 && PW >= 1 && PW <= 4 && FN % 2 == 0 && ST >= 3 && P * (ST - 2) < 64, "tile");
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
-  __shared__ __attribute__((aligned(16))) char smem[ST * STAGE];
+  __shared__ __attribute__((aligned(16))) char smem[ST * STAGE + SCALES];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = w / WGN, wn = w % WGN;
   const int fr = lane & 15, fg = lane >> 4;
@@ -332,6 +334,15 @@ gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   };
+  // the rows' sums of squares: thread = (part, 4 rows), 8 parts each on their way before the ring's first stages
+  [[maybe_unused]] float* scale = (float*)(smem + ST * STAGE);
+  [[maybe_unused]] f32x4_t sq[8];
+  constexpr int RQ = BM / 4, PL = 64 * NW / RQ;  // row quads, parts at a time
+  if constexpr (NORM)
+    if (nrm.ssq)
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        sq[j] = *(const f32x4_t*)(nrm.ssq + (size_t)min(tid / RQ + j * PL, nrm.parts - 1) * 64 + tid % RQ * 4);
   open();
 #pragma unroll 1
   for (int i = 0; i < ST - 1; ++i) {
@@ -339,6 +350,26 @@ gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
     for (int j = 0; j < P; ++j) piece(j);
     next_stage();
   }
+  if constexpr (NORM)
+    if (nrm.ssq) {
+      f32x4_t s{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += tid / RQ + j * PL < nrm.parts ? sq[j] : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int q = tid / RQ + 8 * PL; q < nrm.parts; q += PL) s += *(const f32x4_t*)(nrm.ssq + (size_t)q * 64 + tid % RQ * 4);
+#pragma unroll
+      for (int o = RQ; o < 64; o <<= 1)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += __shfl_xor(s[e], o, 64);
+      if (lane < RQ) *(f32x4_t*)(scale + (w + 1) * BM + lane * 4) = s;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      if (tid < BM) {
+        float t = 0.f;
+#pragma unroll
+        for (int i = 1; i <= NW; ++i) t += scale[i * BM + tid];
+        scale[tid] = rsqrtf(t / nrm.norm_k + nrm.eps);  // (visible at the first stage's barrier)
+      }
+    }
 
   int rd = 0;  // the slot that is read next
   const int sw = (fr >> 1) & 7;
@@ -399,7 +430,8 @@ gemm_ws_kernel(GemmArgs p, WsNorm nrm, int splits) {
       const int m = m0 + wm * WROWS + i * 16 + fr;
       if (m >= p.M) continue;
       float inv = 1.f;
-      if (nrm.ssq) inv = rsqrtf(sum_strided(nrm.ssq + m, nrm.parts, 64) / nrm.norm_k + nrm.eps);
+      if constexpr (NORM)
+        if (nrm.ssq) inv = scale[wm * WROWS + i * 16 + fr];  // (one row block: up to 64 rows)
       if constexpr (EPI == EPI_SWIGLU) {
 #pragma unroll
         for (int j = 0; j < FN; j += 2) {
@@ -721,8 +753,12 @@ static int launch_ws_tile(const GemmArgs& a, int epi, int splits, const WsNorm& 
 // way, and the wider tile then moves less of A: 64 x 8192 x 4096 22.8 us at four splits vs 24.0 at two of 64 x 64. Splits are
 // short, and eight waves fill and drain faster: with the reduce, 64 x 4096 x 4096 14.4 us vs 15.8 with four (8 splits), x 14336
 // 28.5 / 30.2, 64 x 6144 x 4096 18.2 / 18.9 (4); unsplit 64 x 28672 x 4096 42.9 / 40.3.
+// Up to 32 rows only wide ones come here (kernels.py, dk_wide).
 // W is read once where there is one row block only: not worth a place in the caches then.
 static int launch_ws(const GemmArgs& a, int epi, int splits, const WsNorm& nrm, hipStream_t s) {
+  if (a.M <= 32 && splits == 1)
+    return a.N <= 16384 ? launch_ws_tile<32, 64, 2, 2, true>(a, epi, splits, nrm, s)
+                        : launch_ws_tile<32, 128, 1, 4, true>(a, epi, splits, nrm, s);
   if (a.M <= 64) {
     if (splits > 1) return launch_ws_tile<64, 128, 2, 4, true>(a, epi, splits, nrm, s);
     return a.N <= 16384 ? launch_ws_tile<64, 64, 2, 2, true>(a, epi, splits, nrm, s)
@@ -873,7 +909,7 @@ splitk_reduce_resid_ssq(const float* __restrict__ ws, int splits, int M, int N, 
   if (lane == 0) ssq_out[(size_t)blockIdx.x * 64 + m] = sq;
 }
 
-// gemm_dk's contract (DkArgs semantics, csrc/gemm_dk.hip) for 33..64 rows on the 64x128 streaming
+// gemm_dk's contract (DkArgs semantics, csrc/gemm_dk.hip) for 33..64 rows, and up to 32 without splits, on the streaming
 // tiles: epi NONE / BIAS / SWIGLU with an optional deferred norm of A's rows (ssq_in: the raw
 // residual stream as A, the row scale applied in the reduce, or without splits in the epilogue), or EPI_RESID with optional per-part
 // sums of squares out (ssq_out: [N / 512][64]). splits 1: no reduce (not with ssq_out); else ws holds

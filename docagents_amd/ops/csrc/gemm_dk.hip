@@ -17,6 +17,10 @@
 // A and W fragments are in flight per wave (counted vmcnt waits: the ring is indexed by unrolled
 // slot, loads issued in k order).
 //
+// From K = 4096 on the tiles of an XCD begin at K chunks of their own: all at the same columns of rows a power of two apart,
+// they ask the same few channels at a time. 8192 x 4096, 4 / 16 / 32 rows: 16.7 / 16.9 / 18.3 -> 13.5 / 13.7 / 16.0 us, 6144 x 4096
+// 16.6 / 16.8 / 17.8 -> 13.7 / 14.2 / 17.5, 4096 x 14336 23.6 / 26.3 / 33.3 -> 22.4 / 25.1 / 33.1; a shorter K gains nothing.
+//
 // Deferred RMSNorm (NORM): the decode layer's norms ride here instead of in a reduce launch. The
 // producer of the residual stream (EPI_RESID) writes, next to x, per-(workgroup, row) sums of squares
 // of its bf16 output slice (ssq_out [parts][64]); the consumer reads x itself as A and scales each A
@@ -63,11 +67,12 @@ gemm_dk_kernel(DkArgs p) {
   const int Mb = min(BM, p.M - m0);  // rows of this block
   const int nch = p.K / KC;
   const int kl = nch - 1;
+  const int rot = nch >= 16 ? (tile >> 3) % nch : 0;  // the chunk that this tile begins with
 
   // ---- global -> registers: whole 512-B row segments (32 lanes x 16 B per row), full lines ----
   u32x4_t rw[PF][LW], ra[PF][LA];
   auto gload = [&](u32x4_t (&xw)[LW], u32x4_t (&xa)[LA], int c) {
-    const int k0 = c * KC;
+    const int cr = c + rot, k0 = (cr < nch ? cr : cr - nch) * KC;
 #pragma unroll
     for (int i = 0; i < LW; ++i) {
       const int idx = tid + 256 * i, r = idx >> 5, ch = idx & 31;

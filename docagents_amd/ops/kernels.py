@@ -376,6 +376,14 @@ def dk_fusable(M: int, N: int, K: int, epi: int = EPI_NONE) -> bool:
             and epi in (EPI_NONE, EPI_BIAS, EPI_RESID, *GATED) and (epi not in GATED or N % 32 == 0))
 
 
+def dk_wide(M: int, N: int, K: int, lda: int) -> bool:
+    """Products of up to 32 rows and more than 8192 columns: 32-row streaming tiles (csrc/gemm.hip) cover the CUs without
+    gemm_dk's K split in the workgroup, whose 64-wide tile leaves a CU one workgroup and ends in rounds that are not full.
+    16 rows, dk / streaming us: 28672 x 4096 with the norm 50 / 41 (45 / 40 without), 128256 x 4096 191 / 163, 16384 x 3072
+    21.7 / 20.7, 9216 x 3072 18.3 / 17.6 (32 rows: 22.8 / 20.0), 12608 x 4096 21.6 / 20.8; below the line 8192 x 4096 13.7 / 19.4."""
+    return 1 <= M <= DK_SPLITK_ABOVE and N > 8192 and max(K, lda) <= 8192
+
+
 def _dk_splitk(M: int, N: int) -> bool:
     return DK_SPLITK_ABOVE < M <= 64 and N % 512 == 0
 
@@ -436,6 +444,10 @@ def gemm_dk(a, w, epi: int = EPI_NONE, bias=None, resid=None, out=None, norm_in=
     if ssq_out is not None:
         _req(epi == EPI_RESID and ssq_out.dtype == torch.float32 and ssq_out.is_contiguous()
              and ssq_out.numel() >= dk_parts(N, M) * 64, "bad ssq_out")
+    if dk_wide(M, N, K, a.stride(0)) and ssq_out is None:
+        _check(lib().da_gemm_dk_splitk(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid),
+                                       ldr, M, N, K, epi, _ptr(ssq), parts, K, float(eps), None, None, 1, _stream()), "gemm_dk_wide")
+        return out
     if _dk_splitk(M, N) or (DK_SPLITK_ABOVE < M <= 64 and ssq_out is None):
         # (rows too long for the unsplit tile's 32-bit offsets: the reduce carries the epilogue)
         splits = _dk_splits(N, K, ssq_out is not None or max(K, a.stride(0)) >= 1 << 22)
