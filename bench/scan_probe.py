@@ -1,6 +1,6 @@
 """Dense-scan probe: time the streaming top-k kernels (ops.kernels.topk_dense's route) on one shard
-for several batch sizes, similarity floors (a floor no row passes = pure streaming, no candidate
-work) and rows per wave, to separate HBM streaming from the top-K bookkeeping."""
+for several batch sizes, similarity floors (a floor no row passes: nothing to pick) and least rows per
+wave, to separate HBM streaming from the selection."""
 import argparse
 import json
 import math
@@ -34,7 +34,7 @@ def main():
         base = max(64, math.ceil(N / (256 * 16) / 16) * 16)
         for thr in (-1.0, 0.95):
             for rpw in (base, base * 4):
-                ws = K._workspace(int(lib.da_topk_stream_ws(N, q, a.k, rpw)), dev)
+                ws = K._workspace(int(lib.da_topk_stream_ws(N, q, rpw)), dev)
                 out_s = torch.empty((q, a.k), dtype=torch.float32, device=dev)
                 out_i = torch.empty((q, a.k), dtype=torch.int32, device=dev)
 

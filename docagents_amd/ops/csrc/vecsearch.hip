@@ -122,43 +122,18 @@ topk_dense_kernel(const bf16_t* __restrict__ X, int N, int d, const int* __restr
 }
 
 // ------------------------------------------------------------------------------------------------
-// Streaming dense scan (d % 128 == 0): the whole-shard pass of flat search, IVF coarse probing and
-// k-means assignment, built to run at HBM speed.
-//
-//  * Every wave is an independent worker over its own contiguous run of rows, 16 rows per MFMA
-//    tile, against the workgroup's 16 queries (B fragments from LDS, one copy per workgroup).
-//  * The rows stream from HBM through a ring of R groups (4 MFMA k-steps = 64 B per lane each)
-//    that runs across tile boundaries: group s + R is requested as soon as group s is consumed,
-//    so ~R * 4 KB per wave stay in flight (the old kernel issued one row load, waited, issued the
-//    next: 3.5 TB/s on a 10M x 1024 shard).
-//  * A tile's 16 x 16 scores are tested against each query's running k-th best; only rows that beat
-//    it do any top-K work (TdWave below).
-//  * Up to 16 queries (one query block): topk_dense_stream_kernel, every wave its own rows, the
-//    rows loaded non-temporally straight into the MFMA A registers.
-//  * 17 and more: topk_dense_mq_kernel, the workgroup's 4 waves = 4 (or 8) query blocks over the SAME
-//    rows: each 16-row tile is read from HBM once into LDS and feeds all four waves (B fragments of
-//    a wave's queries live in its registers). Query blocks as separate workgroups over the same
-//    rows, even dispatched back to back to one XCD, missed in L2 and read the shard once per block
-//    (batch 64: 12.1 ms vs 3.6 ms for batch 1, profiles/r5/index/).
-// out [row blocks (padded to 8), Q, K]: one unsorted top-K list per (workgroup, query), ordered and
-// merged by topk_merge_kernel.
-constexpr int TD_G = 4;    // MFMA k-steps (of 32) per load group: 64 B per lane
-
-// One wave's top-K state for its 16 queries over a run of 16-row tiles. Per query, 64 LDS slots:
-// [0, K) the current top-K (unsorted), then one candidate sub-buffer of SB slots for each of the
-// query's 4 lanes; the k-th best score sits in a register of those lanes.
-//  * tile(): a lane's rows that beat the k-th best pass the doc filter / floor and go to ITS
-//    sub-buffer at a lane-local count: no cross-lane traffic on the append path.
-//  * cut(): once a sub-buffer could overflow on the next tile, the query's list + buffered rows (one
-//    per lane, <= 64) are cut to the top K by a radix select on the ballot unit: 32 rounds of ballot
-//    + popcount on an order-preserving integer image of the score find the K-th largest (ties at
-//    the threshold go to the smaller row id), the winners are compacted into [0, K) by mbcnt. The
-//    sorted-list merge it replaces (K rounds of a 6-level shuffle argmax per (tile, query), then
-//    per 48 candidates) stalled the workgroup's load pipeline: 64 queries took 10.5 ms against
-//    3.7 ms with no candidate work (bench/scan_probe.py, profiles/r5/index/).
-// Lists leave unsorted; topk_merge_kernel orders them.
-constexpr int TD_SL = 64;  // LDS slots per (wave, query)
-
+// Streaming dense scan (d = 384, 768, 1024): the whole-shard pass of flat search and IVF coarse probing, built to run at HBM
+// speed. In two launches:
+//  1. a scan that leaves, per query, the best score of every group of 16 rows (a power of two of them from 65536 groups on)
+//     that the filter and the floor let pass: four selects, two cross-lane steps and a store of 4 B per group and query;
+//  2. topk_pick_kernel: the K best groups of a query hold its K best rows (whoever is in another group has K groups before
+//     it, each with a better row, or an equal one of a smaller id); it scores those groups again, with the scan's own
+//     instructions, and orders the rows.
+// A top-K list kept beside the scan starts empty in every workgroup, so with a few hundred to a few thousand rows each nearly
+// every tile held a row that beat the list so far: appending, cutting and merging took 20 - 85 % of a pass. Whole searches, us,
+// lists / groups: 1.25 M x 1024, K = 5, 1 query 506 / 395, 16 600 / 417, 64 708 / 443, 128 795 / 496; 411812 x 768, 113
+// queries, K = 5 309 / 148, K = 20 518 / 161; 75595 x 384, 36 queries, K = 19 159 / 33; 30000 x 1024, 20 queries 69 / 29;
+// 512 x 768 (centroids), 24 queries 27 / 19.
 __device__ __forceinline__ unsigned td_key(float v, int id) {  // larger = better; empty (id < 0) = 0
   const unsigned u = __float_as_uint(v + 0.f);  // (-0 as 0)
   return id < 0 ? 0u : ((u & 0x80000000u) ? ~u : (u | 0x80000000u));
@@ -217,264 +192,220 @@ __device__ __forceinline__ float td_cut(float v, int id, int K, int lane, float*
   return t != t ? -INFINITY : t;  // (a prefix below -FLT_MAX)
 }
 
-struct TdWave {
-  float* cs; int* ci;  // [16][TD_SL] scores / rows
-  int K, SB, lane, fr, fg;
-  float kth;  // this lane's query (fr): its current k-th best score
-  int cnt;    // entries in this lane's sub-buffer
 
-  __device__ __forceinline__ void init(float* s, int* i, int k) {
-    cs = s; ci = i; K = k; SB = (TD_SL - k) / 4;  // K <= 32: SB >= 8
-    lane = threadIdx.x & 63; fr = lane & 15; fg = lane >> 4;
-    kth = -INFINITY; cnt = 0;
-    for (int j = lane; j < 16 * TD_SL; j += 64) { cs[j] = -INFINITY; ci[j] = -1; }
+// What a scan leaves of a run of 16-row tiles for a wave's 16 queries: lane (fr, fg) of query fr keeps groups 4 fg .. 4 fg + 3
+// of every 16 and stores them together. A run's groups are padded to a multiple of 4 with -inf.
+struct GroupMax {
+  float* line;  // this lane's query's groups of this run; null: no such query
+  int slots, lg, g;  // groups of a run (padded), log2 of a group's tiles, groups so far
+  f32x4_t keep;
+  float best;
+
+  __device__ __forceinline__ void init(float* l, int n, int log_tiles) {
+    line = l; slots = n; lg = log_tiles; g = 0;
+    best = -INFINITY;
+    keep = f32x4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
   }
-  // cut the lists of the queries set in `full` (bit q) back to their top K
-  __device__ __forceinline__ void flush(const unsigned long long full) {
-    wave_sync_lds();
-    float kq = -INFINITY;  // lane q < 16: query q's new k-th best
-    for (unsigned long long left = full; left; left &= left - 1) {
-      const int q = __builtin_ctzll(left);
-      // lane j: list slot j (< K) or sub-buffer b = (j - K) / SB entry (j - K) % SB, live below the
-      // count of lane q + 16 b
-      const int b = lane < K ? 0 : min((lane - K) / SB, 3), e = lane < K ? 0 : lane - K - b * SB;
-      const int nb = __shfl(cnt, q + 16 * b, 64);
-      const bool live = lane < K || (lane < K + 4 * SB && e < nb);
-      const float v = live ? cs[q * TD_SL + lane] : -INFINITY;
-      const int id = live ? ci[q * TD_SL + lane] : -1;
-      const float t = td_cut(v, id, K, lane, cs + q * TD_SL, ci + q * TD_SL);
-      if (lane == q) kq = t;
-    }
-    const float kn = __shfl(kq, fr, 64);
-    if ((full >> fr) & 1ull) { kth = kn; cnt = 0; }
+  __device__ __forceinline__ void flush(int at, int fg) {
+    if (line && at + 4 * fg < slots) *(f32x4_t*)(line + at + 4 * fg) = keep;
+    keep = f32x4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
   }
-  // a finished 16 x 16 tile: lane (fr, fg) holds rows row0 + i (row0 = tile base + 4 fg) of query fr
-  // (global query index qrow); rows from `end` on are padding. slot: the doc slot of row fr of the tile, loaded with
-  // its rows (0 without slots): most tiles of a whole-shard pass have a candidate somewhere, and a load of its slot
-  // here had every wave of the workgroup wait for memory once a tile.
-  __device__ __forceinline__ void tile(const f32x4_t& acc, int row0, int end, bool qok, float thr, int slot,
-                                       const unsigned* __restrict__ bitmap, int W, int qrow) {
-    bool cand = false;
+  __device__ __forceinline__ void close(int fg) {  // the group ends
+    const int own = (g >> 2) & 3;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) cand |= qok && row0 + i < end && acc[i] >= thr && acc[i] > kth;
-    if (!__ballot(cand)) return;  // the common case after the first tiles
-    float* bs = cs + fr * TD_SL + K + fg * SB;
-    int* bi = ci + fr * TD_SL + K + fg * SB;
+    for (int i = 0; i < 4; ++i) keep[i] = fg == own && (g & 3) == i ? best : keep[i];
+    best = -INFINITY;
+    if ((++g & 15) == 0) flush(g - 16, fg);
+  }
+  // tile t of the run: lane (fr, fg) holds the scores of rows row0 .. row0 + 3 (row0 = its first row + 4 fg) whose doc slots
+  // are sl (removed rows: -1); rows from `end` on are padding
+  __device__ __forceinline__ void tile(const f32x4_t& acc, int t, int row0, int end, float thr, const int (&sl)[4],
+                                       const unsigned* __restrict__ bits, int W, int fg) {
+    float m = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int row = row0 + i;
-      const int sl = __shfl(slot, 4 * fg + i, 64);
-      bool ok = qok && row < end && acc[i] >= thr && acc[i] > kth && sl >= 0;  // removed rows (slot -1) never match
-      if (ok && bitmap) ok = (sl >> 5) < W && ((bitmap[(size_t)qrow * W + (sl >> 5)] >> (sl & 31)) & 1u);
-      if (ok) { bs[cnt] = acc[i]; bi[cnt] = row; ++cnt; }
+      bool ok = row0 + i < end && sl[i] >= 0 && acc[i] >= thr;
+      if (bits && ok) ok = (sl[i] >> 5) < W && ((bits[sl[i] >> 5] >> (sl[i] & 31)) & 1u);
+      m = fmaxf(m, ok ? acc[i] : -INFINITY);
     }
-    // a lane's next tile adds <= 4: cut the queries with a sub-buffer past SB - 4
-    const unsigned long long over = __ballot(cnt > SB - 4);
-    if (over) flush((over | (over >> 16) | (over >> 32) | (over >> 48)) & 0xffffull);
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+    best = fmaxf(best, max_xhalf(fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]))));
+    if (((t + 1) & ((1 << lg) - 1)) == 0) close(fg);
   }
-  // every list cut to its top K (unsorted) in slots [0, K)
-  __device__ __forceinline__ void finish() {
-    const unsigned long long rest = __ballot(cnt > 0);
-    if (rest) flush((rest | (rest >> 16) | (rest >> 32) | (rest >> 48)) & 0xffffull);
-  }
-  // merge another wave's finished lists (same 16 queries) into this wave's
-  __device__ __forceinline__ void absorb(const float* os, const int* oi, int nq) {
-    wave_sync_lds();
-    for (int q = 0; q < nq; ++q) {
-      const float v = lane < K ? cs[q * TD_SL + lane] : lane < 2 * K ? os[q * TD_SL + lane - K] : -INFINITY;
-      const int id = lane < K ? ci[q * TD_SL + lane] : lane < 2 * K ? oi[q * TD_SL + lane - K] : -1;
-      td_cut(v, id, K, lane, cs + q * TD_SL, ci + q * TD_SL);
-    }
-  }
-  // lists of queries [0, nq) -> out[o0 + q * K + j] (o0: this list's (part, first query) offset)
-  __device__ __forceinline__ void store(int nq, size_t o0, float* __restrict__ os, int* __restrict__ oi) {
-    wave_sync_lds();
-    for (int i = lane; i < nq * K; i += 64) {
-      const int q = i / K, j = i % K;
-      os[o0 + i] = cs[q * TD_SL + j];
-      oi[o0 + i] = ci[q * TD_SL + j];
-    }
+  __device__ __forceinline__ void finish(int tiles, int fg) {
+    if (tiles & ((1 << lg) - 1)) close(fg);
+    for (int at = g & ~15; at < slots; at += 16) flush(at, fg);
   }
 };
 
-// NG = d / 128 load groups per 16-row tile (3, 6, 8: d = 384, 768, 1024): the ring holds one whole
-// tile ahead (NG * 4 KB per wave in flight), every load of the loop body unconditional (clamped),
-// so the compiler's vmcnt waits stay counted.
+typedef __attribute__((address_space(3))) void* vs_lds_t;
+
+// Up to 16 queries: a wave has a run of rows to itself. A tile is 16 rows x d in LDS, by LDS-DMA in column groups of 128 (256 B
+// of a row: 16-B chunk c of row r at c ^ r), and a group's place is filled with the next tile's as soon as its fragments are
+// in registers: no barrier, counted waits; the queries' fragments stay in registers.
+// (Rows loaded straight into the MFMA's A registers are requests of 64 B, of which a CU has no more on their way than of
+// whole lines.)
+// Bound by HBM: 1.25 M x 1024 at 6.5 TB/s with one query, 6.1 with 16 (5.1 and 4.3 by registers, with lists).
 template <int NG>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 1)
 topk_dense_stream_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict__ slots,
                          const bf16_t* __restrict__ Qv, int Q, const unsigned* __restrict__ bitmap, int W, float thr,
-                         int K, int rows_per_wave, int nqb, float* __restrict__ out_s, int* __restrict__ out_i) {
-  constexpr int d = NG * 32 * TD_G;
-  constexpr int qstr = d * 2 + 16;
-  __shared__ __attribute__((aligned(16))) char sQ[16 * qstr];   // [16][d] bf16, rows padded by 16 B
-  __shared__ float cs_all[4][16 * TD_SL];  // per wave: top-K lists + candidate buffers (TdWave)
-  __shared__ int ci_all[4][16 * TD_SL];
-
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+                         int rows_per_wave, float* __restrict__ gm, int GT, int run_slots, int lg) {
+  constexpr int d = NG * 128, RB = d * 2, NK = d / 32, TB = 16 * RB;
+  __shared__ __attribute__((aligned(16))) char sX[4 * TB];
+  __shared__ __attribute__((aligned(16))) int sS[4][2][64];  // doc slots of this tile and the next
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fg = lane >> 4;
-  // XCD-grouped block order: blocks b and b + 8 i share an XCD; the nqb query blocks of row block rb
-  // are b = (rb / 8) * 8 nqb + j * 8 + rb % 8
-  const int b = blockIdx.x, per = 8 * nqb;
-  const int grp = b / per, rem = b % per;
-  const int qb = rem / 8, rb = grp * 8 + rem % 8;
-  const int qbase = qb * 16, nq = min(16, Q - qbase);
-  for (int i = tid; i < 16 * (d / 8); i += 256) {
-    const int r = i / (d / 8), c = i % (d / 8);
-    u32x4_t v = u32x4_t{0, 0, 0, 0};
-    if (r < nq) v = *(const u32x4_t*)(Qv + (size_t)(qbase + r) * d + c * 8);
-    *(u32x4_t*)(sQ + r * qstr + c * 16) = v;
+  const int run = blockIdx.x * 4 + w;
+  const int beg = (int)min((long)N, (long)run * rows_per_wave), end = (int)min((long)N, (long)beg + rows_per_wave);
+  const int ntile = (end - beg + 15) / 16;
+  if (!ntile) return;  // (no barrier below)
+  bf16x8_t bq[NK];
+#pragma unroll
+  for (int kk = 0; kk < NK; ++kk) bq[kk] = *(const bf16x8_t*)(Qv + (size_t)min(fr, Q - 1) * d + kk * 32 + fg * 8);
+  const __amdgpu_buffer_rsrc_t rx =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)beg * d), (short)0, (end - beg) * RB, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(slots ? slots + beg : (const int*)X), (short)0, slots ? (end - beg) * 4 : 0, 0x00020000);
+  unsigned off[4];  // 1 KiB instruction i: rows 4 i .. 4 i + 3 of the group
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = 4 * i + (lane >> 4);
+    off[i] = (unsigned)(r * RB + (((lane & 15) ^ r) << 4));
   }
-  TdWave st;
-  st.init(cs_all[wid], ci_all[wid], K);
-  __syncthreads();
-
-  const int wbeg = (int)min((long)N, ((long)rb * 4 + wid) * rows_per_wave);
-  const int wend = (int)min((long)N, (long)wbeg + rows_per_wave);
-  const int ntile = (wend - wbeg + 15) / 16;
-  const int lrow = N - 1;
-  const int* sp = slots ? slots : (const int*)X;  // (without slots some word of X: loaded all the same, not used)
-  auto gload = [&](u32x4_t (&v)[NG][TD_G], int t) {  // tile t's fragments (rows clamped)
-    const int row = min(wbeg + t * 16 + fr, lrow);
-    const bf16_t* p = X + (size_t)row * d + fg * 8;
+  char* mine = sX + w * TB;
+  auto issue = [&](int t, int g) __attribute__((always_inline)) {
 #pragma unroll
-    for (int g = 0; g < NG; ++g)
-#pragma unroll
-      for (int j = 0; j < TD_G; ++j) v[g][j] = __builtin_nontemporal_load((const u32x4_t*)(p + (g * TD_G + j) * 32));
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (vs_lds_t)(mine + g * 4096 + i * 1024), 16, off[i], t * TB + g * 256, 0, 2);
   };
-  u32x4_t ring[NG][TD_G];
-  gload(ring, 0);
-  int sl_next = sp[min(wbeg + fr, lrow)];
-  const bool qok = fr < nq;
+  auto issue_slots = [&](int t) __attribute__((always_inline)) {  // (rows behind the tile's: out of range or unused)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (vs_lds_t)(&sS[w][t & 1][0]), 4, lane * 4, t * 64, 0, 0);
+  };
+  issue_slots(0);
+#pragma unroll
+  for (int g = 0; g < NG; ++g) issue(0, g);
+#pragma unroll
+  for (int kk = 0; kk < NK; ++kk) asm volatile("" : "+v"(bq[kk]));  // (waited for here, the tile on its way)
+  GroupMax gx;
+  gx.init(fr < Q ? gm + (size_t)fr * GT + (size_t)run * run_slots : nullptr, run_slots, lg);
+  const unsigned* bits = bitmap ? bitmap + (size_t)min(fr, Q - 1) * W : nullptr;
   for (int t = 0; t < ntile; ++t) {
     f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    const int row_next = min(wbeg + (t + 1) * 16 + fr, lrow);
-    const int sl = slots ? sl_next : 0;
-    sl_next = sp[row_next];
-    const bf16_t* pn = X + (size_t)row_next * d + fg * 8;
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (NG - 1)) : "memory");  // this group is in; NG - 1 newer ones at least
+      __builtin_amdgcn_sched_barrier(0);
+      bf16x8_t a[4];
 #pragma unroll
-      for (int j = 0; j < TD_G; ++j) {
-        const int kk = g * TD_G + j;
-        const bf16x8_t bq = *(const bf16x8_t*)(sQ + fr * qstr + kk * 64 + fg * 16);
-        acc = mfma16(__builtin_bit_cast(bf16x8_t, ring[g][j]), bq, acc);
-      }
-      // group g of the NEXT tile into the slot just consumed (one tile of loads stays in flight)
+      for (int j = 0; j < 4; ++j) a[j] = *(const bf16x8_t*)(mine + g * 4096 + fr * 256 + (((4 * j + fg) ^ fr) << 4));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      if (g == 0) issue_slots(t + 1);
+      issue(t + 1, g);
 #pragma unroll
-      for (int j = 0; j < TD_G; ++j)
-        ring[g][j] = __builtin_nontemporal_load((const u32x4_t*)(pn + (g * TD_G + j) * 32));
+      for (int j = 0; j < 4; ++j) acc = mfma16(a[j], bq[4 * g + j], acc);
     }
-    st.tile(acc, wbeg + t * 16 + fg * 4, wend, qok, thr, sl, bitmap, W, qbase + fr);
+    int sl[4] = {0, 0, 0, 0};
+    if (slots) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sl[i] = sS[w][t & 1][4 * fg + i];
+    }
+    gx.tile(acc, t, beg + t * 16 + fg * 4, end, thr, sl, bits, W, fg);
   }
-  st.finish();
-  // the 4 waves' lists -> one per workgroup (wave 0 absorbs the others'), out [rb, Q, K]
-  __syncthreads();
-  if (wid == 0) {
-    for (int w = 1; w < 4; ++w) st.absorb(cs_all[w], ci_all[w], nq);
-    st.store(nq, ((size_t)rb * Q + qbase) * K, out_s, out_i);
-  }
+  gx.finish(ntile, fg);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // pieces past the end write zeros: in before the workgroup's LDS goes
 }
 
 // 17 and more queries: NW waves of 16 queries each per workgroup (8 from 65 queries on, so that a shard is read once
-// for up to 128). rows_per_block rows per workgroup (multiple of 16), grid = row blocks (padded to 8) x query groups:
-// the nqg groups of one row block are dispatched to one XCD back to back. A tile: 16 rows x d, 16 B per thread per load
-// (NL loads) and the rows' doc slots, TD_PF tiles in flight in registers, written to one of two LDS buffers (16-B
-// chunk c of row r at c ^ (r & 15): the 16 rows one ds_read_b128 lane group reads hit 16 distinct slots), one barrier
-// per tile. The queries' fragments stay in registers (d / 8 of them).
-// Bound by HBM, and by what a SIMD does between tiles when it has one wave only: a pass of 128 queries x 1.25 M rows x
-// 1024 took 2304 us with 64 queries per workgroup, slots loaded where a candidate turned up and cuts of always 32
-// rounds, 1087 us with 4 waves of 32 queries each, and 808 us (3.2 TB/s) with two waves per SIMD, whose waits overlap.
-constexpr int TD_PF = 3;
-
+// for up to 128) over the SAME rows. rows_per_block rows per workgroup (multiple of 16), grid = row blocks (padded to 8) x
+// query groups: the nqg groups of one row block are dispatched to one XCD back to back. A stage: 16 rows (d = 384: 32) and
+// their doc slots by LDS-DMA (16-B chunk c of row r at c ^ (r & 15): the 16 rows one ds_read_b128 lane group reads hit 16
+// distinct slots; the slots to each wave's own words), a ring of 2 - 5 stages, one barrier a stage. The queries' fragments
+// stay in registers (d / 8 of them). 1.25 M x 1024: 6.0 TB/s with 17 queries, 5.8 with 64, 5.2 with 128, where a CU's LDS reads
+// (each wave reads the whole stage) and its MFMAs take about as long as its stages; the DMA instructions spread between the
+// MFMAs, or two chains of them, were slower (594 - 622 us for 496).
 template <int NG, int NW>
-__global__ void __launch_bounds__(64 * NW, 1)
+__global__ void __launch_bounds__(64 * NW, 2)
 topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict__ slots,
                      const bf16_t* __restrict__ Qv, int Q, const unsigned* __restrict__ bitmap, int W, float thr,
-                     int K, int rows_per_block, int nqg, float* __restrict__ out_s, int* __restrict__ out_i) {
-  constexpr int d = NG * 128, NK = d / 32, CPR = d / 8, RB = d * 2, TB = 16 * RB, NT = 64 * NW;
-  constexpr int NL = (16 * CPR + NT - 1) / NT;  // 16-B loads of a thread per tile
-  __shared__ __attribute__((aligned(16))) char sX[2][TB];
-  __shared__ float cs_all[NW][16 * TD_SL];
-  __shared__ int ci_all[NW][16 * TD_SL];
+                     int rows_per_block, int nqg, float* __restrict__ gm, int GT, int run_slots, int lg) {
+  constexpr int d = NG * 128, NK = d / 32, CPR = d / 8, RB = d * 2;
+  constexpr int TR = NG == 3 ? 2 : 1, STAGE = TR * 16 * RB, P1 = STAGE / 1024 / NW, P = P1 + 1;
+  constexpr int LDS = NW == 8 ? 160 * 1024 : 80 * 1024, SL = NW * 256;
+  constexpr int ST = LDS / (STAGE + SL) < 5 ? LDS / (STAGE + SL) : 5;
+  static_assert(STAGE % (1024 * NW) == 0 && ST >= 2 && P1 <= 8, "stage");
+  __shared__ __attribute__((aligned(16))) char sX[ST * (STAGE + SL)];
 
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fg = lane >> 4;
   const int b = blockIdx.x, per = 8 * nqg;
   const int grp = b / per, rem = b % per;
   const int qg = rem / 8, rb = grp * 8 + rem % 8;
-  const int qbase = (qg * NW + wid) * 16, nq = max(0, min(16, Q - qbase));
-  const bool qok = fr < nq;
-  // this wave's B fragments: query qbase + fr, columns 32 kk + 8 fg .. + 8
+  const int q = (qg * NW + w) * 16 + fr;
+  const int beg = (int)min((long)N, (long)rb * rows_per_block), end = (int)min((long)N, (long)beg + rows_per_block);
+  const int ntile = (end - beg + 15) / 16, nst = (ntile + TR - 1) / TR;
+  if (!nst) return;  // whole workgroup
+  // this wave's B fragments: query q, columns 32 kk + 8 fg .. + 8
   bf16x8_t bq[NK];
 #pragma unroll
-  for (int kk = 0; kk < NK; ++kk)
-    bq[kk] = *(const bf16x8_t*)(Qv + (size_t)min(qbase + fr, Q - 1) * d + kk * 32 + fg * 8);
-  TdWave st;
-  st.init(cs_all[wid], ci_all[wid], K);
-
-  const int rbeg = (int)min((long)N, (long)rb * rows_per_block);
-  const int rend = (int)min((long)N, (long)rbeg + rows_per_block);
-  const int ntile = (rend - rbeg + 15) / 16;
-  const int tl = max(ntile - 1, 0);
-  // buffer loads: one scalar offset per tile, rows past the workgroup's last return zeros (masked in tile()).
-  // Without slots some words of X are loaded in their place, and not used.
-  const __amdgpu_buffer_rsrc_t rsx = __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)rbeg * d), (short)0,
-                                                                       (rend - rbeg) * RB, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rss = __builtin_amdgcn_make_buffer_rsrc(
-      slots ? (void*)(slots + rbeg) : (void*)(X + (size_t)rbeg * d), (short)0, (rend - rbeg) * 4, 0x00020000);
-  unsigned voff[NL];   // chunk tid + NT i of a tile (one past its end: out of range, loads nothing)
-  int loff[NL];
+  for (int kk = 0; kk < NK; ++kk) bq[kk] = *(const bf16x8_t*)(Qv + (size_t)min(q, Q - 1) * d + kk * 32 + fg * 8);
+  // rows past the workgroup's last are zeros (masked in GroupMax::tile); no slots: an empty resource
+  const __amdgpu_buffer_rsrc_t rx =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)beg * d), (short)0, (end - beg) * RB, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(slots ? slots + beg : (const int*)X), (short)0, slots ? (end - beg) * 4 : 0, 0x00020000);
+  unsigned off[8];
 #pragma unroll
-  for (int i = 0; i < NL; ++i) {
-    const int idx = tid + NT * i, r = idx / CPR, c = idx % CPR;
-    voff[i] = idx < 16 * CPR ? idx * 16u : 0x7ffffff0u;
-    loff[i] = r * RB + ((c ^ (r & 15)) << 4);
+  for (int j = 0; j < P1; ++j) {
+    const int idx = (w * P1 + j) * 64 + lane, r = idx / CPR, c = idx % CPR;
+    off[j] = (unsigned)(r * RB + ((c ^ (r & 15)) << 4));
   }
-  auto gload = [&](u32x4_t (&v)[NL], int& sl, int t) {  // tile t <= tl
+  auto issue = [&](int t, int stage) __attribute__((always_inline)) {
+    char* dst = sX + stage * (STAGE + SL);
 #pragma unroll
-    for (int i = 0; i < NL; ++i)
-      v[i] = __builtin_amdgcn_raw_buffer_load_b128(rsx, voff[i], t * TB, 2);  // non-temporal
-    sl = __builtin_amdgcn_raw_buffer_load_b32(rss, fr * 4, t * 64, 0);
+    for (int j = 0; j < P1; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (vs_lds_t)(dst + (w * P1 + j) * 1024), 16, off[j & 7], t * STAGE, 0, 2);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (vs_lds_t)(dst + STAGE + w * 256), 4, lane * 4, t * (64 * TR), 0, 0);
   };
-  auto lstore = [&](const u32x4_t (&v)[NL], int buf) {
 #pragma unroll
-    for (int i = 0; i < NL; ++i)
-      if ((i + 1) * NT <= 16 * CPR || tid + NT * i < 16 * CPR) *(u32x4_t*)(&sX[buf][loff[i]]) = v[i];
-  };
+  for (int i = 0; i < ST - 1; ++i) issue(i, i);
+#pragma unroll
+  for (int kk = 0; kk < NK; ++kk) asm volatile("" : "+v"(bq[kk]));  // (waited for here, the stages on their way)
   int xo[4];  // where chunk 4 kk + fg of row fr is: the swizzle only touches the chunk's low four bits
 #pragma unroll
   for (int j = 0; j < 4; ++j) xo[j] = fr * RB + (((j * 4 + fg) ^ fr) << 4);
-  __syncthreads();  // the lists' initial values (before any load is in flight: this drains them)
-  u32x4_t ring[TD_PF][NL];
-  int slot[TD_PF];
+  GroupMax gx;
+  gx.init(q < Q ? gm + (size_t)q * GT + (size_t)rb * run_slots : nullptr, run_slots, lg);
+  const unsigned* bits = bitmap ? bitmap + (size_t)min(q, Q - 1) * W : nullptr;
+  int rd = 0, wr = ST - 1;
+  for (int t = 0; t < nst; ++t) {
+    // this wave's pieces of stage t are in (ST - 2 newer stages); after the barrier everyone's, and stage t - 1 has been read
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(P * (ST - 2)) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    issue(t + ST - 1, wr);
+    const char* src = sX + rd * (STAGE + SL);
 #pragma unroll
-  for (int u = 0; u < TD_PF; ++u) {
-    gload(ring[u], slot[u], min(u, tl));
-    asm volatile("" ::: "memory");  // issue order = tile order (counted waits)
-  }
-  // whole groups of TD_PF tiles (no exit inside the unrolled group: the ring keeps fixed registers);
-  // tiles past the end re-read the last one and mask every row
-  for (int t0 = 0; t0 < ntile; t0 += TD_PF) {
-#pragma unroll
-    for (int u = 0; u < TD_PF; ++u) {
-      const int t = t0 + u;
-      const int buf = t & 1, sl = slots ? slot[u] : 0;
-      lstore(ring[u], buf);
-      gload(ring[u], slot[u], min(t + TD_PF, tl));  // clamped past the end: uniform counts
-      // tile t visible to every wave, and every wave is done with tile t - 2 (same buffer): a raw
-      // barrier (__syncthreads() would drain the loads in flight)
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
+    for (int u = 0; u < TR; ++u) {
       f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kk = 0; kk < NK; ++kk)
-        acc = mfma16(*(const bf16x8_t*)(&sX[buf][xo[kk & 3] + (kk >> 2) * 256]), bq[kk], acc);
-      st.tile(acc, rbeg + t * 16 + fg * 4, rend, qok, thr, sl, bitmap, W, qbase + fr);
+        acc = mfma16(*(const bf16x8_t*)(src + u * 16 * RB + xo[kk & 3] + (kk >> 2) * 256), bq[kk], acc);
+      int sl[4] = {0, 0, 0, 0};
+      if (slots) {
+        const u32x4_t v = *(const u32x4_t*)(src + STAGE + w * 256 + u * 64 + fg * 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sl[i] = (int)v[i];
+      }
+      gx.tile(acc, t * TR + u, beg + (t * TR + u) * 16 + fg * 4, end, thr, sl, bits, W, fg);
     }
+    rd = rd + 1 == ST ? 0 : rd + 1;
+    wr = wr + 1 == ST ? 0 : wr + 1;
   }
-  st.finish();
-  st.store(nq, ((size_t)rb * Q + qbase) * K, out_s, out_i);
+  gx.finish(nst * TR, fg);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // pieces past the end write zeros: in before the workgroup's LDS goes
 }
 
 // A wave's unsorted top-K list in LDS: cs / ci hold TL_SL slots, [0, K) the list, the rest room for what is
@@ -647,6 +578,38 @@ topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ 
   }
 }
 
+// Wave 0 (every wave's list is in): the lists of waves 1 .. n - 1 into its own.
+__device__ __forceinline__ void top_join(TopList& top, float (*cs)[TL_SL], int (*ci)[TL_SL], int n) {
+  const int rest = (n - 1) * top.K;
+  for (int e0 = 0; e0 < rest; e0 += 64) {
+    const int e = e0 + top.lane, w = 1 + min(e, max(rest - 1, 0)) / top.K;
+    top.add(cs[w][e % top.K], e < rest ? ci[w][e % top.K] : -1);
+  }
+  wave_sync_lds();
+}
+
+// A wave's list, best first (ties: smaller row id), empty places behind: each row's place by counting the better ones.
+__device__ __forceinline__ void top_order(const TopList& top, float* __restrict__ os, int* __restrict__ oi) {
+  const int K = top.K, lane = top.lane;
+  const float v = lane < K ? top.cs[lane] : -INFINITY;
+  const int id = lane < K ? top.ci[lane] : -1;
+  int rank = 0;
+  for (int j = 0; j < K; ++j) {
+    const float vj = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), j));
+    const int ij = __builtin_amdgcn_readlane(id, j);
+    rank += ij >= 0 && (better(vj, ij, v, id) || (vj == v && ij == id && j < lane));  // (a row named twice)
+  }
+  const int real = __popcll(__ballot(id >= 0));
+  if (id >= 0) {
+    os[rank] = v;
+    oi[rank] = id;
+  }
+  if (lane >= real && lane < K) {
+    os[lane] = -INFINITY;
+    oi[lane] = -1;
+  }
+}
+
 // cand [P, Q, K] -> out [Q, K] sorted desc (ties: smaller row id). One workgroup per query, a wave per 64 candidates
 // up to 16 (TM_WAVES): each wave cuts its share to K, wave 0 joins the lists and orders them by counting the better
 // ones of each. Bound by the chain of cuts (about 1 us each), hence many waves: K rounds of a workgroup-wide argmax
@@ -677,28 +640,153 @@ topk_merge_kernel(const float* __restrict__ cand_s, const int* __restrict__ cand
   }
   __syncthreads();
   if (wid) return;
-  const int rest = (nt / 64 - 1) * K;  // the other waves' lists, one after another
-  for (int e0 = 0; e0 < rest; e0 += 64) {
-    const int e = e0 + lane, w = 1 + min(e, max(rest - 1, 0)) / K;
-    top.add(cs[w][e % K], e < rest ? ci[w][e % K] : -1);
+  top_join(top, cs, ci, nt / 64);
+  top_order(top, os + (size_t)q * K, oi + (size_t)q * K);
+}
+
+// The second half of a scan (see there): per query the K best of its GT groups, their rows scored again (16 rows a wave and
+// step, the query in all of the MFMA's columns), the K best of those in order. Group g is tiles (g % run_slots) << lg .. of
+// run g / run_slots, run_rows rows each.
+// Bound by latency. A cut of a list of 64 takes about 1 us, and 80000 values in any order improve on one many times (lists
+// kept by every wave, as topk_merge_kernel does: 100 us for 80000 groups, K = 5; 49 for 8000, K = 19), so a bound comes first:
+// the K-th best of the threads' own best values, to its upper 20 bits. What reaches it (little more than K values) is
+// collected and cut once, and the same again with the rows that reach the K-th best group. Lists that overflow (thousands
+// of equal scores) are done over by the waves' lists.
+constexpr int TP_WAVES = 8, TP_CAP = 1024;
+
+// The largest bound, to its upper 20 bits, that at least `need` of the 8 keys of each lane reach (0: there are not as many).
+__device__ __forceinline__ unsigned reached_by(const unsigned (&key)[8], int need) {
+  unsigned T = 0;
+  for (int bt = 31; bt >= 12; --bt) {
+    const unsigned t = T | (1u << bt);
+    int c = 0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) c += __popcll(__ballot(key[u] >= t));
+    if (c >= need) T = t;
+    if (c == need) break;
   }
-  wave_sync_lds();
-  const float v = lane < K ? cs[0][lane] : -INFINITY;
-  const int id = lane < K ? ci[0][lane] : -1;
-  int rank = 0;
-  for (int j = 0; j < K; ++j) {
-    const float vj = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), j));
-    const int ij = __builtin_amdgcn_readlane(id, j);
-    rank += ij >= 0 && (better(vj, ij, v, id) || (vj == v && ij == id && j < lane));  // (a row named twice)
+  return T;
+}
+
+template <int NG>
+__global__ void __launch_bounds__(64 * TP_WAVES, 2)
+topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_rows, int lg, const bf16_t* __restrict__ X, int N,
+                 const int* __restrict__ slots, const bf16_t* __restrict__ Qv, const unsigned* __restrict__ bitmap, int W,
+                 float thr, int K, float* __restrict__ os, int* __restrict__ oi) {
+  constexpr int d = NG * 128, NK = d / 32, nt = 64 * TP_WAVES;
+  static_assert(TP_WAVES == 8, "a key of each thread: 8 per lane of a wave");
+  __shared__ float cs[TP_WAVES][TL_SL], cand_s[TP_CAP];
+  __shared__ int ci[TP_WAVES][TL_SL], cand_i[TP_CAP];
+  __shared__ int groups[TK_MAX], count;
+  __shared__ float bound;
+  __shared__ unsigned keys[nt];
+  __shared__ __attribute__((aligned(16))) bf16_t sq[d];
+  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, fr = lane & 15, fg = lane >> 4;
+  for (int i = tid; i < d / 8; i += nt) *(u32x4_t*)(sq + i * 8) = *(const u32x4_t*)(Qv + (size_t)q * d + i * 8);
+  const f32x4_t* line = (const f32x4_t*)(gm + (size_t)q * GT);
+  TopList top;
+  top.init(cs[wid], ci[wid], K);
+  // the best rows or groups so far collected: through wave 0's list, best K of them; overflowed: every wave's own
+  auto collect = [&](float v, int id, bool in) __attribute__((always_inline)) {
+    if (!in) return;
+    const int at = atomicAdd(&count, 1);
+    if (at < TP_CAP) { cand_s[at] = v; cand_i[at] = id; }
+  };
+  auto fold = [&](int n) __attribute__((always_inline)) {  // wave 0
+    for (int j = 0; j < n; j += 64) {
+      const int e = min(j + lane, n - 1);
+      top.add(cand_s[e], j + lane < n ? cand_i[e] : -1);
+    }
+    wave_sync_lds();
+  };
+
+  // ---- groups ----
+  const int nv = GT / 4;
+  float best = -INFINITY;
+  for (int j0 = tid; j0 < nv; j0 += nt * 4) {
+    f32x4_t v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = line[min(j0 + nt * u, nv - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)  // (a value counts for one thread only)
+      if (j0 + nt * u < nv) best = fmaxf(best, fmaxf(fmaxf(v[u][0], v[u][1]), fmaxf(v[u][2], v[u][3])));
   }
-  const int real = __popcll(__ballot(id >= 0));
-  if (id >= 0) {
-    os[(size_t)q * K + rank] = v;
-    oi[(size_t)q * K + rank] = id;
+  keys[tid] = td_key(best, best > -INFINITY ? 0 : -1);
+  if (tid == 0) count = 0;
+  __syncthreads();
+  if (wid == 0) {
+    unsigned key[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) key[u] = keys[u * 64 + lane];
+    const float b = td_unkey(reached_by(key, K));
+    if (lane == 0) bound = b != b ? -INFINITY : b;
   }
-  if (lane >= real && lane < K) {
-    os[(size_t)q * K + lane] = -INFINITY;
-    oi[(size_t)q * K + lane] = -1;
+  __syncthreads();
+  const float T = bound;
+  for (int j0 = tid; j0 < nv; j0 += nt) {
+    const f32x4_t v = line[j0];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) collect(v[e], 4 * j0 + e, v[e] >= T && v[e] > -INFINITY);
+  }
+  __syncthreads();
+  const int found = count;
+  const bool over = found > TP_CAP;
+  __syncthreads();  // (wave 0 writes count below)
+  if (over) {
+    for (int j0 = wid * 64; j0 < GT; j0 += nt) {
+      const int j = j0 + lane;
+      const float v = ((const float*)line)[min(j, GT - 1)];
+      top.add(v, j < GT && v > -INFINITY ? j : -1);
+    }
+    __syncthreads();
+  }
+  if (wid == 0) {
+    if (over) top_join(top, cs, ci, TP_WAVES);
+    else fold(found);
+    if (lane < K) groups[lane] = ci[0][lane];
+    float low = lane < K && ci[0][lane] >= 0 ? cs[0][lane] : lane < K ? -INFINITY : INFINITY;  // the K-th best group
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) low = fminf(low, __shfl_xor(low, o, 64));
+    if (lane == 0) { bound = low; count = 0; }
+  }
+  __syncthreads();
+
+  // ---- their rows ----
+  const float R = bound;
+  top.init(cs[wid], ci[wid], K);
+  for (int again = 0; again < 2; ++again) {
+    for (int it = wid; it < K << lg; it += TP_WAVES) {
+      const int g = groups[it >> lg];
+      if (g < 0) continue;
+      const int run = g / run_slots;
+      const long first = (long)run * run_rows;
+      const int row0 = (int)first + ((((g % run_slots) << lg) + (it & ((1 << lg) - 1))) * 16);
+      const int end = (int)min((long)N, first + run_rows);
+      if (row0 >= end) continue;
+      const bf16_t* xr = X + (size_t)min(row0 + fr, end - 1) * d + fg * 8;
+      bf16x8_t a[NK];
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk) a[kk] = *(const bf16x8_t*)(xr + kk * 32);
+      // lane (fr, fg), fr < 4: row 4 fg + fr of the tile
+      const int row = row0 + 4 * fg + (fr & 3);
+      const int sl = slots ? slots[min(row, end - 1)] : 0;
+      f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk) acc = mfma16(a[kk], *(const bf16x8_t*)(sq + kk * 32 + fg * 8), acc);
+      const float s = fr == 0 ? acc[0] : fr == 1 ? acc[1] : fr == 2 ? acc[2] : acc[3];
+      bool ok = fr < 4 && row < end && sl >= 0 && s >= thr && s > -INFINITY && s >= R;
+      if (ok && bitmap) ok = (sl >> 5) < W && ((bitmap[(size_t)q * W + (sl >> 5)] >> (sl & 31)) & 1u);
+      if (again) top.add(s, ok ? row : -1);
+      else collect(s, row, ok);
+    }
+    __syncthreads();
+    if (again || count <= TP_CAP) {  // (no more writes to count)
+      if (wid) return;
+      if (again) top_join(top, cs, ci, TP_WAVES);
+      else fold(count);
+      top_order(top, os + (size_t)q * K, oi + (size_t)q * K);
+      return;
+    }
   }
 }
 
@@ -753,44 +841,62 @@ DA_EXPORT int da_topk_dense(const void* X, int N, int d, const void* slots, cons
   return topk_merge(cs, ci, nblk, Q, K, out_s, out_i, s);
 }
 
-// The streaming scan (d = 384, 768 or 1024): ws holds (row blocks padded to 8) * 4 * Q * K candidate
-// pairs; rows_per_wave % 16 == 0. hipErrorInvalidValue for shapes it does not take (the caller
-// then uses da_topk_dense).
-static long blocks8(long N, long rows) { return ((N + rows - 1) / rows + 7) / 8 * 8; }
-// rows per workgroup of the shared-tile kernel: one workgroup per CU over the whole shard (each pays the early top-K
-// fill once), one tile at least, 1 GB at most (its 32-bit offsets)
-static int mq_rows(long N) { return (int)min(524288L, max(16L, (N + 256 * 16 - 1) / (256 * 16) * 16)); }
+// The streaming scan (d = 384, 768 or 1024). hipErrorInvalidValue for shapes it does not take (the caller then uses
+// da_topk_dense). Its runs of rows, and their groups in ws: Q lines of `groups` floats.
+struct ScanPlan {
+  int runs, run_rows, run_slots, lg;  // run_slots: a run's groups, padded to 4
+  long groups() const { return (long)runs * run_slots; }
+};
 
-DA_EXPORT size_t da_topk_stream_ws(int N, int Q, int K, int rows_per_wave) {
-  const long parts = Q <= 16 ? blocks8(N, 4L * rows_per_wave) : blocks8(N, mq_rows(N));
-  return (size_t)parts * Q * K * 8;
+// A run is a wave's (up to 16 queries; rows_per_wave at least) or a workgroup's (17 and more), 16 to 524288 rows (32-bit
+// offsets), and as many as one round of resident workgroups needs: a second round starts its pipelines anew, us with 1024
+// waves / 4096: 100000 x 1024, 16 queries, 48.7 / 56.3; 411812 x 768 113.6 / 121.0; 1250000 x 1024 417 / 419.
+// A group is a tile up to 65536 groups, so that the pick reads 256 KB a query at most, and 2, 4, .. tiles from there on.
+static ScanPlan scan_plan(long N, int Q, int rows_per_wave) {
+  const long runs = Q <= 16 ? 1024 : Q <= 64 ? 512 : 256;
+  ScanPlan p;
+  p.run_rows = (int)min(524288L, max(Q <= 16 ? (rows_per_wave + 15L) / 16 * 16 : 16L, (N + runs * 16 - 1) / (runs * 16) * 16));
+  p.runs = (int)((N + p.run_rows - 1) / p.run_rows);
+  p.lg = 0;
+  while ((N >> (4 + p.lg)) > 65536) ++p.lg;
+  const int tiles = p.run_rows / 16 + 1;  // (32-row stages: one tile past the end)
+  p.run_slots = ((tiles + (1 << p.lg) - 1 >> p.lg) + 3) & ~3;
+  return p;
+}
+
+DA_EXPORT size_t da_topk_stream_ws(int N, int Q, int rows_per_wave) {
+  return (size_t)scan_plan(N, Q, rows_per_wave).groups() * Q * 4;
 }
 
 DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slots, const void* Qv, int Q,
-                                   const void* bitmap, int W, float thr, int K, int rows_per_wave, void* ws,
-                                   void* out_s, void* out_i, void* stream) {
-  if ((d != 384 && d != 768 && d != 1024) || K < 1 || K > TK_MAX || rows_per_wave % 16 || rows_per_wave <= 0 ||
-      N < 1)
+                                   const void* bitmap, int W, float thr, int K, int rows_per_wave, void* ws, void* out_s,
+                                   void* out_i, void* stream) {
+  if ((d != 384 && d != 768 && d != 1024) || K < 1 || K > TK_MAX || N < 1 || rows_per_wave < 16)
     return (int)hipErrorInvalidValue;
   if (Q == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  const int rpb = mq_rows(N), qper = Q > 64 ? 128 : 64, nqg = (Q + qper - 1) / qper;
-  const long parts = Q <= 16 ? blocks8(N, 4L * rows_per_wave) : blocks8(N, rpb);
-  if (parts * nqg > 0x7fffffffL) return (int)hipErrorInvalidValue;
-  float* cs = (float*)ws;
-  int* ci = (int*)(cs + (size_t)parts * Q * K);
-#define TDQ(NG, NW)                                                                                     \
-  topk_dense_mq_kernel<NG, NW><<<(int)parts * nqg, 64 * NW, 0, s>>>((const bf16_t*)X, N,                \
-      (const int*)slots, (const bf16_t*)Qv, Q, (const unsigned*)bitmap, W, thr, K, rpb, nqg, cs, ci)
-#define TDS(NG)                                                                                         \
-  do {                                                                                                  \
-    if (Q <= 16)                                                                                        \
-      topk_dense_stream_kernel<NG><<<(int)parts, 256, 0, s>>>((const bf16_t*)X, N, (const int*)slots,   \
-          (const bf16_t*)Qv, Q, (const unsigned*)bitmap, W, thr, K, rows_per_wave, 1, cs, ci);           \
-    else if (Q <= 64)                                                                                   \
-      TDQ(NG, 4);                                                                                       \
-    else                                                                                                \
-      TDQ(NG, 8);                                                                                       \
+  const ScanPlan p = scan_plan(N, Q, rows_per_wave);
+  const int nw = Q > 64 ? 8 : 4, nqg = (Q + 16 * nw - 1) / (16 * nw);
+  const long blocks = Q <= 16 ? (p.runs + 3) / 4 : (long)(p.runs + 7) / 8 * 8 * nqg;
+  if (p.groups() > 0x7fffffffL || blocks > 0x7fffffffL) return (int)hipErrorInvalidValue;
+  float* gm = (float*)ws;
+  const int GT = (int)p.groups();
+#define TDQ(NG, NW)                                                                                                  \
+  topk_dense_mq_kernel<NG, NW><<<(int)blocks, 64 * NW, 0, s>>>((const bf16_t*)X, N, (const int*)slots, (const bf16_t*)Qv, Q, \
+      (const unsigned*)bitmap, W, thr, p.run_rows, nqg, gm, GT, p.run_slots, p.lg)
+#define TDS(NG)                                                                                                      \
+  do {                                                                                                               \
+    if (Q <= 16)                                                                                                     \
+      topk_dense_stream_kernel<NG><<<(int)blocks, 256, 0, s>>>((const bf16_t*)X, N, (const int*)slots,               \
+          (const bf16_t*)Qv, Q, (const unsigned*)bitmap, W, thr, p.run_rows, gm, GT, p.run_slots, p.lg);             \
+    else if (Q <= 64)                                                                                                \
+      TDQ(NG, 4);                                                                                                    \
+    else                                                                                                             \
+      TDQ(NG, 8);                                                                                                    \
+    const int err = (int)hipGetLastError();                                                                          \
+    if (err) return err;                                                                                             \
+    topk_pick_kernel<NG><<<Q, 64 * TP_WAVES, 0, s>>>(gm, GT, p.run_slots, p.run_rows, p.lg, (const bf16_t*)X, N,      \
+        (const int*)slots, (const bf16_t*)Qv, (const unsigned*)bitmap, W, thr, K, (float*)out_s, (int*)out_i);        \
   } while (0)
   switch (d) {
     case 384: TDS(3); break;
@@ -799,9 +905,7 @@ DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slot
   }
 #undef TDS
 #undef TDQ
-  int err = (int)hipGetLastError();
-  if (err) return err;
-  return topk_merge(cs, ci, (int)parts, Q, K, out_s, out_i, s);
+  DA_LAUNCH_CHECK();
 }
 
 DA_EXPORT int da_topk_ranges(const void* X, int d, const void* slots, const void* Qv, int Q, const void* ranges,

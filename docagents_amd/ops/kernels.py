@@ -103,7 +103,7 @@ _SIGS = {
     "da_bert_embed_ln_f16": [c_void_p] * 9 + [c_int, c_int, c_float, c_void_p],
     "da_pool_l2norm_f16": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
     "da_topk_dense_ws": [c_int] * 4,
-    "da_topk_stream_ws": [c_int] * 4,
+    "da_topk_stream_ws": [c_int] * 3,
 }
 # the library part (build.py) of each launcher that is not in "kernels"; da_gemm* are in "gemm"
 _PART_OF = {n: "token" for n in (
@@ -1177,10 +1177,9 @@ def sample_finalize(gathered, ranks: int, out_tok=None, out_lp=None, conf=None, 
 
 # --------------------------------------------------------------------------- vector search
 def _scan_rows(N: int) -> int:
-    """Rows of a wave in the streaming scan of up to 16 queries: 16 waves a CU over the chip (256 CUs), but at least 64 rows
-    each, with 256 workgroups of 4 waves where that leaves CUs idle (one tile of 16 rows each at least: a few hundred
-    centroids). More workgroups than CUs for less each are slower, us in 16 / 32 / 64 rows: 60000 x 1024, one query, 74.8 /
-    56.2 / 45.7 (16 queries 197 / 127 / 126); 30000 42.7 / 33.5 / 40.1; 16000 28.0 / 30.4 / 38.8; 512 x 384 15.1 / 16.9 / 20.5."""
+    """Rows that a wave of the streaming scan of up to 16 queries takes at least (the launcher gives it what one round of
+    workgroups needs, if that is more): 16 waves a CU over the chip (256 CUs), but at least 64 rows each, with 256 workgroups
+    of 4 waves where that leaves CUs idle (one tile of 16 rows each at least: a few hundred centroids)."""
     tiles = lambda waves: math.ceil(N / waves / 16) * 16  # noqa: E731
     return max(min(tiles(256 * 4), 64), tiles(256 * 16), 16)
 
@@ -1204,7 +1203,7 @@ def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_bloc
         # the streaming scan (search-sized batches over a big shard; k-means assignment, with the
         # rows as the queries, keeps the query-major tiles below)
         rpw = _scan_rows(N)
-        ws = _workspace(int(lib().da_topk_stream_ws(N, Q, K, rpw)), X.device)
+        ws = _workspace(int(lib().da_topk_stream_ws(N, Q, rpw)), X.device)
         out_s = torch.empty((Q, K), dtype=torch.float32, device=X.device)
         out_i = torch.empty((Q, K), dtype=torch.int32, device=X.device)
         _check(lib().da_topk_dense_stream(_ptr(X), N, d, _ptr(slots), _ptr(Qv), Q, _ptr(bitmap), W, float(thr), K,
