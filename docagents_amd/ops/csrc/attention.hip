@@ -1257,11 +1257,11 @@ decode_attn_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __restri
 // pair_rows: whole rows, up to 64 of them, two workgroups per CU: paired_row (91 -> 87 us in the first case above).
 template <int D>
 __device__ __forceinline__ int vswz(int r) {
-  return D == 128 ? ((r & 7) << 1) : (((r >> 1) & 3) << 1);
+  return D == 128 ? ((r & 7) << 1) : D == 96 ? ((r >> 2) & 1) << 1 : (((r >> 1) & 3) << 1);
 }
 template <int D>
 __device__ __forceinline__ int kswz(int r) {
-  return D == 128 ? r & 15 : (r >> 1) & 7;
+  return D == 128 ? r & 15 : D == 96 ? (r >> 2) & 3 : (r >> 1) & 7;
 }
 
 // The row that workgroup row z of B <= 64 takes, and its keys: the `round` longest first (a workgroup per CU), then from the
@@ -1466,40 +1466,38 @@ decode_attn_gqa_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __re
   dec_finish<D, G>(po, pm, pl, H, Hkv, nsplit, b, hk, cnt, out, ldo, (int*)(swl + 4), act);
 }
 
-// MHA decode attention on MFMA for few (row, kv head) pairs (batch 1..: the p50 path). The VALU
-// kernel (decode_attn_kernel, G = 1) spends ~2k VALU cycles per 64-key tile on its dot products, so
-// at batch 1 — 32 pairs, a few tiles per wave — it is issue-bound, not HBM-bound (profiles/r5/
-// decode_mfma1/: 2.9 TB/s even with the K/V in the MALL). Here the single query is the N = 16 side of
-// v_mfma_f32_16x16x32_bf16 (column 0 live, 15 zero), exactly the GQA kernel's data path with G = 1:
-// K rows straight into registers (non-temporal), the V tile by LDS-DMA into a wave-private region
-// (XOR chunk swizzle within groups of 4 chunks, so D = 96's 12 chunks per row stay in the row),
-// S^T = K Q^T, softmax over column 0, O^T += V^T P^T with transposed LDS reads. chunk <= 512 keys per
-// split (host-checked) gives every wave at most TWO tiles, and both are requested before any is
-// waited for: one HBM round trip per workgroup. XC: same-XCD split exchange (see dec_finish).
-template <int D>
-__device__ __forceinline__ int vswz1(int r) {
-  return D == 96 ? ((r >> 1) & 3) : vswz<D>(r);
-}
-
+// MHA decode attention (G = 1) on MFMA: the GQA kernel's data path, with the one query in all 16 columns, so that every lane has
+// the weights of its 8 keys. They stay fp32: column 0 of P^T holds their upper 8 bits (as bf16), column 1 the next 8, column 2
+// the last, and the three columns of O^T are added at the end. (Dot products and weighted sums on the VALU, decode_attn_kernel,
+// take it 2000 cycles per 64 keys: this kernel had only launches of up to 32 pairs, K rows by 64-B requests and weights of 16
+// bits, the others the VALU.) us before / after, 32 heads x 96: one row of 60 / 300 / 2935 / 4000 keys 7.6 / 8.5 / 13.2 / 15.0 ->
+// 5.5 / 7.3 / 11.6 / 13.5; rows of 64 - 146 keys, 4 / 12 / 30 / 40 of them, 10.6 / 18.1 / 17.9 / 23.2 -> 6.5 / 7.9 / 14.1 /
+// 16.3; of 500 - 2000 19.0 / 50.8 / 86.7 / 89.1 -> 16.6 / 41.6 / 79.4 / 88.5 (5.9 TB/s). Few keys: bound by the launch, the
+// chain length -> addresses -> keys and the merge, about 5 us.
+// by_len (as in the GQA kernel): even splits of 12 rows of 64 - 146 keys in a cache of 4096 take 10.9 us, of 200 - 500 15.8 (16.5
+// by length).
+// XC: same-XCD split exchange (see dec_finish).
 // RP: fused RoPE + new-token KV write (DecRope, as decode_attn_kernel): q is the raw qkv row; q is
 // rotated into LDS while the tiles fly, key L - 1 enters as one extra online-softmax term of the
 // split that holds it (taken from the qkv row, written into the cache for later steps).
 template <int D, bool XC, bool RP>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 2)
 decode_attn_mfma1_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __restrict__ kc,
                          const bf16_t* __restrict__ vc, const int* __restrict__ lens, const int* __restrict__ slot,
                          const int* __restrict__ pre, int H, int Hkv, int max_seq, int chunk_max, int nsplit,
                          float scale_log2e, float* __restrict__ po, float* __restrict__ pm, float* __restrict__ pl,
-                         bf16_t* __restrict__ out, int ldo, int* __restrict__ cnt, DecRope rope) {
+                         bf16_t* __restrict__ out, int ldo, int* __restrict__ cnt, DecRope rope, int by_len) {
   static_assert(D == 64 || D == 96 || D == 128, "head dim");
-  constexpr int KT = 64, NDS = D / 32, NDT = D / 16, NS = D / 8;
-  constexpr int VBYTES = KT * D * 2, NDMA = VBYTES / 1024;
+  constexpr int KT = 32, NDS = D / 32, NDT = D / 16, NS = D / 8;
+  constexpr int TB = KT * D * 2, ND = TB / 1024, ST = D == 64 ? 2 : 1;
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
-  typedef __attribute__((address_space(1))) const void* gptr_t;
-  __shared__ __attribute__((aligned(16))) char sv[4 * 2 * VBYTES];  // two tiles per wave
-  __shared__ float swm[4], swl[4];
+  // (one array: with several, hipcc has every LDS read wait for the DMA)
+  __shared__ __attribute__((aligned(16))) char ring[4 * ST * 2 * TB + 64 + D * 10];
+  float* swm = (float*)(ring + 4 * ST * 2 * TB);
+  float *swl = swm + 4, *ssn = swm + 8, *skn = swm + 16, *svn = skn + D;
+  bf16_t* sqb = (bf16_t*)(svn + D);
 
-  int split = blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
+  int split = by_len ? blockIdx.z : blockIdx.x, hk = by_len ? blockIdx.x : blockIdx.y, b = by_len ? blockIdx.y : blockIdx.z;
   if constexpr (XC) {  // the same-XCD mapping of decode_attn_kernel
     const int wl = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
     const int s8 = wl >> 3, pair = (s8 / nsplit) * 8 + (wl & 7);
@@ -1507,192 +1505,230 @@ decode_attn_mfma1_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __
     hk = pair % Hkv;
     b = pair / Hkv;
   }
-  const int L = lens[b];
+  const int L = __builtin_amdgcn_readfirstlane(lens[b]);  // (uniform, for the DMA's resources)
   DA_ASSERT(L >= 0 && L <= max_seq && slot[b] >= 0);
-  const int chunk = dec_chunk(L, nsplit, chunk_max);
-  DA_ASSERT(chunk <= 8 * KT);
+  const int act = by_len && cnt ? min(nsplit, max(1, (L + chunk_max - 1) / chunk_max)) : nsplit;  // (see the GQA kernel)
+  if (split >= act) return;
+  const int chunk = dec_chunk(L, act, by_len ? 0x7fffffff : chunk_max);
   const int kstart = split * chunk;
   const bool own_new = RP && kstart <= L - 1 && L - 1 < kstart + chunk;  // this split holds key L - 1
   const int kend = min(RP ? L - 1 : L, kstart + chunk);                  // RP: key L - 1 from the qkv row
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fg = lane >> 4;
-  const size_t cbase = ((size_t)slot[b] * Hkv + hk) * (size_t)max_seq * D;
-  const int P = pre ? pre[2 * b] : 0;  // shared-prefix keys [0, P) live in slot pre[2b + 1]
-  const size_t pbase = P ? ((size_t)pre[2 * b + 1] * Hkv + hk) * (size_t)max_seq * D : cbase;
+  const size_t cbase = ((size_t)__builtin_amdgcn_readfirstlane(slot[b]) * Hkv + hk) * (size_t)max_seq * D;
+  const int P = pre ? __builtin_amdgcn_readfirstlane(pre[2 * b]) : 0;  // shared-prefix keys [0, P) live in slot pre[2b + 1]
+  const size_t pbase = P ? ((size_t)__builtin_amdgcn_readfirstlane(pre[2 * b + 1]) * Hkv + hk) * (size_t)max_seq * D : cbase;
   DA_ASSERT(P % 64 == 0 && P <= L);
   DA_ASSERT(!RP || rope.pos[b] == L - 1);
+  char* mine = ring + w * (ST * 2 * TB);
 
-  // ---- both tiles of this wave requested up front (branch-free: an empty tile reads key 0 of
-  //      the row's own slot, valid memory whose scores are masked) ----
-  const int ta = kstart + w * KT, tb = ta + 4 * KT;
-  u32x4_t kr[2][4][NDS];
-  auto issue = [&](int j, int t0) {
-    const int nk = kend - t0;
-    const bool shared = t0 < P;
-    const bf16_t* kb = nk > 0 ? kc + (shared ? pbase : cbase) + (size_t)t0 * D : kc + cbase;
-    const bf16_t* vb = nk > 0 ? vc + (shared ? pbase : cbase) + (size_t)t0 * D : vc + cbase;
-    const int last = nk > 0 ? min(KT, nk) - 1 : 0;
+  // this thread's element d of the query and (RP) of the new key and value, with its partner in the pair and its angle
+  const bf16_t* qrow = q + (size_t)b * ldq;
+  bf16x8_t qf[NDS];
+  [[maybe_unused]] unsigned rq = 0, rk = 0, rv = 0;
+  [[maybe_unused]] f32x2_t rcs = f32x2_t{1.f, 0.f};
+  const int d = min(tid, D - 1);
+  if constexpr (RP) {
+    rq = *(const unsigned*)(qrow + hk * D + (d & ~1));
+    rk = *(const unsigned*)(qrow + (size_t)(H + hk) * D + (d & ~1));
+    rv = *(const unsigned*)(qrow + (size_t)(H + Hkv + hk) * D + (d & ~1));
+    rcs = *(const f32x2_t*)(rope.cs + ((size_t)max(L - 1, 0) * (D / 2) + (d >> 1)) * 2);
+  } else {
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int ds = 0; ds < NDS; ++ds) qf[ds] = *(const bf16x8_t*)(qrow + hk * D + ds * 32 + fg * 8);
+  }
+  unsigned ko[8], vo[8];  // DMA sources within a tile
 #pragma unroll
-      for (int ds = 0; ds < NDS; ++ds) {
-        const int key = min(16 * t + fr, last);
-        kr[j][t][ds] = __builtin_nontemporal_load((const u32x4_t*)(kb + (size_t)key * D + ds * 32 + fg * 8));
-      }
-    char* myv = sv + (w * 2 + j) * VBYTES;
+  for (int i = 0; i < ND; ++i) {
+    const int p = i * 64 + lane, row = p / NS, sl = p % NS;
+    ko[i] = (unsigned)(row * D * 2 + ((sl ^ kswz<D>(row)) << 4));
+    vo[i] = (unsigned)(row * D * 2 + ((sl ^ vswz<D>(row)) << 4));
+  }
+  __builtin_amdgcn_sched_barrier(0);  // (the loads above are the oldest)
+  auto issue = [&](const bf16_t* cache, const unsigned (&off)[8], int t0, char* dst) __attribute__((always_inline)) {
+    // the tile from key t0 on (none past kend)
+    const int n = __builtin_amdgcn_readfirstlane(max(0, min(KT, kend - t0))) * D * 2;
+    const size_t at = (t0 < P ? pbase : cbase) + (size_t)t0 * D;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(cache + at), (short)0, n, 0x00020000);
 #pragma unroll
-    for (int i = 0; i < NDMA; ++i) {
-      const int pc = i * 64 + lane, row = pc / NS, sl = pc % NS;
-      const int c = sl ^ vswz1<D>(row);
-      const int key = min(row, last);
+    for (int i = 0; i < ND; ++i)
       // aux 2 = nt: the KV stream is read once per step; allocating it in L2 / MALL cost the GEMVs
       // that follow ~3 % (their weights lose cache residency): profiles/r5/decode_mfma1/
-      __builtin_amdgcn_global_load_lds((gptr_t)(vb + (size_t)key * D + c * 8), (lds_ptr_t)(myv + i * 1024), 16, 0, 2);
-    }
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(dst + i * 1024), 16, off[i & 7], 0, 0, 2);
   };
-  issue(0, ta);
-  issue(1, tb);
-
-  bf16x8_t qf[NDS];
-  [[maybe_unused]] __shared__ __attribute__((aligned(16))) bf16_t sqb[RP ? D : 1];
-  [[maybe_unused]] __shared__ float skn[RP ? D : 1], svn[RP ? D : 1];
-  [[maybe_unused]] __shared__ float ssn;
-  if constexpr (RP) {
-    // rotate q (and the new key) at position L - 1, rounded to bf16 like the rope_cache kernel
-    constexpr int HALF = D / 2;
-    const bf16_t* qrow = q + (size_t)b * ldq;
-    if (tid < D) {
-      const int d = tid, i = d >> 1;
-      const float c = rope.cs[((size_t)(L - 1) * HALF + i) * 2], sn = rope.cs[((size_t)(L - 1) * HALF + i) * 2 + 1];
-      auto rot = [&](const bf16_t* hp) {
-        const float x1 = bf2f(hp[d & ~1]), x2 = bf2f(hp[d | 1]);
-        return f2bf((d & 1) ? x2 * c + x1 * sn : x1 * c - x2 * sn);
-      };
-      sqb[d] = rot(qrow + hk * D);
-      if (own_new) {
-        const bf16_t kn = rot(qrow + (size_t)(H + hk) * D), vn = qrow[(size_t)(H + Hkv + hk) * D + d];
-        skn[d] = bf2f(kn);
-        svn[d] = bf2f(vn);
-        const size_t crow = cbase + (size_t)(L - 1) * D;
-        rope.kc[crow + d] = kn;  // for later steps (read back only after this launch)
-        rope.vc[crow + d] = vn;
-      }
-    }
-    __syncthreads();
+  auto landed = [&]() __attribute__((always_inline)) {  // the oldest K or V tile of the ring is in
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ND * (2 * ST - 1)) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
 #pragma unroll
-    for (int ds = 0; ds < NDS; ++ds)
-      qf[ds] = fr == 0 ? *(const bf16x8_t*)(sqb + ds * 32 + fg * 8) : bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+  for (int i = 0; i < ST; ++i) {
+    issue(kc, ko, kstart + (w + 4 * i) * KT, mine + i * 2 * TB);
+    issue(vc, vo, kstart + (w + 4 * i) * KT, mine + i * 2 * TB + TB);
+  }
+  [[maybe_unused]] bf16_t kn = 0;
+  if constexpr (RP) {
+    asm volatile("" : "+v"(rq), "+v"(rk), "+v"(rv), "+v"(rcs));  // (waited for here, the tiles on their way)
+    // rotate q (and the new key) at position L - 1, rounded to bf16 like the rope_cache kernel
+    auto rot = [&](unsigned x) {
+      const float x1 = bf2f((bf16_t)(x & 0xffff)), x2 = bf2f((bf16_t)(x >> 16));
+      return f2bf((d & 1) ? x2 * rcs[0] + x1 * rcs[1] : x1 * rcs[0] - x2 * rcs[1]);
+    };
+    kn = rot(rk);
+    if (tid < D) {
+      sqb[d] = rot(rq);
+      skn[d] = bf2f(kn);
+      svn[d] = bf2f((bf16_t)((d & 1) ? rv >> 16 : rv & 0xffff));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // (__syncthreads() would wait for the tiles)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ds = 0; ds < NDS; ++ds) qf[ds] = *(const bf16x8_t*)(sqb + ds * 32 + fg * 8);
     if (own_new && w == 0) {  // score of the new key (log2 units)
       float part = 0.f;
-      for (int d = lane; d < D; d += 64) part += bf2f(sqb[d]) * skn[d];
+      for (int e = lane; e < D; e += 64) part += bf2f(sqb[e]) * skn[e];
       part = wave_sum(part);
-      if (lane == 0) ssn = part * scale_log2e;
+      if (lane == 0) *ssn = part * scale_log2e;
     }
   } else {
 #pragma unroll
-    for (int ds = 0; ds < NDS; ++ds)
-      qf[ds] = fr == 0 ? *(const bf16x8_t*)(q + (size_t)b * ldq + hk * D + ds * 32 + fg * 8)
-                       : bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+    for (int ds = 0; ds < NDS; ++ds) asm volatile("" : "+v"(qf[ds]));
   }
+  // transposed V reads (see the GQA kernel)
+  const int vr = 4 * fg + (fr >> 2), vx = vswz<D>(vr) >> 1;
+  const unsigned vrow = vr * (D * 2) + ((fr & 3) >> 1) * 16 + (fr & 1) * 8;
   f32x4_t oacc[NDT];
 #pragma unroll
   for (int i = 0; i < NDT; ++i) oacc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_part = 0.f;
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // both tiles' K registers and V regions landed
-
-  auto process = [&](int j, int t0) {
-    const int nk = kend - t0;
-    f32x4_t sacc[4];
+  int stage = 0;
+  for (int t0 = kstart + w * KT; t0 < kend; t0 += 4 * KT) {
+    char* kt = mine + stage * 2 * TB;
+    char* vt = kt + TB;
+    landed();
+    bf16x8_t kf[2][NDS];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      sacc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int ds = 0; ds < NDS; ++ds) sacc[t] = mfma16(__builtin_bit_cast(bf16x8_t, kr[j][t][ds]), qf[ds], sacc[t]);
-    }
+      for (int ds = 0; ds < NDS; ++ds)
+        kf[t][ds] = *(const bf16x8_t*)(kt + (16 * t + fr) * (D * 2) + (((4 * ds + fg) ^ kswz<D>(16 * t + fr)) << 4));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    issue(kc, ko, t0 + 4 * ST * KT, kt);
+    f32x4_t sacc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int ds = 0; ds < NDS; ++ds)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) sacc[t] = mfma16(kf[t][ds], qf[ds], sacc[t]);
     float mx = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int key = 16 * t + 4 * fg + i;
-        const float sc = key < nk ? sacc[t][i] * scale_log2e : -INFINITY;
+        const float sc = t0 + 16 * t + 4 * fg + i < kend ? sacc[t][i] * scale_log2e : -INFINITY;
         sacc[t][i] = sc;
         mx = fmaxf(mx, sc);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = max_xhalf(mx);
-    const float m_new = fmaxf(m_run, mx);
-    const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-    const float alpha = exp2f(m_run - m_use);
-    m_run = m_new;
-    float psum = 0.f;
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+    mx = max_xhalf(fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1])));
+    if (__ballot(mx > m_run)) {  // (a new maximum is rare after the first tiles)
+      const float m_new = fmaxf(m_run, mx);
+      const float alpha = exp2f(m_run - (m_new == -INFINITY ? 0.f : m_new));
+      m_run = m_new;
+      l_part *= alpha;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+      for (int i = 0; i < NDT; ++i) oacc[i] *= alpha;
+    }
+    const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
+    unsigned pw[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float p = __builtin_amdgcn_exp2f(sacc[t][i] - m_use);
-        sacc[t][i] = p;
-        psum += p;
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; i += 2) {
+        unsigned x[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {  // this column's 8 bits of the weight
+          const float p = __builtin_amdgcn_exp2f(sacc[t][i + j] - m_use);
+          l_part += p;
+          const float r1 = p - __uint_as_float(__float_as_uint(p) & 0xffff0000u);
+          const float r2 = r1 - __uint_as_float(__float_as_uint(r1) & 0xffff0000u);
+          x[j] = __float_as_uint(fr == 0 ? p : fr == 1 ? r1 : r2);
+        }
+        pw[2 * t + i / 2] = __builtin_amdgcn_perm(x[1], x[0], 0x07060302u);
       }
-    l_part = l_part * alpha + psum;
+    const bf16x8_t pb = __builtin_bit_cast(bf16x8_t, u32x4_t{pw[0], pw[1], pw[2], pw[3]});
+    landed();
+    const unsigned va0 = (unsigned)(size_t)(lds_ptr_t)vt + vrow;
+    s16x4_t v[2][8];
+    constexpr int HT = NDT % 4 ? 3 : 4;  // d-tiles of a block of transposed reads
 #pragma unroll
-    for (int i = 0; i < NDT; ++i) oacc[i] *= alpha;
-    const char* myv = sv + (w * 2 + j) * VBYTES;
+    for (int h = 0; h < NDT / HT; ++h) {
+      const int dt = HT * h;
+      if constexpr (HT == 4)
+        asm volatile("ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %8 offset:%12\n\t"
+                     "ds_read_b64_tr_b16 %2, %9\n\tds_read_b64_tr_b16 %3, %9 offset:%12\n\t"
+                     "ds_read_b64_tr_b16 %4, %10\n\tds_read_b64_tr_b16 %5, %10 offset:%12\n\t"
+                     "ds_read_b64_tr_b16 %6, %11\n\tds_read_b64_tr_b16 %7, %11 offset:%12\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&v"(v[h][0]), "=&v"(v[h][1]), "=&v"(v[h][2]), "=&v"(v[h][3]), "=&v"(v[h][4]), "=&v"(v[h][5]),
+                       "=&v"(v[h][6]), "=&v"(v[h][7])
+                     : "v"(va0 + ((dt ^ vx) << 5)), "v"(va0 + (((dt + 1) ^ vx) << 5)), "v"(va0 + (((dt + 2) ^ vx) << 5)),
+                       "v"(va0 + (((dt + 3) ^ vx) << 5)), "n"(16 * D * 2)
+                     : "memory");
+      else
+        asm volatile("ds_read_b64_tr_b16 %0, %6\n\tds_read_b64_tr_b16 %1, %6 offset:%9\n\t"
+                     "ds_read_b64_tr_b16 %2, %7\n\tds_read_b64_tr_b16 %3, %7 offset:%9\n\t"
+                     "ds_read_b64_tr_b16 %4, %8\n\tds_read_b64_tr_b16 %5, %8 offset:%9\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&v"(v[h][0]), "=&v"(v[h][1]), "=&v"(v[h][2]), "=&v"(v[h][3]), "=&v"(v[h][4]), "=&v"(v[h][5])
+                     : "v"(va0 + ((dt ^ vx) << 5)), "v"(va0 + (((dt + 1) ^ vx) << 5)), "v"(va0 + (((dt + 2) ^ vx) << 5)),
+                       "n"(16 * D * 2)
+                     : "memory");
+      if (h == NDT / HT - 1) issue(vc, vo, t0 + 4 * ST * KT, vt);
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const u32x4_t pw = u32x4_t{pack_bf2(sacc[2 * c][0], sacc[2 * c][1]), pack_bf2(sacc[2 * c][2], sacc[2 * c][3]),
-                                 pack_bf2(sacc[2 * c + 1][0], sacc[2 * c + 1][1]),
-                                 pack_bf2(sacc[2 * c + 1][2], sacc[2 * c + 1][3])};
-      const bf16x8_t pb = __builtin_bit_cast(bf16x8_t, pw);
-      const int q4 = fr >> 2, p4 = fr & 3;
-#pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) {
-        const int col = dt * 16 + 4 * p4;
-        const int r0 = 32 * c + 4 * fg + q4, r1 = r0 + 16;
-        const s16x4_t lo = lds_read_tr16(myv + r0 * (D * 2) + (((col >> 3) ^ vswz1<D>(r0)) << 4) + (col & 7) * 2);
-        const s16x4_t hi = lds_read_tr16(myv + r1 * (D * 2) + (((col >> 3) ^ vswz1<D>(r1)) << 4) + (col & 7) * 2);
-        const bf16x8_t va = bf16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        oacc[dt] = mfma16(va, pb, oacc[dt]);
+      for (int j = 0; j < HT; ++j) {
+        const s16x4_t lo = v[h][2 * j], hi = v[h][2 * j + 1];
+        oacc[dt + j] = mfma16(bf16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, pb, oacc[dt + j]);
       }
     }
-  };
-  if (ta < kend) process(0, ta);
-  if (tb < kend) process(1, tb);
-
-  // ---- merge the 4 waves (query column 0: lanes fr == 0) through LDS ----
+    stage = stage + 1 == ST ? 0 : stage + 1;
+  }
+  // ---- merge the 4 waves (columns 0 - 2: lanes fr < 3) through LDS ----
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (pieces past the end write zeros)
+  if (RP && own_new && tid < D) {  // for later steps (read back only after this launch)
+    const size_t crow = cbase + (size_t)(L - 1) * D;
+    rope.kc[crow + d] = kn;
+    rope.vc[crow + d] = (bf16_t)((d & 1) ? rv >> 16 : rv & 0xffff);
+  }
   float l_tot = l_part + __shfl_xor(l_part, 16, 64);
   l_tot = sum_xhalf(l_tot);
   if (lane == 0) { swm[w] = m_run; swl[w] = l_tot; }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __syncthreads();  // every wave is done with its V regions
-  float* so = (float*)sv;  // [4][D]: column 0 of each wave's O^T
-  if (fr == 0) {
+  __syncthreads();  // every wave is done with its ring
+  float* so = (float*)ring;  // [4][3][D]
+  if (fr < 3) {
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) so[w * D + dt * 16 + 4 * fg + i] = oacc[dt][i];
+      for (int i = 0; i < 4; ++i) so[(w * 3 + fr) * D + dt * 16 + 4 * fg + i] = oacc[dt][i];
   }
   __syncthreads();
-  for (int d = tid; d < D; d += 256) {
+  if (tid < D) {
     float M = fmaxf(fmaxf(swm[0], swm[1]), fmaxf(swm[2], swm[3]));
-    if (own_new) M = fmaxf(M, ssn);
+    if (own_new) M = fmaxf(M, *ssn);
     const float Mu = (M == -INFINITY) ? 0.f : M;
     float o = 0.f, ls = 0.f;
 #pragma unroll
     for (int ww = 0; ww < 4; ++ww) {
       const float f = exp2f(swm[ww] - Mu);
-      o += so[ww * D + d] * f;
+      o += (so[(ww * 3) * D + d] + (so[(ww * 3 + 1) * D + d] + so[(ww * 3 + 2) * D + d])) * f;
       ls += swl[ww] * f;
     }
     if (own_new) {  // the new token's key: weight exp2(s - M), value straight from the qkv row
-      const float f = exp2f(ssn - Mu);
+      const float f = exp2f(*ssn - Mu);
       o += svn[d] * f;
       ls += f;
     }
-    dec_store(o, M, ls, b, hk, d, H, nsplit, split, D, po, pm, pl, out, ldo, nsplit);
+    dec_store(o, M, ls, b, hk, d, H, nsplit, split, D, po, pm, pl, out, ldo, act);
   }
-  __shared__ int s_last;
-  dec_finish<D, 1, XC>(po, pm, pl, H, Hkv, nsplit, b, hk, cnt, out, ldo, &s_last, nsplit);
+  dec_finish<D, 1, XC>(po, pm, pl, H, Hkv, nsplit, b, hk, cnt, out, ldo, (int*)(ssn + 1), act);
 }
 
 template <int D>
@@ -1734,12 +1770,10 @@ static int launch_decode_v(int G, dim3 grid, hipStream_t s, const bf16_t* q, int
 
 // GQA groups (G >= 2) take the MFMA kernel: 1.8x (Llama-3-8B, G=4) to 5x (Llama-3-70B TP=8, G=8)
 // over the VALU path (profiles/decode_attn_gqa_mfma_r1.json); the VALU kernel covers the other
-// head dims. MHA (G = 1) decode prefetches each wave's next tile (VAR bit 2) when the launch has
-// few (row, kv head) pairs (B * Hkv <= 32: latency-bound), else streams with V issued with K.
-//
-// Measured on MI355X (profiles/decode_attn_variants_r1.json): non-temporal K/V loads + V issued with
-// K reach 6.5 TB/s for MHA (G = 1, Phi-3); with G >= 2 the extra V registers cost more occupancy
-// than they buy, so those keep V after the scores (nt loads only).
+// head dims. So does MHA (G = 1), with decode_attn_mfma1_kernel; DA_DECODE_MFMA1=0 gives it the VALU kernel, which
+// prefetches each wave's next tile (VAR bit 2) when the launch has few (row, kv head) pairs (B * Hkv <= 32), else streams
+// with V issued with K. With G >= 2 the extra V registers cost more occupancy than they buy
+// (profiles/decode_attn_variants_r1.json), so those keep V after the scores (nt loads only).
 constexpr int kDecPrefetchPairs = 32;
 
 template <int D>
@@ -1747,22 +1781,24 @@ static int launch_decode(int G, dim3 grid, hipStream_t s, const bf16_t* q, int l
                          const bf16_t* vc, const int* lens, const int* slot, const int* pre, int H, int Hkv, int max_seq, int chunk,
                          int nsplit, float sl2e, float* po, float* pm, float* pl, bf16_t* out, int ldo,
                          int* cnt, DecRope rope, int xc) {
-  const int by_len = xc >> 1;  // GQA on MFMA: splits by the row's length (bit 1)
+  const int by_len = xc >> 1;  // on MFMA: splits by the row's length (bit 1)
   xc &= 1;
   static int mfma1 = -1;
   if (mfma1 < 0) {
     const char* e = getenv("DA_DECODE_MFMA1");
     mfma1 = (e && e[0] == '0') ? 0 : 1;
   }
-  if (mfma1 && G == 1 && (int)(grid.y * grid.z) <= kDecPrefetchPairs && chunk <= 512) {
+  if (mfma1 && G == 1) {
     if (xc && ((grid.y * grid.z) % 8 || !cnt || nsplit < 2)) return (int)hipErrorInvalidValue;
-#define M1(XCV, RPV) decode_attn_mfma1_kernel<D, XCV, RPV><<<grid, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, \
-                         max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt, rope)
+    const dim3 grid_g = by_len && !xc ? dim3(Hkv, grid.z, nsplit) : grid;
+#define M1(XCV, RPV) decode_attn_mfma1_kernel<D, XCV, RPV><<<grid_g, 256, 0, s>>>(q, ldq, kc, vc, lens, slot, pre, H, Hkv, \
+                         max_seq, chunk, nsplit, sl2e, po, pm, pl, out, ldo, cnt, rope, by_len)
     if (xc) { if (rope.cs) M1(true, true); else M1(true, false); }
     else { if (rope.cs) M1(false, true); else M1(false, false); }
 #undef M1
     return (int)hipGetLastError();
   }
+  if (by_len && G == 1) chunk = 0x7fffffc0;  // (even splits of any length)
   if (xc) {  // same-XCD split exchange (cached ws / counters): the prefetching MHA form only
     if (G != 1 || (int)(grid.y * grid.z) > kDecPrefetchPairs || (grid.y * grid.z) % 8 || !cnt || nsplit < 2)
       return (int)hipErrorInvalidValue;

@@ -971,6 +971,19 @@ def _gqa_split(B: int, Hkv: int, max_len: int):
     return chunk, nsplit, False
 
 
+def _mha_split(B: int, H: int, max_len: int):
+    """(chunk, nsplit, by_len) of a launch with a KV head to each query head whose caller names no chunk: a row's keys over as
+    many of the even splits as hold 256 of them each, or 128 where the launch has up to 32 (row, head) pairs and would leave
+    CUs idle. us even / by length of 64 / 128 / 256, 32 heads x 96 in caches of 4096: one row of 60 7.4 / 5.5 / 5.5 / 5.5, of 500
+    8.0 / 8.1 / 7.5 / 8.3, of 2935 11.7 / 11.7 / 11.6 / 11.6; 4 rows of 64 - 146 8.7 / 9.3 / 7.8 / 6.5, of 200 - 500 9.8 / 10.6 /
+    10.5 / 9.0, of 900 - 3100 26.5 / 26.2 / 26.0 / 25.1; 8 rows 9.3 / 10.0 / 9.9 / 6.9, 12.2 / 13.3 / 13.2 / 13.1, 38.9 / 40.0 /
+    40.2 / 40.4."""
+    chunk, nsplit = _decode_split(B, H, max_len, 0)
+    if nsplit == 1:
+        return chunk, 1, False
+    return (BY_LEN_KEYS if B * H > 32 else BY_LEN_KEYS // 2), nsplit, True
+
+
 # Same-XCD split exchange of the batch-1..small-batch MHA decode attention (attention.hip, VAR bit 3):
 # all splits of a (row, kv head) pair on one XCD, their partials and ticket in cached memory (L2
 # round trips instead of uncached ones). It relies on the launch's workgroup -> XCD round-robin, so
@@ -1047,7 +1060,9 @@ def decode_attn(q, k_cache, v_cache, lens, slot, H, Hkv, D, max_len: int, chunk:
     k / v into the cache at pos (== lens - 1) — the decode step's rope_cache launch folded in."""
     cs, ps = _decode_checks(q, k_cache, v_cache, lens, slot, H, Hkv, D, max_len, pre, rope)
     B = q.shape[0]
-    if chunk <= 0 and H != Hkv and D in (64, 128):
+    if chunk <= 0 and H == Hkv:
+        chunk, nsplit, by_len = _mha_split(B, H, max_len)
+    elif chunk <= 0 and D in (64, 128):
         chunk, nsplit, by_len = _gqa_split(B, Hkv, max_len)
     else:
         (chunk, nsplit), by_len = _decode_split(B, Hkv, max_len, chunk), False
