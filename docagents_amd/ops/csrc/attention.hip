@@ -407,6 +407,203 @@ __device__ __forceinline__ void dma3_lds(__amdgpu_buffer_rsrc_t rs, unsigned lds
       : "memory", "scc");
 }
 
+// Two such pieces.
+__device__ __forceinline__ void dma2_lds(__amdgpu_buffer_rsrc_t rs, unsigned lds, unsigned v0, unsigned v1) {
+  unsigned keep;
+  asm volatile(
+      "s_nop 4\n\t"
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %4\n\t"
+      "s_nop 0\n\t"
+      "buffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
+      "s_add_u32 m0, m0, 0x400\n\t"
+      "s_nop 0\n\t"
+      "buffer_load_dwordx4 %2, %3, 0 offen lds\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(v0), "v"(v1), "s"(rs), "s"(lds)
+      : "memory", "scc");
+}
+
+// Bidirectional attention of the encoders (D = 64, no prefix): flash_attn_v2<64, 4, 1>'s tiles and arithmetic, with Q, K and V
+// by LDS-DMA, in rings of three K and two V tiles: the first of them are on their way with the queries, a K tile has two steps
+// to arrive in, and 40 KB and 128 registers let a CU have four workgroups (a third V tile, three workgroups: 92 us for 86). One
+// barrier a tile. 16-B chunk c of row r is at c ^ (r >> 1) in a K (and Q, O) tile and at c ^ ((r & 2) << 1) in a V tile: both
+// reads are free of bank conflicts. A wave without queries only moves its part of the tiles. Rows go out whole, through LDS.
+// The maximum that weights are relative to moves when it is 2^SPEC_TAU off (rescaling O takes a quarter of a tile's vector
+// instructions, and some row of 32 has a new maximum at most tiles of a short sequence).
+// Bound by the vector ALU (of 64 x 512 rows, 16 heads: 63 % of its cycles, the MFMAs 30 %) and by what is left of a round for
+// ragged sequences. us, by registers one tile ahead with two workgroups a CU / this: 80 texts of 61 - 512 rows, 16 heads, fp16
+// 110 / 86; 64 of 512 118 / 97 (710 TF); 12 heads, bf16: 80 of 61 - 512 78 / 60; one of 400 rows 13.0 / 11.1.
+template <typename T>
+__global__ void __launch_bounds__(256, 4)
+flash_attn_enc_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, int ldq, int ldk,
+                      int ldv, const int* __restrict__ cu, int H, int Hkv, float c, bf16_t* __restrict__ o, int ldo, int rev) {
+  constexpr int D = 64, KT = 64, RB = D * 2, TILE = KT * RB;
+  __shared__ __attribute__((aligned(16))) char smem[5 * TILE];
+  typedef __attribute__((address_space(3))) char lds_char;  // LDS byte offset, not the flat address
+
+  const FaBlock fb = fa_block(rev, 0, H / Hkv);
+  const int b = fb.b, h = fb.h, q0 = fb.qb * 128;
+  const int s0 = __builtin_amdgcn_readfirstlane(cu[b]), L = __builtin_amdgcn_readfirstlane(cu[b + 1]) - s0;
+  if (q0 >= L) return;
+  const int hk = h / (H / Hkv);
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int qr = lane & 31, hi = lane >> 5;
+  const int wq0 = q0 + w * 32;
+  const bool live = wq0 < L;
+  const int ntiles = (L + KT - 1) / KT;
+  const unsigned ring = (unsigned)(size_t)(lds_char*)smem;
+  auto rows_of = [&](const bf16_t* base, int ld, int r0, int n) __attribute__((always_inline)) {  // rows past the sequence: none
+    const int rows = __builtin_amdgcn_readfirstlane(max(0, min(n, L - r0)));
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(base + (size_t)(s0 + r0) * ld), (short)0, rows * ld * 2, 0x00020000);
+  };
+  // piece i of this wave: rows 16 w + 8 i + lane / 8 of a K or V tile (and of the wave's 32 queries, 8 i + lane / 8)
+  unsigned kx[2], vx[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = w * 16 + i * 8 + (lane >> 3);
+    kx[i] = (unsigned)(r * ldk * 2 + (((lane & 7) ^ ((r >> 1) & 7)) << 4));
+    vx[i] = (unsigned)(r * ldv * 2 + (((lane & 7) ^ ((r & 2) << 1)) << 4));
+  }
+  auto issue = [&](int t, int stage) __attribute__((always_inline)) {
+    dma2_lds(rows_of(k + hk * D, ldk, t * KT, KT), __builtin_amdgcn_readfirstlane(ring + stage * TILE + w * 2048), kx[0], kx[1]);
+  };
+  auto issue_v = [&](int t) __attribute__((always_inline)) {
+    dma2_lds(rows_of(v + hk * D, ldv, t * KT, KT), __builtin_amdgcn_readfirstlane(ring + (3 + (t & 1)) * TILE + w * 2048), vx[0], vx[1]);
+  };
+  char* mine = smem + w * 4096;  // this wave's output
+  const int qat = 2 * TILE + (w < 2 ? w : w + 2) * 4096;  // its queries: in the third K and the second V tile
+  {
+    const __amdgpu_buffer_rsrc_t rq = rows_of(q + h * D, ldq, wq0, 32);
+    const unsigned dst = __builtin_amdgcn_readfirstlane(ring + qat);
+    unsigned x[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = i * 8 + (lane >> 3);
+      x[i] = (unsigned)(r * ldq * 2 + (((lane & 7) ^ ((r >> 1) & 7)) << 4));
+    }
+    dma2_lds(rq, dst, x[0], x[1]);
+    dma2_lds(rq, dst + 2048, x[2], x[3]);
+  }
+  issue(0, 0);
+  issue_v(0);
+  issue(1, 1);
+  int xo[4];  // chunk 2 ds + hi of row qr
+#pragma unroll
+  for (int ds = 0; ds < 4; ++ds) xo[ds] = qr * RB + (((2 * ds + hi) ^ ((qr >> 1) & 7)) << 4);
+  // transposed V reads of a 16-key step: row 4 (g >> 1) + li / 4 (and 8 on), columns 32 db + 16 (g & 1) + 4 (li & 3)
+  const int g = lane >> 4, li = lane & 15;
+  int vo[2];
+#pragma unroll
+  for (int db = 0; db < 2; ++db)
+    vo[db] = (4 * (g >> 1) + (li >> 2)) * RB + ((db ^ (li >> 3)) << 6) + (g & 1) * 32 + (li & 3) * 8;
+  f32x16_t oacc[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
+  float m_run = -INFINITY, l_part = 0.f;
+  asm volatile("s_waitcnt vmcnt(6)" ::: "memory");  // the queries; the tiles may be on their way
+  bf16x8_t qf[4];
+#pragma unroll
+  for (int ds = 0; ds < 4; ++ds) qf[ds] = *(const bf16x8_t*)(smem + qat + xo[ds]);
+
+  int rd = 0;
+  for (int t = 0; t < ntiles; ++t) {
+    // this wave's part of tile t is in (K of t + 1 newer); after the barrier everyone's, and the places of t - 1 are free
+    asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    issue_v(t + 1);
+    issue(t + 2, rd == 0 ? 2 : rd - 1);
+    if (live) {
+      const char* sK = smem + rd * TILE;
+      const char* sV = smem + (3 + (t & 1)) * TILE;
+      f32x16_t sacc[2];
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sacc[hh][r] = 0.f;
+      bf16x8_t kfr[2][4];
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+        for (int ds = 0; ds < 4; ++ds) kfr[hh][ds] = *(const bf16x8_t*)(sK + hh * 32 * RB + xo[ds]);
+#pragma unroll
+      for (int ds = 0; ds < 4; ++ds)
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) sacc[hh] = T::mma32(kfr[hh][ds], qf[ds], sacc[hh]);
+      __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);  // DS reads
+      __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);  // MFMAs
+      if (t * KT + KT > L) {
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (t * KT + hh * 32 + 8 * (r >> 2) + 4 * hi + (r & 3) >= L) sacc[hh][r] = -INFINITY;
+      }
+      float mx = sacc[0][0];
+#pragma unroll
+      for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sacc[0][r]);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sacc[1][r]);
+      mx = max_xhalf(mx);
+      if (__any((mx - m_run) * c > SPEC_TAU)) {  // (weights of up to 2^SPEC_TAU are as exact)
+        const float m_new = fmaxf(m_run, mx);
+        const float alpha = exp2f((m_run - m_new) * c);
+        m_run = m_new;
+        l_part *= alpha;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) oacc[i] *= alpha;
+      }
+      const float mc = m_run == -INFINITY ? 0.f : -m_run * c;
+      float psum = 0.f;
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float p = __builtin_amdgcn_exp2f(fmaf(sacc[hh][r], c, mc));
+          sacc[hh][r] = p;
+          psum += p;
+        }
+      l_part += psum;
+      // O^T += V^T P^T over 4 steps of 16 keys: slot (hi, j) -> key 16 kc + 8 (j >> 2) + 4 hi + (j & 3)
+#pragma unroll
+      for (int kc = 0; kc < 4; ++kc) {
+        const int hh = kc >> 1, cb = (kc & 1) * 8;
+        const bf16x8_t pb = __builtin_bit_cast(
+            bf16x8_t, u32x4_t{T::pack2(sacc[hh][cb], sacc[hh][cb + 1]), T::pack2(sacc[hh][cb + 2], sacc[hh][cb + 3]),
+                              T::pack2(sacc[hh][cb + 4], sacc[hh][cb + 5]), T::pack2(sacc[hh][cb + 6], sacc[hh][cb + 7])});
+#pragma unroll
+        for (int db = 0; db < 2; ++db) {
+          const s16x4_t lo = lds_read_tr16(sV + kc * 16 * RB + vo[db]);
+          const s16x4_t up = lds_read_tr16(sV + (kc * 16 + 8) * RB + vo[db]);
+          oacc[db] = T::mma32(bf16x8_t{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]}, pb, oacc[db]);
+        }
+      }
+    }
+    rd = rd == 2 ? 0 : rd + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // (tiles past the end write zeros)
+  __builtin_amdgcn_s_barrier();
+  if (!live) return;
+  const float l_tot = sum_xhalf(l_part);
+  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+#pragma unroll
+  for (int db = 0; db < 2; ++db)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      *(u32x2_t*)(mine + qr * RB + (((db * 4 + e) ^ ((qr >> 1) & 7)) << 4) + hi * 8) =
+          u32x2_t{T::pack2(oacc[db][4 * e] * inv, oacc[db][4 * e + 1] * inv),
+                  T::pack2(oacc[db][4 * e + 2] * inv, oacc[db][4 * e + 3] * inv)};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = i * 8 + (lane >> 3);
+    const u32x4_t row = *(const u32x4_t*)(mine + r * RB + (((lane & 7) ^ ((r >> 1) & 7)) << 4));
+    if (wq0 + r < L) *(u32x4_t*)(o + (size_t)(s0 + wq0 + r) * ldo + h * D + (lane & 7) * 8) = row;
+  }
+}
+
 template <int D, bool SPEC, bool DMA>
 __global__ void __launch_bounds__(256, 2)
 flash_attn_pipe_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
@@ -1899,6 +2096,17 @@ DA_EXPORT int da_decode_attn(const void* q, int ldq, const void* k_cache, const 
 // chunk, profiles/r4/flash_order/).
 constexpr int kFaDispatch = 3;
 
+// The encoders' kernel takes bidirectional attention over own keys, D = 64, rows that 16-B accesses can reach and a tile's rows
+// within 2 GiB.
+template <typename T>
+static bool launch_fa_enc(const void* q, const void* k, const void* v, int ldq, int ldk, int ldv, const void* cu, int B,
+                          int max_seqlen, int H, int Hkv, float sl2e, void* o, int ldo, hipStream_t s) {
+  if (ldo % 8 || ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o) % 16 || max(max(ldq, ldk), ldv) > 1 << 22) return false;
+  flash_attn_enc_kernel<T><<<dim3((max_seqlen + 127) / 128, H, B), 256, 0, s>>>((const bf16_t*)q, (const bf16_t*)k,
+      (const bf16_t*)v, ldq, ldk, ldv, (const int*)cu, H, Hkv, sl2e, (bf16_t*)o, ldo, kFaDispatch);
+  return true;
+}
+
 // fp16 (the encoder's DTYPE=fp16): bidirectional or causal, no shared prefix, 4 waves x 32 queries
 DA_EXPORT int da_flash_attn_f16(const void* q, const void* k, const void* v, int ldq, int ldk, int ldv,
                                 const void* cu_seqlens, int B, int max_seqlen, int H, int Hkv, int D, int causal,
@@ -1908,6 +2116,9 @@ DA_EXPORT int da_flash_attn_f16(const void* q, const void* k, const void* v, int
   const FaPrefix pre{nullptr, nullptr, 0, 0, kFaDispatch};
   dim3 grid((max_seqlen + 127) / 128, H, B);
   hipStream_t s = (hipStream_t)stream;
+  if (D == 64 && !causal && launch_fa_enc<F16T>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv,
+                                                scale * 1.4426950408889634f, o, ldo, s))
+    return (int)hipGetLastError();
 #define FA_ARGS16 (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldq, ldk, ldv, (const int*)cu_seqlens, H, Hkv, \
                   causal, scale * 1.4426950408889634f, (bf16_t*)o, ldo, pre
   switch (D) {
@@ -2011,6 +2222,9 @@ DA_EXPORT int da_flash_attn_v2(const void* q, const void* k, const void* v, int 
     if (dma) return launch_fa_pipe<true>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv, causal, sl2e, o, ldo, pre, s);
     return launch_fa_pipe<false>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv, causal, sl2e, o, ldo, pre, s);
   }
+  if (D == 64 && !causal && pre_len == 0 &&
+      launch_fa_enc<BF16T>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv, sl2e, o, ldo, s))
+    return (int)hipGetLastError();
   if (D == 128) return launch_fa2<8, 1>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv, D, causal, sl2e, o, ldo, pre, s);
   return launch_fa2<4, 1>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv, D, causal, sl2e, o, ldo, pre, s);
 }
