@@ -6,7 +6,7 @@
 //
 // BT x BT tile (64, or 128 where the rows fill the chip), 4 waves of a quarter each, K in 128-byte slices through
 // double-buffered LDS (rows padded to 144 bytes: conflict-free 16-byte reads), the next slice's loads in flight while this
-// one is multiplied.
+// one is multiplied. fp32 operands have gemm_f32_kernel where K allows it.
 #include "seq.h"
 
 enum AnyEpi : int {
@@ -374,6 +374,186 @@ __global__ void __launch_bounds__(256) gemm_rows_kernel(AnyArgs p) {
   }
 }
 
+// fp32 operands, K a multiple of 32: the general kernel's products with operands by LDS-DMA in a ring of four 32-k stages (rows of
+// 128 bytes, 16-byte chunk c of row r at c ^ (r >> 1): conflict-free), one barrier a stage, and K over as many workgroups as
+// fill the chip. 32 rows x 128 columns for up to 32 rows, else 64 x 64; a wave has 32 x 32 of them.
+// Bound by the weights' bytes up to some 40 rows, by v_mfma_f32_16x16x4_f32 (157 TF) from there on. The general kernel, a slice
+// ahead and a workgroup for each 64 columns, took 482 us on average for 4096 columns with K = 4096 and 14336, 20 or 50 rows
+// alike: now 24 and 49, 28 and 72 (82 TF). 300 x 28672 x 4096 1239 -> 580 (121 TF), 8 x 28672 x 4096 267 -> 86 (5.5 TB/s).
+template <int BM>
+struct F32Tile {
+  static constexpr int BN = 4096 / BM, WN = BN / 32, STAGE = (BM + BN) * 128, ST = 4, P = (BM + BN) / 32;
+};
+
+template <int EPI, int BM>
+__global__ void __launch_bounds__(256, 2) gemm_f32_kernel(AnyArgs p, int splits, float* __restrict__ ws) {
+  using C = F32Tile<BM>;
+  constexpr int BN = C::BN, WN = C::WN, STAGE = C::STAGE, ST = C::ST, P = C::P;
+  typedef __attribute__((address_space(3))) void* lds_t;
+  extern __shared__ __attribute__((aligned(16))) char sm[];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wv / WN, wn = wv % WN;
+  const int fr = lane & 15, fg = lane >> 4, z = blockIdx.z;
+  // the row tiles of a column tile and slice beside each other (they read the same weights)
+  const int ntm = (p.M + BM - 1) / BM, ntn = (p.N + BN - 1) / BN;
+  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  const int m0 = id % ntm * BM, n0 = id / ntm % ntn * BN, split = id / (ntm * ntn);
+  const int nk = p.K / 32, k0 = (int)((long)split * nk / splits), kn = (int)((long)(split + 1) * nk / splits) - k0;
+  const int rot = ntm == 1 ? id % ntn % kn : 0;  // (each column tile begins elsewhere: the same columns of all rows are on few channels)
+  const int ra = min(BM, p.M - m0), rw = min(BN, p.N - n0);
+  const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)((const float*)p.A + z * p.sA + (size_t)m0 * p.lda), (short)0, ra * p.lda * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsw = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)((const float*)p.W + z * p.sW + (size_t)n0 * p.K), (short)0, rw * p.K * 4, 0x00020000);
+  unsigned off[8];  // piece wv P + i: 8 rows of A, then of W
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    const int row = (wv * P + i) * 8 + (lane >> 3), ld = row < BM ? p.lda : p.K;
+    off[i & 7] = (unsigned)((row < BM ? row : row - BM) * ld * 4 + (((lane & 7) ^ ((row >> 1) & 7)) << 4));
+  }
+  auto issue = [&](int t, int stage) __attribute__((always_inline)) {  // past the end: out of range, zeros, no traffic
+    const int soff = t < kn ? (k0 + (t + rot < kn ? t + rot : t + rot - kn)) * 128 : 0x7ffffff0;
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      const lds_t dst = (lds_t)(sm + stage * STAGE + (wv * P + i) * 1024);
+      if ((wv * P + i) * 8 < BM) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, dst, 16, off[i & 7], soff, 0, 0);
+      else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsw, dst, 16, off[i & 7], soff, 0, BM == 32 ? 2 : 0);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < ST - 1; ++i) issue(i, i);
+  f32x4_t acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  int at[2];  // chunk 4 ks + fg of row fr (and of the rows 16 on: the same swizzle)
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) at[ks] = fr * 128 + (((4 * ks + fg) ^ (fr >> 1)) << 4);
+  int rd = 0;
+  for (int t = 0; t < kn; ++t) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(P * (ST - 2)) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    issue(t + ST - 1, rd == 0 ? ST - 1 : rd - 1);
+    const char* sa = sm + rd * STAGE + wm * 32 * 128;
+    const char* sw = sm + rd * STAGE + (BM + wn * 32) * 128;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      f32x4_t fa[2], fw[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        fa[i] = *(const f32x4_t*)(sa + i * 2048 + at[ks]);
+        fw[i] = *(const f32x4_t*)(sw + i * 2048 + at[ks]);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[j][e], fa[i][e], acc[i][j], 0, 0, 0);
+    }
+    rd = rd == ST - 1 ? 0 : rd + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (pieces past the end write zeros)
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int m = m0 + wm * 32 + i * 16 + fr, nb = n0 + wn * 32;
+    if (m >= p.M) continue;
+    if (splits > 1) {
+      float* o = ws + ((size_t)(split * gridDim.z + z) * p.M + m) * (ntn * BN) + nb + 4 * fg;
+      *(f32x4_t*)o = acc[i][0];
+      *(f32x4_t*)(o + 16) = acc[i][1];
+    } else if constexpr (any_paired(EPI)) {
+      if (nb >= p.N) continue;
+      f32x4_t u{0.f, 0.f, 0.f, 0.f};
+      if constexpr (EPI == ANY_RGLRU) u = *(const f32x4_t*)((const float*)p.u + (size_t)m * p.ldu + z * (p.N / 2) + nb / 2 + 4 * fg);
+      any_pair<EPI>(p, z, m, nb, fg, acc[i][0], acc[i][1], u);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) any_block<float, EPI>(p, z, m, nb + j * 16 + 4 * fg, acc[i][j]);
+    }
+  }
+}
+
+// The splits' sums and the epilogue: a thread per four columns (paired: four columns of each half).
+template <int EPI>
+__global__ void __launch_bounds__(256) gemm_f32_reduce_kernel(AnyArgs p, int splits, const float* __restrict__ ws, int np) {
+  constexpr int V = any_paired(EPI) ? 8 : 4;
+  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
+  const int z = blockIdx.z, c = (int)(idx % (np / V));
+  const long m = idx / (np / V);
+  if (m >= p.M) return;
+  const int n = any_paired(EPI) ? c / 4 * 32 + c % 4 * 4 : c * 4;
+  const float* src = ws + ((size_t)z * p.M + m) * np + n;
+  const size_t step = (size_t)gridDim.z * p.M * np;
+  f32x4_t x{0.f, 0.f, 0.f, 0.f}, y = x;
+  for (int s0 = 0; s0 < splits; s0 += 4) {  // four on their way together
+    f32x4_t a[4], b[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float* q = src + min(s0 + j, splits - 1) * step;
+      a[j] = *(const f32x4_t*)q;
+      if constexpr (V == 8) b[j] = *(const f32x4_t*)(q + 16);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (s0 + j < splits) {
+        x += a[j];
+        if constexpr (V == 8) y += b[j];
+      }
+  }
+  if constexpr (V == 8) {
+    const int nb = c / 4 * 32, fg = c % 4;
+    if (nb >= p.N) return;
+    f32x4_t u{0.f, 0.f, 0.f, 0.f};
+    if constexpr (EPI == ANY_RGLRU) u = *(const f32x4_t*)((const float*)p.u + m * p.ldu + z * (p.N / 2) + nb / 2 + 4 * fg);
+    any_pair<EPI>(p, z, (int)m, nb, fg, x, y, u);
+  } else {
+    any_block<float, EPI>(p, z, (int)m, n, x);
+  }
+}
+
+// Workgroups along K of an fp32 product (0: the general kernel), each with 8 stages of K at least, by estimate in columns of K:
+// rounds of two workgroups a CU, a split's sums written and read, the second launch. (50 x 28672 x 4096, 448 tiles: whole 141
+// us, in two splits, 1.75 rounds, 146; 32 rows, 224 tiles: in two 90, in three 100.)
+static int f32_splits(long M, long N, long K, int lda, int batch) {
+  if (K % 32 || K > 1 << 21 || lda > 1 << 21) return 0;
+  const long bm = M <= 32 ? 32 : 64, tiles = (M + bm - 1) / bm * ((N + 4096 / bm - 1) / (4096 / bm)) * batch;
+  if (tiles > 0x7fffffffL / 64) return 0;
+  long best = 1, least = 0x7fffffffffffffffL;
+  for (long s = 1; s <= max(1L, min(K / 256, 64L)); ++s) {
+    const long cost = (tiles * s + 511) / 512 * K / s + (s > 1 ? 110 * s * tiles / 512 + 300 : 0);
+    if (cost < least) least = cost, best = s;
+  }
+  return (int)best;
+}
+static size_t f32_ws(long M, long N, int batch, int splits) {
+  const long bn = M <= 32 ? 128 : 64;
+  return splits > 1 ? (size_t)splits * batch * M * ((N + bn - 1) / bn * bn) * 4 : 0;
+}
+// Bytes of partial sums that an fp32 product wants (0: none).
+DA_EXPORT size_t da_gemm_any_ws(int M, int N, int K, int lda, int batch) {
+  return M < 1 || N < 1 || K < 1 || batch < 1 ? 0 : f32_ws(M, N, batch, f32_splits(M, N, K, lda, batch));
+}
+
+template <int EPI, int BM>
+static int launch_f32(const AnyArgs& a, int batch, int splits, float* ws, hipStream_t s) {
+  using C = F32Tile<BM>;
+  constexpr int lds = C::STAGE * C::ST;
+  static const hipError_t e = hipFuncSetAttribute((const void*)gemm_f32_kernel<EPI, BM>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return (int)e;
+  const int ntm = (a.M + BM - 1) / BM, ntn = (a.N + C::BN - 1) / C::BN;
+  gemm_f32_kernel<EPI, BM><<<dim3(ntm * ntn * splits, 1, batch), 256, lds, s>>>(a, splits, ws);
+  if (splits > 1) {
+    const int np = ntn * C::BN;
+    const long n = (long)a.M * (np / (any_paired(EPI) ? 8 : 4));
+    gemm_f32_reduce_kernel<EPI><<<dim3((unsigned)((n + 255) / 256), 1, batch), 256, 0, s>>>(a, splits, ws, np);
+  }
+  DA_LAUNCH_CHECK();
+}
+
 template <typename T, int EPI, int BT>
 static int launch_any(const AnyArgs& a, int batch, hipStream_t s) {
   constexpr int lds = 4 * BT * ANY_ROWB;
@@ -386,7 +566,11 @@ static int launch_any(const AnyArgs& a, int batch, hipStream_t s) {
   DA_LAUNCH_CHECK();
 }
 template <typename T, int EPI>
-static int launch_any_t(const AnyArgs& a, int batch, hipStream_t s) {
+static int launch_any_t(const AnyArgs& a, int batch, float* ws, hipStream_t s) {
+  if constexpr (sizeof(T) == 4) {
+    const int sp = f32_splits(a.M, a.N, a.K, a.lda, batch), splits = sp > 1 && !ws ? 1 : sp;
+    if (splits) return a.M <= 32 ? launch_f32<EPI, 32>(a, batch, splits, ws, s) : launch_f32<EPI, 64>(a, batch, splits, ws, s);
+  }
   if constexpr (sizeof(T) == 2 && (EPI == ANY_SOFTPLUS || EPI == ANY_RGLRU)) {
     if (a.M >= 1024 && a.K <= 256 && a.K % 32 == 0 && a.N % 16 == 0 && a.ldc % 4 == 0 &&
         (EPI != ANY_RGLRU || (a.A == a.u && a.sA == a.N / 2 && a.K == a.N / 2))) {
@@ -413,11 +597,12 @@ static int launch_any_t(const AnyArgs& a, int batch, hipStream_t s) {
 }
 
 // A [M, lda] and W [batch][N, K] of bf16 (f32 = 0) or fp32 (f32 = 1) elements with 16-byte aligned
-// rows, K a multiple of 16 bytes. The result is fp32, with ANY_ACT of the operands' type.
+// rows, K a multiple of 16 bytes. The result is fp32, with ANY_ACT of the operands' type. ws: fp32, da_gemm_any_ws bytes
+// (null: K is not split).
 DA_EXPORT int da_gemm_any(const void* A, int lda, const void* W, void* C, int ldc, const void* bias, int M, int N,
                           int K, int f32, int epi, int batch, long long sA, long long sW, long long sC,
                           long long sBias, const void* u, int ldu, const void* lam, void* decay, void* drive, int ldg,
-                          void* stream) {
+                          void* ws, void* stream) {
   const int e16 = f32 ? 4 : 8;
   if (M < 1 || N < 1 || K < 1 || batch < 1 || K % e16 || lda % e16 || sA % e16 || sW % e16 || (M + 63) / 64 > 65535)
     return (int)hipErrorInvalidValue;
@@ -432,7 +617,7 @@ DA_EXPORT int da_gemm_any(const void* A, int lda, const void* W, void* C, int ld
   a.u = u; a.lam = (const float*)lam; a.decay = (float*)decay; a.drive = (float*)drive; a.ldu = ldu; a.ldg = ldg;
   hipStream_t s = (hipStream_t)stream;
 #define ANY_CASE(E) \
-  case E: return f32 ? launch_any_t<float, E>(a, batch, s) : launch_any_t<bf16_t, E>(a, batch, s);
+  case E: return f32 ? launch_any_t<float, E>(a, batch, (float*)ws, s) : launch_any_t<bf16_t, E>(a, batch, nullptr, s);
   switch (epi) {
     ANY_CASE(ANY_NONE)
     ANY_CASE(ANY_SOFTPLUS)

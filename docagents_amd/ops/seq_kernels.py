@@ -14,7 +14,8 @@ from .seq_batch import PAGE, SeqBatch
 _META = [c_void_p] * 4 + [c_int] * 2
 K._SIGS.update({
     "da_gemm_any": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p] + [c_int] * 6 + [c_longlong] * 4
-                   + [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
+                   + [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p],
+    "da_gemm_any_ws": [c_int] * 5,
     "da_gemm_partials": [c_void_p, c_int, c_void_p] + [c_int] * 5 + [c_void_p, c_void_p],
     "da_stream_step": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_float, c_float, c_int, c_int]
                       + [c_void_p] * 5 + _META + [c_int, c_int, c_void_p],
@@ -43,7 +44,7 @@ K._SIGS.update({
                         c_float, c_float, K.ctypes.c_double] + [c_int] * 4 + [c_void_p, c_int, c_void_p] + [c_int] * 4
                        + _META + [c_int, c_void_p],
 })
-K._PART_OF.update({n: "hybrid" for n in ("da_gemm_any", "da_stream_step", "da_stream_final", "da_causal_conv",
+K._PART_OF.update({n: "hybrid" for n in ("da_gemm_any", "da_gemm_any_ws", "da_stream_step", "da_stream_final", "da_causal_conv",
                                          "da_selective_scan", "da_gated_scan", "da_sigmoid_attn", "da_stream_add", "da_delta_rule",
                                          "da_latent_prep", "da_latent_attn", "da_latent_gather", "da_latent_flash")})
 
@@ -84,6 +85,12 @@ def _scratch(m: SeqBatch, waves: int, fill: int, device, *shapes, deep: int = 1)
     return ws, [*map(_ptr, ws), _ptr(ck), _ptr(base), tot, n]
 
 
+def _split_sums(f32: int, M: int, N: int, Kd: int, lda: int, batch: int, device):
+    """Partial sums of an fp32 product whose K is split over workgroups (the call's own), None: it is not."""
+    n = lib().da_gemm_any_ws(M, N, Kd, lda, batch) if f32 else 0
+    return torch.empty(n // 4, dtype=torch.float32, device=device) if n else None
+
+
 def gemm_any(a, w, bias=None, epi: int = ANY_NONE, coef=None):
     """fp32 [M, N'] = epi(a[M, K] @ w[N, K]^T + bias), a and w both bf16 or both fp32, bias fp32; any M and
     N, K a multiple of 16 bytes. ANY_SOFTPLUS: softplus, times coef (fp32 [N]) if given; ANY_REGLU / ANY_SWIGLU: w
@@ -99,8 +106,9 @@ def gemm_any(a, w, bias=None, epi: int = ANY_NONE, coef=None):
         _f32(coef, "coef", N)
         _req(epi == ANY_SOFTPLUS, "coef goes with softplus")
     out = torch.empty((M, N // 2 if epi in (ANY_REGLU, ANY_SWIGLU) else N), dtype=torch.float32, device=a.device)
+    ws = _split_sums(f32, M, N, Kd, a.stride(0), 1, a.device)
     _check(lib().da_gemm_any(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), M, N, Kd, f32, epi, 1, 0,
-                             0, 0, 0, None, 0, _ptr(coef), None, None, 0, _stream()), "gemm_any")
+                             0, 0, 0, None, 0, _ptr(coef), None, None, 0, _ptr(ws), _stream()), "gemm_any")
     return out
 
 
@@ -115,8 +123,9 @@ def gemm_heads(a, w, stride: int, gate=None):
     if gate is not None:
         _act(gate, "gate", a.dtype)
         _req(gate.shape == out.shape and gate.stride(0) % 4 == 0, "gate")
+    ws = _split_sums(f32, M, N, Kd, a.stride(0), H, a.device)
     _check(lib().da_gemm_any(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), None, M, N, Kd, f32, ANY_ACT, H, stride,
-                             N * Kd, N, 0, _ptr(gate), 0 if gate is None else gate.stride(0), None, None, None, 0,
+                             N * Kd, N, 0, _ptr(gate), 0 if gate is None else gate.stride(0), None, None, None, 0, _ptr(ws),
                              _stream()), "gemm_heads")
     return out
 
@@ -157,8 +166,9 @@ def rglru_gates(u, w, bias, lam):
     _f32(lam, "lam", C)
     decay = torch.empty((T, C), dtype=torch.float32, device=u.device)
     drive = torch.empty_like(decay)
+    ws = _split_sums(f32, T, bw2, bw, u.stride(0), blocks, u.device)
     _check(lib().da_gemm_any(_ptr(u), u.stride(0), _ptr(w), None, 0, _ptr(bias), T, bw2, bw, f32, ANY_RGLRU, blocks, bw,
-                             bw2 * bw, 0, bw2, _ptr(u), u.stride(0), _ptr(lam), _ptr(decay), _ptr(drive), C, _stream()),
+                             bw2 * bw, 0, bw2, _ptr(u), u.stride(0), _ptr(lam), _ptr(decay), _ptr(drive), C, _ptr(ws), _stream()),
            "rglru_gates")
     return decay, drive
 

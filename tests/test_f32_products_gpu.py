@@ -1,0 +1,62 @@
+"""fp32 products with K split over workgroups: ends of row and column tiles, one to many splits, each epilogue, strided rows,
+batches, against 64-bit products; and K that only the general kernel takes."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from docagents_amd.ops import kernels as K
+
+
+def _near(got, want, mag, Kd):
+    # a chain of Kd fp32 additions, products exact to 2^-24; the functions behind it are 1-Lipschitz but for silu (1.1) and
+    # good to 2^-20 of what they return
+    assert ((got.double() - want).abs() <= 1.1 * (Kd + 4) * 2.0 ** -24 * mag + 2.0 ** -20 * (1 + want.abs())).all()
+
+
+@pytest.mark.parametrize("M", [1, 16, 32, 33, 64, 65, 200])
+@pytest.mark.parametrize("N,Kd", [(320, 8192), (36, 32), (160, 288), (4096, 512), (96, 1056), (64, 2052), (130, 4096)])
+@pytest.mark.parametrize("epi", [0, 1, 2, 4])
+def test_products(M, N, Kd, epi):
+    if epi in (2, 4) and N % 32:
+        pytest.skip("halves interleaved by 16")
+    g = torch.Generator(device="cuda").manual_seed(M + N + Kd)
+    a = torch.randn(M, Kd + 8, device="cuda", generator=g)[:, :Kd]
+    w = torch.randn(N, Kd, device="cuda", generator=g) * Kd ** -0.5
+    b = torch.randn(N, device="cuda", generator=g)
+    x, mag = a.double() @ w.double().t() + b.double(), a.double().abs() @ w.double().t().abs() + b.double().abs()
+    got = K.gemm_any(a, w, b, epi)
+    if epi == 1:
+        x = torch.nn.functional.softplus(x)
+    elif epi:
+        x, mag = x.view(M, N // 32, 2, 16), mag.view(M, N // 32, 2, 16)
+        gate = torch.relu(x[:, :, 0]) if epi == 2 else torch.nn.functional.silu(x[:, :, 0])
+        mag = (gate.abs() * mag[:, :, 1] + mag[:, :, 0] * x[:, :, 1].abs()).reshape(M, N // 2)
+        x = (gate * x[:, :, 1]).reshape(M, N // 2)
+    _near(got, x, mag, Kd)
+    assert torch.equal(K.gemm_any(a, w, b, epi), got)
+
+
+@pytest.mark.parametrize("M", [1, 33, 100])
+@pytest.mark.parametrize("H,N,Kd", [(5, 48, 96), (8, 128, 512)])
+def test_heads_and_gates(M, H, N, Kd):
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    a = torch.randn(M, H * (Kd + 16), device="cuda", generator=g)
+    w = torch.randn(H, N, Kd, device="cuda", generator=g) * Kd ** -0.5
+    gate = torch.randn(M, H * N, device="cuda", generator=g)
+    ah = a.view(M, H, Kd + 16)[:, :, :Kd].double().transpose(0, 1)
+    x = (ah @ w.double().transpose(1, 2).contiguous()).transpose(0, 1).reshape(M, H * N)
+    mag = (ah.abs() @ w.double().abs().transpose(1, 2).contiguous()).transpose(0, 1).reshape(M, H * N)
+    _near(K.gemm_heads(a, w, Kd + 16, gate), x * torch.sigmoid(gate.double()), mag, Kd)
+    # the recurrence's gates: rows of both interleaved by 16, blocks of Kd channels
+    u = torch.randn(M, H * Kd, device="cuda", generator=g)
+    wg = torch.randn(H, 2 * Kd, Kd, device="cuda", generator=g) * Kd ** -0.5
+    bias, lam = torch.randn(H, 2 * Kd, device="cuda", generator=g), -torch.rand(H * Kd, device="cuda", generator=g) - 0.1
+    decay, drive = K.rglru_gates(u, wg, bias, lam)
+    y = (u.view(M, H, Kd).double().transpose(0, 1) @ wg.double().transpose(1, 2).contiguous()).transpose(0, 1) + bias.double()
+    y = torch.sigmoid(y.view(M, H, Kd // 16, 2, 16))
+    want = torch.exp(lam.double() * y[:, :, :, 0].reshape(M, H * Kd))
+    assert (decay.double() - want).abs().max() <= 2.0 ** -18
+    want = torch.sqrt(1 - want ** 2) * y[:, :, :, 1].reshape(M, H * Kd) * u.double()
+    assert (drive.double() - want).abs().max() <= 2.0 ** -14
