@@ -212,6 +212,151 @@ gemm256_kernel(GemmArgs p) {
   }
 }
 
+// Smaller fp8 tiles, for products that 256 x 256 ones leave most CUs idle with: BT x BT, 4 waves of a quarter each, the K-steps
+// by LDS-DMA in a ring (the image and swizzle of the kernel above), one barrier a step, counted waits, two workgroups a CU.
+// The same MFMAs in the same order per result, the same roundings: the same bits whatever the tile.
+// Bound by latency: a 256 x 256 tile's prologue, K-steps one behind the other and epilogue take 15 - 27 us, however few rows.
+template <int EPI, int BT>
+__global__ void __launch_bounds__(256, 2)
+gemm_fp8_kernel(GemmArgs p) {
+  constexpr int WT = BT / 2, F = WT / 16, STG = 2 * BT * 128, ST = BT == 64 ? 4 : 2, P = BT / 16;
+  typedef __attribute__((ext_vector_type(8))) int i32x8_t;
+  __shared__ __attribute__((aligned(16))) char smem[ST * STG];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), wm = w >> 1, wn = w & 1;
+  const int fr = lane & 15, fg = lane >> 4;
+  const int ntm = (p.M + BT - 1) / BT;
+  const int t = xcd_remap(blockIdx.x, gridDim.x);
+  const int m0 = t % ntm * BT, n0 = t / ntm * BT, nk = p.K / 128;
+  // piece w P + i: 8 rows of A (waves 0 and 1) or of W; rows past the end are zeros
+  const bool isw = w >= 2;
+  const int ld = isw ? p.K : p.lda;
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      isw ? (void*)((const char*)p.W + (size_t)n0 * p.K) : (void*)((const char*)p.A + (size_t)m0 * p.lda), (short)0,
+      min(BT, isw ? p.N - n0 : p.M - m0) * ld, 0x00020000);
+  unsigned off[8];
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    const int r = ((w & 1) * P + i) * 8 + (lane >> 3);
+    off[i & 7] = (unsigned)(r * ld + (((lane & 7) ^ swz(r)) << 4));
+  }
+  auto issue = [&](int kt, int stage) __attribute__((always_inline)) {  // past the end: out of range, zeros, no traffic
+    const int soff = kt < nk ? kt * 128 : 0x7ffffff0;
+#pragma unroll
+    for (int i = 0; i < P; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(smem + stage * STG + (w * P + i) * 1024), 16, off[i & 7], soff, 0, 0);
+  };
+#pragma unroll
+  for (int i = 0; i < ST - 1; ++i) issue(i, i);
+  f32x4_t acc[F][F];
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  int at[2];  // chunks 2 fg and 2 fg + 1 of row fr (and of the rows 16, 32, .. on: the same swizzle)
+#pragma unroll
+  for (int h = 0; h < 2; ++h) at[h] = fr * 128 + (((2 * fg + h) ^ swz(fr)) << 4);
+  int rd = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    // ST > 2: this step's pieces are in, then everyone's, and the last step has been read. ST = 2: the place is read first
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(P * (ST - 2)) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    issue(kt + ST - 1, rd == 0 ? ST - 1 : rd - 1);
+    const char* sa = smem + rd * STG + wm * WT * 128;
+    const char* sb = smem + rd * STG + (BT + wn * WT) * 128;
+    u32x4_t fa[F][2], fb[F][2];
+#pragma unroll
+    for (int i = 0; i < F; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        fa[i][h] = *(const u32x4_t*)(sa + i * 2048 + at[h]);
+        fb[i][h] = *(const u32x4_t*)(sb + i * 2048 + at[h]);
+      }
+#pragma unroll
+    for (int i = 0; i < F; ++i)
+#pragma unroll
+      for (int j = 0; j < F; ++j)
+        // W first: lane (fr, fg) holds row fr, columns 4 fg .. 4 fg + 3 of each 16 x 16 block
+        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+            __builtin_bit_cast(i32x8_t, __builtin_shufflevector(fb[j][0], fb[j][1], 0, 1, 2, 3, 4, 5, 6, 7)),
+            __builtin_bit_cast(i32x8_t, __builtin_shufflevector(fa[i][0], fa[i][1], 0, 1, 2, 3, 4, 5, 6, 7)), acc[i][j], 0, 0, 0, 127,
+            0, 127);
+    rd = rd == ST - 1 ? 0 : rd + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (pieces past the end write zeros)
+  const int nb = n0 + wn * WT + 4 * fg;
+  f32x4_t swv[F], bv[F];
+#pragma unroll
+  for (int j = 0; j < F; ++j) {
+    const int n = min(nb + j * 16, p.N - 4);
+    swv[j] = *(const f32x4_t*)(p.sw + n);
+    bv[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (p.bias)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) bv[j][q] = bf2f(p.bias[n + q]);
+  }
+#pragma unroll
+  for (int i = 0; i < F; ++i) {
+    const int m = m0 + wm * WT + i * 16 + fr;
+    if (m >= p.M) continue;
+    const float sav = p.sa[m];
+#pragma unroll
+    for (int j = 0; j < F; ++j) {
+      if constexpr (EPI == EPI_SWIGLU) {
+        if (j & 1) continue;
+        const int col = (n0 + wn * WT + j * 16) / 2 + 4 * fg;
+        if (col >= p.N / 2) continue;
+        float v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = silu(acc[i][j][q] * (sav * swv[j][q])) * (acc[i][(j + 1) % F][q] * (sav * swv[(j + 1) % F][q]));
+        *(u32x2_t*)(p.C + (size_t)m * p.ldc + col) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+      } else {
+        const int n = nb + j * 16;
+        if (n >= p.N) continue;
+        float v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          v[q] = fmaf(acc[i][j][q], sav * swv[j][q], bv[j][q]);  // (as the kernel above compiles to)
+          if constexpr (EPI == EPI_GELU) v[q] = gelu_erf(v[q]);
+        }
+        u32x2_t o = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+        if constexpr (EPI == EPI_RESID) {
+          const u32x2_t r = *(const u32x2_t*)(p.resid + (size_t)m * p.ldr + n);
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            o[e] = pack_bf2(bf2f((bf16_t)(o[e] & 0xffff)) + bf2f((bf16_t)(r[e] & 0xffff)),
+                            bf2f((bf16_t)(o[e] >> 16)) + bf2f((bf16_t)(r[e] >> 16)));
+        }
+        *(u32x2_t*)(p.C + (size_t)m * p.ldc + n) = o;
+      }
+    }
+  }
+}
+
+// Which tile, us of 256 / 128 / 64 rows and columns: 64 x 3072 x 768 with GELU (48 tiles of 64) 24.5 / 12.9 / 6.8, 1000 rows (768)
+// 25.9 / 14.1 / 12.6, 2000 (1536; 384 of 128) 27.4 / 18.9 / 19.5, 4000 (768 of 128) 28.5 / 31.0 / 34.5; 3000 x 2304 x 768 (432)
+// 19.5 / 15.3, 4000 (576) 20.0 / 22.5; 1000 x 4096 x 1024 (1024 of 64) 29.1 / 15.4 / 15.4, 4000 (1024 of 128) 33.6 / 40.7.
+static int fp8_tile(long M, long N) {
+  auto tiles = [&](long t) { return (M + t - 1) / t * ((N + t - 1) / t); };
+  if (tiles(64) <= 1024) return 64;
+  return tiles(128) < 512 * ((tiles(256) + 255) / 256) ? 128 : 256;
+}
+
+template <int BT>
+static int launch_fp8(const GemmArgs& a, int epi, hipStream_t s) {
+  const dim3 grid(((a.M + BT - 1) / BT) * ((a.N + BT - 1) / BT));
+  switch (epi) {
+    case EPI_NONE: gemm_fp8_kernel<EPI_NONE, BT><<<grid, 256, 0, s>>>(a); break;
+    case EPI_BIAS: gemm_fp8_kernel<EPI_BIAS, BT><<<grid, 256, 0, s>>>(a); break;
+    case EPI_GELU: gemm_fp8_kernel<EPI_GELU, BT><<<grid, 256, 0, s>>>(a); break;
+    case EPI_SWIGLU: gemm_fp8_kernel<EPI_SWIGLU, BT><<<grid, 256, 0, s>>>(a); break;
+    case EPI_RESID: gemm_fp8_kernel<EPI_RESID, BT><<<grid, 256, 0, s>>>(a); break;
+    default: return (int)hipErrorInvalidValue;
+  }
+  return (int)hipGetLastError();
+}
+
 template <int FP8>
 static int launch256(const GemmArgs& a, int epi, hipStream_t s, dim3 grid, dim3 block) {
   switch (epi) {
@@ -227,6 +372,10 @@ static int launch256(const GemmArgs& a, int epi, hipStream_t s, dim3 grid, dim3 
 
 int launch_gemm256(const GemmArgs& a, int epi, hipStream_t s, int fp8) {
   if (!fp8) return (int)hipErrorInvalidValue;  // bf16: gemm8p
+  const int tile = (long)a.lda * 128 < 0x7fff0000 && (long)a.K * 128 < 0x7fff0000 && a.ldr % 4 == 0 && ((uintptr_t)a.sw & 15) == 0 &&
+                   (((uintptr_t)a.C | (uintptr_t)a.resid) & 7) == 0 ? fp8_tile(a.M, a.N) : 256;
+  if (tile == 64) return launch_fp8<64>(a, epi, s);
+  if (tile == 128) return launch_fp8<128>(a, epi, s);
   const int ntm = (a.M + BM - 1) / BM, ntn = (a.N + BN - 1) / BN;
   dim3 grid(ntm * ntn), block(512);
   return launch256<1>(a, epi, s, grid, block);

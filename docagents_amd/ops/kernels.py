@@ -561,7 +561,7 @@ def quant_weight_fp8(w: torch.Tensor):
 
 
 def gemm_fp8(aq, sa, wq, sw, bias=None, epi: int = EPI_NONE, resid=None, out=None) -> torch.Tensor:
-    """out[M, N] = epi((aq . wq^T) * sa[:, None] * sw[None, :]) with e4m3 operands (256x256 MFMA tile)."""
+    """out[M, N] = epi((aq . wq^T) * sa[:, None] * sw[None, :]) with e4m3 operands (MFMA tiles of 64, 128 or 256 squared)."""
     _req(aq.is_cuda and aq.dtype == FP8 and wq.dtype == FP8, "fp8 operands expected")
     M, K = aq.shape
     N, K2 = wq.shape
