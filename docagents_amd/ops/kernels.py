@@ -338,7 +338,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
             _bf16_cuda(gamma, "gamma"); _req(gamma.numel() == K, "gamma must be [K]")
     ws = None
     if splits <= 0:
-        if tile == 0 and 64 < M < ROW_TILES_BELOW and max(K, a.stride(0)) < 1 << 22:
+        if tile == 0 and M > 64 and _row_tiles_ok(M, N) and max(K, a.stride(0)) < 1 << 22:
             tile, splits = _row_tile(M, N, K, epi)
             ws = _call_partials(splits, M, N, a.device)
         elif tile == 0 and 128 < M < 640:
@@ -664,6 +664,15 @@ _ROW_TILES = {14: (128, 128, 8.46, 0.38, -0.06, -0.22, 1.9, 0.14), 15: (128, 64,
               18: (192, 128, 11.58, 0.46, -0.59, -2.04, 1.81, 0.16)}
 _PHASE_TILES = {7: (256, 10.76, 0.67, 0.64), 10: (128, 7.11, 0.55, 0.37)}
 ROW_TILES_BELOW = 1280
+# From there on small results only, whole, and where the estimate, 10 % up (rows are a larger part of what tiles load), is still
+# below the phase-split kernel's: of 1300 - 5000 rows, us phase-split / streaming: 1300 x 1024 x 1024 16.8 / 11.5, 2000 17.0 / 13.5;
+# 1600 x 768 x 3072 25.1 / 22.3; 1600 x 1024 x 4096 29.3 / 25.2; 3500 x 384 x 1536 22.4 / 17.7; 1300 x 4096 x 4096 54.0 / 46.7.
+# Not 2600 x 1024 x 1024 (18.1 / 19.2), 1600 x 4096 x 1024 (24.5 / 28.3) or 2000 x 3072 x 768 (20.3 / 22.4).
+SMALL_RESULT_ROWS, SMALL_RESULT = 5120, 21 << 18
+
+
+def _row_tiles_ok(M: int, N: int) -> bool:
+    return M < ROW_TILES_BELOW or (M <= SMALL_RESULT_ROWS and M * N <= SMALL_RESULT)
 
 
 def _stream_us(M: int, N: int, K: int):
@@ -674,7 +683,7 @@ def _stream_us(M: int, N: int, K: int):
     for t, (bm, bn, fill, step, again, reduce, part, load) in _ROW_TILES.items():
         tiles = math.ceil(M / bm) * math.ceil(N / bn)
         for s in (1, 2, 4, 8):
-            if s > 1 and (N >= 8192 or ksteps % s or ksteps // s < 4 or tiles * s > 520 or s > most):
+            if s > 1 and (N >= 8192 or M >= ROW_TILES_BELOW or ksteps % s or ksteps // s < 4 or tiles * s > 520 or s > most):
                 continue
             rounds, nk = math.ceil(tiles * s / 256), ksteps // s
             us = fill + rounds * nk * step + (rounds - 1) * again + tiles * s * nk * load / 256
@@ -694,14 +703,15 @@ def _phase_us(M: int, N: int, K: int, epi: int, tile: int) -> float:
 
 @_rule
 def _row_tile(M: int, N: int, K: int, epi: int = EPI_NONE, f16: bool = False):
-    """(tile, splits) of a product of 65 rows to ROW_TILES_BELOW: the fastest by estimate (``_ROW_TILES``). From 640 rows on
+    """(tile, splits) of a product of 65 rows to ROW_TILES_BELOW, and of more with a small result (``_row_tiles_ok``): the fastest
+    by estimate (``_ROW_TILES``). From 640 rows on
     the phase-split kernel picks its own row height, and keeps what is within 3 %. Below, bf16 residuals are added to the
     fp32 sums only (that kernel rounds the product first)."""
     us, tile, splits = _stream_us(M, N, K)
     if K < 128 or (epi == EPI_RESID and M < 640 and not f16):
         return tile, splits
     phase = min((_phase_us(M, N, K, epi, t), t) for t in _PHASE_TILES)
-    if us < phase[0] * (0.97 if M >= 640 else 1):
+    if us * (1.1 if M >= ROW_TILES_BELOW else 1) < phase[0] * (0.97 if M >= 640 else 1):
         return tile, splits
     return (0 if M >= 640 else phase[1]), 1
 
@@ -1374,7 +1384,7 @@ def gemm_f16(a, w, bias=None, epi: int = EPI_NONE, resid=None, out=None) -> torc
         out = torch.empty((M, N), dtype=torch.float16, device=a.device)
     _req(out.dtype == torch.float16 and out.shape == (M, N) and out.stride(1) == 1 and out.stride(0) % 8 == 0, "out")
     stream = torch.cuda.current_stream().cuda_stream
-    tile, splits = _row_tile(M, N, K, epi, True) if M < ROW_TILES_BELOW and max(K, a.stride(0)) < 1 << 22 else (0, 1)
+    tile, splits = _row_tile(M, N, K, epi, True) if _row_tiles_ok(M, N) and max(K, a.stride(0)) < 1 << 22 else (0, 1)
     ws = _call_partials(splits, M, N, a.device)
     tail = _gemm_tail(a.device, stream, M, N, K, epi, tile) if tile in (7, 10) or (tile == 0 and M >= 256) else (None, None)
     _check(lib().da_gemm_f16(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,

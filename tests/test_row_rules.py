@@ -25,3 +25,14 @@ def test_splits(M, N, Kd):
         assert splits == 1 or splits * M * N * 4 <= (32 if M < 256 else 20) << 20
         # a bf16 residual is added to the fp32 sums below 640 rows
         assert f16 or M >= 640 or tile in K._ROW_TILES
+
+
+@pytest.mark.parametrize("M,N,Kd,want", [(1300, 1024, 1024, 15), (2000, 1024, 1024, 15), (2600, 1024, 1024, 0), (1600, 768, 3072, 15),
+                                         (3500, 384, 1536, 15), (1600, 4096, 1024, 0), (5000, 768, 768, 0), (1300, 4096, 4096, 18)])
+def test_small_results_of_many_rows(M, N, Kd, want):
+    assert K._row_tiles_ok(M, N) or want == 0
+    assert not K._row_tiles_ok(M, N) or K._row_tile(M, N, Kd, K.EPI_RESID) == (want, 1)
+
+
+def test_large_results_of_many_rows():
+    assert K._row_tiles_ok(1279, 28672) and not K._row_tiles_ok(1280, 28672) and not K._row_tiles_ok(5121, 384)
