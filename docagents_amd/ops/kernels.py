@@ -181,8 +181,14 @@ def _ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
+def _raw_stream() -> int:
+    """The calling thread's current stream on its current device. (torch.cuda.current_stream() builds a stream object around the
+    same number: 2.8 us of the 8 that a launch took the host; this takes 0.2.)"""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(_raw_stream())
 
 
 def _check(rc: int, name: str):
@@ -349,7 +355,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
             splits = _auto_splits(M, N, K) if tile in (0, 2, 3) or (tile == 9 and M <= 128) else 1
     if splits > 1 and ws is None:
         ws = _workspace(splits * M * N * 4, a.device)
-    stream = torch.cuda.current_stream().cuda_stream
+    stream = _raw_stream()
     # (gemm8p's rows and tiles)
     tail = _gemm_tail(a.device, stream, M, N, K, epi, tile) if tile in (4, 7, 10) or (tile == 0 and M >= 640) else (None, None)
     rc = lib().da_gemm_bf16(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
@@ -1383,7 +1389,7 @@ def gemm_f16(a, w, bias=None, epi: int = EPI_NONE, resid=None, out=None) -> torc
     if out is None:
         out = torch.empty((M, N), dtype=torch.float16, device=a.device)
     _req(out.dtype == torch.float16 and out.shape == (M, N) and out.stride(1) == 1 and out.stride(0) % 8 == 0, "out")
-    stream = torch.cuda.current_stream().cuda_stream
+    stream = _raw_stream()
     tile, splits = _row_tile(M, N, K, epi, True) if _row_tiles_ok(M, N) and max(K, a.stride(0)) < 1 << 22 else (0, 1)
     ws = _call_partials(splits, M, N, a.device)
     tail = _gemm_tail(a.device, stream, M, N, K, epi, tile) if tile in (7, 10) or (tile == 0 and M >= 256) else (None, None)
