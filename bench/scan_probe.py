@@ -34,7 +34,7 @@ def main():
         base = max(64, math.ceil(N / (256 * 16) / 16) * 16)
         for thr in (-1.0, 0.95):
             for rpw in (base, base * 4):
-                ws = K._workspace(int(lib.da_topk_stream_ws(N, q, rpw)), dev)
+                ws = K._workspace(int(lib.da_topk_stream_ws(N, q, a.k, rpw)), dev)
                 out_s = torch.empty((q, a.k), dtype=torch.float32, device=dev)
                 out_i = torch.empty((q, a.k), dtype=torch.int32, device=dev)
 

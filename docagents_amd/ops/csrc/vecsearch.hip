@@ -131,9 +131,9 @@ topk_dense_kernel(const bf16_t* __restrict__ X, int N, int d, const int* __restr
 //     instructions, and orders the rows.
 // A top-K list kept beside the scan starts empty in every workgroup, so with a few hundred to a few thousand rows each nearly
 // every tile held a row that beat the list so far: appending, cutting and merging took 20 - 85 % of a pass. Whole searches, us,
-// lists / groups: 1.25 M x 1024, K = 5, 1 query 506 / 395, 16 600 / 417, 64 708 / 443, 128 795 / 496; 411812 x 768, 113
-// queries, K = 5 309 / 148, K = 20 518 / 161; 75595 x 384, 36 queries, K = 19 159 / 33; 30000 x 1024, 20 queries 69 / 29;
-// 512 x 768 (centroids), 24 queries 27 / 19.
+// lists / groups (few rows: scores, see scan_plan): 1.25 M x 1024, K = 5, 1 query 506 / 395, 16 600 / 417, 64 708 / 443, 128
+// 795 / 496; 411812 x 768, 113 queries, K = 5 309 / 148, K = 20 518 / 161; 75595 x 384, 36 queries, K = 19 159 / 33; 30000 x
+// 1024, 20 queries 69 / 29; 512 x 768 (centroids), 24 queries 27 / 12.
 __device__ __forceinline__ unsigned td_key(float v, int id) {  // larger = better; empty (id < 0) = 0
   const unsigned u = __float_as_uint(v + 0.f);  // (-0 as 0)
   return id < 0 ? 0u : ((u & 0x80000000u) ? ~u : (u | 0x80000000u));
@@ -194,7 +194,8 @@ __device__ __forceinline__ float td_cut(float v, int id, int K, int lane, float*
 
 
 // What a scan leaves of a run of 16-row tiles for a wave's 16 queries: lane (fr, fg) of query fr keeps groups 4 fg .. 4 fg + 3
-// of every 16 and stores them together. A run's groups are padded to a multiple of 4 with -inf.
+// of every 16 and stores them together. A run's groups are padded to a multiple of 4 with -inf. lg < 0: its rows' scores
+// instead, padded to whole tiles.
 struct GroupMax {
   float* line;  // this lane's query's groups of this run; null: no such query
   int slots, lg, g;  // groups of a run (padded), log2 of a group's tiles, groups so far
@@ -221,18 +222,28 @@ struct GroupMax {
   // are sl (removed rows: -1); rows from `end` on are padding
   __device__ __forceinline__ void tile(const f32x4_t& acc, int t, int row0, int end, float thr, const int (&sl)[4],
                                        const unsigned* __restrict__ bits, int W, int fg) {
-    float m = -INFINITY;
+    f32x4_t s;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       bool ok = row0 + i < end && sl[i] >= 0 && acc[i] >= thr;
       if (bits && ok) ok = (sl[i] >> 5) < W && ((bits[sl[i] >> 5] >> (sl[i] & 31)) & 1u);
-      m = fmaxf(m, ok ? acc[i] : -INFINITY);
+      s[i] = ok ? acc[i] : -INFINITY;
     }
+    if (lg < 0) {  // every row's score
+      if (line) *(f32x4_t*)(line + t * 16 + 4 * fg) = s;
+      return;
+    }
+    const float m = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
     const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
     best = fmaxf(best, max_xhalf(fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]))));
     if (((t + 1) & ((1 << lg) - 1)) == 0) close(fg);
   }
   __device__ __forceinline__ void finish(int tiles, int fg) {
+    if (lg < 0) {
+      for (int t = tiles; t * 16 < slots; ++t)
+        if (line) *(f32x4_t*)(line + t * 16 + 4 * fg) = keep;
+      return;
+    }
     if (tiles & ((1 << lg) - 1)) close(fg);
     for (int at = g & ~15; at < slots; at += 16) flush(at, fg);
   }
@@ -743,12 +754,19 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
   if (wid == 0) {
     if (over) top_join(top, cs, ci, TP_WAVES);
     else fold(found);
+    if (lg < 0) {  // these are the rows
+      if (lane < K && ci[0][lane] >= 0) ci[0][lane] = ci[0][lane] / run_slots * run_rows + ci[0][lane] % run_slots;
+      wave_sync_lds();
+      top_order(top, os + (size_t)q * K, oi + (size_t)q * K);
+      return;
+    }
     if (lane < K) groups[lane] = ci[0][lane];
     float low = lane < K && ci[0][lane] >= 0 ? cs[0][lane] : lane < K ? -INFINITY : INFINITY;  // the K-th best group
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) low = fminf(low, __shfl_xor(low, o, 64));
     if (lane == 0) { bound = low; count = 0; }
   }
+  if (lg < 0) return;
   __syncthreads();
 
   // ---- their rows ----
@@ -844,7 +862,7 @@ DA_EXPORT int da_topk_dense(const void* X, int N, int d, const void* slots, cons
 // The streaming scan (d = 384, 768 or 1024). hipErrorInvalidValue for shapes it does not take (the caller then uses
 // da_topk_dense). Its runs of rows, and their groups in ws: Q lines of `groups` floats.
 struct ScanPlan {
-  int runs, run_rows, run_slots, lg;  // run_slots: a run's groups, padded to 4
+  int runs, run_rows, run_slots, lg;  // run_slots: a run's groups, padded to 4; lg < 0: its rows, padded to 16
   long groups() const { return (long)runs * run_slots; }
 };
 
@@ -852,20 +870,24 @@ struct ScanPlan {
 // offsets), and as many as one round of resident workgroups needs: a second round starts its pipelines anew, us with 1024
 // waves / 4096: 100000 x 1024, 16 queries, 48.7 / 56.3; 411812 x 768 113.6 / 121.0; 1250000 x 1024 417 / 419.
 // A group is a tile up to 65536 groups, so that the pick reads 256 KB a query at most, and 2, 4, .. tiles from there on.
-static ScanPlan scan_plan(long N, int Q, int rows_per_wave) {
+// Up to 10000 + 1500 K rows each row's score is left, and nothing is scored again: more to write and to read for fewer steps of
+// the pick, a wave's tile of a group each. us, groups / scores: 464 x 1024, K = 24, 2 queries 36 / 14; 512 x 768, K = 8, 24
+// queries 19 / 12; 10000 x 1024, 24 queries, K = 5 25 / 21, K = 20 39 / 22; 20000 x 768, 128 queries 29 / 33 and 41 / 34;
+// 30000 x 1024, 20 queries 29 / 31 and 45 / 32; 60000 x 384, 128 queries 32 / 47 and 40 / 48.
+static ScanPlan scan_plan(long N, int Q, int K, int rows_per_wave) {
   const long runs = Q <= 16 ? 1024 : Q <= 64 ? 512 : 256;
   ScanPlan p;
   p.run_rows = (int)min(524288L, max(Q <= 16 ? (rows_per_wave + 15L) / 16 * 16 : 16L, (N + runs * 16 - 1) / (runs * 16) * 16));
   p.runs = (int)((N + p.run_rows - 1) / p.run_rows);
-  p.lg = 0;
-  while ((N >> (4 + p.lg)) > 65536) ++p.lg;
+  p.lg = N <= 10000 + 1500L * K ? -1 : 0;
+  while (p.lg >= 0 && (N >> (4 + p.lg)) > 65536) ++p.lg;
   const int tiles = p.run_rows / 16 + 1;  // (32-row stages: one tile past the end)
-  p.run_slots = ((tiles + (1 << p.lg) - 1 >> p.lg) + 3) & ~3;
+  p.run_slots = p.lg < 0 ? tiles * 16 : ((tiles + (1 << p.lg) - 1 >> p.lg) + 3) & ~3;
   return p;
 }
 
-DA_EXPORT size_t da_topk_stream_ws(int N, int Q, int rows_per_wave) {
-  return (size_t)scan_plan(N, Q, rows_per_wave).groups() * Q * 4;
+DA_EXPORT size_t da_topk_stream_ws(int N, int Q, int K, int rows_per_wave) {
+  return (size_t)scan_plan(N, Q, K, rows_per_wave).groups() * Q * 4;
 }
 
 DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slots, const void* Qv, int Q,
@@ -875,7 +897,7 @@ DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slot
     return (int)hipErrorInvalidValue;
   if (Q == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  const ScanPlan p = scan_plan(N, Q, rows_per_wave);
+  const ScanPlan p = scan_plan(N, Q, K, rows_per_wave);
   const int nw = Q > 64 ? 8 : 4, nqg = (Q + 16 * nw - 1) / (16 * nw);
   const long blocks = Q <= 16 ? (p.runs + 3) / 4 : (long)(p.runs + 7) / 8 * 8 * nqg;
   if (p.groups() > 0x7fffffffL || blocks > 0x7fffffffL) return (int)hipErrorInvalidValue;

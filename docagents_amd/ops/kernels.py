@@ -103,7 +103,7 @@ _SIGS = {
     "da_bert_embed_ln_f16": [c_void_p] * 9 + [c_int, c_int, c_float, c_void_p],
     "da_pool_l2norm_f16": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
     "da_topk_dense_ws": [c_int] * 4,
-    "da_topk_stream_ws": [c_int] * 3,
+    "da_topk_stream_ws": [c_int] * 4,
 }
 # the library part (build.py) of each launcher that is not in "kernels"; da_gemm* are in "gemm"
 _PART_OF = {n: "token" for n in (
@@ -1234,7 +1234,7 @@ def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_bloc
         # the streaming scan (search-sized batches over a big shard; k-means assignment, with the
         # rows as the queries, keeps the query-major tiles below)
         rpw = _scan_rows(N)
-        ws = _workspace(int(lib().da_topk_stream_ws(N, Q, rpw)), X.device)
+        ws = _workspace(int(lib().da_topk_stream_ws(N, Q, K, rpw)), X.device)
         out_s = torch.empty((Q, K), dtype=torch.float32, device=X.device)
         out_i = torch.empty((Q, K), dtype=torch.int32, device=X.device)
         _check(lib().da_topk_dense_stream(_ptr(X), N, d, _ptr(slots), _ptr(Qv), Q, _ptr(bitmap), W, float(thr), K,
