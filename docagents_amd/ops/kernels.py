@@ -289,9 +289,16 @@ def _gemm_tail(device, stream: int, M: int, N: int, K: int, epi: int, tile: int 
     return part, cnt
 
 
+def _call_scratch(nbytes: int, device) -> torch.Tensor:
+    """Scratch as the call's own, from the caching allocator (a capture's: from its graph's pool). The workspace of a role is
+    one stream's, and one that grows drops the buffer that captured decode steps still write to: what may outgrow what a
+    generator reserved (the scores or group maxima of a search, up to 67 MB) must not come from there."""
+    return torch.empty(nbytes, dtype=torch.uint8, device=device)
+
+
 def _call_partials(splits: int, M: int, N: int, device):
-    """A product's K-split partials as the call's own (the workspace of a role is one stream's): None if whole."""
-    return torch.empty(splits * M * N, dtype=torch.float32, device=device) if splits > 1 else None
+    """A product's K-split partials as the call's own: None if whole."""
+    return _call_scratch(splits * M * N * 4, device) if splits > 1 else None
 
 
 def gemv_fusable(M: int, N: int, K: int, epi: int = EPI_NONE) -> bool:
@@ -1234,7 +1241,7 @@ def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_bloc
         # the streaming scan (search-sized batches over a big shard; k-means assignment, with the
         # rows as the queries, keeps the query-major tiles below)
         rpw = _scan_rows(N)
-        ws = _workspace(int(lib().da_topk_stream_ws(N, Q, K, rpw)), X.device)
+        ws = _call_scratch(int(lib().da_topk_stream_ws(N, Q, K, rpw)), X.device)
         out_s = torch.empty((Q, K), dtype=torch.float32, device=X.device)
         out_i = torch.empty((Q, K), dtype=torch.int32, device=X.device)
         _check(lib().da_topk_dense_stream(_ptr(X), N, d, _ptr(slots), _ptr(Qv), Q, _ptr(bitmap), W, float(thr), K,
@@ -1245,7 +1252,7 @@ def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_bloc
         nblk = max(1, min(math.ceil(N / 256), max(1, 1024 // qt)))
         rows_per_block = max(64, math.ceil(math.ceil(N / nblk) / 64) * 64)
     nblk = max(1, math.ceil(N / rows_per_block))
-    ws = _workspace(nblk * Q * K * 8, X.device)
+    ws = _call_scratch(nblk * Q * K * 8, X.device)
     out_s = torch.empty((Q, K), dtype=torch.float32, device=X.device)
     out_i = torch.empty((Q, K), dtype=torch.int32, device=X.device)
     _check(lib().da_topk_dense(_ptr(X), N, d, _ptr(slots), _ptr(Qv), Q, _ptr(bitmap), W, float(thr), K,
@@ -1299,7 +1306,7 @@ def _ranges(X, Qv, ranges, range_off, lists, K, thr, max_rows, slots, bitmap, ro
     if Q == 0:
         return out_s, out_i
     splits = max(1, math.ceil(max_rows / rows_per_split))
-    ws = _workspace(splits * Q * K * 8, X.device)
+    ws = _call_scratch(splits * Q * K * 8, X.device)
     _check(lib().da_topk_ranges(_ptr(X), d, _ptr(slots), _ptr(Qv), Q, _ptr(ranges), _ptr(range_off), _ptr(lists),
                                 0 if lists is None else lists.shape[1], _ptr(bitmap),
                                 W, float(thr), K, splits, rows_per_split, _ptr(ws), _ptr(out_s), _ptr(out_i),

@@ -40,7 +40,7 @@ GB = 1e9
 HBM_BYTES = 288 * GB
 PLAN_LIMIT_BYTES = 270 * GB  # what a phase may hold: the rest is the runtime, RCCL and fragmentation
 MAX_PREFILL_TOKENS = 65536   # Generator.max_prefill_tokens default
-RUNTIME_BYTES = 2 * GB       # graph pools, tables, small buffers, allocator rounding (every phase)
+RUNTIME_BYTES = 2 * GB       # graph pools, tables, searches' scratch (67 MB a stream), small buffers, allocator rounding (every phase)
 TAIL_BYTES = 256 * 256 * 256 * 4 + 8192  # 256 workgroups' fp32 partials and their tiles' counters
 TAIL_LANES = 4               # streams that run prefill products
 TP70B_BATCHES = (1, 16)      # tp_decode_70b: decode batches timed

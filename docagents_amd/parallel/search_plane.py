@@ -632,8 +632,8 @@ class SearchPlane:
         stream_ctx = torch.cuda.stream(self.stream) if self.stream is not None else _nullctx()
         ws_ctx = _nullctx()
         if dev.type == "cuda":
-            # the scan kernels' scratch must not be the GPU thread's: its decode graph captured that
-            # workspace's pointer and runs concurrently with this thread (ops/kernels.py workspace_role)
+            # a workspace that this thread's kernels use must not be the GPU thread's: its decode graph captured that
+            # one's pointer and runs concurrently with this thread (ops/kernels.py workspace_role)
             from ..ops.kernels import workspace_role
             ws_ctx = workspace_role("search")
         with stream_ctx, ws_ctx:
