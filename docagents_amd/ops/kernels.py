@@ -534,7 +534,10 @@ def gemm_rope(a, w, pos, cos_sin, H: int, Hkv: int, D: int, slot, k_cache, v_cac
     _req(k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.shape == v_cache.shape
          and k_cache.dim() == 4 and k_cache.shape[1] == Hkv and k_cache.shape[3] == D, "caches")
     plain = K % 64 == 0 and K >= 128 and a.stride(1) == 1 and a.stride(0) % 8 == 0 and w.is_contiguous()
-    if M < 256 or not plain or (a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and _rope_apart(M, N, K)):
+    # (what gemm and rope_cache refuse and the one kernel takes stays with that)
+    apart = (a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and a.stride(0) >= K and cos_sin.shape[-1] == 2
+             and (out is None or out.is_contiguous()) and M >= 256 and _rope_apart(M, N, K))
+    if M < 256 or not plain or apart:
         qkv = gemm(a, w, out=out)
         return rope_cache(qkv, pos, cos_sin, H, Hkv, D, slot=slot, k_cache=k_cache, v_cache=v_cache)
     if out is None:

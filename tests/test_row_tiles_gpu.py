@@ -83,8 +83,9 @@ def test_as_the_rule_has_them(M, N, Kd, dtype):
     assert all(torch.equal(o, got) for o in outs)
 
 
-@pytest.mark.parametrize("M,apart", [(432, True), (1280, False)])
-def test_qkv_projection_either_way(M, apart):
+# (wide: into columns of a wider buffer, which the rotation behind a product does not take)
+@pytest.mark.parametrize("M,apart,wide", [(432, True, False), (1280, False, False), (432, True, True)])
+def test_qkv_projection_either_way(M, apart, wide):
     H, Hkv, D, Kd = 32, 8, 128, 4096
     N = (H + 2 * Hkv) * D
     assert K._rope_apart(M, N, Kd) == apart
@@ -96,7 +97,9 @@ def test_qkv_projection_either_way(M, apart):
     ang = pos.double()[:, None] * 10000.0 ** (-torch.arange(0, D, 2, device="cuda").double() / D)
     cs = torch.stack([ang.cos(), ang.sin()], -1).float().contiguous()
     kc, vc = (torch.zeros(2, Hkv, M, D, device="cuda", dtype=torch.bfloat16) for _ in range(2))
-    got = K.gemm_rope(a, w, pos, cs, H, Hkv, D, slot, kc, vc)
+    buf = torch.full((M, N + 64), 7.0, device="cuda", dtype=torch.bfloat16)
+    got = K.gemm_rope(a, w, pos, cs, H, Hkv, D, slot, kc, vc, out=buf[:, :N] if wide else None)
+    assert (buf[:, N:] == 7).all() and (not wide or got.data_ptr() == buf.data_ptr())
     x = (a.double() @ w.double().T).view(M, H + 2 * Hkv, D)
     c, s = ang.cos()[:, None], ang.sin()[:, None]
     turned = torch.stack([x[..., 0::2] * c - x[..., 1::2] * s, x[..., 1::2] * c + x[..., 0::2] * s], -1).flatten(-2)
