@@ -550,7 +550,7 @@ flash_attn_enc_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k
       mx = max_xhalf(mx);
       if (__any((mx - m_run) * c > SPEC_TAU)) {  // (weights of up to 2^SPEC_TAU are as exact)
         const float m_new = fmaxf(m_run, mx);
-        const float alpha = exp2f((m_run - m_new) * c);
+        const float alpha = exp2f((m_run - (m_new == -INFINITY ? 0.f : m_new)) * c);  // (scores of -inf only: 0, not NaN)
         m_run = m_new;
         l_part *= alpha;
 #pragma unroll

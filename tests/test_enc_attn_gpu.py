@@ -37,3 +37,20 @@ def test_rows(dtype, H, Hkv, lens, rising):
         err = (got[a:a + n].double().view(n, H, D).transpose(0, 1) - want).abs()
         # weights and the result are rounded to the type (half an ulp each); fp16 weights below 2^-14 of the row's scale to 2^-25
         assert (err <= ulp * (mag + want.abs()) / 2 * 1.01 + 2.0 ** -13).all()
+
+
+def test_infinite_scores():
+    """A query whose first 64 scores are -inf in fp32, beside ordinary ones of its wave."""
+    D, H, T = 64, 2, 150
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v = (torch.randn(T, H * D, device="cuda", generator=g) for _ in range(3))
+    q[:, 0], k[:, 0] = 0, 0
+    q[5, 0], k[:64, 0] = 2.0 ** 100, -(2.0 ** 100)
+    q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+    cu = torch.tensor([0, T], device="cuda", dtype=torch.int32)
+    got = K.flash_attn_varlen(q, k, v, cu, T, H, H, D, False).double().view(T, H, D).transpose(0, 1)
+    r = lambda t: t.double().view(T, H, D).transpose(0, 1)  # noqa: E731
+    p = torch.softmax(r(q) @ r(k).transpose(1, 2) * D ** -0.5, -1)
+    want, mag = p @ r(v), p @ r(v).abs()
+    # weights and the result are rounded to the type
+    assert ((got - want).abs() <= 2.0 ** -8 * (mag + want.abs()) * 1.01 + 2.0 ** -13).all()
