@@ -1915,7 +1915,9 @@ decode_attn_mfma1_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __
 #pragma unroll
     for (int ww = 0; ww < 4; ++ww) {
       const float f = exp2f(swm[ww] - Mu);
-      o += (so[(ww * 3) * D + d] + (so[(ww * 3 + 1) * D + d] + so[(ww * 3 + 2) * D + d])) * f;
+      // (an infinite value: the upper bits' sum has it, the others' may be 0 times it, NaN)
+      const float up = so[(ww * 3) * D + d], low = so[(ww * 3 + 1) * D + d] + so[(ww * 3 + 2) * D + d];
+      o += (fabsf(up) < INFINITY ? up + low : up) * f;
       ls += swl[ww] * f;
     }
     if (own_new) {  // the new token's key: weight exp2(s - M), value straight from the qkv row

@@ -48,3 +48,18 @@ def test_rows(B, H, D, S, kind, rope, prefix):
         # weights, are off by some 2^-19 in fp32, and the values are up to 6
         assert ((got[b].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -15).all(), b
     assert torch.equal(K.decode_attn(q, kc, vc, to(lens), to(slot), H, H, D, S, pre=pre, rope=rp), got)
+
+
+@pytest.mark.parametrize("B", [1, 8])
+def test_infinite_value(B):
+    """An infinite value under a weight that is not 0 makes its column infinite, whatever the weight's lower bits are."""
+    H, D, S = 32, 96, 256
+    g = torch.Generator(device="cuda").manual_seed(B)
+    kc, vc = (torch.randn(B, H, S, D, device="cuda", generator=g).bfloat16() for _ in range(2))
+    vc[:, :, 7, 3] = float("inf")
+    vc[:, :, 9, 4] = float("-inf")
+    q = torch.randn(B, H * D, device="cuda", generator=g).bfloat16()
+    lens, slot = torch.full((B,), 200, dtype=torch.int32, device="cuda"), torch.arange(B, dtype=torch.int32, device="cuda")
+    got = K.decode_attn(q, kc, vc, lens, slot, H, H, D, S).view(B, H, D)
+    assert (got[..., 3] == float("inf")).all() and (got[..., 4] == float("-inf")).all()
+    assert got[..., :3].isfinite().all() and got[..., 5:].isfinite().all()
