@@ -471,16 +471,19 @@ __global__ void pool_l2norm_kernel(const bf16_t* __restrict__ h, const int* __re
   }
 }
 
-// The mean of rows of up to 2048 columns: 1024 threads, as many rows at once as that holds (of 1024 columns 8, four of each
-// on their way together), their sums meet in LDS. Bound by latency: a thread per 8 columns that walks the rows alone took 123 us
-// for three texts of 285 - 512 rows x 1024, this 14 (two of 18 - 46 x 768 12, this 4).
-template <typename T>
+// The mean of rows of up to 2048 columns: as many rows at once as the workgroup's threads hold (1024 of them 8 rows of 1024
+// columns), four of each on their way together, whose sums meet in LDS. Bound by latency: a thread per 8 columns that walks the
+// rows alone took 123 us for three texts of 285 - 512 rows x 1024, this 14 (two of 18 - 46 x 768 12, this 4).
+// NT: threads where they and LDS are constants (64 texts of 512 rows x 1024 16.6 us; LDS sized at the launch 19.4), or 0.
+template <typename T, int NT>
 __global__ void __launch_bounds__(1024)
 pool_mean_kernel(const bf16_t* __restrict__ h, const int* __restrict__ cu_seqlens, int D, float* __restrict__ out32,
                  bf16_t* __restrict__ out16) {
   __shared__ float red[16];
-  __shared__ __attribute__((aligned(16))) float part[1024 * 8];
-  const int b = blockIdx.x, nch = D / 8, G = 1024 / nch, g = threadIdx.x / nch, c = threadIdx.x % nch;
+  extern __shared__ __attribute__((aligned(16))) float dyn[];
+  __shared__ __attribute__((aligned(16))) float fixed[NT ? NT * 8 : 1];
+  float* part = NT ? fixed : dyn;  // 8 a thread
+  const int b = blockIdx.x, nch = D / 8, G = (NT ? NT : (int)blockDim.x) / nch, g = threadIdx.x / nch, c = threadIdx.x % nch;
   const int s0 = cu_seqlens[b], n = cu_seqlens[b + 1] - s0, last = max(n - 1, 0);  // (an empty text: row s0)
   float v[8] = {};
   if (g < G)
@@ -657,21 +660,38 @@ DA_EXPORT int da_embed(const void* ids, const void* table, void* y, int T, int D
   DA_LAUNCH_CHECK();
 }
 
+// Threads of a text: 1024 while one round of workgroups has every text; of more texts, what the mean length takes at four rows
+// a thread. us, a thread per 8 columns that walks the rows / 1024 threads / this: 2000 texts of 12 rows x 384 5.9 / 13.8 / 5.1,
+// 5000 of 3 6.1 / 28.9 / 6.0, 20000 of 1 x 768 20.5 / 98 / 19, 1000 of 40 x 384 16.4 / 10.0 / 6.4, 600 of 300 98 / 25 / 25.
+static int pool_threads(int B, int D, int rows) {
+  const int nch = D / 8;
+  if (B <= 512) return 1024;
+  const int g = max(1, min((rows / B + 3) / 4, 1024 / nch));
+  return g == 1024 / nch ? 1024 : (g * nch + 63) / 64 * 64;
+}
+
 template <typename T>
-static int launch_pool(const void* h, const void* cu_seqlens, int B, int D, int mode, void* out32, void* out16, hipStream_t s) {
-  if (mode && D <= 2048)
-    pool_mean_kernel<T><<<B, 1024, 0, s>>>((const bf16_t*)h, (const int*)cu_seqlens, D, (float*)out32, (bf16_t*)out16);
-  else
+static int launch_pool(const void* h, const void* cu_seqlens, int B, int D, int mode, int rows, void* out32, void* out16,
+                       hipStream_t s) {
+  if (mode && D <= 2048) {
+    const int nt = pool_threads(B, D, rows);
+#define POOL(N) \
+  pool_mean_kernel<T, N><<<B, nt, N ? 0 : nt * 32, s>>>((const bf16_t*)h, (const int*)cu_seqlens, D, (float*)out32, (bf16_t*)out16)
+    if (nt == 1024) POOL(1024); else POOL(0);
+#undef POOL
+  } else {
     pool_l2norm_kernel<T><<<B, row_threads(D), 0, s>>>((const bf16_t*)h, (const int*)cu_seqlens, D, mode, (float*)out32,
                                                        (bf16_t*)out16);
+  }
   DA_LAUNCH_CHECK();
 }
 
-DA_EXPORT int da_pool_l2norm(const void* h, const void* cu_seqlens, int B, int D, int mode, void* out32,
+// rows: of h (the texts' mean length).
+DA_EXPORT int da_pool_l2norm(const void* h, const void* cu_seqlens, int B, int D, int mode, int rows, void* out32,
                              void* out16, void* stream) {
   if (!d_ok(D)) return (int)hipErrorInvalidValue;
   if (B == 0) return 0;
-  return launch_pool<BF16T>(h, cu_seqlens, B, D, mode, out32, out16, (hipStream_t)stream);
+  return launch_pool<BF16T>(h, cu_seqlens, B, D, mode, rows, out32, out16, (hipStream_t)stream);
 }
 
 DA_EXPORT int da_quant_fp8_rows(const void* x, int ldx, int M, int K, void* out, int ldo, void* scale, void* stream) {
@@ -695,11 +715,11 @@ DA_EXPORT int da_bert_embed_ln_f16(const void* ids, const void* positions, const
   return launch_bert_ln<F16T>(ids, positions, types, word, pos, type, g, b, y, nullptr, nullptr, T, D, eps, stream);
 }
 
-DA_EXPORT int da_pool_l2norm_f16(const void* h, const void* cu_seqlens, int B, int D, int mode, void* out32,
+DA_EXPORT int da_pool_l2norm_f16(const void* h, const void* cu_seqlens, int B, int D, int mode, int rows, void* out32,
                                  void* out16, void* stream) {
   if (!d_ok(D)) return (int)hipErrorInvalidValue;
   if (B == 0) return 0;
-  return launch_pool<F16T>(h, cu_seqlens, B, D, mode, out32, out16, (hipStream_t)stream);
+  return launch_pool<F16T>(h, cu_seqlens, B, D, mode, rows, out32, out16, (hipStream_t)stream);
 }
 
 // LayerNorm / BERT embeddings + LayerNorm with an additional fused fp8 (e4m3, per-row scale) output.

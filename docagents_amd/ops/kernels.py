@@ -53,7 +53,7 @@ _SIGS = {
     "da_layernorm": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
     "da_bert_embed_ln": [c_void_p] * 9 + [c_int, c_int, c_float, c_void_p],
     "da_embed": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
-    "da_pool_l2norm": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
+    "da_pool_l2norm": [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
     "da_rope_cache": [c_void_p] * 6 + [c_int] * 6 + [c_void_p],
     "da_sample": [c_void_p, c_int, c_int, c_int, c_float, c_uint, c_uint] + [c_void_p] * 9
                  + [c_int] * 6 + [c_void_p],
@@ -101,7 +101,7 @@ _SIGS = {
                           c_int, c_int, c_float, c_void_p, c_int, c_void_p],
     "da_layernorm_f16": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
     "da_bert_embed_ln_f16": [c_void_p] * 9 + [c_int, c_int, c_float, c_void_p],
-    "da_pool_l2norm_f16": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
+    "da_pool_l2norm_f16": [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
     "da_topk_dense_ws": [c_int] * 4,
     "da_topk_stream_ws": [c_int] * 4,
 }
@@ -851,7 +851,7 @@ def pool_l2norm(h, cu_seqlens, mode: int = 0, out32=None, out16=None):
     _req(h.is_contiguous(), "h contiguous")
     if out32 is None and out16 is None:
         out32 = torch.empty((B, D), dtype=torch.float32, device=h.device)
-    _check(lib().da_pool_l2norm(_ptr(h), _ptr(cu_seqlens), B, D, mode, _ptr(out32), _ptr(out16), _stream()),
+    _check(lib().da_pool_l2norm(_ptr(h), _ptr(cu_seqlens), B, D, mode, h.shape[0], _ptr(out32), _ptr(out16), _stream()),
            "pool_l2norm")
     return out32 if out32 is not None else out16
 
@@ -1461,7 +1461,7 @@ def pool_l2norm_f16(h, cu_seqlens, mode: int = 0, out32=None, out16=None):
         _bf16_cuda(out16, "out16")
     if out32 is None and out16 is None:
         out32 = torch.empty((B, D), dtype=torch.float32, device=h.device)
-    _check(lib().da_pool_l2norm_f16(_ptr(h), _ptr(cu_seqlens), B, D, mode, _ptr(out32), _ptr(out16), _stream()),
+    _check(lib().da_pool_l2norm_f16(_ptr(h), _ptr(cu_seqlens), B, D, mode, h.shape[0], _ptr(out32), _ptr(out16), _stream()),
            "pool_l2norm_f16")
     return out32 if out32 is not None else out16
 
