@@ -17,9 +17,12 @@
 // A and W fragments are in flight per wave (counted vmcnt waits: the ring is indexed by unrolled
 // slot, loads issued in k order).
 //
-// From K = 4096 on the tiles of an XCD begin at K chunks of their own: all at the same columns of rows a power of two apart,
-// they ask the same few channels at a time. 8192 x 4096, 4 / 16 / 32 rows: 16.7 / 16.9 / 18.3 -> 13.5 / 13.7 / 16.0 us, 6144 x 4096
-// 16.6 / 16.8 / 17.8 -> 13.7 / 14.2 / 17.5, 4096 x 14336 23.6 / 26.3 / 33.3 -> 22.4 / 25.1 / 33.1; a shorter K gains nothing.
+// Where K is a multiple of 2048 from 4096 on, the tiles of an XCD begin at K chunks of their own: all at the same columns of rows
+// a multiple of 4 KB apart, they ask the same few channels at a time. 8192 x 4096, 4 / 16 / 32 rows: 16.7 / 16.9 / 18.3 -> 13.5 /
+// 13.7 / 16.0 us, 6144 x 4096 16.6 / 16.8 / 17.8 -> 13.7 / 14.2 / 17.5, 4096 x 14336 23.6 / 26.3 / 33.3 -> 22.4 / 25.1 / 33.1. Time
+// with / without, 3072 - 5120 columns, 3 - 32 rows: K = 8192 0.80 - 0.98, 16384 0.76 - 0.96, 6144 0.94 - 1.00, 10240 and 12288 0.97 -
+// 1.00; of other K 4608 1.01 - 1.04, 5120 1.01 - 1.06, 6656 1.01 - 1.05, 7168 1.00 - 1.05, 13824 1.00 - 1.04 (11008 0.95 - 0.99); a
+// shorter K gains nothing.
 //
 // Deferred RMSNorm (NORM): the decode layer's norms ride here instead of in a reduce launch. The
 // producer of the residual stream (EPI_RESID) writes, next to x, per-(workgroup, row) sums of squares
@@ -67,7 +70,7 @@ gemm_dk_kernel(DkArgs p) {
   const int Mb = min(BM, p.M - m0);  // rows of this block
   const int nch = p.K / KC;
   const int kl = nch - 1;
-  const int rot = nch >= 16 ? (tile >> 3) % nch : 0;  // the chunk that this tile begins with
+  const int rot = nch >= 16 && nch % 8 == 0 ? (tile >> 3) % nch : 0;  // the chunk that this tile begins with
 
   // ---- global -> registers: whole 512-B row segments (32 lanes x 16 B per row), full lines ----
   u32x4_t rw[PF][LW], ra[PF][LA];

@@ -41,10 +41,10 @@ def test_wide(M, N, Kd, parts, epi, norm):
     assert ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 8 * (Kd + parts) * 2.0 ** -24 * mag).all()
 
 
-@pytest.mark.parametrize("N,Kd", [(4096, 4096), (6144, 4096 + 256), (1024, 14336)])
+@pytest.mark.parametrize("N,Kd", [(4096, 4096), (6144, 4096 + 256), (1024, 14336), (3072, 6144), (640, 5120)])
 @pytest.mark.parametrize("M", [3, 32, 40])
 def test_rotated_chunks(M, N, Kd):
-    """Narrow products from K = 4096 on: tiles begin at a chunk of their own."""
+    """Narrow products of K = 2048 n from 4096 on: tiles begin at a chunk of their own; of other K at the first."""
     g = torch.Generator(device="cuda").manual_seed(M + N)
     a = torch.randn(M, Kd, device="cuda", generator=g).bfloat16()
     w = (torch.randn(N, Kd, device="cuda", generator=g) * Kd ** -0.5).bfloat16()
