@@ -374,7 +374,7 @@ __global__ void __launch_bounds__(256) gemm_rows_kernel(AnyArgs p) {
   }
 }
 
-// fp32 operands, K a multiple of 32: the general kernel's products with operands by LDS-DMA in a ring of four 32-k stages (rows of
+// fp32 operands, K a multiple of 32 from 128 on: the general kernel's products with operands by LDS-DMA in a ring of four 32-k stages (rows of
 // 128 bytes, 16-byte chunk c of row r at c ^ (r >> 1): conflict-free), one barrier a stage, and K over as many workgroups as
 // fill the chip. 32 rows x 128 columns for up to 32 rows, else 64 x 64; a wave has 32 x 32 of them.
 // Bound by the weights' bytes up to some 40 rows, by v_mfma_f32_16x16x4_f32 (157 TF) from there on. The general kernel, a slice
@@ -517,9 +517,11 @@ __global__ void __launch_bounds__(256) gemm_f32_reduce_kernel(AnyArgs p, int spl
 
 // Workgroups along K of an fp32 product (0: the general kernel), each with 8 stages of K at least, by estimate in columns of K:
 // rounds of two workgroups a CU, a split's sums written and read, the second launch. (50 x 28672 x 4096, 448 tiles: whole 141
-// us, in two splits, 1.75 rounds, 146; 32 rows, 224 tiles: in two 90, in three 100.)
+// us, in two splits, 1.75 rounds, 146; 32 rows, 224 tiles: in two 90, in three 100.) From K = 128 on: gates of 8 blocks x 64,
+// general kernel / ring, 1 row 5.2 / 6.2 us, 32 5.6 / 6.6, 4000 13.9 / 15.6; 64 heads of 512 x 128, 1 row 9.0 / 7.6, 32 11.0 / 9.0,
+// 4000 555 / 583; 33 rows x 2560 x 160 8.9 / 8.1, 800 16.6 / 17.7.
 static int f32_splits(long M, long N, long K, int lda, int batch) {
-  if (K % 32 || K > 1 << 21 || lda > 1 << 21) return 0;
+  if (K % 32 || K < 128 || K > 1 << 21 || lda > 1 << 21) return 0;
   const long bm = M <= 32 ? 32 : 64, tiles = (M + bm - 1) / bm * ((N + 4096 / bm - 1) / (4096 / bm)) * batch;
   if (tiles > 0x7fffffffL / 64) return 0;
   long best = 1, least = 0x7fffffffffffffffL;
