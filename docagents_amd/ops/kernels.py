@@ -672,12 +672,13 @@ def _auto_splits(M: int, N: int, K: int) -> int:
 # Weight-streaming tiles of more than 64 rows (csrc/gemm.hip): code -> rows, columns, and what a product takes on them in us:
 # the first round's fill and drain, a K-step of 64 of a round, each further round, a reduce and its partials per million
 # values, and a unit's K-step on 1/256 of the chip (what all of them load). Phase-split kernel (csrc/gemm8p.hip): code ->
-# rows, fill, a K-step of 256 columns, the same on 1/256 of the chip. Fitted to 598 products of 65 - 1200 rows (projections,
-# feed-forwards and encoder layers 384 - 4096 wide, weights cold; a median of 5 % off): the choice takes 1.008 times the
-# fastest tile on average and at worst 1.2, and 0.81 times the rules before it (25 up to 1.1 times as long, near ties).
-_ROW_TILES = {14: (128, 128, 8.46, 0.38, -0.06, -0.22, 1.9, 0.14), 15: (128, 64, 5.96, 0.25, 0.83, 1.35, 1.96, 0.1),
+# rows, fill, a K-step of 256 columns, the same on 1/256 of the chip. Fitted, with no cost below zero, to 598 products of 65 -
+# 1200 rows (projections, feed-forwards and encoder layers 384 - 4096 wide, weights cold): off by 5 - 7 % on average, by up to 48
+# where all rows of a tile are real and K is 14336. The choice takes 1.008 times the fastest tile on average and at worst 1.2, and
+# 0.81 times the rules before it (12 products longer by more than 2 %, up to 1.11 times).
+_ROW_TILES = {14: (128, 128, 8.37, 0.38, 0.07, 0.0, 1.84, 0.14), 15: (128, 64, 5.96, 0.25, 0.83, 1.35, 1.96, 0.1),
               16: (64, 64, 5.82, 0.16, 1.66, 2.54, 1.26, 0.08), 17: (64, 128, 5.79, 0.26, 0.72, 1.61, 1.78, 0.13),
-              18: (192, 128, 11.58, 0.46, -0.59, -2.04, 1.81, 0.16)}
+              18: (192, 128, 10.64, 0.47, 0.7, 0.0, 1.45, 0.16)}
 _PHASE_TILES = {7: (256, 10.76, 0.67, 0.64), 10: (128, 7.11, 0.55, 0.37)}
 ROW_TILES_BELOW = 1280
 # From there on small results only, whole, and where the estimate, 10 % up (rows are a larger part of what tiles load), is still
@@ -704,7 +705,9 @@ def _stream_us(M: int, N: int, K: int):
             rounds, nk = math.ceil(tiles * s / 256), ksteps // s
             us = fill + rounds * nk * step + (rounds - 1) * again + tiles * s * nk * load / 256
             if s > 1:
-                us = 1.06 * (us + reduce + part * s * M * N * 1e-6)  # (a close call stays whole)
+                # (a close call stays whole; less so with full tiles of 128 rows, which whole K takes longer than estimated:
+                # 128 x 3072 x 3072 18.7 / 15.7 in four splits, 112 x 5120 x 5120 28.4 / 25.9; 80 x 2048 x 2048 10.2 / 10.6)
+                us = (1.03 if 96 < M <= 128 else 1.06) * (us + reduce + part * s * M * N * 1e-6)
             if best is None or us < best[0]:
                 best = us, t, s
     return best
@@ -718,27 +721,32 @@ def _phase_us(M: int, N: int, K: int, epi: int, tile: int) -> float:
 
 
 @_rule
-def _row_tile(M: int, N: int, K: int, epi: int = EPI_NONE, f16: bool = False):
-    """(tile, splits) of a product of 65 rows to ROW_TILES_BELOW, and of more with a small result (``_row_tiles_ok``): the fastest
-    by estimate (``_ROW_TILES``). From 640 rows on
-    the phase-split kernel picks its own row height, and keeps what is within 3 %. Below, bf16 residuals are added to the
-    fp32 sums only (that kernel rounds the product first)."""
+def _row_us(M: int, N: int, K: int, epi: int = EPI_NONE, f16: bool = False):
+    """(us, tile, splits) of a product of 65 rows to ROW_TILES_BELOW, and of more with a small result (``_row_tiles_ok``): the
+    fastest by estimate (``_ROW_TILES``). From 640 rows on the phase-split kernel picks its own row height, and keeps what is
+    within 3 %. Below, bf16 residuals are added to the fp32 sums only (that kernel rounds the product first)."""
     us, tile, splits = _stream_us(M, N, K)
     if K < 128 or (epi == EPI_RESID and M < 640 and not f16):
-        return tile, splits
+        return us, tile, splits
     phase = min((_phase_us(M, N, K, epi, t), t) for t in _PHASE_TILES)
     if us * (1.1 if M >= ROW_TILES_BELOW else 1) < phase[0] * (0.97 if M >= 640 else 1):
-        return tile, splits
-    return (0 if M >= 640 else phase[1]), 1
+        return us, tile, splits
+    return phase[0], (0 if M >= 640 else phase[1]), 1
+
+
+def _row_tile(M: int, N: int, K: int, epi: int = EPI_NONE, f16: bool = False):
+    """(tile, splits) of such a product."""
+    return _row_us(M, N, K, epi, f16)[1:]
 
 
 @_rule
 def _rope_apart(M: int, N: int, K: int) -> bool:
-    """A QKV projection of 256 rows and more as a weight-streaming product and rope_cache behind it (which reads and writes
-    the result once more; the rotation costs the phase-split kernel 4 us): 432 x 6144 x 4096 54 -> 39 us, 300 x 9216 x 3072 46 -> 34,
-    800 x 6144 x 4096 54 -> 50, where 128x256 tiles leave CUs idle."""
+    """A QKV projection of 256 rows and more as a product by itself, on the tile that it has then, and rope_cache behind it (which
+    reads and writes the result once more; the rotation costs the phase-split kernel 4 us): 432 x 6144 x 4096 54 -> 39 us, 300 x 9216
+    x 3072 46 -> 34, 800 x 6144 x 4096 54 -> 50, where 128x256 tiles leave CUs idle, and 1024 x 9216 x 3072 95 -> 69, 1200 x 10240 x
+    8192 212 -> 173, where the last round of a product without the rotation is shared out along K."""
     tiles = math.ceil(M / 256) * math.ceil(N / 256)
-    return M < ROW_TILES_BELOW and (_stream_us(M, N, K)[0] + 4 + M * N * 1e-6
+    return M < ROW_TILES_BELOW and (_row_us(M, N, K)[0] + 4 + M * N * 1e-6
                                     < 0.97 * (_phase_us(M, N, K, EPI_ROPE, 7 if tiles >= 256 else 10) + 4))
 
 

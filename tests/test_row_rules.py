@@ -36,3 +36,11 @@ def test_small_results_of_many_rows(M, N, Kd, want):
 
 def test_large_results_of_many_rows():
     assert K._row_tiles_ok(1279, 28672) and not K._row_tiles_ok(1280, 28672) and not K._row_tiles_ok(5121, 384)
+
+
+def test_estimate():
+    """No cost is negative; full tiles of 128 rows go into splits sooner; a projection is apart from its rotation where the product
+    alone has a shorter last round, also on the phase-split kernel."""
+    assert all(x >= 0 for t in (*K._ROW_TILES.values(), *K._PHASE_TILES.values()) for x in t)
+    assert K._row_tile(128, 3072, 3072) == (15, 4) and K._row_tile(80, 2048, 2048) == (16, 1)
+    assert K._row_tile(1024, 9216, 3072) == (0, 1) and K._rope_apart(1024, 9216, 3072) and not K._rope_apart(512, 9216, 3072)
