@@ -354,11 +354,12 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
         if tile == 0 and M > 64 and _row_tiles_ok(M, N) and max(K, a.stride(0)) < 1 << 22:
             tile, splits = _row_tile(M, N, K, epi)
             ws = _call_partials(splits, M, N, a.device)
-        elif tile == 0 and 128 < M < 640:
-            tile, splits = _mid_tile(M, N, K)
+        elif tile == 0 and 64 < M < 640:  # rows too long for the streaming tiles' offsets: the register-staged 64x128 tile
+            tile, splits = 11, _auto_splits(M, N, K)
+            ws = _call_partials(splits, M, N, a.device)
         else:
             if tile == 0 and M < 640:
-                tile = _decode_tile(M, N)
+                tile = _decode_tile(M)
             splits = _auto_splits(M, N, K) if tile in (0, 2, 3) or (tile == 9 and M <= 128) else 1
     if splits > 1 and ws is None:
         ws = _workspace(splits * M * N * 4, a.device)
@@ -627,17 +628,9 @@ def gemm_resid_norm(a, w, resid, gamma, eps: float, out=None, h_out=None, bias=N
     return h_out
 
 
-def _decode_tile(M: int, N: int = 0) -> int:
-    """Decode-sized M: 32x128 tiles up to 32 rows, else the weight-streaming tile (64x128 to 64 rows,
-    128x128 above; csrc/gemm.hip). 65..128 rows have it only for N >= 20480 (gate/up, LM head), where its
-    tiles cover most of the CUs: one 128x64 register-staged tile per 64 weight rows otherwise (weights
-    cold: 80 x 28672 x 4096 48.5 vs 58 us, 128 x 128256 x 4096 230 vs 255, but 100 x 12288 x 3072 29 vs
-    27 and 128 x 4096 x 4096 21 vs 18). 129..639 rows: ``_mid_tile``."""
-    if M <= 32:
-        return 3
-    if 64 < M <= 128:
-        return 2 if N >= 20480 else 9
-    return 2
+def _decode_tile(M: int) -> int:
+    """The tile of up to 64 rows: 32x128 up to 32, else the weight-streaming tile (csrc/gemm.hip)."""
+    return 3 if M <= 32 else 2
 
 
 @_rule
@@ -647,22 +640,20 @@ def _auto_splits(M: int, N: int, K: int) -> int:
     workgroup (gemm.hip PF) a tile needs fewer splits to cover HBM latency, and fewer splits = fewer
     partial bytes to reduce. From a graph-replayed sweep with weights streamed cold from HBM, as in a real
     decode step (profiles/decode_gemm_prefetch_sweep_r1.jsonl: matches the best split on 17 of 20 Phi-3 /
-    Llama-3-8B shapes at M = 16 / 64, within 0.7 us on the rest). 129..639 rows: ``_mid_stream``."""
+    Llama-3-8B shapes at M = 16 / 64, within 0.7 us on the rest)."""
     if M >= 640:
         return 1
     ksteps = K // 64
-    if 64 < M <= 128:  # (see _decode_tile) wide N: no split; else 4 splits, fewer if K is short
+    if 64 < M <= 128:  # wide N: no split; else 4 splits, fewer if K is short
         if N >= 8192:
             return 1
         s = 4
         while s > 1 and (ksteps % s or ksteps // s < 4):
             s //= 2
         return s
-    if M > 128:
-        return _mid_stream(M, N, K)[1]
-    if M > 32 and N > 8192 and K <= 8192:  # (see _dk_splits)
+    if 32 < M <= 64 and N > 8192 and K <= 8192:  # (see _dk_splits)
         return 1
-    tiles = math.ceil(N / 128)
+    tiles = math.ceil(M / 64) * math.ceil(N / 128)
     s = 1
     while tiles * s * 2 <= 256 and ksteps % (s * 2) == 0 and ksteps // (s * 2) >= 4:
         s *= 2
@@ -748,41 +739,6 @@ def _rope_apart(M: int, N: int, K: int) -> bool:
     tiles = math.ceil(M / 256) * math.ceil(N / 256)
     return M < ROW_TILES_BELOW and (_row_us(M, N, K)[0] + 4 + M * N * 1e-6
                                     < 0.97 * (_phase_us(M, N, K, EPI_ROPE, 7 if tiles >= 256 else 10) + 4))
-
-
-def _reduce_us(M: int, N: int, splits: int) -> float:
-    """The reduce of a split product: a launch, and the partials out and in at 4 TB/s."""
-    return 4 + splits * M * N * 2e-6 if splits > 1 else 0.0
-
-
-def _mid_stream(M: int, N: int, K: int):
-    """(microseconds, splits) of a product of 129..639 rows on the 128x128 streaming tile: rounds of the chip at 0.56 us a
-    K-step of 64, and the reduce (256 x 4096 x 14336 50 us at 4 splits vs 78 at 2; 200 x 28672 x 4096 79 at 1 vs 96 at 2).
-    At most 1024 64x128 blocks of partials below 256 rows and 640 from there: a prefill must not outgrow the workspace
-    that captured decode steps point at."""
-    ksteps, tiles = K // 64, math.ceil(M / 128) * math.ceil(N / 128)
-    most = (1024 if M < 256 else 640) // (math.ceil(M / 64) * math.ceil(N / 128))
-    return min((math.ceil(tiles * s / 256) * (ksteps // s) * 0.56 + _reduce_us(M, N, s), s) for s in (1, 2, 4, 8)
-               if s == 1 or (ksteps % s == 0 and ksteps // s >= 4 and s <= most))
-
-
-@_rule
-def _mid_tile(M: int, N: int, K: int):
-    """(tile, splits) of a product of 129..639 rows: the 128x128 streaming tile (2), or the register-staged 64x128 one (11)
-    over ceil(M / 64) row blocks with up to 4 workgroups a CU below 256 rows and 2.5 from there (32-layer Phi-3 chain,
-    bench/midm_chain.py, profiles/r2/midm_chain.txt). The latter shares a CU, so a round that is not full costs it less:
-    0.36 us a K-step and workgroup of a CU (a third below what it takes by itself: a close call goes to it), and it has no
-    ring to fill (1.5 us). Register / streaming, us: 300 x 12288 x 4096 56 / 72 (288 streaming tiles: two rounds), 448 x
-    9216 x 3072 44 / 59, 160 x 768 x 1024 9.5 / 11.3, 300 x 3072 x 8192 38 / 44; 512 x 4096 x 4096 38 / 32, 200 x 28672 x
-    4096 99 / 79, 256 x 4096 x 14336 61 / 49. Over 1078 shapes none is more than 3 % slower than on the register tile."""
-    ksteps, blocks = K // 64, math.ceil(M / 64) * math.ceil(N / 128)
-    most = 1024 if M < 256 else 640
-    s = 1
-    while blocks * s * 2 <= most and ksteps % (s * 2) == 0 and ksteps // (s * 2) >= 4:
-        s *= 2
-    staged = max(1.0, blocks * s / 256) * (ksteps // s) * 0.36 + _reduce_us(M, N, s)
-    us, splits = _mid_stream(M, N, K)
-    return (2, splits) if us + 1.5 < staged else (11, s)
 
 
 # ------------------------------------------------------------------------------ norms etc.

@@ -15,12 +15,21 @@ def test_wide_products_of_up_to_64_rows(N, Kd, one):
         assert K._dk_splits(N, Kd, reduce=True) >= 2
 
 
-@pytest.mark.parametrize("M,N,Kd,tile", [(300, 12288, 4096, 11), (448, 9216, 3072, 11), (160, 768, 1024, 11), (300, 3072, 8192, 11),
-                                         (129, 320, 14336, 11), (512, 4096, 4096, 2), (200, 28672, 4096, 2),
-                                         (256, 4096, 14336, 2), (639, 3072, 8192, 2)])
+@pytest.mark.parametrize("M,N,Kd,tile", [(300, 12288, 4096, 18), (448, 9216, 3072, 18), (160, 768, 1024, 16), (300, 3072, 8192, 16),
+                                         (129, 320, 14336, 16), (512, 4096, 4096, 15), (200, 28672, 4096, 7),
+                                         (256, 4096, 14336, 14), (639, 3072, 8192, 10)])
 def test_tile_of_129_to_639_rows(M, N, Kd, tile):
-    """A last round of 128x128 tiles that is nearly empty, and short products, are for the register-staged tile."""
-    got, splits = K._mid_tile(M, N, Kd)
+    """Few or short rounds on the streaming tiles, long ones of many columns on the phase-split kernel."""
+    got, splits = K._row_tile(M, N, Kd)
     assert got == tile and (Kd // 64) % splits == 0 and Kd // 64 // splits >= 4
-    # (a prefill must not outgrow the workspace of captured decode steps)
+    # (partials of 32 MB below 256 rows and 20 MB from there)
     assert splits == 1 or splits * -(-M // 64) * -(-N // 128) <= (1024 if M < 256 else 640)
+
+
+@pytest.mark.parametrize("M", [65, 128, 129, 300, 639])
+@pytest.mark.parametrize("N,Kd", [(768, 768), (4096, 4096), (28672, 4096), (64, 1 << 22)])
+def test_splits_of_rows_too_long_for_the_streaming_tiles(M, N, Kd):
+    """One round of 64 x 128 tiles at most, or four splits up to 128 rows; four K-steps a split."""
+    s = K._auto_splits(M, N, Kd)
+    assert (Kd // 64) % s == 0 and (s == 1 or Kd // 64 // s >= 4)
+    assert s <= 4 if M <= 128 else s == 1 or s * -(-M // 64) * -(-N // 128) <= 256

@@ -62,9 +62,10 @@ def test_row_norm_without_splits(M, N, Kd, epi):
     assert ((got - ref).abs() <= U * ref.abs() + 8 * Kd * 2.0 ** -24 * mag).all()
 
 
-@pytest.mark.parametrize("M,N,stages,splits", [(64, 136, 19, 2), (64, 136, 20, 2), (33, 4096 + 8, 28, 3), (48, 320, 4, 32)])
+@pytest.mark.parametrize("M,N,stages,splits", [(64, 136, 19, 2), (64, 136, 20, 2), (33, 4096 + 8, 28, 3), (48, 320, 4, 32), (64, 136, 5, 4),
+                                               (64, 136, 6, 4)])
 def test_split_products_either_side_of_the_ring(M, N, stages, splits):
-    """K splits of up to 64 rows: 20 stages are the first on the ring, shorter ones are staged through registers."""
+    """K splits of up to 64 rows: 6 stages are the first on the ring, shorter ones are staged through registers."""
     Kd = 64 * stages * splits
     a, w, bias, g = _operands(M, N, Kd, Kd + 64)
     resid = torch.randn(M, N, device="cuda", generator=g).bfloat16()
@@ -115,5 +116,18 @@ def test_mid_rows(M, N, Kd, epi):
     ref = {"gelu": torch.nn.functional.gelu, "swiglu": _swiglu}.get(epi, lambda x: x)(ref)
     if resid is not None:
         ref = ref + resid.double()
+    tol = U * ref.abs() + 8 * Kd * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T).max()
+    assert ((got - ref).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("M,N,Kd", [(65, 768, 1024), (200, 320, 512)])
+def test_rows_too_long_for_the_streaming_tiles(M, N, Kd):
+    """Rows 4 M elements apart: the register-staged tile, in splits."""
+    a, w, bias, g = _operands(M, N, Kd)
+    apart = torch.empty(M * (1 << 22), device="cuda", dtype=torch.bfloat16).view(M, 1 << 22)[:, :Kd]
+    apart.copy_(a)
+    assert K._auto_splits(M, N, Kd) > 1
+    got = K.gemm(apart, w, bias, epi=K.EPI_BIAS).double()
+    ref = a.double() @ w.double().T + bias.double()
     tol = U * ref.abs() + 8 * Kd * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T).max()
     assert ((got - ref).abs() <= tol).all()
