@@ -343,6 +343,9 @@ static int fp8_tile(long M, long N) {
   return tiles(128) < 512 * ((tiles(256) + 255) / 256) ? 128 : 256;
 }
 
+// Rows and columns of a product's tiles.
+DA_EXPORT int da_gemm_fp8_tile(int M, int N) { return fp8_tile(M, N); }
+
 template <int BT>
 static int launch_fp8(const GemmArgs& a, int epi, hipStream_t s) {
   const dim3 grid(((a.M + BT - 1) / BT) * ((a.N + BT - 1) / BT));

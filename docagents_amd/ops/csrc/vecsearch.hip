@@ -869,7 +869,8 @@ struct ScanPlan {
 // A run is a wave's (up to 16 queries; rows_per_wave at least) or a workgroup's (17 and more), 16 to 524288 rows (32-bit
 // offsets), and as many as one round of resident workgroups needs: a second round starts its pipelines anew, us with 1024
 // waves / 4096: 100000 x 1024, 16 queries, 48.7 / 56.3; 411812 x 768 113.6 / 121.0; 1250000 x 1024 417 / 419.
-// A group is a tile up to 65536 groups, so that the pick reads 256 KB a query at most, and 2, 4, .. tiles from there on.
+// A group is a tile up to 65536 of them, and 2, 4, .. tiles from there on; with the padding of the runs' ends the pick reads 290 KB
+// a query at most (1.05 and 2.1 M rows 279, scores of 57925 rows with K = 32 290).
 // Up to 10000 + 1500 K rows each row's score is left, and nothing is scored again: more to write and to read for fewer steps of
 // the pick, a wave's tile of a group each. us, groups / scores: 464 x 1024, K = 24, 2 queries 36 / 14; 512 x 768, K = 8, 24
 // queries 19 / 12; 10000 x 1024, 24 queries, K = 5 25 / 21, K = 20 39 / 22; 20000 x 768, 128 queries 29 / 33 and 41 / 34;

@@ -67,6 +67,7 @@ _SIGS = {
     "da_enc_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5
                   + [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_void_p],
     "da_gemm_tail_ws": [c_int] * 5,
+    "da_gemm_fp8_tile": [c_int] * 2,
     "da_gemm8p_ksteps": [c_int] * 5,
     "da_gemm_capture_id": [c_void_p],
     "da_gemm_dk_splitk": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
