@@ -1671,6 +1671,9 @@ decode_attn_gqa_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __re
 // 5.5 / 7.3 / 11.6 / 13.5; rows of 64 - 146 keys, 4 / 12 / 30 / 40 of them, 10.6 / 18.1 / 17.9 / 23.2 -> 6.5 / 7.9 / 14.1 /
 // 16.3; of 500 - 2000 19.0 / 50.8 / 86.7 / 89.1 -> 16.6 / 41.6 / 79.4 / 88.5 (5.9 TB/s). Few keys: bound by the launch, the
 // chain length -> addresses -> keys and the merge, about 5 us.
+// One stage of tiles: with two for D = 64 a CU has two workgroups, which short rows wait for, us two / one (the VALU before): 12
+// heads, 64 rows of 40 - 146 keys 10.8 / 8.1 (8.5), 32 of 200 - 500 15.0 / 12.3 (13.1), 16 of 500 - 2000 19.5 / 16.2 (18.9); long rows
+// lose some of it, 48 of 900 - 3100 51.6 / 55.8 (59.8), one of 4000 among 31 of 200 17.6 / 19.4 (31.7).
 // by_len (as in the GQA kernel): even splits of 12 rows of 64 - 146 keys in a cache of 4096 take 10.9 us, of 200 - 500 15.8 (16.5
 // by length).
 // XC: same-XCD split exchange (see dec_finish).
@@ -1686,7 +1689,7 @@ decode_attn_mfma1_kernel(const bf16_t* __restrict__ q, int ldq, const bf16_t* __
                          bf16_t* __restrict__ out, int ldo, int* __restrict__ cnt, DecRope rope, int by_len) {
   static_assert(D == 64 || D == 96 || D == 128, "head dim");
   constexpr int KT = 32, NDS = D / 32, NDT = D / 16, NS = D / 8;
-  constexpr int TB = KT * D * 2, ND = TB / 1024, ST = D == 64 ? 2 : 1;
+  constexpr int TB = KT * D * 2, ND = TB / 1024, ST = 1;
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   // (one array: with several, hipcc has every LDS read wait for the DMA)
   __shared__ __attribute__((aligned(16))) char ring[4 * ST * 2 * TB + 64 + D * 10];
