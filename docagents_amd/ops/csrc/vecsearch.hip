@@ -661,9 +661,11 @@ topk_merge_kernel(const float* __restrict__ cand_s, const int* __restrict__ cand
 // Bound by latency. A cut of a list of 64 takes about 1 us, and 80000 values in any order improve on one many times (lists
 // kept by every wave, as topk_merge_kernel does: 100 us for 80000 groups, K = 5; 49 for 8000, K = 19), so a bound comes first:
 // the K-th best of the threads' own best values, to its upper 20 bits. What reaches it (little more than K values) is
-// collected and cut once, and the same again with the rows that reach the K-th best group. Lists that overflow (thousands
-// of equal scores) are done over by the waves' lists.
-constexpr int TP_WAVES = 8, TP_CAP = 1024;
+// collected and cut once, and the same again with the rows that reach the K-th best group. Where more than 256 reach it
+// (equal scores), the K-th best is found to its last bit by counting, a pass over the groups for each bit that is open, and its first
+// equals are taken in order. us, lists of every scan / lists of the pick's waves / this: 20000 equal rows x 384, one query, K = 20
+// 155 / 811 / 65, 600000 of 20 kinds, K = 5 181 / 488 / 163, 600000 equal, 64 queries, K = 5 187 / 792 / 187; rows that overflow are done over by the waves' lists.
+constexpr int TP_WAVES = 8, TP_CAP = 1024, TP_FOLD = 256;
 
 // The largest bound, to its upper 20 bits, that at least `need` of the 8 keys of each lane reach (0: there are not as many).
 __device__ __forceinline__ unsigned reached_by(const unsigned (&key)[8], int need) {
@@ -688,9 +690,9 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
   static_assert(TP_WAVES == 8, "a key of each thread: 8 per lane of a wave");
   __shared__ float cs[TP_WAVES][TL_SL], cand_s[TP_CAP];
   __shared__ int ci[TP_WAVES][TL_SL], cand_i[TP_CAP];
-  __shared__ int groups[TK_MAX], count;
+  __shared__ int groups[TK_MAX], count, reach[32], equal[TP_WAVES];
   __shared__ float bound;
-  __shared__ unsigned keys[nt];
+  __shared__ unsigned keys[nt], bkey;
   __shared__ __attribute__((aligned(16))) bf16_t sq[d];
   const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, fr = lane & 15, fg = lane >> 4;
   for (int i = tid; i < d / 8; i += nt) *(u32x4_t*)(sq + i * 8) = *(const u32x4_t*)(Qv + (size_t)q * d + i * 8);
@@ -724,13 +726,15 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
   }
   keys[tid] = td_key(best, best > -INFINITY ? 0 : -1);
   if (tid == 0) count = 0;
+  if (tid < 32) reach[tid] = 0;
   __syncthreads();
   if (wid == 0) {
     unsigned key[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) key[u] = keys[u * 64 + lane];
-    const float b = td_unkey(reached_by(key, K));
-    if (lane == 0) bound = b != b ? -INFINITY : b;
+    const unsigned by = reached_by(key, K);
+    const float b = td_unkey(by);
+    if (lane == 0) { bound = b != b ? -INFINITY : b; bkey = b != b ? 0 : by; }
   }
   __syncthreads();
   const float T = bound;
@@ -740,20 +744,69 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
     for (int e = 0; e < 4; ++e) collect(v[e], 4 * j0 + e, v[e] >= T && v[e] > -INFINITY);
   }
   __syncthreads();
-  const int found = count;
-  const bool over = found > TP_CAP;
-  __syncthreads();  // (wave 0 writes count below)
-  if (over) {
-    for (int j0 = wid * 64; j0 < GT; j0 += nt) {
-      const int j = j0 + lane;
-      const float v = ((const float*)line)[min(j, GT - 1)];
-      top.add(v, j < GT && v > -INFINITY ? j : -1);
+  int found = count;
+  __syncthreads();  // (count is written below)
+  if (found > TP_FOLD) {
+    // the K-th best to its last bit (from bkey to the best), then what is better than it, and as many of its equals as are
+    // missing, first rows first
+    unsigned Tk = 0, kmax = 0;
+    for (int u = 0; u < 8; ++u) kmax = max(kmax, keys[u * 64 + lane]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) kmax = max(kmax, (unsigned)__shfl_xor((int)kmax, o, 64));
+    for (int bt = 31; bt >= 0; --bt) {
+      const unsigned t = Tk | (1u << bt);
+      if (t <= bkey) Tk = t;
+      if (t <= bkey || t > kmax) continue;
+      int c = 0;  // (whole in lane 0, which takes part in every step of its wave)
+      for (int j0 = tid; j0 < nv; j0 += nt) {
+        const f32x4_t v = line[j0];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c += __popcll(__ballot(v[e] > -INFINITY && td_key(v[e], 0) >= t));
+      }
+      if (lane == 0) atomicAdd(&reach[bt], c);
+      __syncthreads();
+      if (reach[bt] >= K) Tk = t;
+    }
+    if (tid == 0) count = 0;
+    __syncthreads();
+    for (int j0 = tid; j0 < nv; j0 += nt) {
+      const f32x4_t v = line[j0];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) collect(v[e], 4 * j0 + e, v[e] > -INFINITY && td_key(v[e], 0) > Tk);
     }
     __syncthreads();
+    found = count;  // (less than K)
+    for (int j0 = 0; j0 < nv && found < K; j0 += nt) {
+      const f32x4_t v = line[min(j0 + tid, nv - 1)];
+      unsigned m = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m |= (unsigned)(j0 + tid < nv && v[e] > -INFINITY && td_key(v[e], 0) == Tk) << e;
+      int at = __popc(m);  // equals up to this lane's last
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int x = __shfl_up(at, o, 64);
+        if (lane >= o) at += x;
+      }
+      if (lane == 63) equal[wid] = at;
+      __syncthreads();
+      int all = found;
+      at += found - __popc(m);
+      for (int w = 0; w < TP_WAVES; ++w) {
+        if (w < wid) at += equal[w];
+        all += equal[w];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if ((m >> e) & 1) {
+          if (at < K) { cand_s[at] = v[e]; cand_i[at] = 4 * (j0 + tid) + e; }
+          ++at;
+        }
+      found = min(all, K);
+      __syncthreads();  // (equal is written again)
+    }
   }
   if (wid == 0) {
-    if (over) top_join(top, cs, ci, TP_WAVES);
-    else fold(found);
+    fold(found);
     if (lg < 0) {  // these are the rows
       if (lane < K && ci[0][lane] >= 0) ci[0][lane] = ci[0][lane] / run_slots * run_rows + ci[0][lane] % run_slots;
       wave_sync_lds();

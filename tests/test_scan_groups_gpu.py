@@ -16,7 +16,8 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("N,d,Q,Kk,cols", [
     (1_100_003, 384, 20, 5, 384), (1_100_003, 384, 3, 32, 4),  # groups of two tiles
     (66_000, 1024, 70, 8, 1024), (66_000, 768, 129, 20, 3),
-    (20_001, 768, 17, 32, 5), (4_100, 384, 16, 20, 6), (70_001, 1024, 1, 5, 2), (17_499, 384, 20, 5, 5), (17_501, 384, 20, 5, 5), (9_000, 768, 33, 3, 2), (100, 768, 65, 32, 768), (17, 1024, 64, 1, 4)])
+    (20_001, 768, 17, 32, 5), (4_100, 384, 16, 20, 6), (70_001, 1024, 1, 5, 2), (17_499, 384, 20, 5, 5), (17_501, 384, 20, 5, 5), (9_000, 768, 33, 3, 2), (100, 768, 65, 32, 768), (17, 1024, 64, 1, 4),
+    (20_000, 384, 5, 20, 0), (2_100, 768, 2, 32, 0), (70_001, 768, 18, 5, 1), (300_000, 1024, 66, 32, 0)])  # (0: all rows equal)
 def test_groups_and_ties(N, d, Q, Kk, cols):
     g = torch.Generator(device=DEV).manual_seed(N + d + Q)
     rand = lambda n: torch.randint(-1, 2, (n, d), device=DEV, generator=g, dtype=torch.int8).to(torch.bfloat16)  # noqa: E731
