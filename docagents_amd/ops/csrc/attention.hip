@@ -1003,7 +1003,7 @@ __device__ __forceinline__ void dec_finish(const float* po, const float* pm, con
                                            int act) {
   if (act == 1 || cnt == nullptr) return;  // no counters: the host launches decode_combine_kernel
   const int tid = threadIdx.x;
-  // Partials and tickets live in UNCACHED memory (da_malloc_uncached: MTYPE UC, L2 bypassed), so
+  // Partials and tickets live in UNCACHED memory (da_malloc_uncached: MTYPE UC, L2 bypassed, L1 not), so
   // device-wide visibility needs only this workgroup's stores to have completed — no
   // __threadfence(), whose L2 write-back + invalidate of the whole cache costs more than the
   // combine launch it replaces (measured: 24.6 -> 48.4 us at batch 1).
@@ -1020,10 +1020,9 @@ __device__ __forceinline__ void dec_finish(const float* po, const float* pm, con
   }
   __syncthreads();
   if (!*s_last) return;
-  auto ld = [](const float* p) -> float {
-    if constexpr (XC) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else return *p;
-  };
+  // Past this CU's L1 (agent scope), for uncached memory too: the maxima and sums of some 10 (row, head) pairs share a line, and a
+  // workgroup that merged one of them here earlier in this launch has left that line, with the others' from before, in L1.
+  auto ld = [](const float* p) -> float { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
   // One online pass over the splits, 8 splits' (m, l, o) loads issued per step: the partials sit in
   // uncached memory (~1-2 us per round trip), so a max pass + a sum pass that each walk the splits
   // one dependent load at a time cost ~2 x nsplit round trips — most of a batch-1 decode attention.

@@ -57,3 +57,29 @@ def test_automatic_split(H, Hkv, D, B, S, route, monkeypatch):
         for _ in range(2):
             got = K.decode_attn(q, kc, vc, lt, slot, H, Hkv, D, max_len=S).float()
             assert bool(((got - want).abs() <= 2.0 ** -7 * (1 + want.abs())).all())
+
+
+@pytest.mark.parametrize("B,Hkv,G,D,S,chunk", [(22, 12, 1, 96, 1088, 0), (22, 12, 1, 64, 1088, 0), (60, 12, 1, 96, 1088, 64),
+                                               (60, 12, 2, 128, 1088, 64)])
+def test_merges_see_this_launchs_sums(B, Hkv, G, D, S, chunk):
+    """Short rows merge while their neighbours' splits still run, and leave a line of the neighbours' maxima and sums in their CU's
+    L1: a merge there afterwards must not read those of the launch before. Questions change from launch to launch."""
+    H, g = Hkv * G, torch.Generator(device=DEV).manual_seed(B)
+    kc, vc = (torch.randn(B, Hkv, S, D, device=DEV, generator=g).bfloat16() for _ in range(2))
+    lens = [1 if i * 7 % 5 < 2 else S if i % 3 else 1 + i * 389 % S for i in range(B)]
+    lt, slot = torch.tensor(lens, dtype=torch.int32, device=DEV), torch.arange(B - 1, -1, -1, dtype=torch.int32, device=DEV)
+    mask = torch.arange(S, device=DEV) >= lt[:, None]
+    cases = []
+    for _ in range(4):
+        q = torch.randn(B, H * D, device=DEV, generator=g).bfloat16()
+        s = (q.float().view(B, Hkv, G, D) @ kc[slot.long()].float().transpose(2, 3).contiguous()) * D ** -0.5
+        p = torch.softmax(s.masked_fill(mask[:, None, None], -torch.inf), -1)
+        v = vc[slot.long()].float()
+        want, mag = (p @ v).reshape(B, -1), (p @ v.abs()).reshape(B, -1)
+        # weights and the result are rounded to bf16
+        cases.append((q, want, 2.0 ** -8 * (want.abs() + 1.02 * mag) + 2.0 ** -12))
+    wrong = torch.zeros((), dtype=torch.int64, device=DEV)
+    for i in range(600):
+        q, want, tol = cases[i % 4]
+        wrong += ((K.decode_attn(q, kc, vc, lt, slot, H, Hkv, D, S, chunk=chunk).float() - want).abs() > tol).sum()
+    assert wrong.item() == 0
