@@ -431,7 +431,8 @@ __device__ __forceinline__ void dma2_lds(__amdgpu_buffer_rsrc_t rs, unsigned lds
 // barrier a tile. 16-B chunk c of row r is at c ^ (r >> 1) in a K (and Q, O) tile and at c ^ ((r & 2) << 1) in a V tile: both
 // reads are free of bank conflicts. A wave without queries only moves its part of the tiles. Rows go out whole, through LDS.
 // The maximum that weights are relative to moves when it is 2^SPEC_TAU off (rescaling O takes a quarter of a tile's vector
-// instructions, and some row of 32 has a new maximum at most tiles of a short sequence).
+// instructions, and some row of 32 has a new maximum at most tiles of a short sequence). bf16: all of them 2^-SPEC_TAU times
+// that, so that sums of values near the type's largest don't leave fp32 (fp16 has no range below for it, and values of 2^16 at most).
 // Bound by the vector ALU (of 64 x 512 rows, 16 heads: 63 % of its cycles, the MFMAs 30 %) and by what is left of a round for
 // ragged sequences. us, by registers one tile ahead with two workgroups a CU / this: 80 texts of 61 - 512 rows, 16 heads, fp16
 // 110 / 86; 64 of 512 118 / 97 (710 TF); 12 heads, bf16: 80 of 61 - 512 78 / 60; one of 400 rows 13.0 / 11.1.
@@ -556,7 +557,7 @@ flash_attn_enc_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k
 #pragma unroll
         for (int i = 0; i < 2; ++i) oacc[i] *= alpha;
       }
-      const float mc = m_run == -INFINITY ? 0.f : -m_run * c;
+      const float mc = m_run == -INFINITY ? 0.f : fmaf(-m_run, c, T::kF16 ? 0.f : -SPEC_TAU);
       float psum = 0.f;
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh)

@@ -54,3 +54,19 @@ def test_infinite_scores():
     want, mag = p @ r(v), p @ r(v).abs()
     # weights and the result are rounded to the type
     assert ((got - want).abs() <= 2.0 ** -8 * (mag + want.abs()) * 1.01 + 2.0 ** -13).all()
+
+
+def test_values_near_the_largest():
+    """A value of 3e38 under weights of a few per cent, where the scores rise along the keys."""
+    D, H, T = 64, 2, 300
+    g = torch.Generator(device="cuda").manual_seed(6)
+    q, k, v = (torch.randn(T, H * D, device="cuda", generator=g) for _ in range(3))
+    k *= torch.linspace(0.05, 2, T, device="cuda").view(-1, 1)
+    v[T - 5:, 3] = 3e38
+    q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+    cu = torch.tensor([0, T], device="cuda", dtype=torch.int32)
+    got = K.flash_attn_varlen(q, k, v, cu, T, H, H, D, False).double().view(T, H, D).transpose(0, 1)
+    r = lambda t: t.double().view(T, H, D).transpose(0, 1)  # noqa: E731
+    p = torch.softmax(r(q) @ r(k).transpose(1, 2) * D ** -0.5, -1)
+    want, mag = p @ r(v), p @ r(v).abs()
+    assert ((got - want).abs() <= 2.0 ** -8 * (mag + want.abs()) * 1.01 + 2.0 ** -13).all()
