@@ -290,16 +290,16 @@ def _gemm_tail(device, stream: int, M: int, N: int, K: int, epi: int, tile: int 
     return part, cnt
 
 
-def _call_scratch(nbytes: int, device) -> torch.Tensor:
-    """Scratch as the call's own, from the caching allocator (a capture's: from its graph's pool). The workspace of a role is
+def _call_scratch(nbytes: int, like) -> torch.Tensor:
+    """Scratch as the call's own, where ``like`` is, from the caching allocator (a capture's: from its graph's pool). The workspace of a role is
     one stream's, and one that grows drops the buffer that captured decode steps still write to: what may outgrow what a
     generator reserved (the scores or group maxima of a search, up to 67 MB) must not come from there."""
-    return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    return like.new_empty(-(-nbytes // like.element_size()))  # (0.7 us less than torch.empty with a type and a device)
 
 
-def _call_partials(splits: int, M: int, N: int, device):
+def _call_partials(splits: int, M: int, N: int, like):
     """A product's K-split partials as the call's own: None if whole."""
-    return _call_scratch(splits * M * N * 4, device) if splits > 1 else None
+    return _call_scratch(splits * M * N * 4, like) if splits > 1 else None
 
 
 def gemv_fusable(M: int, N: int, K: int, epi: int = EPI_NONE) -> bool:
@@ -354,10 +354,10 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
     if splits <= 0:
         if tile == 0 and M > 64 and _row_tiles_ok(M, N) and max(K, a.stride(0)) < 1 << 22:
             tile, splits = _row_tile(M, N, K, epi)
-            ws = _call_partials(splits, M, N, a.device)
+            ws = _call_partials(splits, M, N, a)
         elif tile == 0 and 64 < M < 640:  # rows too long for the streaming tiles' offsets: the register-staged 64x128 tile
             tile, splits = 11, _auto_splits(M, N, K)
-            ws = _call_partials(splits, M, N, a.device)
+            ws = _call_partials(splits, M, N, a)
         else:
             if tile == 0 and M < 640:
                 tile = _decode_tile(M)
@@ -1209,9 +1209,9 @@ def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_bloc
         # the streaming scan (search-sized batches over a big shard; k-means assignment, with the
         # rows as the queries, keeps the query-major tiles below)
         rpw = _scan_rows(N)
-        ws = _call_scratch(int(lib().da_topk_stream_ws(N, Q, K, rpw)), X.device)
-        out_s = torch.empty((Q, K), dtype=torch.float32, device=X.device)
-        out_i = torch.empty((Q, K), dtype=torch.int32, device=X.device)
+        ws = _call_scratch(int(lib().da_topk_stream_ws(N, Q, K, rpw)), X)
+        out_s = X.new_empty((Q, K), dtype=torch.float32)
+        out_i = X.new_empty((Q, K), dtype=torch.int32)
         _check(lib().da_topk_dense_stream(_ptr(X), N, d, _ptr(slots), _ptr(Qv), Q, _ptr(bitmap), W, float(thr), K,
                                           rpw, _ptr(ws), _ptr(out_s), _ptr(out_i), _stream()), "topk_dense_stream")
         return out_s, out_i
@@ -1220,9 +1220,9 @@ def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_bloc
         nblk = max(1, min(math.ceil(N / 256), max(1, 1024 // qt)))
         rows_per_block = max(64, math.ceil(math.ceil(N / nblk) / 64) * 64)
     nblk = max(1, math.ceil(N / rows_per_block))
-    ws = _call_scratch(nblk * Q * K * 8, X.device)
-    out_s = torch.empty((Q, K), dtype=torch.float32, device=X.device)
-    out_i = torch.empty((Q, K), dtype=torch.int32, device=X.device)
+    ws = _call_scratch(nblk * Q * K * 8, X)
+    out_s = X.new_empty((Q, K), dtype=torch.float32)
+    out_i = X.new_empty((Q, K), dtype=torch.int32)
     _check(lib().da_topk_dense(_ptr(X), N, d, _ptr(slots), _ptr(Qv), Q, _ptr(bitmap), W, float(thr), K,
                                rows_per_block, _ptr(ws), _ptr(out_s), _ptr(out_i), _stream()), "topk_dense")
     return out_s, out_i
@@ -1269,12 +1269,12 @@ def _ranges(X, Qv, ranges, range_off, lists, K, thr, max_rows, slots, bitmap, ro
         _req(slots is not None, "bitmap needs slots")
         _req(bitmap.dtype == torch.int32 and bitmap.shape[0] == Q, "bitmap")
         W = bitmap.shape[1]
-    out_s = torch.empty((Q, K), dtype=torch.float32, device=X.device)
-    out_i = torch.empty((Q, K), dtype=torch.int32, device=X.device)
+    out_s = X.new_empty((Q, K), dtype=torch.float32)
+    out_i = X.new_empty((Q, K), dtype=torch.int32)
     if Q == 0:
         return out_s, out_i
     splits = max(1, math.ceil(max_rows / rows_per_split))
-    ws = _call_scratch(splits * Q * K * 8, X.device)
+    ws = _call_scratch(splits * Q * K * 8, X)
     _check(lib().da_topk_ranges(_ptr(X), d, _ptr(slots), _ptr(Qv), Q, _ptr(ranges), _ptr(range_off), _ptr(lists),
                                 0 if lists is None else lists.shape[1], _ptr(bitmap),
                                 W, float(thr), K, splits, rows_per_split, _ptr(ws), _ptr(out_s), _ptr(out_i),
@@ -1366,7 +1366,7 @@ def gemm_f16(a, w, bias=None, epi: int = EPI_NONE, resid=None, out=None) -> torc
     _req(out.dtype == torch.float16 and out.shape == (M, N) and out.stride(1) == 1 and out.stride(0) % 8 == 0, "out")
     stream = _raw_stream()
     tile, splits = _row_tile(M, N, K, epi, True) if _row_tiles_ok(M, N) and max(K, a.stride(0)) < 1 << 22 else (0, 1)
-    ws = _call_partials(splits, M, N, a.device)
+    ws = _call_partials(splits, M, N, a)
     tail = _gemm_tail(a.device, stream, M, N, K, epi, tile) if tile in (7, 10) or (tile == 0 and M >= 256) else (None, None)
     _check(lib().da_gemm_f16(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
                              M, N, K, epi, tile, splits, _ptr(ws), *map(_ptr, tail), c_void_p(stream)), "gemm_f16")
