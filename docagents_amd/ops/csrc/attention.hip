@@ -435,7 +435,7 @@ __device__ __forceinline__ void dma2_lds(__amdgpu_buffer_rsrc_t rs, unsigned lds
 // that, so that sums of values near the type's largest don't leave fp32 (fp16 has no range below for it, and values of 2^16 at most).
 // Bound by the vector ALU (of 64 x 512 rows, 16 heads: 63 % of its cycles, the MFMAs 30 %) and by what is left of a round for
 // ragged sequences. us, by registers one tile ahead with two workgroups a CU / this: 80 texts of 61 - 512 rows, 16 heads, fp16
-// 110 / 86; 64 of 512 118 / 97 (710 TF); 12 heads, bf16: 80 of 61 - 512 78 / 60; one of 400 rows 13.0 / 11.1.
+// 85 / 70; 64 of 512 115 / 97 (710 TF); 12 heads, bf16: 80 of 61 - 512 67 / 55, 64 of 512 85 / 73; one of 400 rows 11.4 / 9.4.
 template <typename T>
 __global__ void __launch_bounds__(256, 4)
 flash_attn_enc_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v, int ldq, int ldk,
