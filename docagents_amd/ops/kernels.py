@@ -736,7 +736,7 @@ def _rope_apart(M: int, N: int, K: int) -> bool:
     """A QKV projection of 256 rows and more as a product by itself, on the tile that it has then, and rope_cache behind it (which
     reads and writes the result once more; the rotation costs the phase-split kernel 4 us): 432 x 6144 x 4096 54 -> 39 us, 300 x 9216
     x 3072 46 -> 34, 800 x 6144 x 4096 54 -> 50, where 128x256 tiles leave CUs idle, and 1024 x 9216 x 3072 95 -> 69, 1200 x 10240 x
-    8192 212 -> 173, where the last round of a product without the rotation is shared out along K."""
+    8192 212 -> 173, where the one kernel has two rounds of 128-row tiles and the product alone one of 256-row ones."""
     tiles = math.ceil(M / 256) * math.ceil(N / 256)
     return M < ROW_TILES_BELOW and (_row_us(M, N, K)[0] + 4 + M * N * 1e-6
                                     < 0.97 * (_phase_us(M, N, K, EPI_ROPE, 7 if tiles >= 256 else 10) + 4))
@@ -1330,7 +1330,8 @@ def spin(us: int, device=None) -> None:
 def gemm8p_persist(on: int = -1) -> int:
     """Persistent tile loop of the prefill GEMM (one workgroup per CU walking its XCD's tiles) on
     (1) / off (0) for later launches; -1 only queries. Returns the previous setting."""
-    _tail_bytes.cache_clear()
+    for rule in (_tail_bytes, _row_us, _rope_apart):  # (the rules that ask which rounds are shared)
+        rule.cache_clear()
     return int(lib().da_gemm8p_persist(int(on)))
 
 

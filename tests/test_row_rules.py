@@ -40,7 +40,18 @@ def test_large_results_of_many_rows():
 
 def test_estimate():
     """No cost is negative; full tiles of 128 rows go into splits sooner; a projection is apart from its rotation where the product
-    alone has a shorter last round, also on the phase-split kernel."""
+    alone has fewer rounds, also on the phase-split kernel."""
     assert all(x >= 0 for t in (*K._ROW_TILES.values(), *K._PHASE_TILES.values()) for x in t)
     assert K._row_tile(128, 3072, 3072) == (15, 4) and K._row_tile(80, 2048, 2048) == (16, 1)
     assert K._row_tile(1024, 9216, 3072) == (0, 1) and K._rope_apart(1024, 9216, 3072) and not K._rope_apart(512, 9216, 3072)
+
+
+def test_choices_follow_the_shared_round():
+    """With the persistent loop off no round is shared, and choices made before are not kept."""
+    shared = K._row_us(700, 10240, 8192)
+    was = K.gemm8p_persist(0)
+    try:
+        alone = K._row_us(700, 10240, 8192)
+    finally:
+        K.gemm8p_persist(was)
+    assert alone[0] > shared[0] and K._row_us(700, 10240, 8192) == shared
