@@ -677,6 +677,7 @@ ROW_TILES_BELOW = 1280
 # below the phase-split kernel's: of 1300 - 5000 rows, us phase-split / streaming: 1300 x 1024 x 1024 16.8 / 11.5, 2000 17.0 / 13.5;
 # 1600 x 768 x 3072 25.1 / 22.3; 1600 x 1024 x 4096 29.3 / 25.2; 3500 x 384 x 1536 22.4 / 17.7; 1300 x 4096 x 4096 54.0 / 46.7.
 # Not 2600 x 1024 x 1024 (18.1 / 19.2), 1600 x 4096 x 1024 (24.5 / 28.3) or 2000 x 3072 x 768 (20.3 / 22.4).
+# Of 44 products that it takes, bf16 and fp16, 43 run in 0.49 - 1.00 of the time and one in 1.07 (1700 x 1024 x 4096 with a residual).
 SMALL_RESULT_ROWS, SMALL_RESULT = 5120, 21 << 18
 
 
