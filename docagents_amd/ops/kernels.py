@@ -392,11 +392,22 @@ def dk_fusable(M: int, N: int, K: int, epi: int = EPI_NONE) -> bool:
 
 
 def dk_wide(M: int, N: int, K: int, lda: int) -> bool:
-    """Products of up to 32 rows and more than 8192 columns: 32-row streaming tiles (csrc/gemm.hip) cover the CUs without
-    gemm_dk's K split in the workgroup, whose 64-wide tile leaves a CU one workgroup and ends in rounds that are not full.
-    16 rows, dk / streaming us: 28672 x 4096 with the norm 50 / 41 (45 / 40 without), 128256 x 4096 191 / 163, 16384 x 3072
-    21.7 / 20.7, 9216 x 3072 18.3 / 17.6 (32 rows: 22.8 / 20.0), 12608 x 4096 21.6 / 20.8; below the line 8192 x 4096 13.7 / 19.4."""
+    """Products of up to 32 rows and more than 8192 columns, which the streaming tiles of csrc/gemm.hip cover the CUs with too."""
     return 1 <= M <= DK_SPLITK_ABOVE and N > 8192 and max(K, lda) <= 8192
+
+
+def _dk_streams(M: int, N: int, K: int, lda: int) -> bool:
+    """More than 16 rows of more than 16384 columns: the streaming tiles share a stage of A among the waves (28672 x 4096, 32
+    rows: 40.6 us, 41.2 on gemm_dk; 16 rows: 40.4 and 38.5; 16384 x 3072, 32 rows: 19.7 and 19.0)."""
+    return M > 16 and N > 16384 and dk_wide(M, N, K, lda)
+
+
+def _dk_whole(M: int, N: int, K: int) -> bool:
+    """33..64 rows that one gemm_dk launch runs faster than streaming tiles (with split-K and a reduce up to 8192 columns): up to
+    16384 columns while K is short, as a workgroup reads all of A. us at 48 / 64 rows, tiles -> gemm_dk: 6144 x 4096
+    17.1 / 18.5 -> 15.2 / 16.7, 8192 x 4096 20.2 / 21.7 -> 16.2 / 17.7, 9216 x 3072 21.4 / 21.6 -> 16.4 / 18.1, 12608 x 4096
+    25.1 / 26.7 -> 22.6 / 24.8; 3072 x 8192 17.5 / 19.0 -> 19.5 / 21.9."""
+    return N <= 16384 and K <= 4096
 
 
 def _dk_splitk(M: int, N: int) -> bool:
@@ -459,13 +470,13 @@ def gemm_dk(a, w, epi: int = EPI_NONE, bias=None, resid=None, out=None, norm_in=
     if ssq_out is not None:
         _req(epi == EPI_RESID and ssq_out.dtype == torch.float32 and ssq_out.is_contiguous()
              and ssq_out.numel() >= dk_parts(N, M) * 64, "bad ssq_out")
-    if dk_wide(M, N, K, a.stride(0)) and ssq_out is None:
+    if _dk_streams(M, N, K, a.stride(0)) and ssq_out is None:
         _check(lib().da_gemm_dk_splitk(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid),
                                        ldr, M, N, K, epi, _ptr(ssq), parts, K, float(eps), None, None, 1, _stream()), "gemm_dk_wide")
         return out
-    if _dk_splitk(M, N) or (DK_SPLITK_ABOVE < M <= 64 and ssq_out is None):
-        # (rows too long for the unsplit tile's 32-bit offsets: the reduce carries the epilogue)
-        splits = _dk_splits(N, K, ssq_out is not None or max(K, a.stride(0)) >= 1 << 22)
+    far = max(K, a.stride(0)) >= 1 << 22  # rows too long for 32-bit offsets within a tile: the reduce carries the epilogue
+    if (_dk_splitk(M, N) and ssq_out is not None) or (ssq_out is None and (far or (M > DK_SPLITK_ABOVE and not _dk_whole(M, N, K)))):
+        splits = _dk_splits(N, K, ssq_out is not None or far)
         ws = _workspace(splits * M * N * 4, a.device) if splits > 1 else None
         _check(lib().da_gemm_dk_splitk(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid),
                                        ldr, M, N, K, epi, _ptr(ssq), parts, K, float(eps), _ptr(ssq_out), _ptr(ws),

@@ -500,11 +500,11 @@ def dk_fusable(M, N, K, epi=EPI_NONE):
 
 
 def dk_parts(N, M=0):
-    """gemm_dk.hip dk_bn for EPI_RESID: row-norm partial sums written per output tile; 33..64 rows
+    """gemm_dk.hip dk_fn for EPI_RESID: row-norm partial sums written per output tile; 33..64 rows
     (the split-K route): one per 512 columns (written by the reduce launch)."""
     if DK_SPLITK_ABOVE < M <= 64 and N % 512 == 0:
         return N // 512
-    bn = 64 if N // 64 >= 192 else (32 if N // 32 >= 192 else 16)
+    bn = 16 if N <= 4096 else 32 if N <= 8192 else 64
     return (N + bn - 1) // bn
 
 
