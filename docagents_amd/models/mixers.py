@@ -9,7 +9,7 @@ it, what it keeps per sequence (``LayerState``), its packed weights and its forw
                        epilogue in fp32, scan (+ D x, silu(z), conv state), output GEMM
     delta rule         [q | k | v | decay rank | gate rank | beta] GEMM, causal conv + silu, decay GEMM whose epilogue
                        leaves log decays in fp32, scan (+ unit norms, beta, conv state), gate GEMM, gated norm of
-                       every head, output GEMM
+                       every head, output GEMM; single tokens: all between the two large GEMMs in one launch
     latent attention   [query rank | latent | rotated key | gates] GEMM, norms + rotation + page write, query GEMM;
                        short portions attend to the cached latents (queries taken into the latent space, results
                        out of it, head by head), long ones to keys and values expanded from them; output GEMM
@@ -242,10 +242,16 @@ class DeltaMixer:
         self.gate = Linear(ops, _pad(heads(w["g2"], H, V), -1, rg), act)
         self.norm = _pad(w["norm"].float(), V)
         self.out = Linear(ops, _pad(heads(w["o"].t(), H, V).t(), hp, -1), act)
+        self.one_step = ops.delta_step_fits(act, H, G, K, V, s.conv, ra, rg)
 
     def __call__(self, h, m: SeqBatch, st: dict, partial=True):
         o, s, C = self.ops, self.s, self.C
         y = self.proj(h)
+        if self.one_step and m.max_len == 1:
+            r = o.delta_step(y, self.conv_w, st["conv"], (self.decay_w, self.dt_bias, self.rate, self.at_decay),
+                             (self.gate.w, self.at_gate), self.at_beta, st["delta"], m, s.dim ** -0.5, self.UNIT_EPS,
+                             norm=(self.norm, s.vdim, self.eps))
+            return self.out(r, partial=partial)
         x = y[:, :C]
         qkv = o.causal_conv(x, self.conv_w, None, st["conv"], m, silu=True)
         decay = o.gemm_any(y[:, self.at_decay:self.at_gate], self.decay_w, self.dt_bias, ANY_SOFTPLUS, coef=self.rate)

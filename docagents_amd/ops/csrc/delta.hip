@@ -9,6 +9,8 @@
 // decays of a tile of tokens are staged in LDS as fp32 (unit norms taken on the way), the next tile's loads in flight
 // meanwhile.
 //
+// delta_step: a batch of single tokens, with the convolution, the low-rank products and the norm around the step (below).
+//
 // delta_chunk: 32 tokens at a time on the matrix cores (below).
 #include "seq.h"
 
@@ -171,6 +173,221 @@ __global__ void __launch_bounds__(256) delta_scan_kernel(DeltaArgs a) {
   // the convolution's state, shared out over the portion's workgroups
   const int wg = blockIdx.y * gridDim.x + blockIdx.x, step = gridDim.x * gridDim.y * 256;
   for (int c = wg * 256 + tid; c < a.conv.C; c += step) conv_state_store<T>(a.conv, a.m, b, c);
+}
+
+// ------------------------------------------------------------------------------- one token, everything behind the projection
+// A decoding row's layer between its input projection and its output product in one launch, a workgroup a row and head:
+// convolution and silu of the head's q, k and v, its log decays and gates (products of the row's low-rank columns, 16
+// channels a wave on the matrix cores, the row in all 16 columns), the step of delta_scan, the gated norm. As five launches
+// (convolution 4.7 - 5.5 us, decays 4.7 - 7.7, gates 4.6 - 5.9, step 4.8 - 52, norm 4.6 - 4.7) the others waited for the
+// start and the end of a launch each; the state (64 KB a head, 268 MB read and written for 64 rows of 32) is what is left.
+// The state is asked for before the first wait, behind what the step needs first; the gates' operands come last.
+struct DeltaStepArgs {
+  const bf16_t* y; int ldy;        // [T][ldy]: C convolved columns [H K | H K | H V], then at_*: decay rank, gate rank, beta
+  const float* conv_w;             // [taps][C]
+  bf16_t* conv_state;              // [slots][taps - 1][C]
+  const bf16_t* decay_w;           // [H K][ra]
+  const float *dt_bias, *rate;     // [H K]
+  const bf16_t* gate_w;            // [H V][rg]
+  const float* norm;               // [V]
+  float* state; bf16_t* o; int ldo;
+  int H, V, C, ra, rg, at_decay, at_gate, at_beta, dim;
+  float q_scale, unit_eps, eps;
+  SeqMeta m;
+};
+
+template <int NS4, int TAPS>  // K = 32 NS4; V <= 128
+__global__ void __launch_bounds__(512, 4) delta_step_kernel(DeltaStepArgs a) {
+  constexpr int K = 32 * NS4, LN = 8, NC = 2, RS = 4;  // RS: K-steps of the low-rank products that are asked for at once
+  __shared__ __attribute__((aligned(16))) float sq[K], sk[K], sa[K], sv[128], sg[128], so[128], sb[1];
+  const int h = blockIdx.x, b = blockIdx.y, t = a.m.cu[b];
+  if (a.m.cu[b + 1] == t) return;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15, fg = lane >> 4;
+  const bool stored = a.m.pos0[b] != 0;
+  const size_t slot = a.m.slot[b];
+  const bf16_t* row = a.y + (size_t)t * a.ldy;
+
+  // ---- what the step needs first: 4 channels of q (wave 0, lanes 0 - 31), k (32 - 63) or v (wave 1) ----
+  const int sl = lane & 31, part = w * 2 + (lane >> 5);  // 0: q, 1: k, 2: v
+  const bool conv = part < 3 && sl < (part == 2 ? a.V / 4 : K / 4);
+  const int cc = part == 2 ? 2 * a.H * K + h * a.V + 4 * sl : part * a.H * K + h * K + 4 * sl;
+  bf16_t* cs = a.conv_state + slot * (TAPS - 1) * a.C + cc;
+  u32x2_t x[TAPS];
+  f32x4_t cw[TAPS];
+  if (conv) {
+#pragma unroll
+    for (int i = 0; i < TAPS; ++i) {
+      x[i] = i + 1 == TAPS ? *(const u32x2_t*)(row + cc) : stored ? *(const u32x2_t*)(cs + (size_t)i * a.C) : u32x2_t{0, 0};
+      cw[i] = *(const f32x4_t*)(a.conv_w + (size_t)i * a.C + cc);
+    }
+  }
+  // channels 16 w .. + 15 of the decays and of the gates; lane (fr < 4, fg) has channel 16 w + 4 fg + fr in the end
+  const int ch = 16 * w + 4 * fg + (fr & 3);
+  const bool dec = 16 * w < K, gat = 16 * w < a.V;
+  float dtb = 0.f, rate = 0.f;
+  if (dec) {
+    dtb = a.dt_bias[h * K + ch];
+    rate = a.rate[h * K + ch];
+  }
+  const bf16_t* dw = a.decay_w + (size_t)(h * K + 16 * w + fr) * a.ra + 8 * fg;
+  const bf16_t* gw = a.gate_w + (size_t)(h * a.V + 16 * w + fr) * a.rg + 8 * fg;
+  bf16x8_t wd[RS], vd[RS];
+  auto ask = [&](bool on, const bf16_t* p, int at, int rank) {
+#pragma unroll
+    for (int s = 0; s < RS; ++s)
+      if (on && 32 * s < rank) {
+        wd[s] = *(const bf16x8_t*)(p + 32 * s);
+        vd[s] = *(const bf16x8_t*)(row + at + 32 * s + 8 * fg);
+      }
+  };
+  auto product = [&](const bf16_t* p, int at, int rank) {
+    f32x4_t z{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < RS; ++s)
+      if (32 * s < rank) z = mfma16(wd[s], vd[s], z);
+    for (int k = 32 * RS; k < rank; k += 32) z = mfma16(*(const bf16x8_t*)(p + k), *(const bf16x8_t*)(row + at + k + 8 * fg), z);
+    return fr == 0 ? z[0] : fr == 1 ? z[1] : fr == 2 ? z[2] : z[3];
+  };
+  ask(dec, dw, a.at_decay, a.ra);
+  asm volatile("" ::: "memory");  // issue order: the state behind them
+
+  // ---- the state: columns NC grp .. of V, 4 channels at 32 i + 4 g ----
+  const int g = tid % LN, grp = tid / LN;
+  f32x4_t S[NC][NS4];
+  float* st[NC];
+  bool live[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    const int c = grp * NC + j;
+    live[j] = c < a.V;
+    st[j] = a.state + ((slot * a.H + h) * a.V + min(c, a.V - 1)) * K + g * 4;
+#pragma unroll
+    for (int i = 0; i < NS4; ++i) S[j][i] = stored ? *(const f32x4_t*)(st[j] + i * LN * 4) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  asm volatile("" ::: "memory");
+
+  if (w < 2) {
+    f32x4_t v{0.f, 0.f, 0.f, 0.f};
+    if (conv) {
+#pragma unroll
+      for (int i = 0; i < TAPS; ++i) {
+        const f32x4_t xi{__uint_as_float(x[i][0] << 16), __uint_as_float(x[i][0] & 0xffff0000u), __uint_as_float(x[i][1] << 16),
+                         __uint_as_float(x[i][1] & 0xffff0000u)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = fmaf(cw[i][e], xi[e], v[e]);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = bf2f(f2bf(act_silu<bf16_t>(v[e])));  // (rounded as the convolution's own launch stores it)
+#pragma unroll
+      for (int i = 0; i + 1 < TAPS; ++i) *(u32x2_t*)(cs + (size_t)i * a.C) = x[i + 1];
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss = fmaf(v[e], v[e], ss);
+    ss = lanes_sum<32>(ss);
+    const float f = part == 2 ? 1.f : (part == 0 ? a.q_scale : 1.f) / sqrtf(ss + a.unit_eps);
+    if (conv) *(f32x4_t*)((part == 0 ? sq : part == 1 ? sk : sv) + 4 * sl) = v * f;
+    if (tid == 96) sb[0] = sigmoid32(bf2f(row[a.at_beta + h]));
+  }
+  if (dec) {
+    const float z = product(dw, a.at_decay, a.ra);
+    if (fr < 4) sa[ch] = __builtin_amdgcn_exp2f(softplus32(z + dtb) * rate);
+  }
+  ask(gat, gw, a.at_gate, a.rg);  // (the gates are needed last)
+  asm volatile("" ::: "memory");
+  lds_barrier();
+
+  f32x4_t kv[NS4];
+  float held[NC], out[NC], u[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) held[j] = out[j] = 0.f;
+#pragma unroll
+  for (int i = 0; i < NS4; ++i) {
+    kv[i] = *(const f32x4_t*)(sk + i * LN * 4 + g * 4);
+    const f32x4_t d = *(const f32x4_t*)(sa + i * LN * 4 + g * 4);
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        S[j][i][e] *= d[e];
+        held[j] = fmaf(S[j][i][e], kv[i][e], held[j]);
+      }
+  }
+  const float beta = sb[0];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) u[j] = beta * (sv[min(grp * NC + j, a.V - 1)] - lanes_sum<LN>(held[j]));
+#pragma unroll
+  for (int i = 0; i < NS4; ++i) {
+    const f32x4_t q = *(const f32x4_t*)(sq + i * LN * 4 + g * 4);
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        S[j][i][e] = fmaf(kv[i][e], u[j], S[j][i][e]);
+        out[j] = fmaf(S[j][i][e], q[e], out[j]);
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    out[j] = lanes_sum<LN>(out[j]);
+    if (g == 0) so[grp * NC + j] = live[j] ? out[j] : 0.f;
+    if (live[j])
+#pragma unroll
+      for (int i = 0; i < NS4; ++i) *(f32x4_t*)(st[j] + i * LN * 4) = S[j][i];
+  }
+  if (gat) {
+    const float z = product(gw, a.at_gate, a.rg);
+    if (fr < 4) sg[ch] = sigmoid32(z);
+  }
+  lds_barrier();
+  if (w) return;
+  const f32x4_t v = *(const f32x4_t*)(so + 4 * sl);
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) ss = fmaf(v[e], v[e], ss);
+  ss = lanes_sum<32>(ss);
+  if (lane >= a.V / 4) return;
+  const float inv = 1.f / sqrtf(ss / a.dim + a.eps);
+  const f32x4_t nw = *(const f32x4_t*)(a.norm + 4 * lane), gt = *(const f32x4_t*)(sg + 4 * lane);
+  f32x4_t r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = v[e] * inv * nw[e] * gt[e];
+  Act<bf16_t>::store4(a.o + (size_t)t * a.ldo + h * a.V + 4 * lane, r);
+}
+
+template <int TAPS>
+static int launch_delta_step(const DeltaStepArgs& a, int K, hipStream_t s) {
+  const dim3 grid(a.H, a.m.B);
+  switch (K) {
+    case 32: delta_step_kernel<1, TAPS><<<grid, 512, 0, s>>>(a); break;
+    case 64: delta_step_kernel<2, TAPS><<<grid, 512, 0, s>>>(a); break;
+    case 96: delta_step_kernel<3, TAPS><<<grid, 512, 0, s>>>(a); break;
+    case 128: delta_step_kernel<4, TAPS><<<grid, 512, 0, s>>>(a); break;
+    default: return (int)hipErrorInvalidValue;
+  }
+  DA_LAUNCH_CHECK();
+}
+
+// Batches of single tokens, bf16: y [T][ldy] as DeltaStepArgs has it, H heads of queries, keys (K = 32, 64, 96, 128 channels)
+// and values (V <= 128, a multiple of 16); ranks multiples of 32; 2 - 4 taps. state and conv_state are replaced.
+DA_EXPORT int da_delta_step(const void* y, int ldy, const void* conv_w, void* conv_state, int taps, const void* decay_w,
+                            const void* dt_bias, const void* rate, int ra, int at_decay, const void* gate_w, int rg, int at_gate,
+                            int at_beta, const void* norm, int dim, float eps, void* state, void* o, int ldo, int H, int K, int V,
+                            float q_scale, float unit_eps, const void* cu, const void* slot, const void* pos0, const void* seq,
+                            int T, int B, void* stream) {
+  if (T < 1 || B < 1 || B > 65535 || H < 1 || V < 16 || V > 128 || V % 16 || ra < 32 || ra % 32 || rg < 32 || rg % 32 || ldy % 8 ||
+      ldo % 4 || at_decay % 8 || at_gate % 8 || dim < 1 || dim > V)
+    return (int)hipErrorInvalidValue;
+  DeltaStepArgs a{(const bf16_t*)y, ldy, (const float*)conv_w, (bf16_t*)conv_state, (const bf16_t*)decay_w, (const float*)dt_bias,
+                  (const float*)rate, (const bf16_t*)gate_w, (const float*)norm, (float*)state, (bf16_t*)o, ldo, H, V,
+                  2 * H * K + H * V, ra, rg, at_decay, at_gate, at_beta, dim, q_scale, unit_eps, eps,
+                  SeqMeta{(const int*)cu, (const int*)slot, (const int*)pos0, (const int*)seq, T, B}};
+  switch (taps) {
+    case 2: return launch_delta_step<2>(a, K, (hipStream_t)stream);
+    case 3: return launch_delta_step<3>(a, K, (hipStream_t)stream);
+    case 4: return launch_delta_step<4>(a, K, (hipStream_t)stream);
+    default: return (int)hipErrorInvalidValue;
+  }
 }
 
 // ------------------------------------------------------------------------------- matrix cores, chunks of 32 tokens

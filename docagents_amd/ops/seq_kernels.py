@@ -25,6 +25,8 @@ K._SIGS.update({
     "da_delta_rule": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int] + [c_int] * 4
                      + [c_float, c_float, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p, c_int, c_void_p] + [c_int] * 4
                      + [c_void_p, c_void_p, c_int, c_void_p] + _META + [c_int, c_void_p],
+    "da_delta_step": [c_void_p, c_int, c_void_p, c_void_p, c_int] + [c_void_p] * 3 + [c_int, c_int, c_void_p, c_int, c_int, c_int,
+                      c_void_p, c_int, c_float, c_void_p, c_void_p] + [c_int] * 4 + [c_float, c_float] + _META + [c_void_p],
     "da_latent_prep": [c_void_p, c_int, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int, c_float, c_void_p,
                        c_void_p, c_int, c_void_p, c_int, c_void_p, c_int] + _META + [c_int, c_void_p],
     "da_latent_attn": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p,
@@ -45,7 +47,7 @@ K._SIGS.update({
                        + _META + [c_int, c_void_p],
 })
 K._PART_OF.update({n: "hybrid" for n in ("da_gemm_any", "da_gemm_any_ws", "da_stream_step", "da_stream_final", "da_causal_conv",
-                                         "da_selective_scan", "da_gated_scan", "da_sigmoid_attn", "da_stream_add", "da_delta_rule",
+                                         "da_selective_scan", "da_gated_scan", "da_sigmoid_attn", "da_stream_add", "da_delta_rule", "da_delta_step",
                                          "da_latent_prep", "da_latent_attn", "da_latent_gather", "da_latent_flash")})
 
 ACTS = (torch.bfloat16, torch.float32)
@@ -397,6 +399,43 @@ def delta_rule(qkv, decay, beta, state, conv_x, conv_state, m: SeqBatch, H: int,
                                float(eps), *_conv_args(conv_x, conv_state, C, qkv.dtype, m), C,
                                1 if m.lens is None else int(m.lens.min()), DELTA_CHUNK_FROM, _ptr(ck), _ptr(base), n,
                                _ptr(frags), *_meta(m), f32, _stream()), "delta_rule")
+    return o
+
+
+def delta_step_fits(act, H: int, G: int, Kd: int, V: int, taps: int, ra: int, rg: int) -> bool:
+    """Whether ``delta_step`` takes a layer's sizes. Heads that share keys are refused: each key head's convolution state
+    has one workgroup that reads and replaces it."""
+    return (act == torch.bfloat16 and H == G and Kd in (32, 64, 96, 128) and V <= 128 and V % 16 == 0 and 2 <= taps <= 4
+            and ra % 32 == 0 and rg % 32 == 0)
+
+
+def delta_step(y, conv_w, conv_state, decay, gate, at_beta: int, state, m: SeqBatch, q_scale: float, unit_eps: float, norm):
+    """A batch of single tokens between a delta layer's input projection y [T, columns] and its output product: ``causal_conv``
+    (silu) of the first columns, log decays (decay = (weight bf16 [H K, rank], bias fp32 [H K], rate fp32 [H K], first column)),
+    ``delta_rule``'s step and its gated norm (gate = (weight bf16 [H V, rank], first column); norm = (weight fp32 [V], true
+    channels of a value head, eps)). state and conv_state are updated. -> [T, H V]."""
+    _, H, V, Kd = state.shape
+    wd, bias, rate, at_decay = decay
+    wg, at_gate = gate
+    weight, dim, eps = norm
+    taps, C = conv_w.shape
+    _act(y, "y", torch.bfloat16)
+    _req(m.max_len == 1 and y.shape[0] == m.T and C == 2 * H * Kd + H * V and y.stride(0) % 8 == 0
+         and y.shape[1] >= max(at_decay + wd.shape[1], at_gate + wg.shape[1], at_beta + H, C), "delta_step columns")
+    for t, name, shape in ((wd, "decay weight", (H * Kd, wd.shape[1])), (wg, "gate weight", (H * V, wg.shape[1]))):
+        _act(t, name, torch.bfloat16)
+        _req(t.is_contiguous() and t.shape == shape, name)
+    _f32(conv_w, "conv_w")
+    _f32(state, "state")
+    for t, name, n in ((bias, "bias", H * Kd), (rate, "rate", H * Kd), (weight, "norm weight", V)):
+        _f32(t, name, n)
+    _req(conv_state.dtype == torch.bfloat16 and conv_state.is_cuda and conv_state.is_contiguous()
+         and conv_state.shape[1:] == (taps - 1, C), "conv state")
+    o = torch.empty((m.T, H * V), dtype=torch.bfloat16, device=y.device)
+    _check(lib().da_delta_step(_ptr(y), y.stride(0), _ptr(conv_w), _ptr(conv_state), taps, _ptr(wd), _ptr(bias), _ptr(rate),
+                               wd.shape[1], at_decay, _ptr(wg), wg.shape[1], at_gate, at_beta, _ptr(weight), dim, float(eps),
+                               _ptr(state), _ptr(o), H * V, H, Kd, V, float(q_scale), float(unit_eps), *_meta(m), _stream()),
+           "delta_step")
     return o
 
 

@@ -208,6 +208,20 @@ def delta_rule(qkv, decay, beta, state, conv_x, conv_state, m: SeqBatch, H: int,
     return (y.flatten(1) * torch.sigmoid(gate.float())).to(qkv.dtype)
 
 
+def delta_step_fits(act, H: int, G: int, K: int, V: int, taps: int, ra: int, rg: int) -> bool:
+    return False
+
+
+def delta_step(y, conv_w, conv_state, decay, gate, at_beta: int, state, m: SeqBatch, q_scale: float, unit_eps: float, norm):
+    _, H, V, K = state.shape
+    (wd, bias, rate, at_decay), (wg, at_gate), (weight, dim, eps) = decay, gate, norm
+    x = y[:, :conv_w.shape[1]]
+    g = gemm_any(y[:, at_decay:at_decay + wd.shape[1]], wd, bias, ANY_SOFTPLUS, coef=rate)
+    qkv = causal_conv(x, conv_w, None, conv_state, m, silu=True)
+    return delta_rule(qkv, g, y[:, at_beta:], state, x, conv_state, m, H, H, q_scale, unit_eps,
+                      (weight, gemm_any(y[:, at_gate:at_gate + wg.shape[1]], wg), dim, eps))
+
+
 def latent_flash_fits(D: int, V: int) -> bool:
     return False
 
