@@ -178,10 +178,11 @@ __global__ void __launch_bounds__(256) delta_scan_kernel(DeltaArgs a) {
 // ------------------------------------------------------------------------------- one token, everything behind the projection
 // A decoding row's layer between its input projection and its output product in one launch, a workgroup a row and head:
 // convolution and silu of the head's q, k and v, its log decays and gates (products of the row's low-rank columns, 16
-// channels a wave on the matrix cores, the row in all 16 columns), the step of delta_scan, the gated norm. As five launches
-// (convolution 4.7 - 5.5 us, decays 4.7 - 7.7, gates 4.6 - 5.9, step 4.8 - 52, norm 4.6 - 4.7) the others waited for the
-// start and the end of a launch each; the state (64 KB a head, 268 MB read and written for 64 rows of 32) is what is left.
-// The state is asked for before the first wait, behind what the step needs first; the gates' operands come last.
+// channels a wave on the matrix cores, the row in all 16 columns), the step of delta_scan, the gated norm. Five launches
+// before (convolution 4.7 - 5.5 us, decays 4.7 - 7.7, gates 4.6 - 5.9, step 4.8 - 52, norm 4.6 - 4.7) took 23.4 us for one row of
+// 32 heads of 128 x 128 and 76 for 64 rows, this one 7.0 and 62: one row is a chain of memory round trips, 64 rows are 268 MB of
+// state read and written at 4.3 TB/s (a large copy: 5). The state is asked for before the first wait, behind what the step
+// needs first; the gates' operands come last.
 struct DeltaStepArgs {
   const bf16_t* y; int ldy;        // [T][ldy]: C convolved columns [H K | H K | H V], then at_*: decay rank, gate rank, beta
   const float* conv_w;             // [taps][C]
@@ -198,156 +199,159 @@ struct DeltaStepArgs {
 
 template <int NS4, int TAPS>  // K = 32 NS4; V <= 128
 __global__ void __launch_bounds__(512, 4) delta_step_kernel(DeltaStepArgs a) {
-  constexpr int K = 32 * NS4, LN = 8, NC = 2, RS = 4;  // RS: K-steps of the low-rank products that are asked for at once
-  __shared__ __attribute__((aligned(16))) float sq[K], sk[K], sa[K], sv[128], sg[128], so[128], sb[1];
+  constexpr int K = 32 * NS4, LN = 8, NC = 2;
+  __shared__ __attribute__((aligned(16))) float sx[3][128], sa[K], sg[128], so[128], ss[4], sb[1];  // sx: q, k (no norms yet), v
   const int h = blockIdx.x, b = blockIdx.y, t = a.m.cu[b];
   if (a.m.cu[b + 1] == t) return;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15, fg = lane >> 4;
   const bool stored = a.m.pos0[b] != 0;
   const size_t slot = a.m.slot[b];
-  const bf16_t* row = a.y + (size_t)t * a.ldy;
+  // Loads through buffer resources: 32-bit offsets, and a sequence that begins reads its slot as zero (an empty resource).
+  auto rsrc = [](const void* p, int bytes) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, bytes, 0x00020000); };
+  constexpr int ALL = 0x7ffffff0;
+  const __amdgpu_buffer_rsrc_t row = rsrc(a.y + (size_t)t * a.ldy, a.ldy * 2);
+  auto load16 = [](const __amdgpu_buffer_rsrc_t& r, int at) { return (bf16_t)__builtin_amdgcn_raw_buffer_load_b16(r, at, 0, 0); };
+  auto frag = [](const __amdgpu_buffer_rsrc_t& r, int at) {
+    return __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0));
+  };
 
-  // ---- what the step needs first: 4 channels of q (wave 0, lanes 0 - 31), k (32 - 63) or v (wave 1) ----
-  const int sl = lane & 31, part = w * 2 + (lane >> 5);  // 0: q, 1: k, 2: v
-  const bool conv = part < 3 && sl < (part == 2 ? a.V / 4 : K / 4);
-  const int cc = part == 2 ? 2 * a.H * K + h * a.V + 4 * sl : part * a.H * K + h * K + 4 * sl;
-  bf16_t* cs = a.conv_state + slot * (TAPS - 1) * a.C + cc;
-  u32x2_t x[TAPS];
-  f32x4_t cw[TAPS];
+  // ---- what the step needs first: a channel of q (waves 0, 1), k (2, 3) or v (4, 5) a lane ----
+  const int part = w >> 1, pc = (w & 1) * 64 + lane;
+  const bool conv = part < 2 ? pc < K : part == 2 && pc < a.V;
+  const int cc = part == 2 ? 2 * a.H * K + h * a.V + pc : part * a.H * K + h * K + pc;
+  bf16_t* cs = a.conv_state + slot * (TAPS - 1) * a.C;
+  const __amdgpu_buffer_rsrc_t rc = rsrc(cs, stored ? (TAPS - 1) * a.C * 2 : 0);
+  bf16_t x[TAPS];
+  float cw[TAPS];
   if (conv) {
 #pragma unroll
     for (int i = 0; i < TAPS; ++i) {
-      x[i] = i + 1 == TAPS ? *(const u32x2_t*)(row + cc) : stored ? *(const u32x2_t*)(cs + (size_t)i * a.C) : u32x2_t{0, 0};
-      cw[i] = *(const f32x4_t*)(a.conv_w + (size_t)i * a.C + cc);
+      x[i] = i + 1 == TAPS ? load16(row, cc * 2) : load16(rc, (i * a.C + cc) * 2);
+      cw[i] = a.conv_w[(size_t)i * a.C + cc];
     }
   }
   // channels 16 w .. + 15 of the decays and of the gates; lane (fr < 4, fg) has channel 16 w + 4 fg + fr in the end
   const int ch = 16 * w + 4 * fg + (fr & 3);
   const bool dec = 16 * w < K, gat = 16 * w < a.V;
+  bf16x8_t wf[2], vf[2];
+  auto ask = [&](const __amdgpu_buffer_rsrc_t& p, int wat, int at, int k0, int rank) __attribute__((always_inline)) {  // two K-steps of 32 from k0
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int k = min(k0 + 32 * s, rank - 32);
+      wf[s] = frag(p, wat + k * 2);
+      vf[s] = frag(row, (at + k + 8 * fg) * 2);
+    }
+  };
+  auto product = [&](const __amdgpu_buffer_rsrc_t& p, int wat, int at, int rank) __attribute__((always_inline)) {  // (the first two are asked for)
+    f32x4_t z{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < rank; k += 64) {
+      if (k) ask(p, wat, at, k, rank);
+      z = mfma16(wf[0], vf[0], z);
+      if (k + 32 < rank) z = mfma16(wf[1], vf[1], z);
+    }
+    return fr == 0 ? z[0] : fr == 1 ? z[1] : fr == 2 ? z[2] : z[3];
+  };
+  const __amdgpu_buffer_rsrc_t dw = rsrc(a.decay_w + (size_t)h * K * a.ra, ALL), gw = rsrc(a.gate_w + (size_t)h * a.V * a.rg, ALL);
+  const int dat = ((16 * w + fr) * a.ra + 8 * fg) * 2, gat_ = ((16 * w + fr) * a.rg + 8 * fg) * 2;
   float dtb = 0.f, rate = 0.f;
   if (dec) {
     dtb = a.dt_bias[h * K + ch];
     rate = a.rate[h * K + ch];
+    ask(dw, dat, a.at_decay, 0, a.ra);
   }
-  const bf16_t* dw = a.decay_w + (size_t)(h * K + 16 * w + fr) * a.ra + 8 * fg;
-  const bf16_t* gw = a.gate_w + (size_t)(h * a.V + 16 * w + fr) * a.rg + 8 * fg;
-  bf16x8_t wd[RS], vd[RS];
-  auto ask = [&](bool on, const bf16_t* p, int at, int rank) {
-#pragma unroll
-    for (int s = 0; s < RS; ++s)
-      if (on && 32 * s < rank) {
-        wd[s] = *(const bf16x8_t*)(p + 32 * s);
-        vd[s] = *(const bf16x8_t*)(row + at + 32 * s + 8 * fg);
-      }
-  };
-  auto product = [&](const bf16_t* p, int at, int rank) {
-    f32x4_t z{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < RS; ++s)
-      if (32 * s < rank) z = mfma16(wd[s], vd[s], z);
-    for (int k = 32 * RS; k < rank; k += 32) z = mfma16(*(const bf16x8_t*)(p + k), *(const bf16x8_t*)(row + at + k + 8 * fg), z);
-    return fr == 0 ? z[0] : fr == 1 ? z[1] : fr == 2 ? z[2] : z[3];
-  };
-  ask(dec, dw, a.at_decay, a.ra);
   asm volatile("" ::: "memory");  // issue order: the state behind them
 
   // ---- the state: columns NC grp .. of V, 4 channels at 32 i + 4 g ----
   const int g = tid % LN, grp = tid / LN;
   f32x4_t S[NC][NS4];
-  float* st[NC];
-  bool live[NC];
+  float* st = a.state + (slot * a.H + h) * a.V * K;
+  const __amdgpu_buffer_rsrc_t rs = rsrc(st, stored ? a.V * K * 4 : 0), rst = rsrc(st, a.V * K * 4);
+  int at[NC];  // (columns past V: outside the resource)
 #pragma unroll
   for (int j = 0; j < NC; ++j) {
-    const int c = grp * NC + j;
-    live[j] = c < a.V;
-    st[j] = a.state + ((slot * a.H + h) * a.V + min(c, a.V - 1)) * K + g * 4;
+    at[j] = ((grp * NC + j) * K + g * 4) * 4;
 #pragma unroll
-    for (int i = 0; i < NS4; ++i) S[j][i] = stored ? *(const f32x4_t*)(st[j] + i * LN * 4) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < NS4; ++i)
+      S[j][i] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, at[j] + i * LN * 16, 0, 0));
   }
   asm volatile("" ::: "memory");
 
-  if (w < 2) {
-    f32x4_t v{0.f, 0.f, 0.f, 0.f};
+  if (part < 3) {
+    float v = 0.f;
     if (conv) {
 #pragma unroll
-      for (int i = 0; i < TAPS; ++i) {
-        const f32x4_t xi{__uint_as_float(x[i][0] << 16), __uint_as_float(x[i][0] & 0xffff0000u), __uint_as_float(x[i][1] << 16),
-                         __uint_as_float(x[i][1] & 0xffff0000u)};
+      for (int i = 0; i < TAPS; ++i) v = fmaf(cw[i], bf2f(x[i]), v);
+      v = bf2f(f2bf(act_silu<bf16_t>(v)));  // (rounded as the convolution's own launch stores it)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = fmaf(cw[i][e], xi[e], v[e]);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = bf2f(f2bf(act_silu<bf16_t>(v[e])));  // (rounded as the convolution's own launch stores it)
-#pragma unroll
-      for (int i = 0; i + 1 < TAPS; ++i) *(u32x2_t*)(cs + (size_t)i * a.C) = x[i + 1];
+      for (int i = 0; i + 1 < TAPS; ++i) cs[i * a.C + cc] = x[i + 1];
     }
-    float ss = 0.f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ss = fmaf(v[e], v[e], ss);
-    ss = lanes_sum<32>(ss);
-    const float f = part == 2 ? 1.f : (part == 0 ? a.q_scale : 1.f) / sqrtf(ss + a.unit_eps);
-    if (conv) *(f32x4_t*)((part == 0 ? sq : part == 1 ? sk : sv) + 4 * sl) = v * f;
-    if (tid == 96) sb[0] = sigmoid32(bf2f(row[a.at_beta + h]));
+    sx[part][pc] = v;
+    if (part < 2) {
+      const float q = wave_sum(v * v);
+      if (lane == 0) ss[w] = q;
+    }
   }
+  if (tid == 511) sb[0] = sigmoid32(bf2f(load16(row, (a.at_beta + h) * 2)));
   if (dec) {
-    const float z = product(dw, a.at_decay, a.ra);
+    const float z = product(dw, dat, a.at_decay, a.ra);
     if (fr < 4) sa[ch] = __builtin_amdgcn_exp2f(softplus32(z + dtb) * rate);
   }
-  ask(gat, gw, a.at_gate, a.rg);  // (the gates are needed last)
+  if (gat) ask(gw, gat_, a.at_gate, 0, a.rg);  // (the gates are needed last)
   asm volatile("" ::: "memory");
   lds_barrier();
 
-  f32x4_t kv[NS4];
+  const float fq = a.q_scale / sqrtf(ss[0] + ss[1] + a.unit_eps), fk = 1.f / sqrtf(ss[2] + ss[3] + a.unit_eps);
   float held[NC], out[NC], u[NC];
 #pragma unroll
   for (int j = 0; j < NC; ++j) held[j] = out[j] = 0.f;
 #pragma unroll
   for (int i = 0; i < NS4; ++i) {
-    kv[i] = *(const f32x4_t*)(sk + i * LN * 4 + g * 4);
-    const f32x4_t d = *(const f32x4_t*)(sa + i * LN * 4 + g * 4);
+    if (i == 2) asm volatile("" ::: "memory");  // (no registers for all of them at once)
+    const f32x4_t kv = *(const f32x4_t*)(sx[1] + i * LN * 4 + g * 4), d = *(const f32x4_t*)(sa + i * LN * 4 + g * 4);
 #pragma unroll
     for (int j = 0; j < NC; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         S[j][i][e] *= d[e];
-        held[j] = fmaf(S[j][i][e], kv[i][e], held[j]);
+        held[j] = fmaf(S[j][i][e], kv[e], held[j]);
       }
   }
   const float beta = sb[0];
 #pragma unroll
-  for (int j = 0; j < NC; ++j) u[j] = beta * (sv[min(grp * NC + j, a.V - 1)] - lanes_sum<LN>(held[j]));
+  for (int j = 0; j < NC; ++j) u[j] = fk * beta * fmaf(-fk, lanes_sum<LN>(held[j]), sx[2][grp * NC + j]);
 #pragma unroll
   for (int i = 0; i < NS4; ++i) {
-    const f32x4_t q = *(const f32x4_t*)(sq + i * LN * 4 + g * 4);
+    if (i == 0 || i == 2) asm volatile("" ::: "memory");
+    const f32x4_t kv = *(const f32x4_t*)(sx[1] + i * LN * 4 + g * 4), q = *(const f32x4_t*)(sx[0] + i * LN * 4 + g * 4);
 #pragma unroll
     for (int j = 0; j < NC; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        S[j][i][e] = fmaf(kv[i][e], u[j], S[j][i][e]);
+        S[j][i][e] = fmaf(kv[e], u[j], S[j][i][e]);
         out[j] = fmaf(S[j][i][e], q[e], out[j]);
       }
   }
 #pragma unroll
   for (int j = 0; j < NC; ++j) {
     out[j] = lanes_sum<LN>(out[j]);
-    if (g == 0) so[grp * NC + j] = live[j] ? out[j] : 0.f;
-    if (live[j])
+    if (g == 0) so[grp * NC + j] = grp * NC + j < a.V ? fq * out[j] : 0.f;
 #pragma unroll
-      for (int i = 0; i < NS4; ++i) *(f32x4_t*)(st[j] + i * LN * 4) = S[j][i];
+    for (int i = 0; i < NS4; ++i)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, S[j][i]), rst, at[j] + i * LN * 16, 0, 0);
   }
   if (gat) {
-    const float z = product(gw, a.at_gate, a.rg);
+    const float z = product(gw, gat_, a.at_gate, a.rg);
     if (fr < 4) sg[ch] = sigmoid32(z);
   }
   lds_barrier();
-  if (w) return;
-  const f32x4_t v = *(const f32x4_t*)(so + 4 * sl);
-  float ss = 0.f;
+  if (w || lane >= 32) return;
+  const f32x4_t v = *(const f32x4_t*)(so + 4 * lane);
+  float sq = 0.f;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) ss = fmaf(v[e], v[e], ss);
-  ss = lanes_sum<32>(ss);
+  for (int e = 0; e < 4; ++e) sq = fmaf(v[e], v[e], sq);
+  sq = lanes_sum<32>(sq);
   if (lane >= a.V / 4) return;
-  const float inv = 1.f / sqrtf(ss / a.dim + a.eps);
+  const float inv = 1.f / sqrtf(sq / a.dim + a.eps);
   const f32x4_t nw = *(const f32x4_t*)(a.norm + 4 * lane), gt = *(const f32x4_t*)(sg + 4 * lane);
   f32x4_t r;
 #pragma unroll
