@@ -10,13 +10,17 @@
 // the layernorm kernel stores.
 //
 // What bounds it is latency: 12 layers' 170 MB are 35 us at HBM's rate, a launch is 4 - 5. So a workgroup is a strip of
-// 16 columns (48 - 256 of them) whose up to 16 waves share K in units of 64, operands go from global memory straight to
-// the MFMA, everything that a wave needs is requested before the first wait (the statistics first: they are merged while
-// the weights are on their way), and the waves' sums meet in LDS once.
-// 32 rows of 12 layers of 768 x 3072 columns: 4.8 us (K = 768), 5.9 (a norm on A), 6.9 (and GELU) and 8.5 (K = 3072) a
-// launch, the question 485 -> 403 us; a dk product, a norm, or a split-K product with its reduce took 5.2 / 7.1, 4.6 and
-// 9.7.
+// 16 columns (48 - 256 of them) whose up to 16 waves take K in units of 64 in turn, and the waves' sums meet in LDS once. A unit
+// arrives by LDS-DMA, 128 B of every row, into a stage that is the wave's own: a CU has 256 requests on their way, and
+// operands straight in MFMA layout are requests of 64 B, twice as many. A wave waits for its own transfers only; the statistics
+// are asked for first and merged while the weights are on their way.
+// 21 rows of 12 layers of 768 x 3072 columns, us a launch, operands straight to the MFMA / by LDS-DMA: K = 3072 8.7 / 6.2, a norm
+// on A 6.3 / 5.4 (without GELU) and 6.7 / 5.9 (with it), K = 768 4.2 / 4.3; the question 375 -> 333 us, 60 tokens through 24
+// layers of 1024 in fp16 1028 -> 926, 16 + 20 through 384 columns 315 -> 311. A dk product, a norm, or a split-K product with
+// its reduce took 5.2 / 7.1, 4.6 and 9.7.
 #include "gemm.h"
+
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 struct EncRowsArgs {
   const bf16_t *A, *W, *bias, *resid;
@@ -28,13 +32,19 @@ struct EncRowsArgs {
   float eps;
 };
 
-// PFU: units of 64 k that a wave has in flight
-template <typename T, int FM, bool LNA, int EPI, int PFU>
-__global__ void __launch_bounds__(1024)
+// The waves' stages (ST of each) and, after the last unit, their sums share LDS: up to enc_waves(FM) waves.
+constexpr int enc_waves(int fm) { return fm == 4 ? 12 : 16; }
+constexpr int enc_stages(int fm) { return fm == 1 ? 2 : 1; }
+
+template <typename T, int FM, bool LNA, int EPI>
+__global__ void __launch_bounds__(64 * enc_waves(FM))
 enc_rows_kernel(EncRowsArgs p) {
-  constexpr int ROWS = FM * 16, SLD = 20;
-  __shared__ __attribute__((aligned(16))) float red[16][ROWS][SLD];
+  constexpr int ROWS = FM * 16, SLD = 20, ST = enc_stages(FM), A_BYTES = ROWS * 128, STAGE = A_BYTES + 2048;
+  constexpr int PA = 2 * FM, P = PA + 2;  // LDS-DMA instructions of a stage
+  static_assert(ROWS * SLD * 4 <= ST * STAGE, "the sums fit the stages");
+  __shared__ __attribute__((aligned(16))) char smem[enc_waves(FM) * ST * STAGE];
   __shared__ float smean[ROWS], srstd[ROWS];
+  float (*red)[ROWS][SLD] = (float (*)[ROWS][SLD])smem;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
   const int fr = lane & 15, fg = lane >> 4;
   const int n0 = blockIdx.x * 16, units = p.K / 64;
@@ -89,28 +99,42 @@ enc_rows_kernel(EncRowsArgs p) {
     }
   }
   asm volatile("" ::: "memory");
-  bf16x8_t wf[PFU][2], af[PFU][2][FM], gf[2], bf[2];
-  auto load = [&](int u0) __attribute__((always_inline)) {
+  // ---- the wave's units w, w + nw, ..: row r's 16-B chunk c of 64 k at slot c ^ (r >> 1 & 7) of its 128 B ----
+  unsigned ao[8], wo[2];  // rows past M: past the resource's end, which reads as zero
 #pragma unroll
-    for (int j = 0; j < PFU; ++j) {
-      const int k = min(u0 + nw * j, units - 1) * 64 + fg * 8;  // (past the end: the last unit again, not used)
+  for (int j = 0; j < PA; ++j) {
+    const int r = 8 * j + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+    ao[j] = r < p.M ? (unsigned)r * (unsigned)(p.lda * 2) + c * 16 : 0x7ffffff0u;
+  }
 #pragma unroll
-      for (int h = 0; h < 2; ++h) wf[j][h] = *(const bf16x8_t*)(p.W + (size_t)(n0 + fr) * p.K + k + 32 * h);
+  for (int j = 0; j < 2; ++j) {
+    const int r = 8 * j + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+    wo[j] = (unsigned)r * (unsigned)(p.K * 2) + c * 16;
+  }
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, (short)0, 0x7fffff00, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)(p.W + (size_t)n0 * p.K), (short)0, 0x7fffff00, 0x00020000);
+  char* ring = smem + w * ST * STAGE;
+  auto ask = [&](int u, int slot) __attribute__((always_inline)) {
+    char* base = ring + slot * STAGE;
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+    for (int j = 0; j < 2; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t)(base + A_BYTES + j * 1024), 16, wo[j], u * 128, 0, 0);
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
-          af[j][h][i] = *(const bf16x8_t*)(p.A + (size_t)min(16 * i + fr, p.M - 1) * p.lda + k + 32 * h);
-      if constexpr (LNA) {
+    for (int j = 0; j < PA; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(base + j * 1024), 16, ao[j & 7], u * 128, 0, 0);
+  };
+  bf16x8_t gf[2], bf[2];
+  auto norm_load = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          gf[h] = *(const bf16x8_t*)(p.g + k + 32 * h);
-          bf[h] = *(const bf16x8_t*)(p.b + k + 32 * h);
-        }
-      }
+    for (int h = 0; h < 2; ++h) {
+      gf[h] = *(const bf16x8_t*)(p.g + u * 64 + fg * 8 + 32 * h);
+      bf[h] = *(const bf16x8_t*)(p.b + u * 64 + fg * 8 + 32 * h);
     }
   };
-  load(w);
+  if constexpr (LNA) norm_load(min(w, units - 1));
+#pragma unroll
+  for (int i = 0; i < ST; ++i)
+    if (w + i * nw < units) ask(w + i * nw, i);
   if (p.st) {
     asm volatile("" ::: "memory");
     stats_merge(4 * w + fg);
@@ -118,37 +142,53 @@ enc_rows_kernel(EncRowsArgs p) {
       stats_load(r);
       stats_merge(r);
     }
-    __syncthreads();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the transfers stay on their way)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
   }
   f32x4_t acc[FM];
 #pragma unroll
   for (int i = 0; i < FM; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int u0 = w;;) {
+  const int sw = (fr >> 1) & 7;
+  const int co[2] = {(fg ^ sw) << 4, ((4 + fg) ^ sw) << 4};
+#pragma unroll 1
+  for (int u = w, slot = 0; u < units; u += nw) {
+    if (LNA && u != w) norm_load(u);
+    // this unit is in: everything but the stage behind it (with a norm: everything)
+    if (!LNA && ST > 1 && u + nw < units) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(P * (ST - 1)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    const char* s = ring + slot * STAGE + fr * 128;
+    bf16x8_t wf[2], af[2][FM];
 #pragma unroll
-    for (int j = 0; j < PFU; ++j) {
-      if (u0 + nw * j >= units) continue;
+    for (int h = 0; h < 2; ++h) {
+      wf[h] = *(const bf16x8_t*)(s + A_BYTES + co[h]);
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-          bf16x8_t a = af[j][h][i];
-          if constexpr (LNA) {
-            const float mean = smean[16 * i + fr], rstd = srstd[16 * i + fr];
-            u32x4_t y;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              y[e] = T::pack2(fmaf((T::to_f((bf16_t)a[2 * e]) - mean) * rstd, T::to_f((bf16_t)gf[h][2 * e]), T::to_f((bf16_t)bf[h][2 * e])),
-                              fmaf((T::to_f((bf16_t)a[2 * e + 1]) - mean) * rstd, T::to_f((bf16_t)gf[h][2 * e + 1]),
-                                   T::to_f((bf16_t)bf[h][2 * e + 1])));
-            a = __builtin_bit_cast(bf16x8_t, y);
-          }
-          acc[i] = T::mma16(wf[j][h], a, acc[i]);  // (W first: a lane has 4 columns of a row)
-        }
+      for (int i = 0; i < FM; ++i) af[h][i] = *(const bf16x8_t*)(s + i * 2048 + co[h]);
     }
-    u0 += nw * PFU;
-    if (u0 >= units) break;
-    load(u0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and read: its stage is free
+    __builtin_amdgcn_sched_barrier(0);
+    if (u + ST * nw < units) ask(u + ST * nw, slot);
+    slot = slot + 1 == ST ? 0 : slot + 1;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        bf16x8_t a = af[h][i];
+        if constexpr (LNA) {
+          const float mean = smean[16 * i + fr], rstd = srstd[16 * i + fr];
+          u32x4_t y;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            y[e] = T::pack2(fmaf((T::to_f((bf16_t)a[2 * e]) - mean) * rstd, T::to_f((bf16_t)gf[h][2 * e]), T::to_f((bf16_t)bf[h][2 * e])),
+                            fmaf((T::to_f((bf16_t)a[2 * e + 1]) - mean) * rstd, T::to_f((bf16_t)gf[h][2 * e + 1]),
+                                 T::to_f((bf16_t)bf[h][2 * e + 1])));
+          a = __builtin_bit_cast(bf16x8_t, y);
+        }
+        acc[i] = T::mma16(wf[h], a, acc[i]);  // (W first: a lane has 4 columns of a row)
+      }
   }
+  __syncthreads();
 #pragma unroll
   for (int i = 0; i < FM; ++i) *(f32x4_t*)&red[w][16 * i + fr][4 * fg] = acc[i];
   __syncthreads();
@@ -192,19 +232,14 @@ enc_rows_kernel(EncRowsArgs p) {
 
 template <typename T, int FM>
 static int enc_rows_launch(const EncRowsArgs& a, int epi, hipStream_t s) {
-  // as many waves as share the units of 64 k evenly, up to 16; at least FM (4 threads an output row)
-  const int units = a.K / 64, per = (units + 15) / 16;
+  // as many waves as share the units of 64 k evenly; at least FM (4 threads an output row)
+  const int units = a.K / 64, per = (units + enc_waves(FM) - 1) / enc_waves(FM);
   const dim3 grid(a.N / 16, (a.M + FM * 16 - 1) / (FM * 16)), block(max((units + per - 1) / per, FM) * 64);
-#define ENC_ROWS(LNA, E, PFU) enc_rows_kernel<T, FM, LNA, E, PFU><<<grid, block, 0, s>>>(a)
-  if (epi == EPI_RESID) {  // (a unit past the end costs what one within it does)
-    if (per == 1) ENC_ROWS(false, EPI_RESID, 1);
-    else if (per == 2 || FM == 4 || (FM == 2 && per != 3)) ENC_ROWS(false, EPI_RESID, 2);
-    else if (per == 3) ENC_ROWS(false, EPI_RESID, FM == 4 ? 2 : 3);
-    else ENC_ROWS(false, EPI_RESID, FM == 1 ? 4 : 2);
-  }
-  else if (epi == EPI_GELU && a.st) ENC_ROWS(true, EPI_GELU, 1);
-  else if (epi == EPI_BIAS && a.st) ENC_ROWS(true, EPI_BIAS, 1);
-  else if (epi == EPI_BIAS) ENC_ROWS(false, EPI_BIAS, 1);
+#define ENC_ROWS(LNA, E) enc_rows_kernel<T, FM, LNA, E><<<grid, block, 0, s>>>(a)
+  if (epi == EPI_RESID) ENC_ROWS(false, EPI_RESID);
+  else if (epi == EPI_GELU && a.st) ENC_ROWS(true, EPI_GELU);
+  else if (epi == EPI_BIAS && a.st) ENC_ROWS(true, EPI_BIAS);
+  else if (epi == EPI_BIAS) ENC_ROWS(false, EPI_BIAS);
   else return (int)hipErrorInvalidValue;
 #undef ENC_ROWS
   return (int)hipGetLastError();
@@ -228,6 +263,7 @@ DA_EXPORT int da_enc_rows(const void* A, int lda, const void* W, void* C, int ld
   if (M < 1 || M > 64 || K < 64 || K % 64 || N < 16 || N % 16 || lda % 8 || ldc % 4 || (st && (!g || !b || width > 1024 || width % 16)))
     return (int)hipErrorInvalidValue;
   if (epi == EPI_RESID && (!resid || ldr % 4 || !st_out || N > 1024)) return (int)hipErrorInvalidValue;
+  if (2ll * ((M - 1) * (long long)lda + K) > 0x7ffff000ll || 32ll * K > 0x7ffff000ll) return (int)hipErrorInvalidValue;  // (32-bit offsets)
   EncRowsArgs a{(const bf16_t*)A, (const bf16_t*)W, (const bf16_t*)bias, (const bf16_t*)resid, (bf16_t*)C, st,
                 (const bf16_t*)g, (const bf16_t*)b, st_out, M, N, K, lda, ldc, ldr, width / 16, eps};
   hipStream_t s = (hipStream_t)stream;
