@@ -43,20 +43,36 @@ struct DkArgs {
   int relu;  // EPI_SWIGLU: the gate's activation is relu, not silu
 };
 
+// The values of four neighbours, as two words.
+template <typename T> __device__ __forceinline__ f32x4_t unpack4(const u32x2_t& u) {
+  return f32x4_t{T::to_f((bf16_t)(u[0] & 0xffff)), T::to_f((bf16_t)(u[0] >> 16)), T::to_f((bf16_t)(u[1] & 0xffff)), T::to_f((bf16_t)(u[1] >> 16))};
+}
+
 // ST stages of a wave's ring, each BM rows of A and BN of W; row r's 16-B chunk c at slot c ^ (r >> 1 & 7), so that the 16
 // rows of a fragment read land on all banks
-template <int FM, int FN, int NW, int ST, int EPI>
+// ROWS: more than one block of BM rows (gridDim.y of them; W's lines are worth a place in the caches then). The blocks of a column
+// tile are neighbours on one XCD.
+template <int FM, int FN, int NW, int ST, int EPI, typename T, bool ROWS>
 __global__ void __launch_bounds__(64 * NW)
 gemm_dk_kernel(DkArgs p) {
   constexpr int BM = 16 * FM, BN = 16 * FN, A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128;
   constexpr int PA = BM / 8, PW = BN / 8, P = PA + PW;  // LDS-DMA instructions of a stage
   constexpr int SLD = BN + 4, RED = NW * BM * SLD * 4;
   constexpr int RING = NW * ST * STAGE, SUMS = RED + NW * 64 * 4;
-  static_assert(P * ST < 64 && PA <= 8 && PW <= 8, "tile");
+  static_assert(P * ST < 64 && PA <= 8 && PW <= 16, "tile");
   __shared__ __attribute__((aligned(16))) char smem[RING > SUMS ? RING : SUMS];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fg = lane >> 4;
-  const int tile = blockIdx.x, n0 = tile * BN, nk = p.K / 64;
+  int tile = blockIdx.x;
+  if constexpr (ROWS) {
+    const int t = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y), m0 = t % (int)gridDim.y * BM;
+    tile = t / (int)gridDim.y;
+    p.M -= m0;
+    p.A += (size_t)m0 * p.lda;
+    p.C += (size_t)m0 * p.ldc;
+    if (EPI == EPI_RESID) p.resid += (size_t)m0 * p.ldr;
+  }
+  const int n0 = tile * BN, nk = p.K / 64;
 
   // deferred norm: thread = (part, 4 rows), 8 parts each on their way before the ring's first stages
   constexpr int RQ = FM == 3 ? 16 : BM / 4, PL = 64 * NW / RQ;  // row quads (a power of two), parts at a time
@@ -66,7 +82,7 @@ gemm_dk_kernel(DkArgs p) {
     for (int j = 0; j < 8; ++j)
       sq[j] = *(const f32x4_t*)(p.ssq_in + (size_t)min(tid / RQ + j * PL, p.ssq_parts - 1) * 64 + tid % RQ * 4);
 
-  unsigned ao[8], wo[8];  // rows past the operands': past the resource's end, which reads as zero
+  unsigned ao[8], wo[16];  // rows past the operands': past the resource's end, which reads as zero
 #pragma unroll
   for (int j = 0; j < PA; ++j) {
     const int r = 8 * j + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
@@ -90,7 +106,7 @@ gemm_dk_kernel(DkArgs p) {
     char* base = ring + slot * STAGE;
 #pragma unroll
     for (int j = 0; j < PW; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t)(base + A_BYTES + j * 1024), 16, wo[j & 7], step * 128, 0, 2);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t)(base + A_BYTES + j * 1024), 16, wo[j & 15], step * 128, 0, ROWS ? 0 : 2);
 #pragma unroll
     for (int j = 0; j < PA; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(base + j * 1024), 16, ao[j & 7], step * 128, 0, 0);
@@ -143,7 +159,7 @@ gemm_dk_kernel(DkArgs p) {
 #pragma unroll
       for (int q = 0; q < FM; ++q)
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[q][j] = mfma16(wf[h][j], af[h][q], acc[q][j]);  // (W first: a lane has 4 columns of a row)
+        for (int j = 0; j < FN; ++j) acc[q][j] = T::mma16(wf[h][j], af[h][q], acc[q][j]);  // (W first: a lane has 4 columns of a row)
     slot = slot + 1 == ST ? 0 : slot + 1;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (transfers past the end write zeros)
@@ -160,7 +176,7 @@ gemm_dk_kernel(DkArgs p) {
 
   constexpr int BNO = EPI == EPI_SWIGLU ? BN / 2 : BN;  // output columns of the tile
   constexpr int CPR = BNO / 4;                          // 4-column pieces of a row
-  static_assert(EPI != EPI_RESID || (CPR & (CPR - 1)) == 0, "a row's pieces meet by lane exchange");
+  static_assert(EPI != EPI_RESID || ROWS || (CPR & (CPR - 1)) == 0, "a row's pieces meet by lane exchange");
 #pragma unroll 1
   for (int t = tid; t < BM * CPR; t += 64 * NW) {
     const int m = t / CPR, c = t % CPR * 4;
@@ -178,9 +194,7 @@ gemm_dk_kernel(DkArgs p) {
       return v;
     };
     auto bias4 = [&](int col) {  // columns of the product
-      const u32x2_t b = p.bias ? *(const u32x2_t*)(p.bias + col) : u32x2_t{0, 0};
-      return f32x4_t{__uint_as_float(b[0] << 16), __uint_as_float(b[0] & 0xffff0000u), __uint_as_float(b[1] << 16),
-                     __uint_as_float(b[1] & 0xffff0000u)};
+      return p.bias ? unpack4<T>(*(const u32x2_t*)(p.bias + col)) : f32x4_t{0.f, 0.f, 0.f, 0.f};
     };
     const int gn = EPI == EPI_SWIGLU ? n0 / 2 + c : n0 + c;
     const bool ok = m < p.M && gn < (EPI == EPI_SWIGLU ? p.N / 2 : p.N);
@@ -196,22 +210,18 @@ gemm_dk_kernel(DkArgs p) {
       const f32x4_t x = total(c), b = bias4(gn);
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = fmaf(x[e], inv, b[e]);
-      if constexpr (EPI == EPI_RESID) {
-        const u32x2_t r = *(const u32x2_t*)(p.resid + (size_t)m * p.ldr + gn);
-        v += f32x4_t{__uint_as_float(r[0] << 16), __uint_as_float(r[0] & 0xffff0000u), __uint_as_float(r[1] << 16),
-                     __uint_as_float(r[1] & 0xffff0000u)};
-      }
-    }
-    const u32x2_t o{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
-    if (ok) *(u32x2_t*)(p.C + (size_t)m * p.ldc + gn) = o;
-    if constexpr (EPI == EPI_RESID) {
-      if (p.ssq_out) {  // sum of squares of the bf16 values the stream now holds
-        float q = 0.f;
+      if constexpr (EPI == EPI_GELU) {
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const float lo = __uint_as_float(o[e] << 16), hi = __uint_as_float(o[e] & 0xffff0000u);
-          q += lo * lo + hi * hi;
-        }
+        for (int e = 0; e < 4; ++e) v[e] = gelu_erf(v[e]);
+      }
+      if constexpr (EPI == EPI_RESID) v += unpack4<T>(*(const u32x2_t*)(p.resid + (size_t)m * p.ldr + gn));
+    }
+    const u32x2_t o{T::pack2(v[0], v[1]), T::pack2(v[2], v[3])};
+    if (ok) *(u32x2_t*)(p.C + (size_t)m * p.ldc + gn) = o;
+    if constexpr (EPI == EPI_RESID && !ROWS) {
+      if (p.ssq_out) {  // sum of squares of the bf16 values the stream now holds
+        const f32x4_t x = unpack4<T>(o);
+        float q = (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
         if (!ok) q = 0.f;
 #pragma unroll
         for (int x = 1; x < CPR; x <<= 1) q += __shfl_xor(q, x, 64);
@@ -232,7 +242,7 @@ template <int FM, int FN, int EPI>
 static int dk_launch3(const DkArgs& a, hipStream_t s) {
   // four waves, as many stages as leave a CU room for two workgroups; at least two, of which one is read
   constexpr int STAGE = (FM + FN) * 2048, FIT = 81920 / (4 * STAGE), ST = FIT < 2 ? 2 : FIT > 4 ? 4 : FIT;
-  gemm_dk_kernel<FM, FN, 4, ST, EPI><<<(a.N + 16 * FN - 1) / (16 * FN), 256, 0, s>>>(a);
+  gemm_dk_kernel<FM, FN, 4, ST, EPI, BF16T, false><<<(a.N + 16 * FN - 1) / (16 * FN), 256, 0, s>>>(a);
   return (int)hipGetLastError();
 }
 
@@ -284,4 +294,55 @@ DA_EXPORT int da_gemm_dk(const void* A, int lda, const void* W, void* C, int ldc
   if (M <= 32) return dk_launch1<2>(a, epi, s);
   if (M <= 48) return dk_launch1<3>(a, epi, s);
   return dk_launch1<4>(a, epi, s);
+}
+
+template <int FM, int FN, int ST, typename T>
+static int dk_rows(const DkArgs& a, int epi, hipStream_t s) {
+  const dim3 grid((a.N + 16 * FN - 1) / (16 * FN), (a.M + 16 * FM - 1) / (16 * FM));
+#define DK_ROWS(E) gemm_dk_kernel<FM, FN, 4, ST, E, T, true><<<grid, 256, 0, s>>>(a)
+  switch (epi) {
+    case EPI_NONE: case EPI_BIAS: DK_ROWS(EPI_NONE); break;
+    case EPI_GELU: DK_ROWS(EPI_GELU); break;
+    case EPI_RESID: DK_ROWS(EPI_RESID); break;
+    case EPI_SWIGLU:
+      if constexpr (FN % 2 == 0 && !T::kF16) {
+        DK_ROWS(EPI_SWIGLU);
+        break;
+      }
+      return (int)hipErrorInvalidValue;
+    default: return (int)hipErrorInvalidValue;
+  }
+#undef DK_ROWS
+  return (int)hipGetLastError();
+}
+
+template <typename T>
+static int dk_rows_tile(const DkArgs& a, int epi, int tile, hipStream_t s) {
+  switch (tile) {
+    case 20: return dk_rows<2, 1, 3, T>(a, epi, s);
+    case 21: return dk_rows<2, 2, 2, T>(a, epi, s);
+    case 22: return dk_rows<4, 2, 2, T>(a, epi, s);
+    case 23: return dk_rows<4, 3, 2, T>(a, epi, s);
+    case 24: return dk_rows<4, 4, 2, T>(a, epi, s);
+    case 25: return dk_rows<4, 6, 2, T>(a, epi, s);
+    default: return (int)hipErrorInvalidValue;
+  }
+}
+
+// More rows than a block, by tiles of their own (kernels.py, _DK_TILES): 20 = 32x16, 21 = 32x32, 22 = 64x32, 23 = 64x48, 24 = 64x64,
+// 25 = 64x96. epi: NONE / BIAS / GELU / RESID, bf16 also SWIGLU / REGLU (N % 32 == 0; not tiles 20 and 23). K % 64 == 0, N % 8 == 0,
+// bf16 or fp16 (f16) throughout.
+DA_EXPORT int da_gemm_dk_rows(const void* A, int lda, const void* W, void* C, int ldc, const void* bias, const void* resid, int ldr,
+                              int M, int N, int K, int epi, int tile, int f16, void* stream) {
+  const int relu = epi == EPI_REGLU;
+  if (relu) epi = EPI_SWIGLU;
+  if (M < 1 || M > 65535 * 32 || K < 64 || K % 64 || N < 8 || N % 8 || lda % 8 || ldc % 4 || (epi == EPI_SWIGLU && N % 32) ||
+      (epi == EPI_RESID && (!resid || ldr % 4)))
+    return (int)hipErrorInvalidValue;
+  if (2ll * (63 * (long long)lda + K) > 0x7ffff000ll || 2ll * 96 * K > 0x7ffff000ll) return (int)hipErrorInvalidValue;
+  DkArgs a{};
+  a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = (bf16_t*)C;
+  a.bias = (const bf16_t*)bias; a.resid = (const bf16_t*)resid;
+  a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc; a.ldr = ldr; a.relu = relu;
+  return f16 ? dk_rows_tile<F16T>(a, epi, tile, (hipStream_t)stream) : dk_rows_tile<BF16T>(a, epi, tile, (hipStream_t)stream);
 }

@@ -64,6 +64,7 @@ _SIGS = {
     "da_gemm_dk": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                    c_int, c_void_p, c_int, c_int, c_float, c_void_p, c_void_p],
     "da_gemm_dk_parts": [c_int],
+    "da_gemm_dk_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 7 + [c_void_p],
     "da_enc_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5
                   + [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_void_p],
     "da_gemm_tail_ws": [c_int] * 5,
@@ -342,6 +343,11 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
         return out
     if (tile == 12 or (tile == 0 and splits <= 0)) and rms is None and dk_fusable(M, N, K, epi):
         return gemm_dk(a, w, epi=epi, bias=bias, resid=resid, out=out)
+    if tile == 0 and splits <= 0 and rms is None and max(K, a.stride(0)) < 1 << 22:
+        tile = _dk_rows_tile(M, N, K, epi)
+    if tile in _DK_TILES:
+        _req(rms is None and splits <= 1, "gemm_dk rows: whole, without a norm")
+        return _gemm_dk_rows(a, w, bias, epi, resid, out, tile)
     if tile == 0 and splits <= 0 and gemv_fusable(M, N, K, epi):
         tile, splits = 6, 1  # batch-1 decode: weight-streaming GEMV, one launch, no split-K workspace
     gamma, eps = (None, 0.0) if rms is None else rms  # rms = (gain or None for unit gain, eps > 0)
@@ -690,6 +696,13 @@ ROW_TILES_BELOW = 1280
 # Not 2600 x 1024 x 1024 (18.1 / 19.2), 1600 x 4096 x 1024 (24.5 / 28.3) or 2000 x 3072 x 768 (20.3 / 22.4).
 # Of 44 products that it takes, bf16 and fp16, 43 run in 0.49 - 1.00 of the time and one in 1.07 (1700 x 1024 x 4096 with a residual).
 SMALL_RESULT_ROWS, SMALL_RESULT = 5120, 21 << 18
+# Tiles of csrc/gemm_dk.hip for more than 64 rows, where K is shared out within a workgroup and nothing waits for a barrier: code ->
+# 16-row groups, 16-column groups, workgroups of a CU at a time, and us: start and end, each further round, a K-step of 64 of a round,
+# of a CU's workgroup, of a workgroup on 1/256 of the chip, a million weights. Fitted, with no cost below zero, to 338 products of 72 -
+# 1280 rows (26 projections, feed-forwards and encoder layers 320 - 16384 wide, weights cold): off by 5 - 7 % on average.
+_DK_TILES = {20: (2, 1, 2, 3.52, 1.42, 0.0, 0.037, 0.033, 0.097), 21: (2, 2, 2, 3.45, 1.12, 0.0, 0.057, 0.039, 0.174),
+             22: (4, 2, 1, 3.88, 1.78, 0.093, 0.0, 0.068, 0.056), 23: (4, 3, 1, 4.29, 2.06, 0.111, 0.0, 0.074, 0.098),
+             24: (4, 4, 1, 4.76, 2.50, 0.132, 0.0, 0.076, 0.148), 25: (4, 6, 1, 5.81, 3.40, 0.172, 0.0, 0.078, 0.202)}
 
 
 def _row_tiles_ok(M: int, N: int) -> bool:
@@ -741,6 +754,36 @@ def _row_us(M: int, N: int, K: int, epi: int = EPI_NONE, f16: bool = False):
 def _row_tile(M: int, N: int, K: int, epi: int = EPI_NONE, f16: bool = False):
     """(tile, splits) of such a product."""
     return _row_us(M, N, K, epi, f16)[1:]
+
+
+@_rule
+def _dk_rows_tile(M: int, N: int, K: int, epi: int = EPI_NONE, f16: bool = False) -> int:
+    """The tile of ``_DK_TILES`` that a product of 65 rows to ROW_TILES_BELOW runs on, 0: those of ``_row_tile`` are faster. Where the
+    estimate is 3 % below theirs, 10 % from 257 rows on, 15 % where K is above 4096 (768 x 320 x 8192 is not: 15.9 / 19.0 us): 155 of
+    the 338 products that it is fitted to, in 0.76 of their time, four of them in 1.02 - 1.03. us, tiles of ``_row_tile`` -> these: 128 x 384 x 1536 8.9 ->
+    4.3, 256 x 768 x 768 6.6 -> 4.3, 256 x 768 x 3072 12.2 -> 7.6, 256 x 1024 x 4096 13.8 -> 8.8, 128 x 4096 x 1024 8.1 -> 6.3,
+    640 x 1024 x 1024 8.2 -> 6.9; 96 x 3072 x 3072 13.0 -> 9.6, 128 x 4096 x 4096 19.8 -> 15.8, 128 x 9216 x 3072 27.4 -> 23.9."""
+    if not 64 < M < ROW_TILES_BELOW:
+        return 0
+    best, ksteps = None, K // 64
+    for t, (fm, fn, beside, start, again, step, wg, load, weights) in _DK_TILES.items():
+        if epi in GATED and fn % 2:
+            continue
+        units = math.ceil(M / (16 * fm)) * math.ceil(N / (16 * fn))
+        per_cu = math.ceil(units / 256)
+        rounds = math.ceil(per_cu / beside)
+        us = start + again * (rounds - 1) + ksteps * (step * rounds + wg * per_cu + load * units / 256) + weights * N * K * 1e-6
+        if best is None or us < best[0]:
+            best = us, t
+    line = 0.85 if K > 4096 else 0.97 if M <= 256 else 0.9
+    return best[1] if best[0] < line * _row_us(M, N, K, epi, f16)[0] else 0
+
+
+def _gemm_dk_rows(a, w, bias, epi: int, resid, out, tile: int):
+    _check(lib().da_gemm_dk_rows(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid),
+                                 0 if resid is None else resid.stride(0), a.shape[0], *w.shape, epi, tile,
+                                 int(a.dtype == torch.float16), _stream()), "gemm_dk_rows")
+    return out
 
 
 @_rule
@@ -1342,7 +1385,7 @@ def spin(us: int, device=None) -> None:
 def gemm8p_persist(on: int = -1) -> int:
     """Persistent tile loop of the prefill GEMM (one workgroup per CU walking its XCD's tiles) on
     (1) / off (0) for later launches; -1 only queries. Returns the previous setting."""
-    for rule in (_tail_bytes, _row_us, _rope_apart):  # (the rules that ask which rounds are shared)
+    for rule in (_tail_bytes, _row_us, _dk_rows_tile, _rope_apart):  # (the rules that ask which rounds are shared)
         rule.cache_clear()
     return int(lib().da_gemm8p_persist(int(on)))
 
@@ -1377,6 +1420,8 @@ def gemm_f16(a, w, bias=None, epi: int = EPI_NONE, resid=None, out=None) -> torc
     if out is None:
         out = torch.empty((M, N), dtype=torch.float16, device=a.device)
     _req(out.dtype == torch.float16 and out.shape == (M, N) and out.stride(1) == 1 and out.stride(0) % 8 == 0, "out")
+    if max(K, a.stride(0)) < 1 << 22 and (tile := _dk_rows_tile(M, N, K, epi, True)):
+        return _gemm_dk_rows(a, w, bias, epi, resid, out, tile)
     stream = _raw_stream()
     tile, splits = _row_tile(M, N, K, epi, True) if _row_tiles_ok(M, N) and max(K, a.stride(0)) < 1 << 22 else (0, 1)
     ws = _call_partials(splits, M, N, a)
