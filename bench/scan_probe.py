@@ -40,7 +40,7 @@ def main():
 
                 def run():
                     K._check(lib.da_topk_dense_stream(K._ptr(X), N, d, None, K._ptr(Qv), q, None, 0, float(thr), a.k,
-                                                      rpw, K._ptr(ws), K._ptr(out_s), K._ptr(out_i), K._stream()), "scan")
+                                                      rpw, K._ptr(ws), K._ptr(out_s), K._ptr(out_i), None, 0, K._stream()), "scan")
                 run(); torch.cuda.synchronize()
                 s0, e0 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
                 s0.record()

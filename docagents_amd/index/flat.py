@@ -45,6 +45,7 @@ class FlatIndex:
         self.lock = threading.RLock()
         self._write_ev = None   # event after the last mutation's device work (None: nothing pending)
         self._read_evs: dict = {}  # reader stream handle -> event after its last read
+        self._read_on = None       # stream handle of the read that is open
         self._depth = 0
 
     # ----------------------------------------------------------------- stream ordering
@@ -82,17 +83,20 @@ class FlatIndex:
     @contextlib.contextmanager
     def reading(self):
         with self.lock:
-            cuda = self.device.type == "cuda"
-            if cuda and self._write_ev is not None:
-                torch.cuda.current_stream(self.device).wait_event(self._write_ev)
+            st = torch.cuda.current_stream(self.device) if self.device.type == "cuda" else None
+            if st is None or st.cuda_stream == self._read_on:  # inside a read on this stream: its wait and its event stand for both
+                yield
+                return
+            if self._write_ev is not None:
+                st.wait_event(self._write_ev)
+            outer, self._read_on = self._read_on, st.cuda_stream
             try:
                 yield
             finally:
-                if cuda:
-                    st = torch.cuda.current_stream(self.device)
-                    ev = torch.cuda.Event()
-                    ev.record(st)
-                    self._read_evs[st.cuda_stream] = ev
+                self._read_on = outer
+                ev = self._read_evs.get(st.cuda_stream) or torch.cuda.Event()
+                ev.record(st)
+                self._read_evs[st.cuda_stream] = ev
 
     # ----------------------------------------------------------------- mutation
     def _grow(self, need: int):
@@ -236,31 +240,37 @@ class FlatIndex:
     def search(self, q: torch.Tensor, k: int, min_sim: float, doc_filters: list[list[str]] | None = None):
         """q [Q, d] unit-norm -> (scores fp32 [Q, k], row idx int32 [Q, k]) on device; -inf / -1 padding.
         doc_filters: per-query list of document ids (None = all documents)."""
+        with self.reading():
+            return self._search(q, k, min_sim, doc_filters, False)
+
+    def _search(self, q, k, min_sim, doc_filters, want_ids: bool):
+        """Scores and rows, or the rows' external ids; in a read."""
         Q = q.shape[0]
         q = q.to(device=self.device, dtype=self.X.dtype).contiguous()
-        with self.reading():
-            if self.n == 0 or Q == 0:
-                return (torch.full((Q, k), float("-inf"), device=self.device),
-                        torch.full((Q, k), -1, dtype=torch.int32, device=self.device))
-            X = self.X[:self.n]
-            if doc_filters is None:
-                return self._dense(X, q, k, min_sim, self.slots_t[:self.n])
-            ranges, off, maxrows = self._ranges_for(doc_filters)
-            if maxrows == 0:
-                return (torch.full((Q, k), float("-inf"), device=self.device),
-                        torch.full((Q, k), -1, dtype=torch.int32, device=self.device))
-            if maxrows * Q > 4 * self.n and self.dim % 32 == 0:
-                # wide filters: one MFMA dense scan + bitmap beats per-query range scans
-                return self._dense(X, q, k, min_sim, self.slots_t[:self.n], doc_filters)
-            rt = h2d(np.asarray(ranges, dtype=np.int32).reshape(-1, 2), self.device)
-            ot = h2d(np.asarray(off, dtype=np.int32), self.device)
-            return self.ops.topk_ranges(X, q, rt, ot, k, min_sim, max_rows=maxrows)
+        ids = self.ids_t[:self.n] if want_ids else None
+        if self.n == 0 or Q == 0:
+            return self._none(Q, k, want_ids)
+        X = self.X[:self.n]
+        if doc_filters is None:
+            return self._dense(X, q, k, min_sim, self.slots_t[:self.n], ids=ids)
+        ranges, off, maxrows = self._ranges_for(doc_filters)
+        if maxrows == 0:
+            return self._none(Q, k, want_ids)
+        if maxrows * Q > 4 * self.n and self.dim % 32 == 0:
+            # wide filters: one MFMA dense scan + bitmap beats per-query range scans
+            return self._dense(X, q, k, min_sim, self.slots_t[:self.n], doc_filters, ids)
+        return self.ops.topk_ranges(X, q, np.asarray(ranges, dtype=np.int32).reshape(-1, 2), np.asarray(off, dtype=np.int32),
+                                    k, min_sim, max_rows=maxrows, ids=ids)
 
-    def _dense(self, X, q, k, min_sim, slots, doc_filters=None):
+    def _none(self, Q: int, k: int, want_ids: bool):
+        return (torch.full((Q, k), float("-inf"), device=self.device),
+                torch.full((Q, k), -1, dtype=torch.int64 if want_ids else torch.int32, device=self.device))
+
+    def _dense(self, X, q, k, min_sim, slots, doc_filters=None, ids=None):
         """MFMA dense scan; doc filter as a bitmap over local doc slots (none without a filter: the scan itself
         leaves out removed rows, slot -1)."""
         bitmap = None if doc_filters is None else self._bitmap(q.shape[0], doc_filters)
-        return self.ops.topk_dense(X, q, k, min_sim, slots=slots, bitmap=bitmap)
+        return self.ops.topk_dense(X, q, k, min_sim, slots=slots, bitmap=bitmap, ids=ids)
 
     def _bitmap(self, Q, doc_filters):
         """int32 [Q, words]: bit s of a query's row is set for the doc slots s that its filter names."""
@@ -290,8 +300,7 @@ class FlatIndex:
         """search + gather_ids as ONE read: (scores fp32 [Q, k], external ids int64 [Q, k]) from the
         same committed state of the shard."""
         with self.reading():
-            s, rows = self.search(q, k, min_sim, doc_filters)
-            return s, self.gather_ids(rows)
+            return self._search(q, k, min_sim, doc_filters, True)
 
     def row_ids(self, rows: np.ndarray) -> np.ndarray:
         out = np.full(rows.shape, -1, dtype=np.int64)

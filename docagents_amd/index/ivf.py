@@ -218,31 +218,32 @@ class IVFFlatIndex(FlatIndex):
         return order.cpu().numpy(), docs
 
     # ------------------------------------------------------------------ search
-    def search(self, q: torch.Tensor, k: int, min_sim: float, doc_filters=None):
-        with self.reading():
-            if self.centroids is None or self.n < self.lists:
-                if self.n >= self.lists and self.n >= 4 * self.lists:
-                    self.train()
-                if self.centroids is None:
-                    return super().search(q, k, min_sim, doc_filters)
-            if self.n - self.trained_n > self.retrain_frac * max(1, self.trained_n):
+    def _search(self, q, k, min_sim, doc_filters, want_ids: bool):
+        if self.centroids is None or self.n < self.lists:
+            if self.n >= self.lists and self.n >= 4 * self.lists:
                 self.train()
-            Q = q.shape[0]
-            q = q.to(device=self.device, dtype=torch.bfloat16).contiguous()
-            probes = min(self.probes, self.lists)
-            if probes <= 32:
-                _, lists = self.ops.topk_dense(self.centroids, q, probes, -2.0)
-            else:  # wide probing: centroid scores as one GEMM, then torch top-k
-                lists = torch.topk(self.ops.gemm(q, self.centroids).float(), probes, dim=1).indices.int()
-            bitmap = None if doc_filters is None else self._bitmap(Q, doc_filters)
-            s1, i1 = self.ops.topk_lists(self.X, q, lists, self.list_off_t, k, min_sim,
-                                         mean_rows=-(-probes * self.trained_n // self.lists),
-                                         max_rows=int(self.most_rows[probes]), slots=self.slots_t, bitmap=bitmap)
-            if self.n > self.trained_n:  # delta rows: exact scan
-                d0 = self.trained_n
-                rt = h2d(np.asarray([[d0, self.n]] * Q, dtype=np.int32), self.device)
-                ot = torch.arange(Q + 1, dtype=torch.int32, device=self.device)
-                s2, i2 = self.ops.topk_ranges(self.X, q, rt, ot, k, min_sim, max_rows=self.n - d0,
-                                              slots=self.slots_t, bitmap=bitmap)
-                s1, i1 = self.ops.topk_merge(torch.stack([s1, s2]), torch.stack([i1, i2]), k)
-            return s1, i1
+            if self.centroids is None:
+                return super()._search(q, k, min_sim, doc_filters, want_ids)
+        if self.n - self.trained_n > self.retrain_frac * max(1, self.trained_n):
+            self.train()
+        Q = q.shape[0]
+        q = q.to(device=self.device, dtype=torch.bfloat16).contiguous()
+        probes = min(self.probes, self.lists)
+        if probes <= 32:
+            _, lists = self.ops.topk_dense(self.centroids, q, probes, -2.0)
+        else:  # wide probing: centroid scores as one GEMM, then torch top-k
+            lists = torch.topk(self.ops.gemm(q, self.centroids).float(), probes, dim=1).indices.int()
+        bitmap = None if doc_filters is None else self._bitmap(Q, doc_filters)
+        ids = self.ids_t[:self.n] if want_ids else None
+        delta = self.n > self.trained_n
+        s1, i1 = self.ops.topk_lists(self.X, q, lists, self.list_off_t, k, min_sim,
+                                     mean_rows=-(-probes * self.trained_n // self.lists),
+                                     max_rows=int(self.most_rows[probes]), slots=self.slots_t, bitmap=bitmap,
+                                     ids=None if delta else ids)
+        if delta:  # delta rows: exact scan
+            d0 = self.trained_n
+            s2, i2 = self.ops.topk_ranges(self.X, q, np.asarray([[d0, self.n]] * Q, dtype=np.int32).reshape(-1, 2),
+                                          np.arange(Q + 1, dtype=np.int32), k, min_sim, max_rows=self.n - d0,
+                                          slots=self.slots_t, bitmap=bitmap)
+            s1, i1 = self.ops.topk_merge(torch.stack([s1, s2]), torch.stack([i1, i2]), k, ids=ids)
+        return s1, i1

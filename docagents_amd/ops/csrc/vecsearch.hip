@@ -11,6 +11,8 @@
 //  * topk_merge:  per query, select the global top-k over all workgroups' candidates (sorted desc,
 //                 ties -> smaller row id first).
 //  * kmeans_accum: centroid sums / counts for IVFFlat training (fp32 atomics, 256-B rows).
+#include <cstring>
+
 #include "common.h"
 
 #define TK_MAX 32
@@ -467,13 +469,23 @@ struct TopList {
 // rows over as many workgroups as fill the chip (388 rows of 8 documents: one workgroup took 105 us, with one load
 // in flight and a shuffle merge of K rounds per 64 rows; 7 workgroups take 15 us. 24 queries over 8 lists of about
 // 780 rows x 768: 162 -> 41 us).
+//
+// A filter's ranges come from the host. Up to TR_TABLE numbers of them ride in the launch's arguments (range_off, then the
+// ranges; a workgroup takes them to LDS in one step); as two copies they took 3.3 us each on the device and about 15 on the
+// host. With the ids looked up by the last kernel and one pair of events a search, one query over 8 of 100000 x 768 rows'
+// documents takes 33 us, 94 before; 24 queries over 8 of 512 lists 65, 78 before.
+constexpr int TR_TABLE = 512;  // 2 of the 4 KB that a launch's arguments may have
+struct RangeTable { int v[TR_TABLE]; };
+
 template <int NCH>
 __global__ void __launch_bounds__(256)
 topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ slots,
                    const bf16_t* __restrict__ Qv, int Q, const int* __restrict__ ranges,
                    const int* __restrict__ range_off, const int* __restrict__ lists, int probes,
                    const unsigned* __restrict__ bitmap, int W, float thr,
-                   int K, int rows_per_split, float* __restrict__ out_s, int* __restrict__ out_i) {
+                   int K, int rows_per_split, float* __restrict__ out_s, int* __restrict__ out_i, int n_table,
+                   const RangeTable table) {
+  __shared__ int st[TR_TABLE];
   __shared__ float sc[2][64];
   __shared__ int sr[2][64];
   __shared__ float cs[TL_SL];
@@ -483,6 +495,9 @@ topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ 
   const int half = lane >> 5, l32 = lane & 31;
   TopList top;
   top.init(cs, ci, K);  // (every wave writes the same empty list; wave 0 keeps it)
+  for (int i = tid; i < n_table; i += 256) st[i] = table.v[i];
+  if (n_table) __syncthreads();
+  const auto range = [&](int i) { return n_table ? st[Q + 1 + i] : ranges[i]; };
   const int nch = d / 8;  // 16-B chunks of a row; this lane has chunks l32 + 32 i
   float qv[NCH][8];
 #pragma unroll
@@ -492,7 +507,7 @@ topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ 
 #pragma unroll
     for (int e = 0; e < 8; ++e) qv[i][e] = bf2f((bf16_t)((e & 1) ? (u[e >> 1] >> 16) : (u[e >> 1] & 0xffff)));
   }
-  const int rb = lists ? q * probes : range_off[q], re = lists ? rb + probes : range_off[q + 1];
+  const int rb = n_table ? st[q] : lists ? q * probes : range_off[q], re = n_table ? st[q + 1] : lists ? rb + probes : range_off[q + 1];
   DA_ASSERT(rb >= 0 && re >= rb);
   const int pbeg = split * rows_per_split, pend = pbeg + rows_per_split;
   __syncthreads();
@@ -505,7 +520,7 @@ topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ 
       const int r = min(r0 + lane, re - 1), l = lists ? lists[r] : 0;
       const bool in = r0 + lane < re && l >= 0;
       const int at = !in ? 0 : lists ? l : 2 * r;
-      const int len = ranges[at + 1] - ranges[at];
+      const int len = range(at + 1) - range(at);
       int sum = in ? len : 0;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
@@ -527,7 +542,7 @@ topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ 
   for (int r = r0; r < re; ++r) {
     const int l = lists ? lists[r] : 0;
     if (l < 0) continue;
-    const int s0 = ranges[lists ? l : 2 * r], s1 = ranges[lists ? l + 1 : 2 * r + 1];
+    const int s0 = range(lists ? l : 2 * r), s1 = range(lists ? l + 1 : 2 * r + 1);
     const int len = s1 - s0;
     const int lo = max(pbeg, pos), hi = min(pend, pos + len);
     for (int p0 = lo; p0 < hi; p0 += 64) {
@@ -599,9 +614,26 @@ __device__ __forceinline__ void top_join(TopList& top, float (*cs)[TL_SL], int (
   wave_sync_lds();
 }
 
+// Where a search's result goes, [Q, K] each: scores, and the rows (oi) or, with the table of external ids [N] (og, oi null),
+// the rows' ids. The last kernel of a search looks them up itself: as a launch of its own that was 2 us on the device and 10
+// on the host, for K numbers a query.
+struct TopOut {
+  float* os;
+  int* oi;
+  const long* ids;
+  long* og;
+  int N;
+  __device__ __forceinline__ void put(size_t o, float v, int row) const {
+    os[o] = v;
+    if (og) og[o] = row >= 0 && row < N ? ids[row] : -1;  // (a bad row index never reads outside the table)
+    else oi[o] = row;
+  }
+};
+
 // A wave's list, best first (ties: smaller row id), empty places behind: each row's place by counting the better ones.
-__device__ __forceinline__ void top_order(const TopList& top, float* __restrict__ os, int* __restrict__ oi) {
+__device__ __forceinline__ void top_order(const TopList& top, const TopOut& out, int q) {
   const int K = top.K, lane = top.lane;
+  const size_t o = (size_t)q * K;
   const float v = lane < K ? top.cs[lane] : -INFINITY;
   const int id = lane < K ? top.ci[lane] : -1;
   int rank = 0;
@@ -611,14 +643,8 @@ __device__ __forceinline__ void top_order(const TopList& top, float* __restrict_
     rank += ij >= 0 && (better(vj, ij, v, id) || (vj == v && ij == id && j < lane));  // (a row named twice)
   }
   const int real = __popcll(__ballot(id >= 0));
-  if (id >= 0) {
-    os[rank] = v;
-    oi[rank] = id;
-  }
-  if (lane >= real && lane < K) {
-    os[lane] = -INFINITY;
-    oi[lane] = -1;
-  }
+  if (id >= 0) out.put(o + rank, v, id);
+  if (lane >= real && lane < K) out.put(o + lane, -INFINITY, -1);
 }
 
 // cand [P, Q, K] -> out [Q, K] sorted desc (ties: smaller row id). One workgroup per query, a wave per 64 candidates
@@ -629,7 +655,7 @@ constexpr int TM_WAVES = 16;
 
 __global__ void __launch_bounds__(64 * TM_WAVES)
 topk_merge_kernel(const float* __restrict__ cand_s, const int* __restrict__ cand_i, int P, int Q, int K,
-                  float* __restrict__ os, int* __restrict__ oi) {
+                  const TopOut out) {
   __shared__ float cs[TM_WAVES][TL_SL];
   __shared__ int ci[TM_WAVES][TL_SL];
   const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nt = blockDim.x;
@@ -652,7 +678,7 @@ topk_merge_kernel(const float* __restrict__ cand_s, const int* __restrict__ cand
   __syncthreads();
   if (wid) return;
   top_join(top, cs, ci, nt / 64);
-  top_order(top, os + (size_t)q * K, oi + (size_t)q * K);
+  top_order(top, out, q);
 }
 
 // The second half of a scan (see there): per query the K best of its GT groups, their rows scored again (16 rows a wave and
@@ -685,7 +711,7 @@ template <int NG>
 __global__ void __launch_bounds__(64 * TP_WAVES, 2)
 topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_rows, int lg, const bf16_t* __restrict__ X, int N,
                  const int* __restrict__ slots, const bf16_t* __restrict__ Qv, const unsigned* __restrict__ bitmap, int W,
-                 float thr, int K, float* __restrict__ os, int* __restrict__ oi) {
+                 float thr, int K, const TopOut out) {
   constexpr int d = NG * 128, NK = d / 32, nt = 64 * TP_WAVES;
   static_assert(TP_WAVES == 8, "a key of each thread: 8 per lane of a wave");
   __shared__ float cs[TP_WAVES][TL_SL], cand_s[TP_CAP];
@@ -810,7 +836,7 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
     if (lg < 0) {  // these are the rows
       if (lane < K && ci[0][lane] >= 0) ci[0][lane] = ci[0][lane] / run_slots * run_rows + ci[0][lane] % run_slots;
       wave_sync_lds();
-      top_order(top, os + (size_t)q * K, oi + (size_t)q * K);
+      top_order(top, out, q);
       return;
     }
     if (lane < K) groups[lane] = ci[0][lane];
@@ -855,7 +881,7 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
       if (wid) return;
       if (again) top_join(top, cs, ci, TP_WAVES);
       else fold(count);
-      top_order(top, os + (size_t)q * K, oi + (size_t)q * K);
+      top_order(top, out, q);
       return;
     }
   }
@@ -882,9 +908,14 @@ __global__ void kmeans_accum_kernel(const bf16_t* __restrict__ X, int N, int d, 
   if (threadIdx.x == 0) atomicAdd(&counts[c], 1.f);
 }
 
-static int topk_merge(const void* cs, const void* ci, int P, int Q, int K, void* out_s, void* out_i, hipStream_t s) {
+// (out: rows, int; with ids [N]: their ids, long)
+static TopOut top_out(void* out_s, void* out, const void* ids, int N) {
+  return ids ? TopOut{(float*)out_s, nullptr, (const long*)ids, (long*)out, N} : TopOut{(float*)out_s, (int*)out, nullptr, nullptr, 0};
+}
+
+static int topk_merge(const void* cs, const void* ci, int P, int Q, int K, const TopOut& out, hipStream_t s) {
   const long waves = min((long)TM_WAVES, max(1L, ((long)P * K + 63) / 64));
-  topk_merge_kernel<<<Q, 64 * (int)waves, 0, s>>>((const float*)cs, (const int*)ci, P, Q, K, (float*)out_s, (int*)out_i);
+  topk_merge_kernel<<<Q, 64 * (int)waves, 0, s>>>((const float*)cs, (const int*)ci, P, Q, K, out);
   DA_LAUNCH_CHECK();
 }
 
@@ -894,8 +925,8 @@ DA_EXPORT size_t da_topk_dense_ws(int N, int Q, int K, int rows_per_block) {
 }
 
 DA_EXPORT int da_topk_dense(const void* X, int N, int d, const void* slots, const void* Qv, int Q, const void* bitmap,
-                            int W, float thr, int K, int rows_per_block, void* ws, void* out_s, void* out_i,
-                            void* stream) {
+                            int W, float thr, int K, int rows_per_block, void* ws, void* out_s, void* out,
+                            const void* ids, int n_ids, void* stream) {
   if (d % 32 || K < 1 || K > TK_MAX || rows_per_block % 64 || rows_per_block <= 0) return (int)hipErrorInvalidValue;
   if (Q == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
@@ -909,7 +940,7 @@ DA_EXPORT int da_topk_dense(const void* X, int N, int d, const void* slots, cons
                                            (const unsigned*)bitmap, W, thr, K, rows_per_block, cs, ci);
   int err = (int)hipGetLastError();
   if (err) return err;
-  return topk_merge(cs, ci, nblk, Q, K, out_s, out_i, s);
+  return topk_merge(cs, ci, nblk, Q, K, top_out(out_s, out, ids, n_ids), s);
 }
 
 // The streaming scan (d = 384, 768 or 1024). hipErrorInvalidValue for shapes it does not take (the caller then uses
@@ -946,7 +977,7 @@ DA_EXPORT size_t da_topk_stream_ws(int N, int Q, int K, int rows_per_wave) {
 
 DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slots, const void* Qv, int Q,
                                    const void* bitmap, int W, float thr, int K, int rows_per_wave, void* ws, void* out_s,
-                                   void* out_i, void* stream) {
+                                   void* out, const void* ids, int n_ids, void* stream) {
   if ((d != 384 && d != 768 && d != 1024) || K < 1 || K > TK_MAX || N < 1 || rows_per_wave < 16)
     return (int)hipErrorInvalidValue;
   if (Q == 0) return 0;
@@ -972,7 +1003,7 @@ DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slot
     const int err = (int)hipGetLastError();                                                                          \
     if (err) return err;                                                                                             \
     topk_pick_kernel<NG><<<Q, 64 * TP_WAVES, 0, s>>>(gm, GT, p.run_slots, p.run_rows, p.lg, (const bf16_t*)X, N,      \
-        (const int*)slots, (const bf16_t*)Qv, (const unsigned*)bitmap, W, thr, K, (float*)out_s, (int*)out_i);        \
+        (const int*)slots, (const bf16_t*)Qv, (const unsigned*)bitmap, W, thr, K, top_out(out_s, out, ids, n_ids));   \
   } while (0)
   switch (d) {
     case 384: TDS(3); break;
@@ -986,12 +1017,15 @@ DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slot
 
 DA_EXPORT int da_topk_ranges(const void* X, int d, const void* slots, const void* Qv, int Q, const void* ranges,
                              const void* range_off, const void* lists, int probes, const void* bitmap, int W,
-                             float thr, int K, int splits, int rows_per_split, void* ws, void* out_s, void* out_i,
-                             void* stream) {
+                             float thr, int K, int splits, int rows_per_split, void* ws, void* out_s, void* out,
+                             const void* ids, int n_ids, const void* host_table, int n_table, void* stream) {
   if (d % 8 || d < 8 || d > 4096 || K < 1 || K > TK_MAX || splits < 1 || rows_per_split < 1 ||
-      (!range_off && (!lists || probes < 0)))
+      (!range_off && !n_table && (!lists || probes < 0)) || n_table < 0 || n_table > TR_TABLE ||
+      (n_table && (lists || !host_table || n_table < Q + 1)))
     return (int)hipErrorInvalidValue;
   if (Q == 0) return 0;
+  RangeTable table;
+  if (n_table) memcpy(table.v, host_table, (size_t)n_table * sizeof(int));
   hipStream_t s = (hipStream_t)stream;
   float* cs = (float*)ws;
   int* ci = (int*)(cs + (size_t)splits * Q * K);
@@ -999,7 +1033,7 @@ DA_EXPORT int da_topk_ranges(const void* X, int d, const void* slots, const void
 #define TRG(NCH)                                                                                                    \
   topk_ranges_kernel<NCH><<<grid, 256, 0, s>>>((const bf16_t*)X, d, (const int*)slots, (const bf16_t*)Qv, Q,        \
                                                (const int*)ranges, (const int*)range_off, (const int*)lists,        \
-                                               probes, (const unsigned*)bitmap, W, thr, K, rows_per_split, cs, ci)
+                                               probes, (const unsigned*)bitmap, W, thr, K, rows_per_split, cs, ci, n_table, table)
   if (d <= 256) TRG(1);
   else if (d <= 512) TRG(2);
   else if (d <= 768) TRG(3);
@@ -1009,13 +1043,14 @@ DA_EXPORT int da_topk_ranges(const void* X, int d, const void* slots, const void
 #undef TRG
   int err = (int)hipGetLastError();
   if (err) return err;
-  return topk_merge(cs, ci, splits, Q, K, out_s, out_i, s);
+  return topk_merge(cs, ci, splits, Q, K, top_out(out_s, out, ids, n_ids), s);
 }
 
-DA_EXPORT int da_topk_merge(void* cand_s, void* cand_i, int P, int Q, int K, void* out_s, void* out_i, void* stream) {
+DA_EXPORT int da_topk_merge(void* cand_s, void* cand_i, int P, int Q, int K, void* out_s, void* out, const void* ids, int n_ids,
+                            void* stream) {
   if (K < 1 || K > TK_MAX) return (int)hipErrorInvalidValue;
   if (Q == 0) return 0;
-  return topk_merge(cand_s, cand_i, P, Q, K, out_s, out_i, (hipStream_t)stream);
+  return topk_merge(cand_s, cand_i, P, Q, K, top_out(out_s, out, ids, n_ids), (hipStream_t)stream);
 }
 
 DA_EXPORT int da_gather_ids(const void* rows, int n, const void* ids, int N, void* out, void* stream) {

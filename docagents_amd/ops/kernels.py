@@ -16,6 +16,7 @@ import os
 import threading
 from pathlib import Path
 
+import numpy as np
 import torch
 
 _LOCK = threading.Lock()
@@ -77,12 +78,13 @@ _SIGS = {
                        c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
                        c_int, c_void_p],
     "da_topk_dense": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_float, c_int,
-                      c_int, c_void_p, c_void_p, c_void_p, c_void_p],
+                      c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     "da_topk_dense_stream": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_float, c_int,
-                             c_int, c_void_p, c_void_p, c_void_p, c_void_p],
+                             c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     "da_topk_ranges": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int,
-                       c_float, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
-    "da_topk_merge": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
+                       c_float, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int,
+                       c_void_p],
+    "da_topk_merge": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     "da_gather_ids": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p],
     "da_kmeans_accum": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
     "da_sample_partial": [c_void_p, c_int, c_int, c_int, c_int, c_float, c_uint, c_uint, c_void_p, c_void_p, c_void_p],
@@ -1245,8 +1247,21 @@ def _scan_rows(N: int) -> int:
     return max(min(tiles(256 * 4), 64), tiles(256 * 16), 16)
 
 
-def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_block: int | None = None):
-    """Exact top-K of Qv @ X^T per query with threshold and optional doc-slot bitmap [Q, W] int32."""
+def _found(Q: int, K: int, ids, like):
+    """A search's results (scores, rows; the rows' external ids where ``ids`` is their table) and the launcher's arguments."""
+    out_s = like.new_empty((Q, K), dtype=torch.float32)
+    if ids is None:
+        out = like.new_empty((Q, K), dtype=torch.int32)
+        return out_s, out, (out_s.data_ptr(), out.data_ptr(), None, 0)
+    _req(ids.is_cuda and ids.dtype == torch.int64 and ids.is_contiguous() and ids.dim() == 1 and ids.numel() > 0,
+         "ids must be int64 [N]")
+    out = like.new_empty((Q, K), dtype=torch.int64)
+    return out_s, out, (out_s.data_ptr(), out.data_ptr(), ids.data_ptr(), ids.numel())
+
+
+def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_block: int | None = None, ids=None):
+    """Exact top-K of Qv @ X^T per query with threshold and optional doc-slot bitmap [Q, W] int32: scores and rows, or
+    (``ids`` int64 [N]) scores and ids[rows], as ``gather_ids`` gives them."""
     _bf16_cuda(X, "X"); _bf16_cuda(Qv, "Qv")
     N, d = X.shape
     Q = Qv.shape[0]
@@ -1265,36 +1280,49 @@ def topk_dense(X, Qv, K: int, thr: float, slots=None, bitmap=None, rows_per_bloc
         # rows as the queries, keeps the query-major tiles below)
         rpw = _scan_rows(N)
         ws = _call_scratch(int(lib().da_topk_stream_ws(N, Q, K, rpw)), X)
-        out_s = X.new_empty((Q, K), dtype=torch.float32)
-        out_i = X.new_empty((Q, K), dtype=torch.int32)
+        out_s, out, args = _found(Q, K, ids, X)
         _check(lib().da_topk_dense_stream(_ptr(X), N, d, _ptr(slots), _ptr(Qv), Q, _ptr(bitmap), W, float(thr), K,
-                                          rpw, _ptr(ws), _ptr(out_s), _ptr(out_i), _stream()), "topk_dense_stream")
-        return out_s, out_i
+                                          rpw, _ptr(ws), *args, _stream()), "topk_dense_stream")
+        return out_s, out
     if rows_per_block is None:
         qt = math.ceil(Q / 16)
         nblk = max(1, min(math.ceil(N / 256), max(1, 1024 // qt)))
         rows_per_block = max(64, math.ceil(math.ceil(N / nblk) / 64) * 64)
     nblk = max(1, math.ceil(N / rows_per_block))
     ws = _call_scratch(nblk * Q * K * 8, X)
-    out_s = X.new_empty((Q, K), dtype=torch.float32)
-    out_i = X.new_empty((Q, K), dtype=torch.int32)
+    out_s, out, args = _found(Q, K, ids, X)
     _check(lib().da_topk_dense(_ptr(X), N, d, _ptr(slots), _ptr(Qv), Q, _ptr(bitmap), W, float(thr), K,
-                               rows_per_block, _ptr(ws), _ptr(out_s), _ptr(out_i), _stream()), "topk_dense")
-    return out_s, out_i
+                               rows_per_block, _ptr(ws), *args, _stream()), "topk_dense")
+    return out_s, out
+
+
+TABLE_MAX = 512  # numbers of a filter's row ranges that ride in a launch's arguments (the kernel's TR_TABLE)
 
 
 def topk_ranges(X, Qv, ranges, range_off, K: int, thr: float, max_rows: int, slots=None, bitmap=None,
-                rows_per_split: int | None = None):
-    """Top-K per query over its own row ranges. ranges int32 [R, 2], range_off int32 [Q+1];
+                rows_per_split: int | None = None, ids=None):
+    """Top-K per query over its own row ranges. ranges int32 [R, 2], range_off int32 [Q+1] (both on the
+    device or both arrays of the host: a few ride in the launch's arguments, more go in one copy);
     max_rows = max total rows of any query (host int) — sets the split count: rows_per_split rows of a query per
     workgroup (default: ``_rows_per_split``)."""
-    _i32(ranges, "ranges"); _i32(range_off, "range_off")
-    _req(range_off.numel() == Qv.shape[0] + 1, "range_off length")
-    return _ranges(X, Qv, ranges, range_off, None, K, thr, max_rows, slots, bitmap,
-                   rows_per_split or _rows_per_split(max_rows, Qv.shape[0]))
+    rows, Q, table = rows_per_split or _rows_per_split(max_rows, Qv.shape[0]), Qv.shape[0], None
+    if isinstance(ranges, np.ndarray):
+        _req(range_off.shape == (Q + 1,) and ranges.shape == (range_off[-1], 2), "range_off length")
+        table = np.concatenate([range_off, ranges.reshape(-1)]).astype(np.int32, copy=False)
+        if table.size > TABLE_MAX:
+            from . import h2d
+            t = h2d(table, X.device)
+            range_off, ranges, table = t[:Q + 1], t[Q + 1:], None
+    if table is None:
+        _i32(ranges, "ranges"); _i32(range_off, "range_off")
+        _req(range_off.numel() == Q + 1, "range_off length")
+    else:
+        ranges = range_off = None
+    return _ranges(X, Qv, ranges, range_off, None, K, thr, max_rows, slots, bitmap, rows, ids, table)
 
 
-def topk_lists(X, Qv, lists, list_off, K: int, thr: float, mean_rows: int, max_rows: int, slots=None, bitmap=None):
+def topk_lists(X, Qv, lists, list_off, K: int, thr: float, mean_rows: int, max_rows: int, slots=None, bitmap=None,
+               ids=None):
     """Top-K per query over the lists it names: lists int32 [Q, probes] (on the device; negative: none), list l =
     rows list_off[l] .. list_off[l + 1] (int32). mean_rows / max_rows: rows of a query, expected / at most (host
     ints). The lists never visit the host: nothing waits for the kernel that chose them."""
@@ -1302,7 +1330,7 @@ def topk_lists(X, Qv, lists, list_off, K: int, thr: float, mean_rows: int, max_r
     _req(lists.dim() == 2 and lists.shape[0] == Qv.shape[0], "lists [Q, probes]")
     # workgroups past a query's rows end at once, but lists of very uneven length must not make too many of them
     rows = max(_rows_per_split(mean_rows, Qv.shape[0]), math.ceil(max_rows / 512 / 64) * 64)
-    return _ranges(X, Qv, list_off, None, lists, K, thr, max_rows, slots, bitmap, rows)
+    return _ranges(X, Qv, list_off, None, lists, K, thr, max_rows, slots, bitmap, rows, ids)
 
 
 def _rows_per_split(rows: int, Q: int) -> int:
@@ -1311,7 +1339,7 @@ def _rows_per_split(rows: int, Q: int) -> int:
     return min(512, max(64, math.ceil(rows * Q / 1024 / 64) * 64))
 
 
-def _ranges(X, Qv, ranges, range_off, lists, K, thr, max_rows, slots, bitmap, rows_per_split):
+def _ranges(X, Qv, ranges, range_off, lists, K, thr, max_rows, slots, bitmap, rows_per_split, ids=None, table=None):
     _bf16_cuda(X, "X"); _bf16_cuda(Qv, "Qv")
     N, d = X.shape
     Q = Qv.shape[0]
@@ -1324,29 +1352,28 @@ def _ranges(X, Qv, ranges, range_off, lists, K, thr, max_rows, slots, bitmap, ro
         _req(slots is not None, "bitmap needs slots")
         _req(bitmap.dtype == torch.int32 and bitmap.shape[0] == Q, "bitmap")
         W = bitmap.shape[1]
-    out_s = X.new_empty((Q, K), dtype=torch.float32)
-    out_i = X.new_empty((Q, K), dtype=torch.int32)
+    out_s, out, args = _found(Q, K, ids, X)
     if Q == 0:
-        return out_s, out_i
+        return out_s, out
     splits = max(1, math.ceil(max_rows / rows_per_split))
     ws = _call_scratch(splits * Q * K * 8, X)
     _check(lib().da_topk_ranges(_ptr(X), d, _ptr(slots), _ptr(Qv), Q, _ptr(ranges), _ptr(range_off), _ptr(lists),
                                 0 if lists is None else lists.shape[1], _ptr(bitmap),
-                                W, float(thr), K, splits, rows_per_split, _ptr(ws), _ptr(out_s), _ptr(out_i),
+                                W, float(thr), K, splits, rows_per_split, _ptr(ws), *args,
+                                None if table is None else table.ctypes.data, 0 if table is None else table.size,
                                 _stream()), "topk_ranges")
-    return out_s, out_i
+    return out_s, out
 
 
-def topk_merge(cand_s, cand_i, K: int):
+def topk_merge(cand_s, cand_i, K: int, ids=None):
     """cand [P, Q, K] -> the best K of each query, sorted."""
     _req(cand_s.dtype == torch.float32 and cand_i.dtype == torch.int32, "dtypes")
     P, Q, K2 = cand_s.shape
     _req(K2 == K, "K mismatch")
     cs, ci = cand_s.contiguous(), cand_i.contiguous()
-    out_s = torch.empty((Q, K), dtype=torch.float32, device=cs.device)
-    out_i = torch.empty((Q, K), dtype=torch.int32, device=cs.device)
-    _check(lib().da_topk_merge(_ptr(cs), _ptr(ci), P, Q, K, _ptr(out_s), _ptr(out_i), _stream()), "topk_merge")
-    return out_s, out_i
+    out_s, out, args = _found(Q, K, ids, cs)
+    _check(lib().da_topk_merge(_ptr(cs), _ptr(ci), P, Q, K, *args, _stream()), "topk_merge")
+    return out_s, out
 
 
 def gather_ids(rows, ids):

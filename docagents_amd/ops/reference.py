@@ -372,7 +372,11 @@ def sample_finalize(gathered, ranks, out_tok=None, out_lp=None, conf=None, activ
                      lens, hist, start, eos)
 
 
-def topk_dense(X, Qv, K, thr, slots=None, bitmap=None, **_):
+def _found(s, rows, ids):
+    return s, rows if ids is None else gather_ids(rows, ids)
+
+
+def topk_dense(X, Qv, K, thr, slots=None, bitmap=None, ids=None, **_):
     s = Qv.float() @ X.float().t()  # [Q, N]
     valid = s >= thr
     if slots is not None:
@@ -383,7 +387,7 @@ def topk_dense(X, Qv, K, thr, slots=None, bitmap=None, **_):
         bits = (words >> (sl & 31).view(1, -1)) & 1
         valid &= bits.bool()
     s = s.masked_fill(~valid, float("-inf"))
-    return _topk_with_ties(s, K)
+    return _found(*_topk_with_ties(s, K), ids)
 
 
 def _topk_with_ties(s, K):
@@ -405,7 +409,7 @@ def _topk_with_ties(s, K):
     return vs, ii
 
 
-def topk_ranges(X, Qv, ranges, range_off, K, thr, max_rows=None, slots=None, bitmap=None, **_):
+def topk_ranges(X, Qv, ranges, range_off, K, thr, max_rows=None, slots=None, bitmap=None, ids=None, **_):
     Q = Qv.shape[0]
     N = X.shape[0]
     s = Qv.float() @ X.float().t()
@@ -424,17 +428,17 @@ def topk_ranges(X, Qv, ranges, range_off, K, thr, max_rows=None, slots=None, bit
         bits = (bitmap[:, (sl >> 5)] >> (sl & 31).view(1, -1)) & 1
         valid &= bits.bool()
     s = s.masked_fill(~valid, float("-inf"))
-    return _topk_with_ties(s, K)
+    return _found(*_topk_with_ties(s, K), ids)
 
 
-def topk_lists(X, Qv, lists, list_off, K, thr, mean_rows=None, max_rows=None, slots=None, bitmap=None):
+def topk_lists(X, Qv, lists, list_off, K, thr, mean_rows=None, max_rows=None, slots=None, bitmap=None, ids=None):
     off = list_off.tolist()
     rg = [[off[x], off[x + 1]] if x >= 0 else [0, 0] for q in lists.tolist() for x in q]
     ro = torch.arange(lists.shape[0] + 1) * lists.shape[1]
-    return topk_ranges(X, Qv, torch.tensor(rg).view(-1, 2), ro, K, thr, slots=slots, bitmap=bitmap)
+    return topk_ranges(X, Qv, torch.tensor(rg).view(-1, 2), ro, K, thr, slots=slots, bitmap=bitmap, ids=ids)
 
 
-def topk_merge(cand_s, cand_i, K):
+def topk_merge(cand_s, cand_i, K, ids=None):
     P, Q, _ = cand_s.shape
     s = cand_s.permute(1, 0, 2).reshape(Q, -1)
     i = cand_i.permute(1, 0, 2).reshape(Q, -1)
@@ -445,7 +449,7 @@ def topk_merge(cand_s, cand_i, K):
     order = torch.argsort(key, dim=1, descending=True, stable=True)
     vs, ii = torch.gather(s, 1, order)[:, :K], torch.gather(i, 1, order)[:, :K]
     ii = torch.where(torch.isinf(vs), torch.full_like(ii, -1), ii)
-    return vs, ii
+    return _found(vs, ii, ids)
 
 
 def gather_ids(rows, ids):

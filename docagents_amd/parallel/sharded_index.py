@@ -33,11 +33,9 @@ class ShardedIndex:
         rank order (len W*B) or None. Returns (scores fp32 [B, k], ids int64 [B, k]) on device."""
         B = q_local.shape[0]
         if self.world == 1:
-            s, rows = self.local.search(q_local, k, min_sim, doc_filters_all)
-            return s, self.local.gather_ids(rows)
+            return self.local.search_ids(q_local, k, min_sim, doc_filters_all)
         qs = all_gather_rows(q_local.contiguous(), self.group)                     # C2
-        s, rows = self.local.search(qs, k, min_sim, doc_filters_all)
-        gid = self.local.gather_ids(rows)                                          # int64 [W*B, k]
+        s, gid = self.local.search_ids(qs, k, min_sim, doc_filters_all)            # int64 [W*B, k]
         P = all_gather_rows(pack_scores_ids(s, gid), self.group)                    # C1 (one buffer)
         S, G = unpack_scores_ids(P)
         S = S.reshape(self.world, self.world * B, k)
