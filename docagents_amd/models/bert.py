@@ -8,6 +8,7 @@ pooling fused with the L2 normalisation. Output vectors are unit-norm like the r
 """
 from __future__ import annotations
 
+import itertools
 import math
 
 import numpy as np
@@ -133,6 +134,8 @@ class BertEncoder:
             x, *xq = x
         elif o.gemm_ln_fit(x.shape[0], h, c.ffn) and not self._one_row(x.shape[0]):
             return self._layers_few_rows(x, cu_seqlens, max_seqlen, o.flash_attn_varlen, o.layernorm)
+        if o.encoder_layers_fit(x.shape[0]):
+            return o.encoder_layers(x, w["layers"], cu_seqlens, max_seqlen, nh, hd, c.eps, xq=xq)
         for L in w["layers"]:
             qkv = self._linear(x, L, "wqkv", L["bqkv"], EPI_BIAS, xq=xq)
             a = o.flash_attn_varlen(qkv[:, :h], qkv[:, h:2 * h], qkv[:, 2 * h:], cu_seqlens, max_seqlen, nh, nh, hd,
@@ -178,6 +181,8 @@ class BertEncoder:
                                 c.eps)
         if o.gemm_ln_fit(x.shape[0], h, c.ffn):
             return self._layers_few_rows(x, cu_seqlens, max_seqlen, o.flash_attn_f16, o.layernorm_f16)
+        if o.encoder_layers_fit(x.shape[0]):
+            return o.encoder_layers(x, w["layers"], cu_seqlens, max_seqlen, nh, hd, c.eps)
         for L in w["layers"]:
             qkv = o.gemm_f16(x, L["wqkv"], bias=L["bqkv"], epi=EPI_BIAS)
             a = o.flash_attn_f16(qkv[:, :h], qkv[:, h:2 * h], qkv[:, 2 * h:], cu_seqlens, max_seqlen, nh, nh, hd)
@@ -195,10 +200,13 @@ class BertEncoder:
             return torch.empty((0, self.cfg.hidden), dtype=torch.float32, device=self.device)
         cu = np.zeros(len(seqs) + 1, dtype=np.int32)
         np.cumsum(lens, out=cu[1:])
-        flat = np.fromiter((t for s in seqs for t in s), dtype=np.int32, count=int(cu[-1]))
-        pos = np.arange(int(cu[-1]), dtype=np.int32) - np.repeat(cu[:-1], lens)
-        dev = self.device
-        ids_t, pos_t, cu_t = h2d(flat, dev), h2d(pos, dev), h2d(cu, dev)
+        T = int(cu[-1])
+        host = np.empty(2 * T + len(cu), dtype=np.int32)  # one copy
+        host[:T] = np.fromiter(itertools.chain.from_iterable(seqs), dtype=np.int32, count=T)
+        host[T:2 * T] = np.arange(T, dtype=np.int32) - np.repeat(cu[:-1], lens)
+        host[2 * T:] = cu
+        d = h2d(host, self.device)
+        ids_t, pos_t, cu_t = d[:T], d[T:2 * T], d[2 * T:]
         hid = self.forward(ids_t, pos_t, cu_t, int(lens.max()))
         mode = 0 if self.cfg.pooling == "cls" else 1
         pool = self.ops.pool_l2norm_f16 if self.fp16 else self.ops.pool_l2norm

@@ -68,6 +68,7 @@ _SIGS = {
     "da_gemm_dk_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 7 + [c_void_p],
     "da_enc_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5
                   + [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_void_p],
+    "da_encoder_layer": [c_void_p, c_int, c_int, c_int, c_void_p],
     "da_gemm_tail_ws": [c_int] * 5,
     "da_gemm_fp8_tile": [c_int] * 2,
     "da_gemm8p_ksteps": [c_int] * 5,
@@ -174,6 +175,12 @@ def lib(parts=()) -> _Kernels:
         if p not in _LOADED:
             load_part(p)
     return _LIB
+
+
+@functools.lru_cache(maxsize=None)
+def _address(name: str) -> int:
+    """A launcher's address, for native code that calls it (its library stays loaded)."""
+    return ctypes.cast(getattr(lib(), name), c_void_p).value
 
 
 def available() -> bool:
@@ -305,6 +312,24 @@ def _call_partials(splits: int, M: int, N: int, like):
     return _call_scratch(splits * M * N * 4, like) if splits > 1 else None
 
 
+def _row_choice(M: int, N: int, K: int, epi: int, lda: int, f16: bool = False):
+    """(tile, splits) of a product of more than 64 rows (fp16: of any). A tile of ``_DK_TILES`` is da_gemm_dk_rows'."""
+    if max(K, lda) < 1 << 22:
+        tile = _dk_rows_tile(M, N, K, epi, f16)
+        if tile:
+            return tile, 1
+        if _row_tiles_ok(M, N):
+            return _row_tile(M, N, K, epi, f16)
+    if f16 or M >= 640:
+        return 0, 1
+    return 11, _auto_splits(M, N, K)  # rows too long for the streaming tiles' offsets: the register-staged 64x128 tile
+
+
+def _has_tail(M: int, tile: int, f16: bool = False) -> bool:
+    """Whether a product runs on the kernels whose last round may be shared (gemm8p's rows and tiles)."""
+    return tile in (7, 10) or (tile == 4 and not f16) or (tile == 0 and M >= (256 if f16 else 640))
+
+
 def gemv_fusable(M: int, N: int, K: int, epi: int = EPI_NONE) -> bool:
     """True when gemm() runs the batch-1 GEMV (which can also fuse the input RMSNorm)."""
     return M == 1 and K % 512 == 0 and N % 4 == 0 and (epi not in GATED or N % 32 == 0)
@@ -345,8 +370,10 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
         return out
     if (tile == 12 or (tile == 0 and splits <= 0)) and rms is None and dk_fusable(M, N, K, epi):
         return gemm_dk(a, w, epi=epi, bias=bias, resid=resid, out=out)
-    if tile == 0 and splits <= 0 and rms is None and max(K, a.stride(0)) < 1 << 22:
-        tile = _dk_rows_tile(M, N, K, epi)
+    ws = None
+    if tile == 0 and splits <= 0 and rms is None and M > 64:
+        tile, splits = _row_choice(M, N, K, epi, a.stride(0))
+        ws = _call_partials(splits, M, N, a)
     if tile in _DK_TILES:
         _req(rms is None and splits <= 1, "gemm_dk rows: whole, without a norm")
         return _gemm_dk_rows(a, w, bias, epi, resid, out, tile)
@@ -358,23 +385,14 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
         _req(eps > 0, "fused RMSNorm needs eps > 0")
         if gamma is not None:
             _bf16_cuda(gamma, "gamma"); _req(gamma.numel() == K, "gamma must be [K]")
-    ws = None
     if splits <= 0:
-        if tile == 0 and M > 64 and _row_tiles_ok(M, N) and max(K, a.stride(0)) < 1 << 22:
-            tile, splits = _row_tile(M, N, K, epi)
-            ws = _call_partials(splits, M, N, a)
-        elif tile == 0 and 64 < M < 640:  # rows too long for the streaming tiles' offsets: the register-staged 64x128 tile
-            tile, splits = 11, _auto_splits(M, N, K)
-            ws = _call_partials(splits, M, N, a)
-        else:
-            if tile == 0 and M < 640:
-                tile = _decode_tile(M)
-            splits = _auto_splits(M, N, K) if tile in (0, 2, 3) or (tile == 9 and M <= 128) else 1
+        if tile == 0 and M < 640:
+            tile = _decode_tile(M)
+        splits = _auto_splits(M, N, K) if tile in (0, 2, 3) or (tile == 9 and M <= 128) else 1
     if splits > 1 and ws is None:
         ws = _workspace(splits * M * N * 4, a.device)
     stream = _raw_stream()
-    # (gemm8p's rows and tiles)
-    tail = _gemm_tail(a.device, stream, M, N, K, epi, tile) if tile in (4, 7, 10) or (tile == 0 and M >= 640) else (None, None)
+    tail = _gemm_tail(a.device, stream, M, N, K, epi, tile) if _has_tail(M, tile) else (None, None)
     rc = lib().da_gemm_bf16(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
                             M, N, K, epi, tile, splits, _ptr(ws), _ptr(gamma), float(eps), *map(_ptr, tail), c_void_p(stream))
     _check(rc, "gemm")
@@ -595,6 +613,94 @@ def quant_weight_fp8(w: torch.Tensor):
     wf = w.float()
     sw = (wf.abs().amax(dim=1) / 448.0).clamp_min(1e-30)
     return (wf / sw[:, None]).clamp(-448, 448).to(FP8).contiguous(), sw.contiguous()
+
+
+class _EncoderProduct(ctypes.Structure):
+    _fields_ = [(n, c_void_p) for n in ("ws", "tail_ws", "tail_cnt")] + [(n, c_int) for n in ("tile", "splits", "rows", "pad")]
+
+
+_ENCODER_WEIGHTS = ("wqkv", "bqkv", "wo", "bo", "ln1_g", "ln1_b", "w1", "b1", "w2", "b2", "ln2_g", "ln2_b")
+
+
+class _EncoderLayer(ctypes.Structure):
+    _fields_ = ([(n, c_void_p) for n in ("gemm", "gemm_rows", "gemm_fp8", "attn", "norm")] + [("w", c_void_p * 14)]
+                + [(n, c_void_p * 3) for n in ("x", "xq", "xscale")] + [("qkv", c_void_p), ("a", c_void_p), ("y", c_void_p * 2)]
+                + [("f", c_void_p), ("cu", c_void_p)] + [("p", _EncoderProduct * 4)]
+                + [(n, c_int) for n in ("kind", "T", "B", "max_len", "heads", "head_dim", "hidden", "ffn")]
+                + [("eps", c_float), ("scale", c_float)])
+
+
+def encoder_layers_fit(rows: int) -> bool:
+    """Whether an encoder's layers take ``encoder_layers`` (fewer rows have products of their own, and captured graphs)."""
+    return rows > 64
+
+
+def encoder_layers(x, layers, cu_seqlens, max_seqlen: int, heads: int, head_dim: int, eps: float, xq=None):
+    """The layers of an encoder over x [T, hidden] (bf16, fp16; with xq = (e4m3 rows, scales) the fp8 products of
+    ``gemm_fp8``) -> [T, hidden]: what gemm / gemm_f16 / gemm_fp8, the attention and the LayerNorms give one by one, with
+    one native call a layer (csrc/encoder_layer.hip). ``layers``: each layer's weights by name."""
+    f16, q8 = x.dtype == torch.float16, xq is not None
+    (_f16_cuda if f16 else _bf16_cuda)(x, "x")
+    _i32(cu_seqlens, "cu_seqlens")
+    T, h = x.shape
+    ffn = layers[0]["w1"].shape[0] if layers else 0
+    _req(T > 64 and x.is_contiguous() and x.data_ptr() % 16 == 0, "x [T, hidden], contiguous")
+    _req(h == heads * head_dim and head_dim in ((64, 96) if f16 else (32, 64, 96, 128)), f"head dim {head_dim} unsupported")
+    _req(h % (128 if q8 else 64) == 0 and ffn % 64 == 0 and (not f16 or min(h, ffn) >= 128), f"hidden {h}, feed-forward {ffn}")
+    stream, L, dt = _raw_stream(), _EncoderLayer(), x.dtype
+    new = lambda n: torch.empty((T, n), dtype=dt, device=x.device)  # noqa: E731
+    # Two sets of buffers, layers in turn: a kernel that writes over what all dies' caches have just read waits for them to give it
+    # up (57 short texts, width 384, fp8: 684 us with one set, 650 with two; 651, 653 and 683 with 3, 8 and 12).
+    sets = [{n: new(c) for n, c in (("qkv", 3 * h), ("a", h), ("y0", h), ("m", h), ("f", ffn), ("y1", h), ("x", h))}
+            for _ in layers[:2]]
+    L.cu = cu_seqlens.data_ptr()
+    if q8:
+        _req(xq[0].dtype == FP8 and xq[0].shape == x.shape and xq[0].is_contiguous() and xq[0].data_ptr() % 16 == 0
+             and xq[1].dtype == torch.float32 and xq[1].numel() >= T, "fp8 rows")
+        L.gemm_fp8 = _address("da_gemm_fp8")
+        for S in sets:
+            for n in ("m8", "x8"):
+                S[n] = (torch.empty((T, h), dtype=FP8, device=x.device), torch.empty(T, dtype=torch.float32, device=x.device))
+    L.gemm, L.gemm_rows = _address("da_gemm_f16" if f16 else "da_gemm_bf16"), _address("da_gemm_dk_rows")
+    L.attn = _address("da_flash_attn_f16" if f16 else "da_flash_attn_v2")
+    L.norm = _address("da_layernorm_f16" if f16 else "da_layernorm_q" if q8 else "da_layernorm")
+    L.kind, L.T, L.B, L.max_len = 1 if f16 else 2 if q8 else 0, T, cu_seqlens.numel() - 1, int(max_seqlen)
+    L.heads, L.head_dim, L.hidden, L.ffn, L.eps, L.scale = heads, head_dim, h, ffn, float(eps), 1.0 / math.sqrt(head_dim)
+    held = []  # (a product's partials and counters serve every layer: one after another on this stream)
+    for p, (N, K, epi, fp8) in zip(L.p, ((3 * h, h, EPI_BIAS, q8), (h, h, EPI_RESID, False), (ffn, h, EPI_GELU, q8),
+                                        (h, ffn, EPI_RESID, False))):
+        if fp8:
+            continue
+        p.tile, p.splits = _row_choice(T, N, K, epi, K, f16)
+        p.rows = p.tile in _DK_TILES
+        if p.rows:
+            continue
+        ws = _call_partials(p.splits, T, N, x)
+        tail = _gemm_tail(x.device, stream, T, N, K, epi, p.tile) if _has_tail(T, p.tile, f16) else (None, None)
+        held.append((ws, tail))
+        p.ws, p.tail_ws, p.tail_cnt = (None if t is None else t.data_ptr() for t in (ws, *tail))
+    wide, square, up, down, row, row3, rowf = (3 * h, h), (h, h), (ffn, h), (h, ffn), (h,), (3 * h,), (ffn,)
+    need = list(zip(_ENCODER_WEIGHTS, (wide, row3, square, row, row, row, up, rowf, down, row, row, row), (dt,) * 12))
+    if q8:
+        need[0], need[6] = ("wqkv_q", wide, FP8), ("w1_q", up, FP8)
+        need += [("wqkv_s", row3, torch.float32), ("w1_s", rowf, torch.float32)]
+    run, at = lib().da_encoder_layer, ctypes.byref(L)
+    for n, layer in enumerate(layers):
+        S = sets[n & 1]
+        L.qkv, L.a, L.f, L.y[:] = S["qkv"].data_ptr(), S["a"].data_ptr(), S["f"].data_ptr(), (S["y0"].data_ptr(), S["y1"].data_ptr())
+        L.x[:] = [t.data_ptr() for t in (x, S["m"], S["x"])]
+        if q8:
+            (L.xq[:], L.xscale[:]) = zip(*(tuple(t.data_ptr() for t in p) for p in (xq, S["m8"], S["x8"])))
+            xq = S["x8"]
+        x = S["x"]
+        for i, (name, shape, dtype) in enumerate(need):
+            t = layer[name]
+            p = t.data_ptr()
+            if t.dtype is not dtype or t.shape != shape or not t.is_cuda or not t.is_contiguous() or (p % 16 and len(shape) == 2):
+                _req(False, f"{name} must be {dtype} {list(shape)} on the GPU, contiguous and aligned")
+            L.w[i] = p
+        _check(run(at, EPI_BIAS, EPI_GELU, EPI_RESID, stream), "encoder_layer")
+    return x
 
 
 def gemm_fp8(aq, sa, wq, sw, bias=None, epi: int = EPI_NONE, resid=None, out=None) -> torch.Tensor:
@@ -1447,12 +1553,12 @@ def gemm_f16(a, w, bias=None, epi: int = EPI_NONE, resid=None, out=None) -> torc
     if out is None:
         out = torch.empty((M, N), dtype=torch.float16, device=a.device)
     _req(out.dtype == torch.float16 and out.shape == (M, N) and out.stride(1) == 1 and out.stride(0) % 8 == 0, "out")
-    if max(K, a.stride(0)) < 1 << 22 and (tile := _dk_rows_tile(M, N, K, epi, True)):
+    tile, splits = _row_choice(M, N, K, epi, a.stride(0), True)
+    if tile in _DK_TILES:
         return _gemm_dk_rows(a, w, bias, epi, resid, out, tile)
     stream = _raw_stream()
-    tile, splits = _row_tile(M, N, K, epi, True) if _row_tiles_ok(M, N) and max(K, a.stride(0)) < 1 << 22 else (0, 1)
     ws = _call_partials(splits, M, N, a)
-    tail = _gemm_tail(a.device, stream, M, N, K, epi, tile) if tile in (7, 10) or (tile == 0 and M >= 256) else (None, None)
+    tail = _gemm_tail(a.device, stream, M, N, K, epi, tile) if _has_tail(M, tile, True) else (None, None)
     _check(lib().da_gemm_f16(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
                              M, N, K, epi, tile, splits, _ptr(ws), *map(_ptr, tail), c_void_p(stream)), "gemm_f16")
     return out

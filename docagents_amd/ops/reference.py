@@ -562,6 +562,10 @@ def gemm_ln_fit(M: int, hidden: int, ffn: int) -> bool:
     return False
 
 
+def encoder_layers_fit(rows: int) -> bool:
+    return False
+
+
 from .seq_reference import (causal_conv, delta_rule, delta_step, delta_step_fits, gated_scan, gemm_any,  # noqa: E402,F401
                             gemm_heads, gemm_partials, latent_attn, latent_flash_fits, latent_prep, partials_fit, rglru_gates, selective_scan,
                             sigmoid_attn, stream_add, stream_final, stream_step)
