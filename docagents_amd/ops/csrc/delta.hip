@@ -402,7 +402,7 @@ DA_EXPORT int da_delta_step(const void* y, int ldy, const void* conv_w, void* co
 //   U  = T (V / rk - (kappa 2^G) S)                                 rows u_t rk_t: what the tokens write
 //   o  = rq ((chi 2^G) S + tril(Q) U)
 //   S <- 2^G_end S + (kappa 2^(G_end - G))^T U
-// delta_prep: a wave per chunk and head forms what does not depend on S (kappa 2^G, chi 2^G, kappa 2^(G_end - G), T, Q), as
+// delta_prep: a workgroup per chunk and head forms what does not depend on S (kappa 2^G, chi 2^G, kappa 2^(G_end - G), T, Q), as
 // MFMA fragments in scratch memory. delta_apply: a wave walks its portion's chunks with 16 columns of V and S by itself,
 // S staying in its accumulators; the waves of a workgroup share the fragments, which are on their way to LDS one and
 // two chunks ahead.
@@ -473,27 +473,34 @@ template <int L> __device__ __forceinline__ float row_lane(float v) {  // lane L
   return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), L << 5 | 0x10));
 }
 
-// LDS of a wave, used in turn: two terms of 32 tokens x 32 channels to be transposed; the solve.
-struct PrepLds {
-  static constexpr int ROW = 80;                                     // bytes of a token's 32 channels
-  static constexpr int SM = 0, SQ = 32 * 36 * 4, SD = 2 * SQ;        // fp32 [32][36] twice, [3][16][17]
-  static constexpr int TOK = SD + 3 * 16 * 17 * 4, BYTES = TOK + 32 * 4;  // b
+// LDS of an item: each wave's (two terms of 32 tokens x 32 channels to be transposed, then what its channels add to M and Q and
+// the tokens' norms), and the solve's.
+template <int KB> struct PrepLds {
+  static constexpr int ROW = 80;                                             // bytes of a token's 32 channels
+  static constexpr int NORMS = 6 * 1024, WAVE = NORMS + 64 * 4;              // [6 blocks][64 lanes][4], then [k, q][32]
+  static constexpr int SM = KB * WAVE, SQ = SM + 32 * 36 * 4, SD = SQ + 32 * 36 * 4;  // fp32 [32][36] twice, [3][16][17]
+  static constexpr int TOK = SD + 3 * 16 * 17 * 4, BYTES = TOK + 32 * 4;     // b
+  static_assert(2 * 32 * ROW <= WAVE, "the staged tile");
 };
-static_assert(2 * 32 * PrepLds::ROW <= PrepLds::TOK, "the staged tile shares the solve's space");
 
+// A workgroup per chunk and head, a wave per 32 channels; then the first wave solves for T while the last one writes Q. Few chunks
+// are bound by the chain of a wave (with one for all channels four loads, each waited for, then the solve), many by memory: the
+// fragments written and the operands read, 550 MB of 192 chunks. us of 4 / 10 / 26 / 64 / 192 chunks of 32 heads, a wave a chunk ->
+// four: 18.5 / 17.8 / 19.2 / 35.6 / 101 -> 11.2 / 13.8 / 18.1 / 33.2 / 96 (at 185 registers, two workgroups a CU, the last four were
+// 12.9 / 20.6 / 36.5 / 108: steep blocks take their values once more).
 template <int KB>
-__global__ void __launch_bounds__(256, 2) delta_prep_kernel(ChunkArgs p) {
+__global__ void __launch_bounds__(64 * KB) delta_prep_kernel(ChunkArgs p) {
   using C = DC<KB>;
+  using P_ = PrepLds<KB>;
   const DeltaArgs& a = p.a;
-  __shared__ __attribute__((aligned(16))) char smem[4 * PrepLds::BYTES];
+  __shared__ __attribute__((aligned(16))) char smem[P_::BYTES];
   constexpr int K = C::K;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, fr = lane & 15, fg = lane >> 4;
-  const int item = blockIdx.x * 4 + wv;
-  if (item >= p.ch.n * a.H) return;  // the waves share nothing: no barriers below
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15, fg = lane >> 4;
+  const int item = blockIdx.x;
   const int ci = item / a.H, h = item % a.H, hk = h / (a.H / a.G);
   const int b = p.ch.ck[2 * ci], s1 = a.m.cu[b + 1], t0 = a.m.cu[b] + p.ch.ck[2 * ci + 1] * CT;
   if (s1 - a.m.cu[b] < a.below) return;
-  char* lds = smem + wv * PrepLds::BYTES;
+  char* lds = smem + wv * P_::WAVE;
   char* out = p.frags + (size_t)item * C::NF * 1024 + lane * 16;
   float* vec = (float*)(p.frags + ((size_t)item * C::NF + C::VEC) * 1024);
   auto wait_own = [] {  // this wave's LDS writes are read back by itself
@@ -531,24 +538,25 @@ __global__ void __launch_bounds__(256, 2) delta_prep_kernel(ChunkArgs p) {
       }
     return r;
   };
+  const float strength = wv == 0 && lane < 32
+                             ? bf2f(((const bf16_t*)a.beta)[(size_t)min(t0 + lane, s1 - 1) * a.ldb + h]) : 0.f;
+  auto half = [&](int i, const u32x2_t& w, int e) {
+    return in[i] ? __uint_as_float(e & 1 ? w[e >> 1] & 0xffff0000u : w[e >> 1] << 16) : 0.f;
+  };
+  int steep = 0;       // diagonal blocks that decay too much for one scale
   f32x4_t M[3], Q[3];  // blocks (0, 0), (1, 1), (1, 0)
 #pragma unroll
   for (int i = 0; i < 3; ++i) M[i] = Q[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float nk[2] = {0.f, 0.f}, nq[2] = {0.f, 0.f};
 
-  Raw next = load(0);
-#pragma unroll 1
-  for (int ks = 0; ks < KB; ++ks) {
-    const Raw r = next;
-    if (ks + 1 < KB) next = load(ks + 1);
+  {
+    const int ks = wv;
+    const Raw r = load(ks);
     Vec8 k[2], q[2], g[2], L[2], P[2], E[2], eT[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      auto half = [&](const u32x2_t& w, int e) {
-        return in[i] ? __uint_as_float(e & 1 ? w[e >> 1] & 0xffff0000u : w[e >> 1] << 16) : 0.f;
-      };
-      k[i] = V8(half(r.k[i][u], e));
-      q[i] = V8(half(r.q[i][u], e));
+      k[i] = V8(half(i, r.k[i][u], e));
+      q[i] = V8(half(i, r.q[i][u], e));
       g[i] = V8(in[i] ? r.g[i][u][e] : 0.f);
 #pragma unroll
       for (int u = 0; u < 2; ++u)
@@ -584,20 +592,7 @@ __global__ void __launch_bounds__(256, 2) delta_prep_kernel(ChunkArgs p) {
         M[i] = mma3(sk, B, M[i]);
         Q[i] = mma3(sq, B, Q[i]);
       } else {
-        const Vec8 l = V8(row_scan(fmaxf(g[i].u[u][e], -24.f)));
-        const Vec8 m0 = V8(row_lane<3>(l.u[u][e])), m1 = V8(row_lane<11>(l.u[u][e]));
-        const bool up = fr >= 8;
-        const Vec8 to = V8(__builtin_amdgcn_exp2f(l.u[u][e] - (up ? m1.u[u][e] : m0.u[u][e])));
-        const Vec8 col = V8(k[i].u[u][e] * __builtin_amdgcn_exp2f((up ? m1.u[u][e] : m0.u[u][e]) - l.u[u][e]));
-        // the step between the middles in two: the factor alone may underflow where the product does not
-        const Vec8 half_step = V8(up ? 1.f : __builtin_amdgcn_exp2f(0.5f * (m1.u[u][e] - m0.u[u][e])));
-        // rows 0 .. 7 against columns 0 .. 7, then rows 8 .. 15 against all
-        Split B = split8(V8(up ? 0.f : col.u[u][e]));
-        M[i] = mma3(split8(V8(up ? 0.f : k[i].u[u][e] * to.u[u][e])), B, M[i]);
-        Q[i] = mma3(split8(V8(up ? 0.f : q[i].u[u][e] * to.u[u][e])), B, Q[i]);
-        B = split8(V8(col.u[u][e] * half_step.u[u][e] * half_step.u[u][e]));
-        M[i] = mma3(split8(V8(up ? k[i].u[u][e] * to.u[u][e] : 0.f)), B, M[i]);
-        Q[i] = mma3(split8(V8(up ? q[i].u[u][e] * to.u[u][e] : 0.f)), B, Q[i]);
+        steep |= 1 << i;
       }
     }
     if (fr == 0)
@@ -607,11 +602,11 @@ __global__ void __launch_bounds__(256, 2) delta_prep_kernel(ChunkArgs p) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const Split v = split8(i ? E[1] : V8(E[0].u[u][e] * eT[1].u[u][e]));
-      char* w = lds + (16 * i + fr) * PrepLds::ROW + fg * 8;
+      char* w = lds + (16 * i + fr) * P_::ROW + fg * 8;
       const u32x4_t hi = __builtin_bit_cast(u32x4_t, v.hi), lo = __builtin_bit_cast(u32x4_t, v.lo);
       *(u32x2_t*)w = u32x2_t{hi[0], hi[1]};
       *(u32x2_t*)(w + 32) = u32x2_t{hi[2], hi[3]};
-      w += 32 * PrepLds::ROW;
+      w += 32 * P_::ROW;
       *(u32x2_t*)w = u32x2_t{lo[0], lo[1]};
       *(u32x2_t*)(w + 32) = u32x2_t{lo[2], lo[3]};
     }
@@ -620,42 +615,97 @@ __global__ void __launch_bounds__(256, 2) delta_prep_kernel(ChunkArgs p) {
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int part = 0; part < 2; ++part) {
-        const char* v = lds + (part * 32 + 4 * fg + (fr >> 2)) * PrepLds::ROW + (c * 16 + 4 * (fr & 3)) * 2;
-        const s16x4_t x = lds_read_tr16(v), y = lds_read_tr16(v + 16 * PrepLds::ROW);
+        const char* v = lds + (part * 32 + 4 * fg + (fr >> 2)) * P_::ROW + (c * 16 + 4 * (fr & 3)) * 2;
+        const s16x4_t x = lds_read_tr16(v), y = lds_read_tr16(v + 16 * P_::ROW);
         *(bf16x8_t*)(out + (C::KM + (2 * ks + c) * 2 + part) * 1024) =
             bf16x8_t{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
       }
-    wait_own();
   }
+  if (steep) {
+    const Raw r = load(wv);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (steep >> i & 1) {
+        const Vec8 k = V8(half(i, r.k[i][u], e)), q = V8(half(i, r.q[i][u], e)), g = V8(in[i] ? r.g[i][u][e] : 0.f);
+        const Vec8 l = V8(row_scan(fmaxf(g.u[u][e], -24.f)));
+        const Vec8 m0 = V8(row_lane<3>(l.u[u][e])), m1 = V8(row_lane<11>(l.u[u][e]));
+        const bool up = fr >= 8;
+        const Vec8 to = V8(__builtin_amdgcn_exp2f(l.u[u][e] - (up ? m1.u[u][e] : m0.u[u][e])));
+        const Vec8 col = V8(k.u[u][e] * __builtin_amdgcn_exp2f((up ? m1.u[u][e] : m0.u[u][e]) - l.u[u][e]));
+        // the step between the middles in two: the factor alone may underflow where the product does not
+        const Vec8 half_step = V8(up ? 1.f : __builtin_amdgcn_exp2f(0.5f * (m1.u[u][e] - m0.u[u][e])));
+        // rows 0 .. 7 against columns 0 .. 7, then rows 8 .. 15 against all
+        Split B = split8(V8(up ? 0.f : col.u[u][e]));
+        M[i] = mma3(split8(V8(up ? 0.f : k.u[u][e] * to.u[u][e])), B, M[i]);
+        Q[i] = mma3(split8(V8(up ? 0.f : q.u[u][e] * to.u[u][e])), B, Q[i]);
+        B = split8(V8(col.u[u][e] * half_step.u[u][e] * half_step.u[u][e]));
+        M[i] = mma3(split8(V8(up ? k.u[u][e] * to.u[u][e] : 0.f)), B, M[i]);
+        Q[i] = mma3(split8(V8(up ? q.u[u][e] * to.u[u][e] : 0.f)), B, Q[i]);
+      }
+  }
+  wait_own();
 
-  // norms and write strengths of the tokens
-  float* sM = (float*)(lds + PrepLds::SM);
-  float* sQ = (float*)(lds + PrepLds::SQ);
-  float* sD = (float*)(lds + PrepLds::SD);
-  float* sB = (float*)(lds + PrepLds::TOK);
+  // the channels' sums, norms and write strengths of the tokens
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    *(f32x4_t*)(lds + i * 1024 + lane * 16) = M[i];
+    *(f32x4_t*)(lds + (3 + i) * 1024 + lane * 16) = Q[i];
+  }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     nk[i] += __shfl_xor(nk[i], 16, 64);
-    nk[i] = sum_xhalf(nk[i]) + a.eps;
+    nk[i] = sum_xhalf(nk[i]);
     nq[i] += __shfl_xor(nq[i], 16, 64);
-    nq[i] = sum_xhalf(nq[i]) + a.eps;
+    nq[i] = sum_xhalf(nq[i]);
     if (fg == 0) {
-      vec[K + 16 * i + fr] = 1.f / sqrtf(nk[i]);
-      vec[K + CT + 16 * i + fr] = a.q_scale / sqrtf(nq[i]);
-      const float bt = bf2f(((const bf16_t*)a.beta)[(size_t)min(t0 + 16 * i + fr, s1 - 1) * a.ldb + h]);
-      sB[16 * i + fr] = in[i] ? sigmoid32(bt) / nk[i] : 0.f;
+      ((float*)(lds + P_::NORMS))[16 * i + fr] = nk[i];
+      ((float*)(lds + P_::NORMS))[32 + 16 * i + fr] = nq[i];
     }
+  }
+  lds_barrier();
+  float* sM = (float*)(smem + P_::SM);
+  float* sQ = (float*)(smem + P_::SQ);
+  float* sD = (float*)(smem + P_::SD);
+  float* sB = (float*)(smem + P_::TOK);
+  auto block = [&](int i) {
+    f32x4_t v = *(const f32x4_t*)(smem + i * 1024 + lane * 16);
+#pragma unroll
+    for (int w = 1; w < KB; ++w) v += *(const f32x4_t*)(smem + w * P_::WAVE + i * 1024 + lane * 16);
+    return v;
+  };
+  if (wv == KB - 1) {  // norms, and Q's lower triangle as fragments
+    float n = 0.f;
+#pragma unroll
+    for (int w = 0; w < KB; ++w) n += ((const float*)(smem + w * P_::WAVE + P_::NORMS))[lane];
+    vec[K + lane] = (lane < 32 ? 1.f : a.q_scale) / sqrtf(n + a.eps);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int r0 = i ? 16 : 0, c0 = i == 1 ? 16 : 0;
+      const f32x4_t q = block(3 + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sQ[(r0 + 4 * fg + e) * 36 + c0 + fr] = q[e];
+    }
+    wait_own();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = 16 * i + fr;
+      put(C::QF + i * 2, split8(V8(16 * u + 4 * fg + e <= r ? sQ[r * 36 + 16 * u + 4 * fg + e] : 0.f)));
+    }
+  }
+  if (wv) return;
+  if (lane < 32) {
+    float n = 0.f;
+#pragma unroll
+    for (int w = 0; w < KB; ++w) n += ((const float*)(smem + w * P_::WAVE + P_::NORMS))[lane];
+    sB[lane] = t0 + lane < s1 ? sigmoid32(strength) / (n + a.eps) : 0.f;
   }
   wait_own();
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const int r0 = i ? 16 : 0, c0 = i == 1 ? 16 : 0;
-    const f32x4_t bt = *(const f32x4_t*)(sB + r0 + 4 * fg);
+    const f32x4_t bt = *(const f32x4_t*)(sB + r0 + 4 * fg), m = block(i);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      sM[(r0 + 4 * fg + e) * 36 + c0 + fr] = M[i][e] * bt[e];
-      sQ[(r0 + 4 * fg + e) * 36 + c0 + fr] = Q[i][e];
-    }
+    for (int e = 0; e < 4; ++e) sM[(r0 + 4 * fg + e) * 36 + c0 + fr] = m[e] * bt[e];
   }
   wait_own();
   // the diagonal blocks' inverses by columns: lanes fg & 1 == blk take block blk, column fr
@@ -672,12 +722,6 @@ __global__ void __launch_bounds__(256, 2) delta_prep_kernel(ChunkArgs p) {
   if (fg < 2)
 #pragma unroll
     for (int r = 0; r < 16; ++r) sD[(blk * 16 + r) * 17 + fr] = x[r];
-  // Q's lower triangle as fragments
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = 16 * i + fr;
-    put(C::QF + i * 2, split8(V8(16 * u + 4 * fg + e <= r ? sQ[r * 36 + 16 * u + 4 * fg + e] : 0.f)));
-  }
   wait_own();
   f32x4_t y{0.f, 0.f, 0.f, 0.f}, z = y;  // the block below the diagonal: -D1 (L10 D0)
 #pragma unroll
@@ -691,15 +735,15 @@ __global__ void __launch_bounds__(256, 2) delta_prep_kernel(ChunkArgs p) {
     z = __builtin_amdgcn_mfma_f32_16x16x4f32(sD[(16 + fr) * 17 + 4 * i + fg], sD[(32 + 4 * i + fg) * 17 + fr], z, 0, 0, 0);
   const float bc = sB[fr], bd = sB[blk * 16 + fr];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) sQ[(16 + 4 * fg + e) * 36 + fr] = -z[e] * bc;
+  for (int e = 0; e < 4; ++e) sM[(16 + 4 * fg + e) * 36 + fr] = -z[e] * bc;
   if (fg < 2)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) sQ[(blk * 16 + r) * 36 + blk * 16 + fr] = x[r] * bd;
+    for (int r = 0; r < 16; ++r) sM[(blk * 16 + r) * 36 + blk * 16 + fr] = x[r] * bd;
   wait_own();
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int r = 16 * i + fr;
-    put(C::TF + i * 2, split8(V8(16 * u + 4 * fg + e <= r ? sQ[r * 36 + 16 * u + 4 * fg + e] : 0.f)));
+    put(C::TF + i * 2, split8(V8(16 * u + 4 * fg + e <= r ? sM[r * 36 + 16 * u + 4 * fg + e] : 0.f)));
   }
 }
 
@@ -894,7 +938,7 @@ static int launch_delta_apply(const ChunkArgs& p, hipStream_t s) {
 template <int KB>
 static int launch_delta_chunk(const ChunkArgs& p, hipStream_t s) {
   const DeltaArgs& a = p.a;
-  delta_prep_kernel<KB><<<(p.ch.n * a.H + 3) / 4, 256, 0, s>>>(p);
+  delta_prep_kernel<KB><<<p.ch.n * a.H, 64 * KB, 0, s>>>(p);
   // a head's columns on one CU where the heads fill the chip, else spread over more
   const long long heads = (long long)a.m.B * a.H;
   if (heads * ((a.V + 127) / 128) >= 256) return launch_delta_apply<KB, 8>(p, s);
