@@ -403,9 +403,9 @@ DA_EXPORT int da_delta_step(const void* y, int ldy, const void* conv_w, void* co
 //   o  = rq ((chi 2^G) S + tril(Q) U)
 //   S <- 2^G_end S + (kappa 2^(G_end - G))^T U
 // delta_prep: a workgroup per chunk and head forms what does not depend on S (kappa 2^G, chi 2^G, kappa 2^(G_end - G), T, Q), as
-// MFMA fragments in scratch memory. delta_apply: a wave walks its portion's chunks with 16 columns of V and S by itself,
-// S staying in its accumulators; the waves of a workgroup share the fragments, which are on their way to LDS one and
-// two chunks ahead.
+// MFMA fragments in scratch memory. delta_apply: a wave (or two, with half of the key channels each) walks its portion's chunks
+// with 16 columns of V and S, S staying in its accumulators; the waves of a workgroup share the fragments, which are on their way
+// to LDS one and two chunks ahead.
 //
 // Every fp32 operand enters its product as two bf16 terms (its rounding and the remainder), three of their four
 // products taken: about 16 bits, accumulated in fp32. The solve of T is in fp32.
@@ -754,33 +754,38 @@ template <int N> __device__ __forceinline__ void vm_wait() {  // all but this wa
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// LDS of NW waves: part A of three chunks (two with 8 waves, whose V takes the space), part B of two; V of the workgroup's
-// columns of two.
-template <int KB, int NW> struct DL {
+// LDS of CG x KS waves: part A of three chunks (two of 128 columns or two slices, whose V or sums take the space), part B of two;
+// V of the workgroup's columns of two; what a slice hands the other.
+template <int KB, int CG, int KS> struct DL {
   using C = DC<KB>;
-  static constexpr int AHEAD = NW == 8 ? 1 : 2, B = (AHEAD + 1) * C::NA, VB = CT * 16 * NW * 2;  // chunks; fragments; bytes
-  static constexpr int V = (B + 2 * C::NB) * 1024, BYTES = V + 2 * VB;
-  static_assert(BYTES <= 160 * 1024, "LDS");
+  static constexpr int NW = CG * KS, AHEAD = CG == 8 || KS > 1 ? 1 : 2;                      // chunks
+  static constexpr int B = (AHEAD + 1) * C::NA, VB = CT * 16 * CG * 2;                       // fragments; bytes
+  static constexpr int V = (B + 2 * C::NB) * 1024, X = V + 2 * VB, BYTES = X + (KS > 1 ? NW * 3072 : 0);
+  static_assert(BYTES <= 160 * 1024 && KB % KS == 0 && KS <= 2, "LDS");
 };
 
-template <int KB, int NW>  // NW waves
-__global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) delta_apply_kernel(ChunkArgs p) {
+template <int KB, int CG, int KS>  // CG groups of 16 columns, each by one wave or by two that take half of the key channels
+__global__ void __launch_bounds__(64 * CG * KS, CG * KS >= 8 ? 2 : 1) delta_apply_kernel(ChunkArgs p) {
   using C = DC<KB>;
-  using D = DL<KB, NW>;
+  using D = DL<KB, CG, KS>;
+  constexpr int NW = CG * KS, SB = KB / KS;  // waves; 32-channel blocks of a slice
   const DeltaArgs& a = p.a;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int K = C::K;
-  const int b = blockIdx.z, h = blockIdx.y;
+  // the workgroups of a head are neighbours on one XCD: its L2 brings their fragments once
+  const int at = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+  const int b = blockIdx.z, h = at / (int)gridDim.x, bx = at % (int)gridDim.x;
   const int t0 = a.m.cu[b], t1 = a.m.cu[b + 1];
   if (t1 - t0 < a.below) return;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, fr = lane & 15, fg = lane >> 4;
-  const int col = blockIdx.x * NW * 16 + wv * 16 + fr, colc = min(col, a.V - 1);
+  const int cg = wv / KS, sl = wv % KS;
+  const int col = bx * CG * 16 + cg * 16 + fr, colc = min(col, a.V - 1);
   const bool live = col < a.V;
-  float* st = a.state + (((size_t)a.m.slot[b] * a.H + h) * a.V + colc) * K + 4 * fg;
-  f32x4_t S[2 * KB];
+  float* st = a.state + (((size_t)a.m.slot[b] * a.H + h) * a.V + colc) * K + sl * SB * 32 + 4 * fg;
+  f32x4_t S[2 * SB];
   const bool stored = a.m.pos0[b] != 0;
 #pragma unroll
-  for (int i = 0; i < 2 * KB; ++i) {
+  for (int i = 0; i < 2 * SB; ++i) {
     S[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     if (stored) S[i] = *(const f32x4_t*)(st + 16 * i);
   }
@@ -807,23 +812,26 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) delta_apply_kernel(C
       __builtin_amdgcn_global_load_lds((frag_g_t)(from + f * 1024), (frag_l_t)(to + f * 1024), 16, 0, 0);
     }
   };
-  // V's tokens x columns, one instruction a wave: 16 bytes a lane, 2 NW lanes a token
+  // V's tokens x columns, one instruction a wave of the first CG: 16 bytes a lane, 2 CG lanes a token
   auto issue_v = [&](int k) {
-    const int i = wv * 64 + lane, c = min(blockIdx.x * NW * 16 + i % (2 * NW) * 8, a.V - 8);
-    const bf16_t* from = (const bf16_t*)a.x + (size_t)min(t0 + min(k, nc - 1) * CT + i / (2 * NW), t1 - 1) * a.ldx + 2 * a.G * K +
+    if (wv >= CG) return;
+    const int i = wv * 64 + lane, c = min(bx * CG * 16 + i % (2 * CG) * 8, a.V - 8);
+    const bf16_t* from = (const bf16_t*)a.x + (size_t)min(t0 + min(k, nc - 1) * CT + i / (2 * CG), t1 - 1) * a.ldx + 2 * a.G * K +
                          h * a.V + c;
     __builtin_amdgcn_global_load_lds((frag_g_t)from, (frag_l_t)(smem + D::V + (k & 1) * D::VB + wv * 1024), 16, 0, 0);
   };
+  constexpr int NO = KS > 1 ? 1 : 2;  // blocks of 16 tokens that this wave reads out, from block sl on
   f32x4_t O[2];
   auto store_o = [&](int t) {
     if (!live) return;
+    t += 16 * sl;
     bf16_t* o = (bf16_t*)a.o + (size_t)(t + 4 * fg) * a.ldo + h * a.V + col;
-    if (t + CT <= t1) {
+    if (t + 16 * NO <= t1) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[(size_t)((i >> 2) * 16 + (i & 3)) * a.ldo] = f2bf(O[i >> 2][i & 3]);
+      for (int i = 0; i < 4 * NO; ++i) o[(size_t)((i >> 2) * 16 + (i & 3)) * a.ldo] = f2bf(O[i >> 2][i & 3]);
     } else {
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < 4 * NO; ++i)
         if (t + 4 * fg + (i >> 2) * 16 + (i & 3) < t1) o[(size_t)((i >> 2) * 16 + (i & 3)) * a.ldo] = f2bf(O[i >> 2][i & 3]);
     }
   };
@@ -847,17 +855,16 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) delta_apply_kernel(C
     auto load_ks = [&](int ks) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        kp[ks & 1][i] = frag(C::KP + (i * KB + ks) * 2);
-        qp[ks & 1][i] = frag(C::QP + (i * KB + ks) * 2);
+        kp[ks & 1][i] = frag(C::KP + (i * KB + sl * SB + ks) * 2);
+        qp[ks & 1][i] = frag(C::QP + (i * KB + sl * SB + ks) * 2);
       }
     };
     load_ks(0);
     f32x4_t rk[2], rq[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      rk[i] = *(const f32x4_t*)(vec + K + 16 * i + 4 * fg);
-      rq[i] = *(const f32x4_t*)(vec + K + CT + 16 * i + 4 * fg);
-    }
+    for (int i = 0; i < 2; ++i) rk[i] = *(const f32x4_t*)(vec + K + 16 * i + 4 * fg);
+#pragma unroll
+    for (int i = 0; i < NO; ++i) rq[i] = *(const f32x4_t*)(vec + K + CT + 16 * (sl + i) + 4 * fg);
     if (k) store_o(t - CT);
     issue_b(k + 1);
     issue_v(k + 1);
@@ -866,15 +873,14 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) delta_apply_kernel(C
 #pragma unroll
     for (int i = 0; i < 2; ++i) R[i] = O[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < KB; ++ks) {
-      if (ks + 1 < KB) {
+    for (int ks = 0; ks < SB; ++ks) {
+      if (ks + 1 < SB) {
         load_ks(ks + 1);
       } else {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          tf[i] = frag(C::TF + i * 2);
-          qf[i] = frag(C::QF + i * 2);
-        }
+        for (int i = 0; i < 2; ++i) tf[i] = frag(C::TF + i * 2);
+#pragma unroll
+        for (int i = 0; i < NO; ++i) qf[i] = frag(C::QF + (sl + i) * 2);
       }
       __builtin_amdgcn_sched_barrier(0);
       const Split B = split8(S[2 * ks], S[2 * ks + 1]);
@@ -885,17 +891,29 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) delta_apply_kernel(C
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    constexpr int PRE = 2 * KB < 4 ? 2 * KB : 4;
-    f32x4_t end[2 * KB];
+    char* hand = smem + D::X + lane * 16;  // to the other slice: its share of the sums, and of the block that the other reads out
+    if constexpr (KS > 1) {
 #pragma unroll
-    for (int i = 0; i < PRE; ++i) km[i] = frag(C::KM + i * 2);
+      for (int i = 0; i < 3; ++i) *(f32x4_t*)(hand + (wv * 3 + i) * 1024) = i < 2 ? R[i] : sl ? O[0] : O[1];
+    }
+    constexpr int PRE = 2 * SB < 4 ? 2 * SB : 4;
+    f32x4_t end[2 * SB];
 #pragma unroll
-    for (int i = 0; i < 2 * KB; ++i) end[i] = *(const f32x4_t*)(vec + 16 * i + 4 * fg);
-    const bf16_t* vl = (const bf16_t*)(smem + D::V + (k & 1) * D::VB) + 4 * fg * 16 * NW + wv * 16 + fr;
+    for (int i = 0; i < PRE; ++i) km[i] = frag(C::KM + (2 * SB * sl + i) * 2);
+#pragma unroll
+    for (int i = 0; i < 2 * SB; ++i) end[i] = *(const f32x4_t*)(vec + 16 * (2 * SB * sl + i) + 4 * fg);
+    const bf16_t* vl = (const bf16_t*)(smem + D::V + (k & 1) * D::VB) + 4 * fg * 16 * CG + cg * 16 + fr;
     unsigned rv[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) rv[i] = vl[((i >> 2) * 16 + (i & 3)) * 16 * NW];
+    for (int i = 0; i < 8; ++i) rv[i] = vl[((i >> 2) * 16 + (i & 3)) * 16 * CG];
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (KS > 1) {  // (either order gives the same sum: both go on with the same U)
+      lds_barrier();
+      const char* other = hand + (wv ^ 1) * 3072;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) R[i] += *(const f32x4_t*)(other + i * 1024);
+      O[0] = (sl ? O[1] : O[0]) + *(const f32x4_t*)(other + 2048);
+    }
     f32x4_t X[2], U[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -908,42 +926,48 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) delta_apply_kernel(C
     for (int i = 0; i < 2; ++i) U[i] = mma3(tf[i], B, f32x4_t{0.f, 0.f, 0.f, 0.f});
     B = split8(U[0], U[1]);
 #pragma unroll
-    for (int i = 0; i < 2 * KB; ++i) S[i] *= end[i];
+    for (int i = 0; i < 2 * SB; ++i) S[i] *= end[i];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) O[i] = mma3(qf[i], B, O[i]) * rq[i];
+    for (int i = 0; i < NO; ++i) O[i] = mma3(qf[i], B, O[i]) * rq[i];
 #pragma unroll
-    for (int i = 0; i < 2 * KB; ++i) {
+    for (int i = 0; i < 2 * SB; ++i) {
       S[i] = mma3(km[i % PRE], B, S[i]);
-      if (i + PRE < 2 * KB) km[i % PRE] = frag(C::KM + (i + PRE) * 2);
+      if (i + PRE < 2 * SB) km[i % PRE] = frag(C::KM + (2 * SB * sl + i + PRE) * 2);
     }
   }
   store_o(t0 + (nc - 1) * CT);
   if (live)
 #pragma unroll
-    for (int i = 0; i < 2 * KB; ++i) *(f32x4_t*)(st + 16 * i) = S[i];
+    for (int i = 0; i < 2 * SB; ++i) *(f32x4_t*)(st + 16 * i) = S[i];
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no transfer to LDS outlives its workgroup
-  const int wg = blockIdx.y * gridDim.x + blockIdx.x, step = gridDim.x * gridDim.y * 64 * NW;
+  const int wg = at, step = gridDim.x * gridDim.y * 64 * NW;
   for (int c = wg * 64 * NW + threadIdx.x; c < a.conv.C; c += step) conv_state_store<bf16_t>(a.conv, a.m, b, c);
 }
 
-template <int KB, int NW>
+template <int KB, int CG, int KS>
 static int launch_delta_apply(const ChunkArgs& p, hipStream_t s) {
-  static const hipError_t e = hipFuncSetAttribute((const void*)delta_apply_kernel<KB, NW>,
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, DL<KB, NW>::BYTES);
+  using D = DL<KB, CG, KS>;
+  static const hipError_t e = hipFuncSetAttribute((const void*)delta_apply_kernel<KB, CG, KS>,
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, D::BYTES);
   if (e != hipSuccess) return (int)e;
   const DeltaArgs& a = p.a;
-  delta_apply_kernel<KB, NW><<<dim3((a.V + 16 * NW - 1) / (16 * NW), a.H, a.m.B), 64 * NW, DL<KB, NW>::BYTES, s>>>(p);
+  delta_apply_kernel<KB, CG, KS><<<dim3((a.V + 16 * CG - 1) / (16 * CG), a.H, a.m.B), 64 * D::NW, D::BYTES, s>>>(p);
   DA_LAUNCH_CHECK();
 }
 template <int KB>
 static int launch_delta_chunk(const ChunkArgs& p, hipStream_t s) {
   const DeltaArgs& a = p.a;
   delta_prep_kernel<KB><<<p.ch.n * a.H, 64 * KB, 0, s>>>(p);
-  // a head's columns on one CU where the heads fill the chip, else spread over more
+  // A head's columns on one CU where the heads fill the chip, else spread over more, and the channels of few heads over two waves.
+  // A chunk takes a wave 2.2 us with all of them (1.6 without its loads: 84 MFMAs and as much again on the vector ALU), 1.8 with
+  // half and two groups of columns a workgroup, 1.65 with one; four slices read too much LDS (2.2). us of 10 / 26 / 64 chunks of
+  // 32 heads, and 32 of 64: whole 27.8 / 62.4 / 142 / 79, halves of two groups 22.1 / 50.4 / 117 / 63.6, of one 21.0 / 46.7 / 108 /
+  // 110 (more workgroups than CUs); 32 of 128: four whole groups 95, two halves 144.
   const long long heads = (long long)a.m.B * a.H;
-  if (heads * ((a.V + 127) / 128) >= 256) return launch_delta_apply<KB, 8>(p, s);
-  if (heads * ((a.V + 63) / 64) >= 256) return launch_delta_apply<KB, 4>(p, s);
-  return launch_delta_apply<KB, 2>(p, s);
+  if (heads * ((a.V + 127) / 128) >= 256) return launch_delta_apply<KB, 8, 1>(p, s);
+  if (heads * ((a.V + 63) / 64) >= 256) return launch_delta_apply<KB, 4, 1>(p, s);
+  if (KB % 2 == 0 && heads * ((a.V + 15) / 16) <= 256) return launch_delta_apply<KB, 1, KB % 2 ? 1 : 2>(p, s);
+  return launch_delta_apply<KB, 2, KB % 2 ? 1 : 2>(p, s);
 }
 
 // o / rms(o) * w * sigmoid(gate), in place, per head: `lanes` lanes a head, U pieces of 4 columns of theirs in registers.
