@@ -37,7 +37,10 @@ struct DkArgs {
   const bf16_t* A; const bf16_t* W; bf16_t* C;
   const bf16_t* bias; const bf16_t* resid;
   const float* ssq_in;  // nullable: [ssq_parts][64] partial sums of squares of A's rows
-  float* ssq_out;       // EPI_RESID (nullable): [gridDim.x][64] sums of squares of this tile's output rows
+  float* ssq_out;       // EPI_RESID (nullable): [N / ssq_bn][64] sums of squares of the output rows, by ssq_bn columns
+  float* ws;            // SPLIT: the workgroups' sums, and a counter per tile that is 0 between launches
+  int* cnt;
+  int splits, ssq_bn;
   int M, N, K, lda, ldc, ldr, ssq_parts, norm_k;
   float eps;
   int relu;  // EPI_SWIGLU: the gate's activation is relu, not silu
@@ -50,9 +53,15 @@ template <typename T> __device__ __forceinline__ f32x4_t unpack4(const u32x2_t& 
 
 // ST stages of a wave's ring, each BM rows of A and BN of W; row r's 16-B chunk c at slot c ^ (r >> 1 & 7), so that the 16
 // rows of a fragment read land on all banks
+// SPLIT: K by `splits` workgroups as well. Each leaves its sums and counts; the last to come, which nobody waits for, adds them up
+// in order and has the epilogue: 2.5 us that a long K repays, whose workgroups otherwise read all of A for few columns each. The
+// sums go past the XCDs' L2s (sc1) to where all of them see them. us of 32 / 24 / 17 rows, whole -> split (tiles of 64 columns by
+// 4 or 5; of 32 by 4 below 3072): 4096 x 14336 29.6 / 27.3 / 26.6 -> 25.9 / 25.1 / 25.5, 3072 x 8192 16.2 / 14.9 / 15.3 -> 15.3 /
+// 15.1 / 14.9, 2048 x 8192 15.4 / 14.0 / 13.9 -> 11.2 / 10.9 / 11.1, 1024 x 4096 9.4 / 8.8 / 8.1 -> 7.9 / 7.8 / 7.8; not 4096 x
+// 8192 (16.8 -> 17.9), 4096 x 4096 (11.0 -> 11.0), nor 33 rows and more, whose streaming tiles share A (4096 x 14336, 64: 28.1, 31.7).
 // ROWS: more than one block of BM rows (gridDim.y of them; W's lines are worth a place in the caches then). The blocks of a column
 // tile are neighbours on one XCD.
-template <int FM, int FN, int NW, int ST, int EPI, typename T, bool ROWS>
+template <int FM, int FN, int NW, int ST, int EPI, typename T, bool ROWS, bool SPLIT>
 __global__ void __launch_bounds__(64 * NW)
 gemm_dk_kernel(DkArgs p) {
   constexpr int BM = 16 * FM, BN = 16 * FN, A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128;
@@ -63,7 +72,8 @@ gemm_dk_kernel(DkArgs p) {
   __shared__ __attribute__((aligned(16))) char smem[RING > SUMS ? RING : SUMS];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fg = lane >> 4;
-  int tile = blockIdx.x;
+  int tile = SPLIT ? blockIdx.x / p.splits : blockIdx.x;
+  const int first = SPLIT ? blockIdx.x % p.splits * NW + w : w, every = SPLIT ? NW * p.splits : NW;  // this wave's K-steps
   if constexpr (ROWS) {
     const int t = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y), m0 = t % (int)gridDim.y * BM;
     tile = t / (int)gridDim.y;
@@ -96,9 +106,9 @@ gemm_dk_kernel(DkArgs p) {
   const char* Wt = (const char*)p.W + (size_t)n0 * p.K * 2;
   char* ring = smem + w * ST * STAGE;
   const int rot = nk >= 64 && nk % 32 == 0 ? (tile >> 3) * 4 % nk : 0;  // the K-step that this tile begins with
-  const int mine = (nk - w + NW - 1) / NW;                              // of this wave
+  const int mine = max(nk - first + every - 1, 0) / every;              // of this wave
   auto issue = [&](int i, int slot) __attribute__((always_inline)) {  // (past the wave's last: no transfer)
-    int step = w + i * NW + rot;
+    int step = first + i * every + rot;
     step = step >= nk ? step - nk : step;
     const int n = i < mine ? 0x7fffff00 : 0;
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, (short)0, n, 0x00020000);
@@ -176,6 +186,51 @@ gemm_dk_kernel(DkArgs p) {
 
   constexpr int BNO = EPI == EPI_SWIGLU ? BN / 2 : BN;  // output columns of the tile
   constexpr int CPR = BNO / 4;                          // 4-column pieces of a row
+  if constexpr (SPLIT) {  // (a thread's pieces here are its pieces below)
+    static_assert(EPI != EPI_SWIGLU && !ROWS && BM * CPR % (64 * NW) == 0, "split");
+    constexpr int IT = BM * CPR / (64 * NW);
+    constexpr unsigned TB = IT * 64 * NW * 16;
+    f32x4_t v[IT];
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+      const int t = tid + i * 64 * NW;
+      v[i] = *(const f32x4_t*)&red[0][t / CPR][t % CPR * 4];
+#pragma unroll
+      for (int x = 1; x < NW; ++x) v[i] += *(const f32x4_t*)&red[x][t / CPR][t % CPR * 4];
+    }
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)p.ws, (short)0, gridDim.x * TB, 0x00020000);
+    const unsigned at = tid * 16u;
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v[i]), rs, at + i * 1024 * NW, blockIdx.x * TB, 16);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores are done; then every wave's
+    __syncthreads();
+    int* last = (int*)(smem + RED);
+    if (tid == 0) *last = __hip_atomic_fetch_add(p.cnt + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == p.splits - 1;
+    __syncthreads();
+    if (!*(volatile int*)last) return;
+    if (tid == 0) __hip_atomic_store(p.cnt + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int i = 0; i < IT; ++i) v[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int q0 = 0; q0 < p.splits; q0 += 4) {
+      u32x4_t x[4][IT];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < IT; ++i)
+          x[q][i] = __builtin_amdgcn_raw_buffer_load_b128(rs, at + i * 1024 * NW, (tile * p.splits + min(q0 + q, p.splits - 1)) * TB, 16);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (q0 + q < p.splits)
+#pragma unroll
+          for (int i = 0; i < IT; ++i) v[i] += __builtin_bit_cast(f32x4_t, x[q][i]);
+    }
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+      const int t = tid + i * 64 * NW;
+      *(f32x4_t*)&red[0][t / CPR][t % CPR * 4] = v[i];
+    }
+  }
   static_assert(EPI != EPI_RESID || ROWS || (CPR & (CPR - 1)) == 0, "a row's pieces meet by lane exchange");
 #pragma unroll 1
   for (int t = tid; t < BM * CPR; t += 64 * NW) {
@@ -190,7 +245,7 @@ gemm_dk_kernel(DkArgs p) {
     auto total = [&](int col) {
       f32x4_t v = *(const f32x4_t*)&red[0][m][col];
 #pragma unroll
-      for (int x = 1; x < NW; ++x) v += *(const f32x4_t*)&red[x][m][col];
+      for (int x = 1; x < (SPLIT ? 1 : NW); ++x) v += *(const f32x4_t*)&red[x][m][col];
       return v;
     };
     auto bias4 = [&](int col) {  // columns of the product
@@ -224,8 +279,9 @@ gemm_dk_kernel(DkArgs p) {
         float q = (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]);
         if (!ok) q = 0.f;
 #pragma unroll
-        for (int x = 1; x < CPR; x <<= 1) q += __shfl_xor(q, x, 64);
-        if (c == 0 && m < p.M) p.ssq_out[(size_t)tile * 64 + m] = q;
+        for (int x = 1; x < CPR; x <<= 1)
+          if (x < p.ssq_bn / 4) q += __shfl_xor(q, x, 64);
+        if (c % p.ssq_bn == 0 && m < p.M && gn < p.N) p.ssq_out[(size_t)(gn / p.ssq_bn) * 64 + m] = q;
       }
     }
   }
@@ -242,7 +298,17 @@ template <int FM, int FN, int EPI>
 static int dk_launch3(const DkArgs& a, hipStream_t s) {
   // four waves, as many stages as leave a CU room for two workgroups; at least two, of which one is read
   constexpr int STAGE = (FM + FN) * 2048, FIT = 81920 / (4 * STAGE), ST = FIT < 2 ? 2 : FIT > 4 ? 4 : FIT;
-  gemm_dk_kernel<FM, FN, 4, ST, EPI, BF16T, false><<<(a.N + 16 * FN - 1) / (16 * FN), 256, 0, s>>>(a);
+  gemm_dk_kernel<FM, FN, 4, ST, EPI, BF16T, false, false><<<(a.N + 16 * FN - 1) / (16 * FN), 256, 0, s>>>(a);
+  return (int)hipGetLastError();
+}
+
+template <int FN>
+static int dk_split(const DkArgs& a, int epi, hipStream_t s) {
+  constexpr int FM = 2, STAGE = (FM + FN) * 2048, FIT = 81920 / (4 * STAGE), ST = FIT < 2 ? 2 : FIT > 4 ? 4 : FIT;
+  const int blocks = (a.N + 16 * FN - 1) / (16 * FN) * a.splits;
+  if (epi == EPI_RESID) gemm_dk_kernel<FM, FN, 4, ST, EPI_RESID, BF16T, false, true><<<blocks, 256, 0, s>>>(a);
+  else if (epi == EPI_NONE || epi == EPI_BIAS) gemm_dk_kernel<FM, FN, 4, ST, EPI_NONE, BF16T, false, true><<<blocks, 256, 0, s>>>(a);
+  else return (int)hipErrorInvalidValue;
   return (int)hipGetLastError();
 }
 
@@ -271,9 +337,15 @@ DA_EXPORT int da_gemm_dk_parts(int N) {
 // epi: EPI_NONE / EPI_BIAS / EPI_RESID / EPI_SWIGLU. ssq_in (nullable): deferred RMSNorm of A's rows
 // over ssq_parts parts (norm over norm_k columns, eps); ssq_out (nullable, EPI_RESID only):
 // [da_gemm_dk_parts(N)][64] floats. 1 <= M <= 64, K % 64 == 0, N % 16 == 0 (SwiGLU: N % 32 == 0).
+// splits > 0 (17 - 32 rows, not SwiGLU, no ssq_in): tiles of 16 fn columns (fn 2 or 4), K by as many workgroups; ws: da_gemm_dk_ws
+// bytes, cnt: a zero per tile.
+DA_EXPORT size_t da_gemm_dk_ws(int N, int fn, int splits) {
+  return (size_t)((N + 16 * fn - 1) / (16 * fn)) * splits * (32 * 16 * fn * 4);
+}
+
 DA_EXPORT int da_gemm_dk(const void* A, int lda, const void* W, void* C, int ldc, const void* bias,
                          const void* resid, int ldr, int M, int N, int K, int epi, const float* ssq_in, int ssq_parts,
-                         int norm_k, float eps, float* ssq_out, void* stream) {
+                         int norm_k, float eps, float* ssq_out, int fn, int splits, void* ws, void* cnt, void* stream) {
   if (M < 1 || M > 64 || K < 64 || K % 64 || N < 16 || N % 16 || lda % 8 || ldc % 8) return (int)hipErrorInvalidValue;
   const int relu = epi == EPI_REGLU;
   if (relu) epi = EPI_SWIGLU;
@@ -281,15 +353,23 @@ DA_EXPORT int da_gemm_dk(const void* A, int lda, const void* W, void* C, int ldc
   if (epi == EPI_RESID && (!resid || ldr % 8)) return (int)hipErrorInvalidValue;
   if (ssq_out && epi != EPI_RESID) return (int)hipErrorInvalidValue;
   if (ssq_in && (ssq_parts < 1 || norm_k < 1 || !(eps > 0.f))) return (int)hipErrorInvalidValue;
+  const int ssq_fn = dk_fn(N, epi);
+  if (splits < 0 || splits > 64 ||
+      (splits && (M <= 16 || M > 32 || ssq_in || !ws || !cnt || (fn != 2 && fn != 4) || (ssq_out && (ssq_fn > fn || N % (16 * ssq_fn))))))
+    return (int)hipErrorInvalidValue;
   // a tile's rows within the resource's reach
-  if (2ll * ((M - 1) * (long long)lda + K) > 0x7ffff000ll || 32ll * dk_fn(N, epi) * K > 0x7ffff000ll) return (int)hipErrorInvalidValue;
+  if (2ll * ((M - 1) * (long long)lda + K) > 0x7ffff000ll || 32ll * (splits ? fn : ssq_fn) * K > 0x7ffff000ll ||
+      (splits && da_gemm_dk_ws(N, fn, splits) > 0x7ffff000u))
+    return (int)hipErrorInvalidValue;
   DkArgs a{};
   a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = (bf16_t*)C;
   a.bias = (const bf16_t*)bias; a.resid = (const bf16_t*)resid;
   a.ssq_in = ssq_in; a.ssq_out = ssq_out;
   a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc; a.ldr = ldr;
   a.ssq_parts = ssq_parts; a.norm_k = norm_k; a.eps = eps; a.relu = relu;
+  a.ws = (float*)ws; a.cnt = (int*)cnt; a.splits = splits; a.ssq_bn = 16 * ssq_fn;
   hipStream_t s = (hipStream_t)stream;
+  if (splits) return fn == 2 ? dk_split<2>(a, epi, s) : dk_split<4>(a, epi, s);
   if (M <= 16) return dk_launch1<1>(a, epi, s);
   if (M <= 32) return dk_launch1<2>(a, epi, s);
   if (M <= 48) return dk_launch1<3>(a, epi, s);
@@ -299,7 +379,7 @@ DA_EXPORT int da_gemm_dk(const void* A, int lda, const void* W, void* C, int ldc
 template <int FM, int FN, int ST, typename T>
 static int dk_rows(const DkArgs& a, int epi, hipStream_t s) {
   const dim3 grid((a.N + 16 * FN - 1) / (16 * FN), (a.M + 16 * FM - 1) / (16 * FM));
-#define DK_ROWS(E) gemm_dk_kernel<FM, FN, 4, ST, E, T, true><<<grid, 256, 0, s>>>(a)
+#define DK_ROWS(E) gemm_dk_kernel<FM, FN, 4, ST, E, T, true, false><<<grid, 256, 0, s>>>(a)
   switch (epi) {
     case EPI_NONE: case EPI_BIAS: DK_ROWS(EPI_NONE); break;
     case EPI_GELU: DK_ROWS(EPI_GELU); break;

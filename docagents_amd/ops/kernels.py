@@ -63,7 +63,8 @@ _SIGS = {
                          c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
     "da_malloc_uncached": [c_longlong, ctypes.POINTER(c_void_p)],
     "da_gemm_dk": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
-                   c_int, c_void_p, c_int, c_int, c_float, c_void_p, c_void_p],
+                   c_int, c_void_p, c_int, c_int, c_float, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p],
+    "da_gemm_dk_ws": [c_int] * 3,
     "da_gemm_dk_parts": [c_int],
     "da_gemm_dk_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 7 + [c_void_p],
     "da_enc_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5
@@ -281,7 +282,11 @@ def _gemm_tail(device, stream: int, M: int, N: int, K: int, epi: int, tile: int 
     nbytes = _tail_bytes(M, N, K, epi, tile) if K >= TAIL_MIN_K else 0
     if not nbytes:
         return None, None
-    part = torch.empty(nbytes // 4, dtype=torch.float32, device=device)
+    return torch.empty(nbytes // 4, dtype=torch.float32, device=device), _counters(device, stream)
+
+
+def _counters(device, stream: int):
+    """The 256 * 8 counters, 0 between launches, of the current stream ``stream``."""
     key = (device.index, stream)
     if torch.cuda.is_current_stream_capturing():
         capture = lib().da_gemm_capture_id(stream)
@@ -289,7 +294,7 @@ def _gemm_tail(device, stream: int, M: int, N: int, K: int, epi: int, tile: int 
         if had != capture:
             cnt = torch.zeros(256 * 8, dtype=torch.int32, device=device)
             _TAIL_CAPTURED[key] = capture, cnt
-        return part, cnt
+        return cnt
     cnt = _TAIL.get(key)
     if cnt is None:
         cnt = torch.zeros(256 * 8, dtype=torch.int32, device=device)
@@ -297,7 +302,7 @@ def _gemm_tail(device, stream: int, M: int, N: int, K: int, epi: int, tile: int 
             cnt = _TAIL.setdefault(key, cnt)
             while len(_TAIL) > TAIL_STREAMS:
                 del _TAIL[next(iter(_TAIL))]
-    return part, cnt
+    return cnt
 
 
 def _call_scratch(nbytes: int, like) -> torch.Tensor:
@@ -436,6 +441,15 @@ def _dk_whole(M: int, N: int, K: int) -> bool:
     return N <= 16384 and K <= 4096
 
 
+def _dk_split(M: int, N: int, K: int, epi: int):
+    """(16-column groups of a tile, workgroups that share its K) of 17..32 rows on gemm_dk, (0, 0): K whole. Where K is at
+    least 2.5 N; fewer columns than 1024 leave tiles of too few steps (measured: csrc/gemm_dk.hip)."""
+    if not (16 < M <= 32 and 1024 <= N <= 8192 and N % 64 == 0 and 2 * K >= 5 * N and epi in (EPI_NONE, EPI_BIAS, EPI_RESID)):
+        return 0, 0
+    fn = 4 if N >= 3072 else 2
+    return fn, min(256 // (N // (16 * fn)), 6)
+
+
 def _dk_splitk(M: int, N: int) -> bool:
     return DK_SPLITK_ABOVE < M <= 64 and N % 512 == 0
 
@@ -508,8 +522,13 @@ def gemm_dk(a, w, epi: int = EPI_NONE, bias=None, resid=None, out=None, norm_in=
                                        ldr, M, N, K, epi, _ptr(ssq), parts, K, float(eps), _ptr(ssq_out), _ptr(ws),
                                        splits, _stream()), "gemm_dk_splitk")
         return out
+    stream, ws, cnt = _raw_stream(), None, None
+    fn, splits = _dk_split(M, N, K, epi) if ssq is None else (0, 0)
+    if splits:
+        ws, cnt = _call_scratch(int(lib().da_gemm_dk_ws(N, fn, splits)), a), _counters(a.device, stream)
     _check(lib().da_gemm_dk(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
-                            M, N, K, epi, _ptr(ssq), parts, K, float(eps), _ptr(ssq_out), _stream()), "gemm_dk")
+                            M, N, K, epi, _ptr(ssq), parts, K, float(eps), _ptr(ssq_out), fn, splits, _ptr(ws), _ptr(cnt),
+                            c_void_p(stream)), "gemm_dk")
     return out
 
 

@@ -1,0 +1,49 @@
+"""Decode products of 17 to 32 rows and a long K, shared by workgroups of which the last to come adds up."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from docagents_amd.ops import kernels as K  # noqa: E402
+
+
+# tiles of 32 and 64 columns; the fewest and most workgroups a tile; K-steps that they share unevenly, and the first N below and above the line
+@pytest.mark.parametrize("N,Kd", [(1024, 2560), (2048, 8192), (3008, 7680), (3072, 8192), (4096, 14336), (4160, 10496), (8192, 20480)])
+@pytest.mark.parametrize("M", [17, 25, 32])
+def test_split_products(M, N, Kd):
+    assert K._dk_split(M, N, Kd, K.EPI_RESID)[1] >= 2
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    a = torch.randn(M, Kd, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(N, Kd, device="cuda", generator=g) * Kd ** -0.5).bfloat16()
+    x = torch.randn(M, N, device="cuda", generator=g).bfloat16()
+    b = torch.randn(N, device="cuda", generator=g).bfloat16()
+    ref = a.double() @ w.double().T
+    mag = (a.double().abs() @ w.double().abs().T).max()
+    near = lambda got, want: ((got.double() - want).abs()  # noqa: E731  (one rounding, and fp32 sums of Kd products)
+                              <= 2.0 ** -8 * want.abs() + 8 * Kd * 2.0 ** -24 * mag).all()
+    parts = K.dk_parts(N, M)
+    ssq = torch.full((parts + 1, 64), -1.0, device="cuda")
+    for _ in range(3):  # (the counters are 0 again after each)
+        got = K.gemm_dk(a, w, epi=K.EPI_RESID, resid=x, ssq_out=ssq)
+        assert near(got, ref + x.double())
+        want = got.double().square().view(M, parts, -1).sum(2).T
+        assert ((ssq[:parts, :M].double() - want).abs() <= 1e-5 * want).all() and (ssq[parts] == -1).all()
+        assert near(K.gemm(a, w), ref) and near(K.gemm(a, w, bias=b, epi=K.EPI_BIAS), ref + b.double())
+
+
+def test_split_products_replayed():
+    M, N, Kd = 24, 3072, 8192
+    a, w = torch.randn(M, Kd, device="cuda").bfloat16(), torch.randn(N, Kd, device="cuda").bfloat16()
+    want = K.gemm(a, w)
+    torch.cuda.synchronize()
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            one = K.gemm(a, w)
+            two = K.gemm(a, w)
+    for _ in range(4):
+        one.zero_(), two.zero_()
+        graph.replay()
+        other = K.gemm(a, w)  # (the same product on the counters of its own stream)
+        torch.cuda.synchronize()
+        assert torch.equal(one, want) and torch.equal(two, want) and torch.equal(other, want)
