@@ -954,7 +954,7 @@ DA_EXPORT int da_gemm_dk_splitk(const void* A, int lda, const void* W, void* C, 
 }
 
 // A . W^T left as `splits` fp32 partials [splits][M][N] in ws (splits = 1: the product itself) for a consumer
-// that sums them in its own pass. Decode-sized tiles: 2 = 64x128, 3 = 32x128, 9 = 128x64.
+// that sums them in its own pass. Decode-sized tiles: 2 = 64x128, 3 = 32x128, 9 = 128x64, 15 = 128x64 streaming.
 DA_EXPORT int da_gemm_partials(const void* A, int lda, const void* W, int M, int N, int K, int tile, int splits,
                                void* ws, void* stream) {
   if (M < 1 || K % 64 || N % 8 || lda % 8 || splits < 1 || (K / 64) % splits || !ws) return (int)hipErrorInvalidValue;
@@ -966,6 +966,7 @@ DA_EXPORT int da_gemm_partials(const void* A, int lda, const void* W, int M, int
     case 2: return launch_decode_tile<64, 128>(a, EPI_PARTIAL, splits, s);
     case 3: return launch_decode_tile<32, 128>(a, EPI_PARTIAL, splits, s);
     case 9: return launch_tile<128, 64, 2, 2, 4>(a, EPI_PARTIAL, splits, s);
+    case 15: return ws_spans(a) ? launch_ws_tile<128, 64, 4, 2, false>(a, EPI_PARTIAL, splits, WsNorm{}, s) : (int)hipErrorInvalidValue;
     default: return (int)hipErrorInvalidValue;
   }
 }
