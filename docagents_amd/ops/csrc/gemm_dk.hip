@@ -54,11 +54,14 @@ template <typename T> __device__ __forceinline__ f32x4_t unpack4(const u32x2_t& 
 // ST stages of a wave's ring, each BM rows of A and BN of W; row r's 16-B chunk c at slot c ^ (r >> 1 & 7), so that the 16
 // rows of a fragment read land on all banks
 // SPLIT: K by `splits` workgroups as well. Each leaves its sums and counts; the last to come, which nobody waits for, adds them up
-// in order and has the epilogue: 2.5 us that a long K repays, whose workgroups otherwise read all of A for few columns each. The
-// sums go past the XCDs' L2s (sc1) to where all of them see them. us of 32 / 24 / 17 rows, whole -> split (tiles of 64 columns by
-// 4 or 5; of 32 by 4 below 3072): 4096 x 14336 29.6 / 27.3 / 26.6 -> 25.9 / 25.1 / 25.5, 3072 x 8192 16.2 / 14.9 / 15.3 -> 15.3 /
-// 15.1 / 14.9, 2048 x 8192 15.4 / 14.0 / 13.9 -> 11.2 / 10.9 / 11.1, 1024 x 4096 9.4 / 8.8 / 8.1 -> 7.9 / 7.8 / 7.8; not 4096 x
-// 8192 (16.8 -> 17.9), 4096 x 4096 (11.0 -> 11.0), nor 33 rows and more, whose streaming tiles share A (4096 x 14336, 64: 28.1, 31.7).
+// in order and has the epilogue: 2.5 us that a long K repays, where few columns leave CUs idle or workgroups read all of A for few
+// columns each. The sums go past the XCDs' L2s (sc1) to where all of them see them. us, whole -> split:
+//   2 / 8 / 16 / 32 rows, tiles of 16 columns by 4: 320 x 8192 8.1 / 9.1 / 10.9 / 14.2 -> 6.2 / 6.6 / 6.9 / 7.7, 128 x 4096 5.1 / 5.9 /
+//     6.7 / 8.5 -> 5.1 / 5.2 / 5.4 / 6.0, 768 x 3072 at 24 / 32 7.2 / 7.7 -> 6.3 / 6.5; of 32 by 4: 1536 x 6144 at 2 / 8 / 16 / 32
+//     7.6 / 8.6 / 9.7 / 13.0 -> 7.8 / 8.1 / 8.4 / 9.2, 2048 x 8192 10.2 / 9.8 / 11.3 / 14.8 -> 10.0 / 10.0 / 10.1 / 10.6
+//   32 / 24 / 17 rows, tiles of 64 columns by 4 or 5: 4096 x 14336 29.6 / 27.3 / 26.6 -> 25.9 / 25.1 / 25.5, 3072 x 8192 16.2 / 14.9 /
+//     15.3 -> 15.3 / 15.1 / 14.9; not 4096 x 8192 (16.8 -> 17.9), 4096 x 4096 (11.0 -> 11.0) or 512 x 2048 (5.8 -> 5.8), nor 33 rows
+//     and more, whose streaming tiles share A (4096 x 14336, 64: 28.1, 31.7).
 // ROWS: more than one block of BM rows (gridDim.y of them; W's lines are worth a place in the caches then). The blocks of a column
 // tile are neighbours on one XCD.
 template <int FM, int FN, int NW, int ST, int EPI, typename T, bool ROWS, bool SPLIT>
@@ -187,13 +190,13 @@ gemm_dk_kernel(DkArgs p) {
   constexpr int BNO = EPI == EPI_SWIGLU ? BN / 2 : BN;  // output columns of the tile
   constexpr int CPR = BNO / 4;                          // 4-column pieces of a row
   if constexpr (SPLIT) {  // (a thread's pieces here are its pieces below)
-    static_assert(EPI != EPI_SWIGLU && !ROWS && BM * CPR % (64 * NW) == 0, "split");
-    constexpr int IT = BM * CPR / (64 * NW);
+    static_assert(EPI != EPI_SWIGLU && !ROWS, "split");
+    constexpr int IT = (BM * CPR + 64 * NW - 1) / (64 * NW);  // (threads past the last piece: that one again)
     constexpr unsigned TB = IT * 64 * NW * 16;
     f32x4_t v[IT];
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-      const int t = tid + i * 64 * NW;
+      const int t = min(tid + i * 64 * NW, BM * CPR - 1);
       v[i] = *(const f32x4_t*)&red[0][t / CPR][t % CPR * 4];
 #pragma unroll
       for (int x = 1; x < NW; ++x) v[i] += *(const f32x4_t*)&red[x][t / CPR][t % CPR * 4];
@@ -228,7 +231,7 @@ gemm_dk_kernel(DkArgs p) {
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
       const int t = tid + i * 64 * NW;
-      *(f32x4_t*)&red[0][t / CPR][t % CPR * 4] = v[i];
+      if (t < BM * CPR) *(f32x4_t*)&red[0][t / CPR][t % CPR * 4] = v[i];
     }
   }
   static_assert(EPI != EPI_RESID || ROWS || (CPR & (CPR - 1)) == 0, "a row's pieces meet by lane exchange");
@@ -302,9 +305,9 @@ static int dk_launch3(const DkArgs& a, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-template <int FN>
+template <int FM, int FN>
 static int dk_split(const DkArgs& a, int epi, hipStream_t s) {
-  constexpr int FM = 2, STAGE = (FM + FN) * 2048, FIT = 81920 / (4 * STAGE), ST = FIT < 2 ? 2 : FIT > 4 ? 4 : FIT;
+  constexpr int STAGE = (FM + FN) * 2048, FIT = 81920 / (4 * STAGE), ST = FIT < 2 ? 2 : FIT > 4 ? 4 : FIT;
   const int blocks = (a.N + 16 * FN - 1) / (16 * FN) * a.splits;
   if (epi == EPI_RESID) gemm_dk_kernel<FM, FN, 4, ST, EPI_RESID, BF16T, false, true><<<blocks, 256, 0, s>>>(a);
   else if (epi == EPI_NONE || epi == EPI_BIAS) gemm_dk_kernel<FM, FN, 4, ST, EPI_NONE, BF16T, false, true><<<blocks, 256, 0, s>>>(a);
@@ -337,10 +340,10 @@ DA_EXPORT int da_gemm_dk_parts(int N) {
 // epi: EPI_NONE / EPI_BIAS / EPI_RESID / EPI_SWIGLU. ssq_in (nullable): deferred RMSNorm of A's rows
 // over ssq_parts parts (norm over norm_k columns, eps); ssq_out (nullable, EPI_RESID only):
 // [da_gemm_dk_parts(N)][64] floats. 1 <= M <= 64, K % 64 == 0, N % 16 == 0 (SwiGLU: N % 32 == 0).
-// splits > 0 (17 - 32 rows, not SwiGLU, no ssq_in): tiles of 16 fn columns (fn 2 or 4), K by as many workgroups; ws: da_gemm_dk_ws
-// bytes, cnt: a zero per tile.
+// splits > 0 (up to 32 rows, not SwiGLU, no ssq_in): tiles of 16 fn columns (fn 1, 2 or, from 17 rows on, 4), K by as many
+// workgroups; ws: da_gemm_dk_ws bytes, cnt: a zero per tile.
 DA_EXPORT size_t da_gemm_dk_ws(int N, int fn, int splits) {
-  return (size_t)((N + 16 * fn - 1) / (16 * fn)) * splits * (32 * 16 * fn * 4);
+  return (size_t)((N + 16 * fn - 1) / (16 * fn)) * splits * (fn == 4 ? 8192 : 4096);
 }
 
 DA_EXPORT int da_gemm_dk(const void* A, int lda, const void* W, void* C, int ldc, const void* bias,
@@ -355,7 +358,7 @@ DA_EXPORT int da_gemm_dk(const void* A, int lda, const void* W, void* C, int ldc
   if (ssq_in && (ssq_parts < 1 || norm_k < 1 || !(eps > 0.f))) return (int)hipErrorInvalidValue;
   const int ssq_fn = dk_fn(N, epi);
   if (splits < 0 || splits > 64 ||
-      (splits && (M <= 16 || M > 32 || ssq_in || !ws || !cnt || (fn != 2 && fn != 4) || (ssq_out && (ssq_fn > fn || N % (16 * ssq_fn))))))
+      (splits && (M > 32 || ssq_in || !ws || !cnt || (fn != 1 && fn != 2 && fn != 4) || (ssq_out && (ssq_fn > fn || N % (16 * ssq_fn))))))
     return (int)hipErrorInvalidValue;
   // a tile's rows within the resource's reach
   if (2ll * ((M - 1) * (long long)lda + K) > 0x7ffff000ll || 32ll * (splits ? fn : ssq_fn) * K > 0x7ffff000ll ||
@@ -369,7 +372,8 @@ DA_EXPORT int da_gemm_dk(const void* A, int lda, const void* W, void* C, int ldc
   a.ssq_parts = ssq_parts; a.norm_k = norm_k; a.eps = eps; a.relu = relu;
   a.ws = (float*)ws; a.cnt = (int*)cnt; a.splits = splits; a.ssq_bn = 16 * ssq_fn;
   hipStream_t s = (hipStream_t)stream;
-  if (splits) return fn == 2 ? dk_split<2>(a, epi, s) : dk_split<4>(a, epi, s);
+  if (splits && M <= 16) return fn == 1 ? dk_split<1, 1>(a, epi, s) : fn == 2 ? dk_split<1, 2>(a, epi, s) : (int)hipErrorInvalidValue;
+  if (splits) return fn == 1 ? dk_split<2, 1>(a, epi, s) : fn == 2 ? dk_split<2, 2>(a, epi, s) : dk_split<2, 4>(a, epi, s);
   if (M <= 16) return dk_launch1<1>(a, epi, s);
   if (M <= 32) return dk_launch1<2>(a, epi, s);
   if (M <= 48) return dk_launch1<3>(a, epi, s);

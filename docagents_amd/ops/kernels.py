@@ -441,13 +441,17 @@ def _dk_whole(M: int, N: int, K: int) -> bool:
     return N <= 16384 and K <= 4096
 
 
+@_rule
 def _dk_split(M: int, N: int, K: int, epi: int):
-    """(16-column groups of a tile, workgroups that share its K) of 17..32 rows on gemm_dk, (0, 0): K whole. Where K is at
-    least 2.5 N; fewer columns than 1024 leave tiles of too few steps (measured: csrc/gemm_dk.hip)."""
-    if not (16 < M <= 32 and 1024 <= N <= 8192 and N % 64 == 0 and 2 * K >= 5 * N and epi in (EPI_NONE, EPI_BIAS, EPI_RESID)):
+    """(16-column groups of a tile, workgroups that share its K) of 2..32 rows on gemm_dk, (0, 0): K whole (both measured:
+    csrc/gemm_dk.hip). From 17 rows on where K is at least 2.5 N and 3072; of fewer rows, whose workgroups read little of A, where K
+    is at least 4 N (up to 8 rows 16 N) and 4096."""
+    if epi not in (EPI_NONE, EPI_BIAS, EPI_RESID) or N % 64 or not 1 < M <= 32:
         return 0, 0
-    fn = 4 if N >= 3072 else 2
-    return fn, min(256 // (N // (16 * fn)), 6)
+    if not (2 * K >= 5 * N and K >= 3072 and N <= 8192 if M > 16 else K >= (4 if M > 8 else 16) * N and K >= 4096 and N <= 2048):
+        return 0, 0
+    fn = 1 if N < 1024 else 2 if N < 3072 else 4
+    return fn, min(256 // (N // (16 * fn)), 6 if fn == 4 else 4)
 
 
 def _dk_splitk(M: int, N: int) -> bool:

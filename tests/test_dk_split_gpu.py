@@ -1,4 +1,4 @@
-"""Decode products of 17 to 32 rows and a long K, shared by workgroups of which the last to come adds up."""
+"""Decode products of a long K, shared by workgroups of which the last to come adds up."""
 import pytest
 import torch
 
@@ -7,9 +7,13 @@ pytestmark = pytest.mark.gpu
 from docagents_amd.ops import kernels as K  # noqa: E402
 
 
-# tiles of 32 and 64 columns; the fewest and most workgroups a tile; K-steps that they share unevenly, and the first N below and above the line
-@pytest.mark.parametrize("N,Kd", [(1024, 2560), (2048, 8192), (3008, 7680), (3072, 8192), (4096, 14336), (4160, 10496), (8192, 20480)])
-@pytest.mark.parametrize("M", [17, 25, 32])
+# tiles of 16, 32 and 64 columns; the fewest and most workgroups a tile; K-steps that they share unevenly, the first N below and above a line
+MANY = [(64, 3072), (960, 3328), (1024, 3072), (2048, 8192), (3008, 7680), (3072, 8192), (4096, 14336), (4160, 10496), (8192, 20480)]
+FEW = [(64, 4096), (320, 8192), (256, 4352), (960, 16384)]
+
+
+@pytest.mark.parametrize("M,N,Kd", [(m, *s) for m in (17, 25, 32) for s in MANY] + [(m, *s) for m in (2, 8) for s in FEW]
+                         + [(m, *s) for m in (9, 16) for s in [*FEW, (1024, 4096), (2048, 8192)]])
 def test_split_products(M, N, Kd):
     assert K._dk_split(M, N, Kd, K.EPI_RESID)[1] >= 2
     g = torch.Generator(device="cuda").manual_seed(M + N)
