@@ -984,8 +984,9 @@ DA_EXPORT int da_gemm_rope(const void* A, int lda, const void* W, void* C, int l
   a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc; a.k_per_split = K;
   a.rope = RopeArgs{(const int*)pos, (const int*)slot, (const float*)cos_sin, (bf16_t*)k_cache, (bf16_t*)v_cache,
                     H, Hkv, D, max_seq, kv_out ? 1 : 0};
-  const long t256 = (long)((M + 255) / 256) * ((N + 255) / 256);
-  return launch_gemm8p(a, EPI_ROPE, (hipStream_t)stream, t256 >= 256 ? 256 : 128);
+  // the row-tile height of fewer rounds: a single round of 256-row tiles on more than half of the chip beats two of 128-row ones (us,
+  // 256 rows only from 256 tiles on -> this: 1400 x 9216 x 3072 96 -> 69, 1792 96 -> 76, 1400 x 6144 x 4096 104 -> 75, 2048 116 -> 81)
+  return launch_gemm8p(a, EPI_ROPE, (hipStream_t)stream, gemm8p_pick_bm(M, N, K, EPI_ROPE));
 }
 
 // Tile selection: big tiles when the grid fills 256 CUs, skinny tiles (+ split-K) for decode-sized M.

@@ -584,7 +584,7 @@ def gemm_rope(a, w, pos, cos_sin, H: int, Hkv: int, D: int, slot, k_cache, v_cac
               kv_out: bool = True) -> torch.Tensor:
     """Prefill QKV projection: qkv = a @ w^T with RoPE applied to the q / k heads and the token's
     k / v written to the KV cache (cache [slots, Hkv, max_seq, D]) — one kernel (gemm8p EPI_ROPE)
-    from 256 rows on, but where ``_rope_apart``; those and shorter prefills run gemm + rope_cache (identical roundings). kv_out=False: the
+    from 256 rows on, but where ``_rope_apart`` (and not ``_rope_round``); those and shorter prefills run gemm + rope_cache (identical roundings). kv_out=False: the
     k / v columns of the result may be left unwritten (the attention reads the cache; see
     flash_attn_varlen kv_cache) — only the q columns are defined."""
     _bf16_cuda(a, "a"); _bf16_cuda(w, "w"); _i32(pos, "pos"); _i32(slot, "slot")
@@ -598,7 +598,7 @@ def gemm_rope(a, w, pos, cos_sin, H: int, Hkv: int, D: int, slot, k_cache, v_cac
     plain = K % 64 == 0 and K >= 128 and a.stride(1) == 1 and a.stride(0) % 8 == 0 and w.is_contiguous()
     # (what gemm and rope_cache refuse and the one kernel takes stays with that)
     apart = (a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and a.stride(0) >= K and cos_sin.shape[-1] == 2
-             and (out is None or out.is_contiguous()) and M >= 256 and _rope_apart(M, N, K))
+             and (out is None or out.is_contiguous()) and M >= 256 and _rope_apart(M, N, K) and not _rope_round(M, N))
     if M < 256 or not plain or apart:
         qkv = gemm(a, w, out=out)
         return rope_cache(qkv, pos, cos_sin, H, Hkv, D, slot=slot, k_cache=k_cache, v_cache=v_cache)
@@ -922,10 +922,21 @@ def _rope_apart(M: int, N: int, K: int) -> bool:
     """A QKV projection of 256 rows and more as a product by itself, on the tile that it has then, and rope_cache behind it (which
     reads and writes the result once more; the rotation costs the phase-split kernel 4 us): 432 x 6144 x 4096 54 -> 39 us, 300 x 9216
     x 3072 46 -> 34, 800 x 6144 x 4096 54 -> 50, where 128x256 tiles leave CUs idle, and 1024 x 9216 x 3072 95 -> 69, 1200 x 10240 x
-    8192 212 -> 173, where the one kernel has two rounds of 128-row tiles and the product alone one of 256-row ones."""
+    8192 212 -> 173, where the one kernel had two rounds of 128-row tiles and the product alone one of 256-row ones. From
+    ROW_TILES_BELOW rows on where the one kernel's last round is short, which the product alone shares out: 2817 x 6144 x 4096
+    158 -> 140, 3600 168 -> 160, 5400 250 -> 237, 1931 x 9216 x 3072 131 -> 127; not 2300 (128 / 131), 3600 (194 / 199) or
+    4100 x 6144 x 4096 (176 / 184). (The estimates are 5 us and 8 % off either way there.)"""
     tiles = math.ceil(M / 256) * math.ceil(N / 256)
-    return M < ROW_TILES_BELOW and (_row_us(M, N, K)[0] + 4 + M * N * 1e-6
-                                    < 0.97 * (_phase_us(M, N, K, EPI_ROPE, 7 if tiles >= 256 else 10) + 4))
+    if M >= ROW_TILES_BELOW:
+        alone = min(_phase_us(M, N, K, EPI_NONE, t) for t in _PHASE_TILES)
+        return tiles > 256 and alone + M * N * 1e-6 - 1 < 1.05 * (_phase_us(M, N, K, EPI_ROPE, 7) + 4)
+    return _row_us(M, N, K)[0] + 4 + M * N * 1e-6 < 0.97 * (_phase_us(M, N, K, EPI_ROPE, 7 if tiles >= 256 else 10) + 4)
+
+
+def _rope_round(M: int, N: int) -> bool:
+    """The one kernel has a single round of 256-row tiles, of more than half of the chip: us, product and rope_cache / one kernel:
+    900 x 9216 x 3072 65 / 62, 1024 69 / 65, 1200 70 / 64. (Of fewer tiles 900 x 6144 x 4096 53 / 57.)"""
+    return 128 < math.ceil(M / 256) * math.ceil(N / 256) <= 256
 
 
 # ------------------------------------------------------------------------------ norms etc.
