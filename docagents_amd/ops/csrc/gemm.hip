@@ -231,7 +231,7 @@ gemm_bf16_kernel(GemmArgs p) {
 
 // ------------------------------------------------------------------------------------------
 // Weight-streaming product (2 rows to some 1000: decoding, short prompts, short texts; bf16, and fp16 for the encoders).
-// K in stages of 64; tiles of 32 x 64, 32 x 128, 64 x 128, 64 x 64, 128 x 64, 128 x 128 and 192 x 128, four or eight waves.
+// K in stages of 64; tiles of 32 x 128, 64 x 128, 64 x 64, 128 x 64, 128 x 128 and 192 x 128, four or eight waves.
 //  * A stage (8 - 24 KB of A, 8 or 16 KB of W) arrives by LDS-DMA in a ring that fills LDS. What a CU can have on its way
 //    beyond the L2 is 32 KB whatever is asked for (57 GB/s from HBM or the last-level cache, 142 GB/s from L2; loads into
 //    registers the same), and A's pieces wait in that queue behind W's, so the tile's bytes per product bound it, not the
@@ -753,12 +753,10 @@ static int launch_ws_tile(const GemmArgs& a, int epi, int splits, const WsNorm& 
 // way, and the wider tile then moves less of A: 64 x 8192 x 4096 22.8 us at four splits vs 24.0 at two of 64 x 64. Splits are
 // short, and eight waves fill and drain faster: with the reduce, 64 x 4096 x 4096 14.4 us vs 15.8 with four (8 splits), x 14336
 // 28.5 / 30.2, 64 x 6144 x 4096 18.2 / 18.9 (4); unsplit 64 x 28672 x 4096 42.9 / 40.3.
-// Up to 32 rows only wide ones come here (kernels.py, dk_wide).
+// Up to 32 rows only those of more than 16384 columns come here (kernels.py, _dk_streams).
 // W is read once where there is one row block only: not worth a place in the caches then.
 static int launch_ws(const GemmArgs& a, int epi, int splits, const WsNorm& nrm, hipStream_t s) {
-  if (a.M <= 32 && splits == 1)
-    return a.N <= 16384 ? launch_ws_tile<32, 64, 2, 2, true>(a, epi, splits, nrm, s)
-                        : launch_ws_tile<32, 128, 1, 4, true>(a, epi, splits, nrm, s);
+  if (a.M <= 32 && splits == 1 && a.N > 16384) return launch_ws_tile<32, 128, 1, 4, true>(a, epi, splits, nrm, s);
   if (a.M <= 64) {
     if (splits > 1) return launch_ws_tile<64, 128, 2, 4, true>(a, epi, splits, nrm, s);
     return a.N <= 16384 ? launch_ws_tile<64, 64, 2, 2, true>(a, epi, splits, nrm, s)

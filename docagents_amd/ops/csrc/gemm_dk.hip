@@ -1,4 +1,4 @@
-// Decode GEMM for 1 <= M <= 64 rows in one launch, without split-K partials (gemm_dk).
+// Decode GEMM for 1 <= M <= 64 rows in one launch (gemm_dk), and products of more rows in blocks of 32 or 64 (da_gemm_dk_rows).
 //
 //   C[M, N'] = epi( rownorm(A)[M, K] . W[N, K]^T )
 //

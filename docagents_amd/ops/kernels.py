@@ -317,6 +317,7 @@ def _call_partials(splits: int, M: int, N: int, like):
     return _call_scratch(splits * M * N * 4, like) if splits > 1 else None
 
 
+@_rule
 def _row_choice(M: int, N: int, K: int, epi: int, lda: int, f16: bool = False):
     """(tile, splits) of a product of more than 64 rows (fp16: of any). A tile of ``_DK_TILES`` is da_gemm_dk_rows'."""
     if max(K, lda) < 1 << 22:
@@ -404,20 +405,20 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias=None, epi: int = EPI_NONE, resid
     return out
 
 
-# Decode GEMMs with 2..64 rows: gemm_dk (csrc/gemm_dk.hip: K split across the 4 waves of a
-# workgroup and summed through LDS, no split-K partials, no reduce launch). False: the 64x128 /
+# Decode GEMMs with 2..64 rows: gemm_dk (csrc/gemm_dk.hip: K-steps dealt out to the 4 waves of a
+# workgroup and summed through LDS; one launch, also where workgroups share K). False: the 64x128 /
 # 32x128 tiles + split-K + reduce (bench/ab_arms.py DA_DECODE_DK=0).
 DECODE_DK = True
-# 33..64 rows keep the gemm_dk layer structure (norms deferred into the consumer) on the streaming
-# tiles: the narrow dk tiles re-read the activation block once per 16-64 weight rows there
-# (bench/midm_chain.py, profiles/r3/dk/), so gemm_dk() routes those rows to da_gemm_dk_splitk
-# (reduce + residual + row sums of squares; the consumer's reduce or epilogue applies the row scale)
+# 33..64 rows keep the gemm_dk layer structure (norms deferred into the consumer); what ``_dk_whole`` does
+# not take, and residuals with row sums, run on the streaming tiles (da_gemm_dk_splitk: reduce + residual
+# + row sums of squares; the consumer's reduce or epilogue applies the row scale): a dk tile reads the
+# activations once per 16-64 weight rows
 DK_MAX_M = 64
 DK_SPLITK_ABOVE = 32
 
 
 def dk_fusable(M: int, N: int, K: int, epi: int = EPI_NONE) -> bool:
-    """True when gemm() runs a decode-sized product on gemm_dk (no split-K)."""
+    """True when gemm() runs a decode-sized product on gemm_dk."""
     return (DECODE_DK and 2 <= M <= DK_MAX_M and K % 256 == 0 and N % 16 == 0
             and epi in (EPI_NONE, EPI_BIAS, EPI_RESID, *GATED) and (epi not in GATED or N % 32 == 0))
 
@@ -443,15 +444,16 @@ def _dk_whole(M: int, N: int, K: int) -> bool:
 
 @_rule
 def _dk_split(M: int, N: int, K: int, epi: int):
-    """(16-column groups of a tile, workgroups that share its K) of 2..32 rows on gemm_dk, (0, 0): K whole (both measured:
-    csrc/gemm_dk.hip). From 17 rows on where K is at least 2.5 N and 3072; of fewer rows, whose workgroups read little of A, where K
-    is at least 4 N (up to 8 rows 16 N) and 4096."""
+    """(16-column groups of a tile, workgroups that share its K, bytes of their sums) of 2..32 rows on gemm_dk, zeros: K whole
+    (both measured: csrc/gemm_dk.hip). From 17 rows on where K is at least 2.5 N and 3072; of fewer rows, whose workgroups read
+    little of A, where K is at least 4 N (up to 8 rows 16 N) and 4096."""
     if epi not in (EPI_NONE, EPI_BIAS, EPI_RESID) or N % 64 or not 1 < M <= 32:
-        return 0, 0
+        return 0, 0, 0
     if not (2 * K >= 5 * N and K >= 3072 and N <= 8192 if M > 16 else K >= (4 if M > 8 else 16) * N and K >= 4096 and N <= 2048):
-        return 0, 0
+        return 0, 0, 0
     fn = 1 if N < 1024 else 2 if N < 3072 else 4
-    return fn, min(256 // (N // (16 * fn)), 6 if fn == 4 else 4)
+    splits = min(256 // (N // (16 * fn)), 6 if fn == 4 else 4)
+    return fn, splits, int(lib().da_gemm_dk_ws(N, fn, splits))
 
 
 def _dk_splitk(M: int, N: int) -> bool:
@@ -488,10 +490,9 @@ def dk_parts(N: int, M: int = 0) -> int:
 
 
 def gemm_dk(a, w, epi: int = EPI_NONE, bias=None, resid=None, out=None, norm_in=None, ssq_out=None):
-    """Decode-sized product (1 <= M <= 64) in one launch without split-K:
+    """Decode-sized product (1 <= M <= 64), in one launch but for what streams in splits:
     out = epi(rownorm(a) @ w^T). norm_in = (ssq, parts, eps): ``a`` is the raw residual stream and
-    each row is scaled by rsqrt(sum of ssq[:parts, row] / K + eps) first (bf16-rounded, as the
-    rmsnorm kernel would; RMSNorm gains folded into w). ssq_out (EPI_RESID only): fp32
+    each row's sums are scaled by rsqrt(sum of ssq[:parts, row] / K + eps) (RMSNorm gains folded into w). ssq_out (EPI_RESID only): fp32
     [dk_parts(N), 64] receives the per-part sums of squares of the new rows, for the next consumer."""
     _bf16_cuda(a, "a"); _bf16_cuda(w, "w")
     M, K = a.shape
@@ -527,9 +528,9 @@ def gemm_dk(a, w, epi: int = EPI_NONE, bias=None, resid=None, out=None, norm_in=
                                        splits, _stream()), "gemm_dk_splitk")
         return out
     stream, ws, cnt = _raw_stream(), None, None
-    fn, splits = _dk_split(M, N, K, epi) if ssq is None else (0, 0)
+    fn, splits, nbytes = _dk_split(M, N, K, epi) if ssq is None else (0, 0, 0)
     if splits:
-        ws, cnt = _call_scratch(int(lib().da_gemm_dk_ws(N, fn, splits)), a), _counters(a.device, stream)
+        ws, cnt = _call_scratch(nbytes, a), _counters(a.device, stream)
     _check(lib().da_gemm_dk(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
                             M, N, K, epi, _ptr(ssq), parts, K, float(eps), _ptr(ssq_out), fn, splits, _ptr(ws), _ptr(cnt),
                             c_void_p(stream)), "gemm_dk")
@@ -893,7 +894,7 @@ def _dk_rows_tile(M: int, N: int, K: int, epi: int = EPI_NONE, f16: bool = False
     estimate is 3 % below theirs, 10 % from 257 rows on, 15 % where K is above 4096 (768 x 320 x 8192 is not: 15.9 / 19.0 us): 155 of
     the 338 products that it is fitted to, in 0.76 of their time, four of them in 1.02 - 1.03. us, tiles of ``_row_tile`` -> these: 128 x 384 x 1536 8.9 ->
     4.3, 256 x 768 x 768 6.6 -> 4.3, 256 x 768 x 3072 12.2 -> 7.6, 256 x 1024 x 4096 13.8 -> 8.8, 128 x 4096 x 1024 8.1 -> 6.3,
-    640 x 1024 x 1024 8.2 -> 6.9; 96 x 3072 x 3072 13.0 -> 9.6, 128 x 4096 x 4096 19.8 -> 15.8, 128 x 9216 x 3072 27.4 -> 23.9."""
+    640 x 1024 x 1024 8.2 -> 6.9; 96 x 3072 x 3072 13.0 -> 9.6, 128 x 4096 x 4096 19.8 -> 15.8."""
     if not 64 < M < ROW_TILES_BELOW:
         return 0
     best, ksteps = None, K // 64
@@ -1552,7 +1553,7 @@ def spin(us: int, device=None) -> None:
 def gemm8p_persist(on: int = -1) -> int:
     """Persistent tile loop of the prefill GEMM (one workgroup per CU walking its XCD's tiles) on
     (1) / off (0) for later launches; -1 only queries. Returns the previous setting."""
-    for rule in (_tail_bytes, _row_us, _dk_rows_tile, _rope_apart):  # (the rules that ask which rounds are shared)
+    for rule in (_tail_bytes, _row_us, _dk_rows_tile, _row_choice, _rope_apart):  # (the rules that ask which rounds are shared)
         rule.cache_clear()
     return int(lib().da_gemm8p_persist(int(on)))
 
