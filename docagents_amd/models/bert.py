@@ -158,16 +158,18 @@ class BertEncoder:
         return c.ffn > 2048 and all(o.gemv_fusable(rows, c.hidden, k) for k in (c.hidden, c.ffn))
 
     def _layers_few_rows(self, x, cu_seqlens, max_seqlen, attn, layernorm):
-        """The layers of a short text: the LayerNorms ride in the products around them, and between layers the residual
-        is the sum y that the next norm reads, with its row statistics (only the last norm is a launch)."""
+        """The layers of a short text: the LayerNorms (and one text's attention) ride in the products around them, and between
+        layers the residual is the sum y that the next norm reads, with its row statistics (only the last norm is a launch)."""
         c, o = self.cfg, self.ops
         h, nh, hd = c.hidden, c.heads, c.head_dim
         st1, st2 = torch.empty((2, 64, 64, 2), dtype=torch.float32, device=x.device)
         norm = None
+        inside = o.attn_ln_fit(x.shape[0], h, nh, cu_seqlens.numel() - 1, self.fp16)
         for L in self.w["layers"]:
-            qkv = o.gemm_ln(x, L["wqkv"], L["bqkv"], norm=norm)
-            a = attn(qkv[:, :h], qkv[:, h:2 * h], qkv[:, 2 * h:], cu_seqlens, max_seqlen, nh, nh, hd, causal=False)
-            y = o.gemm_ln(a, L["wo"], L["bo"], EPI_RESID, norm=norm, resid=x, st_out=st1)
+            a = qkv = o.gemm_ln(x, L["wqkv"], L["bqkv"], norm=norm)
+            if not inside:
+                a = attn(qkv[:, :h], qkv[:, h:2 * h], qkv[:, 2 * h:], cu_seqlens, max_seqlen, nh, nh, hd, causal=False)
+            y = o.gemm_ln(a, L["wo"], L["bo"], EPI_RESID, norm=norm, resid=x, st_out=st1, attn=(nh, cu_seqlens) if inside else None)
             norm = (st1, L["ln1_g"], L["ln1_b"], c.eps)
             f = o.gemm_ln(y, L["w1"], L["b1"], EPI_GELU, norm=norm)
             x = o.gemm_ln(f, L["w2"], L["b2"], EPI_RESID, norm=norm, resid=y, st_out=st2)

@@ -1,4 +1,5 @@
-// Encoder products for few rows (a question: <= 64 tokens), with the LayerNorms between them inside: five launches a layer.
+// Encoder products for few rows (a question: <= 64 tokens), with the LayerNorms between them inside: five launches a layer,
+// four where attention is inside the product behind it.
 //
 //   C[M, N] = epi(LN(A)[M, K] . W[N, K]^T + bias)      epi: none / GELU
 //   C[M, N] = A . W^T + bias + LN(R)                   and the row statistics that the next LN needs
@@ -30,28 +31,48 @@ struct EncRowsArgs {
   float* st_out;          // RESID: the same of the rows of C, a part per 16 columns
   int M, N, K, lda, ldc, ldr, parts;
   float eps;
+  const int* cu;  // attention: the text's first row and its end
+  float c;        // and log2(e) times the scale of the scores
 };
 
 // The waves' stages (ST of each) and, after the last unit, their sums share LDS: up to enc_waves(FM) waves.
 constexpr int enc_waves(int fm) { return fm == 4 ? 12 : 16; }
 constexpr int enc_stages(int fm) { return fm == 1 ? 2 : 1; }
+constexpr int ENC_ATTN_UNITS = 12;  // of 12 KB of LDS
 
-template <typename T, int FM, bool LNA, int EPI>
+// Attention inside the product that takes its output (D != 0: heads of D; A is then q, k and v beside one another, one text of
+// KR rows at most): a unit of 64 k is a head of 64 or two of 32, so its wave attends for the block's 16 rows and the result is
+// its MFMA operand as it stands. S^T = K Q^T leaves a lane keys 16 t + 4 fg + e of its row, which is P's operand if V's rows
+// come in that order, and V's columns are read so that a lane of O^T has 8 in a row. Scores and weights as in the attention
+// kernels: the maximum and the sums in fp32, weights rounded to the type (bf16: of 2^-8 times them, so that sums of the largest
+// values stay in fp32). Rows outside the text read as zero.
+// All strips do the same attention over again. What it costs is its operands (10 KB a wave at 32 rows, which other dies have just
+// written), so they come by LDS-DMA, and only the text's: straight to the MFMA the question took as long as with a launch
+// between, 64 rows 10 % longer. Texts that share blocks had to take turns with V (a NaN of one reaches another through weights
+// of zero), 6 us a layer for seven: one text only. One of 21 tokens through 12 layers of 768: 333
+// -> 302 us, of 20 through 384 (heads of 32) 278 -> 246. More than 12 waves of 12 KB don't fit a CU's LDS.
+template <typename T, int FM, bool LNA, int EPI, int D = 0, int KR = 0>
 __global__ void __launch_bounds__(64 * enc_waves(FM))
 enc_rows_kernel(EncRowsArgs p) {
   constexpr int ROWS = FM * 16, SLD = 20, ST = enc_stages(FM), A_BYTES = ROWS * 128, STAGE = A_BYTES + 2048;
   constexpr int PA = 2 * FM, P = PA + 2;  // LDS-DMA instructions of a stage
-  static_assert(ROWS * SLD * 4 <= ST * STAGE, "the sums fit the stages");
-  __shared__ __attribute__((aligned(16))) char smem[enc_waves(FM) * ST * STAGE];
+  constexpr int RING = D ? KR * 256 + 4096 : ST * STAGE;  // a wave's stages, or its W, Q, K and V
+  static_assert(ROWS * SLD * 4 <= RING, "the sums fit the stages");
+  static_assert(!D || (FM == 1 && !LNA), "attention: 16 rows a block");
+  __shared__ __attribute__((aligned(16))) char smem[(D ? ENC_ATTN_UNITS : enc_waves(FM)) * RING];
   __shared__ float smean[ROWS], srstd[ROWS];
   float (*red)[ROWS][SLD] = (float (*)[ROWS][SLD])smem;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
   const int fr = lane & 15, fg = lane >> 4;
-  const int n0 = blockIdx.x * 16, units = p.K / 64;
+  const int n0 = blockIdx.x * 16, units = p.K / 64, rows = p.M, m0 = blockIdx.y * ROWS;
+  int first = 0, end = 0;  // the text (attention)
+  if constexpr (D != 0) {
+    first = p.cu[0];
+    end = min(p.cu[1], rows);
+  }
   {  // this block's rows
-    const int m0 = blockIdx.y * ROWS;
     p.M -= m0;
-    p.A += (size_t)m0 * p.lda;
+    if (!D) p.A += (size_t)m0 * p.lda;
     p.C += (size_t)m0 * p.ldc;
     if (p.resid) p.resid += (size_t)m0 * p.ldr;
     if (p.st) p.st += m0 * 128;
@@ -99,6 +120,38 @@ enc_rows_kernel(EncRowsArgs p) {
     }
   }
   asm volatile("" ::: "memory");
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, (short)0, 0x7fffff00, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)(p.W + (size_t)n0 * p.K), (short)0, 0x7fffff00, 0x00020000);
+  char* ring = smem + w * RING;
+  constexpr int NT = D ? KR / 16 : 1;
+  if constexpr (D != 0) {  // unit w: 2 KB each of W and Q, then K and V; rows past the last text read as zero
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int r = 8 * j + (lane >> 3);
+      const unsigned at = (unsigned)r * (unsigned)(p.K * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t)(ring + j * 1024), 16, at, w * 128, 0, 0);
+    }
+    auto row = [&](int r, int at) __attribute__((always_inline)) { return r >= first && r < end ? (unsigned)r * (unsigned)(p.lda * 2) + at : 0x7ffffff0u; };
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int r = 8 * j + (lane >> 3);
+      const unsigned at = row(m0 + r, ((lane & 7) ^ ((r >> 1) & 7)) << 4);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(ring + 2048 + j * 1024), 16, at, w * 128, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < KR / 8; ++j) {
+      const int r = 8 * j + (lane >> 3);
+      const unsigned at = row(r, ((lane & 7) ^ ((r >> 1) & 7)) << 4);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(ring + 4096 + j * 1024), 16, at, p.K * 2 + w * 128, 0, 0);
+    }
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < KR / 8; ++j) {  // (last, for the wait: V's chunk c of row r at slot c ^ ((r & 2) << 1))
+      const int r = 8 * j + (lane >> 3);
+      const unsigned at = row(r, ((lane & 7) ^ ((r & 2) << 1)) << 4);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(ring + 4096 + KR * 128 + j * 1024), 16, at, p.K * 4 + w * 128, 0, 0);
+    }
+  }
   // ---- the wave's units w, w + nw, ..: row r's 16-B chunk c of 64 k at slot c ^ (r >> 1 & 7) of its 128 B ----
   unsigned ao[8], wo[2];  // rows past M: past the resource's end, which reads as zero
 #pragma unroll
@@ -111,9 +164,6 @@ enc_rows_kernel(EncRowsArgs p) {
     const int r = 8 * j + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
     wo[j] = (unsigned)r * (unsigned)(p.K * 2) + c * 16;
   }
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, (short)0, 0x7fffff00, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)(p.W + (size_t)n0 * p.K), (short)0, 0x7fffff00, 0x00020000);
-  char* ring = smem + w * ST * STAGE;
   auto ask = [&](int u, int slot) __attribute__((always_inline)) {
     char* base = ring + slot * STAGE;
 #pragma unroll
@@ -134,7 +184,7 @@ enc_rows_kernel(EncRowsArgs p) {
   if constexpr (LNA) norm_load(min(w, units - 1));
 #pragma unroll
   for (int i = 0; i < ST; ++i)
-    if (w + i * nw < units) ask(w + i * nw, i);
+    if (!D && w + i * nw < units) ask(w + i * nw, i);
   if (p.st) {
     asm volatile("" ::: "memory");
     stats_merge(4 * w + fg);
@@ -149,10 +199,78 @@ enc_rows_kernel(EncRowsArgs p) {
   f32x4_t acc[FM];
 #pragma unroll
   for (int i = 0; i < FM; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if constexpr (D != 0) {
+    constexpr int NH = 64 / D;
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(KR / 8) : "memory");  // everything but V
+    __builtin_amdgcn_sched_barrier(0);
+    const int at[2] = {fr * 128 + ((fg ^ ((fr >> 1) & 7)) << 4), fr * 128 + (((4 + fg) ^ ((fr >> 1) & 7)) << 4)};
+    bf16x8_t aw[2], aq[2], ak[4][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      aw[h] = *(const bf16x8_t*)(ring + at[h]);
+      aq[h] = *(const bf16x8_t*)(ring + 2048 + at[h]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) ak[t][h] = *(const bf16x8_t*)(ring + 4096 + t * 2048 + at[h]);
+    }
+    f32x4_t s[2][4];
+    bf16x8_t pf[2][2];
+    float inv[2];
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        s[h][t] = T::mma16(ak[t][h], aq[h], f32x4_t{0.f, 0.f, 0.f, 0.f});
+        if (NH == 1) s[h][t] = T::mma16(ak[t][1], aq[1], s[h][t]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int key = 16 * t + 4 * fg + e;
+          if (key < first || key >= end) s[h][t][e] = -INFINITY;
+          mx = fmaxf(mx, s[h][t][e]);
+        }
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float mc = mx == -INFINITY ? 0.f : fmaf(-mx, p.c, T::kF16 ? 0.f : -8.f);
+      float sum = 0.f;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum += s[h][t][e] = __builtin_amdgcn_exp2f(fmaf(s[h][t][e], p.c, mc));
+      sum += __shfl_xor(sum, 16, 64);
+      sum += __shfl_xor(sum, 32, 64);
+      inv[h] = sum > 0.f ? 1.f / sum : 0.f;
+#pragma unroll
+      for (int t = 0; t < NT; t += 2)
+        pf[h][t / 2] = __builtin_bit_cast(bf16x8_t, u32x4_t{T::pack2(s[h][t][0], s[h][t][1]), T::pack2(s[h][t][2], s[h][t][3]),
+                                                            T::pack2(s[h][t + 1][0], s[h][t + 1][1]), T::pack2(s[h][t + 1][2], s[h][t + 1][3])});
+    }
+    f32x4_t o[4];  // d = 32 (i / 2) + 8 fg + 4 (i & 1) + e of row fr
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // V
+    __builtin_amdgcn_sched_barrier(0);
+    const char* v = ring + 4096 + KR * 128 + (4 * fg + (fr >> 2)) * 128;
+#pragma unroll
+    for (int t = 0; t < NT; t += 2)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int at = ((4 * (i >> 1) + (fr & 3)) ^ ((fr >> 3) << 2)) * 16 + 8 * (i & 1);
+        const s16x4_t lo = lds_read_tr16(v + t * 2048 + at), up = lds_read_tr16(v + (t + 1) * 2048 + at);
+        o[i] = T::mma16(bf16x8_t{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]}, pf[NH == 1 ? 0 : i >> 1][t / 2], o[i]);
+      }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float n = inv[NH == 1 ? 0 : h];
+      const f32x4_t a = o[2 * h], b = o[2 * h + 1];
+      const u32x4_t x{T::pack2(a[0] * n, a[1] * n), T::pack2(a[2] * n, a[3] * n), T::pack2(b[0] * n, b[1] * n), T::pack2(b[2] * n, b[3] * n)};
+      acc[0] = T::mma16(aw[h], __builtin_bit_cast(bf16x8_t, x), acc[0]);
+    }
+  }
   const int sw = (fr >> 1) & 7;
   const int co[2] = {(fg ^ sw) << 4, ((4 + fg) ^ sw) << 4};
 #pragma unroll 1
-  for (int u = w, slot = 0; u < units; u += nw) {
+  for (int u = D ? units : w, slot = 0; u < units; u += nw) {
     if (LNA && u != w) norm_load(u);
     // this unit is in: everything but the stage behind it (with a norm: everything)
     if (!LNA && ST > 1 && u + nw < units) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(P * (ST - 1)) : "memory");
@@ -254,6 +372,12 @@ static int enc_rows_rows(const EncRowsArgs& a, int epi, hipStream_t s) {
   return a.M <= 32 || strips * ((blocks + 1) / 2) <= 256 ? enc_rows_launch<T, 2>(a, epi, s) : enc_rows_launch<T, 4>(a, epi, s);
 }
 
+template <typename T, int D>
+static int enc_attn_rows(const EncRowsArgs& a, hipStream_t s) {
+  enc_rows_kernel<T, 1, false, EPI_RESID, D, 32><<<dim3(a.N / 16, (a.M + 15) / 16), a.K, 0, s>>>(a);  // (a wave a unit)
+  return (int)hipGetLastError();
+}
+
 // epi BIAS / GELU (st: the norm of A's rows, over K columns; GELU only with it) / RESID (st: the norm of resid's rows,
 // over N columns; st_out is written). 1 <= M <= 64, K % 64 == 0, N % 16 == 0, a normed width of at most 1024; bf16 or fp16 throughout.
 DA_EXPORT int da_enc_rows(const void* A, int lda, const void* W, void* C, int ldc, const void* bias, const void* resid,
@@ -268,4 +392,19 @@ DA_EXPORT int da_enc_rows(const void* A, int lda, const void* W, void* C, int ld
                 (const bf16_t*)g, (const bf16_t*)b, st_out, M, N, K, lda, ldc, ldr, width / 16, eps};
   hipStream_t s = (hipStream_t)stream;
   return f16 ? enc_rows_rows<F16T>(a, epi, s) : enc_rows_rows<BF16T>(a, epi, s);
+}
+
+// RESID with A the attention of K / D heads of D (64, and 32 in bf16) over the one text of rows cu[0] .. cu[1] - 1: qkv holds q, k and v, K
+// columns each. M <= 32, K <= 768; the rest as above.
+DA_EXPORT int da_enc_attn_rows(const void* qkv, int lda, const void* W, void* C, int ldc, const void* bias, const void* resid, int ldr,
+                              int M, int N, int K, int D, const int* cu, float c, const float* st, const void* g,
+                              const void* b, float eps, float* st_out, int f16, void* stream) {
+  if (M < 1 || M > 32 || K < 64 || K % 64 || K > 64 * ENC_ATTN_UNITS || N < 16 || N % 16 || N > 1024 || lda % 8 || lda < 3 * K || ldc % 4 || ldr % 4 ||
+      lda > (1 << 22) || (D != 64 && (D != 32 || f16)) || !cu || !resid || !st_out || (st && (!g || !b)))
+    return (int)hipErrorInvalidValue;
+  EncRowsArgs a{(const bf16_t*)qkv, (const bf16_t*)W, (const bf16_t*)bias, (const bf16_t*)resid, (bf16_t*)C, st,
+                (const bf16_t*)g, (const bf16_t*)b, st_out, M, N, K, lda, ldc, ldr, N / 16, eps, cu, c};
+  hipStream_t s = (hipStream_t)stream;
+  if (D == 32) return enc_attn_rows<BF16T, 32>(a, s);
+  return f16 ? enc_attn_rows<F16T, 64>(a, s) : enc_attn_rows<BF16T, 64>(a, s);
 }

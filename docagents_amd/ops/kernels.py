@@ -69,6 +69,8 @@ _SIGS = {
     "da_gemm_dk_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 7 + [c_void_p],
     "da_enc_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5
                   + [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_void_p],
+    "da_enc_attn_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5 + [c_void_p, c_float]
+                       + [c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_void_p],
     "da_encoder_layer": [c_void_p, c_int, c_int, c_int, c_void_p],
     "da_gemm_tail_ws": [c_int] * 5,
     "da_gemm_fp8_tile": [c_int] * 2,
@@ -542,14 +544,25 @@ def gemm_ln_fit(M: int, hidden: int, ffn: int) -> bool:
     return 1 <= M <= 64 and hidden % 64 == 0 and ffn % 64 == 0 and hidden <= 1024
 
 
-def gemm_ln(a, w, bias, epi: int = EPI_BIAS, norm=None, resid=None, st_out=None):
+def attn_ln_fit(M: int, hidden: int, heads: int, texts: int, f16: bool = False) -> bool:
+    """Whether ``gemm_ln`` takes attention inside (``attn``) where an encoder's products take it."""
+    return M <= 32 and hidden <= 768 and hidden in ((64 * heads,) if f16 else (32 * heads, 64 * heads)) and texts == 1
+
+
+def gemm_ln(a, w, bias, epi: int = EPI_BIAS, norm=None, resid=None, st_out=None, attn=None):
     """bf16 or fp16 products of up to 64 rows between LayerNorms. norm = (st, g, b, eps): the rows of ``a`` (EPI_BIAS, EPI_GELU) or
     of ``resid`` (EPI_RESID) are sums whose LayerNorm is taken here, by the statistics st (fp32 [64, 64, 2]) that the
-    EPI_RESID product which made them wrote as its ``st_out``."""
+    EPI_RESID product which made them wrote as its ``st_out``. attn = (heads, cu_seqlens) (EPI_RESID, ``attn_ln_fit``):
+    ``a`` holds q, k and v, and the product is that of their attention's output."""
     f16 = a.dtype == torch.float16
     is_cuda = _f16_cuda if f16 else _bf16_cuda
     is_cuda(a, "a"); is_cuda(w, "w"); is_cuda(bias, "bias")
     M, K = a.shape
+    if attn is not None:
+        heads, cu = attn
+        _i32(cu, "cu_seqlens")
+        _req(K % 3 == 0 and attn_ln_fit(M, K // 3, heads, cu.numel() - 1, f16) and epi == EPI_RESID, "gemm_ln attention")
+        K //= 3
     N = w.shape[0]
     _req(gemm_ln_fit(M, K if epi != EPI_RESID else N, N if epi != EPI_RESID else K) and w.shape[1] == K
          and bias.shape == (N,) and bias.is_contiguous(), f"gemm_ln shape M={M} N={N} K={K}")
@@ -569,6 +582,12 @@ def gemm_ln(a, w, bias, epi: int = EPI_BIAS, norm=None, resid=None, st_out=None)
         is_cuda(resid, "resid")
         _req(resid.shape == (M, N) and resid.stride(1) == 1 and resid.stride(0) % 8 == 0, "bad resid")
     out = torch.empty((M, N), dtype=a.dtype, device=a.device)
+    if attn is not None:
+        D = K // heads
+        _check(lib().da_enc_attn_rows(_ptr(a), a.stride(0), _ptr(w), _ptr(out), N, _ptr(bias), _ptr(resid), resid.stride(0), M, N, K,
+                                     D, _ptr(cu), math.log2(math.e) / math.sqrt(D), _ptr(st), _ptr(g), _ptr(b),
+                                     float(eps), _ptr(st_out), f16, _stream()), "gemm_ln")
+        return out
     _check(lib().da_enc_rows(_ptr(a), a.stride(0), _ptr(w), _ptr(out), N, _ptr(bias), _ptr(resid),
                             0 if resid is None else resid.stride(0), M, N, K, epi, _ptr(st), _ptr(g), _ptr(b), float(eps),
                             _ptr(st_out), f16, _stream()), "gemm_ln")
