@@ -38,7 +38,6 @@ struct EncRowsArgs {
 // The waves' stages (ST of each) and, after the last unit, their sums share LDS: up to enc_waves(FM) waves.
 constexpr int enc_waves(int fm) { return fm == 4 ? 12 : 16; }
 constexpr int enc_stages(int fm) { return fm == 1 ? 2 : 1; }
-constexpr int ENC_ATTN_UNITS = 12;  // of 12 KB of LDS
 
 // Attention inside the product that takes its output (D != 0: heads of D; A is then q, k and v beside one another, one text of
 // KR rows at most): a unit of 64 k is a head of 64 or two of 32, so its wave attends for the block's 16 rows and the result is
@@ -50,17 +49,20 @@ constexpr int ENC_ATTN_UNITS = 12;  // of 12 KB of LDS
 // written), so they come by LDS-DMA, and only the text's: straight to the MFMA the question took as long as with a launch
 // between, 64 rows 10 % longer. Texts that share blocks had to take turns with V (a NaN of one reaches another through weights
 // of zero), 6 us a layer for seven: one text only. One of 21 tokens through 12 layers of 768: 333
-// -> 302 us, of 20 through 384 (heads of 32) 278 -> 246. More than 12 waves of 12 KB don't fit a CU's LDS.
-template <typename T, int FM, bool LNA, int EPI, int D = 0, int KR = 0>
+// -> 302 us, of 20 through 384 (heads of 32) 278 -> 246. 20 through 24
+// of 1024: 811 -> 760, of 60 through 384: 310 -> 285.
+template <typename T, int FM, bool LNA, int EPI, int D = 0, int KR = 0, int UNITS = 0>
 __global__ void __launch_bounds__(64 * enc_waves(FM))
 enc_rows_kernel(EncRowsArgs p) {
   constexpr int ROWS = FM * 16, SLD = 20, ST = enc_stages(FM), A_BYTES = ROWS * 128, STAGE = A_BYTES + 2048;
   constexpr int PA = 2 * FM, P = PA + 2;  // LDS-DMA instructions of a stage
-  constexpr int RING = D ? KR * 256 + 4096 : ST * STAGE;  // a wave's stages, or its W, Q, K and V
+  constexpr bool WIDE = UNITS > 12;  // (W straight to registers, the statistics in LDS after the sums: 160 KB are full)
+  constexpr int RING = D ? KR * 256 + (WIDE ? 2048 : 4096) : ST * STAGE;  // a wave's stages, or its K, V, Q and W
   static_assert(ROWS * SLD * 4 <= RING, "the sums fit the stages");
   static_assert(!D || (FM == 1 && !LNA), "attention: 16 rows a block");
-  __shared__ __attribute__((aligned(16))) char smem[(D ? ENC_ATTN_UNITS : enc_waves(FM)) * RING];
-  __shared__ float smean[ROWS], srstd[ROWS];
+  __shared__ __attribute__((aligned(16))) char smem[(D ? UNITS : enc_waves(FM)) * RING];
+  __shared__ float sstat[WIDE ? 1 : 2 * ROWS];
+  float *smean = WIDE ? (float*)smem + 16 * ROWS * SLD : sstat, *srstd = smean + ROWS;
   float (*red)[ROWS][SLD] = (float (*)[ROWS][SLD])smem;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
   const int fr = lane & 15, fg = lane >> 4;
@@ -124,32 +126,39 @@ enc_rows_kernel(EncRowsArgs p) {
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)(p.W + (size_t)n0 * p.K), (short)0, 0x7fffff00, 0x00020000);
   char* ring = smem + w * RING;
   constexpr int NT = D ? KR / 16 : 1;
-  if constexpr (D != 0) {  // unit w: 2 KB each of W and Q, then K and V; rows past the last text read as zero
+  bf16x8_t aw[2];
+  if constexpr (D != 0) {  // unit w; rows outside the text read as zero
+    if constexpr (WIDE) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int r = 8 * j + (lane >> 3);
-      const unsigned at = (unsigned)r * (unsigned)(p.K * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t)(ring + j * 1024), 16, at, w * 128, 0, 0);
+      for (int h = 0; h < 2; ++h) aw[h] = *(const bf16x8_t*)(p.W + (size_t)(n0 + fr) * p.K + w * 64 + 32 * h + 8 * fg);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int r = 8 * j + (lane >> 3);
+        const unsigned at = (unsigned)r * (unsigned)(p.K * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t)(ring + KR * 256 + 2048 + j * 1024), 16, at, w * 128, 0, 0);
+      }
     }
+    asm volatile("" ::: "memory");
     auto row = [&](int r, int at) __attribute__((always_inline)) { return r >= first && r < end ? (unsigned)r * (unsigned)(p.lda * 2) + at : 0x7ffffff0u; };
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int r = 8 * j + (lane >> 3);
       const unsigned at = row(m0 + r, ((lane & 7) ^ ((r >> 1) & 7)) << 4);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(ring + 2048 + j * 1024), 16, at, w * 128, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(ring + KR * 256 + j * 1024), 16, at, w * 128, 0, 0);
     }
 #pragma unroll
     for (int j = 0; j < KR / 8; ++j) {
       const int r = 8 * j + (lane >> 3);
       const unsigned at = row(r, ((lane & 7) ^ ((r >> 1) & 7)) << 4);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(ring + 4096 + j * 1024), 16, at, p.K * 2 + w * 128, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(ring + j * 1024), 16, at, p.K * 2 + w * 128, 0, 0);
     }
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int j = 0; j < KR / 8; ++j) {  // (last, for the wait: V's chunk c of row r at slot c ^ ((r & 2) << 1))
       const int r = 8 * j + (lane >> 3);
       const unsigned at = row(r, ((lane & 7) ^ ((r & 2) << 1)) << 4);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(ring + 4096 + KR * 128 + j * 1024), 16, at, p.K * 4 + w * 128, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(ring + KR * 128 + j * 1024), 16, at, p.K * 4 + w * 128, 0, 0);
     }
   }
   // ---- the wave's units w, w + nw, ..: row r's 16-B chunk c of 64 k at slot c ^ (r >> 1 & 7) of its 128 B ----
@@ -185,7 +194,7 @@ enc_rows_kernel(EncRowsArgs p) {
 #pragma unroll
   for (int i = 0; i < ST; ++i)
     if (!D && w + i * nw < units) ask(w + i * nw, i);
-  if (p.st) {
+  if (p.st && !WIDE) {
     asm volatile("" ::: "memory");
     stats_merge(4 * w + fg);
     for (int r = 4 * (w + nw) + fg; r - fg < ROWS; r += 4 * nw) {
@@ -204,13 +213,13 @@ enc_rows_kernel(EncRowsArgs p) {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(KR / 8) : "memory");  // everything but V
     __builtin_amdgcn_sched_barrier(0);
     const int at[2] = {fr * 128 + ((fg ^ ((fr >> 1) & 7)) << 4), fr * 128 + (((4 + fg) ^ ((fr >> 1) & 7)) << 4)};
-    bf16x8_t aw[2], aq[2], ak[4][2];
+    bf16x8_t aq[2], ak[4][2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      aw[h] = *(const bf16x8_t*)(ring + at[h]);
-      aq[h] = *(const bf16x8_t*)(ring + 2048 + at[h]);
+      if constexpr (!WIDE) aw[h] = *(const bf16x8_t*)(ring + KR * 256 + 2048 + at[h]);
+      aq[h] = *(const bf16x8_t*)(ring + KR * 256 + at[h]);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) ak[t][h] = *(const bf16x8_t*)(ring + 4096 + t * 2048 + at[h]);
+      for (int t = 0; t < NT; ++t) ak[t][h] = *(const bf16x8_t*)(ring + t * 2048 + at[h]);
     }
     f32x4_t s[2][4];
     bf16x8_t pf[2][2];
@@ -250,7 +259,7 @@ enc_rows_kernel(EncRowsArgs p) {
     for (int i = 0; i < 4; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // V
     __builtin_amdgcn_sched_barrier(0);
-    const char* v = ring + 4096 + KR * 128 + (4 * fg + (fr >> 2)) * 128;
+    const char* v = ring + KR * 128 + (4 * fg + (fr >> 2)) * 128;
 #pragma unroll
     for (int t = 0; t < NT; t += 2)
 #pragma unroll
@@ -309,6 +318,7 @@ enc_rows_kernel(EncRowsArgs p) {
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < FM; ++i) *(f32x4_t*)&red[w][16 * i + fr][4 * fg] = acc[i];
+  if (WIDE && p.st) stats_merge(4 * w + fg);  // (13 waves or more: all rows)
   __syncthreads();
   if (tid >= 4 * ROWS) return;  // (whole waves)
   if (EPI == EPI_RESID && FM == 4 && out && p.st) {  // (no registers for them before)
@@ -374,7 +384,10 @@ static int enc_rows_rows(const EncRowsArgs& a, int epi, hipStream_t s) {
 
 template <typename T, int D>
 static int enc_attn_rows(const EncRowsArgs& a, hipStream_t s) {
-  enc_rows_kernel<T, 1, false, EPI_RESID, D, 32><<<dim3(a.N / 16, (a.M + 15) / 16), a.K, 0, s>>>(a);  // (a wave a unit)
+  const dim3 grid(a.N / 16, (a.M + 15) / 16);
+  if (a.M > 32) enc_rows_kernel<T, 1, false, EPI_RESID, D, 64, 6><<<grid, a.K, 0, s>>>(a);
+  else if (a.K <= 768) enc_rows_kernel<T, 1, false, EPI_RESID, D, 32, 12><<<grid, a.K, 0, s>>>(a);  // (a wave a unit)
+  else enc_rows_kernel<T, 1, false, EPI_RESID, D, 32, 16><<<grid, a.K, 0, s>>>(a);
   return (int)hipGetLastError();
 }
 
@@ -395,11 +408,11 @@ DA_EXPORT int da_enc_rows(const void* A, int lda, const void* W, void* C, int ld
 }
 
 // RESID with A the attention of K / D heads of D (64, and 32 in bf16) over the one text of rows cu[0] .. cu[1] - 1: qkv holds q, k and v, K
-// columns each. M <= 32, K <= 768; the rest as above.
+// columns each. M <= 32, K <= 1024 or M <= 64, K <= 384 (LDS); the rest as above.
 DA_EXPORT int da_enc_attn_rows(const void* qkv, int lda, const void* W, void* C, int ldc, const void* bias, const void* resid, int ldr,
                               int M, int N, int K, int D, const int* cu, float c, const float* st, const void* g,
                               const void* b, float eps, float* st_out, int f16, void* stream) {
-  if (M < 1 || M > 32 || K < 64 || K % 64 || K > 64 * ENC_ATTN_UNITS || N < 16 || N % 16 || N > 1024 || lda % 8 || lda < 3 * K || ldc % 4 || ldr % 4 ||
+  if (M < 1 || M > (K > 384 ? 32 : 64) || K < 64 || K % 64 || K > 1024 || N < 16 || N % 16 || N > 1024 || lda % 8 || lda < 3 * K || ldc % 4 || ldr % 4 ||
       lda > (1 << 22) || (D != 64 && (D != 32 || f16)) || !cu || !resid || !st_out || (st && (!g || !b)))
     return (int)hipErrorInvalidValue;
   EncRowsArgs a{(const bf16_t*)qkv, (const bf16_t*)W, (const bf16_t*)bias, (const bf16_t*)resid, (bf16_t*)C, st,

@@ -546,7 +546,7 @@ def gemm_ln_fit(M: int, hidden: int, ffn: int) -> bool:
 
 def attn_ln_fit(M: int, hidden: int, heads: int, texts: int, f16: bool = False) -> bool:
     """Whether ``gemm_ln`` takes attention inside (``attn``) where an encoder's products take it."""
-    return M <= 32 and hidden <= 768 and hidden in ((64 * heads,) if f16 else (32 * heads, 64 * heads)) and texts == 1
+    return M <= (32 if hidden > 384 else 64) and hidden <= 1024 and hidden in ((64 * heads,) if f16 else (32 * heads, 64 * heads)) and texts == 1
 
 
 def gemm_ln(a, w, bias, epi: int = EPI_BIAS, norm=None, resid=None, st_out=None, attn=None):

@@ -1,4 +1,4 @@
-"""Attention of one text inside the encoder product behind it (up to 32 rows), against 64-bit arithmetic."""
+"""Attention of one text inside the encoder product behind it (up to 32 or 64 rows), against 64-bit arithmetic."""
 import math
 
 import pytest
@@ -21,10 +21,11 @@ def attend(qkv, heads, cu):
     return (t.transpose(0, 1).reshape(M, h) for t in (o, m))
 
 
-# (rows, hidden, heads, text): one row; edges of the 16-row blocks; rows before the text and past it; one unit of K, and 12
+# (rows, hidden, heads, text): one row; edges of the 16-row blocks; rows before the text and past it; one unit of K, 12, 13 and 16
 @pytest.mark.parametrize("M,h,heads,cu", [
     (1, 768, 12, [0, 1]), (16, 128, 4, [0, 16]), (17, 64, 1, [0, 17]), (32, 768, 12, [0, 32]), (31, 384, 12, [0, 31]),
-    (32, 768, 24, [0, 21]), (32, 384, 6, [5, 19]), (32, 512, 8, [17, 18]), (9, 64, 2, [0, 9]), (16, 128, 2, [0, 5])])
+    (32, 768, 24, [0, 21]), (32, 384, 6, [5, 19]), (32, 512, 8, [17, 18]), (9, 64, 2, [0, 9]), (32, 1024, 16, [0, 32]), (19, 832, 13, [0, 17]), (17, 1024, 32, [0, 17]), (64, 384, 12, [0, 64]), (33, 384, 6, [0, 33]),
+    (50, 128, 2, [3, 47]), (16, 128, 2, [0, 5])])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 def test_attention_inside(M, h, heads, cu, dt):
     if dt == torch.float16 and h == 32 * heads:
@@ -55,7 +56,7 @@ def test_what_attention_refuses():
     st, i32 = torch.zeros((64, 64, 2), device="cuda"), lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
     run = lambda M, h, heads, cu: K.gemm_ln(t(M, 3 * h), t(h, h), t(h), K.EPI_RESID, resid=t(M, h), st_out=st, attn=(heads, cu))  # noqa: E731
     run(8, 128, 2, i32([0, 8]))
-    for M, h, heads, cu in [(33, 128, 2, i32([0, 33])), (8, 832, 13, i32([0, 8])), (8, 128, 1, i32([0, 8])),
+    for M, h, heads, cu in [(33, 448, 7, i32([0, 33])), (65, 128, 2, i32([0, 65])), (8, 1088, 17, i32([0, 8])), (8, 128, 1, i32([0, 8])),
                             (8, 128, 2, i32([0, 4, 8])), (8, 128, 2, i32([0, 8]).long()), (8, 128, 2, i32([0, 8]).cpu())]:
         with pytest.raises(ValueError):
             run(M, h, heads, cu)
