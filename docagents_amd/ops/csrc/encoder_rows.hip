@@ -48,9 +48,8 @@ constexpr int enc_stages(int fm) { return fm == 1 ? 2 : 1; }
 // All strips do the same attention over again. What it costs is its operands (10 KB a wave at 32 rows, which other dies have just
 // written), so they come by LDS-DMA, and only the text's: straight to the MFMA the question took as long as with a launch
 // between, 64 rows 10 % longer. Texts that share blocks had to take turns with V (a NaN of one reaches another through weights
-// of zero), 6 us a layer for seven: one text only. One of 21 tokens through 12 layers of 768: 333
-// -> 302 us, of 20 through 384 (heads of 32) 278 -> 246. 20 through 24
-// of 1024: 811 -> 760, of 60 through 384: 310 -> 285.
+// of zero), 6 us a layer for seven: one text only. One of 21 tokens through 12 layers of 768: 333 -> 302 us, of 20 through 384
+// (heads of 32) 278 -> 246, of 60 there 310 -> 285, of 20 through 24 of 1024 811 -> 760.
 template <typename T, int FM, bool LNA, int EPI, int D = 0, int KR = 0, int UNITS = 0>
 __global__ void __launch_bounds__(64 * enc_waves(FM))
 enc_rows_kernel(EncRowsArgs p) {
