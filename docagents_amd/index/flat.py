@@ -45,7 +45,7 @@ class FlatIndex:
         self.lock = threading.RLock()
         self._write_ev = None   # event after the last mutation's device work (None: nothing pending)
         self._read_evs: dict = {}  # reader stream handle -> event after its last read
-        self._read_on = None       # stream handle of the read that is open
+        self._read_on = None       # stream handle of the read that is open, None after a write inside it
         self._depth = 0
 
     # ----------------------------------------------------------------- stream ordering
@@ -79,6 +79,7 @@ class FlatIndex:
                     ev.record(torch.cuda.current_stream(self.device))
                     self._write_ev = ev
                     self._read_evs.clear()  # this write is ordered after every one of them
+                    self._read_on = None    # the open read's wait was for the write before: one inside it waits by itself
 
     @contextlib.contextmanager
     def reading(self):
