@@ -45,7 +45,8 @@ class FlatIndex:
         self.lock = threading.RLock()
         self._write_ev = None   # event after the last mutation's device work (None: nothing pending)
         self._read_evs: dict = {}  # reader stream handle -> event after its last read
-        self._read_on = None       # stream handle of the read that is open, None after a write inside it
+        self._reads: list = []     # streams of the reads that are open, outermost first
+        self._read_on = None       # handle of the innermost one's, None after a write inside it
         self._depth = 0
 
     # ----------------------------------------------------------------- stream ordering
@@ -70,6 +71,9 @@ class FlatIndex:
                     st.wait_event(self._write_ev)
                 for ev in self._read_evs.values():
                     st.wait_event(ev)
+                for r in self._reads:  # (these leave their events when they end)
+                    if r.cuda_stream != st.cuda_stream:
+                        st.wait_stream(r)
             try:
                 yield
             finally:
@@ -91,9 +95,11 @@ class FlatIndex:
             if self._write_ev is not None:
                 st.wait_event(self._write_ev)
             outer, self._read_on = self._read_on, st.cuda_stream
+            self._reads.append(st)
             try:
                 yield
             finally:
+                self._reads.pop()
                 self._read_on = outer
                 ev = self._read_evs.get(st.cuda_stream) or torch.cuda.Event()
                 ev.record(st)

@@ -93,6 +93,16 @@ def test_write_after_each_of_two_reads(index):
         assert w.after(a)
 
 
+def test_write_on_another_stream_inside_a_read(index):
+    a, b, w = streams()
+    with index.read(a):
+        a.work()
+        with index.read(b):
+            b.work()
+            with index.write(w):
+                assert w.after(a) and w.after(b)
+
+
 @pytest.mark.parametrize("same", [False, True])
 def test_nested_read_after_a_write_on_another_stream(index, same):
     a, b, w = streams()
