@@ -94,13 +94,13 @@ class FlatIndex:
                 return
             if self._write_ev is not None:
                 st.wait_event(self._write_ev)
-            outer, self._read_on = self._read_on, st.cuda_stream
+            outer, wrote, self._read_on = self._read_on, self._write_ev, st.cuda_stream
             self._reads.append(st)
             try:
                 yield
             finally:
                 self._reads.pop()
-                self._read_on = outer
+                self._read_on = outer if self._write_ev is wrote else None
                 ev = self._read_evs.get(st.cuda_stream) or torch.cuda.Event()
                 ev.record(st)
                 self._read_evs[st.cuda_stream] = ev

@@ -115,3 +115,13 @@ def test_nested_read_after_a_write_on_another_stream(index, same):
         a.work()
     with index.write(w):
         assert w.after(a) and w.after(b)
+
+
+def test_read_on_the_outer_stream_after_a_write_inside_another_read(index):
+    a, b, w = streams()
+    with index.read(a):
+        with index.read(b):
+            with index.write(w):
+                w.work()
+        with index.read(a):
+            assert a.after(w)
