@@ -12,6 +12,7 @@
 //                 ties -> smaller row id first).
 //  * kmeans_accum: centroid sums / counts for IVFFlat training (fp32 atomics, 256-B rows).
 #include <cstring>
+#include <type_traits>
 
 #include "common.h"
 
@@ -473,19 +474,23 @@ struct TopList {
 // A filter's ranges come from the host. Up to TR_TABLE numbers of them ride in the launch's arguments (range_off, then the
 // ranges; a workgroup takes them to LDS in one step); as two copies they took 3.3 us each on the device and about 15 on the
 // host. With the ids looked up by the last kernel and one pair of events a search, one query over 8 of 100000 x 768 rows'
-// documents takes 33 us, 94 before; 24 queries over 8 of 512 lists 65, 78 before.
+// documents takes 33 us, 94 before. Lists, and ranges that are on the device, have a kernel without the table (scores and merge,
+// us with it -> without: 24 queries over 8 of 512 lists of 400000 x 768 rows 68.7 -> 58.2, 8 over 16 of 256 of 200000 x 384 53 -> 45,
+// 8 ranges of 50 rows a query for 64 queries 21.9 -> 19.7).
 constexpr int TR_TABLE = 512;  // 2 of the 4 KB that a launch's arguments may have
 struct RangeTable { int v[TR_TABLE]; };
+struct NoTable { int v[1]; };
 
-template <int NCH>
+template <int NCH, typename Table>
 __global__ void __launch_bounds__(256)
 topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ slots,
                    const bf16_t* __restrict__ Qv, int Q, const int* __restrict__ ranges,
                    const int* __restrict__ range_off, const int* __restrict__ lists, int probes,
                    const unsigned* __restrict__ bitmap, int W, float thr,
                    int K, int rows_per_split, float* __restrict__ out_s, int* __restrict__ out_i, int n_table,
-                   const RangeTable table) {
-  __shared__ int st[TR_TABLE];
+                   const Table table) {
+  constexpr bool TABLE = std::is_same_v<Table, RangeTable>;
+  __shared__ int st[TABLE ? TR_TABLE : 1];
   __shared__ float sc[2][64];
   __shared__ int sr[2][64];
   __shared__ float cs[TL_SL];
@@ -495,9 +500,12 @@ topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ 
   const int half = lane >> 5, l32 = lane & 31;
   TopList top;
   top.init(cs, ci, K);  // (every wave writes the same empty list; wave 0 keeps it)
-  for (int i = tid; i < n_table; i += 256) st[i] = table.v[i];
-  if (n_table) __syncthreads();
-  const auto range = [&](int i) { return n_table ? st[Q + 1 + i] : ranges[i]; };
+  if constexpr (TABLE) {
+    for (int i = tid; i < n_table; i += 256) st[i] = table.v[i];
+    __syncthreads();
+    lists = nullptr;
+  }
+  const auto range = [&](int i) { return TABLE ? st[Q + 1 + i] : ranges[i]; };
   const int nch = d / 8;  // 16-B chunks of a row; this lane has chunks l32 + 32 i
   float qv[NCH][8];
 #pragma unroll
@@ -507,7 +515,7 @@ topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ 
 #pragma unroll
     for (int e = 0; e < 8; ++e) qv[i][e] = bf2f((bf16_t)((e & 1) ? (u[e >> 1] >> 16) : (u[e >> 1] & 0xffff)));
   }
-  const int rb = n_table ? st[q] : lists ? q * probes : range_off[q], re = n_table ? st[q + 1] : lists ? rb + probes : range_off[q + 1];
+  const int rb = TABLE ? st[q] : lists ? q * probes : range_off[q], re = TABLE ? st[q + 1] : lists ? rb + probes : range_off[q + 1];
   DA_ASSERT(rb >= 0 && re >= rb);
   const int pbeg = split * rows_per_split, pend = pbeg + rows_per_split;
   __syncthreads();
@@ -1024,23 +1032,31 @@ DA_EXPORT int da_topk_ranges(const void* X, int d, const void* slots, const void
       (n_table && (lists || !host_table || n_table < Q + 1)))
     return (int)hipErrorInvalidValue;
   if (Q == 0) return 0;
-  RangeTable table;
-  if (n_table) memcpy(table.v, host_table, (size_t)n_table * sizeof(int));
   hipStream_t s = (hipStream_t)stream;
   float* cs = (float*)ws;
   int* ci = (int*)(cs + (size_t)splits * Q * K);
   dim3 grid(splits, Q);
+  auto launch = [&](const auto& table) {
+    using Table = std::decay_t<decltype(table)>;
 #define TRG(NCH)                                                                                                    \
-  topk_ranges_kernel<NCH><<<grid, 256, 0, s>>>((const bf16_t*)X, d, (const int*)slots, (const bf16_t*)Qv, Q,        \
-                                               (const int*)ranges, (const int*)range_off, (const int*)lists,        \
-                                               probes, (const unsigned*)bitmap, W, thr, K, rows_per_split, cs, ci, n_table, table)
-  if (d <= 256) TRG(1);
-  else if (d <= 512) TRG(2);
-  else if (d <= 768) TRG(3);
-  else if (d <= 1024) TRG(4);
-  else if (d <= 2048) TRG(8);
-  else TRG(16);
+  topk_ranges_kernel<NCH, Table><<<grid, 256, 0, s>>>((const bf16_t*)X, d, (const int*)slots, (const bf16_t*)Qv, Q, \
+                                                      (const int*)ranges, (const int*)range_off, (const int*)lists, \
+                                                      probes, (const unsigned*)bitmap, W, thr, K, rows_per_split, cs, ci, n_table, table)
+    if (d <= 256) TRG(1);
+    else if (d <= 512) TRG(2);
+    else if (d <= 768) TRG(3);
+    else if (d <= 1024) TRG(4);
+    else if (d <= 2048) TRG(8);
+    else TRG(16);
 #undef TRG
+  };
+  if (n_table) {
+    RangeTable table;
+    memcpy(table.v, host_table, (size_t)n_table * sizeof(int));
+    launch(table);
+  } else {
+    launch(NoTable{});
+  }
   int err = (int)hipGetLastError();
   if (err) return err;
   return topk_merge(cs, ci, splits, Q, K, top_out(out_s, out, ids, n_ids), s);

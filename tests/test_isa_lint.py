@@ -116,3 +116,14 @@ def test_whole_tile_products_carry_no_shared_round(tmp_path):
         r"\.name:\s+(\S+)\n(?:(?!\.name:).)*?\.sgpr_spill_count:\s+(\d+)", asm, re.S)}
     whole = {n: c for n, c in spills.items() if re.match(r"_Z13gemm8p_kernelILi[0134]ELi(128|256)E\d*B?F16TLb1ELb0E", n)}
     assert len(whole) == 14 and max(whole.values()) <= 6, whole
+
+
+def test_searches_over_lists_carry_no_table(tmp_path):
+    """The table of a filter's ranges (2 KB of arguments and of LDS) is in instances of its own: searches over lists, which
+    have none, took 5 - 18 % longer with it."""
+    asm = _asm("vecsearch.hip", tmp_path)
+    sizes = {m.group(3): (int(m.group(1)), int(m.group(2))) for m in re.finditer(
+        r"\.group_segment_fixed_size:\s+(\d+)\n(?:(?!\.group_segment_fixed_size:).)*?\.kernarg_segment_size:\s+(\d+)"
+        r"(?:(?!\.group_segment_fixed_size:).)*?\.name:\s+(\S+)\n", asm, re.S) if "topk_ranges_kernel" in m.group(3)}
+    lean = {n for n, (lds, args) in sizes.items() if lds < 2048 and args < 512}
+    assert len(sizes) == 12 and len(lean) == 6, sizes
