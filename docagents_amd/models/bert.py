@@ -223,15 +223,16 @@ class BertEncoder:
     # GEMMs / norms process them (their rows are independent) and flash attention and the pooling
     # read the real length from cu_seqlens, so row 0..L-1 see exactly the unpadded computation.
     GRAPH_BUCKETS = (16, 32, 64, 128)
-    # small batches of short texts (the fast embed lane's micro-batches of questions): one graph per
-    # (sequences, padded tokens) bucket; sequences packed back to back, then padding rows, padded
+    # small batches of short texts (the fast embed lane's micro-batches of questions): (sequences,
+    # padded tokens) buckets; sequences packed back to back, then padding rows, padded
     # sequences of length 0 (cu repeats the real total); every real length <= BATCH_MAX_LEN, which is
     # the max_seqlen the graphs were captured with. Measured: a lane batch took ~5 ms of launches
     # from Python beside the decode thread (profiles/r6/stack: es_embed)
     BATCH_BUCKETS = ((2, 64), (4, 128), (8, 256), (16, 512), (32, 1024), (64, 2048))
     BATCH_MAX_LEN = 128
     # and of texts of 8 and 16 tokens: in a bucket of 32 tokens a text three rows of four are padding (45 texts of 6 - 8 tokens
-    # through a base encoder in fp8: 971 us in 2048 rows, 545 in 512)
+    # through a base encoder in fp8: 971 us in 2048 rows, 545 in 512). Buckets of as many rows share a graph, with offsets for the
+    # most sequences among them: six to capture, not fourteen (preparing a base encoder 59.5 -> 39 ms, the graphs of a small one 254 -> 141 MB)
     SHORT_BUCKETS = ((8, 64), (8, 128), (16, 128), (16, 256), (32, 256), (32, 512), (64, 512), (64, 1024))
 
     def _capture_small(self):
@@ -243,13 +244,13 @@ class BertEncoder:
         side = torch.cuda.Stream(device=dev)
         side.wait_stream(torch.cuda.current_stream(dev))
         Lc = self.BATCH_MAX_LEN
-        # (key, T, max_seqlen, cu): the one-sequence length buckets and the batch buckets
+        # (key, T, max_seqlen, cu): the one-sequence length buckets and the batches' row counts
         shapes = [(("one", T), T, T, [0, T]) for T in self.GRAPH_BUCKETS]
-        for kind, buckets in (("batch", self.BATCH_BUCKETS), ("short", self.SHORT_BUCKETS)):
-            for nb, T in buckets:
-                step = min(Lc, (T - 1) // nb)
-                shapes.append(((kind, nb, T), T, Lc, [i * step for i in range(nb + 1)]))
-        bufs = {}
+        most = {T: max(nb for nb, rows in (*self.BATCH_BUCKETS, *self.SHORT_BUCKETS) if rows == T) for _, T in self.BATCH_BUCKETS}
+        for T, nb in most.items():
+            step = min(Lc, (T - 1) // nb)
+            shapes.append((("batch", T), T, Lc, [i * step for i in range(nb + 1)]))
+        bufs, batch = {}, {}
         # In a workspace role of their own, and EVERY shape warmed before the first capture: the
         # split-K scratch only grows, and a growth after a capture would free the memory that graph
         # captured (an illegal address at its next replay). The scratch is checked unchanged below.
@@ -271,10 +272,10 @@ class BertEncoder:
                     out = pool(self.forward(ids, pos, cu, ms), cu, mode)
                 if key[0] == "one":
                     self._g[T] = (g, ids, cu, out)
-                elif key[0] == "batch":
-                    self._gb[key[1]] = (T, g, ids, pos, cu, out)
                 else:
-                    self._gs[key[1:]] = (T, g, ids, pos, cu, out)
+                    batch[T] = (T, g, ids, pos, cu, out)
+            self._gb = {nb: batch[T] for nb, T in self.BATCH_BUCKETS}
+            self._gs = {(nb, T): batch[T] for nb, T in self.SHORT_BUCKETS}
             if K.workspace_buffer(dev) is not ws0:
                 raise RuntimeError("encoder graph capture grew the enc_graph workspace")
         torch.cuda.current_stream(dev).wait_stream(side)
@@ -340,7 +341,8 @@ class BertEncoder:
         fit += [(T, nb, self._gs[nb, T]) for nb, T in self.SHORT_BUCKETS if nb >= n and T > tot and (nb, T) in self._gs]
         if not fit:
             return None
-        _, b, (T, g, ids, pos, cu, out) = min(fit, key=lambda f: f[:2])
+        T, g, ids, pos, cu, out = min(fit, key=lambda f: f[:2])[2]
+        b = cu.numel() - 1
         host = np.zeros(2 * T + b + 1, dtype=np.int32)
         host[:tot] = np.fromiter((t for q in seqs for t in q), dtype=np.int32, count=tot)
         c = np.zeros(n + 1, dtype=np.int64)
