@@ -678,6 +678,15 @@ def encoder_layers_fit(rows: int) -> bool:
     return rows > 64
 
 
+def _encoder_sets(rows: int, hidden: int, ffn: int) -> int:
+    """Sets of buffers that an encoder's layers take in turn: two while both fit the dies' L2s (8 of 4 MB), one from there on. A kernel
+    that writes over what all dies' caches have just read waits for them to give it up; where the buffers leave the L2s anyway, a
+    second set only makes more of them leave. us of 12 layers, one / two: 512 rows of 384 columns, fp8 401 / 372, 1024 481 / 461, 256 of
+    768 445 / 417, 24 layers of 1024, fp16, 128 995 / 963; 2000 of 384 646 / 644, 1000 of 768, bf16 738 / 734, 3000 1313 / 1456, 4000 1464 /
+    1566, 12000 of 384 1580 / 1712, 8100 of 1024, fp8 5823 / 6013."""
+    return 2 if rows * (8 * hidden + ffn) * 2 <= 16 << 20 else 1
+
+
 def encoder_layers(x, layers, cu_seqlens, max_seqlen: int, heads: int, head_dim: int, eps: float, xq=None):
     """The layers of an encoder over x [T, hidden] (bf16, fp16; with xq = (e4m3 rows, scales) the fp8 products of
     ``gemm_fp8``) -> [T, hidden]: what gemm / gemm_f16 / gemm_fp8, the attention and the LayerNorms give one by one, with
@@ -692,10 +701,8 @@ def encoder_layers(x, layers, cu_seqlens, max_seqlen: int, heads: int, head_dim:
     _req(h % (128 if q8 else 64) == 0 and ffn % 64 == 0 and (not f16 or min(h, ffn) >= 128), f"hidden {h}, feed-forward {ffn}")
     stream, L, dt = _raw_stream(), _EncoderLayer(), x.dtype
     new = lambda n: torch.empty((T, n), dtype=dt, device=x.device)  # noqa: E731
-    # Two sets of buffers, layers in turn: a kernel that writes over what all dies' caches have just read waits for them to give it
-    # up (57 short texts, width 384, fp8: 684 us with one set, 650 with two; 651, 653 and 683 with 3, 8 and 12).
     sets = [{n: new(c) for n, c in (("qkv", 3 * h), ("a", h), ("y0", h), ("m", h), ("f", ffn), ("y1", h), ("x", h))}
-            for _ in layers[:2]]
+            for _ in layers[:_encoder_sets(T, h, ffn)]]
     L.cu = cu_seqlens.data_ptr()
     if q8:
         _req(xq[0].dtype == FP8 and xq[0].shape == x.shape and xq[0].is_contiguous() and xq[0].data_ptr() % 16 == 0
@@ -729,7 +736,7 @@ def encoder_layers(x, layers, cu_seqlens, max_seqlen: int, heads: int, head_dim:
         need += [("wqkv_s", row3, torch.float32), ("w1_s", rowf, torch.float32)]
     run, at = lib().da_encoder_layer, ctypes.byref(L)
     for n, layer in enumerate(layers):
-        S = sets[n & 1]
+        S = sets[n % len(sets)]
         L.qkv, L.a, L.f, L.y[:] = S["qkv"].data_ptr(), S["a"].data_ptr(), S["f"].data_ptr(), (S["y0"].data_ptr(), S["y1"].data_ptr())
         L.x[:] = [t.data_ptr() for t in (x, S["m"], S["x"])]
         if q8:

@@ -26,6 +26,29 @@ def test_layers_are_the_operations(hidden, heads, ffn, dtype, rows, monkeypatch)
     assert torch.isfinite(want).all() and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp8"])
+def test_memory_of_long_batches(dtype, monkeypatch):
+    """A long batch's layers hold no more at a time than the operations do one by one."""
+    rows = 20000
+    cfg = EncoderConfig(name="layers", vocab=500, hidden=1024, layers=3, heads=16, ffn=4096, max_pos=512)
+    enc = BertEncoder(cfg, seed=rows, dtype=dtype)
+    ids = torch.zeros(rows, dtype=torch.int32).cuda()
+    pos = torch.arange(rows, dtype=torch.int32).cuda() % 400
+    cu = torch.arange(0, rows + 1, 400, dtype=torch.int32).cuda()
+
+    def peak():
+        enc.forward(ids, pos, cu, 400)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        held = torch.cuda.memory_allocated()
+        enc.forward(ids, pos, cu, 400)
+        return torch.cuda.max_memory_allocated() - held
+    got = peak()
+    monkeypatch.setattr(enc.ops, "encoder_layers_fit", lambda n: False)
+    # (the buffers of a layer are all there at once, not one by one: a width or two of twelve more)
+    assert got <= 1.2 * peak()
+
+
 def test_bad_weights_are_refused():
     cfg = EncoderConfig(name="layers", vocab=500, hidden=384, layers=1, heads=6, ffn=1536, max_pos=512)
     enc = BertEncoder(cfg, seed=1)
