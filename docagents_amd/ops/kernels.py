@@ -856,11 +856,11 @@ ROW_TILES_BELOW = 1280
 SMALL_RESULT_ROWS, SMALL_RESULT = 5120, 21 << 18
 # Tiles of csrc/gemm_dk.hip for more than 64 rows, where K is shared out within a workgroup and nothing waits for a barrier: code ->
 # 16-row groups, 16-column groups, workgroups of a CU at a time, and us: start and end, each further round, a K-step of 64 of a round,
-# of a CU's workgroup, of a workgroup on 1/256 of the chip, a million weights. Fitted, with no cost below zero, to 338 products of 72 -
-# 1280 rows (26 projections, feed-forwards and encoder layers 320 - 16384 wide, weights cold): off by 5 - 7 % on average.
-_DK_TILES = {20: (2, 1, 2, 3.52, 1.42, 0.0, 0.037, 0.033, 0.097), 21: (2, 2, 2, 3.45, 1.12, 0.0, 0.057, 0.039, 0.174),
-             22: (4, 2, 1, 3.88, 1.78, 0.093, 0.0, 0.068, 0.056), 23: (4, 3, 1, 4.29, 2.06, 0.111, 0.0, 0.074, 0.098),
-             24: (4, 4, 1, 4.76, 2.50, 0.132, 0.0, 0.076, 0.148), 25: (4, 6, 1, 5.81, 3.40, 0.172, 0.0, 0.078, 0.202)}
+# of a CU's workgroup, of a workgroup on 1/256 of the chip, a million weights. Fitted, with no cost below zero, to 1600 products of 65 -
+# 1279 rows (256 - 12288 columns and K, bf16 and fp16, every epilogue, weights cold): off by 5 % on average (20 and 21: 9 and 8).
+_DK_TILES = {20: (2, 1, 2, 3.227, 1.608, 0.0, 0.041, 0.032, 0.03), 21: (2, 2, 2, 3.195, 1.584, 0.0, 0.066, 0.03, 0.14),
+             22: (4, 2, 1, 3.822, 2.207, 0.106, 0.0, 0.047, 0.07), 23: (4, 3, 1, 4.445, 2.823, 0.126, 0.0, 0.05, 0.132),
+             24: (4, 4, 1, 5.0, 3.36, 0.149, 0.0, 0.05, 0.174), 25: (4, 6, 1, 6.87, 5.082, 0.218, 0.0, 0.039, 0.193)}
 
 
 def _row_tiles_ok(M: int, N: int) -> bool:
@@ -917,10 +917,12 @@ def _row_tile(M: int, N: int, K: int, epi: int = EPI_NONE, f16: bool = False):
 @_rule
 def _dk_rows_tile(M: int, N: int, K: int, epi: int = EPI_NONE, f16: bool = False) -> int:
     """The tile of ``_DK_TILES`` that a product of 65 rows to ROW_TILES_BELOW runs on, 0: those of ``_row_tile`` are faster. Where the
-    estimate is 3 % below theirs, 10 % from 257 rows on, 15 % where K is above 4096 (768 x 320 x 8192 is not: 15.9 / 19.0 us): 155 of
-    the 338 products that it is fitted to, in 0.76 of their time, four of them in 1.02 - 1.03. us, tiles of ``_row_tile`` -> these: 128 x 384 x 1536 8.9 ->
+    estimate is 3 % below theirs, 10 % from 257 rows on, 15 % where K is above 4096 (768 x 320 x 8192 is not: 15.9 / 19.0 us): 1025 of
+    the 1600 products that it is fitted to, in 0.63 of their time, seven of them in 1.02 - 1.12; of 500 others 334, two in more than 1.02
+    (850 x 256 x 6656 14.2 / 16.9). us, tiles of ``_row_tile`` -> these: 128 x 384 x 1536 8.9 ->
     4.3, 256 x 768 x 768 6.6 -> 4.3, 256 x 768 x 3072 12.2 -> 7.6, 256 x 1024 x 4096 13.8 -> 8.8, 128 x 4096 x 1024 8.1 -> 6.3,
-    640 x 1024 x 1024 8.2 -> 6.9; 96 x 3072 x 3072 13.0 -> 9.6, 128 x 4096 x 4096 19.8 -> 15.8."""
+    640 x 1024 x 1024 8.2 -> 6.9; 96 x 3072 x 3072 13.0 -> 9.6, 128 x 4096 x 4096 19.8 -> 15.8; not 171 x 5920 x 2688 (18.0 / 20.6),
+    1022 x 1088 x 1216 (10.2 / 11.7) or 1192 x 864 x 1216 (10.9 / 12.6)."""
     if not 64 < M < ROW_TILES_BELOW:
         return 0
     best, ksteps = None, K // 64

@@ -84,3 +84,11 @@ def test_rule(M, N, Kd, epi, want):
     """None up to 64 rows, from 1280 on, and where the other tiles are faster."""
     assert K._dk_rows_tile(M, N, Kd, epi) == want
     assert all(x >= 0 for t in K._DK_TILES.values() for x in t)
+
+
+@pytest.mark.parametrize("M,N,Kd,epi,f16", [(171, 5920, 2688, K.EPI_SWIGLU, False), (140, 5888, 2432, K.EPI_BIAS, False), (255, 4800, 576, K.EPI_NONE, False),
+                                            (777, 1344, 2240, K.EPI_GELU, False), (1022, 1088, 1216, K.EPI_BIAS, False),
+                                            (1192, 864, 1216, K.EPI_GELU, True), (494, 2152, 2112, K.EPI_GELU, True), (210, 4336, 832, K.EPI_RESID, True)])
+def test_rule_keeps_what_is_faster_elsewhere(M, N, Kd, epi, f16):
+    """Products that took 1.05 - 1.3 times as long on the widest tile as on the streaming ones."""
+    assert K._dk_rows_tile(M, N, Kd, epi, f16) == 0
