@@ -753,7 +753,7 @@ static int launch_ws_tile(const GemmArgs& a, int epi, int splits, const WsNorm& 
 // way, and the wider tile then moves less of A: 64 x 8192 x 4096 22.8 us at four splits vs 24.0 at two of 64 x 64. Splits are
 // short, and eight waves fill and drain faster: with the reduce, 64 x 4096 x 4096 14.4 us vs 15.8 with four (8 splits), x 14336
 // 28.5 / 30.2, 64 x 6144 x 4096 18.2 / 18.9 (4); unsplit 64 x 28672 x 4096 42.9 / 40.3.
-// Up to 32 rows only those of more than 16384 columns come here (kernels.py, _dk_streams).
+// Up to 32 rows only products of more than 16384 columns come here (kernels.py, _dk_streams).
 // W is read once where there is one row block only: not worth a place in the caches then.
 static int launch_ws(const GemmArgs& a, int epi, int splits, const WsNorm& nrm, hipStream_t s) {
   if (a.M <= 32 && splits == 1 && a.N > 16384) return launch_ws_tile<32, 128, 1, 4, true>(a, epi, splits, nrm, s);

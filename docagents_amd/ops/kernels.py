@@ -431,9 +431,18 @@ def dk_wide(M: int, N: int, K: int, lda: int) -> bool:
 
 
 def _dk_streams(M: int, N: int, K: int, lda: int) -> bool:
-    """More than 16 rows of more than 16384 columns: the streaming tiles share a stage of A among the waves (28672 x 4096, 32
-    rows: 40.6 us, 41.2 on gemm_dk; 16 rows: 40.4 and 38.5; 16384 x 3072, 32 rows: 19.7 and 19.0)."""
-    return M > 16 and N > 16384 and dk_wide(M, N, K, lda)
+    """Products of more than 16384 columns on the streaming tiles of 128. More than 16 rows: the waves share a stage of A (28672 x 4096,
+    32 rows: 40.6 us, 41.2 on gemm_dk; 16384 x 3072, 32 rows: 19.7 and 19.0). Of fewer where one tile a CU covers the columns in a round
+    that is at most 7/8 full (gemm_dk's second workgroup of a CU then has nothing beside it), or where most of two rounds is, and
+    short products of many. us, streaming / gemm_dk: 17920 x 5120 37 / 41, 16416 x 2048 16.7 / 18.3, 25344 x 6912 56 / 59, 28672 x 2048
+    21.7 / 22.8, 4096 36.9 / 36.8, 50304 x 2048 35.6 / 40.8, 65472 x 512 14.2 / 15.2, 150688 x 768 37.3 / 40.3; not 30976 x 256 (7.5 / 7.1),
+    32064 x 3072 (32.3 / 31.2), 41504 x 3584 (57.8 / 48.0), 70464 x 1280 (38.4 / 34.0) or 128256 x 4096 (153 / 149). Of 303 such
+    products the slower one is taken by more than 3 % at four, by 6 % at most (64064 x 2048)."""
+    if N <= 16384 or not dk_wide(M, N, K, lda):
+        return False
+    if M > 16 or N <= 28672:
+        return M > 16 or 32 * K > N
+    return N > 49152 and (N <= 61440 or K <= (1024 if N > 81920 else 512))
 
 
 def _dk_whole(M: int, N: int, K: int) -> bool:

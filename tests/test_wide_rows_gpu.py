@@ -1,4 +1,4 @@
-"""Wide products of up to 32 rows on the streaming tiles: every epilogue, the rows' norm over few and many parts, ragged edges."""
+"""Wide products of up to 32 rows, on gemm_dk's tiles and on the streaming ones: every epilogue, the rows' norm over few and many parts, ragged edges."""
 import pytest
 import torch
 
@@ -8,13 +8,29 @@ if torch.cuda.is_available():
     from docagents_amd.ops import kernels as K
 
 
-# either side of 16384 columns (64- and 128-wide tiles), one stage and more than the ring holds, parts of the norm past the
+# gemm_dk's tiles of 64 columns (the fourth and the last: the streaming ones), one stage and more than the ring holds, parts of the norm past the
 # 256 that are added up at once
 @pytest.mark.parametrize("M,N,Kd,parts", [(2, 8192 + 16, 256, 1), (17, 8192 + 48, 1024, 300), (32, 16384, 256, 256), (31, 16384 + 32, 768, 511),
                                           (5, 128 * 257, 256, 33), (16, 28672, 1280, 8)])
 @pytest.mark.parametrize("epi", ["none", "bias", "swiglu", "reglu", "resid"])
 @pytest.mark.parametrize("norm", [False, True])
 def test_wide(M, N, Kd, parts, epi, norm):
+    wide(M, N, Kd, parts, epi, norm)
+
+
+# every range that the rule takes to the 128-wide streaming tile: one and most of two rounds of tiles, many of a short K; one
+# stage and more than the ring holds, the first and last row count, columns past a tile
+@pytest.mark.parametrize("M,N,Kd,parts", [(17, 16384 + 16, 256, 1), (32, 128 * 257, 256, 256), (24, 16384 + 128, 1536, 300), (1, 16384 + 16, 768, 5),
+                                          (2, 16384 + 16, 768, 511), (16, 28672, 1280, 8), (9, 49152 + 16, 256, 3), (16, 61440, 512, 33),
+                                          (3, 65536 + 48, 512, 7), (5, 81920 + 16, 1024, 2)])
+@pytest.mark.parametrize("epi", ["none", "bias", "swiglu", "reglu", "resid"])
+@pytest.mark.parametrize("norm", [False, True])
+def test_streaming(M, N, Kd, parts, epi, norm):
+    assert K._dk_streams(M, -(-N // 32) * 32 if epi in ("swiglu", "reglu") else N, Kd, Kd + 64)
+    wide(M, N, Kd, parts, epi, norm)
+
+
+def wide(M, N, Kd, parts, epi, norm):
     if epi in ("swiglu", "reglu"):
         N = -(-N // 32) * 32
     if epi == "resid" and norm:
