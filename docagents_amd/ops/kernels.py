@@ -445,11 +445,15 @@ def _dk_streams(M: int, N: int, K: int, lda: int) -> bool:
     return N > 49152 and (N <= 61440 or K <= (1024 if N > 81920 else 512))
 
 
-def _dk_whole(M: int, N: int, K: int) -> bool:
+def _dk_whole(M: int, N: int, K: int, epi: int = EPI_NONE, norm: bool = False) -> bool:
     """33..64 rows that one gemm_dk launch runs faster than streaming tiles (with split-K and a reduce up to 8192 columns): up to
     16384 columns while K is short, as a workgroup reads all of A. us at 48 / 64 rows, tiles -> gemm_dk: 6144 x 4096
     17.1 / 18.5 -> 15.2 / 16.7, 8192 x 4096 20.2 / 21.7 -> 16.2 / 17.7, 9216 x 3072 21.4 / 21.6 -> 16.4 / 18.1, 12608 x 4096
-    25.1 / 26.7 -> 22.6 / 24.8; 3072 x 8192 17.5 / 19.0 -> 19.5 / 21.9."""
+    25.1 / 26.7 -> 22.6 / 24.8; 3072 x 8192 17.5 / 19.0 -> 19.5 / 21.9. Not 1024 columns and fewer of many rows and a K that eight
+    splits and more share (few workgroups walk all of it): 64 x 128 x 4096 9.2 -> 11.6, 58 x 768 x 4096 10.5 -> 12.0, 56 x 288 x 3584
+    10.0 -> 11.1; but 36 x 288 x 3840 10.1 -> 10.0, 57 x 256 x 3328 (four splits) 12.7 -> 10.7. The norm's row sums cost the reduce more."""
+    if N <= 1024 and epi not in GATED and M * K > (235_000 if norm else 160_000) and _dk_splits(N, K) >= 8:
+        return False
     return N <= 16384 and K <= 4096
 
 
@@ -531,7 +535,7 @@ def gemm_dk(a, w, epi: int = EPI_NONE, bias=None, resid=None, out=None, norm_in=
                                        ldr, M, N, K, epi, _ptr(ssq), parts, K, float(eps), None, None, 1, _stream()), "gemm_dk_wide")
         return out
     far = max(K, a.stride(0)) >= 1 << 22  # rows too long for 32-bit offsets within a tile: the reduce carries the epilogue
-    if (_dk_splitk(M, N) and ssq_out is not None) or (ssq_out is None and (far or (M > DK_SPLITK_ABOVE and not _dk_whole(M, N, K)))):
+    if (_dk_splitk(M, N) and ssq_out is not None) or (ssq_out is None and (far or (M > DK_SPLITK_ABOVE and not _dk_whole(M, N, K, epi, ssq is not None)))):
         splits = _dk_splits(N, K, ssq_out is not None or far)
         ws = _workspace(splits * M * N * 4, a.device) if splits > 1 else None
         _check(lib().da_gemm_dk_splitk(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid),
