@@ -707,8 +707,10 @@ def encoder_layers(x, layers, cu_seqlens, max_seqlen: int, heads: int, head_dim:
     f16, q8 = x.dtype == torch.float16, xq is not None
     (_f16_cuda if f16 else _bf16_cuda)(x, "x")
     _i32(cu_seqlens, "cu_seqlens")
+    if not layers:
+        return x
     T, h = x.shape
-    ffn = layers[0]["w1"].shape[0] if layers else 0
+    ffn = layers[0]["w1"].shape[0]
     _req(T > 64 and x.is_contiguous() and x.data_ptr() % 16 == 0, "x [T, hidden], contiguous")
     _req(h == heads * head_dim and head_dim in ((64, 96) if f16 else (32, 64, 96, 128)), f"head dim {head_dim} unsupported")
     _req(h % (128 if q8 else 64) == 0 and ffn % 64 == 0 and (not f16 or min(h, ffn) >= 128), f"hidden {h}, feed-forward {ffn}")

@@ -27,6 +27,18 @@ def test_layers_are_the_operations(hidden, heads, ffn, dtype, rows, monkeypatch)
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp8"])
+def test_no_layers(dtype, monkeypatch):
+    """Embeddings alone are the result, as for the few rows of a question."""
+    cfg = EncoderConfig(name="layers", vocab=500, hidden=384, layers=0, heads=6, ffn=1536, max_pos=512)
+    enc = BertEncoder(cfg, seed=2, dtype=dtype)
+    ids = torch.arange(80, dtype=torch.int32).cuda()
+    cu = torch.tensor([0, 80], dtype=torch.int32).cuda()
+    got = enc.forward(ids, ids, cu, 80)
+    monkeypatch.setattr(enc.ops, "encoder_layers_fit", lambda n: False)
+    assert torch.equal(got, enc.forward(ids, ids, cu, 80))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp8"])
 def test_memory_of_long_batches(dtype, monkeypatch):
     """A long batch's layers hold no more at a time than the operations do one by one."""
     rows = 20000
