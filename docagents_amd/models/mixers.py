@@ -247,7 +247,7 @@ class DeltaMixer:
     def __call__(self, h, m: SeqBatch, st: dict, partial=True):
         o, s, C = self.ops, self.s, self.C
         y = self.proj(h)
-        if self.one_step and m.max_len == 1:
+        if m.max_len == 1 and 0 < m.T <= self.one_step:
             r = o.delta_step(y, self.conv_w, st["conv"], (self.decay_w, self.dt_bias, self.rate, self.at_decay),
                              (self.gate.w, self.at_gate), self.at_beta, st["delta"], m, s.dim ** -0.5, self.UNIT_EPS,
                              norm=(self.norm, s.vdim, self.eps))

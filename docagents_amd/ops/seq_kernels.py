@@ -404,11 +404,18 @@ def delta_rule(qkv, decay, beta, state, conv_x, conv_state, m: SeqBatch, H: int,
     return o
 
 
-def delta_step_fits(act, H: int, G: int, Kd: int, V: int, taps: int, ra: int, rg: int) -> bool:
-    """Whether ``delta_step`` takes a layer's sizes. Heads that share keys are refused: each key head's convolution state
-    has one workgroup that reads and replaces it."""
-    return (act == torch.bfloat16 and H == G and Kd in (32, 64, 96, 128) and V <= 128 and V % 16 == 0 and 2 <= taps <= 4
-            and ra % 32 == 0 and rg % 32 == 0)
+def delta_step_fits(act, H: int, G: int, Kd: int, V: int, taps: int, ra: int, rg: int) -> int:
+    """The most rows for which ``delta_step`` takes a layer's sizes, 0: for none. Heads that share keys are refused: each key head's
+    convolution state has one workgroup that reads and replaces it.
+    Every row's workgroup reads its head's decay and gate weights: where they are more than the state, up to 128 MB of them in all.
+    us, one launch / the ops of their own: 32 heads of 128 x 128, ranks of 128 (65 KB of weights, 64 of state) 64 rows 50 / 62, 300 255 /
+    274; ranks of 256 16 rows (67 MB) 18 / 25, 64 (268 MB) 64 / 60, 128 135 / 109; of 384 64 rows 79 / 63; 8 heads, 512 64 rows
+    (134 MB) 27 / 28, 128 51 / 44. Longer ranks are a chain of their own: one head, 1024, one row 20.7 / 15.4."""
+    if not (act == torch.bfloat16 and H == G and Kd in (32, 64, 96, 128) and V <= 128 and V % 16 == 0 and 2 <= taps <= 4
+            and ra % 32 == 0 and rg % 32 == 0 and max(ra, rg) <= 512):
+        return 0
+    weights, most = 2 * (Kd * ra + V * rg), 65535
+    return most if weights <= 4 * Kd * V else min(most, ((128 << 20) - 1) // (H * weights))
 
 
 def delta_step(y, conv_w, conv_state, decay, gate, at_beta: int, state, m: SeqBatch, q_scale: float, unit_eps: float, norm):

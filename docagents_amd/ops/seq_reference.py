@@ -208,8 +208,8 @@ def delta_rule(qkv, decay, beta, state, conv_x, conv_state, m: SeqBatch, H: int,
     return (y.flatten(1) * torch.sigmoid(gate.float())).to(qkv.dtype)
 
 
-def delta_step_fits(act, H: int, G: int, K: int, V: int, taps: int, ra: int, rg: int) -> bool:
-    return False
+def delta_step_fits(act, H: int, G: int, K: int, V: int, taps: int, ra: int, rg: int) -> int:
+    return 0
 
 
 def delta_step(y, conv_w, conv_state, decay, gate, at_beta: int, state, m: SeqBatch, q_scale: float, unit_eps: float, norm):
