@@ -138,6 +138,13 @@ def partials_fit(M: int, N: int, Kd: int) -> bool:
     return 1 < M <= 128 and not (M <= K.DK_SPLITK_ABOVE and Kd % 256 == 0)
 
 
+def _partials_tile(M: int, Kd: int, lda: int) -> int:
+    """65..128 rows: the 128x64 streaming tile (us of 92 rows in 4 splits, register-staged -> this: 4096 x 14336 36.4 -> 30.8, 4096 x
+    8192 21.8 -> 20.5, 4096 x 4096 13.6 -> 13.2), the register-staged one where K is shorter than the ring (126 x 2176 x 64 4.5 -> 6.5,
+    96 x 3024 x 128 4.7 -> 5.5, 115 x 1184 x 192 5.0 -> 5.7) or rows are too long for its offsets."""
+    return K._decode_tile(M) if M <= 64 else 15 if 256 <= Kd and max(Kd, lda) < 1 << 22 else 9
+
+
 def gemm_partials(a, w, own: bool = False):
     """bf16 a[M, K] @ w[N, K]^T as fp32 partials [splits, M, N] (their sum is the product), in the shared workspace:
     valid until the next product (own: in a buffer of their own)."""
@@ -146,9 +153,7 @@ def gemm_partials(a, w, own: bool = False):
     N = w.shape[0]
     _req(w.shape[1] == Kd and Kd % 64 == 0 and N % 8 == 0 and M <= 128 and w.is_contiguous() and a.stride(1) == 1
          and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0, "gemm_partials operands")
-    # 65..128 rows: the 128x64 streaming tile (us of 92 rows in 4 splits, register-staged -> this: 4096 x 14336 36.4 -> 30.8, 4096 x
-    # 8192 21.8 -> 20.5, 4096 x 4096 13.6 -> 13.2), the register-staged one where rows are too long for its offsets
-    tile = K._decode_tile(M) if M <= 64 else 15 if max(Kd, a.stride(0)) < 1 << 22 else 9
+    tile = _partials_tile(M, Kd, a.stride(0))
     splits = K._auto_splits(M, N, Kd)
     n = splits * M * N * 4
     ws = torch.empty(n, dtype=torch.uint8, device=a.device) if own else K._workspace(n, a.device)
