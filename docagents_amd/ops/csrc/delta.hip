@@ -772,8 +772,10 @@ __global__ void __launch_bounds__(64 * CG * KS, CG * KS >= 8 ? 2 : 1) delta_appl
   const DeltaArgs& a = p.a;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int K = C::K;
-  // the workgroups of a head are neighbours on one XCD: its L2 brings their fragments once
-  const int at = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+  // The workgroups of a head are neighbours on one XCD: its L2 brings their fragments once. A head with one stays on the XCD that
+  // wrote them where the heads are a multiple of 8 (moved like the others, us: 32 heads of 32 x 16, 307 tokens 25.8, 23.7 in place;
+  // 64 of 32 x 96, 1824 116.4, 113.1; 16 portions of 64 for 32 of 128 x 128 57.0, 54.8).
+  const int at = gridDim.x > 1 ? xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y) : (int)blockIdx.y;
   const int b = blockIdx.z, h = at / (int)gridDim.x, bx = at % (int)gridDim.x;
   const int t0 = a.m.cu[b], t1 = a.m.cu[b + 1];
   if (t1 - t0 < a.below) return;
