@@ -21,9 +21,10 @@
 //   5184 x 4096  13.4 / 15.8 / 18.1 -> 9.7 / 10.9 / 13.1   12608 x 4096 19.4 / 19.8 / 21.3 -> 17.9 / 18.5 / 20.7
 //   16384 x 3072 19.3 / 19.2 / 19.7 -> 17.7 / 18.1 / 19.8  28672 x 4096 40.1 / 40.4 / 40.6 -> 38.5 / 39.2 / 41.4
 //
-// Where K is a multiple of 2048 from 4096 on, the tiles of an XCD begin at K-steps of their own: all at the same columns of
+// Where K is a multiple of 2048, the tiles of an XCD begin at K-steps of their own: all at the same columns of
 // rows a multiple of 4 KB apart, they ask the same few channels at a time (8192 x 4096, 4 rows: 13.7 us without, 12.1 with;
-// 4096 x 14336: 21.8 and 20.1; K = 3072 gains nothing).
+// 4096 x 14336: 21.8 and 20.1; 2 rows, K = 2048: 4096 columns 6.4 and 5.4, 28672 22.4 and 20.0, 128256 83.5 and 74.7, of up to 2048
+// columns 1 % longer, which begin together; K = 3072 gains nothing).
 //
 // Deferred RMSNorm: the decode layer's norms ride here instead of in launches of their own. The producer of the residual
 // stream (EPI_RESID) writes, next to x, per-(workgroup, row) sums of squares of its bf16 output slice (ssq_out
@@ -108,7 +109,7 @@ gemm_dk_kernel(DkArgs p) {
   }
   const char* Wt = (const char*)p.W + (size_t)n0 * p.K * 2;
   char* ring = smem + w * ST * STAGE;
-  const int rot = nk >= 64 && nk % 32 == 0 ? (tile >> 3) * 4 % nk : 0;  // the K-step that this tile begins with
+  const int rot = nk % 32 == 0 && (nk > 32 || p.N > 2048) ? (tile >> 3) * 4 % nk : 0;  // the K-step that this tile begins with
   const int mine = max(nk - first + every - 1, 0) / every;              // of this wave
   auto issue = [&](int i, int slot) __attribute__((always_inline)) {  // (past the wave's last: no transfer)
     int step = first + i * every + rot;
