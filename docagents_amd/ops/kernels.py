@@ -433,14 +433,14 @@ def dk_wide(M: int, N: int, K: int, lda: int) -> bool:
 def _dk_streams(M: int, N: int, K: int, lda: int) -> bool:
     """Products of more than 16384 columns on the streaming tiles of 128. More than 16 rows: the waves share a stage of A (28672 x 4096,
     32 rows: 40.6 us, 41.2 on gemm_dk; 16384 x 3072, 32 rows: 19.7 and 19.0). Of fewer where one tile a CU covers the columns in a round
-    that is at most 7/8 full (gemm_dk's second workgroup of a CU then has nothing beside it), or where most of two rounds is, and
-    short products of many. us, streaming / gemm_dk: 17920 x 5120 37 / 41, 16416 x 2048 16.7 / 18.3, 25344 x 6912 56 / 59, 28672 x 2048
-    21.7 / 22.8, 4096 36.9 / 36.8, 50304 x 2048 35.6 / 40.8, 65472 x 512 14.2 / 15.2, 150688 x 768 37.3 / 40.3; not 30976 x 256 (7.5 / 7.1),
-    32064 x 3072 (32.3 / 31.2), 41504 x 3584 (57.8 / 48.0), 70464 x 1280 (38.4 / 34.0) or 128256 x 4096 (153 / 149). Of 303 such
-    products the slower one is taken by more than 3 % at four, by 6 % at most (64064 x 2048)."""
+    that is less than 7/8 full (gemm_dk's second workgroup of a CU then has nothing beside it), or where most of two rounds is, and
+    short products of many. us, streaming / gemm_dk: 17920 x 5120 37 / 41, 17600 x 6144 44 / 49, 25344 x 6912 56 / 59, 50016 x
+    4096 64 / 69, 50304 x 2048 35.3 / 36.8, 65472 x 512 14.2 / 15.2, 150688 x 768 37.3 / 40.3; not 28672 x 4096 (37.3 / 37.0), 30976 x 256
+    (7.5 / 7.1), 32064 x 3072 (32.3 / 31.2), 41504 x 3584 (57.8 / 48.0), 70464 x 1280 (38.4 / 34.0) or 128256 x 4096 (153 / 149). Of 303
+    such products it takes the slower way by more than 3 % at three, by 4.4 % at most (58688 x 2048 39.0 / 37.4)."""
     if N <= 16384 or not dk_wide(M, N, K, lda):
         return False
-    if M > 16 or N <= 28672:
+    if M > 16 or N < 28672:
         return M > 16 or 32 * K > N
     return N > 49152 and (N <= 61440 or K <= (1024 if N > 81920 else 512))
 
@@ -460,8 +460,8 @@ def _dk_whole(M: int, N: int, K: int, epi: int = EPI_NONE, norm: bool = False) -
 @_rule
 def _dk_split(M: int, N: int, K: int, epi: int):
     """(16-column groups of a tile, workgroups that share its K, bytes of their sums) of 2..32 rows on gemm_dk, zeros: K whole
-    (both measured: csrc/gemm_dk.hip). From 17 rows on where K is at least 2.5 N and 3072; of fewer rows, whose workgroups read
-    little of A, where K is at least 4 N (up to 8 rows 16 N) and 4096."""
+    (both measured: csrc/gemm_dk.hip). Columns in whole 64s, not gated. From 17 rows on up to 8192 columns where K is at least 2.5 N and
+    3072; of fewer rows, whose workgroups read little of A, up to 2048 columns where K is at least 4 N (up to 8 rows 16 N) and 4096."""
     if epi not in (EPI_NONE, EPI_BIAS, EPI_RESID) or N % 64 or not 1 < M <= 32:
         return 0, 0, 0
     if not (2 * K >= 5 * N and K >= 3072 and N <= 8192 if M > 16 else K >= (4 if M > 8 else 16) * N and K >= 4096 and N <= 2048):
@@ -969,7 +969,10 @@ def _rope_apart(M: int, N: int, K: int) -> bool:
     8192 212 -> 173, where the one kernel had two rounds of 128-row tiles and the product alone one of 256-row ones. From
     ROW_TILES_BELOW rows on where the one kernel's last round is short, which the product alone shares out: 2817 x 6144 x 4096
     158 -> 140, 3600 168 -> 160, 5400 250 -> 237, 1931 x 9216 x 3072 131 -> 127; not 2300 (128 / 131), 3600 (194 / 199) or
-    4100 x 6144 x 4096 (176 / 184). (The estimates are 5 us and 8 % off either way there.)"""
+    4100 x 6144 x 4096 (176 / 184). The estimates are 5 us and 8 % off either way there; 1 us and 5 % in favour of apart put the line
+    where it takes the slower way by more than 2 % least often: at 4 of 70 products of five projections (2235 x 9216 x 3072 115 / 123, 4142 x
+    5120 x 3072 117 / 121 and 5010 x 7680 x 5120 290 / 298 stay in one kernel, 3185 x 5120 x 3072 83 / 92 does not, whose kernel is then one
+    of 128-row tiles), at 10 without. The 19 that it takes run in 0.92 of the one kernel's time on average."""
     tiles = math.ceil(M / 256) * math.ceil(N / 256)
     if M >= ROW_TILES_BELOW:
         alone = min(_phase_us(M, N, K, EPI_NONE, t) for t in _PHASE_TILES)
