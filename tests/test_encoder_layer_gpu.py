@@ -70,5 +70,5 @@ def test_bad_weights_are_refused():
     whole = layer["wo"]
     for bad in (whole[:-8], whole.float(), whole.t()):
         layer["wo"] = bad
-        with pytest.raises(Exception):
+        with pytest.raises(ValueError, match="wo must be"):
             enc.forward(ids, ids, cu, 80)

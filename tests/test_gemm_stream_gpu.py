@@ -47,10 +47,15 @@ def test_stream_tile(M, N, Kd, splits, epi):
     assert ((got - ref).abs() <= tol).all()
 
 
-@pytest.mark.parametrize("M,N,Kd", [(33, 8192, 512), (64, 8192 + 32, 512), (40, 16384, 256), (48, 128 * 224 + 32, 256)])
+@pytest.mark.parametrize("M,N,Kd", [(33, 8192, 512), (64, 8192 + 32, 512), (40, 16384, 256), (48, 128 * 224 + 32, 256),
+                                    (33, 8192 + 16, 4352), (64, 16384, 4352), (50, 12288 + 32, 8192), (64, 16384 + 32, 512)])
 @pytest.mark.parametrize("epi", ["none", "swiglu"])
 def test_row_norm_without_splits(M, N, Kd, epi):
-    """Wide products of 33..64 rows: the rows' scale in the epilogue (no partials), either side of the rule's line."""
+    """Wide products of 33..64 rows: the rows' scale in the epilogue (no partials), of gemm_dk (the first three) and of the streaming
+    tiles of 64 and (above 16384 columns) 128."""
+    N = -(-N // 32) * 32 if epi == "swiglu" else N
+    code = K.EPI_SWIGLU if epi == "swiglu" else K.EPI_NONE
+    assert K._dk_whole(M, N, Kd, code, True) == (N <= 16384 and Kd < 4096) and (Kd < 4096 or K._dk_splits(N, Kd) == 1)
     a, w, bias, g = _operands(M, N, Kd)
     parts = 3
     ssq = torch.rand(parts, 64, device="cuda", generator=g) * Kd / parts * 2
