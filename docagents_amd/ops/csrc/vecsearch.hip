@@ -460,158 +460,6 @@ struct TopList {
   }
 };
 
-// Per-query row ranges: ranges [R, 2] (start, end) and range_off [Q + 1], or (lists [Q, probes] != null) rows
-// ranges[l] .. ranges[l + 1] of each list l that the query names (l < 0: none). rows_per_split rows of the query's concatenated ranges per
-// workgroup (grid = (splits, Q)). out [splits, Q, K], unsorted lists (topk_merge_kernel orders them).
-//
-// A half-wave owns a row (16 B per lane and load, NCH loads), four rows of it are on their way together; 64 rows
-// are scored per step and handed to wave 0, which keeps the list while the others score the next 64 (two buffers,
-// one barrier a step). Bound by the latency of a step for few rows, by HBM for many: the caller splits a query's
-// rows over as many workgroups as fill the chip (388 rows of 8 documents: one workgroup took 105 us, with one load
-// in flight and a shuffle merge of K rounds per 64 rows; 7 workgroups take 15 us. 24 queries over 8 lists of about
-// 780 rows x 768: 162 -> 41 us).
-//
-// A filter's ranges come from the host. Up to TR_TABLE numbers of them ride in the launch's arguments (range_off, then the
-// ranges; a workgroup takes them to LDS in one step); as two copies they took 3.3 us each on the device and about 15 on the
-// host. With the ids looked up by the last kernel and one pair of events a search, one query over 8 of 100000 x 768 rows'
-// documents takes 33 us, 94 before. Lists, and ranges that are on the device, have a kernel without the table (scores and merge,
-// us with it -> without: 24 queries over 8 of 512 lists of 400000 x 768 rows 68.7 -> 58.2, 8 over 16 of 256 of 200000 x 384 53 -> 45,
-// 8 ranges of 50 rows a query for 64 queries 21.9 -> 19.7).
-constexpr int TR_TABLE = 512;  // 2 of the 4 KB that a launch's arguments may have
-struct RangeTable { int v[TR_TABLE]; };
-struct NoTable { int v[1]; };
-
-template <int NCH, typename Table>
-__global__ void __launch_bounds__(256)
-topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ slots,
-                   const bf16_t* __restrict__ Qv, int Q, const int* __restrict__ ranges,
-                   const int* __restrict__ range_off, const int* __restrict__ lists, int probes,
-                   const unsigned* __restrict__ bitmap, int W, float thr,
-                   int K, int rows_per_split, float* __restrict__ out_s, int* __restrict__ out_i, int n_table,
-                   const Table table) {
-  constexpr bool TABLE = std::is_same_v<Table, RangeTable>;
-  __shared__ int st[TABLE ? TR_TABLE : 1];
-  __shared__ float sc[2][64];
-  __shared__ int sr[2][64];
-  __shared__ float cs[TL_SL];
-  __shared__ int ci[TL_SL];
-  const int split = blockIdx.x, q = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int half = lane >> 5, l32 = lane & 31;
-  TopList top;
-  top.init(cs, ci, K);  // (every wave writes the same empty list; wave 0 keeps it)
-  if constexpr (TABLE) {
-    for (int i = tid; i < n_table; i += 256) st[i] = table.v[i];
-    __syncthreads();
-    lists = nullptr;
-  }
-  const auto range = [&](int i) { return TABLE ? st[Q + 1 + i] : ranges[i]; };
-  const int nch = d / 8;  // 16-B chunks of a row; this lane has chunks l32 + 32 i
-  float qv[NCH][8];
-#pragma unroll
-  for (int i = 0; i < NCH; ++i) {
-    const int c = l32 + 32 * i;
-    u32x4_t u = *(const u32x4_t*)(Qv + (size_t)q * d + min(c, nch - 1) * 8);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) qv[i][e] = bf2f((bf16_t)((e & 1) ? (u[e >> 1] >> 16) : (u[e >> 1] & 0xffff)));
-  }
-  const int rb = TABLE ? st[q] : lists ? q * probes : range_off[q], re = TABLE ? st[q + 1] : lists ? rb + probes : range_off[q + 1];
-  DA_ASSERT(rb >= 0 && re >= rb);
-  const int pbeg = split * rows_per_split, pend = pbeg + rows_per_split;
-  __syncthreads();
-  // walk the concatenated ranges; position p counts rows across this query's ranges
-  int pos = 0, buf = 0, r0 = rb;
-  if (pbeg > 0 && re - rb > 16) {
-    // to the range that this split begins in: 64 lengths a step and their sums (one range after another, each a load of its
-    // own that the next waits for, the last of 250 splits took 0.3 us for each of 2000 ranges)
-    for (; r0 < re; r0 += 64) {
-      const int r = min(r0 + lane, re - 1), l = lists ? lists[r] : 0;
-      const bool in = r0 + lane < re && l >= 0;
-      const int at = !in ? 0 : lists ? l : 2 * r;
-      const int len = range(at + 1) - range(at);
-      int sum = in ? len : 0;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int below = __shfl_up(sum, o, 64);
-        sum += lane >= o ? below : 0;
-      }
-      const unsigned long long past = __ballot(pos + sum > pbeg);
-      if (past) {
-        const int first = __builtin_ctzll(past);
-        pos += first ? __shfl(sum, first - 1, 64) : 0;
-        r0 += first;
-        break;
-      }
-      pos += __shfl(sum, 63, 64);
-    }
-    r0 = __builtin_amdgcn_readfirstlane(r0);
-    pos = __builtin_amdgcn_readfirstlane(pos);
-  }
-  for (int r = r0; r < re; ++r) {
-    const int l = lists ? lists[r] : 0;
-    if (l < 0) continue;
-    const int s0 = range(lists ? l : 2 * r), s1 = range(lists ? l + 1 : 2 * r + 1);
-    const int len = s1 - s0;
-    const int lo = max(pbeg, pos), hi = min(pend, pos + len);
-    for (int p0 = lo; p0 < hi; p0 += 64) {
-      // 64 rows per step: 8 half-waves x 8 rows, 4 at a time
-#pragma unroll
-      for (int j0 = 0; j0 < 8; j0 += 4) {
-        const int rl = (wid * 2 + half) * 8 + j0;
-        u32x4_t u[4][NCH];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {  // rows and chunks past the end: the last one's
-          const bf16_t* xr = X + (size_t)(s0 + (min(p0 + rl + j, hi - 1) - pos)) * d;
-#pragma unroll
-          for (int i = 0; i < NCH; ++i) u[j][i] = *(const u32x4_t*)(xr + min(l32 + 32 * i, nch - 1) * 8);
-        }
-        float dot[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < NCH; ++i) {
-          const bool in = l32 + 32 * i < nch;
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const float x = bf2f((bf16_t)((e & 1) ? (u[j][i][e >> 1] >> 16) : (u[j][i][e >> 1] & 0xffff)));
-              const float t = dot[j] + qv[i][e] * x;
-              dot[j] = in ? t : dot[j];
-            }
-        }
-#pragma unroll
-        for (int o = 16; o > 0; o >>= 1)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) dot[j] += __shfl_xor(dot[j], o, 64);
-        // lane j of a half-wave hands in row j
-        const float s = (l32 == 0 ? dot[0] : l32 == 1 ? dot[1] : l32 == 2 ? dot[2] : dot[3]);
-        if (l32 < 4) {
-          const int p = p0 + rl + l32, row = s0 + (p - pos);
-          bool ok = p < hi && s >= thr && s != -INFINITY;
-          if (ok && slots) {
-            const int sl = slots[row];
-            ok = sl >= 0 && (!bitmap || ((sl >> 5) < W && ((bitmap[(size_t)q * W + (sl >> 5)] >> (sl & 31)) & 1u)));
-          }
-          sc[buf][rl + l32] = s;
-          sr[buf][rl + l32] = ok ? row : -1;
-        }
-      }
-      __syncthreads();  // this step's scores are in, and the list has taken the last step's
-      if (wid == 0) top.add(sc[buf][lane], sr[buf][lane]);
-      buf ^= 1;
-    }
-    pos += len;
-    if (pos >= pend) break;
-  }
-  if (wid == 0) {
-    wave_sync_lds();
-    if (lane < K) {
-      const size_t o = ((size_t)split * Q + q) * K + lane;
-      out_s[o] = cs[lane];
-      out_i[o] = ci[lane];
-    }
-  }
-}
-
 // Wave 0 (every wave's list is in): the lists of waves 1 .. n - 1 into its own.
 __device__ __forceinline__ void top_join(TopList& top, float (*cs)[TL_SL], int (*ci)[TL_SL], int n) {
   const int rest = (n - 1) * top.K;
@@ -655,6 +503,220 @@ __device__ __forceinline__ void top_order(const TopList& top, const TopOut& out,
   if (lane >= real && lane < K) out.put(o + lane, -INFINITY, -1);
 }
 
+// The lists [P, Q, K] of query q put together by a workgroup of n waves, each with a list in cs / ci: each wave cuts its share
+// to K, wave 0 joins what is left and orders it. Ends with the query's result written.
+template <typename S, typename I>
+__device__ __forceinline__ void top_collect(float (*cs)[TL_SL], int (*ci)[TL_SL], int n, int K, int P, int Q, int q,
+                                            const TopOut& out, S score, I row) {
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nt = n * 64, all = P * K;
+  TopList top;
+  top.init(cs[wid], ci[wid], K);
+  for (int j0 = wid * 64; j0 < all; j0 += nt * 4) {
+    float v[4];
+    int id[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {  // issued together: the lists come from all over the chip's caches
+      const int j = j0 + lane + nt * u, jc = min(j, all - 1);
+      const size_t o = ((size_t)(jc / K) * Q + q) * K + jc % K;
+      v[u] = score(o);
+      id[u] = row(o);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) top.add(v[u], j0 + lane + nt * u < all ? id[u] : -1);
+  }
+  __syncthreads();
+  if (wid) return;
+  top_join(top, cs, ci, n);
+  top_order(top, out, q);
+}
+
+// Per-query row ranges: ranges [R, 2] (start, end) and range_off [Q + 1], or (lists [Q, probes] != null) rows
+// ranges[l] .. ranges[l + 1] of each list l that the query names (l < 0: none). rows_per_split rows of the query's concatenated ranges per
+// workgroup (grid = (splits, Q)). out_s / out_i [splits, Q, K], unsorted lists (topk_merge_kernel orders them, or with counters cnt [Q], zero
+// between launches, the query's last workgroup: out).
+//
+// A half-wave owns a row (16 B per lane and load, NCH loads), four rows of it are on their way together; 64 rows
+// are scored per step and handed to wave 0, which keeps the list while the others score the next 64 (two buffers,
+// one barrier a step). Bound by the latency of a step for few rows, by HBM for many: the caller splits a query's
+// rows over as many workgroups as fill the chip (388 rows of 8 documents: one workgroup took 105 us, with one load
+// in flight and a shuffle merge of K rounds per 64 rows; 7 workgroups take 15 us. 24 queries over 8 lists of about
+// 780 rows x 768: 162 -> 41 us).
+//
+// Few rows are a chain of latencies, so a step of up to 32 rows is one round of loads, the query and the doc slots arrive with the
+// rows and not before or behind them, and (cnt) the lists meet in the query's last workgroup instead of a launch of their own,
+// which costs the host 2 us. us on the device and in all: 384 rows of 768 12.6 and 17.9 -> 10.5 and 15.8, 10 queries of 192
+// 13.9 and 17.2 -> 12.1 and 15.7, 20 rows 8.2 and 17.1 -> 5.3 and 16.0.
+//
+// A filter's ranges come from the host. Up to TR_TABLE numbers of them ride in the launch's arguments (range_off, then the
+// ranges; a workgroup takes them to LDS in one step); as two copies they took 3.3 us each on the device and about 15 on the
+// host. With the ids looked up by the last kernel and one pair of events a search, one query over 8 of 100000 x 768 rows'
+// documents takes 33 us, 94 before. Lists, and ranges that are on the device, have a kernel without the table (scores and merge,
+// us with it -> without: 24 queries over 8 of 512 lists of 400000 x 768 rows 68.7 -> 58.2, 8 over 16 of 256 of 200000 x 384 53 -> 45,
+// 8 ranges of 50 rows a query for 64 queries 21.9 -> 19.7).
+constexpr int TR_TABLE = 512;  // 2 of the 4 KB that a launch's arguments may have
+struct RangeTable { int v[TR_TABLE]; };
+struct NoTable { int v[1]; };
+
+template <int NCH, typename Table>
+__global__ void __launch_bounds__(256)
+topk_ranges_kernel(const bf16_t* __restrict__ X, int d, const int* __restrict__ slots,
+                   const bf16_t* __restrict__ Qv, int Q, const int* __restrict__ ranges,
+                   const int* __restrict__ range_off, const int* __restrict__ lists, int probes,
+                   const unsigned* __restrict__ bitmap, int W, float thr,
+                   int K, int rows_per_split, float* __restrict__ out_s, int* __restrict__ out_i, const TopOut out,
+                   int* __restrict__ cnt, int n_table, const Table table) {
+  constexpr bool TABLE = std::is_same_v<Table, RangeTable>;
+  extern __shared__ __attribute__((aligned(16))) char joined[];  // (cnt: a list of each wave, and a flag)
+  __shared__ int st[TABLE ? TR_TABLE : 1];
+  __shared__ float sc[2][64];
+  __shared__ int sr[2][64];
+  __shared__ float cs[TL_SL];
+  __shared__ int ci[TL_SL];
+  const int split = blockIdx.x, q = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int half = lane >> 5, l32 = lane & 31;
+  TopList top;
+  top.init(cs, ci, K);  // (every wave writes the same empty list; wave 0 keeps it)
+  if constexpr (TABLE) {
+    for (int i = tid; i < n_table; i += 256) st[i] = table.v[i];
+    __syncthreads();
+    lists = nullptr;
+  }
+  const auto range = [&](int i) { return TABLE ? st[Q + 1 + i] : ranges[i]; };
+  const int nch = d / 8;  // 16-B chunks of a row; this lane has chunks l32 + 32 i
+  const auto half_f = [](const u32x4_t& u, int e) { return bf2f((bf16_t)((e & 1) ? (u[e >> 1] >> 16) : (u[e >> 1] & 0xffff))); };
+  u32x4_t qu[NCH];  // (as it is: converted here, the first rows would wait for it)
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) qu[i] = *(const u32x4_t*)(Qv + (size_t)q * d + min(l32 + 32 * i, nch - 1) * 8);
+  const int rb = TABLE ? st[q] : lists ? q * probes : range_off[q], re = TABLE ? st[q + 1] : lists ? rb + probes : range_off[q + 1];
+  DA_ASSERT(rb >= 0 && re >= rb);
+  const int pbeg = split * rows_per_split, pend = pbeg + rows_per_split;
+  __syncthreads();
+  // walk the concatenated ranges; position p counts rows across this query's ranges
+  int pos = 0, buf = 0, r0 = rb;
+  if (pbeg > 0 && re - rb > 16) {
+    // to the range that this split begins in: 64 lengths a step and their sums (one range after another, each a load of its
+    // own that the next waits for, the last of 250 splits took 0.3 us for each of 2000 ranges)
+    for (; r0 < re; r0 += 64) {
+      const int r = min(r0 + lane, re - 1), l = lists ? lists[r] : 0;
+      const bool in = r0 + lane < re && l >= 0;
+      const int at = !in ? 0 : lists ? l : 2 * r;
+      const int len = range(at + 1) - range(at);
+      int sum = in ? len : 0;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int below = __shfl_up(sum, o, 64);
+        sum += lane >= o ? below : 0;
+      }
+      const unsigned long long past = __ballot(pos + sum > pbeg);
+      if (past) {
+        const int first = __builtin_ctzll(past);
+        pos += first ? __shfl(sum, first - 1, 64) : 0;
+        r0 += first;
+        break;
+      }
+      pos += __shfl(sum, 63, 64);
+    }
+    r0 = __builtin_amdgcn_readfirstlane(r0);
+    pos = __builtin_amdgcn_readfirstlane(pos);
+  }
+  for (int r = r0; r < re; ++r) {
+    const int l = lists ? lists[r] : 0;
+    if (l < 0) continue;
+    const int s0 = range(lists ? l : 2 * r), s1 = range(lists ? l + 1 : 2 * r + 1);
+    const int len = s1 - s0;
+    const int lo = max(pbeg, pos), hi = min(pend, pos + len);
+    for (int p0 = lo; p0 < hi; p0 += 64) {
+      // 64 rows per step: 8 half-waves x 8 rows, 4 at a time (up to 32 rows: 4 each, and the others none)
+      const int each = hi - p0 > 32 ? 8 : 4;
+      for (int j0 = 0; j0 < each; j0 += 4) {
+        const int rl = (wid * 2 + half) * each + j0;
+        u32x4_t u[4][NCH];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {  // rows and chunks past the end: the last one's
+          const bf16_t* xr = X + (size_t)(s0 + (min(p0 + rl + j, hi - 1) - pos)) * d;
+#pragma unroll
+          for (int i = 0; i < NCH; ++i) u[j][i] = *(const u32x4_t*)(xr + min(l32 + 32 * i, nch - 1) * 8);
+        }
+        // lane j of a half-wave hands in row j
+        const int p = p0 + rl + (l32 & 3), row = s0 + (min(p, hi - 1) - pos);
+        const int sl = slots ? slots[row] : 0;
+        float dot[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+          const bool in = l32 + 32 * i < nch;
+          float qv[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) qv[e] = half_f(qu[i], e);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float t = dot[j] + qv[e] * half_f(u[j][i], e);
+              dot[j] = in ? t : dot[j];
+            }
+        }
+#pragma unroll
+        for (int o = 16; o > 0; o >>= 1)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) dot[j] += __shfl_xor(dot[j], o, 64);
+        const float s = (l32 == 0 ? dot[0] : l32 == 1 ? dot[1] : l32 == 2 ? dot[2] : dot[3]);
+        if (l32 < 4) {
+          bool ok = p < hi && s >= thr && s != -INFINITY && sl >= 0;
+          if (ok && bitmap) ok = (sl >> 5) < W && ((bitmap[(size_t)q * W + (sl >> 5)] >> (sl & 31)) & 1u);
+          sc[buf][rl + l32] = s;
+          sr[buf][rl + l32] = ok ? row : -1;
+        }
+      }
+      if (each == 4 && tid < 32) sr[buf][32 + tid] = -1;
+      __syncthreads();  // this step's scores are in, and the list has taken the last step's
+      if (wid == 0) top.add(sc[buf][lane], sr[buf][lane]);
+      buf ^= 1;
+    }
+    pos += len;
+    if (pos >= pend) break;
+  }
+  const size_t o = ((size_t)split * Q + q) * K + lane;
+  if (!cnt) {
+    if (wid == 0) {
+      wave_sync_lds();
+      if (lane < K) {
+        out_s[o] = cs[lane];
+        out_i[o] = ci[lane];
+      }
+    }
+    return;
+  }
+  // ---- the query's last workgroup puts the lists together ----
+  if (gridDim.x == 1) {
+    if (wid == 0) {
+      wave_sync_lds();
+      top_order(top, out, q);
+    }
+    return;
+  }
+  int* last = (int*)joined;
+  float (*js)[TL_SL] = (float (*)[TL_SL])(joined + 16);
+  int (*ji)[TL_SL] = (int (*)[TL_SL])(joined + 16 + 4 * TL_SL * sizeof(float));
+  if (wid == 0) {
+    wave_sync_lds();
+    if (lane < K) {  // past the XCDs' L2s, to where all of them see it
+      __hip_atomic_store(out_s + o, cs[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(out_i + o, ci[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (lane == 0) {
+      const bool all = __hip_atomic_fetch_add(cnt + q, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+      if (all) __hip_atomic_store(cnt + q, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+      *last = all;
+    }
+  }
+  __syncthreads();
+  if (!*last) return;
+  const auto ld = [](const auto* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  top_collect(js, ji, 4, K, (int)gridDim.x, Q, q, out, [&](size_t at) { return ld(out_s + at); }, [&](size_t at) { return ld(out_i + at); });
+}
+
 // cand [P, Q, K] -> out [Q, K] sorted desc (ties: smaller row id). One workgroup per query, a wave per 64 candidates
 // up to 16 (TM_WAVES): each wave cuts its share to K, wave 0 joins the lists and orders them by counting the better
 // ones of each. Bound by the chain of cuts (about 1 us each), hence many waves: K rounds of a workgroup-wide argmax
@@ -666,27 +728,8 @@ topk_merge_kernel(const float* __restrict__ cand_s, const int* __restrict__ cand
                   const TopOut out) {
   __shared__ float cs[TM_WAVES][TL_SL];
   __shared__ int ci[TM_WAVES][TL_SL];
-  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nt = blockDim.x;
-  const int n = P * K;
-  TopList top;
-  top.init(cs[wid], ci[wid], K);
-  for (int j0 = wid * 64; j0 < n; j0 += nt * 4) {
-    float v[4];
-    int id[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {  // issued together: the lists come from all over the chip's caches
-      const int j = j0 + lane + nt * u, jc = min(j, n - 1);
-      const size_t o = ((size_t)(jc / K) * Q + q) * K + jc % K;
-      v[u] = cand_s[o];
-      id[u] = j < n ? cand_i[o] : -1;
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) top.add(v[u], id[u]);
-  }
-  __syncthreads();
-  if (wid) return;
-  top_join(top, cs, ci, nt / 64);
-  top_order(top, out, q);
+  top_collect(cs, ci, (int)blockDim.x / 64, K, P, Q, blockIdx.x, out, [&](size_t o) { return cand_s[o]; },
+              [&](size_t o) { return cand_i[o]; });
 }
 
 // The second half of a scan (see there): per query the K best of its GT groups, their rows scored again (16 rows a wave and
@@ -1026,7 +1069,7 @@ DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slot
 DA_EXPORT int da_topk_ranges(const void* X, int d, const void* slots, const void* Qv, int Q, const void* ranges,
                              const void* range_off, const void* lists, int probes, const void* bitmap, int W,
                              float thr, int K, int splits, int rows_per_split, void* ws, void* out_s, void* out,
-                             const void* ids, int n_ids, const void* host_table, int n_table, void* stream) {
+                             const void* ids, int n_ids, const void* host_table, int n_table, void* cnt, void* stream) {
   if (d % 8 || d < 8 || d > 4096 || K < 1 || K > TK_MAX || splits < 1 || rows_per_split < 1 ||
       (!range_off && !n_table && (!lists || probes < 0)) || n_table < 0 || n_table > TR_TABLE ||
       (n_table && (lists || !host_table || n_table < Q + 1)))
@@ -1036,12 +1079,15 @@ DA_EXPORT int da_topk_ranges(const void* X, int d, const void* slots, const void
   float* cs = (float*)ws;
   int* ci = (int*)(cs + (size_t)splits * Q * K);
   dim3 grid(splits, Q);
+  const TopOut result = top_out(out_s, out, ids, n_ids);
+  const size_t lds = cnt && splits > 1 ? 16 + 4 * TL_SL * 8 : 0;
   auto launch = [&](const auto& table) {
     using Table = std::decay_t<decltype(table)>;
 #define TRG(NCH)                                                                                                    \
-  topk_ranges_kernel<NCH, Table><<<grid, 256, 0, s>>>((const bf16_t*)X, d, (const int*)slots, (const bf16_t*)Qv, Q, \
-                                                      (const int*)ranges, (const int*)range_off, (const int*)lists, \
-                                                      probes, (const unsigned*)bitmap, W, thr, K, rows_per_split, cs, ci, n_table, table)
+  topk_ranges_kernel<NCH, Table><<<grid, 256, lds, s>>>((const bf16_t*)X, d, (const int*)slots, (const bf16_t*)Qv, Q,  \
+                                                        (const int*)ranges, (const int*)range_off, (const int*)lists, \
+                                                        probes, (const unsigned*)bitmap, W, thr, K, rows_per_split, cs, ci, \
+                                                        result, (int*)cnt, n_table, table)
     if (d <= 256) TRG(1);
     else if (d <= 512) TRG(2);
     else if (d <= 768) TRG(3);
@@ -1058,8 +1104,8 @@ DA_EXPORT int da_topk_ranges(const void* X, int d, const void* slots, const void
     launch(NoTable{});
   }
   int err = (int)hipGetLastError();
-  if (err) return err;
-  return topk_merge(cs, ci, splits, Q, K, top_out(out_s, out, ids, n_ids), s);
+  if (err || cnt) return err;
+  return topk_merge(cs, ci, splits, Q, K, result, s);
 }
 
 DA_EXPORT int da_topk_merge(void* cand_s, void* cand_i, int P, int Q, int K, void* out_s, void* out, const void* ids, int n_ids,

@@ -87,7 +87,7 @@ _SIGS = {
                              c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     "da_topk_ranges": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int,
                        c_float, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int,
-                       c_void_p],
+                       c_void_p, c_void_p],
     "da_topk_merge": [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     "da_gather_ids": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p],
     "da_kmeans_accum": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
@@ -267,6 +267,7 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
 # (streams run products beside each other) for the TAIL_STREAMS latest streams, and in a capture one per capture and
 # stream, cleared by a node in front of its first such product.
 TAIL_STREAMS = 32
+N_COUNTERS = 256 * 8  # of a set
 TAIL_MIN_K = 1024  # no round of a shorter product is shared (csrc/gemm8p.hip, tail_slices)
 _TAIL: dict = {}  # (device, stream) -> counters, oldest first
 _TAIL_CAPTURED: dict = {}  # (device, stream) -> (capture, counters): kept until the stream's next capture
@@ -288,18 +289,18 @@ def _gemm_tail(device, stream: int, M: int, N: int, K: int, epi: int, tile: int 
 
 
 def _counters(device, stream: int):
-    """The 256 * 8 counters, 0 between launches, of the current stream ``stream``."""
+    """The ``N_COUNTERS`` counters, 0 between launches, of the current stream ``stream``."""
     key = (device.index, stream)
     if torch.cuda.is_current_stream_capturing():
         capture = lib().da_gemm_capture_id(stream)
         had, cnt = _TAIL_CAPTURED.get(key, (0, None))
         if had != capture:
-            cnt = torch.zeros(256 * 8, dtype=torch.int32, device=device)
+            cnt = torch.zeros(N_COUNTERS, dtype=torch.int32, device=device)
             _TAIL_CAPTURED[key] = capture, cnt
         return cnt
     cnt = _TAIL.get(key)
     if cnt is None:
-        cnt = torch.zeros(256 * 8, dtype=torch.int32, device=device)
+        cnt = torch.zeros(N_COUNTERS, dtype=torch.int32, device=device)
         with _LOCK:
             cnt = _TAIL.setdefault(key, cnt)
             while len(_TAIL) > TAIL_STREAMS:
@@ -1522,8 +1523,20 @@ def topk_lists(X, Qv, lists, list_off, K: int, thr: float, mean_rows: int, max_r
 
 def _rows_per_split(rows: int, Q: int) -> int:
     """Rows of a query per workgroup of the range scan: what gives about 1024 workgroups (4 per CU: a workgroup keeps
-    48 KB of rows on their way), from one step of the kernel (64) to 512."""
-    return min(512, max(64, math.ceil(rows * Q / 1024 / 64) * 64))
+    48 KB of rows on their way), from one step of the kernel (64) to 512; half a step where there are few rows in all (us, 64 / 32: one
+    query's 384 rows of 768 12.2 / 10.5, 64 queries of 144 12.8 / 11.8; 6250 rows of 24 queries 47.4 / 62.7)."""
+    return 32 if rows * Q <= RANGE_SMALL else min(512, max(64, math.ceil(rows * Q / 1024 / 64) * 64))
+
+
+RANGE_SMALL = 10240  # rows of all queries up to which a workgroup of the range scan takes half a step
+RANGE_JOIN = 256     # candidates of a query up to which its last workgroup puts them together
+
+
+def _range_join(splits: int, Q: int, K: int) -> bool:
+    """Whether the lists of a query's workgroups meet in the same launch: its four waves take a cut each up to 256 candidates, a
+    launch's up to sixteen more of them at a time (us on the device, in the launch / after it: 60 candidates 10.5 / 10.5,
+    240 15.0 / 15.2, 405 15.0 / 13.2, 960 16.7 / 15.0; one workgroup a query 5.3 / 7.1; the host 15.8 / 17.5)."""
+    return splits * K <= RANGE_JOIN and Q <= N_COUNTERS
 
 
 def _ranges(X, Qv, ranges, range_off, lists, K, thr, max_rows, slots, bitmap, rows_per_split, ids=None, table=None):
@@ -1544,11 +1557,13 @@ def _ranges(X, Qv, ranges, range_off, lists, K, thr, max_rows, slots, bitmap, ro
         return out_s, out
     splits = max(1, math.ceil(max_rows / rows_per_split))
     ws = _call_scratch(splits * Q * K * 8, X)
+    stream = _raw_stream()
+    cnt = _counters(X.device, stream) if _range_join(splits, Q, K) else None
     _check(lib().da_topk_ranges(_ptr(X), d, _ptr(slots), _ptr(Qv), Q, _ptr(ranges), _ptr(range_off), _ptr(lists),
                                 0 if lists is None else lists.shape[1], _ptr(bitmap),
                                 W, float(thr), K, splits, rows_per_split, _ptr(ws), *args,
                                 None if table is None else table.ctypes.data, 0 if table is None else table.size,
-                                _stream()), "topk_ranges")
+                                _ptr(cnt), stream), "topk_ranges")
     return out_s, out
 
 
