@@ -742,7 +742,12 @@ topk_merge_kernel(const float* __restrict__ cand_s, const int* __restrict__ cand
 // (equal scores), the K-th best is found to its last bit by counting, a pass over the groups for each bit that is open, and its first
 // equals are taken in order. us, lists of every scan / lists of the pick's waves / this: 20000 equal rows x 384, one query, K = 20
 // 155 / 811 / 65, 600000 of 20 kinds, K = 5 181 / 488 / 163, 600000 equal, 64 queries, K = 5 187 / 792 / 187; rows that overflow are done over by the waves' lists.
-constexpr int TP_WAVES = 8, TP_CAP = 1024, TP_FOLD = 256;
+// A thread keeps its best four of groups and the largest behind it, so that nearly always one four is read again and not the
+// whole line (5 us of 34 at 40000 groups). Rows of more tiles than waves come through LDS in whole lines: as MFMA operands they are
+// requests of 64 B, 512 a tile, of which a CU has 256 on their way (24 tiles 13.6 -> 8.3 us; of up to 8 tiles the ring is 1 us
+// slower). Whole searches, us: 102624 x 768, 10 queries, K = 20 50.8 -> 45.1, 110468 x 1024, 42, K = 14 64.3 -> 60.0, 52331 x 1024,
+// one, K = 14 41.3 -> 36.3, 10000 x 768, 24, K = 5 17.1 -> 15.2, 958291 x 1024, 18, K = 12 340 -> 335; 20000 x 768, 128, K = 5 26.9 -> 27.3.
+constexpr int TP_WAVES = 8, TP_CAP = 1024, TP_FOLD = 256, TP_RING = 3;
 
 // The largest bound, to its upper 20 bits, that at least `need` of the 8 keys of each lane reach (0: there are not as many).
 __device__ __forceinline__ unsigned reached_by(const unsigned (&key)[8], int need) {
@@ -771,7 +776,9 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
   __shared__ float bound;
   __shared__ unsigned keys[nt], bkey;
   __shared__ __attribute__((aligned(16))) bf16_t sq[d];
-  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, fr = lane & 15, fg = lane >> 4;
+  extern __shared__ __attribute__((aligned(16))) char tp_tiles[];  // (groups of more than TP_WAVES tiles) [TP_WAVES][TP_RING] pieces of 16 rows x 128 columns
+  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fg = lane >> 4;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   for (int i = tid; i < d / 8; i += nt) *(u32x4_t*)(sq + i * 8) = *(const u32x4_t*)(Qv + (size_t)q * d + i * 8);
   const f32x4_t* line = (const f32x4_t*)(gm + (size_t)q * GT);
   TopList top;
@@ -792,15 +799,26 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
 
   // ---- groups ----
   const int nv = GT / 4;
-  float best = -INFINITY;
-  for (int j0 = tid; j0 < nv; j0 += nt * 4) {
-    f32x4_t v[4];
+  float best = -INFINITY, next = -INFINITY;  // of this thread's fours, by their largest: the best, and the one behind it
+  int at4 = 0;
+  auto see = [&](const f32x4_t& v, int j) __attribute__((always_inline)) {  // (a value counts for one thread only)
+    const float m = j < nv ? fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])) : -INFINITY;
+    next = fmaxf(next, fminf(m, best));
+    at4 = m > best ? j : at4;
+    best = fmaxf(best, m);
+  };
+  auto look = [&](auto ahead) __attribute__((always_inline)) {
+    constexpr int U = decltype(ahead)::value;
+    for (int j0 = tid; j0 < nv; j0 += nt * U) {
+      f32x4_t v[U];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = line[min(j0 + nt * u, nv - 1)];
+      for (int u = 0; u < U; ++u) v[u] = line[min(j0 + nt * u, nv - 1)];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)  // (a value counts for one thread only)
-      if (j0 + nt * u < nv) best = fmaxf(best, fmaxf(fmaxf(v[u][0], v[u][1]), fmaxf(v[u][2], v[u][3])));
-  }
+      for (int u = 0; u < U; ++u) see(v[u], j0 + nt * u);
+    }
+  };
+  if (nv <= 4 * nt) look(std::integral_constant<int, 4>{});
+  else look(std::integral_constant<int, 8>{});
   keys[tid] = td_key(best, best > -INFINITY ? 0 : -1);
   if (tid == 0) count = 0;
   if (tid < 32) reach[tid] = 0;
@@ -815,10 +833,13 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
   }
   __syncthreads();
   const float T = bound;
-  for (int j0 = tid; j0 < nv; j0 += nt) {
-    const f32x4_t v = line[j0];
+  if (best >= T && best > -INFINITY) {
+    const bool more = next >= T && next > -INFINITY;  // (then all of them: rarely more than the one)
+    for (int j0 = more ? tid : at4; j0 < nv; j0 += more ? nt : nv) {
+      const f32x4_t v = line[j0];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) collect(v[e], 4 * j0 + e, v[e] >= T && v[e] > -INFINITY);
+      for (int e = 0; e < 4; ++e) collect(v[e], 4 * j0 + e, v[e] >= T && v[e] > -INFINITY);
+    }
   }
   __syncthreads();
   int found = count;
@@ -902,31 +923,76 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
   // ---- their rows ----
   const float R = bound;
   top.init(cs[wid], ci[wid], K);
-  for (int again = 0; again < 2; ++again) {
-    for (int it = wid; it < K << lg; it += TP_WAVES) {
-      const int g = groups[it >> lg];
-      if (g < 0) continue;
-      const int run = g / run_slots;
-      const long first = (long)run * run_rows;
-      const int row0 = (int)first + ((((g % run_slots) << lg) + (it & ((1 << lg) - 1))) * 16);
-      const int end = (int)min((long)N, first + run_rows);
-      if (row0 >= end) continue;
-      const bf16_t* xr = X + (size_t)min(row0 + fr, end - 1) * d + fg * 8;
-      bf16x8_t a[NK];
+  char* mine = tp_tiles + wid * TP_RING * 4096;
+  unsigned off[4];  // 1 KiB instruction i: rows 4 i .. 4 i + 3, 256 B of each: chunk c of row r at c ^ r
 #pragma unroll
-      for (int kk = 0; kk < NK; ++kk) a[kk] = *(const bf16x8_t*)(xr + kk * 32);
+  for (int i = 0; i < 4; ++i) {
+    const int r = 4 * i + (lane >> 4);
+    off[i] = (unsigned)(r * d * 2 + (((lane & 15) ^ r) << 4));
+  }
+  // the wave's i-th tile: its first row, and the end of the run (0: none)
+  auto tile = [&](int i, int& row0, int& end) __attribute__((always_inline)) {
+    const int it = wid + i * TP_WAVES, g = it < K << lg ? groups[it >> lg] : -1;
+    const long first = (long)(g / run_slots) * run_rows;
+    row0 = g < 0 ? 0 : (int)first + ((((g % run_slots) << lg) + (it & ((1 << lg) - 1))) * 16);
+    end = g < 0 ? 0 : (int)min((long)N, first + run_rows);
+    row0 = __builtin_amdgcn_readfirstlane(row0);
+    end = __builtin_amdgcn_readfirstlane(end);
+  };
+  auto issue = [&](int row0, int end, int g, int slot) __attribute__((always_inline)) {  // 128 columns of a tile (rows past the end: zeros)
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)(X + (size_t)row0 * d), (short)0,
+                                                                        max(0, min(end - row0, 16)) * d * 2, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (vs_lds_t)(mine + slot * 4096 + i * 1024), 16, off[i], g * 256, 0, 0);
+  };
+  const int tiles = ((K << lg) - wid + TP_WAVES - 1) / TP_WAVES;
+  const bool one = K << lg <= TP_WAVES;
+  for (int again = 0; again < 2; ++again) {
+    int row0, end, row1 = 0, end1 = 0, slot = 0;
+    tile(0, row0, end);
+    if (!one && tiles > 0)
+#pragma unroll 1
+      for (int g = 0; g < TP_RING; ++g) issue(row0, end, g, g);
+    for (int i = 0; i < tiles; ++i) {
+      tile(i + 1, row1, end1);  // (past the last: no rows)
       // lane (fr, fg), fr < 4: row 4 fg + fr of the tile
       const int row = row0 + 4 * fg + (fr & 3);
-      const int sl = slots ? slots[min(row, end - 1)] : 0;
+      const int sl = slots && row < end ? slots[row] : 0;
       f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (one) {
+        const bf16_t* xr = X + (size_t)max(0, min(row0 + fr, end - 1)) * d + fg * 8;
+        bf16x8_t a[NK];
 #pragma unroll
-      for (int kk = 0; kk < NK; ++kk) acc = mfma16(a[kk], *(const bf16x8_t*)(sq + kk * 32 + fg * 8), acc);
+        for (int kk = 0; kk < NK; ++kk) a[kk] = *(const bf16x8_t*)(xr + kk * 32);
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk) acc = mfma16(a[kk], *(const bf16x8_t*)(sq + kk * 32 + fg * 8), acc);
+      } else {
+#pragma unroll 1
+        for (int g = 0; g < NG; ++g) {
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (TP_RING - 1)) : "memory");  // this group is in, newer ones on their way
+          __builtin_amdgcn_sched_barrier(0);
+          bf16x8_t a[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) a[j] = *(const bf16x8_t*)(mine + slot * 4096 + fr * 256 + (((4 * j + fg) ^ fr) << 4));
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          __builtin_amdgcn_sched_barrier(0);
+          const bool on = g + TP_RING >= NG;  // the next tile's
+          issue(on ? row1 : row0, on ? end1 : end, on ? g + TP_RING - NG : g + TP_RING, slot);
+          slot = slot + 1 == TP_RING ? 0 : slot + 1;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc = mfma16(a[j], *(const bf16x8_t*)(sq + (4 * g + j) * 32 + fg * 8), acc);
+        }
+      }
       const float s = fr == 0 ? acc[0] : fr == 1 ? acc[1] : fr == 2 ? acc[2] : acc[3];
       bool ok = fr < 4 && row < end && sl >= 0 && s >= thr && s > -INFINITY && s >= R;
       if (ok && bitmap) ok = (sl >> 5) < W && ((bitmap[(size_t)q * W + (sl >> 5)] >> (sl & 31)) & 1u);
       if (again) top.add(s, ok ? row : -1);
       else collect(s, row, ok);
+      row0 = row1;
+      end = end1;
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (pieces past the last tile write zeros)
     __syncthreads();
     if (again || count <= TP_CAP) {  // (no more writes to count)
       if (wid) return;
@@ -1053,7 +1119,7 @@ DA_EXPORT int da_topk_dense_stream(const void* X, int N, int d, const void* slot
       TDQ(NG, 8);                                                                                                    \
     const int err = (int)hipGetLastError();                                                                          \
     if (err) return err;                                                                                             \
-    topk_pick_kernel<NG><<<Q, 64 * TP_WAVES, 0, s>>>(gm, GT, p.run_slots, p.run_rows, p.lg, (const bf16_t*)X, N,      \
+    topk_pick_kernel<NG><<<Q, 64 * TP_WAVES, p.lg < 0 || K << p.lg <= TP_WAVES ? 0 : TP_WAVES * TP_RING * 4096, s>>>(gm, GT, p.run_slots, p.run_rows, p.lg, (const bf16_t*)X, N,      \
         (const int*)slots, (const bf16_t*)Qv, (const unsigned*)bitmap, W, thr, K, top_out(out_s, out, ids, n_ids));   \
   } while (0)
   switch (d) {
