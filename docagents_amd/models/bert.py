@@ -239,8 +239,6 @@ class BertEncoder:
         from ..ops import kernels as K
         self._g, self._gb, self._gs = {}, {}, {}
         dev = self.device
-        mode = 0 if self.cfg.pooling == "cls" else 1
-        pool = self.ops.pool_l2norm_f16 if self.fp16 else self.ops.pool_l2norm
         side = torch.cuda.Stream(device=dev)
         side.wait_stream(torch.cuda.current_stream(dev))
         Lc = self.BATCH_MAX_LEN
@@ -256,24 +254,26 @@ class BertEncoder:
         # captured (an illegal address at its next replay). The scratch is checked unchanged below.
         with torch.cuda.stream(side), K.workspace_role("enc_graph"):
             for key, T, ms, cu_l in shapes:
-                ids = torch.zeros(T, dtype=torch.int32, device=dev)
-                pos = torch.arange(T, dtype=torch.int32, device=dev) if key[0] == "one" else \
-                    torch.zeros(T, dtype=torch.int32, device=dev)
-                cu = torch.tensor(cu_l, dtype=torch.int32, device=dev)
+                # ids, (a batch's) positions and offsets beside one another: a call's input is one copy
+                one = key[0] == "one"
+                buf = torch.zeros((1 if one else 2) * T + len(cu_l), dtype=torch.int32, device=dev)
+                ids, cu = buf[:T], buf[-len(cu_l):]
+                pos = torch.arange(T, dtype=torch.int32, device=dev) if one else buf[T:2 * T]
+                cu.copy_(torch.tensor(cu_l, dtype=torch.int32))
                 for _ in range(2):  # warm: allocations and workspaces before any capture
-                    pool(self.forward(ids, pos, cu, ms), cu, mode)
-                bufs[key] = (T, ms, ids, pos, cu)
+                    self._pool(self.forward(ids, pos, cu, ms), cu)
+                bufs[key] = (T, ms, buf, ids, pos, cu)
             side.synchronize()
             ws0 = K.workspace_buffer(dev)
-            for key, (T, ms, ids, pos, cu) in sorted(bufs.items(), key=lambda kv: -kv[1][0]):
+            for key, (T, ms, buf, ids, pos, cu) in sorted(bufs.items(), key=lambda kv: -kv[1][0]):
                 g = torch.cuda.CUDAGraph()
                 # thread_local: a capture must not trip over the serving threads' own CUDA calls
                 with torch.cuda.graph(g, stream=side, capture_error_mode="thread_local"):
-                    out = pool(self.forward(ids, pos, cu, ms), cu, mode)
+                    hid = self.forward(ids, pos, cu, ms)
                 if key[0] == "one":
-                    self._g[T] = (g, ids, cu, out)
+                    self._g[T] = (g, buf, cu, hid, pos)  # (the graph reads the positions too)
                 else:
-                    batch[T] = (T, g, ids, pos, cu, out)
+                    batch[T] = (T, g, buf, cu, hid)
             self._gb = {nb: batch[T] for nb, T in self.BATCH_BUCKETS}
             self._gs = {(nb, T): batch[T] for nb, T in self.SHORT_BUCKETS}
             if K.workspace_buffer(dev) is not ws0:
@@ -303,23 +303,32 @@ class BertEncoder:
         T = next(b for b in self.GRAPH_BUCKETS if b >= L)
         if T not in self._g:
             return self.encode_packed([seq])
-        g, ids, cu, out = self._g[T]
-        host = torch.zeros(T + 2, dtype=torch.int32)
-        host[:L] = torch.tensor(seq, dtype=torch.int32)
+        g, buf, cu, hid, _ = self._g[T]
+        host = np.zeros(T + 2, dtype=np.int32)
+        host[:L] = seq
         host[T + 1] = L
-        # The graphs' static buffers (ids / cu / out and the enc_graph workspace) are shared by every
-        # caller, and callers run on streams of their own (the fast embed lane, the GPU thread).
-        # Host order is not device order: each use waits on the device for the previous use's
-        # clone (event chain) before its copies overwrite the inputs.
+        return self._replay(g, buf, host, hid, cu)
+
+    def _pool(self, hid, cu):
+        pool = self.ops.pool_l2norm_f16 if self.fp16 else self.ops.pool_l2norm
+        return pool(hid, cu, 0 if self.cfg.pooling == "cls" else 1)
+
+    def _replay(self, g, buf, host, hid, cu) -> torch.Tensor:
+        """A captured graph on the input ``host``, and the embeddings of the texts that ``cu`` bounds in its result.
+
+        The graphs' static buffers (input, hidden states and the enc_graph workspace) are shared by every caller, and callers
+        run on streams of their own (the fast embed lane, the GPU thread). Host order is not device order: each use waits on
+        the device for the previous use's pooling (event chain) before its copy overwrites the input. The input is one copy
+        from pinned memory, and the pooling, which ends in a tensor of the call's own, is launched behind the graph
+        (three copies on the device and a clone around it: a question 350 us, 343 so)."""
+        staged = torch.from_numpy(host).pin_memory()
         with self._g_lock:
             cur = torch.cuda.current_stream(self.device)
             if self._g_done is not None:
                 cur.wait_event(self._g_done)
-            dev = h2d(host.numpy(), self.device)
-            ids.copy_(dev[:T])
-            cu.copy_(dev[T:])
+            buf.copy_(staged, non_blocking=True)
             g.replay()
-            res = out.clone()
+            res = self._pool(hid, cu)
             if self._g_done is None:
                 self._g_done = torch.cuda.Event()
             self._g_done.record(cur)
@@ -341,7 +350,7 @@ class BertEncoder:
         fit += [(T, nb, self._gs[nb, T]) for nb, T in self.SHORT_BUCKETS if nb >= n and T > tot and (nb, T) in self._gs]
         if not fit:
             return None
-        T, g, ids, pos, cu, out = min(fit, key=lambda f: f[:2])[2]
+        T, g, buf, cu, hid = min(fit, key=lambda f: f[:2])[2]
         b = cu.numel() - 1
         host = np.zeros(2 * T + b + 1, dtype=np.int32)
         host[:tot] = np.fromiter((t for q in seqs for t in q), dtype=np.int32, count=tot)
@@ -350,20 +359,7 @@ class BertEncoder:
         host[T:T + tot] = np.arange(tot) - np.repeat(c[:-1], lens)
         host[2 * T:2 * T + n + 1] = c
         host[2 * T + n + 1:] = tot  # padded sequences: length 0
-        with self._g_lock:  # the same device-side ordering as encode_one (shared workspace)
-            cur = torch.cuda.current_stream(self.device)
-            if self._g_done is not None:
-                cur.wait_event(self._g_done)
-            d = h2d(host, self.device)
-            ids.copy_(d[:T])
-            pos.copy_(d[T:2 * T])
-            cu.copy_(d[2 * T:])
-            g.replay()
-            res = out[:n].clone()
-            if self._g_done is None:
-                self._g_done = torch.cuda.Event()
-            self._g_done.record(cur)
-        return res
+        return self._replay(g, buf, host, hid, cu[:n + 1])
 
     def flops_per_token(self, seqlen: int) -> float:
         c = self.cfg
