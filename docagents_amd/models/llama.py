@@ -352,14 +352,25 @@ class LlamaDecoder:
         x = o.embed(ids, self.w["embed"])
         hook = self.layer_hook
         kv_from_cache = bool(getattr(o, "flash_kv_cache_ok", lambda *_: False)(D, True))
+        # up to 64 tokens: the decode step's products, which have the norms and the rotation in them: seven launches a layer for nine,
+        # which the host takes longer for than the device (52 tokens through a 3.8B 3493 -> 2558 us, 38 through an 8B 3689 -> 3486)
+        few = self._dk_decode(x.shape[0]) and o.dk_rope_fits(x.shape[0], *self.w["layers"][0]["wqkv"].shape, x.stride(0))
+        if few:
+            parts, norm = o.dk_parts(c.hidden, x.shape[0]), None
+            sa, sb = torch.empty((2, 512 * 64), dtype=torch.float32, device=x.device)
         for li, L in enumerate(self.w["layers"]):
             if hook is not None:  # e.g. move the rest of a prefill to another (CU-masked) stream
                 hook(li)
-            h = o.rmsnorm(x, L["ln_attn"], c.eps)
-            # QKV projection + RoPE + KV-cache write in one kernel (gemm8p EPI_ROPE epilogue); where the
+            # QKV projection + RoPE + KV-cache write in one kernel (gemm8p EPI_ROPE epilogue, gemm_dk's); where the
             # attention reads its keys from the cache (Phi-3's D = 96), k / v go to the cache only
-            qkv = o.gemm_rope(h, L["wqkv"], pos, self.cos_sin, hl, kl, D, slot_tok, cache.k(li), cache.v(li),
-                              kv_out=not kv_from_cache)
+            if few:
+                h = x if li else o.rmsnorm(x, L["ln_attn"], c.eps)
+                qkv = o.gemm_dk_rope(h, L["wqkv"], pos, self.cos_sin, hl, kl, D, slot_tok, cache.k(li), cache.v(li),
+                                     norm_in=norm, kv_out=not kv_from_cache)
+            else:
+                h = o.rmsnorm(x, L["ln_attn"], c.eps)
+                qkv = o.gemm_rope(h, L["wqkv"], pos, self.cos_sin, hl, kl, D, slot_tok, cache.k(li), cache.v(li),
+                                  kv_out=not kv_from_cache)
             pre = None if prefix is None else (cache.k(li)[prefix[0]], cache.v(li)[prefix[0]], prefix[1])
             if kv_from_cache:
                 a = o.flash_attn_varlen(qkv[:, :hl * D], None, None, cu, max_seqlen, hl, kl, D, causal=True,
@@ -368,7 +379,13 @@ class LlamaDecoder:
                 a = o.flash_attn_varlen(qkv[:, :hl * D], qkv[:, hl * D:(hl + kl) * D], qkv[:, (hl + kl) * D:], cu,
                                         max_seqlen, hl, kl, D, causal=True, prefix=pre)
             del qkv, h
-            x = self._attn_out_and_mlp(L, a, x)
+            if few:
+                o.gemm_dk(a, L["wo"], epi=EPI_RESID, resid=x, out=x, ssq_out=sa)
+                g = o.gemm_dk(x, L["w_gu"], epi=EPI_SWIGLU, norm_in=(sa, parts, c.eps))
+                o.gemm_dk(g, L["w_down"], epi=EPI_RESID, resid=x, out=x, ssq_out=sb)
+                norm = (sb, parts, c.eps)
+            else:
+                x = self._attn_out_and_mlp(L, a, x)
         return self._logits(x.index_select(0, last_idx), gather=not local_logits)
 
     # ------------------------------------------------------------- decode (graph-capturable)
@@ -438,9 +455,18 @@ class LlamaDecoder:
         sa, sb = st.ssq
         parts = o.dk_parts(c.hidden, x.shape[0])
         a_in, norm = o.rmsnorm(x, layers[0]["ln_attn"], c.eps, out=st.h), None
+        D, hl, kl, cache = c.head_dim, self.hl, self.kl, self.cache
+        # GQA: the rotation and the cache write ride in the projection (MHA: in the attention kernel)
+        rotated = hl != kl and _FUSED_ROPE_DECODE and o.dk_rope_fits(x.shape[0], *layers[0]["wqkv"].shape, a_in.stride(0))
         for li, L in enumerate(layers):
-            qkv = o.gemm_dk(a_in, L["wqkv"], out=st.qkv, norm_in=norm)
-            a = self._decode_attn(qkv, li, st)
+            if rotated:
+                qkv = o.gemm_dk_rope(a_in, L["wqkv"], st.pos, self.cos_sin, hl, kl, D, st.slot, cache.k(li), cache.v(li),
+                                     norm_in=norm, out=st.qkv, kv_out=False)
+                a = o.decode_attn(qkv, cache.k(li), cache.v(li), st.lens, st.slot, hl, kl, D, max_len=cache.max_seq,
+                                  pre=st.pre, out=st.attn)
+            else:
+                qkv = o.gemm_dk(a_in, L["wqkv"], out=st.qkv, norm_in=norm)
+                a = self._decode_attn(qkv, li, st)
             o.gemm_dk(a, L["wo"], epi=EPI_RESID, resid=x, out=x, ssq_out=sa)               # x += o
             g = o.gemm_dk(x, L["w_gu"], epi=EPI_SWIGLU, norm_in=(sa, parts, c.eps))        # norm(x) -> gate/up
             o.gemm_dk(g, L["w_down"], epi=EPI_RESID, resid=x, out=x, ssq_out=sb)           # x += mlp

@@ -45,6 +45,7 @@ struct DkArgs {
   int M, N, K, lda, ldc, ldr, ssq_parts, norm_k;
   float eps;
   int relu;  // EPI_SWIGLU: the gate's activation is relu, not silu
+  RopeArgs rope;  // EPI_ROPE
 };
 
 // The values of four neighbours, as two words.
@@ -95,6 +96,25 @@ gemm_dk_kernel(DkArgs p) {
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       sq[j] = *(const f32x4_t*)(p.ssq_in + (size_t)min(tid / RQ + j * PL, p.ssq_parts - 1) * 64 + tid % RQ * 4);
+
+  // rotation: this thread's pieces of the result (their heads, positions and slots), cos and sin on their way before the ring too
+  constexpr int BNO = EPI == EPI_SWIGLU ? BN / 2 : BN;  // output columns of the tile
+  constexpr int CPR = BNO / 4;                          // 4-column pieces of a row
+  constexpr int RI = EPI == EPI_ROPE ? (BM * CPR + 64 * NW - 1) / (64 * NW) : 1;
+  [[maybe_unused]] int rpos[RI], rslot[RI];
+  [[maybe_unused]] f32x4_t rcs[RI];
+  if constexpr (EPI == EPI_ROPE) {
+#pragma unroll
+    for (int i = 0; i < RI; ++i) {
+      const int m = min((tid + i * 64 * NW) / CPR, p.M - 1);
+      rpos[i] = p.rope.pos[m];
+      rslot[i] = p.rope.slot[m];
+    }
+#pragma unroll
+    for (int i = 0; i < RI; ++i)  // (columns of v: not used)
+      rcs[i] = *(const f32x4_t*)(p.rope.cs + (size_t)min(max(rpos[i], 0), p.rope.max_seq - 1) * p.rope.D +
+                                 (n0 + (tid + i * 64 * NW) % CPR * 4) % p.rope.D);
+  }
 
   unsigned ao[8], wo[16];  // rows past the operands': past the resource's end, which reads as zero
 #pragma unroll
@@ -188,8 +208,6 @@ gemm_dk_kernel(DkArgs p) {
   if (p.ssq_in && lane < RQ) *(f32x4_t*)(sums + w * 64 + lane * 4) = ss;
   __syncthreads();
 
-  constexpr int BNO = EPI == EPI_SWIGLU ? BN / 2 : BN;  // output columns of the tile
-  constexpr int CPR = BNO / 4;                          // 4-column pieces of a row
   if constexpr (SPLIT) {  // (a thread's pieces here are its pieces below)
     static_assert(EPI != EPI_SWIGLU && !ROWS, "split");
     constexpr int IT = (BM * CPR + 64 * NW - 1) / (64 * NW);  // (threads past the last piece: that one again)
@@ -236,6 +254,40 @@ gemm_dk_kernel(DkArgs p) {
     }
   }
   static_assert(EPI != EPI_RESID || ROWS || (CPR & (CPR - 1)) == 0, "a row's pieces meet by lane exchange");
+  if constexpr (EPI == EPI_ROPE) {  // rotated as the kernel behind a product does it: the rounded values in fp32, and rounded again
+    const RopeArgs& R = p.rope;
+    const int qw = R.H * R.D, kw = R.Hkv * R.D;
+#pragma unroll
+    for (int i = 0; i < RI; ++i) {
+      const int t = tid + i * 64 * NW, m = t / CPR, c = t % CPR * 4, gn = n0 + c;
+      if (t >= BM * CPR || m >= p.M || gn >= p.N) continue;
+      float inv = 1.f;
+      if (p.ssq_in) {
+        float v = 0.f;
+#pragma unroll
+        for (int x = 0; x < NW; ++x) v += sums[x * 64 + m];
+        inv = rsqrtf(v / p.norm_k + p.eps);
+      }
+      f32x4_t v = *(const f32x4_t*)&red[0][m][c];
+#pragma unroll
+      for (int x = 1; x < NW; ++x) v += *(const f32x4_t*)&red[x][m][c];
+      u32x2_t o{T::pack2(v[0] * inv, v[1] * inv), T::pack2(v[2] * inv, v[3] * inv)};
+      const int kind = gn < qw ? 0 : gn < qw + kw ? 1 : 2, rel = gn - (kind == 0 ? 0 : kind == 1 ? qw : qw + kw);
+      if (kind < 2) {
+        const f32x4_t x = unpack4<T>(o), cs = rcs[i];
+        o = u32x2_t{T::pack2(x[0] * cs[0] - x[1] * cs[1], x[1] * cs[0] + x[0] * cs[1]),
+                    T::pack2(x[2] * cs[2] - x[3] * cs[3], x[3] * cs[2] + x[2] * cs[3])};
+      }
+      if (kind > 0) {
+        DA_ASSERT(rpos[i] >= 0 && rpos[i] < R.max_seq && rslot[i] >= 0);
+        bf16_t* cache = kind == 1 ? R.kc : R.vc;
+        *(u32x2_t*)(cache + (((size_t)rslot[i] * R.Hkv + rel / R.D) * R.max_seq + rpos[i]) * R.D + rel % R.D) = o;
+        if (!R.kv_out) continue;
+      }
+      *(u32x2_t*)(p.C + (size_t)m * p.ldc + gn) = o;
+    }
+    return;
+  }
 #pragma unroll 1
   for (int t = tid; t < BM * CPR; t += 64 * NW) {
     const int m = t / CPR, c = t % CPR * 4;
@@ -328,6 +380,10 @@ static int dk_launch1(const DkArgs& a, int epi, hipStream_t s) {
       return fn == 1   ? dk_launch3<FM, 1, EPI_RESID>(a, s)
              : fn == 2 ? dk_launch3<FM, 2, EPI_RESID>(a, s) : dk_launch3<FM, 4, EPI_RESID>(a, s);
     case EPI_SWIGLU: return fn == 2 ? dk_launch3<FM, 2, EPI_SWIGLU>(a, s) : dk_launch3<FM, 4, EPI_SWIGLU>(a, s);
+    case EPI_ROPE:
+      return fn == 1   ? dk_launch3<FM, 1, EPI_ROPE>(a, s)
+             : fn == 2 ? dk_launch3<FM, 2, EPI_ROPE>(a, s)
+             : fn == 3 ? dk_launch3<FM, 3, EPI_ROPE>(a, s) : dk_launch3<FM, 4, EPI_ROPE>(a, s);
     default: return (int)hipErrorInvalidValue;
   }
 }
@@ -379,6 +435,30 @@ DA_EXPORT int da_gemm_dk(const void* A, int lda, const void* W, void* C, int ldc
   if (M <= 32) return dk_launch1<2>(a, epi, s);
   if (M <= 48) return dk_launch1<3>(a, epi, s);
   return dk_launch1<4>(a, epi, s);
+}
+
+// The QKV projection: rows rotated by their positions (interleaved pairs), k and v to the cache (and, with kv_out, to C too).
+// ssq_in as above. A launch behind the product read the result and wrote it again, 2.8 - 5.2 us a layer; here positions, cosines and
+// sines of a thread's pieces arrive beside the weights, and the epilogue takes 0.5 - 0.7 us longer (64 x 6144 x 4096 17.3 + 4.8 -> 18.0).
+// A step of an 8B at 2 / 11 / 26 / 62 rows 3025 / 3157 / 3831 / 6027 -> 2983 / 3104 / 3791 / 5962 us.
+DA_EXPORT int da_gemm_dk_rope(const void* A, int lda, const void* W, void* C, int ldc, int M, int N, int K, const float* ssq_in,
+                             int ssq_parts, int norm_k, float eps, const void* pos, const void* slot, const void* cos_sin,
+                             void* k_cache, void* v_cache, int H, int Hkv, int D, int max_seq, int kv_out, void* stream) {
+  if (M < 1 || M > 64 || K < 64 || K % 64 || N < 16 || N % 16 || lda % 8 || ldc % 8 || D < 8 || D % 8 || N != (H + 2 * Hkv) * D ||
+      !pos || !slot || !cos_sin || !k_cache || !v_cache || max_seq < 1 || (ssq_in && (ssq_parts < 1 || norm_k < 1 || !(eps > 0.f))))
+    return (int)hipErrorInvalidValue;
+  if (2ll * ((M - 1) * (long long)lda + K) > 0x7ffff000ll || 128ll * K > 0x7ffff000ll) return (int)hipErrorInvalidValue;
+  DkArgs a{};
+  a.A = (const bf16_t*)A; a.W = (const bf16_t*)W; a.C = (bf16_t*)C;
+  a.ssq_in = ssq_in; a.ssq_parts = ssq_parts; a.norm_k = norm_k; a.eps = eps;
+  a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc;
+  a.rope = RopeArgs{(const int*)pos, (const int*)slot, (const float*)cos_sin, (bf16_t*)k_cache, (bf16_t*)v_cache, H, Hkv, D, max_seq,
+                    kv_out ? 1 : 0};
+  hipStream_t s = (hipStream_t)stream;
+  if (M <= 16) return dk_launch1<1>(a, EPI_ROPE, s);
+  if (M <= 32) return dk_launch1<2>(a, EPI_ROPE, s);
+  if (M <= 48) return dk_launch1<3>(a, EPI_ROPE, s);
+  return dk_launch1<4>(a, EPI_ROPE, s);
 }
 
 template <int FM, int FN, int ST, typename T>

@@ -64,6 +64,8 @@ _SIGS = {
     "da_malloc_uncached": [c_longlong, ctypes.POINTER(c_void_p)],
     "da_gemm_dk": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                    c_int, c_void_p, c_int, c_int, c_float, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p],
+    "da_gemm_dk_rope": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_float]
+                       + [c_void_p] * 5 + [c_int] * 5 + [c_void_p],
     "da_gemm_dk_ws": [c_int] * 3,
     "da_gemm_dk_parts": [c_int],
     "da_gemm_dk_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 7 + [c_void_p],
@@ -550,6 +552,38 @@ def gemm_dk(a, w, epi: int = EPI_NONE, bias=None, resid=None, out=None, norm_in=
     _check(lib().da_gemm_dk(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), _ptr(bias), _ptr(resid), ldr,
                             M, N, K, epi, _ptr(ssq), parts, K, float(eps), _ptr(ssq_out), fn, splits, _ptr(ws), _ptr(cnt),
                             c_void_p(stream)), "gemm_dk")
+    return out
+
+
+def dk_rope_fits(M: int, N: int, K: int, lda: int) -> bool:
+    """Whether ``gemm_dk_rope`` takes a QKV projection that gemm_dk runs as one plain launch."""
+    return (dk_fusable(M, N, K) and max(K, lda) < 1 << 22 and not _dk_streams(M, N, K, lda) and not _dk_split(M, N, K, EPI_NONE)[1]
+            and (M <= DK_SPLITK_ABOVE or _dk_whole(M, N, K, EPI_NONE, True)))
+
+
+def gemm_dk_rope(a, w, pos, cos_sin, H: int, Hkv: int, D: int, slot, k_cache, v_cache, norm_in=None, out=None, kv_out: bool = True):
+    """gemm_dk of a QKV projection with the q / k heads rotated and k / v written to the cache, in one launch (``dk_rope_fits``): the
+    same values as the product and ``rope_cache`` behind it. norm_in as gemm_dk's, kv_out as gemm_rope's."""
+    _bf16_cuda(a, "a"); _bf16_cuda(w, "w"); _i32(pos, "pos"); _i32(slot, "slot")
+    M, K = a.shape
+    N = w.shape[0]
+    _req(dk_rope_fits(M, N, K, a.stride(0)) and w.shape[1] == K and N == (H + 2 * Hkv) * D and D % 8 == 0, f"gemm_dk_rope shape M={M} N={N} K={K}")
+    _req(a.stride(1) == 1 and a.stride(0) % 8 == 0 and w.is_contiguous(), "gemm_dk_rope layout")
+    _req(a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0, "operands must be 16-B aligned")
+    _req(pos.numel() >= M and slot.numel() >= M, "pos / slot length")
+    _req(cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and cos_sin.shape[-1] == 2 and cos_sin.shape[1] == D // 2, "cos_sin")
+    _req(k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.shape == v_cache.shape
+         and k_cache.dim() == 4 and k_cache.shape[1] == Hkv and k_cache.shape[3] == D, "caches")
+    if out is None:
+        out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
+    _bf16_cuda(out, "out")
+    _req(out.shape == (M, N) and out.stride(1) == 1 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0, "bad out")
+    ssq, parts, eps = (None, 0, 0.0) if norm_in is None else norm_in
+    if ssq is not None:
+        _req(ssq.dtype == torch.float32 and ssq.is_contiguous() and ssq.numel() >= parts * 64, "bad ssq_in")
+    _check(lib().da_gemm_dk_rope(_ptr(a), a.stride(0), _ptr(w), _ptr(out), out.stride(0), M, N, K, _ptr(ssq), parts, K, float(eps),
+                                 _ptr(pos), _ptr(slot), _ptr(cos_sin), _ptr(k_cache), _ptr(v_cache), H, Hkv, D, k_cache.shape[2],
+                                 int(kv_out), _stream()), "gemm_dk_rope")
     return out
 
 

@@ -503,6 +503,16 @@ def dk_fusable(M, N, K, epi=EPI_NONE):
             and epi in (EPI_NONE, EPI_BIAS, EPI_RESID, *GATED) and (epi not in GATED or N % 32 == 0))
 
 
+def dk_rope_fits(M, N, K, lda):
+    return dk_fusable(M, N, K)
+
+
+def gemm_dk_rope(a, w, pos, cos_sin, H, Hkv, D, slot, k_cache, v_cache, norm_in=None, out=None, kv_out=True):
+    """The QKV projection of gemm_dk.hip: rotation of q / k and the cache write behind the (deferred-norm) product."""
+    qkv = gemm_dk(a, w, norm_in=norm_in, out=out)
+    return rope_cache(qkv, pos, cos_sin, H, Hkv, D, slot=slot, k_cache=k_cache, v_cache=v_cache)
+
+
 def dk_parts(N, M=0):
     """gemm_dk.hip dk_fn for EPI_RESID: row-norm partial sums written per output tile; 33..64 rows
     (the split-K route): one per 512 columns (written by the reduce launch)."""

@@ -1,0 +1,47 @@
+"""The decode-sized QKV projection with rotation and cache write inside, against the product and ``rope_cache`` behind it."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from docagents_amd.ops import kernels as K
+    from docagents_amd.ops.reference import rope_table
+
+DEV = "cuda"
+
+
+# heads of 64, 96 and 128; tiles of 16 to 64 columns, a last one that is not full, heads that end inside a tile; every row block
+@pytest.mark.parametrize("H,Hkv,D,k", [(4, 2, 64, 256), (8, 8, 96, 512), (32, 8, 128, 1024), (32, 32, 96, 768), (40, 8, 128, 512), (33, 1, 64, 256)])
+@pytest.mark.parametrize("M", [1, 2, 16, 17, 33, 48, 49, 64])
+def test_rotated_projection(H, Hkv, D, k, M):
+    g = torch.Generator(device=DEV).manual_seed(M * 7 + H)
+    N, slots, seq = (H + 2 * Hkv) * D, 5, 300
+    a = torch.randn(M, k, device=DEV, generator=g).bfloat16()
+    w = (torch.randn(N, k, device=DEV, generator=g) * k ** -0.5).bfloat16()
+    at = torch.randperm(slots * seq - 1, device=DEV, generator=g)[:M]  # (no two rows at one place)
+    at[-1] = slots * seq - 1
+    slot, pos = (at // seq).int(), (at % seq).int()
+    cs = rope_table(seq, D, 10000.0, torch.device(DEV))
+    ssq = torch.rand(3, 64, device=DEV, generator=g) * k
+    for norm in (None, (ssq, 3, 1e-5)):
+        if not K.dk_rope_fits(M, N, k, k):
+            assert M < 2  # (one row: the matrix-vector product's)
+            return
+        kc, vc = (torch.full((slots, Hkv, seq, D), 7.0, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+        want = K.gemm_dk(a, w, norm_in=norm)
+        plain = want.clone()
+        K.rope_cache(want, pos, cs, H, Hkv, D, slot=slot, k_cache=kc.clone(), v_cache=vc.clone())
+        got = K.gemm_dk_rope(a, w, pos, cs, H, Hkv, D, slot, kc, vc, norm_in=norm)
+        # the same rounded values rotated in fp32, by products contracted as the compiler likes: a rounding to bf16 apart at most
+        assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=2.0 ** -9 * float(plain.abs().max()))
+        assert float((got != want).float().mean()) < 0.01
+        assert torch.equal(got[:, (H + Hkv) * D:], plain[:, (H + Hkv) * D:])
+        for c, o in ((kc, got[:, H * D:(H + Hkv) * D]), (vc, got[:, (H + Hkv) * D:])):
+            assert torch.equal(c[slot.long(), :, pos.long()], o.reshape(-1, Hkv, D))
+        touched = torch.zeros(slots, seq, dtype=torch.bool, device=DEV)
+        touched[slot.long(), pos.long()] = True
+        assert bool((kc.transpose(1, 2)[~touched] == 7).all()) and bool((vc.transpose(1, 2)[~touched] == 7).all())
+        only_q = torch.full((M, N), 3.0, device=DEV, dtype=torch.bfloat16)
+        K.gemm_dk_rope(a, w, pos, cs, H, Hkv, D, slot, kc, vc, norm_in=norm, out=only_q, kv_out=False)
+        assert torch.equal(only_q[:, :H * D], got[:, :H * D]) and bool((only_q[:, H * D:] == 3).all())
