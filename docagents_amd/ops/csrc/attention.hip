@@ -2173,7 +2173,7 @@ static int launch_fa2(const void* q, const void* k, const void* v, int ldq, int 
 // at D = 64, profiles/r2/attn_bench_v5.txt) with the speculative softmax (654 -> 689 TF/s,
 // profiles/r3/attn_bench_spec.txt) and LDS-DMA K / V tiles when the prefix is whole 64-key tiles and
 // the operands 16-B aligned (711 TF/s); every other shape the 4-wave flash_attn_v2_kernel (8 waves
-// at D = 128: Llama-3 prefill, profiles/r2/attn_bench_v4.txt).
+// at D = 128 where fa_eight_waves).
 template <int D, bool DMA>
 static constexpr int fa_pipe_smem() {
   return 3 * ((DMA ? 64 * D * 2 : FA2Cfg<D, 4, 1>::KBUF) + FA2Cfg<D, 4, 1>::VBUF);
@@ -2194,6 +2194,17 @@ static int launch_fa_pipe(const void* q, const void* k, const void* v, int ldq, 
       (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldq, ldk, ldv, (const int*)cu_seqlens, H, Hkv, causal, sl2e,
       (bf16_t*)o, ldo, pre);
   return (int)hipGetLastError();
+}
+
+// D = 128: 256 queries a workgroup, two waves a SIMD that share the staged tiles, or 128 and one. A tile's chain (scores, exponentials,
+// sums) is what a workgroup takes its time for, so one wave a SIMD is nearly twice as fast where the chip has workgroups to spare,
+// and shorter blocks leave less behind the causal diagonal; with many blocks of long prompts the tiles' second reading
+// costs more. Both give the same bits. us, 8 waves / 4, 32 heads over 8: 139 + 138 queries behind 320 keys 21.9 / 18.6, 277 16.2 / 12.5,
+// 820 31.1 / 25.0, 1750 62.2 / 52.0, 1900 + 2000 + 1700 behind 256 171 / 161, 64 x 100 behind 256 129 / 80, 2048 70.5 / 59.6, 2560 88 / 79,
+// 2816 94 / 86; 4 x 2048 190 / 191, 3072 102 / 102, 3600 135 / 146, 8192 560 / 590, 2 x 2560 140 / 142, 6 x 3000 620 / 630.
+static bool fa_eight_waves(int max_seqlen, int H, int B) {
+  const long blocks = (long)((max_seqlen + 255) / 256) * H * B;
+  return max_seqlen > 2816 || (max_seqlen > 2048 && blocks > 400);
 }
 
 // pre_k / pre_v: shared-prefix K/V of KV head 0 in a cache slot (nullptr / pre_len 0: none),
@@ -2230,6 +2241,7 @@ DA_EXPORT int da_flash_attn_v2(const void* q, const void* k, const void* v, int 
   if (D == 64 && !causal && pre_len == 0 &&
       launch_fa_enc<BF16T>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv, sl2e, o, ldo, s))
     return (int)hipGetLastError();
-  if (D == 128) return launch_fa2<8, 1>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv, D, causal, sl2e, o, ldo, pre, s);
+  if (D == 128 && fa_eight_waves(max_seqlen, H, B))
+    return launch_fa2<8, 1>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv, D, causal, sl2e, o, ldo, pre, s);
   return launch_fa2<4, 1>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv, D, causal, sl2e, o, ldo, pre, s);
 }
