@@ -28,6 +28,46 @@ class DocEntry:
     rows: int = 0
 
 
+class _Read:
+    """``FlatIndex.reading`` as a context. (Searches of few rows wait for the host: one question over 8 documents of 100000 x 768 rows took it
+    30 us, 18 of them the launch and its arguments; with this and without arrays in between 25.)"""
+    __slots__ = ("index", "stream", "outer", "wrote")
+
+    def __init__(self, index):
+        self.index = index
+
+    def __enter__(self):
+        ix, self.stream = self.index, None
+        ix.lock.acquire()
+        try:
+            if ix.device.type != "cuda":
+                return
+            st = torch.cuda.current_stream(ix.device)
+            if st.cuda_stream == ix._read_on:  # inside a read on this stream: its wait and its event stand for both
+                return
+            if ix._write_ev is not None:
+                st.wait_event(ix._write_ev)
+            self.outer, self.wrote, ix._read_on = ix._read_on, ix._write_ev, st.cuda_stream
+            ix._reads.append(st)
+            self.stream = st
+        except BaseException:
+            ix.lock.release()
+            raise
+
+    def __exit__(self, *exc):
+        ix, st = self.index, self.stream
+        try:
+            if st is not None:
+                ix._reads.pop()
+                ix._read_on = self.outer if ix._write_ev is self.wrote else None
+                handle = st.cuda_stream
+                ev = ix._read_evs.get(handle) or torch.cuda.Event()
+                ev.record(st)
+                ix._read_evs[handle] = ev
+        finally:
+            ix.lock.release()
+
+
 class FlatIndex:
     kind = "flat"
 
@@ -85,25 +125,8 @@ class FlatIndex:
                     self._read_evs.clear()  # this write is ordered after every one of them
                     self._read_on = None    # the open read's wait was for the write before: one inside it waits by itself
 
-    @contextlib.contextmanager
     def reading(self):
-        with self.lock:
-            st = torch.cuda.current_stream(self.device) if self.device.type == "cuda" else None
-            if st is None or st.cuda_stream == self._read_on:  # inside a read on this stream: its wait and its event stand for both
-                yield
-                return
-            if self._write_ev is not None:
-                st.wait_event(self._write_ev)
-            outer, wrote, self._read_on = self._read_on, self._write_ev, st.cuda_stream
-            self._reads.append(st)
-            try:
-                yield
-            finally:
-                self._reads.pop()
-                self._read_on = outer if self._write_ev is wrote else None
-                ev = self._read_evs.get(st.cuda_stream) or torch.cuda.Event()
-                ev.record(st)
-                self._read_evs[st.cuda_stream] = ev
+        return _Read(self)
 
     # ----------------------------------------------------------------- mutation
     def _grow(self, need: int):
@@ -230,6 +253,7 @@ class FlatIndex:
 
     # ----------------------------------------------------------------- search
     def _ranges_for(self, doc_filters):
+        """(every query's row ranges, one after another, where each query's begin and end, the most rows of one)"""
         ranges, off, maxrows = [], [0], 0
         for f in doc_filters:
             tot = 0
@@ -237,10 +261,10 @@ class FlatIndex:
                 e = self.docs.get(d)
                 if e is None:
                     continue
-                for a, b in e.ranges:
-                    ranges.append((a, b))
-                    tot += b - a
-            off.append(len(ranges))
+                for r in e.ranges:
+                    ranges += r
+                    tot += r[1] - r[0]
+            off.append(len(ranges) // 2)
             maxrows = max(maxrows, tot)
         return ranges, off, maxrows
 
@@ -257,17 +281,15 @@ class FlatIndex:
         ids = self.ids_t[:self.n] if want_ids else None
         if self.n == 0 or Q == 0:
             return self._none(Q, k, want_ids)
-        X = self.X[:self.n]
         if doc_filters is None:
-            return self._dense(X, q, k, min_sim, self.slots_t[:self.n], ids=ids)
+            return self._dense(self.X[:self.n], q, k, min_sim, self.slots_t[:self.n], ids=ids)
         ranges, off, maxrows = self._ranges_for(doc_filters)
         if maxrows == 0:
             return self._none(Q, k, want_ids)
         if maxrows * Q > 4 * self.n and self.dim % 32 == 0:
             # wide filters: one MFMA dense scan + bitmap beats per-query range scans
-            return self._dense(X, q, k, min_sim, self.slots_t[:self.n], doc_filters, ids)
-        return self.ops.topk_ranges(X, q, np.asarray(ranges, dtype=np.int32).reshape(-1, 2), np.asarray(off, dtype=np.int32),
-                                    k, min_sim, max_rows=maxrows, ids=ids)
+            return self._dense(self.X[:self.n], q, k, min_sim, self.slots_t[:self.n], doc_filters, ids)
+        return self.ops.topk_ranges(self.X, q, ranges, off, k, min_sim, max_rows=maxrows, ids=ids)  # (they name rows below n only)
 
     def _none(self, Q: int, k: int, want_ids: bool):
         return (torch.full((Q, k), float("-inf"), device=self.device),

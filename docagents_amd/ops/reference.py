@@ -414,11 +414,11 @@ def topk_ranges(X, Qv, ranges, range_off, K, thr, max_rows=None, slots=None, bit
     N = X.shape[0]
     s = Qv.float() @ X.float().t()
     allowed = torch.zeros((Q, N), dtype=torch.bool, device=X.device)
-    ro = range_off.tolist()
-    rg = ranges.tolist()
+    ro = range_off if isinstance(range_off, list) else range_off.tolist()
+    rg = ranges if isinstance(ranges, list) else ranges.reshape(-1).tolist()
     for q in range(Q):
         for r in range(ro[q], ro[q + 1]):
-            a, b = rg[r]
+            a, b = rg[2 * r:2 * r + 2]
             allowed[q, a:b] = True
     valid = allowed & (s >= thr)
     if slots is not None:
