@@ -162,6 +162,9 @@ class BertEncoder:
         layers the residual is the sum y that the next norm reads, with its row statistics (only the last norm is a launch)."""
         c, o = self.cfg, self.ops
         h, nh, hd = c.hidden, c.heads, c.head_dim
+        layers = self.w["layers"]
+        if o.enc_text_fits(x.shape[0], h, c.ffn, len(layers), nh, cu_seqlens.numel() - 1, self.fp16):
+            return layernorm(o.enc_text(x, layers, cu_seqlens, nh, c.eps), layers[-1]["ln2_g"], layers[-1]["ln2_b"], c.eps)
         st1, st2 = torch.empty((2, 64, 64, 2), dtype=torch.float32, device=x.device)
         norm = None
         inside = o.attn_ln_fit(x.shape[0], h, nh, cu_seqlens.numel() - 1, self.fp16)

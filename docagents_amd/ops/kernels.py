@@ -67,6 +67,8 @@ _SIGS = {
     "da_gemm_dk_rope": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_float]
                        + [c_void_p] * 5 + [c_int] * 5 + [c_void_p],
     "da_gemm_dk_ws": [c_int] * 3,
+    "da_enc_text_ws": [c_int] * 6,
+    "da_enc_text": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p] + [c_int] * 4 + [c_float, c_float, c_int, c_void_p],
     "da_gemm_dk_parts": [c_int],
     "da_gemm_dk_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 7 + [c_void_p],
     "da_enc_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5
@@ -644,6 +646,40 @@ def gemm_ln(a, w, bias, epi: int = EPI_BIAS, norm=None, resid=None, st_out=None,
     _check(lib().da_enc_rows(_ptr(a), a.stride(0), _ptr(w), _ptr(out), N, _ptr(bias), _ptr(resid),
                             0 if resid is None else resid.stride(0), M, N, K, epi, _ptr(st), _ptr(g), _ptr(b), float(eps),
                             _ptr(st_out), f16, _stream()), "gemm_ln")
+    return out
+
+
+ENC_TEXT_MIN_LAYERS = 4  # (two take as long as launches one by one)
+
+
+def enc_text_fits(M: int, hidden: int, ffn: int, layers: int, heads: int, texts: int, f16: bool = False) -> bool:
+    """Whether ``enc_text`` takes the layers of an encoder."""
+    return (M <= 32 and ENC_TEXT_MIN_LAYERS <= layers <= 32 and hidden % 64 == 0 and ffn % 64 == 0 and ffn <= 4096
+            and attn_ln_fit(M, hidden, heads, texts, f16))
+
+
+def enc_text(x, layers, cu, heads: int, eps: float):
+    """All layers of one text of up to 32 rows in one launch (csrc/encoder_text.hip): x [M, h] -> the last layer's sum before
+    its norm. layers: dicts of wqkv, bqkv, wo, bo, ln1_g, ln1_b, w1, b1, w2, b2, ln2_g, ln2_b."""
+    f16 = x.dtype == torch.float16
+    is_cuda = _f16_cuda if f16 else _bf16_cuda
+    is_cuda(x, "x"); _i32(cu, "cu_seqlens")
+    M, h = x.shape
+    f = layers[0]["w1"].shape[0]
+    _req(enc_text_fits(M, h, f, len(layers), heads, cu.numel() - 1, f16) and x.is_contiguous() and x.data_ptr() % 16 == 0, "enc_text shape")
+    shapes = {"wqkv": (3 * h, h), "bqkv": (3 * h,), "wo": (h, h), "bo": (h,), "ln1_g": (h,), "ln1_b": (h,), "w1": (f, h), "b1": (f,),
+              "w2": (h, f), "b2": (h,), "ln2_g": (h,), "ln2_b": (h,)}
+    table = []
+    for L in layers:
+        for name, shape in shapes.items():
+            t = L[name]
+            is_cuda(t, name)
+            _req(t.shape == shape and t.is_contiguous() and t.data_ptr() % 16 == 0, f"enc_text {name}")
+            table.append(t.data_ptr())
+    ws = torch.empty(int(lib().da_enc_text_ws(M, h, f, len(layers), h // heads, f16)), dtype=torch.uint8, device=x.device)
+    out = torch.empty_like(x)
+    _check(lib().da_enc_text(_ptr(x), (c_void_p * len(table))(*table), len(layers), _ptr(out), _ptr(ws), _ptr(cu), M, h, f, h // heads,
+                             float(eps), math.log2(math.e) / math.sqrt(h // heads), f16, _stream()), "enc_text")
     return out
 
 

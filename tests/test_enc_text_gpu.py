@@ -1,0 +1,110 @@
+"""A short text's encoder layers in one launch, against 64-bit arithmetic and the launches one by one."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from docagents_amd.models.bert import BertEncoder
+from docagents_amd.models.configs import EncoderConfig
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from docagents_amd.ops import kernels as K
+
+
+def make(h, f, heads, layers, dt, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(h + f + layers + seed)
+    r = lambda *s, a=1.0: (torch.randn(*s, device="cuda", generator=g) * a).to(dt)  # noqa: E731
+    out = []
+    for _ in range(layers):
+        out.append({"wqkv": r(3 * h, h, a=1.5 * h ** -0.5), "bqkv": r(3 * h, a=0.2), "wo": r(h, h, a=h ** -0.5), "bo": r(h, a=0.2),
+                    "w1": r(f, h, a=h ** -0.5), "b1": r(f, a=0.2), "w2": r(h, f, a=f ** -0.5), "b2": r(h, a=0.2),
+                    **{f"ln{i}_{n}": (r(h, a=0.1).float() + (n == "g")).to(dt) for i in (1, 2) for n in "gb"}})
+    return out, r
+
+
+def in64(x, layers, cu, heads, eps):
+    """(the last sum in 64 bits)"""
+    x, (a, b), h = x.double(), cu, x.shape[1]
+    d = lambda t: t.double()  # noqa: E731
+    for i, L in enumerate(layers):
+        q, k, v = (t.reshape(-1, heads, h // heads).transpose(0, 1) for t in (x[a:b] @ d(L["wqkv"]).T + d(L["bqkv"])).split(h, 1))
+        p = ((q @ k.transpose(1, 2).contiguous()) * (h // heads) ** -0.5).softmax(-1)
+        o = torch.zeros_like(x)
+        o[a:b] = (p @ v).transpose(0, 1).reshape(-1, h)
+        y = F.layer_norm(x + o @ d(L["wo"]).T + d(L["bo"]), (h,), d(L["ln1_g"]), d(L["ln1_b"]), eps)
+        s = y + F.gelu(y @ d(L["w1"]).T + d(L["b1"])) @ d(L["w2"]).T + d(L["b2"])
+        x = F.layer_norm(s, (h,), d(L["ln2_g"]), d(L["ln2_b"]), eps)
+    return s
+
+
+def apart(x, layers, cu, heads, eps):
+    """(the launches one by one)"""
+    st1, st2 = torch.empty((2, 64, 64, 2), dtype=torch.float32, device="cuda")
+    norm = None
+    for L in layers:
+        qkv = K.gemm_ln(x, L["wqkv"], L["bqkv"], norm=norm)
+        y = K.gemm_ln(qkv, L["wo"], L["bo"], K.EPI_RESID, norm=norm, resid=x, st_out=st1, attn=(heads, cu))
+        norm = (st1, L["ln1_g"], L["ln1_b"], eps)
+        x = K.gemm_ln(K.gemm_ln(y, L["w1"], L["b1"], K.EPI_GELU, norm=norm), L["w2"], L["b2"], K.EPI_RESID, norm=norm, resid=y, st_out=st2)
+        norm = (st2, L["ln2_g"], L["ln2_b"], eps)
+    return x
+
+
+# one row; the edges of both row blocks; rows outside the text; units of K fewer than waves, as many, and 2 to 4 a wave; the most layers
+@pytest.mark.parametrize("M,h,f,heads,layers,cu", [
+    (1, 64, 64, 1, 4, [0, 1]), (16, 384, 1536, 12, 6, [0, 16]), (17, 384, 1536, 6, 5, [0, 17]), (32, 768, 3072, 12, 12, [0, 21]),
+    (16, 768, 3072, 12, 12, [0, 7]), (31, 1024, 4096, 16, 4, [3, 29]), (32, 1024, 4096, 32, 24, [0, 32]), (9, 832, 1088, 13, 4, [0, 9]),
+    (32, 128, 2112, 2, 32, [17, 18]), (2, 512, 4032, 8, 4, [0, 2])])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_layers(M, h, f, heads, layers, cu, dt):
+    if dt == torch.float16 and h == 32 * heads:
+        heads //= 2  # (heads of 32: bf16 only)
+    L, r = make(h, f, heads, layers, dt)
+    c = torch.tensor(cu, dtype=torch.int32, device="cuda")
+    assert K.enc_text_fits(M, h, f, layers, heads, 1, dt == torch.float16)
+    for seed in range(3):  # (new activations in the same buffers: nothing of the launch before)
+        x = r(M, h)
+        got, one = (fn(x, L, c, heads, 1e-12)[cu[0]:cu[1]].double() for fn in (K.enc_text, apart))
+        ref = in64(x, L, cu, heads, 1e-12)[cu[0]:cu[1]]
+        e, e1 = (float((t - ref).norm() / ref.norm()) for t in (got, one))
+        # the same roundings in the same places, of sums in another order: errors of one size. A layer rounds about eight
+        # times, by 2^-9 (2^-12) of values of about one each, which add as independent ones over the layers
+        u = 2.0 ** -9 if dt == torch.bfloat16 else 2.0 ** -12
+        assert e < 1.25 * e1 + u and e < 4 * (8 * layers) ** 0.5 * u, (e, e1)
+        for _ in range(10):
+            assert torch.equal(K.enc_text(x, L, c, heads, 1e-12)[cu[0]:cu[1]].double(), got)
+
+
+@pytest.mark.parametrize("T", [16, 32])
+def test_replays(T):
+    """Captured: each replay has its own input's result, with eager launches of the same stream between them."""
+    L, r = make(768, 3072, 12, 12, torch.bfloat16)
+    cu, x = torch.tensor([0, T], dtype=torch.int32, device="cuda"), r(T, 768)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        K.enc_text(x, L, cu, 12, 1e-12)
+        s.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            out = K.enc_text(x, L, cu, 12, 1e-12)
+        for _ in range(6):
+            x.copy_(r(T, 768))
+            want = K.enc_text(x, L, cu, 12, 1e-12)
+            g.replay()
+            assert torch.equal(out, want)
+            assert torch.equal(K.enc_text(x, L, cu, 12, 1e-12), want)
+
+
+def test_which_texts_take_it(monkeypatch):
+    """One text of up to 32 rows from ENC_TEXT_MIN_LAYERS layers on; others as before."""
+    calls, real = [], K.enc_text
+    monkeypatch.setattr(K, "enc_text", lambda *a: calls.append(1) or real(*a))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    for layers in (K.ENC_TEXT_MIN_LAYERS - 1, K.ENC_TEXT_MIN_LAYERS):
+        enc = BertEncoder(EncoderConfig("e", vocab=100, hidden=128, layers=layers, heads=2, ffn=256), "cuda")
+        for T, cu in ((32, [0, 32]), (33, [0, 33]), (32, [0, 16, 32])):
+            calls.clear()
+            enc.forward(i32([7] * T), i32(list(range(T))), i32(cu), T)
+            assert len(calls) == (layers >= K.ENC_TEXT_MIN_LAYERS and T == 32 and len(cu) == 2)
