@@ -336,9 +336,12 @@ topk_dense_stream_kernel(const bf16_t* __restrict__ X, int N, const int* __restr
 // query groups: the nqg groups of one row block are dispatched to one XCD back to back. A stage: 16 rows (d = 384: 32) and
 // their doc slots by LDS-DMA (16-B chunk c of row r at c ^ (r & 15): the 16 rows one ds_read_b128 lane group reads hit 16
 // distinct slots; the slots to each wave's own words), a ring of 2 - 5 stages, one barrier a stage. The queries' fragments
-// stay in registers (d / 8 of them). 1.25 M x 1024: 6.0 TB/s with 17 queries, 5.8 with 64, 5.2 with 128, where a CU's LDS reads
+// stay in registers (d / 8 of them). 1.25 M x 1024: 6.0 TB/s with 17 queries, 5.8 with 64, 5.4 with 128, where a CU's LDS reads
 // (each wave reads the whole stage) and its MFMAs take about as long as its stages; the DMA instructions spread between the
-// MFMAs, or two chains of them, were slower (594 - 622 us for 496).
+// MFMAs, two chains of them, or four waves of 32 queries each were slower (594 - 657 us for 496). A stage's transfers are asked for
+// behind its products: in front of them all waves wait for one another's requests before their first read (us, in front / behind,
+// whole searches: 1.25 M x 1024, 128 queries 497 / 478, 96 492 / 467, 64 435 / 433; 600000 x 768, 128 218 / 197, 40 175 / 172; 600000 x 384,
+// 128 140 / 134; 100000 x 1024, 100 58.6 / 55.4; 30000 x 384, 90 21.9 / 22.0).
 template <int NG, int NW>
 __global__ void __launch_bounds__(64 * NW, 2)
 topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict__ slots,
@@ -399,7 +402,6 @@ topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict_
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    issue(t + ST - 1, wr);
     const char* src = sX + rd * (STAGE + SL);
 #pragma unroll
     for (int u = 0; u < TR; ++u) {
@@ -407,6 +409,7 @@ topk_dense_mq_kernel(const bf16_t* __restrict__ X, int N, const int* __restrict_
 #pragma unroll
       for (int kk = 0; kk < NK; ++kk)
         acc = mfma16(*(const bf16x8_t*)(src + u * 16 * RB + xo[kk & 3] + (kk >> 2) * 256), bq[kk], acc);
+      if (u == TR - 1) issue(t + ST - 1, wr);  // (behind the LDS reads, which its writes would hold up, and beside the maxima)
       int sl[4] = {0, 0, 0, 0};
       if (slots) {
         const u32x4_t v = *(const u32x4_t*)(src + STAGE + w * 256 + u * 64 + fg * 16);
