@@ -2,8 +2,8 @@
 //
 // A layer is four products that wait for one another (csrc/encoder_rows.hip: QKV; attention and its output product; the
 // feed-forward's two), each of which takes 1 - 2 us of a launch of 5.5 - 7: the rest is its begin and end, and weights that are asked
-// for when it begins. Here a workgroup of 16 waves takes tasks (two strips of 16 columns of the wide products, a strip of a block of 16 rows
-// of the others), one after another, from a counter, asks for a task's weights at once, and then for its activations until they are there.
+// for when it begins. Here a workgroup of 16 waves takes tasks (16 rows of a strip of 16 columns, of two
+// or four of the wide products), one after another, from a counter, asks for a task's weights at once, and then for its activations until they are there.
 //
 // Waiting. Nobody counts what is done: the activations are their own flags. All bits of the workspace are set before the launch, a layer has a
 // place of its own in it, and every 8 B there are written once, by one store past the die's L2, never with all bits set (a NaN that would is
@@ -15,10 +15,11 @@
 //
 // Activations are in strips of 16 columns, [strip][row][16], so that a store of a task fills its lines, and MFMA operands come straight from
 // there in whole lines; V alone goes through LDS. What is left of a product is a chain: 1 us from the last store to the operand, norm 0.4,
-// MFMAs and the waves' sums 0.6 - 0.9, epilogue 0.7.
+// MFMAs and the waves' sums 0.6 - 0.9, epilogue 0.7. (A row block a task, also in the wide products: the norm of 32 rows in one took 0.4 longer.
+// Waiting for one word first, or for one of the product before, so that waits read less: 165 - 184 us for 172, 16 rows of 768 columns.)
 //
-// us, launches one by one / this, bf16: 12 layers of 384 x 1536, 16 and 32 rows 216 / 149 and 220 / 185, of 768 x 3072 255 / 173 and 274 / 220, 4 of them
-// 93.5 / 81.7 and 2 47.5 / 47.0, 24 of 1024 x 4096 667 / 393 and (fp16) 722 / 523. A question of 21 tokens, 768 columns: 343 -> 245.
+// us, launches one by one / this, bf16: 12 layers of 384 x 1536, 16 and 32 rows 215 / 140 and 219 / 149, of 768 x 3072 253 / 173 and 273 / 190, 24 of
+// 1024 x 4096 670 / 404 and 730 / 460; 4 of 768, 32 rows 93.5 / 72, 2 47.5 / 42.
 #include <cstring>
 
 #include "gemm.h"
@@ -87,18 +88,19 @@ __device__ __forceinline__ float tx_rows(float v, Op op) {
   return op(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
-template <typename T, int MB, int D>
+// MB blocks of 16 rows, heads of D, NS strips a task of the wide products.
+template <typename T, int MB, int D, int NS>
 __global__ void __launch_bounds__(64 * TX_WAVES)
 enc_text_kernel(const TextArgs p) {
-  constexpr int R = 16 * MB, NS = 2, RED = NS * R * 16;  // NS: strips of a task with all rows
+  constexpr int R = 16 * MB, RED = NS * 256 > R * 32 ? NS * 256 : R * 32;
   constexpr int SC = 16;  // loads past the L2s
   __shared__ __attribute__((aligned(16))) float red[TX_WAVES][RED];  // each wave's sums; attention: its V before
-  __shared__ float smean[R], srstd[R];
+  __shared__ float smean[16], srstd[16];
   __shared__ int snext;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = p.h, f = p.f, hs = h / 16;
-  const int per = 3 * hs / NS + hs * MB + f / (16 * NS) + hs * MB, total = per * p.layers;
-  auto tasks = [&](int phase) __attribute__((always_inline)) { return phase & 1 ? hs * MB : (phase == TX_QKV ? 3 * hs : f / 16) / NS; };
+  const int per = (3 * hs / NS + hs + f / (16 * NS) + hs) * MB, total = per * p.layers;
+  auto tasks = [&](int phase) __attribute__((always_inline)) { return MB * (phase & 1 ? hs : (phase == TX_QKV ? 3 * hs : f / 16) / NS); };
   const size_t layer_bytes = (size_t)R * 2 * (5 * h + f) + 2 * (size_t)hs * R * 8;
   const unsigned S = R * 32;
   const int first = p.cu[0], end = min(p.cu[1], p.M);
@@ -119,8 +121,8 @@ enc_text_kernel(const TextArgs p) {
         index -= tasks(e);
         phase = e + 1;
       }
-    const bool wide = !(phase & 1);  // all rows; otherwise a row block a task
-    const int strip = wide ? index * NS : index / MB, m0 = MB > 1 && !wide ? index % MB * 16 : 0;
+    const bool wide = !(phase & 1);
+    const int strip = index / MB * (wide ? NS : 1), m0 = index % MB * 16;
     int lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane));  // (addresses of every phase kept from task to task would not fit the registers)
     const int tid = w * 64 + lane, fr = lane & 15, fg = lane >> 4;
@@ -130,11 +132,11 @@ enc_text_kernel(const TextArgs p) {
     const int K = phase == TX_DOWN ? f : h, units = K / 64;
     const bool second = phase == TX_QKV || phase == TX_OUT;  // the norm before this task's operand or residual: the layer before's second
     const bf16_t *g = second ? P.g2 : L.g1, *b = second ? P.b2 : L.b1;
-    const bool own = w < (wide ? MB * NS : 1), normed = layer > 0 || phase >= TX_UP;
+    const bool own = w < (wide ? NS : 1), normed = layer > 0 || phase >= TX_UP;
     u32x2_t ob{0, 0}, og{0, 0}, obb{0, 0};
     if (own) {
       const bf16_t* bias = phase == TX_QKV ? L.bqkv : phase == TX_OUT ? L.bo : phase == TX_UP ? L.c1 : L.c2;
-      const int oc = (strip + w / MB) * 16 + 4 * (lane & 3);
+      const int oc = (strip + w) * 16 + 4 * (lane & 3);
       ob = *(const u32x2_t*)(bias + oc);
       if (!wide) {
         og = *(const u32x2_t*)(g + oc);
@@ -168,30 +170,29 @@ enc_text_kernel(const TextArgs p) {
         __builtin_amdgcn_s_sleep(1);
       }
     };
-    const int om = m0 + (tid >> 2) % R;  // the result's row of this thread, and its strip
-    const int ostrip = strip + (wide ? w / MB : 0);
+    const int om = m0 + (lane >> 2), ostrip = strip + (wide ? w : 0);  // the result's row of this thread, and its strip
     const bool out = own && om < end;
     // beside the operand: the residual, and the statistics of four of the rows that are normed here, 16 lanes each
     unsigned long long orr = 0, q[4] = {};
-    const bool stats = normed && w < R / 4;
+    const bool stats = normed && w < 4;
     auto beside = [&](const TextMat& m) __attribute__((always_inline)) {
       const auto ld = [](const void* a) { return __hip_atomic_load((const unsigned long long*)a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
       if (!wide && out) orr = ld(m.p + strip * m.strip + om * m.row + 8 * (tid & 3));
       if (stats) {
-        const float2* st = (second ? (float2*)((char*)st1 - layer_bytes) + hs * R : st1) + 4 * w + fg;
+        const float2* st = (second ? (float2*)((char*)st1 - layer_bytes) + hs * R : st1) + m0 + 4 * w + fg;
 #pragma unroll
         for (int e = 0; e < 4; ++e) q[e] = ld(st + min(fr + 16 * e, hs - 1) * R);
       }
     };
     auto missing = [&]() __attribute__((always_inline)) {
       bool no = (layer > 0 || phase == TX_DOWN) && orr == TX_EMPTY;  // (the input is there)
-      if (stats && 4 * w + fg < end) {
+      if (stats && m0 + 4 * w + fg < end) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) no |= q[e] == TX_EMPTY;
       }
       return no;
     };
-    auto sums = [&](const f32x4_t& acc, int block) __attribute__((always_inline)) { *(f32x4_t*)&red[w][(16 * block + fr) * 16 + 4 * fg] = acc; };
+    auto sums = [&](const f32x4_t& acc, int j) __attribute__((always_inline)) { if (w < units) *(f32x4_t*)&red[w][(16 * j + fr) * 16 + 4 * fg] = acc; };
     auto statistics = [&]() __attribute__((always_inline)) {
       if (!stats) return;
       float2 sq[4];
@@ -331,12 +332,10 @@ enc_text_kernel(const TextArgs p) {
         }
       sums(acc[0], 0);
     } else {
-      f32x4_t acc[NS][MB];
+      f32x4_t acc[NS];
 #pragma unroll
-      for (int j = 0; j < NS; ++j)
-#pragma unroll
-        for (int n = 0; n < MB; ++n) acc[j][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      bf16x8_t wf[NS][2] = {}, af[MB][2] = {};
+      for (int j = 0; j < NS; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      bf16x8_t wf[NS][2] = {}, af[2] = {};
       float gf[2][8] = {}, bf[2][8] = {};
       if (w < units) {
 #pragma unroll
@@ -358,45 +357,32 @@ enc_text_kernel(const TextArgs p) {
         beside(m);
         if (w >= units) return missing();
 #pragma unroll
-        for (int n = 0; n < MB; ++n)
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-            af[n][i] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rs, chunk(m, i, 16 * n + fr, 16 * n + fr < end), 4 * w * m.strip, SC));
+        for (int i = 0; i < 2; ++i)
+          af[i] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rs, chunk(m, i, m0 + fr, m0 + fr < end), 4 * w * m.strip, SC));
         bool no = missing();
-#pragma unroll
-        for (int n = 0; n < MB; ++n) no |= tx_empty(__builtin_bit_cast(u32x4_t, af[n][0])) || tx_empty(__builtin_bit_cast(u32x4_t, af[n][1]));
+        no |= tx_empty(__builtin_bit_cast(u32x4_t, af[0]));
+        no |= tx_empty(__builtin_bit_cast(u32x4_t, af[1]));
         return no && layer + phase > 0;  // (the input is there)
       });
       statistics();
       if (normed) tx_barrier();
       if (w < units) {
         if (normed) {
-          float mean[MB], rstd[MB];
+          const float mean = smean[fr], rstd = srstd[fr];
 #pragma unroll
-          for (int n = 0; n < MB; ++n) {
-            mean[n] = smean[16 * n + fr];
-            rstd[n] = srstd[16 * n + fr];
+          for (int i = 0; i < 2; ++i) {
+            const auto norm = [&](int e) __attribute__((always_inline)) { return fmaf((T::to_f((bf16_t)af[i][e]) - mean) * rstd, gf[i][e], bf[i][e]); };
+            af[i] = __builtin_bit_cast(bf16x8_t, u32x4_t{T::pack2(norm(0), norm(1)), T::pack2(norm(2), norm(3)),
+                                                         T::pack2(norm(4), norm(5)), T::pack2(norm(6), norm(7))});
           }
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int n = 0; n < MB; ++n) {
-              const auto norm = [&](int e) __attribute__((always_inline)) { return fmaf((T::to_f((bf16_t)af[n][i][e]) - mean[n]) * rstd[n], gf[i][e], bf[i][e]); };
-              af[n][i] = __builtin_bit_cast(bf16x8_t, u32x4_t{T::pack2(norm(0), norm(1)), T::pack2(norm(2), norm(3)),
-                                                              T::pack2(norm(4), norm(5)), T::pack2(norm(6), norm(7))});
-            }
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int n = 0; n < MB; ++n)
-#pragma unroll
-            for (int j = 0; j < NS; ++j) acc[j][n] = T::mma16(wf[j][i], af[n][i], acc[j][n]);
+          for (int j = 0; j < NS; ++j) acc[j] = T::mma16(wf[j][i], af[i], acc[j]);
       }
 #pragma unroll
-      for (int j = 0; j < NS; ++j)
-#pragma unroll
-        for (int n = 0; n < MB; ++n) sums(acc[j][n], j * MB + n);
+      for (int j = 0; j < NS; ++j) sums(acc[j], j);
     }
     tx_barrier();
     take(TX_WAVES - 1);
@@ -405,8 +391,15 @@ enc_text_kernel(const TextArgs p) {
     // ---- the result ----
     const float* rd = &red[0][4 * tid];
     f32x4_t v = *(const f32x4_t*)rd;
+    int u = 1;
+    for (; u + 4 < units && u + 4 < TX_WAVES; u += 5) {  // (waves past the units have no sums)
+      f32x4_t s[5];
 #pragma unroll
-    for (int u = 1; u < TX_WAVES; ++u) v += *(const f32x4_t*)(rd + u * RED);
+      for (int j = 0; j < 5; ++j) s[j] = *(const f32x4_t*)(rd + (u + j) * RED);
+#pragma unroll
+      for (int j = 0; j < 5; ++j) v += s[j];
+    }
+    for (; u < min(units, TX_WAVES); ++u) v += *(const f32x4_t*)(rd + u * RED);
     const auto val = [](const u32x2_t& o, int e) { return T::to_f((bf16_t)(e & 1 ? o[e >> 1] >> 16 : o[e >> 1] & 0xffff)); };
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] += val(ob, e);
@@ -415,7 +408,7 @@ enc_text_kernel(const TextArgs p) {
       for (int e = 0; e < 4; ++e) v[e] = gelu_erf(v[e]);
     } else if (!wide) {
       const u32x2_t rb = __builtin_bit_cast(u32x2_t, orr);
-      const float mean = smean[om], rstd = srstd[om];
+      const float mean = smean[om - m0], rstd = srstd[om - m0];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float r = val(rb, e);
@@ -467,8 +460,14 @@ DA_EXPORT int da_enc_text(const void* x, const void* const* layers, int n, void*
   a.M = M; a.h = h; a.f = f; a.layers = n; a.eps = eps; a.c = c;
   hipStream_t s = (hipStream_t)stream;
   enc_text_empty_kernel<<<512, 256, 0, s>>>((u32x4_t*)ws, bytes / 16, (u32x4_t*)out, M * h / 8);
-#define ENC_TEXT(T, DD)                                                             \
-  (M <= 16 ? enc_text_kernel<T, 1, DD><<<256, 64 * TX_WAVES, 0, s>>>(a) : enc_text_kernel<T, 2, DD><<<256, 64 * TX_WAVES, 0, s>>>(a))
+  // strips a task: four of 33 - 64 KB of activations share the block's norm and its reading, two leave fewer weights to a task (us, four / two:
+  // 32 rows of 1024 columns, 24 layers 484 / 555, of 768, 12 209 / 216, of 512, 8 126 / 121, of 384, 12 178 / 168; 16 rows of 768 198 / 173, one 191)
+#define ENC_TEXT(T, DD)                                                                     \
+  do {                                                                                      \
+    if (M <= 16) enc_text_kernel<T, 1, DD, 2><<<256, 64 * TX_WAVES, 0, s>>>(a);             \
+    else if (h <= 512) enc_text_kernel<T, 2, DD, 2><<<256, 64 * TX_WAVES, 0, s>>>(a);       \
+    else enc_text_kernel<T, 2, DD, 4><<<256, 64 * TX_WAVES, 0, s>>>(a);                     \
+  } while (0)
   if (D == 32) ENC_TEXT(BF16T, 32);
   else if (f16) ENC_TEXT(F16T, 64);
   else ENC_TEXT(BF16T, 64);
