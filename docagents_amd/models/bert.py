@@ -61,6 +61,7 @@ class BertEncoder:
         import threading
         self._g_lock = threading.Lock()  # encode_one: the captured graphs' static buffers
         self._g_done = None              # event: the last graph use's output copied out
+        self._text = None                # one short text's plan (ops.enc_text_pooled), set with the graphs
 
     def _linear(self, x, L, name, bias, epi, resid=None, xq=None):
         """fp8 path: ``xq = (q, scale)`` when the producer (a LayerNorm) already emitted the
@@ -246,7 +247,10 @@ class BertEncoder:
         side.wait_stream(torch.cuda.current_stream(dev))
         Lc = self.BATCH_MAX_LEN
         # (key, T, max_seqlen, cu): the one-sequence length buckets and the batches' row counts
-        shapes = [(("one", T), T, T, [0, T]) for T in self.GRAPH_BUCKETS]
+        c = self.cfg
+        text = [not self.fp8 and self.ops.enc_text_fits(T, c.hidden, c.ffn, len(self.w["layers"]), c.heads, 1, self.fp16) for T in self.GRAPH_BUCKETS]
+        self._text = K.TextPlan(self.w, c.heads, c.eps) if any(text) else None  # (short texts: three launches, and no graph)
+        shapes = [(("one", T), T, T, [0, T]) for T, fits in zip(self.GRAPH_BUCKETS, text) if not fits]
         most = {T: max(nb for nb, rows in (*self.BATCH_BUCKETS, *self.SHORT_BUCKETS) if rows == T) for _, T in self.BATCH_BUCKETS}
         for T, nb in most.items():
             step = min(Lc, (T - 1) // nb)
@@ -292,7 +296,7 @@ class BertEncoder:
             except Exception as e:  # noqa: BLE001 - the eager encoder still serves
                 import logging
                 logging.getLogger(__name__).warning("encoder graph capture failed, eager path: %r", e)
-                self._g, self._gb, self._gs = {}, {}, {}
+                self._g, self._gb, self._gs, self._text = {}, {}, {}, None
 
     def encode_one(self, seq: list[int]) -> torch.Tensor:
         """One token sequence -> unit-norm embedding fp32 [1, H]: a captured graph when it fits a
@@ -304,6 +308,12 @@ class BertEncoder:
         if getattr(self, "_g", None) is None:
             self.prepare_graphs()
         T = next(b for b in self.GRAPH_BUCKETS if b >= L)
+        if self._text is not None and T not in self._g and T <= 32:
+            host = np.zeros(2 * L + 2, dtype=np.int32)
+            host[:L] = seq
+            host[L:2 * L] = np.arange(L)
+            host[2 * L + 1] = L
+            return self.ops.enc_text_pooled(self._text, h2d(host, self.device), self._pool_mode)
         if T not in self._g:
             return self.encode_packed([seq])
         g, buf, cu, hid, _ = self._g[T]
@@ -312,9 +322,13 @@ class BertEncoder:
         host[T + 1] = L
         return self._replay(g, buf, host, hid, cu)
 
+    @property
+    def _pool_mode(self) -> int:
+        return 0 if self.cfg.pooling == "cls" else 1
+
     def _pool(self, hid, cu):
         pool = self.ops.pool_l2norm_f16 if self.fp16 else self.ops.pool_l2norm
-        return pool(hid, cu, 0 if self.cfg.pooling == "cls" else 1)
+        return pool(hid, cu, self._pool_mode)
 
     def _replay(self, g, buf, host, hid, cu) -> torch.Tensor:
         """A captured graph on the input ``host``, and the embeddings of the texts that ``cu`` bounds in its result.

@@ -439,6 +439,102 @@ __global__ void __launch_bounds__(256) enc_text_empty_kernel(u32x4_t* ws, long n
   for (long i = blockIdx.x * 256l + threadIdx.x; i < n_out; i += gridDim.x * 256l) out[i] = u32x4_t{0, 0, 0, 0};
 }
 
+template <typename T>
+__device__ __forceinline__ void tx_load(const bf16_t* p, float (&v)[8]) {
+  const bf16x8_t u = *(const bf16x8_t*)p;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = T::to_f((bf16_t)u[e]);
+}
+
+// LayerNorm of a row of D <= 1024 columns, a wave: lane's columns 8 (lane + 64 i) + e, as the layernorm kernel does it.
+template <typename T>
+__device__ __forceinline__ void tx_norm(float (&v)[2][8], const bf16_t* g, const bf16_t* b, int lane, int D, float eps) {
+  float s = 0.f, var = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s += (lane + 64 * i) * 8 < D ? v[i][e] : 0.f;
+  const float mean = wave_sum(s) / D;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) var += (lane + 64 * i) * 8 < D ? (v[i][e] - mean) * (v[i][e] - mean) : 0.f;
+  const float inv = rsqrtf(wave_sum(var) / D + eps);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float gv[8], bv[8];
+    const int c = min((lane + 64 * i) * 8, D - 8);
+    tx_load<T>(g + c, gv);
+    tx_load<T>(b + c, bv);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[i][e] = (v[i][e] - mean) * inv * gv[e] + bv[e];
+  }
+}
+
+// The first of three launches for a text: its embeddings (a block a row) beside the emptied workspace.
+template <typename T>
+__global__ void __launch_bounds__(256)
+enc_text_begin_kernel(const int* ids, const int* positions, const bf16_t* word, const bf16_t* pos, const bf16_t* type, const bf16_t* g,
+                      const bf16_t* b, bf16_t* x, int M, int D, float eps, u32x4_t* ws, long n) {
+  const int lane = threadIdx.x & 63, row = blockIdx.x;
+  if (row >= M) {
+    for (long i = (blockIdx.x - M) * 256l + threadIdx.x; i < n; i += (gridDim.x - M) * 256l) ws[i] = u32x4_t{~0u, ~0u, ~0u, ~0u};
+    return;
+  }
+  if (threadIdx.x >= 64) return;
+  const size_t wi = (size_t)ids[row] * D, pi = (size_t)positions[row] * D;
+  float v[2][8];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float q[8], t[8];
+    const int c = min((lane + 64 * i) * 8, D - 8);
+    tx_load<T>(word + wi + c, v[i]);
+    tx_load<T>(pos + pi + c, q);
+    tx_load<T>(type + c, t);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[i][e] = v[i][e] + q[e] + t[e];
+  }
+  tx_norm<T>(v, g, b, lane, D, eps);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if ((lane + 64 * i) * 8 < D) *(u32x4_t*)(x + (size_t)row * D + (lane + 64 * i) * 8) = u32x4_t{T::pack2(v[i][0], v[i][1]), T::pack2(v[i][2], v[i][3]),
+                                                                            T::pack2(v[i][4], v[i][5]), T::pack2(v[i][6], v[i][7])};
+}
+
+// The last one: the norm behind the layers, the pooling (mode 0: the text's first row, 1: the mean of its rows) and the unit norm, in fp32.
+template <typename T>
+__global__ void __launch_bounds__(64 * TX_WAVES)
+enc_text_end_kernel(const bf16_t* y, const bf16_t* g, const bf16_t* b, const int* cu, int M, int D, float eps, int mode, float* out) {
+  __shared__ __attribute__((aligned(16))) float part[TX_WAVES][1024];
+  __shared__ float red[16];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, first = min(max(cu[0], 0), M - 1), n = mode ? max(min(cu[1], M) - first, 1) : 1;
+  float a[2][8] = {};
+  for (int r = w; r < n; r += TX_WAVES) {
+    float v[2][8];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) tx_load<T>(y + (size_t)(first + r) * D + min((lane + 64 * i) * 8, D - 8), v[i]);
+    tx_norm<T>(v, g, b, lane, D, eps);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a[i][e] += T::to_f(T::from_f(v[i][e]));  // (rounded as the rows are)
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if ((lane + 64 * i) * 8 < D) part[w][(lane + 64 * i) * 8 + e] = a[i][e];
+  __syncthreads();
+  float v = 0.f;
+  if ((int)threadIdx.x < D) {
+#pragma unroll
+    for (int i = 0; i < TX_WAVES; ++i) v += part[i][threadIdx.x];
+    v *= 1.f / (float)n;
+  }
+  const float ss = block_sum(v * v, red), inv = ss > 0.f ? rsqrtf(ss) : 1.f;
+  if ((int)threadIdx.x < D) out[threadIdx.x] = v * inv;
+}
+
 // Bytes of da_enc_text's workspace; 0: it does not take such a text.
 DA_EXPORT long long da_enc_text_ws(int M, int h, int f, int layers, int D, int f16) {
   if (M < 1 || M > 32 || layers < 1 || layers > TX_LAYERS || h < 64 || h % 64 || h > 64 * TX_WAVES || f < 64 || f % 64 || f > 256 * TX_WAVES ||
@@ -450,16 +546,13 @@ DA_EXPORT long long da_enc_text_ws(int M, int h, int f, int layers, int D, int f
 
 // x [M, h] through the layers (pointers of TextLayer each, of the host): out [M, h] is the last layer's sum before its norm. One text, rows
 // cu[0] .. cu[1] - 1.
-DA_EXPORT int da_enc_text(const void* x, const void* const* layers, int n, void* out, void* ws, const int* cu, int M, int h, int f, int D,
-                         float eps, float c, int f16, void* stream) {
+static int enc_text(const void* x, const void* const* layers, int n, void* out, void* ws, const int* cu, int M, int h, int f, int D, float eps,
+                    float c, int f16, hipStream_t s) {
   const long long bytes = da_enc_text_ws(M, h, f, n, D, f16);
-  if (!bytes || !x || !layers || !out || !ws || !cu) return (int)hipErrorInvalidValue;
   TextArgs a{};
   std::memcpy(a.L, layers, n * sizeof(TextLayer));
   a.x = (const bf16_t*)x; a.out = (bf16_t*)out; a.ws = (char*)ws; a.ticket = (int*)((char*)ws + bytes - 256); a.cu = cu;
   a.M = M; a.h = h; a.f = f; a.layers = n; a.eps = eps; a.c = c;
-  hipStream_t s = (hipStream_t)stream;
-  enc_text_empty_kernel<<<512, 256, 0, s>>>((u32x4_t*)ws, bytes / 16, (u32x4_t*)out, M * h / 8);
   // strips a task: four of 33 - 64 KB of activations share the block's norm and its reading, two leave fewer weights to a task (us, four / two:
   // 32 rows of 1024 columns, 24 layers 484 / 555, of 768, 12 209 / 216, of 512, 8 126 / 121, of 384, 12 178 / 168; 16 rows of 768 198 / 173, one 191)
 #define ENC_TEXT(T, DD)                                                                     \
@@ -472,5 +565,32 @@ DA_EXPORT int da_enc_text(const void* x, const void* const* layers, int n, void*
   else if (f16) ENC_TEXT(F16T, 64);
   else ENC_TEXT(BF16T, 64);
 #undef ENC_TEXT
+  return (int)hipGetLastError();
+}
+
+DA_EXPORT int da_enc_text(const void* x, const void* const* layers, int n, void* out, void* ws, const int* cu, int M, int h, int f, int D,
+                         float eps, float c, int f16, void* stream) {
+  const long long bytes = da_enc_text_ws(M, h, f, n, D, f16);
+  if (!bytes || !x || !layers || !out || !ws || !cu) return (int)hipErrorInvalidValue;
+  enc_text_empty_kernel<<<512, 256, 0, (hipStream_t)stream>>>((u32x4_t*)ws, bytes / 16, (u32x4_t*)out, M * h / 8);
+  return enc_text(x, layers, n, out, ws, cu, M, h, f, D, eps, c, f16, (hipStream_t)stream);
+}
+
+// The whole encoder of such a text: ids and positions [M] to its pooled unit vector, out fp32 [h]. emb: word, position and type tables, their
+// norm's gain and shift. x, y [M, h]: scratch. Three launches behind one call want no graph, whose end the next call's
+// copy waits 18 us for, nor a text filled up to a length: a question 218 -> 200 us.
+DA_EXPORT int da_enc_text_pooled(const void* ids, const void* positions, const void* const* emb, const void* const* layers, int n, void* x, void* y,
+                                void* ws, const int* cu, int M, int h, int f, int D, float eps, float c, int mode, void* out, int f16,
+                                void* stream) {
+  const long long bytes = da_enc_text_ws(M, h, f, n, D, f16);
+  if (!bytes || !ids || !positions || !emb || !layers || !x || !y || !ws || !cu || !out) return (int)hipErrorInvalidValue;
+  hipStream_t s = (hipStream_t)stream;
+  const bf16_t *const *e = (const bf16_t* const*)emb, *const *last = (const bf16_t* const*)layers + (size_t)12 * (n - 1);
+  const auto begin = f16 ? enc_text_begin_kernel<F16T> : enc_text_begin_kernel<BF16T>;
+  begin<<<M + 512, 256, 0, s>>>((const int*)ids, (const int*)positions, e[0], e[1], e[2], e[3], e[4], (bf16_t*)x, M, h, eps, (u32x4_t*)ws, bytes / 16);
+  const int err = enc_text(x, layers, n, y, ws, cu, M, h, f, D, eps, c, f16, s);
+  if (err) return err;
+  const auto end = f16 ? enc_text_end_kernel<F16T> : enc_text_end_kernel<BF16T>;
+  end<<<1, 64 * TX_WAVES, 0, s>>>((const bf16_t*)y, last[10], last[11], cu, M, h, eps, mode, (float*)out);
   return (int)hipGetLastError();
 }

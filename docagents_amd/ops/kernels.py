@@ -68,6 +68,7 @@ _SIGS = {
                        + [c_void_p] * 5 + [c_int] * 5 + [c_void_p],
     "da_gemm_dk_ws": [c_int] * 3,
     "da_enc_text_ws": [c_int] * 6,
+    "da_enc_text_pooled": [c_void_p] * 4 + [c_int] + [c_void_p] * 4 + [c_int] * 4 + [c_float, c_float, c_int, c_void_p, c_int, c_void_p],
     "da_enc_text": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p] + [c_int] * 4 + [c_float, c_float, c_int, c_void_p],
     "da_gemm_dk_parts": [c_int],
     "da_gemm_dk_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 7 + [c_void_p],
@@ -658,15 +659,8 @@ def enc_text_fits(M: int, hidden: int, ffn: int, layers: int, heads: int, texts:
             and attn_ln_fit(M, hidden, heads, texts, f16))
 
 
-def enc_text(x, layers, cu, heads: int, eps: float):
-    """All layers of one text of up to 32 rows in one launch (csrc/encoder_text.hip): x [M, h] -> the last layer's sum before
-    its norm. layers: dicts of wqkv, bqkv, wo, bo, ln1_g, ln1_b, w1, b1, w2, b2, ln2_g, ln2_b."""
-    f16 = x.dtype == torch.float16
-    is_cuda = _f16_cuda if f16 else _bf16_cuda
-    is_cuda(x, "x"); _i32(cu, "cu_seqlens")
-    M, h = x.shape
-    f = layers[0]["w1"].shape[0]
-    _req(enc_text_fits(M, h, f, len(layers), heads, cu.numel() - 1, f16) and x.is_contiguous() and x.data_ptr() % 16 == 0, "enc_text shape")
+def _text_layers(layers, h: int, f: int, is_cuda):
+    """The layers' pointers (csrc/encoder_text.hip, TextLayer), and how many."""
     shapes = {"wqkv": (3 * h, h), "bqkv": (3 * h,), "wo": (h, h), "bo": (h,), "ln1_g": (h,), "ln1_b": (h,), "w1": (f, h), "b1": (f,),
               "w2": (h, f), "b2": (h,), "ln2_g": (h,), "ln2_b": (h,)}
     table = []
@@ -676,10 +670,55 @@ def enc_text(x, layers, cu, heads: int, eps: float):
             is_cuda(t, name)
             _req(t.shape == shape and t.is_contiguous() and t.data_ptr() % 16 == 0, f"enc_text {name}")
             table.append(t.data_ptr())
-    ws = torch.empty(int(lib().da_enc_text_ws(M, h, f, len(layers), h // heads, f16)), dtype=torch.uint8, device=x.device)
+    return (c_void_p * len(table))(*table), len(layers)
+
+
+def enc_text(x, layers, cu, heads: int, eps: float):
+    """All layers of one text of up to 32 rows in one launch (csrc/encoder_text.hip): x [M, h] -> the last layer's sum before
+    its norm (rows behind the text: zeros). layers: dicts of wqkv, bqkv, wo, bo, ln1_g, ln1_b, w1, b1, w2, b2, ln2_g, ln2_b."""
+    f16 = x.dtype == torch.float16
+    is_cuda = _f16_cuda if f16 else _bf16_cuda
+    is_cuda(x, "x"); _i32(cu, "cu_seqlens")
+    M, h = x.shape
+    f, D = layers[0]["w1"].shape[0], h // heads
+    _req(enc_text_fits(M, h, f, len(layers), heads, cu.numel() - 1, f16) and x.is_contiguous() and x.data_ptr() % 16 == 0, "enc_text shape")
+    table, n = _text_layers(layers, h, f, is_cuda)
+    ws = torch.empty(int(lib().da_enc_text_ws(M, h, f, n, D, f16)), dtype=torch.uint8, device=x.device)
     out = torch.empty_like(x)
-    _check(lib().da_enc_text(_ptr(x), (c_void_p * len(table))(*table), len(layers), _ptr(out), _ptr(ws), _ptr(cu), M, h, f, h // heads,
-                             float(eps), math.log2(math.e) / math.sqrt(h // heads), f16, _stream()), "enc_text")
+    _check(lib().da_enc_text(_ptr(x), table, n, _ptr(out), _ptr(ws), _ptr(cu), M, h, f, D, float(eps), math.log2(math.e) / math.sqrt(D), f16,
+                             _stream()), "enc_text")
+    return out
+
+
+class TextPlan:
+    """An encoder's weights (word, pos, type, emb_ln_g, emb_ln_b, layers) as ``enc_text_pooled`` takes them: the tensors, checked once."""
+
+    def __init__(self, w: dict, heads: int, eps: float):
+        self.f16 = w["word"].dtype == torch.float16
+        is_cuda = _f16_cuda if self.f16 else _bf16_cuda
+        self.emb, self.weights = [w[k] for k in ("word", "pos", "type", "emb_ln_g", "emb_ln_b")], w["layers"]
+        self.h, self.f, self.D, self.eps = w["word"].shape[1], self.weights[0]["w1"].shape[0], w["word"].shape[1] // heads, float(eps)
+        for t in self.emb:
+            is_cuda(t, "embeddings")
+            _req(t.shape[-1] == self.h and t.is_contiguous() and t.data_ptr() % 16 == 0, "TextPlan embeddings")
+        _req(enc_text_fits(1, self.h, self.f, len(self.weights), heads, 1, self.f16), "TextPlan shape")
+        self.weights = [dict(L) for L in self.weights]  # (kept as they are)
+        self.table, self.n = _text_layers(self.weights, self.h, self.f, is_cuda)
+        self.emb_table = (c_void_p * 5)(*(t.data_ptr() for t in self.emb))
+
+
+def enc_text_pooled(plan: TextPlan, tokens, mode: int) -> torch.Tensor:
+    """The whole encoder of one text of n <= 32 tokens, in three launches: the unit vector of its pooled rows (mode as pool_l2norm's),
+    fp32 [1, h]. tokens int32 [2 n + 2]: ids, positions, 0 and n."""
+    _i32(tokens, "tokens")
+    n, h = tokens.numel() // 2 - 1, plan.h
+    _req(1 <= n <= 32 and tokens.numel() == 2 * n + 2 and tokens.device == plan.emb[0].device, "enc_text_pooled tokens")
+    size, row = int(lib().da_enc_text_ws(n, h, plan.f, plan.n, plan.D, plan.f16)), n * h * 2
+    ws = torch.empty(size + 2 * row, dtype=torch.uint8, device=tokens.device)
+    out = torch.empty((1, h), dtype=torch.float32, device=tokens.device)
+    at, t = ws.data_ptr(), tokens.data_ptr()
+    _check(lib().da_enc_text_pooled(t, t + 4 * n, plan.emb_table, plan.table, plan.n, at + size, at + size + row, at, t + 8 * n, n, h, plan.f, plan.D,
+                                    plan.eps, math.log2(math.e) / math.sqrt(plan.D), mode, out.data_ptr(), plan.f16, _raw_stream()), "enc_text_pooled")
     return out
 
 

@@ -108,3 +108,33 @@ def test_which_texts_take_it(monkeypatch):
             calls.clear()
             enc.forward(i32([7] * T), i32(list(range(T))), i32(cu), T)
             assert len(calls) == (layers >= K.ENC_TEXT_MIN_LAYERS and T == 32 and len(cu) == 2)
+
+
+@pytest.mark.parametrize("h,f,heads,pooling,dtype", [(128, 256, 4, "cls", "bf16"), (768, 3072, 12, "mean", "bf16"), (1024, 4096, 16, "cls", "fp16"),
+                                                     (576, 1088, 9, "mean", "fp16")])
+def test_whole_text(h, f, heads, pooling, dtype):
+    """A question in three launches (embeddings; layers; norm and pooling) against the launches one by one; a result stays as it is when
+    the next question runs, on whichever stream."""
+    enc = BertEncoder(EncoderConfig("e", vocab=500, hidden=h, layers=5, heads=heads, ffn=f, pooling=pooling), "cuda", dtype=dtype)
+    g = torch.Generator().manual_seed(h)
+    for L in enc.w["layers"]:
+        for k in ("wqkv", "wo", "w1", "w2"):
+            L[k].mul_(3)  # (layers that matter beside the stream)
+    enc.prepare_graphs()
+    assert set(enc._g) == {64, 128}
+    other, had = torch.cuda.Stream(), []
+    for n in (1, 2, 15, 16, 17, 21, 31, 32, 33, 7):
+        seq = torch.randint(5, 500, (n,), generator=g).tolist()
+        with torch.cuda.stream(other if n % 2 else torch.cuda.default_stream()):
+            v = enc.encode_one(seq)
+        torch.cuda.synchronize()
+        ids, pos, cu = (torch.tensor(t, dtype=torch.int32, device="cuda") for t in (seq, list(range(n)), [0, n]))
+        with pytest.MonkeyPatch.context() as m:
+            m.setattr(K, "enc_text_fits", lambda *a: False)
+            want = enc._pool(enc.forward(ids, pos, cu, n), cu)
+        assert v.shape == want.shape and v.dtype == torch.float32
+        # roundings of the type, about 8 a layer, add as independent ones in both
+        u = 2.0 ** -9 if dtype == "bf16" else 2.0 ** -12
+        assert float((v - want).norm()) < 2 * (8 * 5) ** 0.5 * u and abs(float(v.norm()) - 1) < 1e-5
+        had.append((v, v.clone()))
+    assert all(torch.equal(a, b) for a, b in had)
