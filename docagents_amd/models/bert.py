@@ -225,7 +225,8 @@ class BertEncoder:
     # ~1.7 ms for a 20-token question, most of the p50 query's embed phase. One graph per padded
     # length bucket replays them in one submission. The rows past the real length are padding: the
     # GEMMs / norms process them (their rows are independent) and flash attention and the pooling
-    # read the real length from cu_seqlens, so row 0..L-1 see exactly the unpadded computation.
+    # read the real length from cu_seqlens, so row 0..L-1 see exactly the unpadded computation. (Texts that ops.enc_text_pooled takes have
+    # no graph: three launches of as many rows as they have.)
     GRAPH_BUCKETS = (16, 32, 64, 128)
     # small batches of short texts (the fast embed lane's micro-batches of questions): (sequences,
     # padded tokens) buckets; sequences packed back to back, then padding rows, padded
@@ -299,8 +300,8 @@ class BertEncoder:
                 self._g, self._gb, self._gs, self._text = {}, {}, {}, None
 
     def encode_one(self, seq: list[int]) -> torch.Tensor:
-        """One token sequence -> unit-norm embedding fp32 [1, H]: a captured graph when it fits a
-        length bucket on a GPU, else the eager packed path."""
+        """One token sequence -> unit-norm embedding fp32 [1, H]: on a GPU three launches for a short text, a captured
+        graph when it fits a length bucket, else the eager packed path."""
         L = len(seq)
         if self.device.type != "cuda" or L == 0 or L > min(self.GRAPH_BUCKETS[-1], self.cfg.max_pos) or \
                 torch.cuda.is_current_stream_capturing():
@@ -308,7 +309,7 @@ class BertEncoder:
         if getattr(self, "_g", None) is None:
             self.prepare_graphs()
         T = next(b for b in self.GRAPH_BUCKETS if b >= L)
-        if self._text is not None and T not in self._g and T <= 32:
+        if self._text is not None and T not in self._g and T <= 64:
             host = np.zeros(2 * L + 2, dtype=np.int32)
             host[:L] = seq
             host[L:2 * L] = np.arange(L)

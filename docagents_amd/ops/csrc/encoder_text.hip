@@ -1,4 +1,4 @@
-// A short text's encoder layers (one text, up to 32 rows) in one launch.
+// A short text's encoder layers (one text, up to 64 rows) in one launch.
 //
 // A layer is four products that wait for one another (csrc/encoder_rows.hip: QKV; attention and its output product; the
 // feed-forward's two), each of which takes 1 - 2 us of a launch of 5.5 - 7: the rest is its begin and end, and weights that are asked
@@ -18,8 +18,9 @@
 // MFMAs and the waves' sums 0.6 - 0.9, epilogue 0.7. (A row block a task, also in the wide products: the norm of 32 rows in one took 0.4 longer.
 // Waiting for one word first, or for one of the product before, so that waits read less: 165 - 184 us for 172, 16 rows of 768 columns.)
 //
-// us, launches one by one / this, bf16: 12 layers of 384 x 1536, 16 and 32 rows 215 / 140 and 219 / 149, of 768 x 3072 253 / 173 and 273 / 190, 24 of
-// 1024 x 4096 670 / 404 and 730 / 460; 4 of 768, 32 rows 93.5 / 72, 2 47.5 / 42.
+// us, launches one by one / this, bf16: 12 layers of 384 x 1536, 16, 32, 48 and 64 rows 215 / 142, 219 / 150, 244 / 189 and 255 / 194, of 768 x 3072
+// 253 / 171, 273 / 187, 346 / 284 and 350 / 290, 24 of 1024 x 4096, 16, 32 and 64 rows 670 / 396, 730 / 439 and 904 / 770; 4 of 768, 32 rows 93.5 / 72,
+// 2 47.5 / 42.
 #include <cstring>
 
 #include "gemm.h"
@@ -155,7 +156,7 @@ enc_text_kernel(const TextArgs p) {
     const TextMat x = layer ? TextMat{at(layer - 1) + (size_t)(4 * h + f) * R * 2, S, 32} : TextMat{(char*)p.x, 32, (unsigned)h * 2};
     char* base = at(layer);
     const TextMat qkv{base, S, 32}, y{base + (size_t)3 * h * R * 2, S, 32}, mid{base + (size_t)4 * h * R * 2, S, 32};
-    float2* st1 = (float2*)(base + (size_t)(5 * h + f) * R * 2);  // [strip][R]
+    float2* st1 = (float2*)(base + (size_t)(5 * h + f) * R * 2);  // [4 rows][strip][row]
     auto pieces = [&](const TextMat& m) __attribute__((always_inline)) {
       return __builtin_amdgcn_make_buffer_rsrc((void*)m.p, (short)0, 0x7fffff00, 0x00020000);
     };
@@ -179,9 +180,9 @@ enc_text_kernel(const TextArgs p) {
       const auto ld = [](const void* a) { return __hip_atomic_load((const unsigned long long*)a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
       if (!wide && out) orr = ld(m.p + strip * m.strip + om * m.row + 8 * (tid & 3));
       if (stats) {
-        const float2* st = (second ? (float2*)((char*)st1 - layer_bytes) + hs * R : st1) + m0 + 4 * w + fg;
+        const float2* st = (second ? (float2*)((char*)st1 - layer_bytes) + hs * R : st1) + (m0 / 4 + w) * hs * 4 + fg;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) q[e] = ld(st + min(fr + 16 * e, hs - 1) * R);
+        for (int e = 0; e < 4; ++e) q[e] = ld(st + min(fr + 16 * e, hs - 1) * 4);
       }
     };
     auto missing = [&]() __attribute__((always_inline)) {
@@ -252,14 +253,14 @@ enc_text_kernel(const TextArgs p) {
       }
       statistics();
       if (w < units) {
-        constexpr int NH = 64 / D, NT = MB;
-        f32x4_t s[NH][2];
-        bf16x8_t pf[NH];
+        constexpr int NH = 64 / D, NT = MB, NP = (MB + 1) / 2;  // keys: blocks of 16, and pairs of them
+        f32x4_t s[NH][2 * NP];
+        bf16x8_t pf[NH][NP];
         float inv[NH];
 #pragma unroll
         for (int i = 0; i < NH; ++i) {
           float mx = -INFINITY;
-          s[i][1] = f32x4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+          s[i][2 * NP - 1] = f32x4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
           for (int n = 0; n < NT; ++n) {
             s[i][n] = T::mma16(af[1 + n][i], af[0][i], f32x4_t{0.f, 0.f, 0.f, 0.f});
@@ -275,21 +276,28 @@ enc_text_kernel(const TextArgs p) {
           const float mc = mx == -INFINITY ? 0.f : fmaf(-mx, p.c, T::kF16 ? 0.f : -8.f);
           float all = 0.f;
 #pragma unroll
-          for (int n = 0; n < 2; ++n)
+          for (int n = 0; n < 2 * NP; ++n)
 #pragma unroll
             for (int e = 0; e < 4; ++e) all += s[i][n][e] = __builtin_amdgcn_exp2f(fmaf(s[i][n][e], p.c, mc));
           all = tx_rows(all, [](float a, float b) { return a + b; });
           inv[i] = all > 0.f ? 1.f / all : 0.f;
-          pf[i] = __builtin_bit_cast(bf16x8_t, u32x4_t{T::pack2(s[i][0][0], s[i][0][1]), T::pack2(s[i][0][2], s[i][0][3]),
-                                                       T::pack2(s[i][1][0], s[i][1][1]), T::pack2(s[i][1][2], s[i][1][3])});
+#pragma unroll
+          for (int n = 0; n < NP; ++n) {
+            const f32x4_t a = s[i][2 * n], b = s[i][2 * n + 1];
+            pf[i][n] = __builtin_bit_cast(bf16x8_t, u32x4_t{T::pack2(a[0], a[1]), T::pack2(a[2], a[3]), T::pack2(b[0], b[1]), T::pack2(b[2], b[3])});
+          }
         }
         f32x4_t o[4];  // d = 32 (i / 2) + 8 fg + 4 (i & 1) + e of row fr
         const char* v = (const char*)red[w] + (4 * fg + (fr >> 2)) * 32;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int c = 4 * (i >> 1) + (fr & 3), a = (c >> 1) * R * 32 + (c & 1) * 16 + 8 * (i & 1);
-          const s16x4_t lo = lds_read_tr16(v + a), up = MB == 2 ? lds_read_tr16(v + 16 * 32 + a) : s16x4_t{0, 0, 0, 0};
-          o[i] = T::mma16(bf16x8_t{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]}, pf[NH == 1 ? 0 : i >> 1], f32x4_t{0.f, 0.f, 0.f, 0.f});
+          o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int n = 0; n < NP; ++n) {
+            const s16x4_t lo = lds_read_tr16(v + n * 1024 + a), up = MB > 1 ? lds_read_tr16(v + n * 1024 + 512 + a) : s16x4_t{0, 0, 0, 0};
+            o[i] = T::mma16(bf16x8_t{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]}, pf[NH == 1 ? 0 : i >> 1][n], o[i]);
+          }
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -428,7 +436,7 @@ enc_text_kernel(const TextArgs p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) d = fmaf(z[e] - m, z[e] - m, d);
       d = tx_sum4(d);
-      if (out && (tid & 3) == 0) tx_put((phase == TX_OUT ? st1 : st1 + hs * R) + strip * R + om, __builtin_bit_cast(unsigned long long, float2{m, d}));
+      if (out && (tid & 3) == 0) tx_put((phase == TX_OUT ? st1 : st1 + hs * R) + ((om >> 2) * hs + strip) * 4 + (om & 3), __builtin_bit_cast(unsigned long long, float2{m, d}));
     }
   }
 }
@@ -537,10 +545,10 @@ enc_text_end_kernel(const bf16_t* y, const bf16_t* g, const bf16_t* b, const int
 
 // Bytes of da_enc_text's workspace; 0: it does not take such a text.
 DA_EXPORT long long da_enc_text_ws(int M, int h, int f, int layers, int D, int f16) {
-  if (M < 1 || M > 32 || layers < 1 || layers > TX_LAYERS || h < 64 || h % 64 || h > 64 * TX_WAVES || f < 64 || f % 64 || f > 256 * TX_WAVES ||
+  if (M < 1 || M > 64 || layers < 1 || layers > TX_LAYERS || h < 64 || h % 64 || h > 64 * TX_WAVES || f < 64 || f % 64 || f > 256 * TX_WAVES ||
       (D != 64 && (D != 32 || f16)))
     return 0;
-  const long long R = M <= 16 ? 16 : 32;
+  const long long R = M <= 16 ? 16 : M <= 32 ? 32 : 64;
   return layers * (R * 2 * (5ll * h + f) + 2 * (h / 16) * R * 8) + 256;  // (and the ticket)
 }
 
@@ -553,11 +561,13 @@ static int enc_text(const void* x, const void* const* layers, int n, void* out, 
   std::memcpy(a.L, layers, n * sizeof(TextLayer));
   a.x = (const bf16_t*)x; a.out = (bf16_t*)out; a.ws = (char*)ws; a.ticket = (int*)((char*)ws + bytes - 256); a.cu = cu;
   a.M = M; a.h = h; a.f = f; a.layers = n; a.eps = eps; a.c = c;
-  // strips a task: four of 33 - 64 KB of activations share the block's norm and its reading, two leave fewer weights to a task (us, four / two:
-  // 32 rows of 1024 columns, 24 layers 484 / 555, of 768, 12 209 / 216, of 512, 8 126 / 121, of 384, 12 178 / 168; 16 rows of 768 198 / 173, one 191)
+  // strips a task: with four fewer tasks read a block's activations and take its norm, with two a task has fewer weights (us, four / two: 32 rows
+  // of 1024 columns, 24 layers 484 / 555, of 768, 12 209 / 216, of 512, 8 126 / 121, of 384, 12 178 / 168; 64 rows of 768 290 / 334, of 384
+  // 194 / 204; 16 rows of 768 198 / 173, one 191)
 #define ENC_TEXT(T, DD)                                                                     \
   do {                                                                                      \
     if (M <= 16) enc_text_kernel<T, 1, DD, 2><<<256, 64 * TX_WAVES, 0, s>>>(a);             \
+    else if (M > 32) enc_text_kernel<T, 4, DD, 4><<<256, 64 * TX_WAVES, 0, s>>>(a);            \
     else if (h <= 512) enc_text_kernel<T, 2, DD, 2><<<256, 64 * TX_WAVES, 0, s>>>(a);       \
     else enc_text_kernel<T, 2, DD, 4><<<256, 64 * TX_WAVES, 0, s>>>(a);                     \
   } while (0)

@@ -655,8 +655,8 @@ ENC_TEXT_MIN_LAYERS = 4  # (two take as long as launches one by one)
 
 def enc_text_fits(M: int, hidden: int, ffn: int, layers: int, heads: int, texts: int, f16: bool = False) -> bool:
     """Whether ``enc_text`` takes the layers of an encoder."""
-    return (M <= 32 and ENC_TEXT_MIN_LAYERS <= layers <= 32 and hidden % 64 == 0 and ffn % 64 == 0 and ffn <= 4096
-            and attn_ln_fit(M, hidden, heads, texts, f16))
+    return (1 <= M <= 64 and ENC_TEXT_MIN_LAYERS <= layers <= 32 and hidden % 64 == 0 and hidden <= 1024 and ffn % 64 == 0 and 64 <= ffn <= 4096
+            and hidden in ((64 * heads,) if f16 else (32 * heads, 64 * heads)) and texts == 1)
 
 
 def _text_layers(layers, h: int, f: int, is_cuda):
@@ -674,7 +674,7 @@ def _text_layers(layers, h: int, f: int, is_cuda):
 
 
 def enc_text(x, layers, cu, heads: int, eps: float):
-    """All layers of one text of up to 32 rows in one launch (csrc/encoder_text.hip): x [M, h] -> the last layer's sum before
+    """All layers of one text of up to 64 rows in one launch (csrc/encoder_text.hip): x [M, h] -> the last layer's sum before
     its norm (rows behind the text: zeros). layers: dicts of wqkv, bqkv, wo, bo, ln1_g, ln1_b, w1, b1, w2, b2, ln2_g, ln2_b."""
     f16 = x.dtype == torch.float16
     is_cuda = _f16_cuda if f16 else _bf16_cuda
@@ -708,11 +708,11 @@ class TextPlan:
 
 
 def enc_text_pooled(plan: TextPlan, tokens, mode: int) -> torch.Tensor:
-    """The whole encoder of one text of n <= 32 tokens, in three launches: the unit vector of its pooled rows (mode as pool_l2norm's),
+    """The whole encoder of one text of n <= 64 tokens, in three launches: the unit vector of its pooled rows (mode as pool_l2norm's),
     fp32 [1, h]. tokens int32 [2 n + 2]: ids, positions, 0 and n."""
     _i32(tokens, "tokens")
     n, h = tokens.numel() // 2 - 1, plan.h
-    _req(1 <= n <= 32 and tokens.numel() == 2 * n + 2 and tokens.device == plan.emb[0].device, "enc_text_pooled tokens")
+    _req(1 <= n <= 64 and tokens.numel() == 2 * n + 2 and tokens.device == plan.emb[0].device, "enc_text_pooled tokens")
     size, row = int(lib().da_enc_text_ws(n, h, plan.f, plan.n, plan.D, plan.f16)), n * h * 2
     ws = torch.empty(size + 2 * row, dtype=torch.uint8, device=tokens.device)
     out = torch.empty((1, h), dtype=torch.float32, device=tokens.device)

@@ -41,21 +41,23 @@ def in64(x, layers, cu, heads, eps):
 def apart(x, layers, cu, heads, eps):
     """(the launches one by one)"""
     st1, st2 = torch.empty((2, 64, 64, 2), dtype=torch.float32, device="cuda")
-    norm = None
+    norm, h, attn = None, x.shape[1], K.flash_attn_f16 if x.dtype == torch.float16 else K.flash_attn_varlen
     for L in layers:
-        qkv = K.gemm_ln(x, L["wqkv"], L["bqkv"], norm=norm)
-        y = K.gemm_ln(qkv, L["wo"], L["bo"], K.EPI_RESID, norm=norm, resid=x, st_out=st1, attn=(heads, cu))
+        qkv, inside = K.gemm_ln(x, L["wqkv"], L["bqkv"], norm=norm), K.attn_ln_fit(x.shape[0], h, heads, 1, x.dtype == torch.float16)
+        a = qkv if inside else attn(qkv[:, :h], qkv[:, h:2 * h], qkv[:, 2 * h:], cu, x.shape[0], heads, heads, h // heads, causal=False)
+        y = K.gemm_ln(a, L["wo"], L["bo"], K.EPI_RESID, norm=norm, resid=x, st_out=st1, attn=(heads, cu) if inside else None)
         norm = (st1, L["ln1_g"], L["ln1_b"], eps)
         x = K.gemm_ln(K.gemm_ln(y, L["w1"], L["b1"], K.EPI_GELU, norm=norm), L["w2"], L["b2"], K.EPI_RESID, norm=norm, resid=y, st_out=st2)
         norm = (st2, L["ln2_g"], L["ln2_b"], eps)
     return x
 
 
-# one row; the edges of both row blocks; rows outside the text; units of K fewer than waves, as many, and 2 to 4 a wave; the most layers
+# one row; the edges of the row blocks; rows outside the text; units of K fewer than waves, as many, and 2 to 4 a wave; the most layers
 @pytest.mark.parametrize("M,h,f,heads,layers,cu", [
     (1, 64, 64, 1, 4, [0, 1]), (16, 384, 1536, 12, 6, [0, 16]), (17, 384, 1536, 6, 5, [0, 17]), (32, 768, 3072, 12, 12, [0, 21]),
     (16, 768, 3072, 12, 12, [0, 7]), (31, 1024, 4096, 16, 4, [3, 29]), (32, 1024, 4096, 32, 24, [0, 32]), (9, 832, 1088, 13, 4, [0, 9]),
-    (32, 128, 2112, 2, 32, [17, 18]), (2, 512, 4032, 8, 4, [0, 2])])
+    (32, 128, 2112, 2, 32, [17, 18]), (2, 512, 4032, 8, 4, [0, 2]), (33, 384, 1536, 12, 6, [0, 33]), (64, 1024, 4096, 16, 6, [0, 64]),
+    (48, 768, 3072, 24, 5, [0, 48]), (49, 832, 1088, 13, 4, [0, 49]), (64, 768, 3072, 12, 6, [0, 41]), (63, 64, 4096, 1, 4, [20, 50])])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 def test_layers(M, h, f, heads, layers, cu, dt):
     if dt == torch.float16 and h == 32 * heads:
@@ -76,7 +78,7 @@ def test_layers(M, h, f, heads, layers, cu, dt):
             assert torch.equal(K.enc_text(x, L, c, heads, 1e-12)[cu[0]:cu[1]].double(), got)
 
 
-@pytest.mark.parametrize("T", [16, 32])
+@pytest.mark.parametrize("T", [16, 32, 64])
 def test_replays(T):
     """Captured: each replay has its own input's result, with eager launches of the same stream between them."""
     L, r = make(768, 3072, 12, 12, torch.bfloat16)
@@ -98,16 +100,16 @@ def test_replays(T):
 
 
 def test_which_texts_take_it(monkeypatch):
-    """One text of up to 32 rows from ENC_TEXT_MIN_LAYERS layers on; others as before."""
+    """One text of up to 64 rows from ENC_TEXT_MIN_LAYERS layers on; others as before."""
     calls, real = [], K.enc_text
     monkeypatch.setattr(K, "enc_text", lambda *a: calls.append(1) or real(*a))
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
     for layers in (K.ENC_TEXT_MIN_LAYERS - 1, K.ENC_TEXT_MIN_LAYERS):
         enc = BertEncoder(EncoderConfig("e", vocab=100, hidden=128, layers=layers, heads=2, ffn=256), "cuda")
-        for T, cu in ((32, [0, 32]), (33, [0, 33]), (32, [0, 16, 32])):
+        for T, cu in ((64, [0, 64]), (65, [0, 65]), (32, [0, 16, 32])):
             calls.clear()
             enc.forward(i32([7] * T), i32(list(range(T))), i32(cu), T)
-            assert len(calls) == (layers >= K.ENC_TEXT_MIN_LAYERS and T == 32 and len(cu) == 2)
+            assert len(calls) == (layers >= K.ENC_TEXT_MIN_LAYERS and T == 64 and len(cu) == 2)
 
 
 @pytest.mark.parametrize("h,f,heads,pooling,dtype", [(128, 256, 4, "cls", "bf16"), (768, 3072, 12, "mean", "bf16"), (1024, 4096, 16, "cls", "fp16"),
@@ -121,9 +123,9 @@ def test_whole_text(h, f, heads, pooling, dtype):
         for k in ("wqkv", "wo", "w1", "w2"):
             L[k].mul_(3)  # (layers that matter beside the stream)
     enc.prepare_graphs()
-    assert set(enc._g) == {64, 128}
+    assert set(enc._g) == {128}
     other, had = torch.cuda.Stream(), []
-    for n in (1, 2, 15, 16, 17, 21, 31, 32, 33, 7):
+    for n in (1, 2, 15, 16, 17, 21, 31, 32, 33, 7, 48, 64, 65, 3):
         seq = torch.randint(5, 500, (n,), generator=g).tolist()
         with torch.cuda.stream(other if n % 2 else torch.cuda.default_stream()):
             v = enc.encode_one(seq)
