@@ -18,9 +18,9 @@
 // MFMAs and the waves' sums 0.6 - 0.9, epilogue 0.7. (A row block a task, also in the wide products: the norm of 32 rows in one took 0.4 longer.
 // Waiting for one word first, or for one of the product before, so that waits read less: 165 - 184 us for 172, 16 rows of 768 columns.)
 //
-// us, launches one by one / this, bf16: 12 layers of 384 x 1536, 16, 32, 48 and 64 rows 215 / 142, 219 / 150, 244 / 189 and 255 / 194, of 768 x 3072
-// 253 / 171, 273 / 187, 346 / 284 and 350 / 290, 24 of 1024 x 4096, 16, 32 and 64 rows 670 / 396, 730 / 439 and 904 / 770; 4 of 768, 32 rows 93.5 / 72,
-// 2 47.5 / 42.
+// us, launches one by one / this, bf16: 12 layers of 384 x 1536, 16, 32, 48 and 64 rows 215 / 142, 219 / 150, 244 / 168 and 255 / 175, of 768 x 3072
+// 253 / 171, 273 / 187, 346 / 223 and 350 / 265, 24 of 1024 x 4096, 16, 32, 36 and 64 rows 670 / 396, 730 / 439, 865 / 593 and 907 / 723; 4 of 768,
+// 32 rows 93.5 / 72, 2 47.5 / 42.
 #include <cstring>
 
 #include "gemm.h"
@@ -222,6 +222,19 @@ enc_text_kernel(const TextArgs p) {
       {
         const auto rs = pieces(qkv);
         u32x4_t v[R / 8] = {};
+        auto vread = [&]() __attribute__((always_inline)) {
+#pragma unroll
+          for (int j = 0; j < R / 8; ++j) {  // V, [4 strips][R rows][32 B]
+            const int e = j * 64 + lane, r = e / 2 % R;
+            v[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, r >= first && r < end ? e * 16 : 0x7ffffff0u, (2 * hs + 4 * w) * S, SC);
+          }
+        };
+        auto vmiss = [&]() __attribute__((always_inline)) {
+          bool no = false;
+#pragma unroll
+          for (int j = 0; j < R / 8; ++j) no |= tx_empty(v[j]);
+          return no;
+        };
         poll([&] {
           beside(x);
           if (w >= units) return missing();
@@ -233,21 +246,21 @@ enc_text_kernel(const TextArgs p) {
 #pragma unroll
             for (int i = 0; i < 2; ++i)
               u[2 + 2 * n + i] = __builtin_amdgcn_raw_buffer_load_b128(rs, chunk(qkv, i, 16 * n + fr, 16 * n + fr >= first && 16 * n + fr < end), (hs + 4 * w) * S, SC);
-#pragma unroll
-          for (int j = 0; j < R / 8; ++j) {  // V, [4 strips][R rows][32 B]
-            const int e = j * 64 + lane, r = e / 2 % R;
-            v[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, r >= first && r < end ? e * 16 : 0x7ffffff0u, (2 * hs + 4 * w) * S, SC);
-          }
+          if constexpr (MB <= 2) vread();
           bool no = missing();
 #pragma unroll
           for (int i = 0; i < 2 + 2 * MB; ++i) {
             no |= tx_empty(u[i]);
             af[i / 2][i % 2] = __builtin_bit_cast(bf16x8_t, u[i]);
           }
-#pragma unroll
-          for (int j = 0; j < R / 8; ++j) no |= tx_empty(v[j]);
+          if constexpr (MB <= 2) no |= vmiss();
           return no;
         });
+        if (MB > 2 && w < units)  // (all at once does not fit the registers: 64 rows of 768 columns 290 us, 265 so)
+          poll([&] {
+            vread();
+            return vmiss();
+          });
 #pragma unroll
         for (int j = 0; j < R / 8; ++j) *(u32x4_t*)((char*)red[w] + (j * 64 + lane) * 16) = v[j];
       }
@@ -295,7 +308,7 @@ enc_text_kernel(const TextArgs p) {
           o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int n = 0; n < NP; ++n) {
-            const s16x4_t lo = lds_read_tr16(v + n * 1024 + a), up = MB > 1 ? lds_read_tr16(v + n * 1024 + 512 + a) : s16x4_t{0, 0, 0, 0};
+            const s16x4_t lo = lds_read_tr16(v + n * 1024 + a), up = 2 * n + 1 < MB ? lds_read_tr16(v + n * 1024 + 512 + a) : s16x4_t{0, 0, 0, 0};
             o[i] = T::mma16(bf16x8_t{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]}, pf[NH == 1 ? 0 : i >> 1][n], o[i]);
           }
         }
@@ -548,7 +561,7 @@ DA_EXPORT long long da_enc_text_ws(int M, int h, int f, int layers, int D, int f
   if (M < 1 || M > 64 || layers < 1 || layers > TX_LAYERS || h < 64 || h % 64 || h > 64 * TX_WAVES || f < 64 || f % 64 || f > 256 * TX_WAVES ||
       (D != 64 && (D != 32 || f16)))
     return 0;
-  const long long R = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+  const long long R = (M + 15) / 16 * 16;
   return layers * (R * 2 * (5ll * h + f) + 2 * (h / 16) * R * 8) + 256;  // (and the ticket)
 }
 
@@ -563,13 +576,14 @@ static int enc_text(const void* x, const void* const* layers, int n, void* out, 
   a.M = M; a.h = h; a.f = f; a.layers = n; a.eps = eps; a.c = c;
   // strips a task: with four fewer tasks read a block's activations and take its norm, with two a task has fewer weights (us, four / two: 32 rows
   // of 1024 columns, 24 layers 484 / 555, of 768, 12 209 / 216, of 512, 8 126 / 121, of 384, 12 178 / 168; 64 rows of 768 290 / 334, of 384
-  // 194 / 204; 16 rows of 768 198 / 173, one 191)
-#define ENC_TEXT(T, DD)                                                                     \
-  do {                                                                                      \
-    if (M <= 16) enc_text_kernel<T, 1, DD, 2><<<256, 64 * TX_WAVES, 0, s>>>(a);             \
-    else if (M > 32) enc_text_kernel<T, 4, DD, 4><<<256, 64 * TX_WAVES, 0, s>>>(a);            \
-    else if (h <= 512) enc_text_kernel<T, 2, DD, 2><<<256, 64 * TX_WAVES, 0, s>>>(a);       \
-    else enc_text_kernel<T, 2, DD, 4><<<256, 64 * TX_WAVES, 0, s>>>(a);                     \
+  // 194 / 204; 16 rows of 768 198 / 173, with one 191)
+#define ENC_TEXT(T, DD)                                                                \
+  do {                                                                                 \
+    if (M <= 16) enc_text_kernel<T, 1, DD, 2><<<256, 64 * TX_WAVES, 0, s>>>(a);        \
+    else if (M > 48) enc_text_kernel<T, 4, DD, 4><<<256, 64 * TX_WAVES, 0, s>>>(a);    \
+    else if (M > 32) enc_text_kernel<T, 3, DD, 4><<<256, 64 * TX_WAVES, 0, s>>>(a);    \
+    else if (h <= 512) enc_text_kernel<T, 2, DD, 2><<<256, 64 * TX_WAVES, 0, s>>>(a);  \
+    else enc_text_kernel<T, 2, DD, 4><<<256, 64 * TX_WAVES, 0, s>>>(a);                \
   } while (0)
   if (D == 32) ENC_TEXT(BF16T, 32);
   else if (f16) ENC_TEXT(F16T, 64);
