@@ -650,7 +650,7 @@ def gemm_ln(a, w, bias, epi: int = EPI_BIAS, norm=None, resid=None, st_out=None,
     return out
 
 
-ENC_TEXT_MIN_LAYERS = 4  # (two take as long as launches one by one)
+ENC_TEXT_MIN_LAYERS = 4  # (two: 45 us for 48 of launches one by one; 4: 74 for 94)
 
 
 def enc_text_fits(M: int, hidden: int, ffn: int, layers: int, heads: int, texts: int, f16: bool = False) -> bool:
@@ -668,7 +668,7 @@ def _text_layers(layers, h: int, f: int, is_cuda):
         for name, shape in shapes.items():
             t = L[name]
             is_cuda(t, name)
-            _req(t.shape == shape and t.is_contiguous() and t.data_ptr() % 16 == 0, f"enc_text {name}")
+            _req(t.shape == shape and t.is_contiguous() and (t.dim() == 1 or t.data_ptr() % 16 == 0), f"enc_text {name}")
             table.append(t.data_ptr())
     return (c_void_p * len(table))(*table), len(layers)
 
@@ -700,7 +700,7 @@ class TextPlan:
         self.h, self.f, self.D, self.eps = w["word"].shape[1], self.weights[0]["w1"].shape[0], w["word"].shape[1] // heads, float(eps)
         for t in self.emb:
             is_cuda(t, "embeddings")
-            _req(t.shape[-1] == self.h and t.is_contiguous() and t.data_ptr() % 16 == 0, "TextPlan embeddings")
+            _req(t.shape[-1] == self.h and t.is_contiguous(), "TextPlan embeddings")
         _req(enc_text_fits(1, self.h, self.f, len(self.weights), heads, 1, self.f16), "TextPlan shape")
         self.weights = [dict(L) for L in self.weights]  # (kept as they are)
         self.table, self.n = _text_layers(self.weights, self.h, self.f, is_cuda)

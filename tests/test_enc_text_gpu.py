@@ -140,3 +140,41 @@ def test_whole_text(h, f, heads, pooling, dtype):
         assert float((v - want).norm()) < 2 * (8 * 5) ** 0.5 * u and abs(float(v.norm()) - 1) < 1e-5
         had.append((v, v.clone()))
     assert all(torch.equal(a, b) for a, b in had)
+
+
+def test_what_it_refuses():
+    """Shapes beyond the kernel's go the other way; wrong operands raise as the products one by one do."""
+    for M, h, f, layers, heads, texts, f16 in [(65, 768, 3072, 12, 12, 1, False), (0, 768, 3072, 12, 12, 1, False), (8, 1088, 3072, 12, 17, 1, False),
+                                               (8, 768, 4160, 12, 12, 1, False), (8, 768, 3072, 33, 12, 1, False), (8, 768, 3072, 12, 12, 2, False),
+                                               (8, 768, 3072, 12, 24, 1, True), (8, 768, 3072, 12, 8, 1, False), (8, 720, 3072, 12, 12, 1, False)]:
+        assert not K.enc_text_fits(M, h, f, layers, heads, texts, f16)
+    L, r = make(128, 256, 2, 4, torch.bfloat16)
+    cu, x = torch.tensor([0, 8], dtype=torch.int32, device="cuda"), r(8, 128)
+    K.enc_text(x, L, cu, 2, 1e-12)
+    off = torch.zeros(129, dtype=torch.bfloat16, device="cuda")[1:]  # (vectors may lie anywhere)
+    assert torch.equal(K.enc_text(x, [{**L[0], "bo": off}, *L[1:]], cu, 2, 1e-12), K.enc_text(x, [{**L[0], "bo": off.clone()}, *L[1:]], cu, 2, 1e-12))
+    for bad in ({"wo": L[0]["wo"].half()}, {"wo": L[0]["wo"].cpu()}, {"w1": L[0]["w1"][:, ::2]}, {"bqkv": L[0]["bo"]}):
+        with pytest.raises(ValueError):
+            K.enc_text(x, [{**L[0], **bad}, *L[1:]], cu, 2, 1e-12)
+    for args in ((x.t().contiguous().t(), cu), (x, cu.long()), (x, cu.cpu()), (r(65, 128), cu)):
+        with pytest.raises(ValueError):
+            K.enc_text(args[0], L, args[1], 2, 1e-12)
+
+
+def test_beside_one_another():
+    """Texts on several streams at once, beside products that fill the chip: each takes its tasks in order on whatever room it gets."""
+    L, r = make(768, 3072, 12, 6, torch.bfloat16)
+    xs, cu = [r(n, 768) for n in (16, 32, 48, 64)], [torch.tensor([0, n], dtype=torch.int32, device="cuda") for n in (16, 32, 48, 64)]
+    want = [K.enc_text(x, L, c, 12, 1e-12) for x, c in zip(xs, cu)]
+    a, b = r(4096, 4096), r(8192, 4096)
+    streams = [torch.cuda.Stream() for _ in range(5)]
+    torch.cuda.synchronize()
+    got = [[] for _ in xs]
+    for _ in range(8):
+        with torch.cuda.stream(streams[4]):
+            K.gemm(a, b)
+        for i, (x, c) in enumerate(zip(xs, cu)):
+            with torch.cuda.stream(streams[i]):
+                got[i].append(K.enc_text(x, L, c, 12, 1e-12))
+    torch.cuda.synchronize()
+    assert all(torch.equal(g, w) for gs, w in zip(got, want) for g in gs)
