@@ -254,7 +254,7 @@ gemm_dk_kernel(DkArgs p) {
     }
   }
   static_assert(EPI != EPI_RESID || ROWS || (CPR & (CPR - 1)) == 0, "a row's pieces meet by lane exchange");
-  if constexpr (EPI == EPI_ROPE) {  // rotated as the kernel behind a product does it: the rounded values in fp32, and rounded again
+  if constexpr (EPI == EPI_ROPE) {  // rotated as the kernel behind a product does it (the same bits): the rounded values in fp32, and rounded again
     const RopeArgs& R = p.rope;
     const int qw = R.H * R.D, kw = R.Hkv * R.D;
 #pragma unroll
@@ -275,8 +275,8 @@ gemm_dk_kernel(DkArgs p) {
       const int kind = gn < qw ? 0 : gn < qw + kw ? 1 : 2, rel = gn - (kind == 0 ? 0 : kind == 1 ? qw : qw + kw);
       if (kind < 2) {
         const f32x4_t x = unpack4<T>(o), cs = rcs[i];
-        o = u32x2_t{T::pack2(x[0] * cs[0] - x[1] * cs[1], x[1] * cs[0] + x[0] * cs[1]),
-                    T::pack2(x[2] * cs[2] - x[3] * cs[3], x[3] * cs[2] + x[2] * cs[3])};
+        o = u32x2_t{T::pack2(fmaf(x[0], cs[0], -(x[1] * cs[1])), fmaf(x[1], cs[0], x[0] * cs[1])),
+                    T::pack2(fmaf(x[2], cs[2], -(x[3] * cs[3])), fmaf(x[3], cs[2], x[2] * cs[3]))};
       }
       if (kind > 0) {
         DA_ASSERT(rpos[i] >= 0 && rpos[i] < R.max_seq && rslot[i] >= 0);

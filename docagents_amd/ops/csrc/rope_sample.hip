@@ -47,8 +47,8 @@ rope_cache_kernel(bf16_t* __restrict__ qkv, const int* __restrict__ pos, const i
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float x1 = bf2f(a[e] & 0xffff), x2 = bf2f(a[e] >> 16);
-      const float o1 = x1 * cc[e] - x2 * sn[e];
-      const float o2 = x2 * cc[e] + x1 * sn[e];
+      const float o1 = fmaf(x1, cc[e], -(x2 * sn[e]));
+      const float o2 = fmaf(x2, cc[e], x1 * sn[e]);
       r[e] = pack_bf2(o1, o2);
     }
     *(u32x4_t*)hp = r;
