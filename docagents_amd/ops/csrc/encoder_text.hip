@@ -13,6 +13,8 @@
 // of workgroups on the chip. A wait has an end of its own after some seconds, and then a result of NaNs.
 // A ticket is taken when the task before is done: taken ahead, a task of the next product began behind later ones (768 columns, 32 rows: 400 us for 229).
 //
+// Sums, statistics and roundings are in the order of the launches one by one (attention inside the output product): in bf16 the same bits.
+//
 // Activations are in strips of 16 columns, [strip][row][16], so that a store of a task fills its lines, and MFMA operands come straight from
 // there in whole lines; V alone goes through LDS. What is left of a product is a chain: 1 us from the last store to the operand, norm 0.4,
 // MFMAs and the waves' sums 0.6 - 0.9, epilogue 0.7. (A row block a task, also in the wide products: the norm of 32 rows in one took 0.4 longer.
@@ -69,15 +71,16 @@ template <int CTRL>
 __device__ __forceinline__ float tx_dpp(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
-// Sums over 4 and 16 lanes beside one another, in each of them: lanes ^ 1, ^ 2, then 7 - lane and 15 - lane.
+// Sums over 4 lanes beside one another, in each of them: lanes ^ 1, ^ 2; over 16: ^ 8, ^ 4, ^ 2, ^ 1 (as rotations, which come to that).
 __device__ __forceinline__ float tx_sum4(float v) {
   v += tx_dpp<0xb1>(v);
   return v + tx_dpp<0x4e>(v);
 }
 __device__ __forceinline__ float tx_sum16(float v) {
-  v = tx_sum4(v);
-  v += tx_dpp<0x141>(v);
-  return v + tx_dpp<0x140>(v);
+  v += tx_dpp<0x128>(v);
+  v += tx_dpp<0x124>(v);
+  v += tx_dpp<0x122>(v);
+  return v + tx_dpp<0x121>(v);
 }
 // op over lanes l, l ^ 16, l ^ 32 and l ^ 48
 template <typename Op>
@@ -131,6 +134,8 @@ enc_text_kernel(const TextArgs p) {
     // ---- weights ----
     const TextLayer &L = p.L[layer], &P = p.L[max(layer - 1, 0)];
     const int K = phase == TX_DOWN ? f : h, units = K / 64;
+    // as many waves as share the units evenly: wave w takes units w, w + nw, ..
+    const int nw = units <= TX_WAVES ? units : units <= 2 * TX_WAVES ? (units + 1) / 2 : units <= 3 * TX_WAVES ? (units + 2) / 3 : (units + 3) / 4;
     const bool second = phase == TX_QKV || phase == TX_OUT;  // the norm before this task's operand or residual: the layer before's second
     const bf16_t *g = second ? P.g2 : L.g1, *b = second ? P.b2 : L.b1;
     const bool own = w < (wide ? NS : 1), normed = layer > 0 || phase >= TX_UP;
@@ -156,7 +161,7 @@ enc_text_kernel(const TextArgs p) {
     const TextMat x = layer ? TextMat{at(layer - 1) + (size_t)(4 * h + f) * R * 2, S, 32} : TextMat{(char*)p.x, 32, (unsigned)h * 2};
     char* base = at(layer);
     const TextMat qkv{base, S, 32}, y{base + (size_t)3 * h * R * 2, S, 32}, mid{base + (size_t)4 * h * R * 2, S, 32};
-    float2* st1 = (float2*)(base + (size_t)(5 * h + f) * R * 2);  // [4 rows][strip][row]
+    float2* st1 = (float2*)(base + (size_t)(5 * h + f) * R * 2);  // [4 rows][strip % 4][strip / 4][row]
     auto pieces = [&](const TextMat& m) __attribute__((always_inline)) {
       return __builtin_amdgcn_make_buffer_rsrc((void*)m.p, (short)0, 0x7fffff00, 0x00020000);
     };
@@ -182,7 +187,7 @@ enc_text_kernel(const TextArgs p) {
       if (stats) {
         const float2* st = (second ? (float2*)((char*)st1 - layer_bytes) + hs * R : st1) + (m0 / 4 + w) * hs * 4 + fg;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) q[e] = ld(st + min(fr + 16 * e, hs - 1) * 4);
+        for (int e = 0; e < 4; ++e) q[e] = ld(st + (e * (hs / 4) + min(fr, hs / 4 - 1)) * 4);  // strip 4 fr + e
       }
     };
     auto missing = [&]() __attribute__((always_inline)) {
@@ -193,7 +198,7 @@ enc_text_kernel(const TextArgs p) {
       }
       return no;
     };
-    auto sums = [&](const f32x4_t& acc, int j) __attribute__((always_inline)) { if (w < units) *(f32x4_t*)&red[w][(16 * j + fr) * 16 + 4 * fg] = acc; };
+    auto sums = [&](const f32x4_t& acc, int j) __attribute__((always_inline)) { if (w < nw) *(f32x4_t*)&red[w][(16 * j + fr) * 16 + 4 * fg] = acc; };
     auto statistics = [&]() __attribute__((always_inline)) {
       if (!stats) return;
       float2 sq[4];
@@ -201,11 +206,11 @@ enc_text_kernel(const TextArgs p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         sq[e] = __builtin_bit_cast(float2, q[e]);
-        a += fr + 16 * e < hs ? sq[e].x : 0.f;
+        a += fr < hs / 4 ? sq[e].x : 0.f;
       }
       const float m = tx_sum16(a) / hs;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v += fr + 16 * e < hs ? fmaf(16.f * (sq[e].x - m), sq[e].x - m, sq[e].y) : 0.f;
+      for (int e = 0; e < 4; ++e) v += fr < hs / 4 ? fmaf(16.f * (sq[e].x - m), sq[e].x - m, sq[e].y) : 0.f;
       v = tx_sum16(v);
       if (fr == 0) {
         smean[4 * w + fg] = m;
@@ -323,31 +328,32 @@ enc_text_kernel(const TextArgs p) {
       sums(acc[0], 0);
     } else if (phase == TX_DOWN) {
       f32x4_t acc[1]{f32x4_t{0.f, 0.f, 0.f, 0.f}};
+      const auto unit = [&](int n) { return w < nw ? w + n * nw : units; };
       bf16x8_t wf[4][2] = {}, af[4][2] = {};
 #pragma unroll
       for (int n = 0; n < 4; ++n)
-        if (w + n * TX_WAVES < units) weights(w + n * TX_WAVES, strip, wf[n]);
+        if (unit(n) < units) weights(unit(n), strip, wf[n]);
       asm volatile("" ::: "memory");
       const auto rs = pieces(mid);
       poll([&] {
         beside(y);
 #pragma unroll
         for (int n = 0; n < 4; ++n)
-          if (w + n * TX_WAVES < units) {
+          if (unit(n) < units) {
 #pragma unroll
             for (int i = 0; i < 2; ++i)
-              af[n][i] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rs, chunk(mid, i, m0 + fr, m0 + fr < end), 4 * (w + n * TX_WAVES) * S, SC));
+              af[n][i] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rs, chunk(mid, i, m0 + fr, m0 + fr < end), 4 * unit(n) * S, SC));
           }
         bool no = missing();
 #pragma unroll
         for (int n = 0; n < 4; ++n)
-          if (w + n * TX_WAVES < units) no |= tx_empty(__builtin_bit_cast(u32x4_t, af[n][0])) || tx_empty(__builtin_bit_cast(u32x4_t, af[n][1]));
+          if (unit(n) < units) no |= tx_empty(__builtin_bit_cast(u32x4_t, af[n][0])) || tx_empty(__builtin_bit_cast(u32x4_t, af[n][1]));
         return no;
       });
       statistics();
 #pragma unroll
       for (int n = 0; n < 4; ++n)
-        if (w + n * TX_WAVES < units) {
+        if (unit(n) < units) {
 #pragma unroll
           for (int i = 0; i < 2; ++i) acc[0] = T::mma16(wf[n][i], af[n][i], acc[0]);
         }
@@ -413,14 +419,14 @@ enc_text_kernel(const TextArgs p) {
     const float* rd = &red[0][4 * tid];
     f32x4_t v = *(const f32x4_t*)rd;
     int u = 1;
-    for (; u + 4 < units && u + 4 < TX_WAVES; u += 5) {  // (waves past the units have no sums)
+    for (; u + 4 < nw; u += 5) {
       f32x4_t s[5];
 #pragma unroll
       for (int j = 0; j < 5; ++j) s[j] = *(const f32x4_t*)(rd + (u + j) * RED);
 #pragma unroll
       for (int j = 0; j < 5; ++j) v += s[j];
     }
-    for (; u < min(units, TX_WAVES); ++u) v += *(const f32x4_t*)(rd + u * RED);
+    for (; u < nw; ++u) v += *(const f32x4_t*)(rd + u * RED);
     const auto val = [](const u32x2_t& o, int e) { return T::to_f((bf16_t)(e & 1 ? o[e >> 1] >> 16 : o[e >> 1] & 0xffff)); };
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] += val(ob, e);
@@ -449,7 +455,7 @@ enc_text_kernel(const TextArgs p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) d = fmaf(z[e] - m, z[e] - m, d);
       d = tx_sum4(d);
-      if (out && (tid & 3) == 0) tx_put((phase == TX_OUT ? st1 : st1 + hs * R) + ((om >> 2) * hs + strip) * 4 + (om & 3), __builtin_bit_cast(unsigned long long, float2{m, d}));
+      if (out && (tid & 3) == 0) tx_put((phase == TX_OUT ? st1 : st1 + hs * R) + ((om >> 2) * hs + (strip & 3) * (hs / 4) + (strip >> 2)) * 4 + (om & 3), __builtin_bit_cast(unsigned long long, float2{m, d}));
     }
   }
 }
@@ -465,6 +471,11 @@ __device__ __forceinline__ void tx_load(const bf16_t* p, float (&v)[8]) {
   const bf16x8_t u = *(const bf16x8_t*)p;
 #pragma unroll
   for (int e = 0; e < 8; ++e) v[e] = T::to_f((bf16_t)u[e]);
+}
+
+template <typename T>
+__device__ __forceinline__ u32x4_t tx_pack(const float (&v)[8]) {
+  return u32x4_t{T::pack2(v[0], v[1]), T::pack2(v[2], v[3]), T::pack2(v[4], v[5]), T::pack2(v[6], v[7])};
 }
 
 // LayerNorm of a row of D <= 1024 columns, a wave: lane's columns 8 (lane + 64 i) + e, as the layernorm kernel does it.
@@ -518,18 +529,20 @@ enc_text_begin_kernel(const int* ids, const int* positions, const bf16_t* word, 
   tx_norm<T>(v, g, b, lane, D, eps);
 #pragma unroll
   for (int i = 0; i < 2; ++i)
-    if ((lane + 64 * i) * 8 < D) *(u32x4_t*)(x + (size_t)row * D + (lane + 64 * i) * 8) = u32x4_t{T::pack2(v[i][0], v[i][1]), T::pack2(v[i][2], v[i][3]),
-                                                                            T::pack2(v[i][4], v[i][5]), T::pack2(v[i][6], v[i][7])};
+    if ((lane + 64 * i) * 8 < D) *(u32x4_t*)(x + (size_t)row * D + (lane + 64 * i) * 8) = tx_pack<T>(v[i]);
 }
 
-// The last one: the norm behind the layers, the pooling (mode 0: the text's first row, 1: the mean of its rows) and the unit norm, in fp32.
+// The last one: the norm behind the layers, the pooling (mode 0: the text's first row, 1: the mean of its rows) and the unit norm, in fp32. Rows and
+// sums in the order of the pooling kernels: the same bits.
 template <typename T>
 __global__ void __launch_bounds__(64 * TX_WAVES)
 enc_text_end_kernel(const bf16_t* y, const bf16_t* g, const bf16_t* b, const int* cu, int M, int D, float eps, int mode, float* out) {
-  __shared__ __attribute__((aligned(16))) float part[TX_WAVES][1024];
+  constexpr int NT = 64 * TX_WAVES;
+  __shared__ __attribute__((aligned(16))) char smem[64 * 1024 * 2];  // the normed rows, and then each thread's sums
   __shared__ float red[16];
+  bf16_t* rows = (bf16_t*)smem;
+  float* part = (float*)smem;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, first = min(max(cu[0], 0), M - 1), n = mode ? max(min(cu[1], M) - first, 1) : 1;
-  float a[2][8] = {};
   for (int r = w; r < n; r += TX_WAVES) {
     float v[2][8];
 #pragma unroll
@@ -537,23 +550,39 @@ enc_text_end_kernel(const bf16_t* y, const bf16_t* g, const bf16_t* b, const int
     tx_norm<T>(v, g, b, lane, D, eps);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) a[i][e] += T::to_f(T::from_f(v[i][e]));  // (rounded as the rows are)
+      if ((lane + 64 * i) * 8 < D) *(u32x4_t*)(rows + r * D + (lane + 64 * i) * 8) = tx_pack<T>(v[i]);
   }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      if ((lane + 64 * i) * 8 < D) part[w][(lane + 64 * i) * 8 + e] = a[i][e];
   __syncthreads();
-  float v = 0.f;
-  if ((int)threadIdx.x < D) {
+  // threads of 8 columns, and each the rows gr, gr + G, ..
+  const int nch = D / 8, G = NT / nch, gr = threadIdx.x / nch, c = threadIdx.x % nch;
+  float v[8] = {}, ss = 0.f;
+  if (gr < G)
+    for (int t = gr; t < n; t += G) {
+      float a[8];
+      tx_load<T>(rows + t * D + c * 8, a);
 #pragma unroll
-    for (int i = 0; i < TX_WAVES; ++i) v += part[i][threadIdx.x];
-    v *= 1.f / (float)n;
+      for (int e = 0; e < 8; ++e) v[e] += a[e];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < 8; ++e) part[threadIdx.x * 8 + e] = v[e];
+  __syncthreads();
+  if (gr == 0) {
+    for (int i = 1; i < min(G, n); ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += part[(i * nch + c) * 8 + e];
+    const float invn = 1.f / (float)n;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      v[e] *= invn;
+      ss += v[e] * v[e];
+    }
   }
-  const float ss = block_sum(v * v, red), inv = ss > 0.f ? rsqrtf(ss) : 1.f;
-  if ((int)threadIdx.x < D) out[threadIdx.x] = v * inv;
+  ss = block_sum(ss, red);
+  const float inv = ss > 0.f ? rsqrtf(ss) : 1.f;
+  if (gr) return;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) out[c * 8 + e] = v[e] * inv;
 }
 
 // Bytes of da_enc_text's workspace; 0: it does not take such a text.

@@ -70,9 +70,12 @@ def test_layers(M, h, f, heads, layers, cu, dt):
         got, one = (fn(x, L, c, heads, 1e-12)[cu[0]:cu[1]].double() for fn in (K.enc_text, apart))
         ref = in64(x, L, cu, heads, 1e-12)[cu[0]:cu[1]]
         e, e1 = (float((t - ref).norm() / ref.norm()) for t in (got, one))
-        # the same roundings in the same places, of sums in another order: errors of one size. A layer rounds about eight
+        # with attention inside the products, one by one: the same sums in the same order, and in bf16 the same bits (in fp16 the
+        # compiler rounds some norms within the fma, and which ones differs from kernel to kernel). Where it is a launch of its
+        # own the sums are in another order: the same roundings in the same places, errors of one size. A layer rounds about eight
         # times, by 2^-9 (2^-12) of values of about one each, which add as independent ones over the layers
         u = 2.0 ** -9 if dt == torch.bfloat16 else 2.0 ** -12
+        assert torch.equal(got, one) or dt == torch.float16 or not K.attn_ln_fit(M, h, heads, 1)
         assert e < 1.25 * e1 + u and e < 4 * (8 * layers) ** 0.5 * u, (e, e1)
         for _ in range(10):
             assert torch.equal(K.enc_text(x, L, c, heads, 1e-12)[cu[0]:cu[1]].double(), got)
@@ -133,8 +136,10 @@ def test_whole_text(h, f, heads, pooling, dtype):
         ids, pos, cu = (torch.tensor(t, dtype=torch.int32, device="cuda") for t in (seq, list(range(n)), [0, n]))
         with pytest.MonkeyPatch.context() as m:
             m.setattr(K, "enc_text_fits", lambda *a: False)
+            m.setattr(enc, "_one_row", lambda rows: False)
             want = enc._pool(enc.forward(ids, pos, cu, n), cu)
         assert v.shape == want.shape and v.dtype == torch.float32
+        assert torch.equal(v, want) or dtype == "fp16" or not K.attn_ln_fit(n, h, heads, 1)
         # roundings of the type, about 8 a layer, add as independent ones in both
         u = 2.0 ** -9 if dtype == "bf16" else 2.0 ** -12
         assert float((v - want).norm()) < 2 * (8 * 5) ** 0.5 * u and abs(float(v.norm()) - 1) < 1e-5
