@@ -108,10 +108,18 @@ class Engine:
         return self.enc_cfg.hidden
 
     # ------------------------------------------------------------------ embeddings
-    def embed(self, texts: list[str], preprocess: bool = True, out_dtype=torch.bfloat16) -> torch.Tensor:
-        """Unit-norm embeddings [n, d] on the engine device (1:1 with ``texts``)."""
+    def embed(self, texts: list[str], preprocess: bool = True, out_dtype=torch.bfloat16, checked: bool = False) -> torch.Tensor:
+        """Unit-norm embeddings [n, d] on the engine device (1:1 with ``texts``). checked: the host waits for those that
+        ``BertEncoder.check`` is about, and asks it."""
         if self.encoder is None:
             raise RuntimeError("encoder not loaded")
+        if checked:
+            had = self.encoder.text_launches
+            out = self.embed(texts, preprocess, out_dtype)
+            if self.encoder.text_launches != had:
+                torch.cuda.current_stream(self.device).synchronize()
+                self.encoder.check()
+            return out
         if preprocess:
             texts = [preprocess_text(t) for t in texts]
         n = len(texts)
@@ -157,6 +165,12 @@ class Engine:
         self.stats["embed_texts"] += n
         self.stats["embed_s"] += time.perf_counter() - t0
         return out
+
+    def embed_host(self, texts: list[str], preprocess: bool = True) -> np.ndarray:
+        """``embed`` as fp32 rows of the host."""
+        v = self.embed(texts, preprocess, out_dtype=torch.float32).cpu().numpy()
+        self.encoder.check()
+        return v
 
     def embed_one(self, text: str) -> torch.Tensor:
         """Embed(text): error on empty-after-preprocessing input (openai.go:44-47)."""

@@ -147,7 +147,7 @@ class EngineGroup:
         e = self.engine
         if cmd == "embed":
             faults.maybe_fail("engine.embed")
-            return e.embed(a["texts"], a.get("preprocess", True), out_dtype=torch.float32).cpu().numpy()
+            return e.embed_host(a["texts"], a.get("preprocess", True))
         if cmd in ("answer", "summarize"):
             # every TP rank of the replica runs every generation on its weight shard; the leader's
             # result is the replica's (identical on all TP ranks)
@@ -181,7 +181,7 @@ class EngineGroup:
             if mine:
                 faults.maybe_fail("engine.embed")
                 texts = [t for _, _, ts in mine for t in ts]
-                v = e.embed(texts, True)
+                v = e.embed(texts, True, checked=True)
                 o = 0
                 for doc_id, keys, ts in mine:
                     self._put(doc_id, np.asarray(keys, dtype=np.int64), v[o:o + len(ts)])
@@ -380,13 +380,13 @@ class EngineServer:
         e = self.group.engine
         faults.maybe_fail("engine.embed")
         if e.device.type != "cuda":
-            return e.embed(texts, preprocess, out_dtype=torch.float32).cpu().numpy()
+            return e.embed_host(texts, preprocess)
         from ..ops import kernels as K
         if self._fast_stream is None:
             torch.cuda.set_device(e.device)
             self._fast_stream = torch.cuda.Stream(device=e.device)
         with torch.cuda.stream(self._fast_stream), K.workspace_role("fast"):
-            return e.embed(texts, preprocess, out_dtype=torch.float32).cpu().numpy()
+            return e.embed_host(texts, preprocess)
 
     async def _embed_fast(self, texts, preprocess: bool):
         """Queue query-sized texts for the fast lane; the lane runs every text queued while its

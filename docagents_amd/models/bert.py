@@ -62,6 +62,10 @@ class BertEncoder:
         self._g_lock = threading.Lock()  # encode_one: the captured graphs' static buffers
         self._g_done = None              # event: the last graph use's output copied out
         self._text = None                # one short text's plan (ops.enc_text_pooled), set with the graphs
+        self._waits = None
+        if self.device.type == "cuda":
+            with torch.cuda.device(self.device):
+                self._waits = self.ops.TextWaits()
 
     def _linear(self, x, L, name, bias, epi, resid=None, xq=None):
         """fp8 path: ``xq = (q, scale)`` when the producer (a LayerNorm) already emitted the
@@ -165,7 +169,7 @@ class BertEncoder:
         h, nh, hd = c.hidden, c.heads, c.head_dim
         layers = self.w["layers"]
         if o.enc_text_fits(x.shape[0], h, c.ffn, len(layers), nh, cu_seqlens.numel() - 1, self.fp16):
-            return layernorm(o.enc_text(x, layers, cu_seqlens, nh, c.eps), layers[-1]["ln2_g"], layers[-1]["ln2_b"], c.eps)
+            return layernorm(o.enc_text(x, layers, cu_seqlens, nh, c.eps, self._waits), layers[-1]["ln2_g"], layers[-1]["ln2_b"], c.eps)
         st1, st2 = torch.empty((2, 64, 64, 2), dtype=torch.float32, device=x.device)
         norm = None
         inside = o.attn_ln_fit(x.shape[0], h, nh, cu_seqlens.numel() - 1, self.fp16)
@@ -250,7 +254,7 @@ class BertEncoder:
         # (key, T, max_seqlen, cu): the one-sequence length buckets and the batches' row counts
         c = self.cfg
         text = [not self.fp8 and self.ops.enc_text_fits(T, c.hidden, c.ffn, len(self.w["layers"]), c.heads, 1, self.fp16) for T in self.GRAPH_BUCKETS]
-        self._text = K.TextPlan(self.w, c.heads, c.eps) if any(text) else None  # (short texts: three launches, and no graph)
+        self._text = K.TextPlan(self.w, c.heads, c.eps, self._waits) if any(text) else None  # (short texts: three launches, and no graph)
         shapes = [(("one", T), T, T, [0, T]) for T, fits in zip(self.GRAPH_BUCKETS, text) if not fits]
         most = {T: max(nb for nb, rows in (*self.BATCH_BUCKETS, *self.SHORT_BUCKETS) if rows == T) for _, T in self.BATCH_BUCKETS}
         for T, nb in most.items():
@@ -298,6 +302,17 @@ class BertEncoder:
                 import logging
                 logging.getLogger(__name__).warning("encoder graph capture failed, eager path: %r", e)
                 self._g, self._gb, self._gs, self._text = {}, {}, {}, None
+
+    @property
+    def text_launches(self) -> int:
+        """How many launches ``check`` has been about."""
+        return 0 if self._waits is None else self._waits.launches
+
+    def check(self) -> None:
+        """KernelError if a short text's one launch gave a wait up, which leaves NaNs for its embedding: for who has waited for an embedding
+        and is about to use it. (The next such launch asks too.)"""
+        if self._waits is not None:
+            self._waits.check()
 
     def encode_one(self, seq: list[int]) -> torch.Tensor:
         """One token sequence -> unit-norm embedding fp32 [1, H]: on a GPU three launches for a short text, a captured

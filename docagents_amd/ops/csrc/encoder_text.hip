@@ -10,7 +10,7 @@
 // another one); whoever reads them, past the L2s too, reads again until that is gone. That is a store and a load between two products;
 // with a counter per product (store, its acknowledgement, an addition, its reading, the load) they were 7 us apart.
 // Tasks are taken in order and wait for earlier ones only, and whoever took a task runs: the first that is not done always ends, with any number
-// of workgroups on the chip. A wait has an end of its own after some seconds, and then a result of NaNs.
+// of workgroups on the chip. A wait has an end of its own all the same, after some seconds; then the result is NaNs, and a word of the host says so.
 // A ticket is taken when the task before is done: taken ahead, a task of the next product began behind later ones (768 columns, 32 rows: 400 us for 229).
 //
 // Sums, statistics and roundings are in the order of the launches one by one (attention inside the output product): in bf16 the same bits.
@@ -20,14 +20,15 @@
 // MFMAs and the waves' sums 0.6 - 0.9, epilogue 0.7. (A row block a task, also in the wide products: the norm of 32 rows in one took 0.4 longer.
 // Waiting for one word first, or for one of the product before, so that waits read less: 165 - 184 us for 172, 16 rows of 768 columns.)
 //
-// us, launches one by one / this, bf16: 12 layers of 384 x 1536, 16, 32, 48 and 64 rows 215 / 142, 219 / 150, 244 / 168 and 255 / 175, of 768 x 3072
-// 253 / 171, 273 / 187, 346 / 223 and 350 / 265, 24 of 1024 x 4096, 16, 32, 36 and 64 rows 670 / 396, 730 / 439, 865 / 593 and 907 / 723; 4 of 768,
-// 32 rows 93.5 / 72, 2 47.5 / 42.
+// us, launches one by one / this, bf16: 12 layers of 384 x 1536, 16, 32, 48 and 64 rows 215 / 142, 217 / 156, 242 / 174 and 256 / 177, of 768 x 3072
+// 253 / 170, 274 / 193, 346 / 231 and 347 / 270, 24 of 1024 x 4096, 16, 32, 36 and 64 rows 670 / 387, 730 / 461, 868 / 618 and 901 / 752; 4 of 768,
+// 32 rows 93 / 74, 2 48 / 44. (That a wait which runs out is told costs 0.6 %: 21 rows of 768 columns 187.3 -> 190.0. Matrices are chosen by
+// value: by reference the scalars that go to lanes and back are 55 to 73 a variant for 50 to 59.)
 #include <cstring>
 
 #include "gemm.h"
 
-constexpr int TX_LAYERS = 32, TX_WAVES = 16, TX_POLLS = 1 << 22;
+constexpr int TX_LAYERS = 32, TX_WAVES = 16;
 
 enum { TX_QKV, TX_OUT, TX_UP, TX_DOWN };
 
@@ -42,7 +43,9 @@ struct TextArgs {
   char* ws;         // per layer: qkv, the first sum, the feed-forward's middle, the second sum, and both sums' statistics; all bits set
   int* ticket;      // the last one taken; -1
   const int* cu;
+  int* gave_up;  // of the host's memory, or null: 1 where a wait ran out
   int M, h, f, layers;
+  int polls;  // minus the readings of a wait
   float eps, c;  // c: log2(e) times the scale of the scores
 };
 
@@ -101,6 +104,8 @@ enc_text_kernel(const TextArgs p) {
   __shared__ __attribute__((aligned(16))) float red[TX_WAVES][RED];  // each wave's sums; attention: its V before
   __shared__ float smean[16], srstd[16];
   __shared__ int snext;
+  __shared__ int sgave;  // (in LDS: the pointer would take registers in every task)
+  if (threadIdx.x == 0) sgave = 0;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = p.h, f = p.f, hs = h / 16;
   const int per = (3 * hs / NS + hs + f / (16 * NS) + hs) * MB, total = per * p.layers;
@@ -115,7 +120,10 @@ enc_text_kernel(const TextArgs p) {
   for (take(0);;) {
     tx_barrier();  // (the task before this one is done with LDS)
     const int t = __builtin_amdgcn_readfirstlane(snext);
-    if (t >= total) return;
+    if (t >= total) {
+      if (threadIdx.x == 0 && sgave && p.gave_up) __hip_atomic_store(p.gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      return;
+    }
     // ---- the task ----
     const int layer = t / per;
     int index = t - layer * per, phase = TX_QKV;
@@ -170,11 +178,13 @@ enc_text_kernel(const TextArgs p) {
       return in ? (2 * i + (fg >> 1)) * m.strip + r * m.row + (fg & 1) * 16 : 0x7ffffff0u;
     };
     auto poll = [&](auto read) __attribute__((always_inline)) {
+      int n = p.polls;
 #pragma clang loop unroll(disable)
-      for (int n = 0; n < TX_POLLS; ++n) {
+      for (; n < 0; ++n) {
         if (!__any(read())) break;
         __builtin_amdgcn_s_sleep(1);
       }
+      if (n == 0) sgave = 1;
     };
     const int om = m0 + (lane >> 2), ostrip = strip + (wide ? w : 0);  // the result's row of this thread, and its strip
     const bool out = own && om < end;
@@ -378,7 +388,7 @@ enc_text_kernel(const TextArgs p) {
         }
       }
       asm volatile("" ::: "memory");
-      const TextMat& m = phase == TX_QKV ? x : y;
+      const TextMat m = phase == TX_QKV ? x : y;
       const auto rs = pieces(m);
       poll([&] {
         beside(m);
@@ -444,7 +454,7 @@ enc_text_kernel(const TextArgs p) {
     }
     const u32x2_t o{T::pack2(v[0], v[1]), T::pack2(v[2], v[3])};
     const TextMat sum = layer + 1 < p.layers ? TextMat{base + (size_t)(4 * h + f) * R * 2, S, 32} : TextMat{(char*)p.out, 32, (unsigned)h * 2};
-    const TextMat& C = phase == TX_QKV ? qkv : phase == TX_OUT ? y : phase == TX_UP ? mid : sum;
+    const TextMat C = phase == TX_QKV ? qkv : phase == TX_OUT ? y : phase == TX_UP ? mid : sum;
     if (out) tx_put(C.p + ostrip * C.strip + om * C.row + 8 * (tid & 3), __builtin_bit_cast(unsigned long long, o));
     if (!wide) {  // statistics of the values as stored
       float z[4];
@@ -597,11 +607,12 @@ DA_EXPORT long long da_enc_text_ws(int M, int h, int f, int layers, int D, int f
 // x [M, h] through the layers (pointers of TextLayer each, of the host): out [M, h] is the last layer's sum before its norm. One text, rows
 // cu[0] .. cu[1] - 1.
 static int enc_text(const void* x, const void* const* layers, int n, void* out, void* ws, const int* cu, int M, int h, int f, int D, float eps,
-                    float c, int f16, hipStream_t s) {
+                    float c, int f16, int* gave_up, int polls, hipStream_t s) {
   const long long bytes = da_enc_text_ws(M, h, f, n, D, f16);
   TextArgs a{};
   std::memcpy(a.L, layers, n * sizeof(TextLayer));
   a.x = (const bf16_t*)x; a.out = (bf16_t*)out; a.ws = (char*)ws; a.ticket = (int*)((char*)ws + bytes - 256); a.cu = cu;
+  a.gave_up = gave_up; a.polls = -polls;
   a.M = M; a.h = h; a.f = f; a.layers = n; a.eps = eps; a.c = c;
   // strips a task: with four fewer tasks read a block's activations and take its norm, with two a task has fewer weights (us, four / two: 32 rows
   // of 1024 columns, 24 layers 484 / 555, of 768, 12 209 / 216, of 512, 8 126 / 121, of 384, 12 178 / 168; 64 rows of 768 290 / 334, of 384
@@ -622,11 +633,11 @@ static int enc_text(const void* x, const void* const* layers, int n, void* out, 
 }
 
 DA_EXPORT int da_enc_text(const void* x, const void* const* layers, int n, void* out, void* ws, const int* cu, int M, int h, int f, int D,
-                         float eps, float c, int f16, void* stream) {
+                         float eps, float c, int f16, int* gave_up, int polls, void* stream) {
   const long long bytes = da_enc_text_ws(M, h, f, n, D, f16);
   if (!bytes || !x || !layers || !out || !ws || !cu) return (int)hipErrorInvalidValue;
   enc_text_empty_kernel<<<512, 256, 0, (hipStream_t)stream>>>((u32x4_t*)ws, bytes / 16, (u32x4_t*)out, M * h / 8);
-  return enc_text(x, layers, n, out, ws, cu, M, h, f, D, eps, c, f16, (hipStream_t)stream);
+  return enc_text(x, layers, n, out, ws, cu, M, h, f, D, eps, c, f16, gave_up, polls, (hipStream_t)stream);
 }
 
 // The whole encoder of such a text: ids and positions [M] to its pooled unit vector, out fp32 [h]. emb: word, position and type tables, their
@@ -634,16 +645,19 @@ DA_EXPORT int da_enc_text(const void* x, const void* const* layers, int n, void*
 // copy waits 18 us for, nor a text filled up to a length: a question 218 -> 200 us.
 DA_EXPORT int da_enc_text_pooled(const void* ids, const void* positions, const void* const* emb, const void* const* layers, int n, void* x, void* y,
                                 void* ws, const int* cu, int M, int h, int f, int D, float eps, float c, int mode, void* out, int f16,
-                                void* stream) {
+                                int* gave_up, int polls, void* stream) {
   const long long bytes = da_enc_text_ws(M, h, f, n, D, f16);
   if (!bytes || !ids || !positions || !emb || !layers || !x || !y || !ws || !cu || !out) return (int)hipErrorInvalidValue;
   hipStream_t s = (hipStream_t)stream;
   const bf16_t *const *e = (const bf16_t* const*)emb, *const *last = (const bf16_t* const*)layers + (size_t)12 * (n - 1);
   const auto begin = f16 ? enc_text_begin_kernel<F16T> : enc_text_begin_kernel<BF16T>;
   begin<<<M + 512, 256, 0, s>>>((const int*)ids, (const int*)positions, e[0], e[1], e[2], e[3], e[4], (bf16_t*)x, M, h, eps, (u32x4_t*)ws, bytes / 16);
-  const int err = enc_text(x, layers, n, y, ws, cu, M, h, f, D, eps, c, f16, s);
+  const int err = enc_text(x, layers, n, y, ws, cu, M, h, f, D, eps, c, f16, gave_up, polls, s);
   if (err) return err;
   const auto end = f16 ? enc_text_end_kernel<F16T> : enc_text_end_kernel<BF16T>;
   end<<<1, 64 * TX_WAVES, 0, s>>>((const bf16_t*)y, last[10], last[11], cu, M, h, eps, mode, (float*)out);
   return (int)hipGetLastError();
 }
+
+// The device's address of pinned host memory.
+DA_EXPORT int da_host_address(void* host, void** out) { return (int)hipHostGetDevicePointer(out, host, 0); }

@@ -68,8 +68,9 @@ _SIGS = {
                        + [c_void_p] * 5 + [c_int] * 5 + [c_void_p],
     "da_gemm_dk_ws": [c_int] * 3,
     "da_enc_text_ws": [c_int] * 6,
-    "da_enc_text_pooled": [c_void_p] * 4 + [c_int] + [c_void_p] * 4 + [c_int] * 4 + [c_float, c_float, c_int, c_void_p, c_int, c_void_p],
-    "da_enc_text": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p] + [c_int] * 4 + [c_float, c_float, c_int, c_void_p],
+    "da_enc_text_pooled": [c_void_p] * 4 + [c_int] + [c_void_p] * 4 + [c_int] * 4 + [c_float, c_float, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p],
+    "da_host_address": [c_void_p, ctypes.POINTER(c_void_p)],
+    "da_enc_text": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p] + [c_int] * 4 + [c_float, c_float, c_int, c_void_p, c_int, c_void_p],
     "da_gemm_dk_parts": [c_int],
     "da_gemm_dk_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 7 + [c_void_p],
     "da_enc_rows": [c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 5
@@ -659,6 +660,31 @@ def enc_text_fits(M: int, hidden: int, ffn: int, layers: int, heads: int, texts:
             and hidden in ((64 * heads,) if f16 else (32 * heads, 64 * heads)) and texts == 1)
 
 
+TEXT_POLLS = 1 << 22  # readings of a wait in csrc/encoder_text.hip, of 1 us and more each
+
+
+class TextWaits:
+    """Where an encoder's ``enc_text`` launches say that a wait ran out (no order of their workgroups does that; the result is NaNs then): a
+    pinned word of the host, which a reader sees once it has waited for the launch."""
+
+    def __init__(self):
+        self._word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self._value, at = c_int.from_address(self._word.data_ptr()), c_void_p()
+        _check(lib().da_host_address(self._word.data_ptr(), ctypes.byref(at)), "host_address")
+        self.at, self.launches = at.value, 0
+
+    def begin(self) -> None:
+        """Before a launch."""
+        self.check()
+        self.launches += 1
+
+    def check(self) -> None:
+        """KernelError, once, if a wait ran out in a launch that has run since the last check."""
+        if self._value.value:
+            self._value.value = 0
+            raise KernelError("enc_text: a wait ran out, the text's embedding is NaNs")
+
+
 def _text_layers(layers, h: int, f: int, is_cuda):
     """The layers' pointers (csrc/encoder_text.hip, TextLayer), and how many."""
     shapes = {"wqkv": (3 * h, h), "bqkv": (3 * h,), "wo": (h, h), "bo": (h,), "ln1_g": (h,), "ln1_b": (h,), "w1": (f, h), "b1": (f,),
@@ -673,9 +699,12 @@ def _text_layers(layers, h: int, f: int, is_cuda):
     return (c_void_p * len(table))(*table), len(layers)
 
 
-def enc_text(x, layers, cu, heads: int, eps: float):
+def enc_text(x, layers, cu, heads: int, eps: float, waits: TextWaits | None = None):
     """All layers of one text of up to 64 rows in one launch (csrc/encoder_text.hip): x [M, h] -> the last layer's sum before
-    its norm (rows behind the text: zeros). layers: dicts of wqkv, bqkv, wo, bo, ln1_g, ln1_b, w1, b1, w2, b2, ln2_g, ln2_b."""
+    its norm (rows behind the text: zeros). layers: dicts of wqkv, bqkv, wo, bo, ln1_g, ln1_b, w1, b1, w2, b2, ln2_g, ln2_b.
+    waits: told of a wait that runs out, and asked first about the launches before."""
+    if waits is not None:
+        waits.begin()
     f16 = x.dtype == torch.float16
     is_cuda = _f16_cuda if f16 else _bf16_cuda
     is_cuda(x, "x"); _i32(cu, "cu_seqlens")
@@ -686,15 +715,15 @@ def enc_text(x, layers, cu, heads: int, eps: float):
     ws = torch.empty(int(lib().da_enc_text_ws(M, h, f, n, D, f16)), dtype=torch.uint8, device=x.device)
     out = torch.empty_like(x)
     _check(lib().da_enc_text(_ptr(x), table, n, _ptr(out), _ptr(ws), _ptr(cu), M, h, f, D, float(eps), math.log2(math.e) / math.sqrt(D), f16,
-                             _stream()), "enc_text")
+                             waits and waits.at, TEXT_POLLS, _stream()), "enc_text")
     return out
 
 
 class TextPlan:
-    """An encoder's weights (word, pos, type, emb_ln_g, emb_ln_b, layers) as ``enc_text_pooled`` takes them: the tensors, checked once."""
+    """An encoder's weights (word, pos, type, emb_ln_g, emb_ln_b, layers) as ``enc_text_pooled`` takes them: the tensors, checked once. waits as ``enc_text``'s."""
 
-    def __init__(self, w: dict, heads: int, eps: float):
-        self.f16 = w["word"].dtype == torch.float16
+    def __init__(self, w: dict, heads: int, eps: float, waits: TextWaits | None = None):
+        self.waits, self.f16 = waits, w["word"].dtype == torch.float16
         is_cuda = _f16_cuda if self.f16 else _bf16_cuda
         self.emb, self.weights = [w[k] for k in ("word", "pos", "type", "emb_ln_g", "emb_ln_b")], w["layers"]
         self.h, self.f, self.D, self.eps = w["word"].shape[1], self.weights[0]["w1"].shape[0], w["word"].shape[1] // heads, float(eps)
@@ -710,6 +739,8 @@ class TextPlan:
 def enc_text_pooled(plan: TextPlan, tokens, mode: int) -> torch.Tensor:
     """The whole encoder of one text of n <= 64 tokens, in three launches: the unit vector of its pooled rows (mode as pool_l2norm's),
     fp32 [1, h]. tokens int32 [2 n + 2]: ids, positions, 0 and n."""
+    if plan.waits is not None:
+        plan.waits.begin()
     _i32(tokens, "tokens")
     n, h = tokens.numel() // 2 - 1, plan.h
     _req(1 <= n <= 64 and tokens.numel() == 2 * n + 2 and tokens.device == plan.emb[0].device, "enc_text_pooled tokens")
@@ -718,7 +749,8 @@ def enc_text_pooled(plan: TextPlan, tokens, mode: int) -> torch.Tensor:
     out = torch.empty((1, h), dtype=torch.float32, device=tokens.device)
     at, t = ws.data_ptr(), tokens.data_ptr()
     _check(lib().da_enc_text_pooled(t, t + 4 * n, plan.emb_table, plan.table, plan.n, at + size, at + size + row, at, t + 8 * n, n, h, plan.f, plan.D,
-                                    plan.eps, math.log2(math.e) / math.sqrt(plan.D), mode, out.data_ptr(), plan.f16, _raw_stream()), "enc_text_pooled")
+                                    plan.eps, math.log2(math.e) / math.sqrt(plan.D), mode, out.data_ptr(), plan.f16,
+                                    plan.waits and plan.waits.at, TEXT_POLLS, _raw_stream()), "enc_text_pooled")
     return out
 
 

@@ -136,7 +136,7 @@ def test_whole_text(h, f, heads, pooling, dtype):
         ids, pos, cu = (torch.tensor(t, dtype=torch.int32, device="cuda") for t in (seq, list(range(n)), [0, n]))
         with pytest.MonkeyPatch.context() as m:
             m.setattr(K, "enc_text_fits", lambda *a: False)
-            m.setattr(enc, "_one_row", lambda rows: False)
+            m.setattr(BertEncoder, "_one_row", lambda self, rows: False)
             want = enc._pool(enc.forward(ids, pos, cu, n), cu)
         assert v.shape == want.shape and v.dtype == torch.float32
         assert torch.equal(v, want) or dtype == "fp16" or not K.attn_ln_fit(n, h, heads, 1)
@@ -183,3 +183,48 @@ def test_beside_one_another():
                 got[i].append(K.enc_text(x, L, c, 12, 1e-12))
     torch.cuda.synchronize()
     assert all(torch.equal(g, w) for gs, w in zip(got, want) for g in gs)
+
+
+def test_a_wait_that_runs_out_is_told(monkeypatch):
+    """A wait that ends before its words are there (here after one reading) leaves NaNs, and the next check or launch raises; later
+    texts are as ever. Waits that do not end early say nothing, nor do NaNs that the input makes."""
+    enc = BertEncoder(EncoderConfig("e", vocab=100, hidden=768, layers=12, heads=12, ffn=3072), "cuda")
+    enc.prepare_graphs()
+    seq = list(range(5, 26))
+    want = enc.encode_one(seq)
+    torch.cuda.synchronize()
+    enc.check()
+    for call in (enc.encode_one, lambda s: enc.encode_packed([s])):
+        with monkeypatch.context() as m:
+            m.setattr(K, "TEXT_POLLS", 1)
+            v = call(seq)
+            torch.cuda.synchronize()
+        assert bool(v.isnan().any())
+        with pytest.raises(K.KernelError):
+            enc.check()
+        enc.check()
+        assert torch.equal(enc.encode_one(seq), want)
+    with monkeypatch.context() as m:
+        m.setattr(K, "TEXT_POLLS", 1)
+        enc.encode_one(seq)
+        torch.cuda.synchronize()
+    with pytest.raises(K.KernelError):  # (who did not ask hears of it at the next text)
+        enc.encode_one(seq)
+    assert torch.equal(enc.encode_one(seq), want)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("where", ["x", "bqkv", "bo", "b1", "b2", "ln1_b"])
+def test_words_of_set_bits(where, dt):
+    """NaNs of all bits set, as words that are not there yet have them, are values like others: no wait waits for them."""
+    L, r = make(128, 256, 2, 4, dt)
+    x, cu, waits = r(17, 128), torch.tensor([0, 17], dtype=torch.int32, device="cuda"), K.TextWaits()
+    t = x[3] if where == "x" else L[1][where]
+    t.view(torch.int16)[:] = -1
+    a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    a.record()
+    got = K.enc_text(x, L, cu, 2, 1e-12, waits)
+    b.record()
+    torch.cuda.synchronize()
+    waits.check()
+    assert a.elapsed_time(b) < 1000 and bool(got[3].isnan().all())
