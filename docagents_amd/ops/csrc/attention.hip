@@ -2198,13 +2198,22 @@ static int launch_fa_pipe(const void* q, const void* k, const void* v, int ldq, 
 
 // D = 128: 256 queries a workgroup, two waves a SIMD that share the staged tiles, or 128 and one. A tile's chain (scores, exponentials,
 // sums) is what a workgroup takes its time for, so one wave a SIMD is nearly twice as fast where the chip has workgroups to spare,
-// and shorter blocks leave less behind the causal diagonal; with many blocks of long prompts the tiles' second reading
-// costs more. Both give the same bits. us, 8 waves / 4, 32 heads over 8: 139 + 138 queries behind 320 keys 21.9 / 18.6, 277 16.2 / 12.5,
-// 820 31.1 / 25.0, 1750 62.2 / 52.0, 1900 + 2000 + 1700 behind 256 171 / 161, 64 x 100 behind 256 129 / 80, 2048 70.5 / 59.6, 2560 88 / 79,
-// 2816 94 / 86; 4 x 2048 190 / 191, 3072 102 / 102, 3600 135 / 146, 8192 560 / 590, 2 x 2560 140 / 142, 6 x 3000 620 / 630.
-static bool fa_eight_waves(int max_seqlen, int H, int B) {
-  const long blocks = (long)((max_seqlen + 255) / 256) * H * B;
-  return max_seqlen > 2816 || (max_seqlen > 2048 && blocks > 400);
+// and shorter blocks leave less behind the causal diagonal and the texts' ends; with many blocks the tiles' second reading costs more, the more
+// the longer the shared head (pre) that all of them walk and the less the diagonal is of that. Both give the same bits.
+// us, 8 waves / 4, 32 heads over 8: 139 + 138 queries behind 320 keys 21.9 / 18.6, 277 16.2 / 12.5, 820 31.1 / 25.0, 1750 62.2 / 52.0, 1900 + 2000 +
+// 1700 behind 256 171 / 161, 64 x 100 behind 256 129 / 80, 2048 65 / 57, behind 1024 100 / 93, 2560 82 / 73, 2816 91 / 83; 3072 99 / 100,
+// 3600 135 / 146, 8192 560 / 590, 2 x 2560 136 / 139, 6 x 3000 620 / 630.
+// Blocks that have a CU each: 700 behind 4096 151 / 127, behind 16384 533 / 487. One round of both, a long head: 1500 behind 4096 181 / 177, behind 16384
+// 556 / 597, 2048 behind 4096 202 / 208; 64 heads over 8, 507 + 350 behind 3000 126 / 137; 40 heads, 481 + 360 + 250 behind 3000 122 / 133. More of
+// them: 2 x 2048 behind 1024 and 4096 157 / 174 and 370 / 402, 16 x 1500 864 / 904 and 2111 / 2269, 2560 behind 1024 122 / 142; of shorter texts by
+// their lengths, 8 to 882 behind 3000 480 / 402, 16 to 484 875 / 792, 16 x 700 behind 4096 950 / 1032.
+static bool fa_eight_waves(int max_seqlen, int H, int B, int pre_len) {
+  const auto blocks = [&](int n, int rows) { return (long)((n + rows - 1) / rows) * H * B; };
+  if (max_seqlen > 2816 || (max_seqlen > 2048 && blocks(max_seqlen, 256) > 400)) return true;
+  const int some = B > 1 ? (max_seqlen * 3 + 3) / 4 : max_seqlen;  // (the others' lengths are not known here)
+  if (blocks(some, 128) <= 256) return false;
+  if (blocks(some, 256) <= 256) return pre_len > max_seqlen / 2 * 3;
+  return max_seqlen > 1408 && pre_len >= 512;
 }
 
 // pre_k / pre_v: shared-prefix K/V of KV head 0 in a cache slot (nullptr / pre_len 0: none),
@@ -2241,7 +2250,7 @@ DA_EXPORT int da_flash_attn_v2(const void* q, const void* k, const void* v, int 
   if (D == 64 && !causal && pre_len == 0 &&
       launch_fa_enc<BF16T>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv, sl2e, o, ldo, s))
     return (int)hipGetLastError();
-  if (D == 128 && fa_eight_waves(max_seqlen, H, B))
+  if (D == 128 && fa_eight_waves(max_seqlen, H, B, pre_len))
     return launch_fa2<8, 1>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv, D, causal, sl2e, o, ldo, pre, s);
   return launch_fa2<4, 1>(q, k, v, ldq, ldk, ldv, cu_seqlens, B, max_seqlen, H, Hkv, D, causal, sl2e, o, ldo, pre, s);
 }

@@ -12,7 +12,9 @@ DEV = "cuda"
 
 # one query, a block of 128 and one more, of 256 and one more; four waves to 2048 queries, to 2816 of few blocks, and eight
 @pytest.mark.parametrize("H,Hkv,lens,P", [(4, 2, [1], 0), (4, 1, [128, 5, 129], 70), (4, 4, [256, 257], 0), (4, 2, [2048], 33),
-                                          (4, 2, [2049, 3], 0), (41, 41, [2100, 9], 0), (4, 1, [2816], 0), (4, 1, [2817], 0)])
+                                          (4, 2, [2049, 3], 0), (41, 41, [2100, 9], 0), (4, 1, [2816], 0), (4, 1, [2817], 0),
+                                          # behind a long head: one round of blocks (128 x 2 of 256 queries) and more
+                                          (64, 8, [507, 130], 759), (64, 8, [507, 130], 760), (64, 64, [1409], 511), (64, 8, [1409], 512)])
 def test_prefill_of_heads_of_128(H, Hkv, lens, P):
     g = torch.Generator(device=DEV).manual_seed(sum(lens) + H)
     D, T = 128, sum(lens)
