@@ -1639,7 +1639,7 @@ def topk_ranges(X, Qv, ranges, range_off, K: int, thr: float, max_rows: int, slo
     device or both arrays of the host, or lists of their numbers: a few ride in the launch's arguments, more go in one copy);
     max_rows = max total rows of any query (host int) — sets the split count: rows_per_split rows of a query per
     workgroup (default: ``_rows_per_split``)."""
-    rows, Q, table = rows_per_split or _rows_per_split(max_rows, Qv.shape[0]), Qv.shape[0], None
+    rows, Q, table = rows_per_split or _rows_per_split(max_rows, Qv.shape[0], K), Qv.shape[0], None
     if isinstance(ranges, list):
         _req(len(range_off) == Q + 1 and len(ranges) == 2 * range_off[-1], "range_off length")
         size = len(range_off) + len(ranges)
@@ -1672,18 +1672,22 @@ def topk_lists(X, Qv, lists, list_off, K: int, thr: float, mean_rows: int, max_r
     _i32(lists, "lists"); _i32(list_off, "list_off")
     _req(lists.dim() == 2 and lists.shape[0] == Qv.shape[0], "lists [Q, probes]")
     # workgroups past a query's rows end at once, but lists of very uneven length must not make too many of them
-    rows = max(_rows_per_split(mean_rows, Qv.shape[0]), math.ceil(max_rows / 512 / 64) * 64)
+    rows = max(_rows_per_split(mean_rows, Qv.shape[0], K), math.ceil(max_rows / 512 / 64) * 64)
     return _ranges(X, Qv, list_off, None, lists, K, thr, max_rows, slots, bitmap, rows, ids)
 
 
-def _rows_per_split(rows: int, Q: int) -> int:
+def _rows_per_split(rows: int, Q: int, K: int) -> int:
     """Rows of a query per workgroup of the range scan: what gives about 1024 workgroups (4 per CU: a workgroup keeps
     48 KB of rows on their way), from one step of the kernel (64) to 512; half a step where there are few rows in all (us, 64 / 32: one
-    query's 384 rows of 768 12.2 / 10.5, 64 queries of 144 12.8 / 11.8; 6250 rows of 24 queries 47.4 / 62.7)."""
-    return 32 if rows * Q <= RANGE_SMALL else min(512, max(64, math.ceil(rows * Q / 1024 / 64) * 64))
+    query's 384 rows of 768 12.2 / 10.5, 64 queries of 144 12.8 / 11.8; 6250 rows of 24 queries 47.4 / 62.7) and twice the lists are
+    still few to put together (on the device, of 384 columns: K = 10, 1500 rows, 470 candidates of half steps 20.6 / 18.1, 2200, 690 17.4 /
+    18.2; K = 20, 600, 380 21.0 / 18.8, 1500, 940 19.9 / 22.8; K = 32, 300, 320 22.5 / 19.4, 600, 608 19.9 / 25.0, 6400, 6400 40 / 48)."""
+    half = rows * Q <= RANGE_SMALL and math.ceil(rows / 32) * K <= RANGE_HALF
+    return 32 if half else min(512, max(64, math.ceil(rows * Q / 1024 / 64) * 64))
 
 
 RANGE_SMALL = 10240  # rows of all queries up to which a workgroup of the range scan takes half a step
+RANGE_HALF = 512     # and candidates of a query that half steps leave
 RANGE_JOIN = 256     # candidates of a query up to which its last workgroup puts them together
 
 

@@ -12,7 +12,7 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("d", [384, 1024])
-@pytest.mark.parametrize("rows,Kk", [(1, 5), (31, 32), (32, 1), (33, 32), (64, 5), (65, 32), (256, 32), (257, 32), (700, 5)])
+@pytest.mark.parametrize("rows,Kk", [(1, 5), (31, 32), (32, 1), (33, 32), (64, 5), (65, 32), (256, 32), (257, 32), (700, 5), (512, 32), (513, 32)])
 def test_lists_that_meet_in_the_launch(d, rows, Kk):
     """One row, half a step, a step and one row more, one workgroup, 256 candidates and one list more; queries with fewer
     rows, and none; by ranges of the host and by lists, with removed rows; the same launch again finds its counters at zero."""
@@ -47,6 +47,13 @@ def test_lists_that_meet_in_the_launch(d, rows, Kk):
                 assert torch.allclose(dots[i, (got[i, :m] - 1) // 3], want[:m], rtol=0, atol=d * 2.0 ** -22)
                 assert got[i, :m].unique().numel() == m and bool(torch.isin(got[i, :m], ids[r]).all())
                 assert got[i, m:].tolist() == [-1] * (Kk - m) and bool((s[i, m:] == -float("inf")).all())
+
+
+@pytest.mark.parametrize("rows,Q,Kk,split", [(512, 1, 32, 32), (513, 1, 32, 64), (6400, 1, 32, 64), (1600, 3, 10, 32), (10240, 1, 1, 32), (10241, 1, 1, 64),
+                                             (10240, 1, 2, 64), (2000, 10, 5, 64), (65536, 1, 5, 64), (65537, 1, 5, 128)])
+def test_half_steps(rows, Q, Kk, split):
+    """Half steps for few rows in all, and no more candidates of them than are soon put together."""
+    assert K._rows_per_split(rows, Q, Kk) == split
 
 
 def test_streams_have_counters_of_their_own():
