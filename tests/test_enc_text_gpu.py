@@ -78,7 +78,8 @@ def test_layers(M, h, f, heads, layers, cu, dt):
         assert torch.equal(got, one) or dt == torch.float16 or not K.attn_ln_fit(M, h, heads, 1)
         assert e < 1.25 * e1 + u and e < 4 * (8 * layers) ** 0.5 * u, (e, e1)
         for _ in range(10):
-            assert torch.equal(K.enc_text(x, L, c, heads, 1e-12)[cu[0]:cu[1]].double(), got)
+            again = K.enc_text(x, L, c, heads, 1e-12)
+            assert torch.equal(again[cu[0]:cu[1]].double(), got) and not bool(again[cu[1]:].any())  # (rows behind the text: zeros)
 
 
 @pytest.mark.parametrize("T", [16, 32, 64])
@@ -156,8 +157,6 @@ def test_what_it_refuses():
     L, r = make(128, 256, 2, 4, torch.bfloat16)
     cu, x = torch.tensor([0, 8], dtype=torch.int32, device="cuda"), r(8, 128)
     K.enc_text(x, L, cu, 2, 1e-12)
-    off = torch.zeros(129, dtype=torch.bfloat16, device="cuda")[1:]  # (vectors may lie anywhere)
-    assert torch.equal(K.enc_text(x, [{**L[0], "bo": off}, *L[1:]], cu, 2, 1e-12), K.enc_text(x, [{**L[0], "bo": off.clone()}, *L[1:]], cu, 2, 1e-12))
     for bad in ({"wo": L[0]["wo"].half()}, {"wo": L[0]["wo"].cpu()}, {"w1": L[0]["w1"][:, ::2]}, {"bqkv": L[0]["bo"]}):
         with pytest.raises(ValueError):
             K.enc_text(x, [{**L[0], **bad}, *L[1:]], cu, 2, 1e-12)
@@ -228,3 +227,31 @@ def test_words_of_set_bits(where, dt):
     torch.cuda.synchronize()
     waits.check()
     assert a.elapsed_time(b) < 1000 and bool(got[3].isnan().all())
+
+
+def shifted(t):
+    """The same values two bytes behind a 16-B address."""
+    out = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape).copy_(t)
+    assert out.data_ptr() % 16 == 2
+    return out
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("name", ["bqkv", "bo", "b1", "b2", "ln1_g", "ln1_b", "ln2_g", "ln2_b"])
+def test_vectors_at_any_address(name, dt):
+    """Vectors of the layers may lie anywhere, as the products one by one take them."""
+    L, r = make(320, 640, 5, 4, dt)
+    cu, x = torch.tensor([0, 19], dtype=torch.int32, device="cuda"), r(19, 320)
+    assert torch.equal(K.enc_text(x, [{**one, name: shifted(one[name])} for one in L], cu, 5, 1e-12), K.enc_text(x, L, cu, 5, 1e-12))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("pooling", ["cls", "mean"])
+def test_embeddings_at_any_address(dtype, pooling):
+    """So may the embeddings' tables, their norm and the last one."""
+    enc = BertEncoder(EncoderConfig("e", vocab=50, hidden=320, layers=4, heads=5, ffn=640, pooling=pooling), "cuda", dtype=dtype)
+    w = {k: shifted(v) if k != "layers" else v[:-1] + [{**v[-1], **{n: shifted(v[-1][n]) for n in ("ln2_g", "ln2_b")}}] for k, v in enc.w.items()}
+    seq = [3, 49, 7, 7, 20]
+    tokens = torch.tensor([*seq, *range(5), 0, 5], dtype=torch.int32, device="cuda")
+    a, b = (K.enc_text_pooled(K.TextPlan(t, 5, 1e-12), tokens, enc._pool_mode) for t in (w, enc.w))
+    assert torch.equal(a, b) and torch.equal(a, enc.encode_one(seq))
