@@ -23,7 +23,7 @@
 // us, launches one by one / this, bf16: 12 layers of 384 x 1536, 16, 32, 48 and 64 rows 215 / 142, 217 / 156, 242 / 174 and 256 / 177, of 768 x 3072
 // 253 / 170, 274 / 193, 346 / 231 and 347 / 270, 24 of 1024 x 4096, 16, 32, 36 and 64 rows 670 / 387, 730 / 461, 868 / 618 and 901 / 752; 4 of 768,
 // 32 rows 93 / 74, 2 48 / 44. (That a wait which runs out is told costs 0.6 %: 21 rows of 768 columns 187.3 -> 190.0. Matrices are chosen by
-// value: by reference the scalars that go to lanes and back are 55 to 73 a variant for 50 to 59.)
+// value: by reference the scalars that go to lanes and back are 55 to 73 a variant for 52 to 64.)
 #include <cstring>
 
 #include "gemm.h"
@@ -604,6 +604,19 @@ DA_EXPORT long long da_enc_text_ws(int M, int h, int f, int layers, int D, int f
   return layers * (R * 2 * (5ll * h + f) + 2 * (h / 16) * R * 8) + 256;  // (and the ticket)
 }
 
+// Workgroups: as many as two neighbouring products have tasks, whose weights travel while the product before is taken; each has a CU to itself, so
+// that with 256 nothing else runs until the last task. us, 256 / 192 / 144 workgroups, 12 layers of 768, 16 rows 170 / 171 / 170 (144 of two
+// products), 32 rows 192 / 191 / 245 (192), 64 rows 270 / 302 / 416; of 384, 32 rows 156 / 155 / 151 (144), 48 174 / 173 / 169 (144), 64 176 / 172 /
+// 193 (192). Wider ones take all: their weights are longer on the way (24 of 1024, 16 rows 385 / 413 / 470, 32 460 / 586 / 683).
+// Beside decode steps (of a 3.8B, one row; a question of 21 tokens and 768 columns after another, 5 ms apart / at once; the launches one by one):
+// a step 1.80 / 7.5 ms with 256, 1.78 / 3.2 with 192 (1.76 / 1.95), a question 250 / 232 us, 258 / 233 (597 / 573). Of 1024 columns, 256: a step 1.90 / 15.7
+// ms (1.81 / 2.13), a question 524 / 497 us (1346 / 1324).
+static int enc_text_grid(int M, int h, int f, int ns) {
+  const int mb = (M + 15) / 16, out = h / 16 * mb, qkv = 3 * out / ns, up = f / 16 * mb / ns;
+  const int two = out + (qkv > up ? qkv : up);
+  return h > 768 || two > 256 ? 256 : two < 96 ? 96 : (two + 15) / 16 * 16;
+}
+
 // x [M, h] through the layers (pointers of TextLayer each, of the host): out [M, h] is the last layer's sum before its norm. One text, rows
 // cu[0] .. cu[1] - 1.
 static int enc_text(const void* x, const void* const* layers, int n, void* out, void* ws, const int* cu, int M, int h, int f, int D, float eps,
@@ -617,13 +630,14 @@ static int enc_text(const void* x, const void* const* layers, int n, void* out, 
   // strips a task: with four fewer tasks read a block's activations and take its norm, with two a task has fewer weights (us, four / two: 32 rows
   // of 1024 columns, 24 layers 484 / 555, of 768, 12 209 / 216, of 512, 8 126 / 121, of 384, 12 178 / 168; 64 rows of 768 290 / 334, of 384
   // 194 / 204; 16 rows of 768 198 / 173, with one 191)
-#define ENC_TEXT(T, DD)                                                                \
-  do {                                                                                 \
-    if (M <= 16) enc_text_kernel<T, 1, DD, 2><<<256, 64 * TX_WAVES, 0, s>>>(a);        \
-    else if (M > 48) enc_text_kernel<T, 4, DD, 4><<<256, 64 * TX_WAVES, 0, s>>>(a);    \
-    else if (M > 32) enc_text_kernel<T, 3, DD, 4><<<256, 64 * TX_WAVES, 0, s>>>(a);    \
-    else if (h <= 512) enc_text_kernel<T, 2, DD, 2><<<256, 64 * TX_WAVES, 0, s>>>(a);  \
-    else enc_text_kernel<T, 2, DD, 4><<<256, 64 * TX_WAVES, 0, s>>>(a);                \
+  const int ns = M <= 16 || (M <= 32 && h <= 512) ? 2 : 4, grid = enc_text_grid(M, h, f, ns);
+#define ENC_TEXT(T, DD)                                                                 \
+  do {                                                                                  \
+    if (M <= 16) enc_text_kernel<T, 1, DD, 2><<<grid, 64 * TX_WAVES, 0, s>>>(a);        \
+    else if (M > 48) enc_text_kernel<T, 4, DD, 4><<<grid, 64 * TX_WAVES, 0, s>>>(a);    \
+    else if (M > 32) enc_text_kernel<T, 3, DD, 4><<<grid, 64 * TX_WAVES, 0, s>>>(a);    \
+    else if (ns == 2) enc_text_kernel<T, 2, DD, 2><<<grid, 64 * TX_WAVES, 0, s>>>(a);   \
+    else enc_text_kernel<T, 2, DD, 4><<<grid, 64 * TX_WAVES, 0, s>>>(a);                \
   } while (0)
   if (D == 32) ENC_TEXT(BF16T, 32);
   else if (f16) ENC_TEXT(F16T, 64);
