@@ -20,11 +20,13 @@
 // MFMAs and the waves' sums 0.6 - 0.9, epilogue 0.7. (A row block a task, also in the wide products: the norm of 32 rows in one took 0.4 longer.
 // Waiting for one word first, or for one of the product before, so that waits read less: 165 - 184 us for 172, 16 rows of 768 columns.)
 //
-// us, launches one by one / this, bf16: 12 layers of 384 x 1536, 16, 32, 48 and 64 rows 215 / 142, 217 / 156, 242 / 174 and 256 / 177, of 768 x 3072
-// 253 / 170, 274 / 193, 346 / 231 and 347 / 270, 24 of 1024 x 4096, 16, 32, 36 and 64 rows 670 / 387, 730 / 461, 868 / 618 and 901 / 752; 4 of 768,
-// 32 rows 93 / 74, 2 48 / 44. (That a wait which runs out is told costs 0.6 %: 21 rows of 768 columns 187.3 -> 190.0. Matrices are chosen by
-// value: by reference the scalars that go to lanes and back are 55 to 73 a variant for 52 to 64.)
+// Each phase has code of its own: as one loop body with the phase a value, its choices and the scalars that went to lanes and back were on the chain
+// (12 layers of 768, 21 rows 187.5 -> 175.0, 24 of 1024, 32 rows 460 -> 446). That a wait which runs out is told costs 0.6 %.
+// us, launches one by one / this, bf16: 12 layers of 384 x 1536, 16, 32, 48 and 64 rows 215 / 132, 217 / 140, 242 / 158 and 255 / 164, of 768 x 3072
+// 253 / 161, 274 / 178, 346 / 217 and 348 / 253, 24 of 1024 x 4096, 16, 32, 36 and 64 rows 673 / 370, 731 / 446, 868 / 592 and 899 / 705; 4 of 768,
+// 32 rows 94 / 69, 2 48 / 42.
 #include <cstring>
+#include <type_traits>
 
 #include "gemm.h"
 
@@ -117,23 +119,10 @@ enc_text_kernel(const TextArgs p) {
   auto take = [&](int wave) __attribute__((always_inline)) {
     if (threadIdx.x == wave * 64) snext = __hip_atomic_fetch_add(p.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
   };
-  for (take(0);;) {
-    tx_barrier();  // (the task before this one is done with LDS)
-    const int t = __builtin_amdgcn_readfirstlane(snext);
-    if (t >= total) {
-      if (threadIdx.x == 0 && sgave && p.gave_up) __hip_atomic_store(p.gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-      return;
-    }
-    // ---- the task ----
-    const int layer = t / per;
-    int index = t - layer * per, phase = TX_QKV;
-#pragma unroll
-    for (int e = TX_QKV; e < TX_DOWN; ++e)
-      if (phase == e && index >= tasks(e)) {
-        index -= tasks(e);
-        phase = e + 1;
-      }
-    const bool wide = !(phase & 1);
+  // A task of the phase, which is a constant: each has code of its own.
+  auto task = [&](auto of, const int layer, const int index) __attribute__((always_inline)) {
+    constexpr int phase = decltype(of)::value;
+    constexpr bool wide = !(phase & 1);
     const int strip = index / MB * (wide ? NS : 1), m0 = index % MB * 16;
     int lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane));  // (addresses of every phase kept from task to task would not fit the registers)
@@ -423,7 +412,7 @@ enc_text_kernel(const TextArgs p) {
     }
     tx_barrier();
     take(TX_WAVES - 1);
-    if (!own) continue;
+    if (!own) return;
 
     // ---- the result ----
     const float* rd = &red[0][4 * tid];
@@ -466,6 +455,29 @@ enc_text_kernel(const TextArgs p) {
       for (int e = 0; e < 4; ++e) d = fmaf(z[e] - m, z[e] - m, d);
       d = tx_sum4(d);
       if (out && (tid & 3) == 0) tx_put((phase == TX_OUT ? st1 : st1 + hs * R) + ((om >> 2) * hs + (strip & 3) * (hs / 4) + (strip >> 2)) * 4 + (om & 3), __builtin_bit_cast(unsigned long long, float2{m, d}));
+    }
+  };
+  for (take(0);;) {
+    tx_barrier();  // (the task before this one is done with LDS)
+    const int t = __builtin_amdgcn_readfirstlane(snext);
+    if (t >= total) {
+      if (threadIdx.x == 0 && sgave && p.gave_up) __hip_atomic_store(p.gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      return;
+    }
+    // ---- the task ----
+    const int layer = t / per;
+    int index = t - layer * per, phase = TX_QKV;
+#pragma unroll
+    for (int e = TX_QKV; e < TX_DOWN; ++e)
+      if (phase == e && index >= tasks(e)) {
+        index -= tasks(e);
+        phase = e + 1;
+      }
+    switch (phase) {
+      case TX_QKV: task(std::integral_constant<int, TX_QKV>{}, layer, index); break;
+      case TX_OUT: task(std::integral_constant<int, TX_OUT>{}, layer, index); break;
+      case TX_UP: task(std::integral_constant<int, TX_UP>{}, layer, index); break;
+      default: task(std::integral_constant<int, TX_DOWN>{}, layer, index);
     }
   }
 }
@@ -605,12 +617,12 @@ DA_EXPORT long long da_enc_text_ws(int M, int h, int f, int layers, int D, int f
 }
 
 // Workgroups: as many as two neighbouring products have tasks, whose weights travel while the product before is taken; each has a CU to itself, so
-// that with 256 nothing else runs until the last task. us, 256 / 192 / 144 workgroups, 12 layers of 768, 16 rows 170 / 171 / 170 (144 of two
-// products), 32 rows 192 / 191 / 245 (192), 64 rows 270 / 302 / 416; of 384, 32 rows 156 / 155 / 151 (144), 48 174 / 173 / 169 (144), 64 176 / 172 /
-// 193 (192). Wider ones take all: their weights are longer on the way (24 of 1024, 16 rows 385 / 413 / 470, 32 460 / 586 / 683).
-// Beside decode steps (of a 3.8B, one row; a question of 21 tokens and 768 columns after another, 5 ms apart / at once; the launches one by one):
-// a step 1.80 / 7.5 ms with 256, 1.78 / 3.2 with 192 (1.76 / 1.95), a question 250 / 232 us, 258 / 233 (597 / 573). Of 1024 columns, 256: a step 1.90 / 15.7
-// ms (1.81 / 2.13), a question 524 / 497 us (1346 / 1324).
+// that with 256 nothing else runs until the last task. us, 256 / 192 / 144 workgroups, 12 layers of 768, 16 rows 157 / 157 / 160 (144 of two
+// products), 32 rows 180 / 178 / 223 (192), 64 rows 253 / 279 / 382; of 384, 32 rows 143 / 142 / 140 (144), 48 162 / 162 / 159 (144), 64 168 / 164 /
+// 182 (192). Wider ones take all: their weights are longer on the way (24 of 1024, 16 rows 369 / 391 / 440, 32 446 / 545 / 631).
+// Beside decode steps (of a 3.8B, one row, 1.72 ms alone; questions of 21 tokens and 768 columns 5 ms apart / one upon another; the launches one by one):
+// a step 1.80 / 6.8 ms with 256, 1.77 / 3.3 with 192 (1.76 / 1.95), a question 247 / 222 us, 251 / 219 (597 / 573). Of 1024 columns: a step 1.90 / 15.1 ms
+// with 256, 1.85 / 4.0 with 192 (1.81 / 2.13), a question 498 / 478 us, 623 / 608 (1346 / 1324).
 static int enc_text_grid(int M, int h, int f, int ns) {
   const int mb = (M + 15) / 16, out = h / 16 * mb, qkv = 3 * out / ns, up = f / 16 * mb / ns;
   const int two = out + (qkv > up ? qkv : up);

@@ -131,12 +131,11 @@ def test_searches_over_lists_carry_no_table(tmp_path):
 
 
 def test_short_texts_keep_their_vectors(tmp_path):
-    """A short text's layers in one launch: 16 waves have 128 vector registers each, all of them used. Scalars go to lanes and back (52 - 64 of
+    """A short text's layers in one launch: 16 waves have 128 vector registers each, all of them used. Scalars go to lanes and back (54 - 62 of
     them; each is on the way from one product to the next), no vector goes to memory."""
     asm = _asm("encoder_text.hip", tmp_path)
     spills = {m.group(1): (int(m.group(2)), int(m.group(3))) for m in re.finditer(
         r"\.name:\s+(\S+)\n(?:(?!\.name:).)*?\.sgpr_spill_count:\s+(\d+)(?:(?!\.name:).)*?\.vgpr_spill_count:\s+(\d+)", asm, re.S)
         if "enc_text_kernel" in m.group(1)}
-    assert len(spills) == 15 and max(s for s, _ in spills.values()) <= 66 and not any(v for _, v in spills.values()), spills
-    for n, (body, _) in _kernels(asm).items():
-        assert "scratch_" not in body, n
+    assert len(spills) == 15 and max(s for s, _ in spills.values()) <= 64 and not any(v for _, v in spills.values()), spills
+    assert not any(scratch for _, scratch in _kernels(asm).values())
