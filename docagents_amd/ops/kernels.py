@@ -602,7 +602,8 @@ def gemm_ln_fit(M: int, hidden: int, ffn: int) -> bool:
 
 
 def attn_ln_fit(M: int, hidden: int, heads: int, texts: int, f16: bool = False) -> bool:
-    """Whether ``gemm_ln`` takes attention inside (``attn``) where an encoder's products take it."""
+    """Whether ``gemm_ln`` takes attention inside (``attn``) where an encoder's products take it: one short text of an encoder that ``enc_text``
+    refuses (fewer than ENC_TEXT_MIN_LAYERS layers, where it is the faster way, more than 32, a feed-forward of more than 4096 columns)."""
     return M <= (32 if hidden > 384 else 64) and hidden <= 1024 and hidden in ((64 * heads,) if f16 else (32 * heads, 64 * heads)) and texts == 1
 
 
@@ -651,7 +652,7 @@ def gemm_ln(a, w, bias, epi: int = EPI_BIAS, norm=None, resid=None, st_out=None,
     return out
 
 
-ENC_TEXT_MIN_LAYERS = 4  # (two: 45 us for 48 of launches one by one; 4: 74 for 94)
+ENC_TEXT_MIN_LAYERS = 4  # (two: 42 us for 48 of launches one by one; 4: 69 for 94)
 
 
 def enc_text_fits(M: int, hidden: int, ffn: int, layers: int, heads: int, texts: int, f16: bool = False) -> bool:
@@ -672,16 +673,26 @@ class TextWaits:
         self._value, at = c_int.from_address(self._word.data_ptr()), c_void_p()
         _check(lib().da_host_address(self._word.data_ptr(), ctypes.byref(at)), "host_address")
         self.at, self.launches = at.value, 0
+        self._lock, self._ran_out, self._told = threading.Lock(), 0, threading.local()
 
     def begin(self) -> None:
         """Before a launch."""
         self.check()
-        self.launches += 1
+        with self._lock:
+            self.launches += 1
 
     def check(self) -> None:
-        """KernelError, once, if a wait ran out in a launch that has run since the last check."""
+        """KernelError if a wait ran out in a launch that has run since this thread's last check (whose launch it was is not known: each thread
+        that uses the encoder is told once)."""
+        told = getattr(self._told, "n", None)
+        if told is None:
+            told = self._told.n = self._ran_out
         if self._value.value:
-            self._value.value = 0
+            with self._lock:
+                self._ran_out += bool(self._value.value)
+                self._value.value = 0
+        if self._ran_out != told:
+            self._told.n = self._ran_out
             raise KernelError("enc_text: a wait ran out, the text's embedding is NaNs")
 
 
@@ -764,7 +775,8 @@ def gemm_rope(a, w, pos, cos_sin, H: int, Hkv: int, D: int, slot, k_cache, v_cac
               kv_out: bool = True) -> torch.Tensor:
     """Prefill QKV projection: qkv = a @ w^T with RoPE applied to the q / k heads and the token's
     k / v written to the KV cache (cache [slots, Hkv, max_seq, D]) — one kernel (gemm8p EPI_ROPE)
-    from 256 rows on, but where ``_rope_apart`` (and not ``_rope_round``); those and shorter prefills run gemm + rope_cache (identical roundings). kv_out=False: the
+    from 256 rows on, but where ``_rope_apart`` (and not ``_rope_round``); those and 65 - 255 rows run gemm + rope_cache (identical
+    roundings). Fewer take that way too, where a decoder does not use ``gemm_dk_rope`` for them. kv_out=False: the
     k / v columns of the result may be left unwritten (the attention reads the cache; see
     flash_attn_varlen kv_cache) — only the q columns are defined."""
     _bf16_cuda(a, "a"); _bf16_cuda(w, "w"); _i32(pos, "pos"); _i32(slot, "slot")

@@ -1,4 +1,6 @@
 """A short text's encoder layers in one launch, against 64-bit arithmetic and the launches one by one."""
+import threading
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -210,6 +212,32 @@ def test_a_wait_that_runs_out_is_told(monkeypatch):
     with pytest.raises(K.KernelError):  # (who did not ask hears of it at the next text)
         enc.encode_one(seq)
     assert torch.equal(enc.encode_one(seq), want)
+
+
+def test_each_thread_is_told():
+    """Two threads with texts of one encoder: who asks first does not keep it from the other."""
+    waits, ask = K.TextWaits(), [threading.Event() for _ in range(2)]
+    told = [[], []]
+
+    def thread(i):
+        waits.check()
+        ask[i].set()
+        ran_out.wait(10)
+        for _ in range(2):
+            try:
+                waits.check()
+            except K.KernelError:
+                told[i].append(1)
+    ran_out, threads = threading.Event(), [threading.Thread(target=thread, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for a in ask:
+        assert a.wait(10)
+    waits._word[0] = 1
+    ran_out.set()
+    for t in threads:
+        t.join()
+    assert told == [[1], [1]]
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
