@@ -417,8 +417,8 @@ class LlamaDecoder:
 
     def _decode_attn(self, qkv, li: int, st: "DecodeState"):
         """RoPE + new-token cache write + decode attention. MHA (Phi-3): one launch — the attention
-        kernel rotates q / the new k itself and writes the new k / v to the cache; GQA: rope_cache,
-        then the MFMA decode kernel."""
+        kernel rotates q / the new k itself and writes the new k / v to the cache. GQA: rope_cache, then the MFMA decode
+        kernel, for rows whose projection does not rotate them itself (``dk_rope_fits``: one row, more than 64, a TP slice)."""
         c, o, cache = self.cfg, self.ops, self.cache
         D, hl, kl = c.head_dim, self.hl, self.kl
         if hl == kl and _FUSED_ROPE_DECODE:
