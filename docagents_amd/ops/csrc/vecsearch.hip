@@ -750,6 +750,8 @@ topk_merge_kernel(const float* __restrict__ cand_s, const int* __restrict__ cand
 // requests of 64 B, 512 a tile, of which a CU has 256 on their way (24 tiles 13.6 -> 8.3 us; of up to 8 tiles the ring is 1 us
 // slower). Whole searches, us: 102624 x 768, 10 queries, K = 20 50.8 -> 45.1, 110468 x 1024, 42, K = 14 64.3 -> 60.0, 52331 x 1024,
 // one, K = 14 41.3 -> 36.3, 10000 x 768, 24, K = 5 17.1 -> 15.2, 958291 x 1024, 18, K = 12 340 -> 335; 20000 x 768, 128, K = 5 26.9 -> 27.3.
+// Groups that are none (few rows reach the least similarity) are no tiles: 100000 x 1024, 17 queries, K = 32, rows of 0.95 and more 47.2 us
+// with the ring's steps left out for them, 60.0 without.
 constexpr int TP_WAVES = 8, TP_CAP = 1024, TP_FOLD = 256, TP_RING = 3;
 
 // The largest bound, to its upper 20 bits, that at least `need` of the 8 keys of each lane reach (0: there are not as many).
@@ -775,7 +777,7 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
   static_assert(TP_WAVES == 8, "a key of each thread: 8 per lane of a wave");
   __shared__ float cs[TP_WAVES][TL_SL], cand_s[TP_CAP];
   __shared__ int ci[TP_WAVES][TL_SL], cand_i[TP_CAP];
-  __shared__ int groups[TK_MAX], count, reach[32], equal[TP_WAVES];
+  __shared__ int groups[TK_MAX], n_groups, count, reach[32], equal[TP_WAVES];
   __shared__ float bound;
   __shared__ unsigned keys[nt], bkey;
   __shared__ __attribute__((aligned(16))) bf16_t sq[d];
@@ -914,7 +916,9 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
       top_order(top, out, q);
       return;
     }
-    if (lane < K) groups[lane] = ci[0][lane];
+    const unsigned long long real = __ballot(lane < K && ci[0][min(lane, K - 1)] >= 0);  // (fewer than K where few rows reach thr)
+    if ((real >> lane) & 1) groups[__popcll(real & ((1ull << lane) - 1))] = ci[0][lane];
+    if (lane == 0) n_groups = __popcll(real);
     float low = lane < K && ci[0][lane] >= 0 ? cs[0][lane] : lane < K ? -INFINITY : INFINITY;  // the K-th best group
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) low = fminf(low, __shfl_xor(low, o, 64));
@@ -933,9 +937,10 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
     const int r = 4 * i + (lane >> 4);
     off[i] = (unsigned)(r * d * 2 + (((lane & 15) ^ r) << 4));
   }
+  const int all = n_groups << lg;
   // the wave's i-th tile: its first row, and the end of the run (0: none)
   auto tile = [&](int i, int& row0, int& end) __attribute__((always_inline)) {
-    const int it = wid + i * TP_WAVES, g = it < K << lg ? groups[it >> lg] : -1;
+    const int it = wid + i * TP_WAVES, g = it < all ? groups[it >> lg] : -1;
     const long first = (long)(g / run_slots) * run_rows;
     row0 = g < 0 ? 0 : (int)first + ((((g % run_slots) << lg) + (it & ((1 << lg) - 1))) * 16);
     end = g < 0 ? 0 : (int)min((long)N, first + run_rows);
@@ -949,8 +954,8 @@ topk_pick_kernel(const float* __restrict__ gm, int GT, int run_slots, int run_ro
     for (int i = 0; i < 4; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (vs_lds_t)(mine + slot * 4096 + i * 1024), 16, off[i], g * 256, 0, 0);
   };
-  const int tiles = ((K << lg) - wid + TP_WAVES - 1) / TP_WAVES;
-  const bool one = K << lg <= TP_WAVES;
+  const int tiles = (all - wid + TP_WAVES - 1) / TP_WAVES;
+  const bool one = all <= TP_WAVES;
   for (int again = 0; again < 2; ++again) {
     int row0, end, row1 = 0, end1 = 0, slot = 0;
     tile(0, row0, end);
